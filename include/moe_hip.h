@@ -206,16 +206,15 @@ typedef struct MoeForwardArgs {
   int add_residual;              /* out = x + moe_out, added in f32 before the one bf16 rounding */
 } MoeForwardArgs;
 
-/* Host-side objects moe_forward creates.  No device memory is ever allocated.  With a shared expert (SI > 0) the
- * call (a) creates, on the first such call on a device, ONE side stream for that device (default priority, kept until
- * the process ends, shared by every caller stream and host thread) and (b) creates two or three hipEvents per call and
- * destroys them before returning (quantised activations ready, shared expert done, and for large batches a fork
- * at the call's start), so that calls on different streams share no event state.  Consequences: if the caller's
- * stream is being captured into a HIP graph, the side stream joins that capture through the first of these events
- * for the length of the call; a second host thread that makes an
- * eager moe_forward call on the same device while another thread is inside a capturing call would enqueue onto a
- * capturing stream -- that combination is unsupported (serialise such calls, or capture on one thread only).  Without
- * a shared expert no stream or event is created. */
+/* Host-side objects moe_forward creates.  No device memory is ever allocated.  A large batch (M * D above 2 M elements)
+ * with a shared expert (SI > 0) runs the shared expert beside the routing chain: the call (a) creates, on the first such
+ * call on a device, ONE side stream for that device (default priority, kept until the process ends, shared by every
+ * caller stream and host thread) and (b) uses three hipEvents per host thread and device, created on first use, so
+ * that calls of different threads share no event state.  Consequences: if the caller's stream is being captured into
+ * a HIP graph, the side stream joins that capture through the first of these events for the length of the call; a
+ * second host thread that makes such an eager call on the same device while another thread is inside a capturing one
+ * would enqueue onto a capturing stream -- that combination is unsupported (serialise such calls, or capture on one
+ * thread only).  Every other call creates neither stream nor event. */
 MOE_API size_t moe_forward_workspace_bytes(int M, int D, int E, int k, int I, int SI);
 MOE_API int moe_forward(const MoeForwardArgs* args, void* ws, size_t ws_bytes, moe_stream_t stream);
 

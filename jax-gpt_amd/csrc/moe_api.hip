@@ -86,11 +86,11 @@ struct Carver {
 };
 
 struct ForwardBuffers {
-  int32_t *idx, *group_sizes, *group_offsets, *sorted_token_ids, *inv_perm, *dense_off;
+  int32_t *idx, *group_sizes, *group_offsets, *sorted_token_ids, *inv_perm;
   float *w, *sx, *sh, *shs, *shared_gate, *sx_listed, *sx_blocked;
   uint8_t *xq, *hq, *hsq;
-  void *y, *ys, *permute_ws, *gemm_ws, *gemm_ws_shared, *router_ws, *normed;
-  size_t permute_ws_bytes, gemm_ws_bytes, gemm_ws_shared_bytes, router_ws_bytes, total;
+  void *y, *ys, *permute_ws, *gemm_ws, *router_ws, *normed;
+  size_t permute_ws_bytes, gemm_ws_bytes, router_ws_bytes, total;
 };
 
 ForwardBuffers carve(void* ws, int M, int D, int E, int k, int I, int SI, bool router) {
@@ -103,14 +103,10 @@ ForwardBuffers carve(void* ws, int M, int D, int E, int k, int I, int SI, bool r
   b.group_offsets = (int32_t*)c.take((size_t)(E + 1) * 4);
   b.sorted_token_ids = (int32_t*)c.take(R * 4);
   b.inv_perm = (int32_t*)c.take(R * 4);
-  b.dense_off = (int32_t*)c.take(8);   // (stands in for the shared expert's group offsets, which its pre-built tile list makes unread)
   b.permute_ws_bytes = moe_permute_workspace_bytes(M, k, E);
   b.permute_ws = c.take(b.permute_ws_bytes);
   b.gemm_ws_bytes = moe_gemm_workspace_bytes((int)R, E, I > D ? I : D);
   b.gemm_ws = c.take(b.gemm_ws_bytes);        // tile list of the routed GEMMs (gate/up and down share it)
-  // the shared expert runs beside the routed ones on its own stream: its launches need their own work lists
-  b.gemm_ws_shared_bytes = SI ? moe_gemm_workspace_bytes(M, 1, SI > D ? SI : D) : 0;
-  b.gemm_ws_shared = SI ? c.take(b.gemm_ws_shared_bytes) : nullptr;
   b.xq = (uint8_t*)c.take((size_t)M * D);
   b.sx = (float*)c.take((size_t)M * (D / 128) * 4);
   // block-major copies of the activation scales for large batches (GemmScales): routed rows in sorted order,
@@ -141,6 +137,10 @@ int quantise(const MoeForwardArgs* a, const ForwardBuffers& b, float* sx_blocked
     return moe_rmsnorm_quant_impl(a->x, a->norm_weight, a->norm_eps, a->M, a->D, b.normed, b.xq, b.sx, sx_blocked, stream);
   return moe_quant_act_impl(a->x, a->M, a->D, b.xq, b.sx, sx_blocked, stream);
 }
+
+// Whether a call with a shared expert runs it inside the routed launches (true) or on the side stream.  From about
+// 2 M activation elements on, the shared expert's GEMMs fill the gap that routing and permutation leave.
+bool small_batch(int M, int D) { return (long long)M * D <= (1ll << 21); }
 }  // namespace
 
 extern "C" size_t moe_forward_workspace_bytes(int M, int D, int E, int k, int I, int SI) {
@@ -197,27 +197,21 @@ extern "C" int moe_forward(const MoeForwardArgs* a, void* ws, size_t ws_bytes, m
               "forward: unknown routing %d", a->routing);
   int rc;
 
-  // With a shared expert the call forks: the side stream runs the shared expert while the caller's stream routes,
-  // permutes and runs the routed experts; the combine waits for the shared expert's output.  (Event record / wait
-  // is also the pattern a capturing caller's graph turns into forks and joins.)
-  //   Large batches fork at once: the side stream quantises the activations and starts the shared expert while the
-  // caller's stream routes and permutes; the routed gate/up GEMM waits for the quantised activations.
-  //   Small batches are bound by launch latency, so nothing may stand between the caller's stream and the routed
-  // GEMMs: the activations are quantised on the caller's stream, the side stream waits for them, and the shared
-  // expert's launches are enqueued after the routed ones (they still run beside them: the routed GEMMs take far longer).
-  const bool small_batch = (long long)a->M * a->D <= (1ll << 21);
+  // The shared expert.  Small batches run it inside the routed experts' two GEMM launches: they are bound by launches
+  // and by the host work behind them, and a second stream costs seven more of those (two events recorded and waited
+  // for, three launches) where one more group of work items costs none: 1 token of the mini layer 97 -> 51 us, of the
+  // DeepSeek-V3 layer 115 -> 100 us, 64 tokens of it 973 -> 965 us.
+  //   Large batches fork at once: the side stream quantises the activations and runs the shared expert while the
+  // caller's stream routes and permutes; the routed gate/up GEMM waits for the quantised activations, the combine for
+  // the shared expert's output.  (Event record / wait is also the pattern that a capturing caller's graph turns into
+  // forks and joins.)
+  const bool fork = a->SI && !small_batch(a->M, a->D);
   hipStream_t side = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_quant = nullptr, ev_join = nullptr;
+  CallEvents* ev = nullptr;
   int rc_shared = MOE_OK;
-  bool quant_joined = true;
-  bool side_forked = false;   // the side stream has been made to wait for work of this call on the caller's stream
-  // the shared expert's one group and its tile list (they depend on M alone: enqueued ahead of the quantiser where
-  // the side stream runs it, so that nothing stands between the quantiser and the shared gate/up GEMM)
-  auto list_shared = [&]() {
-    if (!rc_shared)
-      rc_shared = moe_gemm_build_dense_tile_list(a->M, b.gemm_ws_shared, b.gemm_ws_shared_bytes, (moe_stream_t)side);
-  };
-  auto launch_shared = [&]() {
+  bool quant_joined = !fork;
+  DenseGemm shared_gateup{}, shared_down{};
+  if (a->SI) {
     GemmScales sc = moe_row_major_scales(a->D, a->SI);
     const float* sx_shared = b.sx;
     if (blocked_scales) {   // (block-major scales in token order: written by the quantiser itself)
@@ -225,76 +219,43 @@ extern "C" int moe_forward(const MoeForwardArgs* a, void* ws, size_t ws_bytes, m
       sc.in_row = 1, sc.in_kb = a->M, sc.in_listed = true;
       if (!a->out_shs) sc.out_row = 1, sc.out_cb = a->M;   // (a debug copy of the h scales keeps the documented layout)
     }
-    if (!rc_shared)
-      rc_shared = moe_gemm_gateup_impl(b.xq, sx_shared, nullptr, a->ws_gate, a->sws_gate, a->ws_up, a->sws_up, b.dense_off,
-                                       1, a->M, a->D, a->SI, hsq, shs, b.gemm_ws_shared, b.gemm_ws_shared_bytes, true, sc,
-                                       (moe_stream_t)side);
-    if (!rc_shared)   // same rows, same tile height: the list the gate/up launch built serves the down launch too
-      rc_shared = moe_gemm_down_impl(hsq, shs, a->ws_down, a->sws_down, b.dense_off, 1, a->M, a->SI, a->D, ys,
-                                     b.gemm_ws_shared, b.gemm_ws_shared_bytes, true,
-                                     GemmScales{sc.out_row, sc.out_cb, true, 0, 0}, (moe_stream_t)side);
-  };
-  bool shared_pending = false;
+    shared_gateup = DenseGemm{{b.xq, sx_shared, nullptr, a->ws_gate, a->sws_gate, a->ws_up, a->sws_up, a->D, a->SI, hsq, shs, sc}, a->M};
+    shared_down = DenseGemm{{hsq, shs, nullptr, a->ws_down, a->sws_down, nullptr, nullptr, a->SI, a->D, ys, nullptr,
+                             GemmScales{sc.out_row, sc.out_cb, true, 0, 0}}, a->M};
+  }
+  float* sx_blocked = a->SI && blocked_scales ? b.sx_blocked : nullptr;
   // Where the quantiser would run on the caller's stream just ahead of the routing kernel, the routing launch
   // carries its blocks instead (QuantJob: the two are independent; one launch less and they overlap).  Not with
   // an RMSNorm in front: the router then reads what the quantiser writes.
-  const bool quant_in_route = (!a->SI || small_batch) && !a->norm_weight && a->M > 0;
+  const bool quant_in_route = !fork && !a->norm_weight;
   QuantJob quant_job{};
-  if (quant_in_route &&
-      (rc = moe_quant_act_job(a->x, a->M, a->D, b.xq, b.sx, (a->SI && blocked_scales) ? b.sx_blocked : nullptr, &quant_job)))
-    return rc;
-  if (a->SI) {
+  if (quant_in_route) {
+    if ((rc = moe_quant_act_job(a->x, a->M, a->D, b.xq, b.sx, sx_blocked, &quant_job))) return rc;
+  } else if (!fork) {
+    if ((rc = quantise(a, b, sx_blocked, stream))) return rc;
+  } else {
     if ((rc = side_stream(&side))) return rc;
-    CallEvents* ev = nullptr;
     if ((rc = call_events(&ev))) return rc;
-    ev_fork = ev->fork, ev_quant = ev->quant, ev_join = ev->join;
-    if (!small_batch) {
-      hipError_t e = hipEventRecord(ev_fork, main_s);
-      if (e == hipSuccess) e = hipStreamWaitEvent(side, ev_fork, 0);
-      if (e != hipSuccess) return moe_check_hip(e, "forward: fork");
-      side_forked = true;
-    }
-    if (small_batch) {
-      if (!quant_in_route) {
-        rc_shared = quantise(a, b, blocked_scales ? b.sx_blocked : nullptr, stream);
-        if (!rc_shared) rc_shared = moe_check_hip(hipEventRecord(ev_quant, main_s), "forward: quant event");
-        if (!rc_shared) {
-          rc_shared = moe_check_hip(hipStreamWaitEvent(side, ev_quant, 0), "forward: fork");
-          side_forked = !rc_shared;
-        }
-      }   // (else: the same record and wait follow the routing launch, below)
-      shared_pending = true;
-    } else {
-      quant_joined = false;
-      list_shared();
-      if (!rc_shared) rc_shared = quantise(a, b, blocked_scales ? b.sx_blocked : nullptr, (moe_stream_t)side);
-      if (!rc_shared) rc_shared = moe_check_hip(hipEventRecord(ev_quant, side), "forward: quant event");
-      launch_shared();
-    }
-  } else if (!quant_in_route) {
-    if ((rc = quantise(a, b, nullptr, stream))) return rc;
+    hipError_t e = hipEventRecord(ev->fork, main_s);
+    if (e == hipSuccess) e = hipStreamWaitEvent(side, ev->fork, 0);
+    if (e != hipSuccess) return moe_check_hip(e, "forward: fork");
+    rc_shared = quantise(a, b, sx_blocked, (moe_stream_t)side);
+    if (!rc_shared) rc_shared = moe_check_hip(hipEventRecord(ev->quant, side), "forward: quant event");
+    if (!rc_shared) rc_shared = moe_gemm_gateup_impl(nullptr, &shared_gateup, (moe_stream_t)side);
+    if (!rc_shared) rc_shared = moe_gemm_down_impl(nullptr, &shared_down, (moe_stream_t)side);
   }
   // Once the side stream has been forked off this call, the join is enqueued on every path out of here, so that the
-  // caller's stream (or the graph it is being captured into) never loses track of the side stream.  Before the
-  // fork the side stream holds nothing of this call, and a wait on it would tie the caller's stream -- under
-  // capture: the caller's graph -- to work that does not belong to it.
+  // caller's stream (or the graph it is being captured into) never loses track of the side stream.
   auto join = [&](int code) {
-    if (!a->SI) return code;
-    if (shared_pending && side_forked && !code && !rc_shared) {
-      list_shared();
-      launch_shared();
-    }
-    shared_pending = false;
-    if (!side_forked) return code ? code : rc_shared;
-    hipError_t e1 = hipEventRecord(ev_join, side);
-    hipError_t e2 = hipStreamWaitEvent(main_s, ev_join, 0);
+    if (!fork) return code;
+    hipError_t e1 = hipEventRecord(ev->join, side);
+    hipError_t e2 = hipStreamWaitEvent(main_s, ev->join, 0);
     if (code) return code;
     if (rc_shared) return rc_shared;
     if (e1 != hipSuccess) return moe_check_hip(e1, "forward: join");
     return moe_check_hip(e2, "forward: join");
   };
 
-  if (small_batch && rc_shared) return join(rc_shared);
   // With a router weight the routing kernel adds the matmul's split-K partial sums itself: the (M, E) logits
   // are written only when out_logits asks for them.
   LogitSource src{a->logits, nullptr, 0, a->E, nullptr, nullptr};
@@ -303,7 +264,7 @@ extern "C" int moe_forward(const MoeForwardArgs* a, void* ws, size_t ws_bytes, m
     // the router reads the normalised activations, which the (possibly forked) quantiser writes
     if (a->norm_weight && !quant_joined) {
       if (rc_shared) return join(rc_shared);
-      if ((rc = moe_check_hip(hipStreamWaitEvent(main_s, ev_quant, 0), "forward: quant join"))) return join(rc);
+      if ((rc = moe_check_hip(hipStreamWaitEvent(main_s, ev->quant, 0), "forward: quant join"))) return join(rc);
       quant_joined = true;
     }
     int splits = 0, n_cols = 0;
@@ -321,12 +282,6 @@ extern "C" int moe_forward(const MoeForwardArgs* a, void* ws, size_t ws_bytes, m
     rc = moe_route_sigmoid_grouped_impl(src, a->bias, a->M, a->E, a->n_group, a->topk_group, a->k, a->renorm,
                                         a->routed_scale, idx, w, stream, carried);
   if (rc) return join(rc);
-  if (quant_in_route && a->SI) {   // the side stream's shared expert waits for the activations quantised above
-    hipError_t e = hipEventRecord(ev_quant, main_s);
-    if (e == hipSuccess) e = hipStreamWaitEvent(side, ev_quant, 0);
-    if (e != hipSuccess) return join(moe_check_hip(e, "forward: quant event"));
-    side_forked = true;
-  }
   // the permutation kernels also list the routed GEMMs' row tiles (they hold every expert's row range anyway)
   TileList tiles;
   if ((rc = moe_gemm_tile_list(R, a->E, b.gemm_ws, b.gemm_ws_bytes, &tiles))) return join(rc);
@@ -335,7 +290,7 @@ extern "C" int moe_forward(const MoeForwardArgs* a, void* ws, size_t ws_bytes, m
     return join(rc);
   if (!quant_joined) {
     if (rc_shared) return join(rc_shared);
-    if ((rc = moe_check_hip(hipStreamWaitEvent(main_s, ev_quant, 0), "forward: quant join"))) return join(rc);
+    if ((rc = moe_check_hip(hipStreamWaitEvent(main_s, ev->quant, 0), "forward: quant join"))) return join(rc);
   }
   GemmScales sc = moe_row_major_scales(a->D, a->I);
   const float* sx_routed = b.sx;
@@ -345,12 +300,14 @@ extern "C" int moe_forward(const MoeForwardArgs* a, void* ws, size_t ws_bytes, m
     sc.in_row = 1, sc.in_kb = R, sc.in_listed = true;
     if (!a->out_sh) sc.out_row = 1, sc.out_cb = R;
   }
-  if ((rc = moe_gemm_gateup_impl(b.xq, sx_routed, stid, a->w_gate, a->sw_gate, a->w_up, a->sw_up, b.group_offsets, a->E,
-                                 R, a->D, a->I, hq, sh, b.gemm_ws, b.gemm_ws_bytes, true, sc, stream)))
-    return join(rc);
-  if ((rc = moe_gemm_down_impl(hq, sh, a->w_down, a->sw_down, b.group_offsets, a->E, R, a->I, a->D, y,
-                               b.gemm_ws, b.gemm_ws_bytes, true, GemmScales{sc.out_row, sc.out_cb, true, 0, 0}, stream)))
-    return join(rc);
+  const RoutedGemm routed_gateup{{b.xq, sx_routed, stid, a->w_gate, a->sw_gate, a->w_up, a->sw_up, a->D, a->I, hq, sh, sc},
+                                 b.group_offsets, a->E, R, b.gemm_ws, b.gemm_ws_bytes, true};
+  const RoutedGemm routed_down{{hq, sh, nullptr, a->w_down, a->sw_down, nullptr, nullptr, a->I, a->D, y, nullptr,
+                                GemmScales{sc.out_row, sc.out_cb, true, 0, 0}},
+                               b.group_offsets, a->E, R, b.gemm_ws, b.gemm_ws_bytes, true};
+  const bool together = a->SI && !fork;
+  if ((rc = moe_gemm_gateup_impl(&routed_gateup, together ? &shared_gateup : nullptr, stream))) return join(rc);
+  if ((rc = moe_gemm_down_impl(&routed_down, together ? &shared_down : nullptr, stream))) return join(rc);
   if ((rc = join(MOE_OK))) return rc;
   return moe_combine(y, w, inv, a->SI ? ys : nullptr, shared_gate, a->add_residual ? a->x : nullptr, a->M, a->k,
                      a->D, a->out, stream);

@@ -273,7 +273,6 @@ int moe_route_sigmoid_grouped_impl(const LogitSource& src, const float* bias, in
 // own.  moe_gemm_tile_list describes the list the GEMMs of (R rows, E experts) expect in ws, so that the permutation
 // kernels, which hold every expert's row range anyway, can write it (moe_permute_impl) and no launch is spent on it.
 int moe_gemm_tile_list(int R, int E, void* ws, size_t ws_bytes, TileList* list);
-int moe_gemm_build_dense_tile_list(int R, void* ws, size_t ws_bytes, moe_stream_t stream);
 // the activation quantisers with an optional second copy of the scales, block-major in row order ((K/128, R): what
 // GemmScales{1, R} reads) -- spares the shared expert of a large batch the separate transposition
 int moe_quant_act_impl(const void* x_bf16, int R, int K, uint8_t* xq, float* sx, float* sx_blocked, moe_stream_t stream);
@@ -294,13 +293,38 @@ struct GemmScales {
   bool stream_out;       // down only, set by the launch: y is stored with non-temporal stores
 };
 inline GemmScales moe_row_major_scales(int K, int I) { return GemmScales{K / 128, 1, false, I / 128, 1}; }
-int moe_gemm_gateup_impl(const uint8_t* xq, const float* sx, const int32_t* row_ids, const uint8_t* w_gate,
-                         const float* sw_gate, const uint8_t* w_up, const float* sw_up, const int32_t* group_offsets,
-                         int E, int R, int D, int I, uint8_t* hq, float* sh, void* ws, size_t ws_bytes, bool list_built,
-                         GemmScales sc, moe_stream_t stream);
-int moe_gemm_down_impl(const uint8_t* hq, const float* sh, const uint8_t* w_down, const float* sw_down,
-                       const int32_t* group_offsets, int E, int R, int I, int D, void* y_bf16, void* ws,
-                       size_t ws_bytes, bool list_built, GemmScales sc, moe_stream_t stream);
+// Operands of one grouped GEMM.  Gate/up: w0 = gate, w1 = up, K = D, N = I, out = h codes, out_scale = h scales; down:
+// w0 = down, K = I, N = D, out = y (w1, sw1, out_scale and row_ids null).
+struct GemmOperands {
+  const uint8_t* xq;
+  const float* sx;
+  const int32_t* row_ids;
+  const uint8_t* w0;
+  const float* sw0;
+  const uint8_t* w1;
+  const float* sw1;
+  int K, N;
+  void* out;
+  float* out_scale;
+  GemmScales sc;
+};
+// the routed experts: R rows in E groups through a work list in ws, which the launch builds unless it is there already
+struct RoutedGemm {
+  GemmOperands op;
+  const int32_t* group_offsets;
+  int E, R;
+  void* ws;
+  size_t ws_bytes;
+  bool list_built;
+};
+// one group of all rows (the shared expert): no list, no workspace
+struct DenseGemm {
+  GemmOperands op;
+  int rows;
+};
+// One launch for either or both (nullptr: none).
+int moe_gemm_gateup_impl(const RoutedGemm* routed, const DenseGemm* dense, moe_stream_t stream);
+int moe_gemm_down_impl(const RoutedGemm* routed, const DenseGemm* dense, moe_stream_t stream);
 
 #define MOE_REQUIRE(cond, code, ...) \
   do {                               \

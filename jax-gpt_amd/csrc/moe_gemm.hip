@@ -75,16 +75,12 @@ constexpr int ROTC = 2;       // MFMA groups by which wave set 1 trails wave set
 
 // One workgroup lists the row tiles of every expert (an expert's tiles side by side; which expert where: see
 // moe_tile_first); thread e owns expert e.
-// (dense_rows >= 0: one group of that many rows, whatever group_offsets holds -- the shared expert)
-__global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __restrict__ group_offsets, int E,
-                                                          TileList l, int dense_rows) {
+__global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __restrict__ group_offsets, int E, TileList l) {
   __shared__ int s_rows[1024];
   __shared__ int s_key[1024];
   const int e = threadIdx.x;
   int start = 0, rows = 0;
-  if (dense_rows >= 0) {
-    rows = e == 0 ? dense_rows : 0;
-  } else if (e < E) {
+  if (e < E) {
     start = group_offsets[e];
     rows = group_offsets[e + 1] - start;
   }
@@ -607,72 +603,103 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
   }
 }
 
-template <int MODE>
-__global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(
-    const uint8_t* __restrict__ xq, const float* __restrict__ sx, const int32_t* __restrict__ row_ids,
-    const uint8_t* __restrict__ w0, const float* __restrict__ sw0, const uint8_t* __restrict__ w1,
-    const float* __restrict__ sw1, TileHeader* hdr, const TileEntry* __restrict__ tiles, int K,
-    int N, void* __restrict__ out, float* __restrict__ out_scale, const GemmScales sc) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  // work items = (row tile, column block) pairs in [expert][column block][row tile] order, dealt to the 8 XCDs in
-  // contiguous ranges of about equal cost (workgroup ids are issued round-robin over XCDs)
-  const int ncb = MODE == MODE_GATEUP ? N / 128 : (N + 255) / 256;
-  const int xcd = blockIdx.x & 7;
-  int item_id = (int)((hdr->xcd_q[xcd] * ncb) >> kTileQBits) + (int)(blockIdx.x >> 3);
-  const int share_end = (int)((hdr->xcd_q[xcd + 1] * ncb) >> kTileQBits);
-  if (item_id >= share_end) {
-    // behind the XCD's fixed share: the pool of the smallest experts' items, drawn one at a time by whoever gets
-    // there (TileHeader); an XCD may draw up to twice its eighth of it
-    const int pool_first = hdr->n_static * ncb;
-    const int pool_items = (hdr->n_tiles - hdr->n_static) * ncb;
-    if (pool_items == 0 || item_id - share_end >= moe_pool_workgroups(pool_items)) return;   // (uniform: the whole workgroup leaves)
-    int* slot = (int*)lds;
-    if (threadIdx.x == 0) *slot = atomicAdd(&hdr->pool_next[MODE], 1);   // (the one field of the list a GEMM writes)
-    __syncthreads();
-    const int drawn = *slot;
-    __syncthreads();   // (the work item's first copies overwrite the slot)
-    if (drawn >= pool_items) return;
-    item_id = pool_first + drawn;
+// Column block and row tile of the `local`-th work item of an expert of nt row tiles and ncb column blocks.
+__device__ __forceinline__ void expert_item(int local, int nt, int ncb, int& col_block, int& rt) {
+  if (nt < 16) {
+    col_block = nt == 1 ? local : local / nt;
+    rt = local - col_block * nt;
+    return;
   }
+  // An expert of many row tiles goes through its column blocks once per group of 8 to 11 row tiles: the 32 CUs
+  // of an XCD then work on about 8 row tiles x 4 column blocks at a time (12 distinct operand tiles per K step)
+  // instead of 32 row tiles of one column block (33 distinct tiles, every CU pulling the same weight lines at
+  // once): 32 row tiles per expert ran 19 % slower than 8.  Below 16 tiles a split does not pay (11 tiles as
+  // 6 + 5 measured 1 % slower than unsplit).
+  const int ng = nt >> 3;
+  const int base = nt / ng, extra = nt - base * ng;   // the first `extra` groups hold base + 1 tiles
+  const int big = (base + 1) * ncb * extra;
+  int sz, l2, t0;
+  if (local < big) {
+    sz = base + 1;
+    const int g = local / (sz * ncb);
+    l2 = local - g * sz * ncb;
+    t0 = g * sz;
+  } else {
+    sz = base;
+    const int l = local - big, g = l / (sz * ncb);
+    l2 = l - g * sz * ncb;
+    t0 = extra * (base + 1) + g * sz;
+  }
+  col_block = l2 / sz;
+  rt = t0 + (l2 - col_block * sz);
+}
+
+// The first dense_blocks workgroups serve `dense`, one group of dense_rows rows (the shared expert), whose work items
+// follow from the row count alone; the rest serve the routed experts through the work list (hdr null: none).  A
+// decode-sized layer runs both in one launch: the shared expert's items are few and as long as the others', and the
+// launches, the second stream and the events between them cost it more than the arithmetic.  DENSE false: routed
+// items only, as a kernel of its own, because choosing between the two operand sets costs every item of a large
+// launch some 0.7 us (0.8 % of the prefill step).
+template <int MODE, bool DENSE>
+__global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands routed, TileHeader* hdr,
+                                                            const TileEntry* __restrict__ tiles, const GemmOperands dense,
+                                                            int dense_rows, int dense_blocks) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const bool is_dense = DENSE && (int)blockIdx.x < dense_blocks;   // (dense_blocks is a multiple of 8: the XCD is blockIdx % 8 for both)
+  const int xcd = blockIdx.x & 7;
+  const int K = is_dense ? dense.K : routed.K, N = is_dense ? dense.N : routed.N;
+  const int ncb = MODE == MODE_GATEUP ? N / 128 : (N + 255) / 256;
   Item item;
-  {
+  if (is_dense) {
+    // contiguous eighths of the items, so that row tiles that share a weight slab run under one L2
+    const int nt = moe_tile_count(dense_rows), items = nt * ncb;
+    const int per = dense_blocks >> 3;
+    const int local = xcd * per + (int)(blockIdx.x >> 3);
+    if (local >= items) return;
+    int rt, t0, tn;
+    expert_item(local, nt, ncb, item.col_block, rt);
+    moe_tile_span(dense_rows, nt, rt, t0, tn);
+    item.expert = 0;
+    item.row_start = t0;
+    item.row_count = tn;
+  } else {
+    // work items = (row tile, column block) pairs in [expert][column block][row tile] order, dealt to the 8 XCDs in
+    // contiguous ranges of about equal cost (workgroup ids are issued round-robin over XCDs)
+    int item_id = (int)((hdr->xcd_q[xcd] * ncb) >> kTileQBits) + (((int)blockIdx.x - (DENSE ? dense_blocks : 0)) >> 3);
+    const int share_end = (int)((hdr->xcd_q[xcd + 1] * ncb) >> kTileQBits);
+    if (item_id >= share_end) {
+      // behind the XCD's fixed share: the pool of the smallest experts' items, drawn one at a time by whoever gets
+      // there (TileHeader); an XCD may draw up to twice its eighth of it
+      const int pool_first = hdr->n_static * ncb;
+      const int pool_items = (hdr->n_tiles - hdr->n_static) * ncb;
+      if (pool_items == 0 || item_id - share_end >= moe_pool_workgroups(pool_items)) return;   // (uniform: the whole workgroup leaves)
+      int* slot = (int*)lds;
+      if (threadIdx.x == 0) *slot = atomicAdd(&hdr->pool_next[MODE], 1);   // (the one field of the list a GEMM writes)
+      __syncthreads();
+      const int drawn = *slot;
+      __syncthreads();   // (the work item's first copies overwrite the slot)
+      if (drawn >= pool_items) return;
+      item_id = pool_first + drawn;
+    }
     const TileEntry te = tiles[item_id / ncb];   // entries [first_tile, first_tile + tiles) all describe this expert
     const int nt = moe_tile_count(te.rows);
-    const int local = item_id - te.first_tile * ncb;
-    int rt;
-    if (nt < 16) {
-      item.col_block = nt == 1 ? local : local / nt;
-      rt = local - item.col_block * nt;
-    } else {
-      // An expert of many row tiles goes through its column blocks once per group of 8 to 11 row tiles: the 32 CUs
-      // of an XCD then work on about 8 row tiles x 4 column blocks at a time (12 distinct operand tiles per K step)
-      // instead of 32 row tiles of one column block (33 distinct tiles, every CU pulling the same weight lines at
-      // once): 32 row tiles per expert ran 19 % slower than 8.  Below 16 tiles a split does not pay (11 tiles as
-      // 6 + 5 measured 1 % slower than unsplit).
-      const int ng = nt >> 3;
-      const int base = nt / ng, extra = nt - base * ng;   // the first `extra` groups hold base + 1 tiles
-      const int big = (base + 1) * ncb * extra;
-      int sz, l2, t0;
-      if (local < big) {
-        sz = base + 1;
-        const int g = local / (sz * ncb);
-        l2 = local - g * sz * ncb;
-        t0 = g * sz;
-      } else {
-        sz = base;
-        const int l = local - big, g = l / (sz * ncb);
-        l2 = l - g * sz * ncb;
-        t0 = extra * (base + 1) + g * sz;
-      }
-      item.col_block = l2 / sz;
-      rt = t0 + (l2 - item.col_block * sz);
-    }
-    item.expert = te.expert;
-    int t0, tn;
+    int rt, t0, tn;
+    expert_item(item_id - te.first_tile * ncb, nt, ncb, item.col_block, rt);
     moe_tile_span(te.rows, nt, rt, t0, tn);
+    item.expert = te.expert;
     item.row_start = te.row_start + t0;
     item.row_count = tn;
   }
+  const uint8_t* xq = is_dense ? dense.xq : routed.xq;
+  const float* sx = is_dense ? dense.sx : routed.sx;
+  const int32_t* row_ids = is_dense ? nullptr : routed.row_ids;
+  const uint8_t* w0 = is_dense ? dense.w0 : routed.w0;
+  const float* sw0 = is_dense ? dense.sw0 : routed.sw0;
+  const uint8_t* w1 = is_dense ? dense.w1 : routed.w1;
+  const float* sw1 = is_dense ? dense.sw1 : routed.sw1;
+  void* out = is_dense ? dense.out : routed.out;
+  float* out_scale = is_dense ? dense.out_scale : routed.out_scale;
+  const GemmScales sc = is_dense ? dense.sc : routed.sc;
   const int rows = __builtin_amdgcn_readfirstlane(item.row_count);
 #define MOE_ITEM(XF) item_body<MODE, XF>(item, lds, xq, sx, row_ids, w0, sw0, w1, sw1, K, N, out, out_scale, sc)
   switch ((rows + 31) >> 5) {
@@ -695,31 +722,67 @@ TileList tile_list(void* ws, int R, int E) {
   return TileList{max_tiles_for(R, E), (TileHeader*)ws, (TileEntry*)((char*)ws + sizeof(TileHeader))};
 }
 
+int check_operands(const GemmOperands& op, int rows, int E, int mode, const char* what) {
+  MOE_REQUIRE((rows == 0 || (op.xq && op.sx && op.out && (mode == MODE_DOWN || op.out_scale))) && op.w0 && op.sw0 &&
+                  (mode == MODE_DOWN || (op.w1 && op.sw1)), MOE_ERR_NULL, "%s: null pointer", what);
+  MOE_REQUIRE(E >= 1 && E <= 1024 && rows >= 0 && op.K > 0 && op.N > 0 && op.K % 128 == 0 && op.N % 128 == 0, MOE_ERR_BAD_SHAPE,
+              "%s: need contraction and output sizes in multiples of 128 and 1 <= E <= 1024, got E=%d rows=%d K=%d N=%d", what, E,
+              rows, op.K, op.N);
+  MOE_REQUIRE(MOE_ALIGNED16(op.xq) && MOE_ALIGNED16(op.w0) && MOE_ALIGNED16(op.w1) && MOE_ALIGNED16(op.out), MOE_ERR_BAD_ALIGN,
+              "%s: pointers must be 16-byte aligned", what);
+  MOE_REQUIRE((long long)rows * op.sc.in_row * 4 <= (1ll << 32) &&
+                  (mode == MODE_DOWN || (long long)rows * op.sc.out_row + (long long)(op.N / 128) * op.sc.out_cb <= (1ll << 40)),
+              MOE_ERR_BAD_SHAPE, "%s: scale array out of the addressable range", what);
+  MOE_REQUIRE(op.K <= MAX_KB * BK, MOE_ERR_BAD_SHAPE, "%s: contraction length %d exceeds %d", what, op.K, MAX_KB * BK);
+  MOE_REQUIRE((long long)op.N * op.K <= (1ll << 32) && (long long)rows * op.K <= (1ll << 32), MOE_ERR_BAD_SHAPE,
+              "%s: one expert matrix and the activation array must each stay within 4 GB (N=%d K=%d rows=%d)", what, op.N, op.K, rows);
+  return MOE_OK;
+}
+
 template <int MODE>
-int launch(const uint8_t* xq, const float* sx, const int32_t* row_ids, const uint8_t* w0, const float* sw0,
-           const uint8_t* w1, const float* sw1, const int32_t* group_offsets, int E, int R, int K, int N,
-           void* out, float* out_scale, void* ws, size_t ws_bytes, bool list_built, GemmScales sc, hipStream_t s) {
-  const size_t need = moe_gemm_workspace_bytes(R, E, N);
-  MOE_REQUIRE(ws_bytes >= need, MOE_ERR_WORKSPACE_TOO_SMALL, "gemm: workspace %zu < %zu", ws_bytes, need);
-  MOE_REQUIRE(K <= MAX_KB * BK, MOE_ERR_BAD_SHAPE, "gemm: contraction length %d exceeds %d", K, MAX_KB * BK);
-  MOE_REQUIRE((long long)N * K <= (1ll << 32) && (long long)R * K <= (1ll << 32), MOE_ERR_BAD_SHAPE,
-              "gemm: one expert matrix and the activation array must each stay within 4 GB (N=%d K=%d R=%d)", N, K, R);
-  if (R == 0) return MOE_OK;
-  const TileList l = tile_list(ws, R, E);
-  if (!list_built) hipLaunchKernelGGL(build_tiles_kernel, dim3(1), dim3(1024), 0, s, group_offsets, E, l, -1);
-  static std::atomic<unsigned long long> lds_raised{0};
-  if (int rc = moe_raise_lds_limit((const void*)grouped_gemm_kernel<MODE>, CLS_LDS_BYTES, lds_raised)) return rc;
+int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
+  const char* what = MODE == MODE_GATEUP ? "gemm_gateup" : "gemm_down";
   // An output that the memory-side cache (256 MB) cannot hold until the combine reads it goes past the caches
   // (config 3: 0.94 GB, step -0.6 %); a smaller one stays cached (config 5: 235 MB, 0.4 % slower when streamed).
-  sc.stream_out = MODE == MODE_DOWN && (size_t)R * N * 2 > ((size_t)192 << 20);
-  const long long max_items = (long long)l.max_tiles * col_blocks(MODE, N);
-  MOE_REQUIRE(max_items < (1ll << 30), MOE_ERR_BAD_SHAPE, "gemm: %lld work items exceed the grid limit", max_items);
-  // sized by the worst case of the largest XCD share (moe_xcd_share_cap_q) and of an XCD's draws from the pool;
-  // surplus workgroups exit at once
-  const long long pool_max = (long long)moe_pool_tile_limit(l.max_tiles) * col_blocks(MODE, N);
-  const int grid = 8 * (int)((max_items + 7) / 8 + 2 + moe_pool_workgroups(pool_max));
-  hipLaunchKernelGGL((grouped_gemm_kernel<MODE>), dim3(grid), dim3(NT), CLS_LDS_BYTES, s, xq, sx, row_ids, w0, sw0, w1,
-                     sw1, l.hdr, l.tiles, K, N, out, out_scale, sc);
+  auto streamed = [](int rows, int N) { return MODE == MODE_DOWN && (size_t)rows * N * 2 > ((size_t)192 << 20); };
+  GemmOperands routed{}, dense{};
+  TileList l{};
+  int dense_rows = 0;
+  long long dense_blocks = 0, grid = 0;
+  if (dn) {
+    if (int rc = check_operands(dn->op, dn->rows, 1, MODE, what)) return rc;
+    dense = dn->op;
+    dense.sc.stream_out = streamed(dn->rows, dense.N);
+    dense_rows = dn->rows;
+    dense_blocks = 8 * (((long long)moe_tile_count(dense_rows) * col_blocks(MODE, dense.N) + 7) / 8);
+    grid = dense_blocks;
+  }
+  if (rt) {
+    MOE_REQUIRE(rt->group_offsets && rt->ws, MOE_ERR_NULL, "%s: null pointer", what);
+    if (int rc = check_operands(rt->op, rt->R, rt->E, MODE, what)) return rc;
+    MOE_REQUIRE(MOE_ALIGNED16(rt->ws), MOE_ERR_BAD_ALIGN, "%s: pointers must be 16-byte aligned", what);
+    const size_t need = moe_gemm_workspace_bytes(rt->R, rt->E, rt->op.N);
+    MOE_REQUIRE(rt->ws_bytes >= need, MOE_ERR_WORKSPACE_TOO_SMALL, "%s: workspace %zu < %zu", what, rt->ws_bytes, need);
+    if (rt->R > 0) {
+      routed = rt->op;
+      routed.sc.stream_out = streamed(rt->R, routed.N);
+      l = tile_list(rt->ws, rt->R, rt->E);
+      // sized by the worst case of the largest XCD share (moe_xcd_share_cap_q) and of an XCD's draws from the pool;
+      // surplus workgroups exit at once
+      const long long max_items = (long long)l.max_tiles * col_blocks(MODE, routed.N);
+      const long long pool_max = (long long)moe_pool_tile_limit(l.max_tiles) * col_blocks(MODE, routed.N);
+      grid += 8 * ((max_items + 7) / 8 + 2 + moe_pool_workgroups(pool_max));
+    }
+  }
+  MOE_REQUIRE(grid < (1ll << 30), MOE_ERR_BAD_SHAPE, "%s: %lld work items exceed the grid limit", what, grid);
+  if (grid == 0) return MOE_OK;
+  if (l.hdr && !rt->list_built)
+    hipLaunchKernelGGL(build_tiles_kernel, dim3(1), dim3(1024), 0, s, rt->group_offsets, rt->E, l);
+  static std::atomic<unsigned long long> lds_raised[2] = {};
+  auto* kernel = dn ? grouped_gemm_kernel<MODE, true> : grouped_gemm_kernel<MODE, false>;
+  if (int rc = moe_raise_lds_limit((const void*)kernel, CLS_LDS_BYTES, lds_raised[dn != nullptr])) return rc;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(NT), CLS_LDS_BYTES, s, routed, l.hdr, l.tiles, dense, dense_rows,
+                     (int)dense_blocks);
   return moe_check_hip(hipGetLastError(), "gemm launch");
 }
 
@@ -730,29 +793,35 @@ extern "C" size_t moe_gemm_workspace_bytes(int R, int E, int N_out) {
   return sizeof(TileHeader) + (size_t)max_tiles_for(R, E) * sizeof(TileEntry) + 256;
 }
 
-int moe_gemm_gateup_impl(const uint8_t* xq, const float* sx, const int32_t* row_ids, const uint8_t* w_gate,
-                         const float* sw_gate, const uint8_t* w_up, const float* sw_up, const int32_t* group_offsets,
-                         int E, int R, int D, int I, uint8_t* hq, float* sh, void* ws, size_t ws_bytes, bool list_built,
-                         GemmScales sc, moe_stream_t stream) {
-  MOE_REQUIRE((R == 0 || (xq && sx && hq && sh)) && w_gate && sw_gate && w_up && sw_up && group_offsets && ws, MOE_ERR_NULL,
-              "gemm_gateup: null pointer");
-  MOE_REQUIRE(E >= 1 && E <= 1024 && R >= 0 && D > 0 && I > 0 && D % 128 == 0 && I % 128 == 0, MOE_ERR_BAD_SHAPE,
-              "gemm_gateup: need D %% 128 == 0 and I %% 128 == 0 and 1 <= E <= 1024, got E=%d R=%d D=%d I=%d", E, R, D, I);
-  MOE_REQUIRE(MOE_ALIGNED16(xq) && MOE_ALIGNED16(w_gate) && MOE_ALIGNED16(w_up) && MOE_ALIGNED16(hq) && MOE_ALIGNED16(ws),
-              MOE_ERR_BAD_ALIGN, "gemm_gateup: pointers must be 16-byte aligned");
-  MOE_REQUIRE((long long)R * sc.in_row * 4 <= (1ll << 32) && (long long)R * sc.out_row + (long long)(I / 128) * sc.out_cb <= (1ll << 40),
-              MOE_ERR_BAD_SHAPE, "gemm_gateup: scale array out of the addressable range");
-  return launch<MODE_GATEUP>(xq, sx, row_ids, w_gate, sw_gate, w_up, sw_up, group_offsets, E, R, D, I, hq, sh, ws,
-                             ws_bytes, list_built, sc, (hipStream_t)stream);
+int moe_gemm_gateup_impl(const RoutedGemm* routed, const DenseGemm* dense, moe_stream_t stream) {
+  return launch<MODE_GATEUP>(routed, dense, (hipStream_t)stream);
 }
+int moe_gemm_down_impl(const RoutedGemm* routed, const DenseGemm* dense, moe_stream_t stream) {
+  return launch<MODE_DOWN>(routed, dense, (hipStream_t)stream);
+}
+
+namespace {
+int gateup(const uint8_t* xq, const float* sx, const int32_t* row_ids, const uint8_t* w_gate, const float* sw_gate,
+           const uint8_t* w_up, const float* sw_up, const int32_t* group_offsets, int E, int R, int D, int I, uint8_t* hq,
+           float* sh, void* ws, size_t ws_bytes, GemmScales sc, moe_stream_t stream) {
+  const RoutedGemm r{{xq, sx, row_ids, w_gate, sw_gate, w_up, sw_up, D, I, hq, sh, sc}, group_offsets, E, R, ws, ws_bytes, false};
+  return moe_gemm_gateup_impl(&r, nullptr, stream);
+}
+int down(const uint8_t* hq, const float* sh, const uint8_t* w_down, const float* sw_down, const int32_t* group_offsets, int E,
+         int R, int I, int D, void* y_bf16, void* ws, size_t ws_bytes, GemmScales sc, moe_stream_t stream) {
+  const RoutedGemm r{{hq, sh, nullptr, w_down, sw_down, nullptr, nullptr, I, D, y_bf16, nullptr, sc}, group_offsets, E, R, ws,
+                     ws_bytes, false};
+  return moe_gemm_down_impl(&r, nullptr, stream);
+}
+}  // namespace
 
 extern "C" int moe_gemm_gateup_swiglu_fp8(const uint8_t* xq, const float* sx, const int32_t* row_ids,
                                           const uint8_t* w_gate, const float* sw_gate, const uint8_t* w_up,
                                           const float* sw_up, const int32_t* group_offsets, int E, int R, int D,
                                           int I, uint8_t* hq, float* sh, void* ws, size_t ws_bytes,
                                           moe_stream_t stream) {
-  return moe_gemm_gateup_impl(xq, sx, row_ids, w_gate, sw_gate, w_up, sw_up, group_offsets, E, R, D, I, hq, sh, ws,
-                              ws_bytes, false, moe_row_major_scales(D, I), stream);
+  return gateup(xq, sx, row_ids, w_gate, sw_gate, w_up, sw_up, group_offsets, E, R, D, I, hq, sh, ws, ws_bytes,
+                moe_row_major_scales(D, I), stream);
 }
 
 namespace {
@@ -773,8 +842,7 @@ extern "C" int moe_gemm_gateup_swiglu_fp8_layout(const uint8_t* xq, const float*
   GemmScales sc = moe_row_major_scales(D, I);
   if (sx_layout == MOE_SCALES_BLOCK_MAJOR) sc.in_row = 1, sc.in_kb = R, sc.in_listed = true;
   if (sh_layout == MOE_SCALES_BLOCK_MAJOR) sc.out_row = 1, sc.out_cb = R;
-  return moe_gemm_gateup_impl(xq, sx, row_ids, w_gate, sw_gate, w_up, sw_up, group_offsets, E, R, D, I, hq, sh, ws,
-                              ws_bytes, false, sc, stream);
+  return gateup(xq, sx, row_ids, w_gate, sw_gate, w_up, sw_up, group_offsets, E, R, D, I, hq, sh, ws, ws_bytes, sc, stream);
 }
 
 namespace {
@@ -810,29 +878,14 @@ extern "C" int moe_gemm_gateup_swiglu_fp8_static(const uint8_t* xq, const float*
   if (int rc = static_scratch(&ws)) return rc;
   // the tile list (header and every entry the GEMM reads) is rewritten by this call's first kernel: nothing of
   // an earlier call's contents is read
-  return moe_gemm_gateup_impl(xq, sx, row_ids, w_gate, sw_gate, w_up, sw_up, group_offsets, E, R, D, I, hq, sh, ws,
-                              MOE_STATIC_SCRATCH_BYTES, false, moe_row_major_scales(D, I), stream);
-}
-
-int moe_gemm_down_impl(const uint8_t* hq, const float* sh, const uint8_t* w_down, const float* sw_down,
-                       const int32_t* group_offsets, int E, int R, int I, int D, void* y_bf16, void* ws,
-                       size_t ws_bytes, bool list_built, GemmScales sc, moe_stream_t stream) {
-  MOE_REQUIRE((R == 0 || (hq && sh && y_bf16)) && w_down && sw_down && group_offsets && ws, MOE_ERR_NULL,
-              "gemm_down: null pointer");
-  MOE_REQUIRE(E >= 1 && E <= 1024 && R >= 0 && D > 0 && I > 0 && D % 128 == 0 && I % 128 == 0, MOE_ERR_BAD_SHAPE,
-              "gemm_down: need D %% 128 == 0 and I %% 128 == 0 and 1 <= E <= 1024, got E=%d R=%d I=%d D=%d", E, R, I, D);
-  MOE_REQUIRE(MOE_ALIGNED16(hq) && MOE_ALIGNED16(w_down) && MOE_ALIGNED16(y_bf16) && MOE_ALIGNED16(ws), MOE_ERR_BAD_ALIGN,
-              "gemm_down: pointers must be 16-byte aligned");
-  MOE_REQUIRE((long long)R * sc.in_row * 4 <= (1ll << 32), MOE_ERR_BAD_SHAPE, "gemm_down: scale array out of the addressable range");
-  return launch<MODE_DOWN>(hq, sh, nullptr, w_down, sw_down, nullptr, nullptr, group_offsets, E, R, I, D, y_bf16,
-                           nullptr, ws, ws_bytes, list_built, sc, (hipStream_t)stream);
+  return gateup(xq, sx, row_ids, w_gate, sw_gate, w_up, sw_up, group_offsets, E, R, D, I, hq, sh, ws, MOE_STATIC_SCRATCH_BYTES,
+                moe_row_major_scales(D, I), stream);
 }
 
 extern "C" int moe_gemm_down_fp8(const uint8_t* hq, const float* sh, const uint8_t* w_down, const float* sw_down,
                                  const int32_t* group_offsets, int E, int R, int I, int D, void* y_bf16, void* ws,
                                  size_t ws_bytes, moe_stream_t stream) {
-  return moe_gemm_down_impl(hq, sh, w_down, sw_down, group_offsets, E, R, I, D, y_bf16, ws, ws_bytes, false,
-                            moe_row_major_scales(I, D), stream);
+  return down(hq, sh, w_down, sw_down, group_offsets, E, R, I, D, y_bf16, ws, ws_bytes, moe_row_major_scales(I, D), stream);
 }
 
 extern "C" int moe_gemm_down_fp8_layout(const uint8_t* hq, const float* sh, const uint8_t* w_down, const float* sw_down,
@@ -841,16 +894,7 @@ extern "C" int moe_gemm_down_fp8_layout(const uint8_t* hq, const float* sh, cons
   if (int rc = check_layout(sh_layout, "gemm_down: sh")) return rc;
   GemmScales sc = moe_row_major_scales(I, D);
   if (sh_layout == MOE_SCALES_BLOCK_MAJOR) sc.in_row = 1, sc.in_kb = R, sc.in_listed = true;
-  return moe_gemm_down_impl(hq, sh, w_down, sw_down, group_offsets, E, R, I, D, y_bf16, ws, ws_bytes, false, sc, stream);
-}
-
-// Builds, ahead of the GEMM launches, the list that they read from ws when they are told list_built = true:
-// one group of R rows (the shared expert).
-int moe_gemm_build_dense_tile_list(int R, void* ws, size_t ws_bytes, moe_stream_t stream) {
-  TileList l;
-  if (int rc = moe_gemm_tile_list(R, 1, ws, ws_bytes, &l)) return rc;
-  hipLaunchKernelGGL(build_tiles_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, (const int32_t*)nullptr, 1, l, R);
-  return moe_check_hip(hipGetLastError(), "gemm tiles launch");
+  return down(hq, sh, w_down, sw_down, group_offsets, E, R, I, D, y_bf16, ws, ws_bytes, sc, stream);
 }
 
 // The tile list that the GEMM launches of (R rows, E experts) read from ws when they are told list_built = true.
