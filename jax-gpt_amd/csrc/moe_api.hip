@@ -275,18 +275,12 @@ extern "C" int moe_forward(const MoeForwardArgs* a, void* ws, size_t ws_bytes, m
     if (a->w_shared_gate) shared_gate = gate_out;
     src = LogitSource{nullptr, (const float*)b.router_ws, splits, n_cols, a->out_logits, gate_out};
   }
-  const QuantJob* carried = quant_in_route ? &quant_job : nullptr;
-  if (a->routing == MOE_ROUTING_SOFTMAX)
-    rc = moe_route_softmax_impl(src, a->M, a->E, a->k, a->renorm, idx, w, stream, carried);
-  else
-    rc = moe_route_sigmoid_grouped_impl(src, a->bias, a->M, a->E, a->n_group, a->topk_group, a->k, a->renorm,
-                                        a->routed_scale, idx, w, stream, carried);
-  if (rc) return join(rc);
-  // the permutation kernels also list the routed GEMMs' row tiles (they hold every expert's row range anyway)
+  // routing, the sort by expert and the routed GEMMs' work list (the sort holds every expert's row range anyway)
   TileList tiles;
   if ((rc = moe_gemm_tile_list(R, a->E, b.gemm_ws, b.gemm_ws_bytes, &tiles))) return join(rc);
-  if ((rc = moe_permute_impl(idx, a->M, a->k, a->E, gsz, b.group_offsets, stid, nullptr, inv, b.permute_ws,
-                             b.permute_ws_bytes, tiles, stream)))
+  const RouteArgs route{src, a->bias, a->M, a->E, a->k, a->renorm, a->n_group, a->topk_group, a->routed_scale, idx, w};
+  const PermuteOut sort{gsz, b.group_offsets, stid, nullptr, inv, a->k, tiles};
+  if ((rc = moe_route_impl(a->routing, route, quant_in_route ? &quant_job : nullptr, &sort, b.permute_ws, b.permute_ws_bytes, stream)))
     return join(rc);
   if (!quant_joined) {
     if (rc_shared) return join(rc_shared);

@@ -94,16 +94,20 @@ __host__ __device__ inline void moe_tile_span(int rows, int nt, int t, int& star
 // Where an expert's tiles go in the work list.  The grouped GEMM deals contiguous eighths of the list to the 8 XCDs
 // (tiles that share a weight slab then share an L2), so the eighths should cost about the same: with group sizes
 // as skewed as a biased router makes them, natural expert order leaves one XCD with up to a tenth more work than the
-// average, and the launch ends with its slowest XCD.  The experts are therefore ranked by size (ties: lower index
-// first) and dealt to eight bins in snake order (0..7, 7..0, ...); the list holds bin after bin.
-// Called by every thread of a workgroup of 2^n >= E threads (at most 1024); thread e owns expert e (rows = 0 for
-// e >= E); lds_rows and lds_key are int[blockDim.x] arrays in LDS.  Returns the index of expert e's first tile and, in
-// *total_tiles, the length of the list, and writes the list header.
+// average, and the launch ends with its slowest XCD.  The experts are therefore ranked by size (in units of 32 rows)
+// and dealt to eight bins in snake order (0..7, 7..0, ...); the list holds bin after bin.
+// Called by every thread of a workgroup of 1024; thread e owns expert e (rows = 0 where there is none); lds_a and lds_b
+// are int[1024] in LDS.  Returns the index of expert e's first tile and writes the list header.
 //
 // The header's XCD shares are cut by cost, not by count: a row tile of u 32-row units costs about 8 + u (measured:
 // 63 us for a 32-row tile of the gate/up GEMM against 112 us for a 256-row one, and the same ratio for the down
 // GEMM), and equal counts left the XCD with the tallest tiles some 3 % more work than the average.  All tiles of an
 // expert cost alike, so a cut inside an expert sits at the same fraction of its items as of its cost.
+//
+// One workgroup, between two launches that wait for it, so it is written for few steps: the ranking is a counting sort
+// over size classes, an expert's place in the list follows from its rank in closed form, and the tiles and cost in
+// front of it are one scan over the list.  (Comparing every expert with every other took 10, 17 and 45 us at 128, 256
+// and 512 experts; this takes 4.)
 __device__ inline int moe_tile_cost(int rows) { return 8 * moe_tile_count(rows) + ((rows + 31) >> 5); }   // (< 2^31 for 2^32 / 128 rows)
 __device__ inline void moe_tile_even_shares(TileHeader* hdr, int n_static, int n_tiles) {   // one thread
   hdr->n_tiles = n_tiles;
@@ -111,64 +115,60 @@ __device__ inline void moe_tile_even_shares(TileHeader* hdr, int n_static, int n
   hdr->pool_next[0] = hdr->pool_next[1] = 0;
   for (int k = 0; k <= 8; ++k) hdr->xcd_q[k] = (((long long)n_static << kTileQBits) * k) >> 3;
 }
-__device__ inline int moe_tile_first(int e, int E, int rows, int* lds_rows, int* lds_key, int* total_tiles,
-                                     TileHeader* hdr, int max_tiles) {
+// exclusive sums of (a, b) over the workgroup's 1024 threads, and the totals
+__device__ __forceinline__ void moe_scan_1024(int& a, int& b, int& all_a, int& all_b) {
+  __shared__ int wave_a[16], wave_b[16];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int a0 = a, b0 = b;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int oa = __shfl_up(a, off, MOE_WAVE), ob = __shfl_up(b, off, MOE_WAVE);
+    if (lane >= off) a += oa, b += ob;
+  }
+  if (lane == 63) wave_a[wv] = a, wave_b[wv] = b;
+  __syncthreads();
+  int pa = 0, pb = 0;
+  all_a = all_b = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    if (w == wv) pa = all_a, pb = all_b;
+    all_a += wave_a[w], all_b += wave_b[w];
+  }
+  a += pa - a0;
+  b += pb - b0;
+  __syncthreads();   // (the wave totals may be overwritten)
+}
+__device__ inline int moe_tile_first(int e, int rows, int* lds_a, int* lds_b, TileHeader* hdr, int max_tiles) {
   __shared__ long long cut_q[9];
   __shared__ int tail_tiles[kTailRounds];   // tiles of the last, last but one, ... round of the ranking
-  __shared__ int sums[4];                   // non-empty experts; tiles, tiles outside the pool and their cost
-  __shared__ int acc_first[1024], acc_cost[1024];
-  // The two walks over all experts (the ranking; the tiles and cost in front of an expert) are shared out: with
-  // epad = E rounded up to a power of two (at least a wavefront), the workgroup's threads form blockDim / epad parts,
-  // thread (part, e2) walks the part's slice of the experts on behalf of expert e2, and the parts' sums meet in LDS
-  // (against one thread per expert walking them all: 2 us less of a 17 us launch at 128 experts; most of such a
-  // launch is its start -- arguments, first instruction lines, first loads -- and not its arithmetic).
-  int epad = 64;
-  while (epad < E) epad <<= 1;
-  const int parts = (int)blockDim.x / epad;          // >= 1: the caller has at least E threads, a power of two of them
-  const int e2 = e & (epad - 1), part = e / epad;
-  const int span = (epad + parts - 1) / parts;
-  const int o0 = part * span, o1 = o0 + span < E ? o0 + span : E;
-  const bool helper = part < parts && e2 < E;
-  lds_rows[e] = e < E ? rows : 0;
-  lds_key[e] = 0;   // (first the ranks' accumulator)
-  acc_first[e] = 0;
-  acc_cost[e] = 0;
-  if (e < 4) sums[e] = 0;
+  const int nt = moe_tile_count(rows);
+  // rank: largest class first, inside a class in any order (1023 = the largest class and everything above it)
+  const int cls = rows > 0 ? 1023 - min((rows + 31) >> 5, 1023) : 0;
+  lds_a[e] = 0;
   if (e < kTailRounds) tail_tiles[e] = 0;
   __syncthreads();
-  if (helper) {
-    const int mine = lds_rows[e2];
-    int ahead = 0;
-#pragma unroll 8
-    for (int o = o0; o < o1; ++o) {
-      const int r = lds_rows[o];
-      ahead += (r > mine || (r == mine && o < e2)) ? 1 : 0;
-    }
-    if (ahead) atomicAdd(&lds_key[e2], ahead);
-  }
-  {
-    const unsigned long long busy = __ballot(e < E && rows > 0);
-    if ((e & 63) == 0 && busy) atomicAdd(&sums[0], __popcll(busy));
-  }
+  const int order = rows > 0 ? atomicAdd(&lds_a[cls], 1) : 0;
   __syncthreads();
-  int key = e;
-  const int rank = lds_key[e], nz = sums[0];
+  int before = lds_a[e], unused = 0, nz, unused_all;   // nz: experts with rows
+  moe_scan_1024(before, unused, nz, unused_all);
+  lds_b[e] = before;
+  __syncthreads();
+  const int rank = lds_b[cls] + order;
   const int nr = (nz + 7) >> 3;   // rounds that hold a non-empty expert
   const int tail = nr / 4 < kTailRounds ? nr / 4 : kTailRounds;   // (3 rounds = 24 experts over the 8 bins; 6 measured no better)
   const int round = rank >> 3;
-  if (e < E && rows > 0 && round >= nr - tail) atomicAdd(&tail_tiles[nr - 1 - round], moe_tile_count(rows));
+  if (rows > 0 && round >= nr - tail) atomicAdd(&tail_tiles[nr - 1 - round], nt);
   __syncthreads();
   // The pool: as many of the tail rounds, from the last one, as fit the launch's spare workgroups.
   int pooled = 0;
-  for (int t = 0, sum = 0; e < E && t < tail; ++t) {
+  for (int t = 0, sum = 0; t < tail; ++t) {
     sum += tail_tiles[t];
     if (sum > moe_pool_tile_limit(max_tiles)) break;
     pooled = t + 1;
   }
-  if (e < E && rows > 0 && round >= nr - pooled) {
-    key = 1024 + rank;   // behind every bin (keys below 1024), the tallest of the pool first
-  } else if (e < E) {
-    const int posn = rank & 7;
+  const int n_fixed = pooled ? (nr - pooled) * 8 : nz;   // experts in fixed shares; the others, last in rank, are the pool
+  int at = rank;                                         // place in the list
+  if (rank < n_fixed) {
     // Inside a bin the experts alternate between the large and the small end of the ranking (largest, smallest,
     // second largest, ...): tall tiles are matrix work on lines that mostly hit L2, short tiles are weight streams
     // from HBM, and a launch that runs them side by side from start to end keeps both busy and its power draw even
@@ -176,56 +176,44 @@ __device__ inline int moe_tile_first(int e, int E, int rows, int* lds_rows, int*
     // The smallest experts of a bin stay at its end (those that the pool does not take): the launch ends with its
     // shortest items.
     const int mixed = nr - tail;
-    const int pos = round >= mixed ? round : (round < (mixed + 1) / 2 ? 2 * round : 2 * (mixed - 1 - round) + 1);
-    key = ((round & 1) ? 7 - posn : posn) * 128 + pos;   // E <= 1024: at most 128 rounds
+    auto position = [&](int r) { return r >= mixed ? r : r < (mixed + 1) / 2 ? 2 * r : 2 * (mixed - 1 - r) + 1; };
+    const int bin = (round & 1) ? 7 - (rank & 7) : rank & 7;
+    // full rounds give every bin one expert; a last round of `part` experts gives one to some bins
+    const int full = n_fixed >> 3, part = n_fixed & 7;
+    const bool odd = full & 1;
+    const bool has_part = odd ? bin >= 8 - part : bin < part;
+    at = bin * full + (odd ? max(0, bin - (8 - part)) : min(bin, part)) + position(round) -
+         (part && !has_part && position(full) < position(round) ? 1 : 0);
   }
-  lds_key[e] = key;
-  if (e < E) {   // the whole list's tiles, and the tiles and cost of the fixed shares (outside the pool)
-    const int t = moe_tile_count(rows);
-    if (t) {
-      atomicAdd(&sums[1], t);
-      if (key < 1024) {
-        atomicAdd(&sums[2], t);
-        atomicAdd(&sums[3], moe_tile_cost(rows));
-      }
-    }
+  lds_a[e] = 0;   // (the class counts were read before the scan's barriers, lds_b's prefixes before the last one)
+  lds_b[e] = 0;
+  __syncthreads();
+  if (rows > 0) {
+    lds_a[at] = nt;
+    lds_b[at] = at < n_fixed ? moe_tile_cost(rows) : 0;   // (the pool has no part in the shares)
   }
   __syncthreads();
-  if (helper) {
-    const int key2 = lds_key[e2];
-    int tiles_before = 0, cost_before_part = 0;
-#pragma unroll 8
-    for (int o = o0; o < o1; ++o) {
-      const int ko = lds_key[o], ro = lds_rows[o];
-      const int t = moe_tile_count(ro);
-      const int c = ko < 1024 ? 8 * t + ((ro + 31) >> 5) : 0;   // (not in the pool)
-      const bool before = ko < key2;
-      tiles_before += before ? t : 0;
-      cost_before_part += before ? c : 0;
-    }
-    if (tiles_before) atomicAdd(&acc_first[e2], tiles_before);
-    if (cost_before_part) atomicAdd(&acc_cost[e2], cost_before_part);
-  }
+  int tiles_before = lds_a[e], cost_before = lds_b[e], total, cost_all;
+  moe_scan_1024(tiles_before, cost_before, total, cost_all);
+  lds_a[e] = tiles_before;
+  lds_b[e] = cost_before;
   __syncthreads();
-  const int first = acc_first[e], cost_before = acc_cost[e];
-  const int total = sums[1], n_static = sums[2], cost_all = sums[3];
-  *total_tiles = total;
+  const int first = lds_a[at & 1023], mine_before = lds_b[at & 1023];
+  const int fixed_tiles = n_fixed < 1024 ? lds_a[n_fixed] : total;
   // cut k sits where the cost of the fixed shares reaches k/8 of their whole: inside exactly one expert, whose
   // thread places it
-  if (e < E && rows > 0 && key < 1024) {
-    const long long mine = moe_tile_cost(rows);
-    const int nt = moe_tile_count(rows);
+  if (rows > 0 && at < n_fixed) {
+    const long long mine = (long long)moe_tile_cost(rows) * 8;
     for (int k = 1; k < 8; ++k) {
-      const long long at = (long long)cost_all * k - (long long)cost_before * 8;   // (cost units x 8)
-      if (at >= 0 && at < mine * 8)   // (float: the cut need not be exact, only inside this expert's tiles)
-        cut_q[k] = ((long long)first << kTileQBits) +
-                   (long long)((float)at / (float)(mine * 8) * (float)nt * (float)(1 << kTileQBits));
+      const long long d = (long long)cost_all * k - (long long)mine_before * 8;   // (cost units x 8)
+      if (d >= 0 && d < mine)   // (float: the cut need not be exact, only inside this expert's tiles)
+        cut_q[k] = ((long long)first << kTileQBits) + (long long)((float)d / (float)mine * (float)nt * (float)(1 << kTileQBits));
     }
   }
   __syncthreads();
   if (e == 0) {
     const int n = total < max_tiles ? total : max_tiles;
-    const int ns = n_static < n ? n_static : n;
+    const int ns = fixed_tiles < n ? fixed_tiles : n;
     cut_q[0] = 0;
     cut_q[8] = (long long)ns << kTileQBits;
     bool fits = ns > 0 && total <= max_tiles;
@@ -251,8 +239,8 @@ struct LogitSource {
 int moe_router_partials(const void* x_bf16, int M, int D, const void* w_router_bf16, int E,
                         const void* w_shared_gate_bf16, void* ws, size_t ws_bytes, int* splits_used, int* n_cols,
                         moe_stream_t stream);
-// An activation quantisation that a routing launch carries along (moe_quant_device.h): `blocks` blocks of 256
-// 16-byte pieces behind the routing kernel's own blocks.  blocks == 0: none.
+// An activation quantisation (moe_quant_device.h): blocks of blockDim.x 16-byte pieces, in a launch of its own or
+// behind the routing kernel's own blocks.
 struct QuantJob {
   const void* x;        // (R, K) bf16
   long long n_pieces;   // R * K / 8
@@ -261,14 +249,32 @@ struct QuantJob {
   uint8_t* xq;
   float* sx;
   float* sx_blocked;    // optional (K/128, R) copy of the scales
-  unsigned blocks;
 };
+inline unsigned moe_quant_blocks(const QuantJob& q, int threads) { return (unsigned)((q.n_pieces + threads - 1) / threads); }
 int moe_quant_act_job(const void* x_bf16, int R, int K, uint8_t* xq, float* sx, float* sx_blocked, QuantJob* job);
-int moe_route_softmax_impl(const LogitSource& src, int M, int E, int k, int renorm, int32_t* idx, float* w,
-                           moe_stream_t stream, const QuantJob* quant = nullptr);
-int moe_route_sigmoid_grouped_impl(const LogitSource& src, const float* bias, int M, int E, int n_group,
-                                   int topk_group, int k, int renorm, float routed_scale, int32_t* idx, float* w,
-                                   moe_stream_t stream, const QuantJob* quant = nullptr);
+// What the sort by expert writes (sort_order, sorted_token_ids, inv_perm: null to skip; tl.tiles null: no work list).
+struct PermuteOut {
+  int32_t *group_sizes, *group_offsets, *sorted_token_ids, *sort_order, *inv_perm;
+  int k;
+  TileList tl;
+};
+// One routing call: the selection, and with it (optional) an activation quantisation and the sort by expert.
+struct RouteArgs {
+  LogitSource src;
+  const float* bias;   // sigmoid_grouped only, or null
+  int M, E, k, renorm;
+  int n_group, topk_group;
+  float routed_scale;
+  int32_t* idx;
+  float* w;
+};
+int moe_route_impl(int routing, const RouteArgs& a, const QuantJob* quant, const PermuteOut* sort, void* permute_ws,
+                   size_t permute_ws_bytes, moe_stream_t stream);
+// chunks of the flat list that get a histogram each, at most
+int moe_permute_max_chunks(int E);
+// the sort's second launch: chunk_hist [n_chunks][E] (null when n_chunks == 1)
+int moe_permute_place(const int32_t* idx, int R, int E, int chunk, int n_chunks, const int32_t* chunk_hist, const PermuteOut& o,
+                      moe_stream_t stream);
 // grouped GEMMs with an optional pre-built tile list in ws (moe_gemm.hip); the extern "C" entry points build their
 // own.  moe_gemm_tile_list describes the list the GEMMs of (R rows, E experts) expect in ws, so that the permutation
 // kernels, which hold every expert's row range anyway, can write it (moe_permute_impl) and no launch is spent on it.
@@ -278,9 +284,7 @@ int moe_gemm_tile_list(int R, int E, void* ws, size_t ws_bytes, TileList* list);
 int moe_quant_act_impl(const void* x_bf16, int R, int K, uint8_t* xq, float* sx, float* sx_blocked, moe_stream_t stream);
 int moe_rmsnorm_quant_impl(const void* x_bf16, const float* weight, float eps, int M, int D, void* normed_bf16,
                            uint8_t* xq, float* sx, float* sx_blocked, moe_stream_t stream);
-int moe_permute_impl(const int32_t* idx, int M, int k, int E, int32_t* group_sizes, int32_t* group_offsets,
-                     int32_t* sorted_token_ids, int32_t* sort_order, int32_t* inv_perm, void* ws, size_t ws_bytes,
-                     TileList tiles, moe_stream_t stream);
+int moe_permute_impl(const int32_t* idx, int M, int k, int E, const PermuteOut& o, void* ws, size_t ws_bytes, moe_stream_t stream);
 // Where the grouped GEMMs find an activation scale and put an h scale, in floats: scale of (row, 128-wide K block kb)
 // = s[row * in_row + kb * in_kb].  The public entry points use the row-major arrays of the quantisers ({K/128, 1});
 // moe_forward hands large batches block-major arrays in row-list order ({1, R}, in_listed = true: indexed by the

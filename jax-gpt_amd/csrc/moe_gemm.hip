@@ -85,8 +85,7 @@ __global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __rest
     rows = group_offsets[e + 1] - start;
   }
   const int tiles = moe_tile_count(rows);
-  int total = 0;
-  const int first = moe_tile_first(e, E, rows, s_rows, s_key, &total, l.hdr, l.max_tiles);
+  const int first = moe_tile_first(e, rows, s_rows, s_key, l.hdr, l.max_tiles);
   for (int t = 0; t < tiles; ++t)
     if (first + t < l.max_tiles) l.tiles[first + t] = TileEntry{e, start, rows, first};   // (cannot overflow for consistent offsets)
 }

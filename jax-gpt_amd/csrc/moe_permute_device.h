@@ -1,0 +1,96 @@
+// The stable counting sort's placing step as device functions of one workgroup, shared by its own kernel
+// (moe_permute.hip) and by the routing kernel of a small batch (moe_route.hip), which sorts what it has just selected.
+#pragma once
+#include "moe_common.h"
+
+constexpr int kMaxE = 1024;
+constexpr int kPlaceThreads = 1024;
+constexpr int kPlaceWaves = kPlaceThreads / MOE_WAVE;
+// Batches up to this many (token, slot) entries are one chunk, and their few, short row tiles are listed in plain
+// expert order with equal XCD shares.
+constexpr int kSmallRows = 2048;
+
+// waves that count and place: one counter per expert each, at most 32 KB of LDS in all
+__host__ __device__ inline int moe_place_waves(int E) { return E > 512 ? kPlaceWaves / 2 : kPlaceWaves; }
+__host__ __device__ inline size_t moe_place_lds_ints(int E) { return (size_t)moe_place_waves(E) * E; }
+
+#ifdef __HIPCC__
+// lanes of this wave whose expert id equals mine (ids < 2^bits); inactive lanes pass id = -1
+__device__ __forceinline__ unsigned long long match_any(int id, int bits) {
+  unsigned long long m = __ballot(id >= 0);
+  for (int b = 0; b < bits; ++b) {
+    unsigned long long set = __ballot((id >> b) & 1);
+    m &= ((id >> b) & 1) ? set : ~set;
+  }
+  return id >= 0 ? m : 0ull;
+}
+
+__device__ __forceinline__ int ilog2_ceil(int n) { return n <= 1 ? 0 : 32 - __clz(n - 1); }
+
+// Counts or places the entries [first, first + n) of the flat list, wave w a contiguous share of them in flat order, so
+// that a wave's own counters and the popcount of the match mask below a lane give stable ranks.  `next` is [waves][E]:
+// PLACE false: += the wave's entries per expert; true: next free output position, advanced as entries are placed.
+template <bool PLACE>
+__device__ __forceinline__ void place_pass(const int32_t* ids, int first, int n, int E, int* next, const PermuteOut& o) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, waves = moe_place_waves(E);
+  if (wv >= waves) return;
+  const int bits = ilog2_ceil(E);
+  const int span = (n + waves * MOE_WAVE - 1) / (waves * MOE_WAVE) * MOE_WAVE;   // uniform
+  int* mine = next + wv * E;
+  for (int i0 = wv * span; i0 < min(n, (wv + 1) * span); i0 += MOE_WAVE) {
+    const int i = i0 + lane;
+    int id = i < n ? ids[i] : -1;
+    if (id >= E) id = -1;   // out-of-range ids are dropped rather than corrupting LDS
+    const unsigned long long m = match_any(id, bits);
+    const int rank = __popcll(m & ((1ull << lane) - 1ull));
+    if (id >= 0) {
+      int pos = 0;
+      if (PLACE) pos = mine[id] + rank;             // every lane of a class reads before its leader bumps the counter
+      if (rank == 0) mine[id] += __popcll(m);       // (one writer per counter and instruction)
+      if (PLACE) {
+        const int f = first + i;
+        if (o.sort_order) o.sort_order[pos] = f;
+        if (o.sorted_token_ids) o.sorted_token_ids[pos] = f / o.k;
+        if (o.inv_perm) o.inv_perm[f] = pos;
+      }
+    }
+  }
+}
+
+// The whole sort of one chunk (n entries starting at flat index 0) in one workgroup of kPlaceThreads; ids may be in
+// LDS.  next: moe_place_lds_ints(E) ints of LDS.  The caller synchronises before the call (ids written, LDS free).
+__device__ __forceinline__ void permute_one_chunk(const int32_t* ids, int n, int E, int* next, const PermuteOut& o) {
+  const int e = threadIdx.x, waves = moe_place_waves(E);
+  for (int i = threadIdx.x; i < waves * E; i += kPlaceThreads) next[i] = 0;
+  __syncthreads();
+  place_pass<false>(ids, 0, n, E, next, o);
+  __syncthreads();
+  int rows = 0;
+  if (e < E)
+    for (int w = 0; w < waves; ++w) rows += next[w * E + e];
+  const int nt = moe_tile_count(rows);
+  int row_start = rows, tile_start = nt, rows_all, tiles_all;
+  moe_scan_1024(row_start, tile_start, rows_all, tiles_all);
+  if (e < E) {
+    int run = row_start;
+    for (int w = 0; w < waves; ++w) {
+      const int c = next[w * E + e];
+      next[w * E + e] = run;
+      run += c;
+    }
+    o.group_sizes[e] = rows;
+    o.group_offsets[e] = row_start;
+    if (e == E - 1) o.group_offsets[E] = row_start + rows;
+    if (o.tl.tiles) {
+      for (int t = 0; t < nt; ++t)
+        if (tile_start + t < o.tl.max_tiles) o.tl.tiles[tile_start + t] = TileEntry{e, row_start, rows, tile_start};
+      if (e == 0) {
+        const int all = min(tiles_all, o.tl.max_tiles);
+        moe_tile_even_shares(o.tl.hdr, all, all);
+      }
+    }
+  }
+  __syncthreads();
+  place_pass<true>(ids, 0, n, E, next, o);
+}
+#endif

@@ -121,16 +121,15 @@ int moe_quant_act_job(const void* x_bf16, int R, int K, uint8_t* xq, float* sx, 
   MOE_REQUIRE(R >= 0 && K > 0 && K % MOE_QBLOCK == 0, MOE_ERR_BAD_SHAPE, "quant_act: K=%d must be a positive multiple of 128 (R=%d)", K, R);
   MOE_REQUIRE(MOE_ALIGNED16(x_bf16) && MOE_ALIGNED16(xq), MOE_ERR_BAD_ALIGN, "quant_act: pointers must be 16-byte aligned");
   const long long pieces = (long long)R * K / 8;
-  const long long blocks = (pieces + 255) / 256;
-  MOE_REQUIRE(blocks < (1ll << 31), MOE_ERR_BAD_SHAPE, "quant_act: too many elements");
-  *job = QuantJob{x_bf16, pieces, K / 128, R, xq, sx, sx_blocked, (unsigned)blocks};
+  MOE_REQUIRE(pieces < (1ll << 38), MOE_ERR_BAD_SHAPE, "quant_act: too many elements");
+  *job = QuantJob{x_bf16, pieces, K / 128, R, xq, sx, sx_blocked};
   return MOE_OK;
 }
 int moe_quant_act_impl(const void* x_bf16, int R, int K, uint8_t* xq, float* sx, float* sx_blocked, moe_stream_t stream) {
   QuantJob job;
   if (int rc = moe_quant_act_job(x_bf16, R, K, xq, sx, sx_blocked, &job)) return rc;
   if (R == 0) return MOE_OK;
-  hipLaunchKernelGGL(quant_act_kernel, dim3(job.blocks), dim3(256), 0, (hipStream_t)stream, job);
+  hipLaunchKernelGGL(quant_act_kernel, dim3(moe_quant_blocks(job, 256)), dim3(256), 0, (hipStream_t)stream, job);
   return moe_check_hip(hipGetLastError(), "quant_act launch");
 }
 

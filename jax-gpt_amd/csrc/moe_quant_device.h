@@ -1,4 +1,4 @@
-// The 1x128 activation quantiser as a device function of one 256-thread block, shared by its own kernel
+// The 1x128 activation quantiser as a device function of one block (whole wavefronts), shared by its own kernel
 // (moe_quant.hip) and by the routing kernels (moe_route.hip), whose launch can carry the quantiser's blocks behind
 // its own: the two are independent, and on a latency-bound path one launch runs them side by side.
 // scale = 448/amax, q = e4m3(clamp(x*scale, +-448)), stored scale = 1/scale (replaces the per-row quantiser of
@@ -8,9 +8,9 @@
 
 struct alignas(16) moe_bf16x8 { bf16_t v[8]; };
 
-// 16 lanes per 128-wide group, 8 bf16 (16 B) per lane; `block` = index of the 256-piece block
+// 16 lanes per 128-wide group, 8 bf16 (16 B) per lane; `block` = index of the block of blockDim.x pieces
 __device__ __forceinline__ void moe_quant_act_block(const QuantJob& q, long long block) {
-  const long long p = block * 256 + threadIdx.x;
+  const long long p = block * blockDim.x + threadIdx.x;
   const bool ok = p < q.n_pieces;
   moe_bf16x8 in = {};
   if (ok) in = ((const moe_bf16x8*)q.x)[p];

@@ -1,4 +1,4 @@
-// Routing kernels: one wavefront per token.
+// Routing: one wavefront per token, and with it the rest of what stands in front of the grouped GEMMs.
 //
 // Selection is exact integer work on order-preserving keys, so the indices do
 // not depend on any transcendental: softmax routing ranks the logits (softmax
@@ -7,294 +7,401 @@
 // operations (no fused multiply-add; this file is compiled with
 // -ffp-contract=off) that a CPU can repeat bit for bit.
 //
-// Replaces jax_gpt/models/qwen35/moe.py:51-53 (softmax, lax.top_k, renormalise).
+// Replaces jax_gpt/models/qwen35/moe.py:51-53 (softmax, lax.top_k, renormalise) and, for a whole layer, the
+// counting half of :58-80.
 #include "moe_common.h"
+#include "moe_permute_device.h"
 #include "moe_quant_device.h"
 
 namespace {
 
-// value-descending, ties -> lower index: larger key wins.  key 0 = absent.
-__device__ __forceinline__ unsigned long long make_key(float v, unsigned idx) {
-  unsigned u = __float_as_uint(v + 0.0f);  // -0 -> +0
-  u = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-  return ((unsigned long long)u << 32) | (unsigned long long)(0xffffffffu - idx);
+// 32-bit keys: larger key = larger value (-0 equals +0); 0 = absent
+__device__ __forceinline__ unsigned make_key(float v) {
+  const unsigned u = __float_as_uint(v + 0.0f);  // -0 -> +0
+  return max((u & 0x80000000u) ? ~u : (u | 0x80000000u), 1u);   // (a NaN of all ones is still present)
 }
-__device__ __forceinline__ float key_value(unsigned long long key) {
-  unsigned u = (unsigned)(key >> 32);
-  u = (u & 0x80000000u) ? (u & 0x7fffffffu) : ~u;
-  return __uint_as_float(u);
-}
-__device__ __forceinline__ unsigned key_index(unsigned long long key) {
-  return 0xffffffffu - (unsigned)(key & 0xffffffffu);
+__device__ __forceinline__ float key_value(unsigned u) {
+  return __uint_as_float((u & 0x80000000u) ? (u & 0x7fffffffu) : ~u);
 }
 
-// Wave-wide maximum of 64-bit keys, result in every lane.  Inside a row of 16 lanes the partners are reached with
-// DPP lane permutations (a few cycles each: xor 1, xor 2, mirror of 8, mirror of 16 -- a maximum does not care
-// which partner it meets, only that the set closes); the four row maxima are then read as scalars.  The same
-// reduction over ds_bpermute takes about 100 cycles per step, and routing is a chain of some thirty reductions.
-template <int CTRL> __device__ __forceinline__ unsigned long long dpp_max_u64(unsigned long long k) {
-  const int lo = (int)(unsigned)(k & 0xffffffffu), hi = (int)(unsigned)(k >> 32);
-  const unsigned olo = (unsigned)__builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xF, 0xF, false);
-  const unsigned ohi = (unsigned)__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xF, 0xF, false);
-  const unsigned long long o = ((unsigned long long)ohi << 32) | olo;
-  return o > k ? o : k;
+// Lane permutations inside a row of 16 lanes (DPP, a few cycles each): xor 1, xor 2, mirror of 8, mirror of 16 -- a
+// maximum does not care which partner it meets, only that the set closes.  Reductions over ds_bpermute cost about
+// 100 cycles per step, and routing is a chain of reductions.
+template <int CTRL> __device__ __forceinline__ unsigned dpp(unsigned v) {
+  return (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xF, 0xF, false);
 }
-__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long k) {
-  k = dpp_max_u64<0xB1>(k);    // quad_perm [1,0,3,2]: lane ^ 1
-  k = dpp_max_u64<0x4E>(k);    // quad_perm [2,3,0,1]: lane ^ 2
-  k = dpp_max_u64<0x141>(k);   // row_half_mirror: lane i <-> 7 - i within 8
-  k = dpp_max_u64<0x140>(k);   // row_mirror: lane i <-> 15 - i within 16
-  unsigned long long best = 0ull;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(k & 0xffffffffu), 16 * r);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(k >> 32), 16 * r);
-    const unsigned long long o = ((unsigned long long)hi << 32) | lo;
-    best = o > best ? o : best;
-  }
-  return best;
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_MIRROR8 = 0x141, DPP_MIRROR16 = 0x140, DPP_ROR4 = 0x124, DPP_ROR8 = 0x128;
+
+// wave-wide maximum, as a scalar: row maxima by DPP, the four rows as scalars
+__device__ __forceinline__ unsigned wave_max(unsigned k) {
+  k = max(k, dpp<DPP_XOR1>(k));
+  k = max(k, dpp<DPP_XOR2>(k));
+  k = max(k, dpp<DPP_MIRROR8>(k));
+  k = max(k, dpp<DPP_MIRROR16>(k));
+  const unsigned a = (unsigned)__builtin_amdgcn_readlane((int)k, 0), b = (unsigned)__builtin_amdgcn_readlane((int)k, 16);
+  const unsigned c = (unsigned)__builtin_amdgcn_readlane((int)k, 32), d = (unsigned)__builtin_amdgcn_readlane((int)k, 48);
+  return max(max(a, b), max(c, d));
 }
-__device__ __forceinline__ float wave_max_f32(float v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, MOE_WAVE));
-  return v;
-}
+// wave-wide sum in the pairing of a butterfly (partner lane ^ 32, 16, 8, 4, 2, 1), which fixes the rounding.  After the
+// step over 8 lanes i and i ^ 8 hold the same value, so a rotation by 4 meets what lane ^ 4 holds.
 __device__ __forceinline__ float wave_sum_f32(float v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = __fadd_rn(v, __shfl_xor(v, off, MOE_WAVE));
+  v = __fadd_rn(v, __shfl_xor(v, 32, MOE_WAVE));
+  v = __fadd_rn(v, __shfl_xor(v, 16, MOE_WAVE));
+  v = __fadd_rn(v, __uint_as_float(dpp<DPP_ROR8>(__float_as_uint(v))));
+  v = __fadd_rn(v, __uint_as_float(dpp<DPP_ROR4>(__float_as_uint(v))));
+  v = __fadd_rn(v, __uint_as_float(dpp<DPP_XOR2>(__float_as_uint(v))));
+  v = __fadd_rn(v, __uint_as_float(dpp<DPP_XOR1>(__float_as_uint(v))));
   return v;
 }
-
-constexpr int kWavesPerBlock = 4;
-
-// Logit (t, e).  In partial mode: the slices added in slice order, one bf16 rounding (what the router's own
-// finishing pass computes, moe_router.hip), optionally copied out.
-__device__ __forceinline__ float fetch_logit(const LogitSource& src, int M, int E, int t, int e) {
-  if (!src.partial) return src.logits[(size_t)t * E + e];
-  const size_t MN = (size_t)M * src.N, at = (size_t)t * src.N + e;
-  float s = src.partial[at];
-  for (int z = 1; z < src.splits; ++z) s = __fadd_rn(s, src.partial[(size_t)z * MN + at]);
-  const float v = bf16_to_f32(f32_to_bf16(s));
-  if (src.out_logits) src.out_logits[(size_t)t * E + e] = v;
-  return v;
-}
-// the shared expert's gate rides in column E of the partial sums: one lane per token finishes it
-__device__ __forceinline__ void finish_shared_gate(const LogitSource& src, int M, int E, int t) {
-  if (!src.partial || !src.shared_gate || src.N <= E) return;
-  const size_t MN = (size_t)M * src.N, at = (size_t)t * src.N + E;
-  float s = src.partial[at];
-  for (int z = 1; z < src.splits; ++z) s = __fadd_rn(s, src.partial[(size_t)z * MN + at]);
-  src.shared_gate[t] = bf16_to_f32(f32_to_bf16(sigmoid_det(bf16_to_f32(f32_to_bf16(s)))));
+__device__ __forceinline__ float lane_f32(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
-// VPL = values per lane; element e lives in lane e%64, slot e/64.
-template <int VPL>
-__global__ __launch_bounds__(kWavesPerBlock* MOE_WAVE) void route_softmax_kernel(
-    const LogitSource src, int M, int E, int k, int renorm, int32_t* __restrict__ idx,
-    float* __restrict__ w, const QuantJob quant) {
-  const unsigned route_blocks = gridDim.x - quant.blocks;
-  if (blockIdx.x >= route_blocks) {   // the blocks behind the routing blocks quantise the activations (QuantJob)
-    moe_quant_act_block(quant, blockIdx.x - route_blocks);
-    return;
-  }
+// the k best of the wave's keys in order, ties to the lower index.  BLOCKED: element e lives in lane e / VPL, slot
+// e % VPL; otherwise in lane e % 64, slot e / 64.  Lane i keeps the i-th: its index, key and (SCORES) score.
+template <int VPL, bool BLOCKED, bool SCORES>
+__device__ __forceinline__ void select_topk(unsigned (&key)[VPL], const float* score, int k, int& my_idx, unsigned& my_key,
+                                            float& my_score) {
   const int lane = threadIdx.x & 63;
-  const int t = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
-  if (t >= M) return;
-  if (lane == 0) finish_shared_gate(src, M, E, t);
-  float v[VPL];
-  unsigned long long key[VPL];
-  float mx = -INFINITY;
-#pragma unroll
-  for (int s = 0; s < VPL; ++s) {
-    int e = lane + 64 * s;
-    bool ok = e < E;
-    v[s] = ok ? fetch_logit(src, M, E, t, e) : -INFINITY;
-    key[s] = ok ? make_key(v[s], (unsigned)e) : 0ull;
-    mx = fmaxf(mx, v[s]);
-  }
-  mx = wave_max_f32(mx);
-  float part = 0.f;
-#pragma unroll
-  for (int s = 0; s < VPL; ++s)
-    if (lane + 64 * s < E) part = __fadd_rn(part, exp_det(__fsub_rn(v[s], mx)));
-  const float denom = wave_sum_f32(part);
-
-  int my_idx = 0;
-  float my_p = 0.f, psum = 0.f;
   for (int sel = 0; sel < k; ++sel) {
-    unsigned long long best = 0ull;
+    unsigned local = key[0];
 #pragma unroll
-    for (int s = 0; s < VPL; ++s) best = key[s] > best ? key[s] : best;
-    best = wave_max_u64(best);
-    const unsigned e = key_index(best);
+    for (int s = 1; s < VPL; ++s) local = max(local, key[s]);
+    const unsigned best = wave_max(local);
+    int owner = 0, slot = 0;
+    if (BLOCKED) {
+      owner = (int)__builtin_ctzll(__ballot(local == best));
 #pragma unroll
-    for (int s = 0; s < VPL; ++s)
-      if (key[s] == best) key[s] = 0ull;
-    const float p = __fdiv_rn(exp_det(__fsub_rn(key_value(best), mx)), denom);
-    psum = __fadd_rn(psum, p);
-    if (lane == sel) {
-      my_idx = (int)e;
-      my_p = p;
-    }
-  }
-  if (lane < k) {
-    idx[(size_t)t * k + lane] = my_idx;
-    w[(size_t)t * k + lane] = renorm ? __fdiv_rn(my_p, psum) : my_p;
-  }
-}
-
-template <int VPL>
-__global__ __launch_bounds__(kWavesPerBlock* MOE_WAVE) void route_sigmoid_grouped_kernel(
-    const LogitSource src, const float* __restrict__ bias, int M, int E, int n_group,
-    int topk_group, int k, int renorm, float routed_scale, int32_t* __restrict__ idx,
-    float* __restrict__ w, const QuantJob quant) {
-  const unsigned route_blocks = gridDim.x - quant.blocks;
-  if (blockIdx.x >= route_blocks) {   // the blocks behind the routing blocks quantise the activations (QuantJob)
-    moe_quant_act_block(quant, blockIdx.x - route_blocks);
-    return;
-  }
-  const int lane = threadIdx.x & 63;
-  const int t = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
-  if (t >= M) return;
-  if (lane == 0) finish_shared_gate(src, M, E, t);
-  const int per = E / n_group;
-  float score[VPL];
-  unsigned long long key[VPL];
-  int gid[VPL];   // group of each slot's expert (one integer division per slot, not one per group and slot)
+      for (int s = VPL - 1; s >= 0; --s)
+        if ((unsigned)__builtin_amdgcn_readlane((int)key[s], owner) == best) slot = s;
+    } else {
 #pragma unroll
-  for (int s = 0; s < VPL; ++s) {
-    int e = lane + 64 * s;
-    bool ok = e < E;
-    score[s] = ok ? sigmoid_det(fetch_logit(src, M, E, t, e)) : 0.f;
-    float choice = __fadd_rn(score[s], (ok && bias) ? bias[e] : 0.f);
-    key[s] = ok ? make_key(choice, (unsigned)e) : 0ull;
-    gid[s] = ok ? e / per : -1;
-  }
-  // group score = sum of the two best choice scores of the group (lane g keeps group g's)
-  unsigned long long gkey = 0ull;
-  for (int g = 0; g < n_group; ++g) {
-    unsigned long long b1 = 0ull, b2 = 0ull;
-#pragma unroll
-    for (int s = 0; s < VPL; ++s) {
-      bool in = gid[s] == g;
-      b1 = (in && key[s] > b1) ? key[s] : b1;
-    }
-    b1 = wave_max_u64(b1);
-    float gs = key_value(b1);
-    if (per >= 2) {
-#pragma unroll
-      for (int s = 0; s < VPL; ++s) {
-        bool in = gid[s] == g && key[s] < b1;
-        b2 = (in && key[s] > b2) ? key[s] : b2;
+      for (int s = VPL - 1; s >= 0; --s) {
+        const unsigned long long in = __ballot(key[s] == best);
+        if (in) owner = (int)__builtin_ctzll(in), slot = s;
       }
-      b2 = wave_max_u64(b2);
-      gs = __fadd_rn(gs, key_value(b2));
     }
-    if (lane == g) gkey = make_key(gs, (unsigned)g);
-  }
-  unsigned long long keep = 0ull;  // bit g set = group g kept
-  for (int sel = 0; sel < topk_group; ++sel) {
-    unsigned long long best = wave_max_u64(gkey);
-    if (gkey == best) gkey = 0ull;
-    keep |= 1ull << key_index(best);
-  }
-#pragma unroll
-  for (int s = 0; s < VPL; ++s) {
-    const int g = gid[s];
-    if (g < 0 || g >= n_group || !((keep >> g) & 1ull)) key[s] = 0ull;
-  }
-  int my_idx = 0;
-  float my_w = 0.f, wsum = 0.f;
-  for (int sel = 0; sel < k; ++sel) {
-    unsigned long long best = 0ull;
-#pragma unroll
-    for (int s = 0; s < VPL; ++s) best = key[s] > best ? key[s] : best;
-    best = wave_max_u64(best);
-    const unsigned e = key_index(best);
     float sv = 0.f;
 #pragma unroll
     for (int s = 0; s < VPL; ++s) {
-      if (key[s] == best) key[s] = 0ull;
-      if ((int)(e >> 6) == s) sv = score[s];
+      if (SCORES) {
+        const float v = lane_f32(score[s], owner);
+        sv = s == slot ? v : sv;
+      }
+      if (s == slot && lane == owner) key[s] = 0u;
     }
-    sv = __shfl(sv, (int)(e & 63u), MOE_WAVE);
-    wsum = __fadd_rn(wsum, sv);
     if (lane == sel) {
-      my_idx = (int)e;
-      my_w = sv;
+      my_idx = BLOCKED ? owner * VPL + slot : owner + 64 * slot;
+      my_key = best;
+      my_score = sv;
     }
   }
-  if (lane < k) {
-    float r = my_w;
-    if (renorm) r = __fdiv_rn(r, __fadd_rn(wsum, 1e-20f));
-    idx[(size_t)t * k + lane] = my_idx;
-    w[(size_t)t * k + lane] = __fmul_rn(r, routed_scale);
+}
+// sum of the first k lanes' values in lane order
+__device__ __forceinline__ float sum_first(float v, int k) {
+  float s = 0.f;
+  for (int i = 0; i < k; ++i) s = __fadd_rn(s, lane_f32(v, i));
+  return s;
+}
+
+constexpr int ROUTE_SOFTMAX = MOE_ROUTING_SOFTMAX, ROUTE_GROUPED = MOE_ROUTING_SIGMOID_GROUPED;
+
+// One token's selection by one wave.  row: its logits (global memory or LDS).  Returns the chosen expert (lane < k).
+template <int VPL>
+__device__ __forceinline__ int route_softmax_token(const RouteArgs& a, const float* row, int t) {
+  const int lane = threadIdx.x & 63;
+  float v[VPL];
+  unsigned key[VPL], top = 0u;
+#pragma unroll
+  for (int s = 0; s < VPL; ++s) {
+    const int e = lane + 64 * s;
+    v[s] = e < a.E ? row[e] : -INFINITY;
+    key[s] = e < a.E ? make_key(v[s]) : 0u;
+    top = max(top, key[s]);
+  }
+  const float mx = key_value(wave_max(top));
+  float part = 0.f;
+#pragma unroll
+  for (int s = 0; s < VPL; ++s)
+    if (lane + 64 * s < a.E) part = __fadd_rn(part, exp_det(__fsub_rn(v[s], mx)));
+  const float denom = wave_sum_f32(part);
+  int my_idx = 0;
+  unsigned my_key = 0u;
+  float unused;
+  select_topk<VPL, false, false>(key, nullptr, a.k, my_idx, my_key, unused);
+  const float p = __fdiv_rn(exp_det(__fsub_rn(key_value(my_key), mx)), denom);
+  const float psum = sum_first(p, a.k);
+  if (lane < a.k) {
+    a.idx[(size_t)t * a.k + lane] = my_idx;
+    a.w[(size_t)t * a.k + lane] = a.renorm ? __fdiv_rn(p, psum) : p;
+  }
+  return my_idx;
+}
+
+template <int VPL>
+__device__ __forceinline__ int route_grouped_token(const RouteArgs& a, const float* row, int t) {
+  const int lane = threadIdx.x & 63, E = a.E, n_group = a.n_group;
+  float score[VPL];
+  unsigned key[VPL];
+#pragma unroll
+  for (int s = 0; s < VPL; ++s) {
+    const int e = lane * VPL + s;
+    const bool ok = e < E;
+    score[s] = ok ? sigmoid_det(row[e]) : 0.f;
+    const float choice = __fadd_rn(score[s], (ok && a.bias) ? a.bias[e] : 0.f);
+    key[s] = ok ? make_key(choice) : 0u;
+  }
+  if (a.topk_group < n_group) {
+    // group score = sum of the two best choice scores of the group; a group is kept if fewer than topk_group of the
+    // groups score higher (ties: lower index)
+    const int per = E / n_group, lpg = per / VPL;   // experts and lanes per group
+    if (lpg * VPL == per && (lpg & (lpg - 1)) == 0 && lpg >= 1 && lpg <= 16 && per >= 2) {
+      // every group is a run of 1, 2, 4, 8 or 16 lanes: all groups' two best at once, by DPP
+      unsigned m1 = key[0], m2 = 0u;
+#pragma unroll
+      for (int s = 1; s < VPL; ++s) {
+        m2 = max(m2, min(m1, key[s]));
+        m1 = max(m1, key[s]);
+      }
+      auto meet = [&](unsigned o1, unsigned o2) {
+        m2 = max(min(m1, o1), max(m2, o2));
+        m1 = max(m1, o1);
+      };
+      if (lpg > 1) meet(dpp<DPP_XOR1>(m1), dpp<DPP_XOR1>(m2));
+      if (lpg > 2) meet(dpp<DPP_XOR2>(m1), dpp<DPP_XOR2>(m2));
+      if (lpg > 4) meet(dpp<DPP_MIRROR8>(m1), dpp<DPP_MIRROR8>(m2));
+      if (lpg > 8) meet(dpp<DPP_MIRROR16>(m1), dpp<DPP_MIRROR16>(m2));
+      const int g = lane / lpg;
+      const unsigned gkey = make_key(__fadd_rn(key_value(m1), key_value(m2)));
+      int rank = 0;
+      for (int o = 0; o < n_group; ++o) {
+        const unsigned ok = (unsigned)__builtin_amdgcn_readlane((int)gkey, o * lpg);
+        rank += (ok > gkey || (ok == gkey && o < g)) ? 1 : 0;
+      }
+      const bool keep = rank < a.topk_group;
+#pragma unroll
+      for (int s = 0; s < VPL; ++s) key[s] = keep ? key[s] : 0u;
+    } else {   // groups that lie across lanes in any way: one at a time (lane g keeps group g's score)
+      unsigned gkey = 0u;
+      int gid[VPL];
+#pragma unroll
+      for (int s = 0; s < VPL; ++s) gid[s] = lane * VPL + s < E ? (lane * VPL + s) / per : -1;
+      for (int g = 0; g < n_group; ++g) {
+        unsigned m = 0u;
+#pragma unroll
+        for (int s = 0; s < VPL; ++s) m = max(m, gid[s] == g ? key[s] : 0u);
+        const unsigned b1 = wave_max(m);
+        float gs = key_value(b1);
+        if (per >= 2) {
+          int same = 0;
+          m = 0u;
+#pragma unroll
+          for (int s = 0; s < VPL; ++s) {
+            same += __popcll(__ballot(gid[s] == g && key[s] == b1));
+            m = max(m, gid[s] == g && key[s] < b1 ? key[s] : 0u);
+          }
+          const unsigned b2 = same > 1 ? b1 : wave_max(m);
+          gs = __fadd_rn(gs, key_value(b2));
+        }
+        if (lane == g) gkey = make_key(gs);
+      }
+      int rank = 0;
+      for (int o = 0; o < n_group; ++o) {
+        const unsigned ok = (unsigned)__builtin_amdgcn_readlane((int)gkey, o);
+        rank += (ok > gkey || (ok == gkey && o < lane)) ? 1 : 0;
+      }
+      const unsigned long long keep = __ballot(lane < n_group && rank < a.topk_group);   // bit g set = group g kept
+#pragma unroll
+      for (int s = 0; s < VPL; ++s)
+        if (gid[s] < 0 || !((keep >> gid[s]) & 1ull)) key[s] = 0u;
+    }
+  }
+  int my_idx = 0;
+  unsigned my_key = 0u;
+  float my_w = 0.f;
+  select_topk<VPL, true, true>(key, score, a.k, my_idx, my_key, my_w);
+  const float wsum = sum_first(my_w, a.k);
+  if (lane < a.k) {
+    const float r = a.renorm ? __fdiv_rn(my_w, __fadd_rn(wsum, 1e-20f)) : my_w;
+    a.idx[(size_t)t * a.k + lane] = my_idx;
+    a.w[(size_t)t * a.k + lane] = __fmul_rn(r, a.routed_scale);
+  }
+  return my_idx;
+}
+
+template <int N> __device__ __forceinline__ void add_slices(float& s, const float*& q, size_t stride) {
+  float v[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) v[j] = *(q += stride);
+#pragma unroll
+  for (int j = 0; j < N; ++j) s = __fadd_rn(s, v[j]);
+}
+
+// Workgroup c routes tokens [c * tokens_per_block, +tokens_per_block).  Around the selection:
+//  - LogitSource's partial sums are added by the whole workgroup for as many tokens as it has waves (a token's columns
+//    are contiguous in every slice: independent coalesced loads, eight in flight per thread) and the waves then read
+//    the rounded logits from LDS.  One wave summing its own token one load at a time took 87 us for 32 tokens of 513
+//    columns in 32 slices, most of the layer's overhead; this way 9 us.
+//  - chunk_hist: the workgroup's selections are counted for the sort by expert (one row of E counts per workgroup).
+//  - sort_here (one workgroup routes the whole batch): the sort itself follows in the same launch.
+//  - the blocks behind the routing blocks quantise the activations: independent work, one launch less.
+struct RouteJob {
+  int blocks, tokens_per_block, batch;   // batch: tokens whose partial sums are added at a time
+  int32_t* chunk_hist;                   // [blocks][E] or null
+};
+constexpr int kSortHereTokens = 8;
+
+template <int VPL, int KIND, bool SORT_HERE>
+__global__ __launch_bounds__(1024) void route_kernel(const RouteArgs a, const RouteJob job, const QuantJob quant, const PermuteOut sort) {
+  if ((int)blockIdx.x >= job.blocks) {
+    moe_quant_act_block(quant, (int)blockIdx.x - job.blocks);
+    return;
+  }
+  extern __shared__ __attribute__((aligned(16))) int lds[];   // [ids when sort_here][E counts][logits or the sort's counters]
+  int* ids = lds;
+  int* hist = lds + (SORT_HERE ? kSmallRows : 0);
+  float* rows = (float*)(hist + a.E);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  const int first = blockIdx.x * job.tokens_per_block, last = min(a.M, first + job.tokens_per_block);
+  if (!SORT_HERE && job.chunk_hist)
+    for (int e = threadIdx.x; e < a.E; e += blockDim.x) hist[e] = 0;
+  __syncthreads();
+  const int N = a.src.N;
+  for (int t0 = first; t0 < last; t0 += job.batch) {
+    const int nt = min(job.batch, last - t0);
+    if (a.src.partial) {
+      if (t0 > first) __syncthreads();   // (the waves are done with the batch before)
+      const size_t MN = (size_t)a.M * N;
+      const float* p = a.src.partial + (size_t)t0 * N;
+      for (int i = threadIdx.x; i < nt * N; i += blockDim.x) {
+        const float* q = p + i;
+        float s = *q;
+        int z = 1;   // the slices in slice order, a batch of independent loads at a time
+        for (; z + 8 <= a.src.splits; z += 8) add_slices<8>(s, q, MN);
+        for (; z + 4 <= a.src.splits; z += 4) add_slices<4>(s, q, MN);
+        for (; z < a.src.splits; ++z) add_slices<1>(s, q, MN);
+        rows[i] = bf16_to_f32(f32_to_bf16(s));   // what the router's own finishing pass computes
+      }
+      __syncthreads();
+    }
+    for (int tt = wave; tt < nt; tt += waves) {
+      const int t = t0 + tt;
+      const float* row = a.src.partial ? rows + tt * N : a.src.logits + (size_t)t * a.E;
+      if (a.src.partial) {
+        if (a.src.out_logits)
+          for (int e = lane; e < a.E; e += MOE_WAVE) a.src.out_logits[(size_t)t * a.E + e] = row[e];
+        if (lane == 0 && a.src.shared_gate && N > a.E)   // the shared expert's gate rides in column E
+          a.src.shared_gate[t] = bf16_to_f32(f32_to_bf16(sigmoid_det(row[a.E])));
+      }
+      const int chosen = KIND == ROUTE_SOFTMAX ? route_softmax_token<VPL>(a, row, t) : route_grouped_token<VPL>(a, row, t);
+      if (lane < a.k) {
+        if (!SORT_HERE && job.chunk_hist) atomicAdd(&hist[chosen], 1);
+        if (SORT_HERE) ids[t * a.k + lane] = chosen;
+      }
+    }
+  }
+  if (!SORT_HERE && job.chunk_hist) {
+    __syncthreads();
+    for (int e = threadIdx.x; e < a.E; e += blockDim.x) job.chunk_hist[(size_t)blockIdx.x * a.E + e] = hist[e];
+  }
+  if (SORT_HERE) {
+    __syncthreads();
+    permute_one_chunk(ids, a.M * a.k, a.E, hist, sort);   // (the counters take the place of counts and logits)
   }
 }
 
-int check_route_args(const LogitSource& src, int M, int E, int k, const int32_t* idx, const float* w) {
-  MOE_REQUIRE(M == 0 || ((src.logits || src.partial) && idx && w), MOE_ERR_NULL, "route: null pointer");
+int check_route_args(int routing, const RouteArgs& a) {
+  const LogitSource& src = a.src;
+  const int M = a.M, E = a.E, k = a.k;
+  MOE_REQUIRE(M == 0 || ((src.logits || src.partial) && a.idx && a.w), MOE_ERR_NULL, "route: null pointer");
   MOE_REQUIRE(!src.partial || (src.splits >= 1 && src.N >= E), MOE_ERR_BAD_SHAPE, "route: bad partial-sum layout");
   MOE_REQUIRE(M >= 0 && E >= 1 && E <= 1024, MOE_ERR_BAD_SHAPE, "route: need 1 <= E <= 1024, got E=%d M=%d", E, M);
   MOE_REQUIRE(k >= 1 && k <= 32 && k <= E, MOE_ERR_BAD_SHAPE, "route: need 1 <= k <= min(32,E), got k=%d E=%d", k, E);
+  if (routing == MOE_ROUTING_SIGMOID_GROUPED) {
+    MOE_REQUIRE(a.n_group >= 1 && a.n_group <= 64 && E % a.n_group == 0, MOE_ERR_BAD_SHAPE,
+                "route: n_group=%d must divide E=%d and be <= 64", a.n_group, E);
+    MOE_REQUIRE(a.topk_group >= 1 && a.topk_group <= a.n_group, MOE_ERR_BAD_SHAPE,
+                "route: topk_group=%d out of range for n_group=%d", a.topk_group, a.n_group);
+    MOE_REQUIRE(k <= a.topk_group * (E / a.n_group), MOE_ERR_BAD_SHAPE,
+                "route: k=%d exceeds the %d experts of the kept groups", k, a.topk_group * (E / a.n_group));
+  }
   return MOE_OK;
+}
+
+template <int KIND, bool SORT_HERE>
+void launch_route(int vpl, dim3 grid, dim3 block, size_t lds, hipStream_t s, const RouteArgs& a, const RouteJob& job,
+                  const QuantJob& q, const PermuteOut& o) {
+  if (vpl <= 1) hipLaunchKernelGGL((route_kernel<1, KIND, SORT_HERE>), grid, block, lds, s, a, job, q, o);
+  else if (vpl <= 2) hipLaunchKernelGGL((route_kernel<2, KIND, SORT_HERE>), grid, block, lds, s, a, job, q, o);
+  else if (vpl <= 4) hipLaunchKernelGGL((route_kernel<4, KIND, SORT_HERE>), grid, block, lds, s, a, job, q, o);
+  else if (vpl <= 8) hipLaunchKernelGGL((route_kernel<8, KIND, SORT_HERE>), grid, block, lds, s, a, job, q, o);
+  else hipLaunchKernelGGL((route_kernel<16, KIND, SORT_HERE>), grid, block, lds, s, a, job, q, o);
 }
 
 }  // namespace
 
-static_assert(kWavesPerBlock * MOE_WAVE == 256, "a routing block doubles as a quantiser block of 256 pieces");
-#define DISPATCH_VPL(E, KERNEL, ...)                                                      \
-  do {                                                                                    \
-    dim3 grid((M + kWavesPerBlock - 1) / kWavesPerBlock + qj.blocks), block(kWavesPerBlock* MOE_WAVE); \
-    int vpl = ((E) + 63) / 64;                                                            \
-    if (vpl <= 1) hipLaunchKernelGGL(KERNEL<1>, grid, block, 0, s, __VA_ARGS__);          \
-    else if (vpl <= 2) hipLaunchKernelGGL(KERNEL<2>, grid, block, 0, s, __VA_ARGS__);     \
-    else if (vpl <= 4) hipLaunchKernelGGL(KERNEL<4>, grid, block, 0, s, __VA_ARGS__);     \
-    else if (vpl <= 8) hipLaunchKernelGGL(KERNEL<8>, grid, block, 0, s, __VA_ARGS__);     \
-    else hipLaunchKernelGGL(KERNEL<16>, grid, block, 0, s, __VA_ARGS__);                  \
-  } while (0)
-
-int moe_route_softmax_impl(const LogitSource& src, int M, int E, int k, int renorm, int32_t* idx, float* w,
-                           moe_stream_t stream, const QuantJob* quant) {
-  int rc = check_route_args(src, M, E, k, idx, w);
-  if (rc) return rc;
-  MOE_REQUIRE(!quant || M > 0, MOE_ERR_BAD_SHAPE, "route: nothing to carry a quantisation with");
-  if (M == 0) return MOE_OK;
+int moe_route_impl(int routing, const RouteArgs& a, const QuantJob* quant, const PermuteOut* sort, void* permute_ws,
+                   size_t permute_ws_bytes, moe_stream_t stream) {
+  if (int rc = check_route_args(routing, a)) return rc;
+  MOE_REQUIRE((!quant && !sort) || a.M > 0, MOE_ERR_BAD_SHAPE, "route: nothing to carry a quantisation or a sort with");
+  MOE_REQUIRE(!sort || (permute_ws && permute_ws_bytes >= moe_permute_workspace_bytes(a.M, a.k, a.E)), MOE_ERR_WORKSPACE_TOO_SMALL,
+              "route: permutation workspace too small");
+  MOE_REQUIRE(!sort || (long long)a.M * a.k < (1ll << 31), MOE_ERR_BAD_SHAPE, "route: M*k overflows int32");
+  if (a.M == 0) return MOE_OK;
+  const int R = a.M * a.k;
+  RouteJob job{};
+  // Partial sums: a token per workgroup while there are few tokens (the summing is the work then); ready logits: a
+  // token per wave.  Many tokens: as many per workgroup as keep the sort's histograms few.
+  const int max_chunks = moe_permute_max_chunks(a.E);
+  int tpb = a.src.partial ? 1 : 4;
+  if ((a.M + max_chunks - 1) / max_chunks > tpb) tpb = (a.M + max_chunks - 1) / max_chunks;
+  // One workgroup takes a batch whose partial sums (if any) it can add about as fast as many would: the sort needs no
+  // launch of its own then.
+  const bool sort_here = sort && a.M <= kSortHereTokens && R <= kSmallRows &&
+                  (!a.src.partial || (long long)a.M * a.src.N * a.src.splits <= 65536);
+  if (sort_here) tpb = a.M;
+  const int threads = sort_here || tpb >= 8 ? 1024 : 256;
+  job.tokens_per_block = tpb;
+  job.blocks = (a.M + tpb - 1) / tpb;
+  const bool one_chunk = R <= kSmallRows;   // the placing kernel counts such a list itself
+  job.chunk_hist = sort && !sort_here && !one_chunk ? (int32_t*)permute_ws : nullptr;
+  job.batch = tpb;
+  size_t ints = (sort_here ? kSmallRows : 0) + (size_t)a.E;
+  size_t tail = 0;
+  if (a.src.partial) {
+    const int room = 12288 / a.src.N;   // 48 KB of logits (N <= 1025)
+    const int waves = threads / MOE_WAVE;
+    job.batch = waves < room ? waves : room;
+    if (job.batch > tpb) job.batch = tpb;
+    tail = (size_t)job.batch * a.src.N;
+  }
+  if (sort_here && moe_place_lds_ints(a.E) > tail) tail = moe_place_lds_ints(a.E);
+  const size_t lds = (ints + tail) * sizeof(int);
+  const QuantJob q = quant ? *quant : QuantJob{};
+  const PermuteOut o = sort ? *sort : PermuteOut{};
+  const dim3 grid(job.blocks + (quant ? moe_quant_blocks(q, threads) : 0)), block(threads);
+  const int vpl = (a.E + 63) / 64;
   hipStream_t s = (hipStream_t)stream;
-  const QuantJob qj = quant ? *quant : QuantJob{};
-  DISPATCH_VPL(E, route_softmax_kernel, src, M, E, k, renorm, idx, w, qj);
-  return moe_check_hip(hipGetLastError(), "route_softmax launch");
+  const auto launch = routing == MOE_ROUTING_SOFTMAX ? (sort_here ? launch_route<ROUTE_SOFTMAX, true> : launch_route<ROUTE_SOFTMAX, false>)
+                                                      : (sort_here ? launch_route<ROUTE_GROUPED, true> : launch_route<ROUTE_GROUPED, false>);
+  launch(vpl, grid, block, lds, s, a, job, q, o);
+  if (int rc = moe_check_hip(hipGetLastError(), "route launch")) return rc;
+  if (!sort || sort_here) return MOE_OK;
+  if (one_chunk) return moe_permute_place(a.idx, R, a.E, kSmallRows, 1, nullptr, o, stream);
+  return moe_permute_place(a.idx, R, a.E, tpb * a.k, job.blocks, job.chunk_hist, o, stream);
 }
 
 extern "C" int moe_route_softmax_topk(const float* logits, int M, int E, int k, int renorm,
                                       int32_t* idx, float* w, moe_stream_t stream) {
-  return moe_route_softmax_impl(LogitSource{logits, nullptr, 0, E, nullptr, nullptr}, M, E, k, renorm, idx, w, stream, nullptr);
-}
-
-int moe_route_sigmoid_grouped_impl(const LogitSource& src, const float* bias, int M, int E, int n_group,
-                                   int topk_group, int k, int renorm, float routed_scale, int32_t* idx, float* w,
-                                   moe_stream_t stream, const QuantJob* quant) {
-  int rc = check_route_args(src, M, E, k, idx, w);
-  if (rc) return rc;
-  MOE_REQUIRE(!quant || M > 0, MOE_ERR_BAD_SHAPE, "route: nothing to carry a quantisation with");
-  MOE_REQUIRE(n_group >= 1 && n_group <= 64 && E % n_group == 0, MOE_ERR_BAD_SHAPE,
-              "route: n_group=%d must divide E=%d and be <= 64", n_group, E);
-  MOE_REQUIRE(topk_group >= 1 && topk_group <= n_group, MOE_ERR_BAD_SHAPE,
-              "route: topk_group=%d out of range for n_group=%d", topk_group, n_group);
-  MOE_REQUIRE(k <= topk_group * (E / n_group), MOE_ERR_BAD_SHAPE,
-              "route: k=%d exceeds the %d experts of the kept groups", k, topk_group * (E / n_group));
-  if (M == 0) return MOE_OK;
-  hipStream_t s = (hipStream_t)stream;
-  const QuantJob qj = quant ? *quant : QuantJob{};
-  DISPATCH_VPL(E, route_sigmoid_grouped_kernel, src, bias, M, E, n_group, topk_group, k, renorm,
-               routed_scale, idx, w, qj);
-  return moe_check_hip(hipGetLastError(), "route_sigmoid_grouped launch");
+  const RouteArgs a{LogitSource{logits, nullptr, 0, E, nullptr, nullptr}, nullptr, M, E, k, renorm, 1, 1, 1.f, idx, w};
+  return moe_route_impl(MOE_ROUTING_SOFTMAX, a, nullptr, nullptr, nullptr, 0, stream);
 }
 
 extern "C" int moe_route_sigmoid_grouped(const float* logits, const float* bias, int M, int E,
                                          int n_group, int topk_group, int k, int renorm,
                                          float routed_scale, int32_t* idx, float* w,
                                          moe_stream_t stream) {
-  return moe_route_sigmoid_grouped_impl(LogitSource{logits, nullptr, 0, E, nullptr, nullptr}, bias, M, E, n_group,
-                                        topk_group, k, renorm, routed_scale, idx, w, stream, nullptr);
+  const RouteArgs a{LogitSource{logits, nullptr, 0, E, nullptr, nullptr}, bias, M, E, k, renorm, n_group, topk_group,
+                    routed_scale, idx, w};
+  return moe_route_impl(MOE_ROUTING_SIGMOID_GROUPED, a, nullptr, nullptr, nullptr, 0, stream);
 }
