@@ -206,7 +206,7 @@ typedef struct MoeForwardArgs {
   int add_residual;              /* out = x + moe_out, added in f32 before the one bf16 rounding */
 } MoeForwardArgs;
 
-/* Host-side objects moe_forward creates.  No device memory is ever allocated.  A large batch (M * D above 2 M elements)
+/* Host-side objects moe_forward creates.  No device memory is ever allocated.  A large batch (M * D above 16 M elements)
  * with a shared expert (SI > 0) runs the shared expert beside the routing chain: the call (a) creates, on the first such
  * call on a device, ONE side stream for that device (default priority, kept until the process ends, shared by every
  * caller stream and host thread) and (b) uses three hipEvents per host thread and device, created on first use, so
@@ -217,6 +217,9 @@ typedef struct MoeForwardArgs {
  * thread only).  Every other call creates neither stream nor event. */
 MOE_API size_t moe_forward_workspace_bytes(int M, int D, int E, int k, int I, int SI);
 MOE_API int moe_forward(const MoeForwardArgs* args, void* ws, size_t ws_bytes, moe_stream_t stream);
+/* The same for a caller whose activations are f32 (moe.py:282): args->x and args->out are (M, D) f32; x is rounded to
+ * bf16 on the way in and out holds the bf16 results, as if moe_convert stood on either side. */
+MOE_API int moe_forward_f32(const MoeForwardArgs* args, void* ws, size_t ws_bytes, moe_stream_t stream);
 
 #ifdef __cplusplus
 }

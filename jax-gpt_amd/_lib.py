@@ -66,6 +66,7 @@ SIGNATURES = {
     "moe_convert": (_I, [_P, _I, _P, _I, C.c_longlong, _P]),
     "moe_forward_workspace_bytes": (_Z, [_I, _I, _I, _I, _I, _I]),
     "moe_forward": (_I, [C.POINTER(MoeForwardArgs), _P, _Z, _P]),
+    "moe_forward_f32": (_I, [C.POINTER(MoeForwardArgs), _P, _Z, _P]),
 }
 
 

@@ -130,17 +130,22 @@ ForwardBuffers carve(void* ws, int M, int D, int E, int k, int I, int SI, bool r
 }  // namespace
 
 namespace {
-// the activations the layer computes from: x itself, or its RMS-normalised form (kept in bf16 for the router)
+// The activations that the router's matmul and the experts compute from: x itself, its RMS-normalised form or, from f32
+// input, its bf16 rounding; the latter two are kept in b.normed for the matmul.
 // (sx_blocked: an optional second copy of the scales, block-major in token order, for the shared expert of a large batch)
-int quantise(const MoeForwardArgs* a, const ForwardBuffers& b, float* sx_blocked, moe_stream_t stream) {
+bool quantiser_feeds_router(const MoeForwardArgs* a, int io_f32) { return a->norm_weight || (io_f32 && a->w_router); }
+int quantise(const MoeForwardArgs* a, int io_f32, const ForwardBuffers& b, float* sx_blocked, moe_stream_t stream) {
   if (a->norm_weight)
-    return moe_rmsnorm_quant_impl(a->x, a->norm_weight, a->norm_eps, a->M, a->D, b.normed, b.xq, b.sx, sx_blocked, stream);
-  return moe_quant_act_impl(a->x, a->M, a->D, b.xq, b.sx, sx_blocked, stream);
+    return moe_rmsnorm_quant_impl(a->x, io_f32, a->norm_weight, a->norm_eps, a->M, a->D, b.normed, b.xq, b.sx, sx_blocked, stream);
+  return moe_quant_act_impl(a->x, io_f32, quantiser_feeds_router(a, io_f32) ? b.normed : nullptr, a->M, a->D, b.xq, b.sx, sx_blocked, stream);
 }
 
-// Whether a call with a shared expert runs it inside the routed launches (true) or on the side stream.  From about
-// 2 M activation elements on, the shared expert's GEMMs fill the gap that routing and permutation leave.
-bool small_batch(int M, int D) { return (long long)M * D <= (1ll << 21); }
+// Whether a call with a shared expert runs it inside the routed launches (true) or on the side stream.  The shared
+// expert's GEMMs can fill the gap that quantising, routing and sorting leave in front of the routed ones, for the price
+// of two streams' events.  Measured, together against forked: 4000 tokens of the mini layer 72 / 105 us, 2047 tokens of
+// the Qwen3.5 layer 1269 / 1294 us, 4096 tokens 1456 / 1481; the DeepSeek-V3 layer at 777 tokens 1508 / 1513, at 2048
+// 1975 / 1970, at 4096 2518 / 2505, at 8192 3847 / 3830 us.
+bool small_batch(int M, int D) { return (long long)M * D <= (1ll << 24); }
 }  // namespace
 
 extern "C" size_t moe_forward_workspace_bytes(int M, int D, int E, int k, int I, int SI) {
@@ -148,7 +153,7 @@ extern "C" size_t moe_forward_workspace_bytes(int M, int D, int E, int k, int I,
   return carve(nullptr, M, D, E, k, I, SI, true).total;   // room for the router whether or not a call uses it
 }
 
-extern "C" int moe_forward(const MoeForwardArgs* a, void* ws, size_t ws_bytes, moe_stream_t stream) {
+static int forward(const MoeForwardArgs* a, int io_f32, void* ws, size_t ws_bytes, moe_stream_t stream) {
   MOE_REQUIRE(a && ws, MOE_ERR_NULL, "forward: null args or workspace");
   MOE_REQUIRE(a->M >= 0 && a->D > 0 && a->E >= 1 && a->k >= 1 && a->I > 0 && a->SI >= 0, MOE_ERR_BAD_SHAPE,
               "forward: bad dims M=%d D=%d E=%d k=%d I=%d SI=%d", a->M, a->D, a->E, a->k, a->I, a->SI);
@@ -225,21 +230,21 @@ extern "C" int moe_forward(const MoeForwardArgs* a, void* ws, size_t ws_bytes, m
   }
   float* sx_blocked = a->SI && blocked_scales ? b.sx_blocked : nullptr;
   // Where the quantiser would run on the caller's stream just ahead of the routing kernel, the routing launch
-  // carries its blocks instead (QuantJob: the two are independent; one launch less and they overlap).  Not with
-  // an RMSNorm in front: the router then reads what the quantiser writes.
-  const bool quant_in_route = !fork && !a->norm_weight;
+  // carries its blocks instead (QuantJob: the two are independent; one launch less and they overlap).  Not where the
+  // router reads what the quantiser writes.
+  const bool quant_in_route = !fork && !quantiser_feeds_router(a, io_f32);
   QuantJob quant_job{};
   if (quant_in_route) {
-    if ((rc = moe_quant_act_job(a->x, a->M, a->D, b.xq, b.sx, sx_blocked, &quant_job))) return rc;
+    if ((rc = moe_quant_act_job(a->x, io_f32, nullptr, a->M, a->D, b.xq, b.sx, sx_blocked, &quant_job))) return rc;
   } else if (!fork) {
-    if ((rc = quantise(a, b, sx_blocked, stream))) return rc;
+    if ((rc = quantise(a, io_f32, b, sx_blocked, stream))) return rc;
   } else {
     if ((rc = side_stream(&side))) return rc;
     if ((rc = call_events(&ev))) return rc;
     hipError_t e = hipEventRecord(ev->fork, main_s);
     if (e == hipSuccess) e = hipStreamWaitEvent(side, ev->fork, 0);
     if (e != hipSuccess) return moe_check_hip(e, "forward: fork");
-    rc_shared = quantise(a, b, sx_blocked, (moe_stream_t)side);
+    rc_shared = quantise(a, io_f32, b, sx_blocked, (moe_stream_t)side);
     if (!rc_shared) rc_shared = moe_check_hip(hipEventRecord(ev->quant, side), "forward: quant event");
     if (!rc_shared) rc_shared = moe_gemm_gateup_impl(nullptr, &shared_gateup, (moe_stream_t)side);
     if (!rc_shared) rc_shared = moe_gemm_down_impl(nullptr, &shared_down, (moe_stream_t)side);
@@ -261,14 +266,14 @@ extern "C" int moe_forward(const MoeForwardArgs* a, void* ws, size_t ws_bytes, m
   LogitSource src{a->logits, nullptr, 0, a->E, nullptr, nullptr};
   const float* shared_gate = nullptr;
   if (a->w_router) {
-    // the router reads the normalised activations, which the (possibly forked) quantiser writes
-    if (a->norm_weight && !quant_joined) {
+    const bool from_quantiser = quantiser_feeds_router(a, io_f32);
+    if (from_quantiser && !quant_joined) {   // (the quantiser was forked)
       if (rc_shared) return join(rc_shared);
       if ((rc = moe_check_hip(hipStreamWaitEvent(main_s, ev->quant, 0), "forward: quant join"))) return join(rc);
       quant_joined = true;
     }
     int splits = 0, n_cols = 0;
-    if ((rc = moe_router_partials(a->norm_weight ? b.normed : a->x, a->M, a->D, a->w_router, a->E, a->w_shared_gate,
+    if ((rc = moe_router_partials(from_quantiser ? b.normed : a->x, a->M, a->D, a->w_router, a->E, a->w_shared_gate,
                                   b.router_ws, b.router_ws_bytes, &splits, &n_cols, stream)))
       return join(rc);
     float* gate_out = a->out_shared_gate ? a->out_shared_gate : b.shared_gate;   // (written by the routing kernel)
@@ -303,6 +308,13 @@ extern "C" int moe_forward(const MoeForwardArgs* a, void* ws, size_t ws_bytes, m
   if ((rc = moe_gemm_gateup_impl(&routed_gateup, together ? &shared_gateup : nullptr, stream))) return join(rc);
   if ((rc = moe_gemm_down_impl(&routed_down, together ? &shared_down : nullptr, stream))) return join(rc);
   if ((rc = join(MOE_OK))) return rc;
-  return moe_combine(y, w, inv, a->SI ? ys : nullptr, shared_gate, a->add_residual ? a->x : nullptr, a->M, a->k,
-                     a->D, a->out, stream);
+  return moe_combine_impl(y, w, inv, a->SI ? ys : nullptr, shared_gate, a->add_residual ? a->x : nullptr, io_f32, a->M, a->k,
+                          a->D, a->out, stream);
+}
+
+extern "C" int moe_forward(const MoeForwardArgs* a, void* ws, size_t ws_bytes, moe_stream_t stream) {
+  return forward(a, 0, ws, ws_bytes, stream);
+}
+extern "C" int moe_forward_f32(const MoeForwardArgs* a, void* ws, size_t ws_bytes, moe_stream_t stream) {
+  return forward(a, 1, ws, ws_bytes, stream);
 }

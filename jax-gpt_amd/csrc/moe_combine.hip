@@ -11,15 +11,15 @@
 
 namespace {
 
-struct alignas(16) bf16x8 { bf16_t v[8]; };
+typedef moe_bf16x8 bf16x8;
 constexpr int kMaxK = 32;
 
 __global__ __launch_bounds__(256) void combine_kernel(const bf16x8* __restrict__ y, const float* __restrict__ w,
                                                      const int32_t* __restrict__ inv_perm,
                                                      const bf16x8* __restrict__ shared,
                                                      const float* __restrict__ shared_gate,
-                                                     const bf16x8* __restrict__ residual, int k, int D8,
-                                                     bf16x8* __restrict__ out) {
+                                                     const void* __restrict__ residual, int io_f32, int k, int D8,
+                                                     void* __restrict__ out) {
   __shared__ int pos[kMaxK];
   __shared__ float wt[kMaxK];
   const int t = blockIdx.x;
@@ -52,14 +52,23 @@ __global__ __launch_bounds__(256) void combine_kernel(const bf16x8* __restrict__
       }
     }
     if (residual) {
-      bf16x8 v = residual[(size_t)t * D8 + c];
+      const bf16x8 v = load_bf16x8(residual, io_f32, (size_t)t * D8 + c);
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[i] = __fadd_rn(acc[i], bf16_to_f32(v.v[i]));
     }
     bf16x8 o;
 #pragma unroll
     for (int i = 0; i < 8; ++i) o.v[i] = f32_to_bf16(acc[i]);
-    __builtin_nontemporal_store(*(v4i*)&o, (v4i*)&out[(size_t)t * D8 + c]);
+    if (io_f32) {
+      v4f lo, hi;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) lo[i] = bf16_to_f32(o.v[i]), hi[i] = bf16_to_f32(o.v[4 + i]);
+      v4f* dst = (v4f*)out + 2 * ((size_t)t * D8 + c);
+      __builtin_nontemporal_store(lo, dst);
+      __builtin_nontemporal_store(hi, dst + 1);
+    } else {
+      __builtin_nontemporal_store(*(v4i*)&o, (v4i*)out + (size_t)t * D8 + c);
+    }
   }
 }
 
@@ -68,11 +77,15 @@ __global__ __launch_bounds__(256) void combine_kernel(const bf16x8* __restrict__
 extern "C" int moe_combine(const void* y_bf16, const float* w, const int32_t* inv_perm,
                            const void* shared_bf16, const float* shared_gate, const void* residual_bf16, int M,
                            int k, int D, void* out_bf16, moe_stream_t stream) {
-  MOE_REQUIRE(M == 0 || (y_bf16 && w && inv_perm && out_bf16), MOE_ERR_NULL, "combine: null pointer");
+  return moe_combine_impl(y_bf16, w, inv_perm, shared_bf16, shared_gate, residual_bf16, 0, M, k, D, out_bf16, stream);
+}
+int moe_combine_impl(const void* y_bf16, const float* w, const int32_t* inv_perm, const void* shared_bf16, const float* shared_gate,
+                     const void* residual, int io_f32, int M, int k, int D, void* out, moe_stream_t stream) {
+  MOE_REQUIRE(M == 0 || (y_bf16 && w && inv_perm && out), MOE_ERR_NULL, "combine: null pointer");
   MOE_REQUIRE(M >= 0 && k >= 1 && k <= kMaxK && D > 0 && D % 8 == 0, MOE_ERR_BAD_SHAPE,
               "combine: need 1 <= k <= %d and D %% 8 == 0, got M=%d k=%d D=%d", kMaxK, M, k, D);
-  MOE_REQUIRE(MOE_ALIGNED16(y_bf16) && MOE_ALIGNED16(out_bf16) && MOE_ALIGNED16(shared_bf16) &&
-                  MOE_ALIGNED16(residual_bf16), MOE_ERR_BAD_ALIGN,
+  MOE_REQUIRE(MOE_ALIGNED16(y_bf16) && MOE_ALIGNED16(out) && MOE_ALIGNED16(shared_bf16) &&
+                  MOE_ALIGNED16(residual), MOE_ERR_BAD_ALIGN,
               "combine: pointers must be 16-byte aligned");
   MOE_REQUIRE(shared_bf16 || !shared_gate, MOE_ERR_NULL, "combine: a shared gate needs a shared expert output");
   if (M == 0) return MOE_OK;
@@ -80,6 +93,6 @@ extern "C" int moe_combine(const void* y_bf16, const float* w, const int32_t* in
   int split = 1;
   while (split < 8 && (long long)M * split < 1024 && (D / 8) / (split * 2) >= 64) split *= 2;
   hipLaunchKernelGGL(combine_kernel, dim3(M, split), dim3(256), 0, (hipStream_t)stream, (const bf16x8*)y_bf16, w, inv_perm,
-                     (const bf16x8*)shared_bf16, shared_gate, (const bf16x8*)residual_bf16, k, D / 8, (bf16x8*)out_bf16);
+                     (const bf16x8*)shared_bf16, shared_gate, residual, io_f32, k, D / 8, out);
   return moe_check_hip(hipGetLastError(), "combine launch");
 }

@@ -242,7 +242,9 @@ int moe_router_partials(const void* x_bf16, int M, int D, const void* w_router_b
 // An activation quantisation (moe_quant_device.h): blocks of blockDim.x 16-byte pieces, in a launch of its own or
 // behind the routing kernel's own blocks.
 struct QuantJob {
-  const void* x;        // (R, K) bf16
+  const void* x;        // (R, K) bf16, or f32 (x_f32), which is rounded to bf16 first
+  int x_f32;
+  void* x_bf16;         // optional (R, K) copy of the rounded f32 values
   long long n_pieces;   // R * K / 8
   int groups_per_row;   // K / 128
   int R;
@@ -251,7 +253,7 @@ struct QuantJob {
   float* sx_blocked;    // optional (K/128, R) copy of the scales
 };
 inline unsigned moe_quant_blocks(const QuantJob& q, int threads) { return (unsigned)((q.n_pieces + threads - 1) / threads); }
-int moe_quant_act_job(const void* x_bf16, int R, int K, uint8_t* xq, float* sx, float* sx_blocked, QuantJob* job);
+int moe_quant_act_job(const void* x, int x_f32, void* x_bf16, int R, int K, uint8_t* xq, float* sx, float* sx_blocked, QuantJob* job);
 // What the sort by expert writes (sort_order, sorted_token_ids, inv_perm: null to skip; tl.tiles null: no work list).
 struct PermuteOut {
   int32_t *group_sizes, *group_offsets, *sorted_token_ids, *sort_order, *inv_perm;
@@ -281,9 +283,14 @@ int moe_permute_place(const int32_t* idx, int R, int E, int chunk, int n_chunks,
 int moe_gemm_tile_list(int R, int E, void* ws, size_t ws_bytes, TileList* list);
 // the activation quantisers with an optional second copy of the scales, block-major in row order ((K/128, R): what
 // GemmScales{1, R} reads) -- spares the shared expert of a large batch the separate transposition
-int moe_quant_act_impl(const void* x_bf16, int R, int K, uint8_t* xq, float* sx, float* sx_blocked, moe_stream_t stream);
-int moe_rmsnorm_quant_impl(const void* x_bf16, const float* weight, float eps, int M, int D, void* normed_bf16,
+// (x_f32: x holds f32 values, rounded to bf16 first)
+int moe_quant_act_impl(const void* x, int x_f32, void* x_bf16, int R, int K, uint8_t* xq, float* sx, float* sx_blocked,
+                       moe_stream_t stream);
+int moe_rmsnorm_quant_impl(const void* x, int x_f32, const float* weight, float eps, int M, int D, void* normed_bf16,
                            uint8_t* xq, float* sx, float* sx_blocked, moe_stream_t stream);
+// the combine with the residual and the output in bf16 or (io_f32) f32, the output rounded to bf16 either way
+int moe_combine_impl(const void* y_bf16, const float* w, const int32_t* inv_perm, const void* shared_bf16, const float* shared_gate,
+                     const void* residual, int io_f32, int M, int k, int D, void* out, moe_stream_t stream);
 int moe_permute_impl(const int32_t* idx, int M, int k, int E, const PermuteOut& o, void* ws, size_t ws_bytes, moe_stream_t stream);
 // Where the grouped GEMMs find an activation scale and put an h scale, in floats: scale of (row, 128-wide K block kb)
 // = s[row * in_row + kb * in_kb].  The public entry points use the row-major arrays of the quantisers ({K/128, 1});
@@ -353,6 +360,17 @@ __device__ __forceinline__ unsigned pack2_bf16(float lo, float hi) {
   typedef __bf16 bf16x2_hw __attribute__((ext_vector_type(2)));
   const bf16x2_hw b = __builtin_convertvector((f32x2){lo, hi}, bf16x2_hw);
   return __builtin_bit_cast(unsigned, b);
+}
+
+struct alignas(16) moe_bf16x8 { bf16_t v[8]; };
+// eight neighbouring values as bf16: 16 bytes of bf16, or 32 of f32 rounded (piece p of an array)
+__device__ __forceinline__ moe_bf16x8 load_bf16x8(const void* x, int is_f32, size_t p) {
+  if (!is_f32) return ((const moe_bf16x8*)x)[p];
+  const v4f lo = ((const v4f*)x)[2 * p], hi = ((const v4f*)x)[2 * p + 1];
+  moe_bf16x8 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r.v[i] = f32_to_bf16(lo[i]), r.v[4 + i] = f32_to_bf16(hi[i]);
+  return r;
 }
 
 // scale = 448/amax (1 when the group is all zero); both quotients are IEEE-rounded

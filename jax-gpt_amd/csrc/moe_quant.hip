@@ -21,20 +21,19 @@ __global__ __launch_bounds__(256) void quant_act_kernel(const QuantJob q) { moe_
 // with individually rounded operations.
 constexpr int kNormPieces = 4;   // D <= 256 * 8 * 4 = 8192
 
-__global__ __launch_bounds__(256) void rmsnorm_quant_kernel(const bf16x8* __restrict__ x, const float* __restrict__ weight,
+__global__ __launch_bounds__(256) void rmsnorm_quant_kernel(const void* __restrict__ x, int x_f32, const float* __restrict__ weight,
                                                            float eps, int D, bf16x8* __restrict__ normed,
                                                            uint2* __restrict__ xq, float* __restrict__ sx,
                                                            float* __restrict__ sx_blocked) {
   __shared__ float wave_sum[4];
   const int row = blockIdx.x, P = D / 8, t = threadIdx.x;
-  const bf16x8* xr = x + (size_t)row * P;
   float f[kNormPieces][8];
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < kNormPieces; ++i) {
     const int p = t + 256 * i;
     bf16x8 in = {};
-    if (p < P) in = xr[p];
+    if (p < P) in = load_bf16x8(x, x_f32, (size_t)row * P + p);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       f[i][j] = bf16_to_f32(in.v[j]);
@@ -113,21 +112,22 @@ __global__ __launch_bounds__(256) void quant_weight_kernel(const T* __restrict__
 }  // namespace
 
 extern "C" int moe_quant_act(const void* x_bf16, int R, int K, uint8_t* xq, float* sx, moe_stream_t stream) {
-  return moe_quant_act_impl(x_bf16, R, K, xq, sx, nullptr, stream);
+  return moe_quant_act_impl(x_bf16, 0, nullptr, R, K, xq, sx, nullptr, stream);
 }
 // checks the arguments of an activation quantisation and describes it (for its own launch, or a routing launch's)
-int moe_quant_act_job(const void* x_bf16, int R, int K, uint8_t* xq, float* sx, float* sx_blocked, QuantJob* job) {
-  MOE_REQUIRE(R == 0 || (x_bf16 && xq && sx), MOE_ERR_NULL, "quant_act: null pointer");
+int moe_quant_act_job(const void* x, int x_f32, void* x_bf16, int R, int K, uint8_t* xq, float* sx, float* sx_blocked, QuantJob* job) {
+  MOE_REQUIRE(R == 0 || (x && xq && sx), MOE_ERR_NULL, "quant_act: null pointer");
   MOE_REQUIRE(R >= 0 && K > 0 && K % MOE_QBLOCK == 0, MOE_ERR_BAD_SHAPE, "quant_act: K=%d must be a positive multiple of 128 (R=%d)", K, R);
-  MOE_REQUIRE(MOE_ALIGNED16(x_bf16) && MOE_ALIGNED16(xq), MOE_ERR_BAD_ALIGN, "quant_act: pointers must be 16-byte aligned");
+  MOE_REQUIRE(MOE_ALIGNED16(x) && MOE_ALIGNED16(xq), MOE_ERR_BAD_ALIGN, "quant_act: pointers must be 16-byte aligned");
   const long long pieces = (long long)R * K / 8;
   MOE_REQUIRE(pieces < (1ll << 38), MOE_ERR_BAD_SHAPE, "quant_act: too many elements");
-  *job = QuantJob{x_bf16, pieces, K / 128, R, xq, sx, sx_blocked};
+  *job = QuantJob{x, x_f32, x_bf16, pieces, K / 128, R, xq, sx, sx_blocked};
   return MOE_OK;
 }
-int moe_quant_act_impl(const void* x_bf16, int R, int K, uint8_t* xq, float* sx, float* sx_blocked, moe_stream_t stream) {
+int moe_quant_act_impl(const void* x, int x_f32, void* x_bf16, int R, int K, uint8_t* xq, float* sx, float* sx_blocked,
+                       moe_stream_t stream) {
   QuantJob job;
-  if (int rc = moe_quant_act_job(x_bf16, R, K, xq, sx, sx_blocked, &job)) return rc;
+  if (int rc = moe_quant_act_job(x, x_f32, x_bf16, R, K, xq, sx, sx_blocked, &job)) return rc;
   if (R == 0) return MOE_OK;
   hipLaunchKernelGGL(quant_act_kernel, dim3(moe_quant_blocks(job, 256)), dim3(256), 0, (hipStream_t)stream, job);
   return moe_check_hip(hipGetLastError(), "quant_act launch");
@@ -135,18 +135,18 @@ int moe_quant_act_impl(const void* x_bf16, int R, int K, uint8_t* xq, float* sx,
 
 extern "C" int moe_rmsnorm_quant(const void* x_bf16, const float* weight, float eps, int M, int D, void* normed_bf16,
                                  uint8_t* xq, float* sx, moe_stream_t stream) {
-  return moe_rmsnorm_quant_impl(x_bf16, weight, eps, M, D, normed_bf16, xq, sx, nullptr, stream);
+  return moe_rmsnorm_quant_impl(x_bf16, 0, weight, eps, M, D, normed_bf16, xq, sx, nullptr, stream);
 }
-int moe_rmsnorm_quant_impl(const void* x_bf16, const float* weight, float eps, int M, int D, void* normed_bf16,
+int moe_rmsnorm_quant_impl(const void* x, int x_f32, const float* weight, float eps, int M, int D, void* normed_bf16,
                            uint8_t* xq, float* sx, float* sx_blocked, moe_stream_t stream) {
-  MOE_REQUIRE((M == 0 || (x_bf16 && xq && sx)) && weight, MOE_ERR_NULL, "rmsnorm_quant: null pointer");
+  MOE_REQUIRE((M == 0 || (x && xq && sx)) && weight, MOE_ERR_NULL, "rmsnorm_quant: null pointer");
   MOE_REQUIRE(M >= 0 && D > 0 && D % MOE_QBLOCK == 0 && D <= 256 * 8 * kNormPieces, MOE_ERR_BAD_SHAPE,
               "rmsnorm_quant: D=%d must be a multiple of 128, at most %d (M=%d)", D, 256 * 8 * kNormPieces, M);
-  MOE_REQUIRE(MOE_ALIGNED16(x_bf16) && MOE_ALIGNED16(xq) && MOE_ALIGNED16(normed_bf16), MOE_ERR_BAD_ALIGN,
+  MOE_REQUIRE(MOE_ALIGNED16(x) && MOE_ALIGNED16(xq) && MOE_ALIGNED16(normed_bf16), MOE_ERR_BAD_ALIGN,
               "rmsnorm_quant: pointers must be 16-byte aligned");
   if (M == 0) return MOE_OK;
-  hipLaunchKernelGGL(rmsnorm_quant_kernel, dim3(M), dim3(256), 0, (hipStream_t)stream, (const bf16x8*)x_bf16, weight, eps,
-                     D, (bf16x8*)normed_bf16, (uint2*)xq, sx, sx_blocked);
+  hipLaunchKernelGGL(rmsnorm_quant_kernel, dim3(M), dim3(256), 0, (hipStream_t)stream, x, x_f32, weight, eps, D,
+                     (bf16x8*)normed_bf16, (uint2*)xq, sx, sx_blocked);
   return moe_check_hip(hipGetLastError(), "rmsnorm_quant launch");
 }
 

@@ -6,14 +6,13 @@
 #pragma once
 #include "moe_common.h"
 
-struct alignas(16) moe_bf16x8 { bf16_t v[8]; };
-
 // 16 lanes per 128-wide group, 8 bf16 (16 B) per lane; `block` = index of the block of blockDim.x pieces
 __device__ __forceinline__ void moe_quant_act_block(const QuantJob& q, long long block) {
   const long long p = block * blockDim.x + threadIdx.x;
   const bool ok = p < q.n_pieces;
   moe_bf16x8 in = {};
-  if (ok) in = ((const moe_bf16x8*)q.x)[p];
+  if (ok) in = load_bf16x8(q.x, q.x_f32, p);
+  if (ok && q.x_bf16) ((moe_bf16x8*)q.x_bf16)[p] = in;
   float f[8], amax = 0.f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {

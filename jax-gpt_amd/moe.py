@@ -444,7 +444,14 @@ def moe_experts(x, router_logits, *, top_k, experts, routing="softmax", bias=Non
     Returns (M, D) bf16, plus, if return_debug, a dict of the integer intermediates and of the quantised
     SwiGLU output the down GEMMs consumed (`hq` (R, I) e4m3 codes as uint8 and `sh` (R, I/128), sorted order;
     `hsq` (M, SI) and `shs` for the shared expert) and of the down GEMMs' rows (`y` (R, D), `ys` (M, D))."""
-    x = _dev(x, torch.bfloat16, "x")
+    return _forward(x, router_logits, top_k, experts, routing, bias, n_group, topk_group, renorm, routed_scale, shared,
+                    return_debug, gate_weight, shared_expert_gate_weight, norm_weight, norm_eps, add_residual)
+
+
+def _forward(x, router_logits, top_k, experts, routing, bias, n_group, topk_group, renorm, routed_scale, shared, return_debug,
+             gate_weight, shared_expert_gate_weight, norm_weight, norm_eps, add_residual, io_f32=False):
+    """`moe_experts`, with x and the output in f32 if io_f32 (x is rounded to bf16, the output holds bf16 values)."""
+    x = _dev(x, torch.float32 if io_f32 else torch.bfloat16, "x")
     wr = wsg = None
     if gate_weight is not None:
         if router_logits is not None:
@@ -510,7 +517,7 @@ def moe_experts(x, router_logits, *, top_k, experts, routing="softmax", bias=Non
         a.ws_gate, a.ws_up, a.ws_down = swg.data_ptr(), swu.data_ptr(), swd.data_ptr()
         a.sws_gate, a.sws_up, a.sws_down = ssg.data_ptr(), ssu.data_ptr(), ssd.data_ptr()
     a.SI = SI
-    out = _empty((M, D), torch.bfloat16, x)
+    out = _empty((M, D), x.dtype, x)
     a.out = out.data_ptr()
     dbg = None
     if return_debug:
@@ -538,7 +545,7 @@ def moe_experts(x, router_logits, *, top_k, experts, routing="softmax", bias=Non
         a.out_sorted_token_ids, a.out_inv_perm = dbg["sorted_token_ids"].data_ptr(), dbg["inv_perm"].data_ptr()
     nbytes = lib().moe_forward_workspace_bytes(M, D, E, top_k, I, SI)
     ws = _empty((max(nbytes, 16),), torch.uint8, x)
-    check(lib().moe_forward(C.byref(a), _ptr(ws), nbytes, _stream()))
+    check((lib().moe_forward_f32 if io_f32 else lib().moe_forward)(C.byref(a), _ptr(ws), nbytes, _stream()))
     del keep
     return (out, dbg) if return_debug else out
 
@@ -566,18 +573,14 @@ def moe_layer(x, params, n_experts_per_token, n_devices=1, axis_name="tp", mesh=
     x_flat = x.reshape(B * T, D)
     if x_flat.dtype not in (torch.bfloat16, torch.float32):
         raise TypeError(f"x: expected bf16 or f32 activations, got {x.dtype}")
-    if x_flat.dtype == torch.float32:               # the path computes from bf16 activations
-        x_flat = convert(_dev(x_flat, torch.float32, "x"), torch.bfloat16)
     shared = None
     if params.get("shared_gate_proj") is not None:
         shared = dict(gate_proj=params["shared_gate_proj"], up_proj=params["shared_up_proj"],
                       down_proj=params["shared_down_proj"])
-    out = moe_experts(x_flat, None, top_k=n_experts_per_token,
-                      experts=dict(gate_proj=params["gate_proj"], up_proj=params["up_proj"],
-                                   down_proj=params["down_proj"]),
-                      routing="softmax", shared=shared, gate_weight=params["gate_weight"],
-                      shared_expert_gate_weight=params.get("shared_expert_gate_weight") if shared is not None else None,
-                      norm_weight=_norm_weight, norm_eps=_norm_eps, add_residual=_add_residual)
-    if x.dtype == torch.float32:                    # moe.py:282: back to the caller's dtype
-        out = convert(out, torch.float32)
+    # f32 activations: the path computes from their bf16 rounding and returns the caller's dtype (moe.py:282)
+    out = _forward(x_flat, None, n_experts_per_token,
+                   dict(gate_proj=params["gate_proj"], up_proj=params["up_proj"], down_proj=params["down_proj"]),
+                   "softmax", None, 1, 1, True, 1.0, shared, False, params["gate_weight"],
+                   params.get("shared_expert_gate_weight") if shared is not None else None,
+                   _norm_weight, _norm_eps, _add_residual, io_f32=x_flat.dtype == torch.float32)
     return out.reshape(B, T, D)
