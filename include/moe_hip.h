@@ -154,6 +154,11 @@ MOE_API int moe_router_logits(const void* x_bf16, int M, int D, const void* w_ro
                       const void* w_shared_gate_bf16, float* logits, float* shared_gate, void* ws,
                       size_t ws_bytes, moe_stream_t stream);
 
+/* moe.py:37-55 whole (moe_routing): the router's matmul and the softmax selection, without the logits in between.
+ * ws: moe_router_workspace_bytes(M, D, E). */
+MOE_API int moe_routing(const void* x_bf16, int M, int D, const void* w_router_bf16, int E, int k, int renorm, int32_t* idx,
+                float* w, void* ws, size_t ws_bytes, moe_stream_t stream);
+
 /* primitives.py:16-32 (rms_norm, Qwen3.5 convention: x / sqrt(mean(x^2) + eps) * (1 + weight), result in
  * bf16) as called in front of the MoE layer (block.py:54, :88), fused with the 1x128 quantisation of the
  * normalised row.  weight (D) f32; normed_bf16 (M, D) may be NULL when only the fp8 form is needed.
@@ -220,6 +225,10 @@ MOE_API int moe_forward(const MoeForwardArgs* args, void* ws, size_t ws_bytes, m
 /* The same for a caller whose activations are f32 (moe.py:282): args->x and args->out are (M, D) f32; x is rounded to
  * bf16 on the way in and out holds the bf16 results, as if moe_convert stood on either side. */
 MOE_API int moe_forward_f32(const MoeForwardArgs* args, void* ws, size_t ws_bytes, moe_stream_t stream);
+/* moe.py:97-114 (expert_forward_single): the same path behind a selection that the caller has made, idx (M, k) int32
+ * and w (M, k) f32.  args->logits, w_router, bias and the routing fields are not read; out_idx and out_w stay unwritten. */
+MOE_API int moe_forward_selected(const MoeForwardArgs* args, const int32_t* idx, const float* w, void* ws, size_t ws_bytes,
+                         moe_stream_t stream);
 
 #ifdef __cplusplus
 }

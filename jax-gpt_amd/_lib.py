@@ -67,12 +67,16 @@ SIGNATURES = {
     "moe_forward_workspace_bytes": (_Z, [_I, _I, _I, _I, _I, _I]),
     "moe_forward": (_I, [C.POINTER(MoeForwardArgs), _P, _Z, _P]),
     "moe_forward_f32": (_I, [C.POINTER(MoeForwardArgs), _P, _Z, _P]),
+    "moe_forward_selected": (_I, [C.POINTER(MoeForwardArgs), _P, _P, _P, _Z, _P]),
+    "moe_routing": (_I, [_P, _I, _I, _P, _I, _I, _I, _P, _P, _P, _Z, _P]),
 }
 
 
 def lib():
     """Load libmoe_hip.so.  Raises if it has not been built: there is no fallback."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib

@@ -153,13 +153,14 @@ extern "C" size_t moe_forward_workspace_bytes(int M, int D, int E, int k, int I,
   return carve(nullptr, M, D, E, k, I, SI, true).total;   // room for the router whether or not a call uses it
 }
 
-static int forward(const MoeForwardArgs* a, int io_f32, void* ws, size_t ws_bytes, moe_stream_t stream) {
+// given_idx / given_w: a selection that the caller has made (no routing), or null
+static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx, const float* given_w, void* ws, size_t ws_bytes, moe_stream_t stream) {
   MOE_REQUIRE(a && ws, MOE_ERR_NULL, "forward: null args or workspace");
   MOE_REQUIRE(a->M >= 0 && a->D > 0 && a->E >= 1 && a->k >= 1 && a->I > 0 && a->SI >= 0, MOE_ERR_BAD_SHAPE,
               "forward: bad dims M=%d D=%d E=%d k=%d I=%d SI=%d", a->M, a->D, a->E, a->k, a->I, a->SI);
   MOE_REQUIRE(a->D % 128 == 0 && a->I % 128 == 0 && a->SI % 128 == 0, MOE_ERR_BAD_SHAPE,
               "forward: D=%d, I=%d and SI=%d must be multiples of 128", a->D, a->I, a->SI);
-  MOE_REQUIRE((a->M == 0 || (a->x && (a->logits || a->w_router) && a->out)) && a->w_gate && a->w_up && a->w_down && a->sw_gate && a->sw_up && a->sw_down,
+  MOE_REQUIRE((a->M == 0 || (a->x && (a->logits || a->w_router || given_idx) && a->out)) && a->w_gate && a->w_up && a->w_down && a->sw_gate && a->sw_up && a->sw_down,
               MOE_ERR_NULL, "forward: null tensor pointer");
   if (a->SI)
     MOE_REQUIRE(a->ws_gate && a->ws_up && a->ws_down && a->sws_gate && a->sws_up && a->sws_down, MOE_ERR_NULL,
@@ -175,7 +176,8 @@ static int forward(const MoeForwardArgs* a, int io_f32, void* ws, size_t ws_byte
   MOE_REQUIRE(a->w_shared_gate || !a->out_shared_gate, MOE_ERR_NULL, "forward: out_shared_gate needs w_shared_gate");
   ForwardBuffers b = carve(ws, a->M, a->D, a->E, a->k, a->I, a->SI, true);
   int32_t* idx = a->out_idx ? a->out_idx : b.idx;
-  float* w = a->out_w ? a->out_w : b.w;
+  float* w_own = a->out_w ? a->out_w : b.w;
+  const float* w = given_idx ? given_w : w_own;
   int32_t* gsz = a->out_group_sizes ? a->out_group_sizes : b.group_sizes;
   int32_t* stid = a->out_sorted_token_ids ? a->out_sorted_token_ids : b.sorted_token_ids;
   int32_t* inv = a->out_inv_perm ? a->out_inv_perm : b.inv_perm;
@@ -198,7 +200,7 @@ static int forward(const MoeForwardArgs* a, int io_f32, void* ws, size_t ws_byte
   // few scale lines either way and is spared the extra launch
   const bool blocked_scales = R > 2048;
   hipStream_t main_s = (hipStream_t)stream;
-  MOE_REQUIRE(a->routing == MOE_ROUTING_SOFTMAX || a->routing == MOE_ROUTING_SIGMOID_GROUPED, MOE_ERR_BAD_SHAPE,
+  MOE_REQUIRE(given_idx || a->routing == MOE_ROUTING_SOFTMAX || a->routing == MOE_ROUTING_SIGMOID_GROUPED, MOE_ERR_BAD_SHAPE,
               "forward: unknown routing %d", a->routing);
   int rc;
 
@@ -265,7 +267,7 @@ static int forward(const MoeForwardArgs* a, int io_f32, void* ws, size_t ws_byte
   // are written only when out_logits asks for them.
   LogitSource src{a->logits, nullptr, 0, a->E, nullptr, nullptr};
   const float* shared_gate = nullptr;
-  if (a->w_router) {
+  if (a->w_router && !given_idx) {
     const bool from_quantiser = quantiser_feeds_router(a, io_f32);
     if (from_quantiser && !quant_joined) {   // (the quantiser was forked)
       if (rc_shared) return join(rc_shared);
@@ -283,10 +285,12 @@ static int forward(const MoeForwardArgs* a, int io_f32, void* ws, size_t ws_byte
   // routing, the sort by expert and the routed GEMMs' work list (the sort holds every expert's row range anyway)
   TileList tiles;
   if ((rc = moe_gemm_tile_list(R, a->E, b.gemm_ws, b.gemm_ws_bytes, &tiles))) return join(rc);
-  const RouteArgs route{src, a->bias, a->M, a->E, a->k, a->renorm, a->n_group, a->topk_group, a->routed_scale, idx, w};
+  const RouteArgs route{src, a->bias, a->M, a->E, a->k, a->renorm, a->n_group, a->topk_group, a->routed_scale, idx, w_own};
   const PermuteOut sort{gsz, b.group_offsets, stid, nullptr, inv, a->k, tiles};
-  if ((rc = moe_route_impl(a->routing, route, quant_in_route ? &quant_job : nullptr, &sort, b.permute_ws, b.permute_ws_bytes, stream)))
-    return join(rc);
+  const QuantJob* carried = quant_in_route ? &quant_job : nullptr;
+  rc = given_idx ? moe_permute_impl(given_idx, a->M, a->k, a->E, sort, b.permute_ws, b.permute_ws_bytes, carried, stream)
+                 : moe_route_impl(a->routing, route, carried, &sort, b.permute_ws, b.permute_ws_bytes, stream);
+  if (rc) return join(rc);
   if (!quant_joined) {
     if (rc_shared) return join(rc_shared);
     if ((rc = moe_check_hip(hipStreamWaitEvent(main_s, ev->quant, 0), "forward: quant join"))) return join(rc);
@@ -313,8 +317,14 @@ static int forward(const MoeForwardArgs* a, int io_f32, void* ws, size_t ws_byte
 }
 
 extern "C" int moe_forward(const MoeForwardArgs* a, void* ws, size_t ws_bytes, moe_stream_t stream) {
-  return forward(a, 0, ws, ws_bytes, stream);
+  return forward(a, 0, nullptr, nullptr, ws, ws_bytes, stream);
 }
 extern "C" int moe_forward_f32(const MoeForwardArgs* a, void* ws, size_t ws_bytes, moe_stream_t stream) {
-  return forward(a, 1, ws, ws_bytes, stream);
+  return forward(a, 1, nullptr, nullptr, ws, ws_bytes, stream);
+}
+extern "C" int moe_forward_selected(const MoeForwardArgs* a, const int32_t* idx, const float* w, void* ws, size_t ws_bytes,
+                                    moe_stream_t stream) {
+  MOE_REQUIRE(a && (a->M == 0 || (idx && w)), MOE_ERR_NULL, "forward: null selection");
+  MOE_REQUIRE(!a->w_router && !a->w_shared_gate, MOE_ERR_NULL, "forward: a selection that is given leaves the router nothing to do");
+  return forward(a, 0, idx, w, ws, ws_bytes, stream);
 }

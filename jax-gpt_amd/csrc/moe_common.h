@@ -274,9 +274,9 @@ int moe_route_impl(int routing, const RouteArgs& a, const QuantJob* quant, const
                    size_t permute_ws_bytes, moe_stream_t stream);
 // chunks of the flat list that get a histogram each, at most
 int moe_permute_max_chunks(int E);
-// the sort's second launch: chunk_hist [n_chunks][E] (null when n_chunks == 1)
+// the sort's second launch: chunk_hist [n_chunks][E]; or, n_chunks == 1 and chunk_hist null, all of it (quant: carried along)
 int moe_permute_place(const int32_t* idx, int R, int E, int chunk, int n_chunks, const int32_t* chunk_hist, const PermuteOut& o,
-                      moe_stream_t stream);
+                      const QuantJob* quant, moe_stream_t stream);
 // grouped GEMMs with an optional pre-built tile list in ws (moe_gemm.hip); the extern "C" entry points build their
 // own.  moe_gemm_tile_list describes the list the GEMMs of (R rows, E experts) expect in ws, so that the permutation
 // kernels, which hold every expert's row range anyway, can write it (moe_permute_impl) and no launch is spent on it.
@@ -291,7 +291,9 @@ int moe_rmsnorm_quant_impl(const void* x, int x_f32, const float* weight, float 
 // the combine with the residual and the output in bf16 or (io_f32) f32, the output rounded to bf16 either way
 int moe_combine_impl(const void* y_bf16, const float* w, const int32_t* inv_perm, const void* shared_bf16, const float* shared_gate,
                      const void* residual, int io_f32, int M, int k, int D, void* out, moe_stream_t stream);
-int moe_permute_impl(const int32_t* idx, int M, int k, int E, const PermuteOut& o, void* ws, size_t ws_bytes, moe_stream_t stream);
+// the whole sort; its first launch carries the quantisation, if any
+int moe_permute_impl(const int32_t* idx, int M, int k, int E, const PermuteOut& o, void* ws, size_t ws_bytes, const QuantJob* quant,
+                     moe_stream_t stream);
 // Where the grouped GEMMs find an activation scale and put an h scale, in floats: scale of (row, 128-wide K block kb)
 // = s[row * in_row + kb * in_kb].  The public entry points use the row-major arrays of the quantisers ({K/128, 1});
 // moe_forward hands large batches block-major arrays in row-list order ({1, R}, in_listed = true: indexed by the

@@ -13,13 +13,18 @@
 // (chunks x E counts per workgroup, at most 256 KB from L2) cheaper than a third launch that would scan them once.
 #include "moe_common.h"
 #include "moe_permute_device.h"
+#include "moe_quant_device.h"
 
 namespace {
 
 constexpr int kHistThreads = 256;
 
 __global__ __launch_bounds__(kHistThreads) void hist_kernel(const int32_t* __restrict__ ids, int R, int E, int chunk,
-                                                           int32_t* __restrict__ chunk_hist) {
+                                                           int n_chunks, int32_t* __restrict__ chunk_hist, const QuantJob quant) {
+  if ((int)blockIdx.x >= n_chunks) {   // the blocks behind quantise the activations (QuantJob)
+    moe_quant_act_block(quant, (int)blockIdx.x - n_chunks);
+    return;
+  }
   extern __shared__ int hist[];  // E
   for (int e = threadIdx.x; e < E; e += kHistThreads) hist[e] = 0;
   __syncthreads();
@@ -34,9 +39,13 @@ __global__ __launch_bounds__(kHistThreads) void hist_kernel(const int32_t* __res
 
 __global__ __launch_bounds__(kPlaceThreads) void place_kernel(const int32_t* __restrict__ ids, int R, int E, int chunk,
                                                              int n_chunks, const int32_t* __restrict__ chunk_hist,
-                                                             const PermuteOut o) {
+                                                             const PermuteOut o, const QuantJob quant) {
   extern __shared__ int smem[];   // [waves][E]
   if (n_chunks == 1) {
+    if (blockIdx.x > 0) {   // the blocks behind quantise the activations (QuantJob)
+      moe_quant_act_block(quant, (int)blockIdx.x - 1);
+      return;
+    }
     permute_one_chunk(ids, R, E, smem, o);
     return;
   }
@@ -108,10 +117,11 @@ extern "C" size_t moe_permute_workspace_bytes(int M, int k, int E) {
 }
 
 int moe_permute_place(const int32_t* idx, int R, int E, int chunk, int n_chunks, const int32_t* chunk_hist, const PermuteOut& o,
-                      moe_stream_t stream) {
+                      const QuantJob* quant, moe_stream_t stream) {
   const bool places = R > 0 && (o.sorted_token_ids || o.sort_order || o.inv_perm);
-  hipLaunchKernelGGL(place_kernel, dim3(n_chunks == 1 || !places ? 1 : n_chunks + 1), dim3(kPlaceThreads),
-                     moe_place_lds_ints(E) * sizeof(int), (hipStream_t)stream, idx, R, E, chunk, n_chunks, chunk_hist, o);
+  const unsigned blocks = n_chunks > 1 ? (places ? n_chunks + 1 : 1) : 1 + (quant ? moe_quant_blocks(*quant, kPlaceThreads) : 0);
+  hipLaunchKernelGGL(place_kernel, dim3(blocks), dim3(kPlaceThreads), moe_place_lds_ints(E) * sizeof(int), (hipStream_t)stream,
+                     idx, R, E, chunk, n_chunks, chunk_hist, o, quant ? *quant : QuantJob{});
   return moe_check_hip(hipGetLastError(), "permute launch");
 }
 
@@ -119,10 +129,11 @@ extern "C" int moe_permute(const int32_t* idx, int M, int k, int E, int32_t* gro
                            int32_t* group_offsets, int32_t* sorted_token_ids, int32_t* sort_order,
                            int32_t* inv_perm, void* ws, size_t ws_bytes, moe_stream_t stream) {
   return moe_permute_impl(idx, M, k, E, PermuteOut{group_sizes, group_offsets, sorted_token_ids, sort_order, inv_perm, k,
-                                                   TileList{0, nullptr, nullptr}}, ws, ws_bytes, stream);
+                                                   TileList{0, nullptr, nullptr}}, ws, ws_bytes, nullptr, stream);
 }
 
-int moe_permute_impl(const int32_t* idx, int M, int k, int E, const PermuteOut& o, void* ws, size_t ws_bytes, moe_stream_t stream) {
+int moe_permute_impl(const int32_t* idx, int M, int k, int E, const PermuteOut& o, void* ws, size_t ws_bytes, const QuantJob* quant,
+                     moe_stream_t stream) {
   MOE_REQUIRE((idx || M == 0) && o.group_sizes && o.group_offsets && ws, MOE_ERR_NULL, "permute: null pointer");
   MOE_REQUIRE(M >= 0 && k >= 1 && E >= 1 && E <= kMaxE, MOE_ERR_BAD_SHAPE,
               "permute: need k >= 1 and 1 <= E <= %d, got M=%d k=%d E=%d", kMaxE, M, k, E);
@@ -130,12 +141,12 @@ int moe_permute_impl(const int32_t* idx, int M, int k, int E, const PermuteOut& 
   MOE_REQUIRE(ws_bytes >= moe_permute_workspace_bytes(M, k, E), MOE_ERR_WORKSPACE_TOO_SMALL,
               "permute: workspace %zu < %zu", ws_bytes, moe_permute_workspace_bytes(M, k, E));
   const int R = M * k;
-  if (R <= kSmallRows) return moe_permute_place(idx, R, E, kSmallRows, 1, nullptr, o, stream);
+  if (R <= kSmallRows) return moe_permute_place(idx, R, E, kSmallRows, 1, nullptr, o, quant, stream);
   const int max_chunks = moe_permute_max_chunks(E);
   int chunk = (int)(((long long)R + max_chunks - 1) / max_chunks);
   chunk = chunk < 256 ? 256 : chunk;
   const int n_chunks = (int)(((long long)R + chunk - 1) / chunk);
-  hipLaunchKernelGGL(hist_kernel, dim3(n_chunks), dim3(kHistThreads), E * sizeof(int), (hipStream_t)stream, idx, R, E, chunk,
-                     (int32_t*)ws);
-  return moe_permute_place(idx, R, E, chunk, n_chunks, (const int32_t*)ws, o, stream);
+  hipLaunchKernelGGL(hist_kernel, dim3(n_chunks + (quant ? moe_quant_blocks(*quant, kHistThreads) : 0)), dim3(kHistThreads),
+                     E * sizeof(int), (hipStream_t)stream, idx, R, E, chunk, n_chunks, (int32_t*)ws, quant ? *quant : QuantJob{});
+  return moe_permute_place(idx, R, E, chunk, n_chunks, (const int32_t*)ws, o, nullptr, stream);
 }

@@ -387,8 +387,8 @@ int moe_route_impl(int routing, const RouteArgs& a, const QuantJob* quant, const
   launch(vpl, grid, block, lds, s, a, job, q, o);
   if (int rc = moe_check_hip(hipGetLastError(), "route launch")) return rc;
   if (!sort || sort_here) return MOE_OK;
-  if (one_chunk) return moe_permute_place(a.idx, R, a.E, kSmallRows, 1, nullptr, o, stream);
-  return moe_permute_place(a.idx, R, a.E, tpb * a.k, job.blocks, job.chunk_hist, o, stream);
+  if (one_chunk) return moe_permute_place(a.idx, R, a.E, kSmallRows, 1, nullptr, o, nullptr, stream);
+  return moe_permute_place(a.idx, R, a.E, tpb * a.k, job.blocks, job.chunk_hist, o, nullptr, stream);
 }
 
 extern "C" int moe_route_softmax_topk(const float* logits, int M, int E, int k, int renorm,
@@ -404,4 +404,12 @@ extern "C" int moe_route_sigmoid_grouped(const float* logits, const float* bias,
   const RouteArgs a{LogitSource{logits, nullptr, 0, E, nullptr, nullptr}, bias, M, E, k, renorm, n_group, topk_group,
                     routed_scale, idx, w};
   return moe_route_impl(MOE_ROUTING_SIGMOID_GROUPED, a, nullptr, nullptr, nullptr, 0, stream);
+}
+
+extern "C" int moe_routing(const void* x_bf16, int M, int D, const void* w_router_bf16, int E, int k, int renorm, int32_t* idx,
+                           float* w, void* ws, size_t ws_bytes, moe_stream_t stream) {
+  int splits = 0, n_cols = 0;
+  if (int rc = moe_router_partials(x_bf16, M, D, w_router_bf16, E, nullptr, ws, ws_bytes, &splits, &n_cols, stream)) return rc;
+  const RouteArgs a{LogitSource{nullptr, (const float*)ws, splits, n_cols, nullptr, nullptr}, nullptr, M, E, k, renorm, 1, 1, 1.f, idx, w};
+  return moe_route_impl(MOE_ROUTING_SOFTMAX, a, nullptr, nullptr, nullptr, 0, stream);
 }

@@ -34,15 +34,21 @@ ROUTING = {"softmax": 0, "sigmoid_grouped": 1}
 # plumbing
 # ----------------------------------------------------------------------------
 
+# A decode-sized call is bound by the host work in front of its launches, so this layer stays short: pointers travel as
+# plain integers, the stream comes from torch's C binding (a torch.cuda.Stream object costs 3 us), and the tensors that
+# callers normally hand in (on the GPU, of the right type, contiguous) pass one test each.
+
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t):
-    return C.c_void_p(0) if t is None else C.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _dev(t, dtype=None, name="tensor"):
+    if isinstance(t, torch.Tensor) and t.is_cuda and (dtype is None or t.dtype == dtype) and t.is_contiguous():
+        return t
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name}: expected a torch.Tensor, got {type(t).__name__}")
     if not t.is_cuda:
@@ -196,7 +202,7 @@ def _cached(src, tag, build):
     and dropped when the source tensor is garbage-collected or has been modified in place."""
     key = (tag, id(src))
     hit = _derived.get(key)
-    if hit is not None and hit[0]() is src and hit[1] == src._version:
+    if hit is not None and hit[1] == src._version and hit[0]() is src:
         return hit[2]
     val = build()
     if hit is None or hit[0]() is not src:
@@ -225,9 +231,14 @@ def _expert_weight(w, name, dense=False):
     """Accept a block-fp8 dict; a per-row fp8 dict of the reference (re-quantised per block once, cached); or a plain
     (E, in, out) array as the reference stores unquantised experts (model.py:98-101), transposed and quantised
     once.  `dense`: a 2-D layer of the shared expert, (in, out) plain or (out, in) fp8 (fp8.py:123-143).
-    Returns (codes (E, N, K) uint8, scale_inv (E, N/128, K/128) f32)."""
+    Returns (codes (E, N, K) bytes, scale_inv (E, N/128, K/128) f32)."""
     if isinstance(w, dict) and "w" in w:
         q, s = w["w"], w["scale_inv"]
+        if (q.dtype == torch.float8_e4m3fn and s.dtype == torch.float32 and q.is_cuda and s.is_cuda and q.dim() == 3
+                and q.is_contiguous() and s.is_contiguous()):
+            E, N, K = q.shape
+            if s.shape == (E, N // 128, K // 128):
+                return q, s
         if _per_row_scales(q, s):
             return _cached(q, ("per_row", dense, id(s), s._version), lambda: _requantise_per_row(q, s, dense))
         if q.dim() == 2:
@@ -358,14 +369,11 @@ def combine(y, weights, inv_perm, shared=None, shared_gate=None, residual=None):
 
 def expert_forward_single(x, expert_indices, expert_weights, gate_proj, up_proj, down_proj):
     """moe.py:97-114: sort/group, grouped SwiGLU, weighted scatter back.  x (M, D) bf16."""
-    x = _dev(x, torch.bfloat16, "x")
-    wg, _ = _expert_weight(gate_proj, "gate_proj")
-    E = wg.shape[0]
-    sg = permute(expert_indices, E)
-    xq, sx = quant_act(x)
-    hq, sh = gemm_gateup_swiglu(xq, sx, gate_proj, up_proj, sg["group_offsets"], row_ids=sg["sorted_token_ids"])
-    y = gemm_down(hq, sh, down_proj, sg["group_offsets"])
-    return combine(y, expert_weights, sg["inv_perm"])
+    idx = _dev(expert_indices, torch.int32, "expert_indices")
+    w = _dev(expert_weights, torch.float32, "expert_weights")
+    if idx.dim() != 2 or w.shape != idx.shape or idx.shape[0] != x.shape[0]:
+        raise ValueError(f"expert_indices {tuple(idx.shape)} and expert_weights {tuple(w.shape)} must both be ({x.shape[0]}, k)")
+    return _forward(x, None, idx.shape[1], dict(gate_proj=gate_proj, up_proj=up_proj, down_proj=down_proj), selected=(idx, w))
 
 
 def shared_expert_forward(x, gate_proj, up_proj, down_proj):
@@ -427,7 +435,18 @@ def router_logits(x, gate_weight, shared_expert_gate_weight=None):
 
 def moe_routing(x, gate_weight, n_experts_per_token):
     """moe.py:37-55: router matmul, f32 softmax, top-k, renormalise.  x (M, D) bf16, gate_weight (D, E)."""
-    return route_softmax_topk(router_logits(x, gate_weight), n_experts_per_token)
+    x = _dev(x, torch.bfloat16, "x")
+    wr = _router_weight(gate_weight, "gate_weight")
+    E, D = wr.shape
+    M, k = x.shape[0], n_experts_per_token
+    if x.shape[1] != D:
+        raise ValueError(f"gate_weight: expected ({x.shape[1]}, E), got a weight for hidden size {D}")
+    idx = _empty((M, k), torch.int32, x)
+    w = _empty((M, k), torch.float32, x)
+    nbytes = lib().moe_router_workspace_bytes(M, D, E)
+    ws = _empty((max(nbytes, 16),), torch.uint8, x)
+    check(lib().moe_routing(_ptr(x), M, D, _ptr(wr), E, k, 1, _ptr(idx), _ptr(w), _ptr(ws), nbytes, _stream()))
+    return idx, w
 
 
 def moe_experts(x, router_logits, *, top_k, experts, routing="softmax", bias=None, n_group=1, topk_group=1,
@@ -448,9 +467,11 @@ def moe_experts(x, router_logits, *, top_k, experts, routing="softmax", bias=Non
                     return_debug, gate_weight, shared_expert_gate_weight, norm_weight, norm_eps, add_residual)
 
 
-def _forward(x, router_logits, top_k, experts, routing, bias, n_group, topk_group, renorm, routed_scale, shared, return_debug,
-             gate_weight, shared_expert_gate_weight, norm_weight, norm_eps, add_residual, io_f32=False):
-    """`moe_experts`, with x and the output in f32 if io_f32 (x is rounded to bf16, the output holds bf16 values)."""
+def _forward(x, router_logits, top_k, experts, routing="softmax", bias=None, n_group=1, topk_group=1, renorm=True,
+             routed_scale=1.0, shared=None, return_debug=False, gate_weight=None, shared_expert_gate_weight=None,
+             norm_weight=None, norm_eps=1e-6, add_residual=False, io_f32=False, selected=None):
+    """`moe_experts`, with x and the output in f32 if io_f32 (x is rounded to bf16, the output holds bf16 values), and
+    with `selected` = (indices, weights) in place of the routing."""
     x = _dev(x, torch.float32 if io_f32 else torch.bfloat16, "x")
     wr = wsg = None
     if gate_weight is not None:
@@ -463,7 +484,7 @@ def _forward(x, router_logits, top_k, experts, routing, bias, n_group, topk_grou
     else:
         if shared_expert_gate_weight is not None:
             raise ValueError("shared_expert_gate_weight needs gate_weight (the router runs inside the call)")
-        logits = _dev(router_logits, torch.float32, "router_logits")
+        logits = None if selected else _dev(router_logits, torch.float32, "router_logits")
     if routing not in ROUTING:
         raise ValueError(f"routing must be one of {sorted(ROUTING)}, got {routing!r}")
     M, D = x.shape
@@ -486,7 +507,8 @@ def _forward(x, router_logits, top_k, experts, routing, bias, n_group, topk_grou
     a.routing, a.n_group, a.topk_group, a.renorm, a.routed_scale = ROUTING[routing], n_group, topk_group, int(renorm), routed_scale
     nw = None
     if norm_weight is not None:
-        nw = _dev(norm_weight.to(torch.float32), torch.float32, "norm_weight")
+        nw = norm_weight if norm_weight.dtype == torch.float32 else norm_weight.to(torch.float32)
+        nw = _dev(nw, torch.float32, "norm_weight")
         if tuple(nw.shape) != (D,):
             raise ValueError(f"norm_weight: expected ({D},), got {tuple(nw.shape)}")
         a.norm_weight, a.norm_eps = nw.data_ptr(), float(norm_eps)
@@ -543,9 +565,13 @@ def _forward(x, router_logits, top_k, experts, routing, bias, n_group, topk_grou
         a.out_idx, a.out_w = dbg["indices"].data_ptr(), dbg["weights"].data_ptr()
         a.out_group_sizes = dbg["group_sizes"].data_ptr()
         a.out_sorted_token_ids, a.out_inv_perm = dbg["sorted_token_ids"].data_ptr(), dbg["inv_perm"].data_ptr()
-    nbytes = lib().moe_forward_workspace_bytes(M, D, E, top_k, I, SI)
+    L = lib()
+    nbytes = L.moe_forward_workspace_bytes(M, D, E, top_k, I, SI)
     ws = _empty((max(nbytes, 16),), torch.uint8, x)
-    check((lib().moe_forward_f32 if io_f32 else lib().moe_forward)(C.byref(a), _ptr(ws), nbytes, _stream()))
+    if selected:
+        check(L.moe_forward_selected(C.byref(a), _ptr(selected[0]), _ptr(selected[1]), _ptr(ws), nbytes, _stream()))
+    else:
+        check((L.moe_forward_f32 if io_f32 else L.moe_forward)(C.byref(a), _ptr(ws), nbytes, _stream()))
     del keep
     return (out, dbg) if return_debug else out
 
@@ -580,7 +606,8 @@ def moe_layer(x, params, n_experts_per_token, n_devices=1, axis_name="tp", mesh=
     # f32 activations: the path computes from their bf16 rounding and returns the caller's dtype (moe.py:282)
     out = _forward(x_flat, None, n_experts_per_token,
                    dict(gate_proj=params["gate_proj"], up_proj=params["up_proj"], down_proj=params["down_proj"]),
-                   "softmax", None, 1, 1, True, 1.0, shared, False, params["gate_weight"],
-                   params.get("shared_expert_gate_weight") if shared is not None else None,
-                   _norm_weight, _norm_eps, _add_residual, io_f32=x_flat.dtype == torch.float32)
+                   shared=shared, gate_weight=params["gate_weight"],
+                   shared_expert_gate_weight=params.get("shared_expert_gate_weight") if shared is not None else None,
+                   norm_weight=_norm_weight, norm_eps=_norm_eps, add_residual=_add_residual,
+                   io_f32=x_flat.dtype == torch.float32)
     return out.reshape(B, T, D)
