@@ -437,6 +437,10 @@ __device__ __forceinline__ void dma16(const uint8_t* base, unsigned off, unsigne
   const unsigned m0v = __builtin_amdgcn_readfirstlane(lds_addr);
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0v), "v"(off), "s"(base) : "memory", "m0");
 }
+__device__ __forceinline__ void dma16_nt(const uint8_t* base, unsigned off, unsigned lds_addr) {   // for lines that are read once
+  const unsigned m0v = __builtin_amdgcn_readfirstlane(lds_addr);
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(m0v), "v"(off), "s"(base) : "memory", "m0");
+}
 __device__ __forceinline__ void dma4(const uint8_t* base, unsigned off, unsigned lds_addr) {
   const unsigned m0v = __builtin_amdgcn_readfirstlane(lds_addr);
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(m0v), "v"(off), "s"(base) : "memory", "m0");
