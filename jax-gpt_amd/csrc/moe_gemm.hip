@@ -119,7 +119,7 @@ __device__ __forceinline__ int swz(int row, int chunk) { return row * BK + ((chu
 // group j + 1 -- FMA quadruple f just before MFMA f, which overwrites p[f] -- so the matrix core works on the next
 // group while the vector ALU finishes the last one, with one set of result registers.  The last group of a step is
 // finished behind the next step's barrier, while that step's first fragments travel from LDS.
-template <int XF, int MODE = MODE_GATEUP> struct Cls {
+template <int XF, int MODE = MODE_GATEUP, bool ONCE = true> struct Cls {
   static constexpr int BM = 32 * XF, HALF = BM / 2;
   // Two rings: weight tiles (32 KB each) and activation tiles with their scales.  Where 160 KB allow it the weight
   // ring is one stage deeper than the activation ring (160 to 224 rows: three weight stages, two activation
@@ -141,11 +141,13 @@ template <int XF, int MODE = MODE_GATEUP> struct Cls {
   static constexpr bool W_EARLY = XF == 8 && MODE == MODE_GATEUP;
   static constexpr int EARLY_G = 3;   // the group behind which the weight copies of a W_EARLY step begin (2 and 4: within 1 %)
   static constexpr int X_PRE = X_NST - 1, W_PRE = W_NST - 1 + (W_EARLY ? 1 : 0);   // steps that a copy runs ahead of its use
-  // The weight copies' cache policy.  An expert of several row tiles has tiles of more than 96 rows (moe_tile_span), so
-  // a shorter one is its expert's only reader: its weight lines are fetched once and marked non-temporal, which leaves
-  // the memory-side cache alone.  A read-only stream reaches 7.1 TB/s that way and 6.3 without (4 GiB, any grid); 64
-  // tokens of the DeepSeek-V3 layer went from 1010 to 864 us, gate/up and down at 6.7 TB/s instead of 5.8.
-  static constexpr bool W_ONCE = XF <= 3;
+  // The weight copies' cache policy.  ONCE: the item's expert has one row tile (or two that stay close, see the
+  // dispatch), so that its weight lines are fetched once and marked non-temporal, which leaves the memory-side cache
+  // alone.  A read-only stream reaches 7.1 TB/s that way and 6.3 without (4 GiB, any grid); 64 tokens of the
+  // DeepSeek-V3 layer went from 1010 to 864 us, gate/up and down at 6.7 TB/s instead of 5.8.  An expert of several row
+  // tiles has tiles of more than 96 rows (moe_tile_span), so the shorter classes exist in this form only.
+  static constexpr bool W_ONCE = ONCE;
+  static_assert(ONCE || XF > 3, "an expert of several row tiles has none this short");
   static constexpr int X_STAGE_S_OFF = BM * BK;                // the scales behind the tile
   // + 256: every copying wave copies 64 scale slots from its first one on (no lane mask, which would cut the
   // unrolled K step into blocks); the surplus lanes rewrite other waves' slots with the same values or land in this pad
@@ -200,15 +202,15 @@ constexpr int CLS_FLAG_OFF = CLS_WSCALE_OFF + 2 * MAX_KB * 4;  // [4] early_flag
 constexpr int CLS_LDS_BYTES = CLS_FLAG_OFF + 16;              // 160016; the epilogues stage through the ring (<= 128 KB)
 static_assert(CLS_LDS_BYTES <= 160 * 1024, "LDS");
 
-struct Item { int expert, row_start, row_count, col_block; };
+struct Item { int expert, row_start, row_count, col_block, tiles; };
 
-template <int MODE, int XF>
+template <int MODE, int XF, bool ONCE>
 __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const uint8_t* __restrict__ xq,
                                           const float* __restrict__ sx, const int32_t* __restrict__ row_ids,
                                           const uint8_t* __restrict__ w0, const float* __restrict__ sw0,
                                           const uint8_t* __restrict__ w1, const float* __restrict__ sw1, int K, int N,
                                           void* __restrict__ out, float* __restrict__ out_scale, const GemmScales sc) {
-  using C = Cls<XF, MODE>;
+  using C = Cls<XF, MODE, ONCE>;
   constexpr int BM = C::BM, HALF = C::HALF;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -668,6 +670,7 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
     expert_item(local, nt, ncb, item.col_block, rt);
     moe_tile_span(dense_rows, nt, rt, t0, tn);
     item.expert = 0;
+    item.tiles = nt;
     item.row_start = t0;
     item.row_count = tn;
   } else {
@@ -695,6 +698,7 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
     expert_item(item_id - te.first_tile * ncb, nt, ncb, item.col_block, rt);
     moe_tile_span(te.rows, nt, rt, t0, tn);
     item.expert = te.expert;
+    item.tiles = nt;
     item.row_start = te.row_start + t0;
     item.row_count = tn;
   }
@@ -709,17 +713,24 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
   float* out_scale = is_dense ? dense.out_scale : routed.out_scale;
   const GemmScales sc = is_dense ? dense.sc : routed.sc;
   const int rows = __builtin_amdgcn_readfirstlane(item.row_count);
-#define MOE_ITEM(XF) item_body<MODE, XF>(item, lds, xq, sx, row_ids, w0, sw0, w1, sw1, K, N, out, out_scale, sc)
+  // Two row tiles of an expert read the same weight lines; over a short K they stay close enough to find them in L2
+  // (non-temporal lines leave it first), over a long one the later tile needs the memory-side cache.  Qwen3-MoE, 4096
+  // tokens (K = 2048, 768): 269 us with one-tile experts alone marked, 261 with two; DeepSeek-V3 gate/up (K = 7168) at
+  // 4096 tokens: 2426 / 2438 us of the step; all experts whatever their tiles: 8192 tokens 3731 / 3946 us.
+  const bool once = __builtin_amdgcn_readfirstlane(item.tiles) <= (K <= 2048 ? 2 : 1);
+#define MOE_ITEM(XF, ONCE) item_body<MODE, XF, ONCE>(item, lds, xq, sx, row_ids, w0, sw0, w1, sw1, K, N, out, out_scale, sc)
+#define MOE_CLASS(XF) if (once) MOE_ITEM(XF, true); else MOE_ITEM(XF, false); break
   switch ((rows + 31) >> 5) {
-    case 8: MOE_ITEM(8); break;
-    case 7: MOE_ITEM(7); break;
-    case 6: MOE_ITEM(6); break;
-    case 5: MOE_ITEM(5); break;
-    case 4: MOE_ITEM(4); break;
-    case 3: MOE_ITEM(3); break;
-    case 2: MOE_ITEM(2); break;
-    default: MOE_ITEM(1); break;
+    case 8: MOE_CLASS(8);
+    case 7: MOE_CLASS(7);
+    case 6: MOE_CLASS(6);
+    case 5: MOE_CLASS(5);
+    case 4: MOE_CLASS(4);
+    case 3: MOE_ITEM(3, true); break;
+    case 2: MOE_ITEM(2, true); break;
+    default: MOE_ITEM(1, true); break;
   }
+#undef MOE_CLASS
 #undef MOE_ITEM
 }
 int col_blocks(int mode, int N) { return mode == MODE_GATEUP ? N / 128 : (N + 255) / 256; }
