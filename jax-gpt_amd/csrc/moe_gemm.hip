@@ -577,7 +577,11 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
       const int r = ld_row + 64 * i;
       if (r < item.row_count) {
         v4i v = *(const v4i*)(tile + swz(r, ld_chunk));
-        *(v4i*)(hq + (size_t)(item.row_start + r) * I + item.col_block * 128 + ld_chunk * 16) = v;
+        v4i* dst = (v4i*)(hq + (size_t)(item.row_start + r) * I + item.col_block * 128 + ld_chunk * 16);
+        // (a launch of short tiles is a weight stream, which plain stores slow down: 777 tokens of the DeepSeek-V3 layer
+        // 1394 -> 1386 us, 1000 of Qwen3-MoE 154 -> 150.5; shorter and taller tiles leave h where the down GEMM finds it)
+        if (XF == 2 || XF == 3) __builtin_nontemporal_store(v, dst);
+        else *dst = v;
       }
     }
   } else {
