@@ -76,7 +76,8 @@ struct TileList {
 // An expert with `rows` rows gets ceil(rows / 256) row tiles whose heights, counted in units of 32 rows, differ by
 // at most one: no tile computes more than 31 rows of padding, and tiles that share a weight slab take about the same
 // time per K step and walk it together, so the later reader finds it in L2.
-__host__ __device__ inline int moe_tile_count(int rows) { return rows <= 0 ? 0 : (rows + 255) >> 8; }
+constexpr int kTileRows = 288;
+__host__ __device__ inline int moe_tile_count(int rows) { return rows <= 0 ? 0 : (rows + kTileRows - 1) / kTileRows; }
 // first row (relative to the expert's first) and row count of tile t of nt
 __host__ __device__ inline void moe_tile_span(int rows, int nt, int t, int& start, int& count) {
   if (nt == 1) {   // (integer division costs some forty instructions on this hardware: the one-tile case takes none)
@@ -303,7 +304,7 @@ struct GemmScales {
   int in_row, in_kb;
   bool in_listed;
   int out_row, out_cb;   // gate/up only: scale of (row, column block cb) of h = sh[row * out_row + cb * out_cb]
-  bool stream_out;       // down only, set by the launch: y is stored with non-temporal stores
+  bool out_through;      // set by the launch: the output's stores go through the L2 at once
 };
 inline GemmScales moe_row_major_scales(int K, int I) { return GemmScales{K / 128, 1, false, I / 128, 1}; }
 // Operands of one grouped GEMM.  Gate/up: w0 = gate, w1 = up, K = D, N = I, out = h codes, out_scale = h scales; down:
@@ -444,6 +445,11 @@ __device__ __forceinline__ void dma16_nt(const uint8_t* base, unsigned off, unsi
 __device__ __forceinline__ void dma4(const uint8_t* base, unsigned off, unsigned lds_addr) {
   const unsigned m0v = __builtin_amdgcn_readfirstlane(lds_addr);
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(m0v), "v"(off), "s"(base) : "memory", "m0");
+}
+// a 16-byte store; `through`: the L2 passes it on at once instead of when the line falls out of it
+__device__ __forceinline__ void store16(v4i* dst, v4i v, bool through) {
+  if (through) asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(dst), "v"(v) : "memory");
+  else *dst = v;
 }
 __device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xC07F); }   // lgkmcnt = 0, other counters untouched
 template <int N> __device__ __forceinline__ void wait_vm() {

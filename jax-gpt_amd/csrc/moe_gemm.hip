@@ -127,7 +127,7 @@ template <int XF, int MODE = MODE_GATEUP, bool ONCE = true> struct Cls {
   // blocks and comes from L2.  Measured on the loop's skeleton, weights two steps ahead instead of one: 5-7 % on a
   // weight slab that four workgroups share or that a workgroup streams alone, nothing when every line is an L2 hit.
   static constexpr int X_NST = XF >= 5 ? 2 : XF >= 2 ? 3 : 4;
-  static constexpr int W_NST = XF == 8 ? 2 : XF >= 2 ? 3 : 4;
+  static constexpr int W_NST = XF >= 8 ? 2 : XF >= 2 ? 3 : 4;
   // A weight stage is read once per step: every wave loads its four weight fragments into registers when it enters
   // the step, and from then on the stage is free.  With W_EARLY the next tenant's copies are issued right there, in
   // the middle of the step, and not behind the next barrier: the weights of step kb + 2 are then in flight while step
@@ -138,7 +138,7 @@ template <int XF, int MODE = MODE_GATEUP, bool ONCE = true> struct Cls {
   // heights of skewed routing; the down GEMM (16 K steps at the DeepSeek-V3 shape) gained 2 % in the first case and
   // lost 1 % in the second, and the classes with three weight stages cannot gain: their copies complete in issue
   // order behind the activation copies of the step before, which must have landed a step earlier.
-  static constexpr bool W_EARLY = XF == 8 && MODE == MODE_GATEUP;
+  static constexpr bool W_EARLY = XF >= 8 && MODE == MODE_GATEUP;
   static constexpr int EARLY_G = 3;   // the group behind which the weight copies of a W_EARLY step begin (2 and 4: within 1 %)
   static constexpr int X_PRE = X_NST - 1, W_PRE = W_NST - 1 + (W_EARLY ? 1 : 0);   // steps that a copy runs ahead of its use
   // The weight copies' cache policy.  ONCE: the item's expert has one row tile (or two that stay close, see the
@@ -147,7 +147,7 @@ template <int XF, int MODE = MODE_GATEUP, bool ONCE = true> struct Cls {
   // DeepSeek-V3 layer went from 1010 to 864 us, gate/up and down at 6.7 TB/s instead of 5.8.  An expert of several row
   // tiles has tiles of more than 96 rows (moe_tile_span), so the shorter classes exist in this form only.
   static constexpr bool W_ONCE = ONCE;
-  static_assert(ONCE || XF > 3, "an expert of several row tiles has none this short");
+  static_assert(ONCE || XF > 4, "an expert of several row tiles has none this short");
   static constexpr int X_STAGE_S_OFF = BM * BK;                // the scales behind the tile
   // + 256: every copying wave copies 64 scale slots from its first one on (no lane mask, which would cut the
   // unrolled K step into blocks); the surplus lanes rewrite other waves' slots with the same values or land in this pad
@@ -159,7 +159,9 @@ template <int XF, int MODE = MODE_GATEUP, bool ONCE = true> struct Cls {
   // can feed it (2-3 % over all eight waves copying).  Wave v copies 8 weight row groups (the rows that it reads
   // itself), activation row groups v, v + 4, ... and 64 scale slots.
   static constexpr int X_OPS = XF;                     // activation copies per copying wave and step
-  static constexpr int XS_OPS = X_OPS + 1;             // + 1 scale copy
+  static constexpr int S_OPS = BM > 256 ? 2 : 1;       // scale copies: 64 slots each, four waves
+  static constexpr int XS_OPS = X_OPS + S_OPS;
+  static constexpr bool S_LATE = XF == 9;              // read a group's scale with its fragment (registers: 144 are accumulators)
   static constexpr int OPS = 8 + XS_OPS;               // + 8 weight row groups
   // Copies complete in the order of their issue, so within a step those with the earlier deadline go first: with
   // the deeper weight ring the activation copies (and scales), then the weights; with rings of one depth the
@@ -167,7 +169,8 @@ template <int XF, int MODE = MODE_GATEUP, bool ONCE = true> struct Cls {
   static constexpr bool X_FIRST = W_PRE > X_PRE;
   static constexpr bool is_w(int i) { return X_FIRST ? i >= XS_OPS : i < 8; }
   static constexpr int w_index(int i) { return X_FIRST ? i - XS_OPS : i; }
-  static constexpr bool is_s(int i) { return X_FIRST ? i == X_OPS : i == OPS - 1; }
+  static constexpr bool is_s(int i) { return X_FIRST ? i >= X_OPS && i < XS_OPS : i >= 8 + X_OPS; }
+  static constexpr int s_index(int i) { return X_FIRST ? i - X_OPS : i - 8 - X_OPS; }
   static constexpr int x_index(int i) { return X_FIRST ? i : i - 8; }
   // what may still be in flight when a step starts that found every later copy issued: the activation stages and
   // weight stages of the steps after it
@@ -195,7 +198,7 @@ template <int XF, int MODE = MODE_GATEUP, bool ONCE = true> struct Cls {
   }
 };
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
-constexpr int CLS_RING = cmax(cmax(cmax(Cls<8>::RING_BYTES, Cls<7>::RING_BYTES), cmax(Cls<6>::RING_BYTES, Cls<5>::RING_BYTES)),
+constexpr int CLS_RING = cmax(cmax(cmax(cmax(Cls<9>::RING_BYTES, Cls<8>::RING_BYTES), Cls<7>::RING_BYTES), cmax(Cls<6>::RING_BYTES, Cls<5>::RING_BYTES)),
                               cmax(cmax(Cls<4>::RING_BYTES, Cls<3>::RING_BYTES), cmax(Cls<2>::RING_BYTES, Cls<1>::RING_BYTES)));
 constexpr int CLS_WSCALE_OFF = CLS_RING;                       // [2][MAX_KB] weight block scales of the work item
 constexpr int CLS_FLAG_OFF = CLS_WSCALE_OFF + 2 * MAX_KB * 4;  // [4] early_flag: the step whose weight fragments wave (wi, 1) holds, + 1
@@ -245,15 +248,17 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
     if (row_ids) g = row_ids[g];
     xoff[i] = (unsigned)g * (unsigned)K + piece * 16;
   }
-  const int sbase = BM >= 64 ? min(cv * 64, BM - 64) : 0;   // first of the 64 scale slots this wave copies
-  unsigned soff;
-  {
-    const int p = min(sbase + lane, BM - 1);   // slots past the tile land in the pad
+  // first of the 64 scale slots that this wave copies (a second copy, all four waves the same, where 256 are not all)
+  auto sbase = [&](int i) { return i > 0 ? BM - 64 : BM >= 64 ? min(cv * 64, BM - 64) : 0; };
+  unsigned soff[C::S_OPS];
+#pragma unroll
+  for (int i = 0; i < C::S_OPS; ++i) {
+    const int p = min(sbase(i) + lane, BM - 1);   // slots past the tile land in the pad
     const int q = p % HALF;
     const int r = 16 * (2 * (q % XF) + p / HALF) + q / XF;
     int g = item.row_start + min(r, item.row_count - 1);
     if (row_ids && !sc.in_listed) g = row_ids[g];
-    soff = (unsigned)g * (unsigned)sc.in_row * 4u;
+    soff[i] = (unsigned)g * (unsigned)sc.in_row * 4u;
   }
   const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)lds);
   // copies of step t's operands: weight row group w of this wave, activation row group x, the scales
@@ -271,14 +276,14 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
   auto copy_x = [&](int t, int x) {
     dma16(xq + (size_t)t * BK, xoff[x], lds0 + C::X_RING_OFF + (unsigned)(t % C::X_NST) * C::X_STAGE_BYTES + (x * 4 + cv) * 1024u);
   };
-  auto copy_s = [&](int t) {
-    dma4((const uint8_t*)(sx + (size_t)t * sc.in_kb), soff,
-         lds0 + C::X_RING_OFF + (unsigned)(t % C::X_NST) * C::X_STAGE_BYTES + C::X_STAGE_S_OFF + sbase * 4u);
+  auto copy_s = [&](int t, int i) {
+    dma4((const uint8_t*)(sx + (size_t)t * sc.in_kb), soff[i],
+         lds0 + C::X_RING_OFF + (unsigned)(t % C::X_NST) * C::X_STAGE_BYTES + C::X_STAGE_S_OFF + sbase(i) * 4u);
   };
   // operation i of the copies that step kb issues: each kind runs its ring's depth ahead of its use
   auto issue_op = [&](int kb, int i) {
     if (C::is_w(i)) copy_w(kb + C::W_PRE, C::w_index(i));
-    else if (C::is_s(i)) copy_s(kb + C::X_PRE);
+    else if (C::is_s(i)) copy_s(kb + C::X_PRE, C::s_index(i));
     else copy_x(kb + C::X_PRE, C::x_index(i));
   };
   if (xj == 0) {
@@ -405,9 +410,11 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
 #pragma unroll
       for (int f = 0; f < 4; ++f) wf[f] = read_frag(wt + wfrag_off[f]);
       float sxv[XF];
+      const uint8_t* sp = xs + C::X_STAGE_S_OFF + xj * HALF * 4 + fr * XF * 4;
       {
-        const uint8_t* sp = xs + C::X_STAGE_S_OFF + xj * HALF * 4 + fr * XF * 4;
-        if constexpr (XF % 4 == 0) {
+        if constexpr (C::S_LATE) {
+          sxv[0] = *(const float*)sp;
+        } else if constexpr (XF % 4 == 0) {
 #pragma unroll
           for (int j = 0; j < XF; j += 4) {
             const v4f a = *(const v4f*)(sp + j * 4);
@@ -431,10 +438,14 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
       fence();
 #pragma unroll
       for (int j = 0; j < NG; ++j) {
-        if (j + 1 < NG) xf[(j + 1) & 1] = read_frag(xt + (j + 1) * 32 * BK);
+        if (j + 1 < NG) {
+          xf[(j + 1) & 1] = read_frag(xt + (j + 1) * 32 * BK);
+          if (C::S_LATE) sxv[j + 1] = *(const float*)(sp + (j + 1) * 4);
+        }
         if (ROT > 0 && j == 0) {
 #pragma unroll
           for (int i = 0; i < ROT; ++i) {
+            if (C::S_LATE) sxv[NG + i] = *(const float*)(sp + (NG + i) * 4);
             held[i] = read_frag(xt + (NG + i) * 32 * BK);
             hc0[i] = sxv[NG + i] * s0;
             hc1[i] = sxv[NG + i] * s1;
@@ -447,10 +458,10 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
         }
         // pinned order: the next group's fragment reads first (a whole group of latency cover), then FMA quadruple f
         // just before MFMA f (left alone the compiler puts all 16 FMAs before the 4 MFMAs: down GEMM 3-6 % slower)
-        if (j + 1 < NG) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        if (j + 1 < NG) __builtin_amdgcn_sched_group_barrier(0x100, C::S_LATE ? 3 : 2, 0);
         if (ROT > 0 && j == 0) {
 #pragma unroll
-          for (int i = 0; i < ROT; ++i) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+          for (int i = 0; i < ROT; ++i) __builtin_amdgcn_sched_group_barrier(0x100, C::S_LATE ? 3 : 2, 0);
         }
 #pragma unroll
         for (int f = 0; f < 4; ++f) {
@@ -523,7 +534,7 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
 #pragma unroll
     for (int f = 0; f < 4; ++f) fm(f, XF - 1, pc0, pc1);
   };
-  constexpr int ROT1 = XF > ROTC ? ROTC : XF - 1;   // (fewer groups than that: what there is)
+  constexpr int ROT1 = XF == 9 ? 1 : XF > ROTC ? ROTC : XF - 1;   // (fewer groups than that: what there is)
   if (xj == 0) run(std::integral_constant<int, 0>{}, std::true_type{});
   else run(std::integral_constant<int, ROT1>{}, std::false_type{});
   __syncthreads();   // every wave is done reading the ring before the epilogue reuses LDS
@@ -578,10 +589,7 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
       if (r < item.row_count) {
         v4i v = *(const v4i*)(tile + swz(r, ld_chunk));
         v4i* dst = (v4i*)(hq + (size_t)(item.row_start + r) * I + item.col_block * 128 + ld_chunk * 16);
-        // (a launch of short tiles is a weight stream, which plain stores slow down: 777 tokens of the DeepSeek-V3 layer
-        // 1394 -> 1386 us, 1000 of Qwen3-MoE 154 -> 150.5; shorter and taller tiles leave h where the down GEMM finds it)
-        if (XF == 2 || XF == 3) __builtin_nontemporal_store(v, dst);
-        else *dst = v;
+        store16(dst, v, sc.out_through);
       }
     }
   } else {
@@ -610,8 +618,7 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
       if (r < item.row_count && c32 * 8 < ncols) {
         v4i v = *(const v4i*)(tile + r * 512 + ((c32 ^ (r & 7)) << 4));
         v4i* dst = (v4i*)(y + (size_t)(item.row_start + r) * N + wrow0 + c32 * 8);
-        if (sc.stream_out) __builtin_nontemporal_store(v, dst);
-        else *dst = v;
+        store16(dst, v, sc.out_through);
       }
     }
   }
@@ -725,11 +732,12 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
 #define MOE_ITEM(XF, ONCE) item_body<MODE, XF, ONCE>(item, lds, xq, sx, row_ids, w0, sw0, w1, sw1, K, N, out, out_scale, sc)
 #define MOE_CLASS(XF) if (once) MOE_ITEM(XF, true); else MOE_ITEM(XF, false); break
   switch ((rows + 31) >> 5) {
+    case 9: MOE_CLASS(9);
     case 8: MOE_CLASS(8);
     case 7: MOE_CLASS(7);
     case 6: MOE_CLASS(6);
     case 5: MOE_CLASS(5);
-    case 4: MOE_CLASS(4);
+    case 4: MOE_ITEM(4, true); break;
     case 3: MOE_ITEM(3, true); break;
     case 2: MOE_ITEM(2, true); break;
     default: MOE_ITEM(1, true); break;
@@ -739,7 +747,7 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
 }
 int col_blocks(int mode, int N) { return mode == MODE_GATEUP ? N / 128 : (N + 255) / 256; }
 
-int max_tiles_for(int R, int E) { return (int)((long long)(R + 255) / 256 + (E < R ? E : R)); }
+int max_tiles_for(int R, int E) { return (int)(((long long)R + kTileRows - 1) / kTileRows + (E < R ? E : R)); }
 
 TileList tile_list(void* ws, int R, int E) {
   return TileList{max_tiles_for(R, E), (TileHeader*)ws, (TileEntry*)((char*)ws + sizeof(TileHeader))};
@@ -765,9 +773,14 @@ int check_operands(const GemmOperands& op, int rows, int E, int mode, const char
 template <int MODE>
 int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
   const char* what = MODE == MODE_GATEUP ? "gemm_gateup" : "gemm_down";
-  // An output that the memory-side cache (256 MB) cannot hold until the combine reads it goes past the caches
-  // (config 3: 0.94 GB, step -0.6 %); a smaller one stays cached (config 5: 235 MB, 0.4 % slower when streamed).
-  auto streamed = [](int rows, int N) { return MODE == MODE_DOWN && (size_t)rows * N * 2 > ((size_t)192 << 20); };
+  // A launch of short tiles is a weight stream, and writes in between cost the HBM far more than their bytes (512
+  // experts of 40 rows, down GEMM of K = 1024: 416 us with plain stores, 345 with none, at 6 % of the bytes).  Written
+  // through at once they cost half of that (380 us): DeepSeek-V3, 777 tokens 1395 -> 1370 us; full layer, 4096 tokens
+  // 1420 -> 1387.  An output that the L2s can keep until its reader comes stays there, and a launch of taller tiles
+  // has other limits (Qwen3-MoE, 2000 tokens = 125 rows an expert: 195 us plain, 200 through).
+  auto through = [](int rows, int E, int N) {
+    return (size_t)rows * N * (MODE == MODE_DOWN ? 2 : 1) > ((size_t)4 << 20) && rows <= 96ll * E;
+  };
   GemmOperands routed{}, dense{};
   TileList l{};
   int dense_rows = 0;
@@ -775,7 +788,7 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
   if (dn) {
     if (int rc = check_operands(dn->op, dn->rows, 1, MODE, what)) return rc;
     dense = dn->op;
-    dense.sc.stream_out = streamed(dn->rows, dense.N);
+    dense.sc.out_through = through(dn->rows, 1, dense.N);
     dense_rows = dn->rows;
     dense_blocks = 8 * (((long long)moe_tile_count(dense_rows) * col_blocks(MODE, dense.N) + 7) / 8);
     grid = dense_blocks;
@@ -788,7 +801,7 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
     MOE_REQUIRE(rt->ws_bytes >= need, MOE_ERR_WORKSPACE_TOO_SMALL, "%s: workspace %zu < %zu", what, rt->ws_bytes, need);
     if (rt->R > 0) {
       routed = rt->op;
-      routed.sc.stream_out = streamed(rt->R, routed.N);
+      routed.sc.out_through = through(rt->R, rt->E, routed.N);
       l = tile_list(rt->ws, rt->R, rt->E);
       // sized by the worst case of the largest XCD share (moe_xcd_share_cap_q) and of an XCD's draws from the pool;
       // surplus workgroups exit at once
