@@ -66,18 +66,20 @@ __host__ __device__ inline long long moe_xcd_share_cap_q(int max_tiles) {
   return ((long long)max_tiles << kTileQBits) >> 3;
 }
 struct TileEntry {
-  int expert, row_start, rows, first_tile;
+  int expert_tiles;   // expert (10 bits), then its number of row tiles (a list holds at most 2^25 / 288 of them)
+  int row_start, rows, first_tile;
 };
 struct TileList {
   int max_tiles;
+  int tile_rows;      // rows of a full tile: a multiple of 32, at most kTileRows
   TileHeader* hdr;
   TileEntry* tiles;
 };
-// An expert with `rows` rows gets ceil(rows / 256) row tiles whose heights, counted in units of 32 rows, differ by
+// An expert with `rows` rows gets ceil(rows / tile_rows) row tiles whose heights, counted in units of 32 rows, differ by
 // at most one: no tile computes more than 31 rows of padding, and tiles that share a weight slab take about the same
 // time per K step and walk it together, so the later reader finds it in L2.
 constexpr int kTileRows = 288;
-__host__ __device__ inline int moe_tile_count(int rows) { return rows <= 0 ? 0 : (rows + kTileRows - 1) / kTileRows; }
+__host__ __device__ inline int moe_tile_count(int rows, int tile_rows) { return rows <= 0 ? 0 : (rows + tile_rows - 1) / tile_rows; }
 // first row (relative to the expert's first) and row count of tile t of nt
 __host__ __device__ inline void moe_tile_span(int rows, int nt, int t, int& start, int& count) {
   if (nt == 1) {   // (integer division costs some forty instructions on this hardware: the one-tile case takes none)
@@ -97,7 +99,7 @@ __host__ __device__ inline void moe_tile_span(int rows, int nt, int t, int& star
 // as skewed as a biased router makes them, natural expert order leaves one XCD with up to a tenth more work than the
 // average, and the launch ends with its slowest XCD.  The experts are therefore ranked by size (in units of 32 rows)
 // and dealt to eight bins in snake order (0..7, 7..0, ...); the list holds bin after bin.
-// Called by every thread of a workgroup of 1024; thread e owns expert e (rows = 0 where there is none); lds_a and lds_b
+// Called by every thread of a workgroup of 1024; thread e owns expert e (rows = nt = 0 where there is none); lds_a and lds_b
 // are int[1024] in LDS.  Returns the index of expert e's first tile and writes the list header.
 //
 // The header's XCD shares are cut by cost, not by count: a row tile of u 32-row units costs about 8 + u (measured:
@@ -109,7 +111,7 @@ __host__ __device__ inline void moe_tile_span(int rows, int nt, int t, int& star
 // over size classes, an expert's place in the list follows from its rank in closed form, and the tiles and cost in
 // front of it are one scan over the list.  (Comparing every expert with every other took 10, 17 and 45 us at 128, 256
 // and 512 experts; this takes 4.)
-__device__ inline int moe_tile_cost(int rows) { return 8 * moe_tile_count(rows) + ((rows + 31) >> 5); }   // (< 2^31 for 2^32 / 128 rows)
+__device__ inline int moe_tile_cost(int rows, int tiles) { return 8 * tiles + ((rows + 31) >> 5); }   // (< 2^31 for 2^32 / 128 rows)
 __device__ inline void moe_tile_even_shares(TileHeader* hdr, int n_static, int n_tiles) {   // one thread
   hdr->n_tiles = n_tiles;
   hdr->n_static = n_static;
@@ -139,10 +141,9 @@ __device__ __forceinline__ void moe_scan_1024(int& a, int& b, int& all_a, int& a
   b += pb - b0;
   __syncthreads();   // (the wave totals may be overwritten)
 }
-__device__ inline int moe_tile_first(int e, int rows, int* lds_a, int* lds_b, TileHeader* hdr, int max_tiles) {
+__device__ inline int moe_tile_first(int e, int rows, int nt, int* lds_a, int* lds_b, TileHeader* hdr, int max_tiles) {
   __shared__ long long cut_q[9];
   __shared__ int tail_tiles[kTailRounds];   // tiles of the last, last but one, ... round of the ranking
-  const int nt = moe_tile_count(rows);
   // rank: largest class first, inside a class in any order (1023 = the largest class and everything above it)
   const int cls = rows > 0 ? 1023 - min((rows + 31) >> 5, 1023) : 0;
   lds_a[e] = 0;
@@ -191,7 +192,7 @@ __device__ inline int moe_tile_first(int e, int rows, int* lds_a, int* lds_b, Ti
   __syncthreads();
   if (rows > 0) {
     lds_a[at] = nt;
-    lds_b[at] = at < n_fixed ? moe_tile_cost(rows) : 0;   // (the pool has no part in the shares)
+    lds_b[at] = at < n_fixed ? moe_tile_cost(rows, nt) : 0;   // (the pool has no part in the shares)
   }
   __syncthreads();
   int tiles_before = lds_a[e], cost_before = lds_b[e], total, cost_all;
@@ -204,7 +205,7 @@ __device__ inline int moe_tile_first(int e, int rows, int* lds_a, int* lds_b, Ti
   // cut k sits where the cost of the fixed shares reaches k/8 of their whole: inside exactly one expert, whose
   // thread places it
   if (rows > 0 && at < n_fixed) {
-    const long long mine = (long long)moe_tile_cost(rows) * 8;
+    const long long mine = (long long)moe_tile_cost(rows, nt) * 8;
     for (int k = 1; k < 8; ++k) {
       const long long d = (long long)cost_all * k - (long long)mine_before * 8;   // (cost units x 8)
       if (d >= 0 && d < mine)   // (float: the cut need not be exact, only inside this expert's tiles)
@@ -281,7 +282,16 @@ int moe_permute_place(const int32_t* idx, int R, int E, int chunk, int n_chunks,
 // grouped GEMMs with an optional pre-built tile list in ws (moe_gemm.hip); the extern "C" entry points build their
 // own.  moe_gemm_tile_list describes the list the GEMMs of (R rows, E experts) expect in ws, so that the permutation
 // kernels, which hold every expert's row range anyway, can write it (moe_permute_impl) and no launch is spent on it.
-int moe_gemm_tile_list(int R, int E, void* ws, size_t ws_bytes, TileList* list);
+// tile_rows: moe_gemm_tile_rows of the GEMMs that will read it.
+int moe_gemm_tile_list(int R, int E, int tile_rows, void* ws, size_t ws_bytes, TileList* list);
+// Rows of a full tile for R rows in E groups and, in the same launches, dense_rows rows of a dense group; [0] gate/up,
+// [1] down: column blocks per row tile and K steps (0: that GEMM does not read the list).
+struct TileShape {
+  int R, E;
+  int ncb[2], kb[2];
+  int dense_rows, dense_ncb[2];
+};
+int moe_gemm_tile_rows(const TileShape& t);
 // the activation quantisers with an optional second copy of the scales, block-major in row order ((K/128, R): what
 // GemmScales{1, R} reads) -- spares the shared expert of a large batch the separate transposition
 // (x_f32: x holds f32 values, rounded to bf16 first)
@@ -322,14 +332,14 @@ struct GemmOperands {
   float* out_scale;
   GemmScales sc;
 };
-// the routed experts: R rows in E groups through a work list in ws, which the launch builds unless it is there already
+// the routed experts: R rows in E groups through a work list in ws, which the launch builds unless it is there already (list_tile_rows)
 struct RoutedGemm {
   GemmOperands op;
   const int32_t* group_offsets;
   int E, R;
   void* ws;
   size_t ws_bytes;
-  bool list_built;
+  int list_tile_rows;   // of the list that is there already, or 0: none is
 };
 // one group of all rows (the shared expert): no list, no workspace
 struct DenseGemm {

@@ -84,10 +84,10 @@ __global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __rest
     start = group_offsets[e];
     rows = group_offsets[e + 1] - start;
   }
-  const int tiles = moe_tile_count(rows);
-  const int first = moe_tile_first(e, rows, s_rows, s_key, l.hdr, l.max_tiles);
+  const int tiles = moe_tile_count(rows, l.tile_rows);
+  const int first = moe_tile_first(e, rows, tiles, s_rows, s_key, l.hdr, l.max_tiles);
   for (int t = 0; t < tiles; ++t)
-    if (first + t < l.max_tiles) l.tiles[first + t] = TileEntry{e, start, rows, first};   // (cannot overflow for consistent offsets)
+    if (first + t < l.max_tiles) l.tiles[first + t] = TileEntry{e | tiles << 10, start, rows, first};   // (cannot overflow for consistent offsets)
 }
 
 // ---- the kernel ------------------------------------------------------------------------------------------------
@@ -144,10 +144,9 @@ template <int XF, int MODE = MODE_GATEUP, bool ONCE = true> struct Cls {
   // The weight copies' cache policy.  ONCE: the item's expert has one row tile (or two that stay close, see the
   // dispatch), so that its weight lines are fetched once and marked non-temporal, which leaves the memory-side cache
   // alone.  A read-only stream reaches 7.1 TB/s that way and 6.3 without (4 GiB, any grid); 64 tokens of the
-  // DeepSeek-V3 layer went from 1010 to 864 us, gate/up and down at 6.7 TB/s instead of 5.8.  An expert of several row
-  // tiles has tiles of more than 96 rows (moe_tile_span), so the shorter classes exist in this form only.
+  // DeepSeek-V3 layer went from 1010 to 864 us, gate/up and down at 6.7 TB/s instead of 5.8.  Tiles of up to 128
+  // rows are their expert's only one in every launch that fills the chip, so these classes exist in this form only.
   static constexpr bool W_ONCE = ONCE;
-  static_assert(ONCE || XF > 4, "an expert of several row tiles has none this short");
   static constexpr int X_STAGE_S_OFF = BM * BK;                // the scales behind the tile
   // + 256: every copying wave copies 64 scale slots from its first one on (no lane mask, which would cut the
   // unrolled K step into blocks); the surplus lanes rewrite other waves' slots with the same values or land in this pad
@@ -664,7 +663,7 @@ __device__ __forceinline__ void expert_item(int local, int nt, int ncb, int& col
 template <int MODE, bool DENSE>
 __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands routed, TileHeader* hdr,
                                                             const TileEntry* __restrict__ tiles, const GemmOperands dense,
-                                                            int dense_rows, int dense_blocks) {
+                                                            int dense_rows, int dense_tiles, int dense_blocks) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const bool is_dense = DENSE && (int)blockIdx.x < dense_blocks;   // (dense_blocks is a multiple of 8: the XCD is blockIdx % 8 for both)
   const int xcd = blockIdx.x & 7;
@@ -673,7 +672,7 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
   Item item;
   if (is_dense) {
     // contiguous eighths of the items, so that row tiles that share a weight slab run under one L2
-    const int nt = moe_tile_count(dense_rows), items = nt * ncb;
+    const int nt = dense_tiles, items = nt * ncb;
     const int per = dense_blocks >> 3;
     const int local = xcd * per + (int)(blockIdx.x >> 3);
     if (local >= items) return;
@@ -704,11 +703,11 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
       item_id = pool_first + drawn;
     }
     const TileEntry te = tiles[item_id / ncb];   // entries [first_tile, first_tile + tiles) all describe this expert
-    const int nt = moe_tile_count(te.rows);
+    const int nt = te.expert_tiles >> 10;
     int rt, t0, tn;
     expert_item(item_id - te.first_tile * ncb, nt, ncb, item.col_block, rt);
     moe_tile_span(te.rows, nt, rt, t0, tn);
-    item.expert = te.expert;
+    item.expert = te.expert_tiles & 1023;
     item.tiles = nt;
     item.row_start = te.row_start + t0;
     item.row_count = tn;
@@ -747,10 +746,12 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
 }
 int col_blocks(int mode, int N) { return mode == MODE_GATEUP ? N / 128 : (N + 255) / 256; }
 
-int max_tiles_for(int R, int E) { return (int)(((long long)R + kTileRows - 1) / kTileRows + (E < R ? E : R)); }
+int max_tiles_for(int R, int E, int tile_rows) { return (int)(((long long)R + tile_rows - 1) / tile_rows + (E < R ? E : R)); }
+// fewest work items at which every launch takes full tiles (moe_gemm_tile_rows)
+constexpr int kFullTileItems = 768;
 
-TileList tile_list(void* ws, int R, int E) {
-  return TileList{max_tiles_for(R, E), (TileHeader*)ws, (TileEntry*)((char*)ws + sizeof(TileHeader))};
+TileList tile_list(void* ws, int R, int E, int tile_rows) {
+  return TileList{max_tiles_for(R, E, tile_rows), tile_rows, (TileHeader*)ws, (TileEntry*)((char*)ws + sizeof(TileHeader))};
 }
 
 int check_operands(const GemmOperands& op, int rows, int E, int mode, const char* what) {
@@ -781,16 +782,20 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
   auto through = [](int rows, int E, int N) {
     return (size_t)rows * N * (MODE == MODE_DOWN ? 2 : 1) > ((size_t)4 << 20) && rows <= 96ll * E;
   };
+  auto own_tile_rows = [](int rows, int E, const GemmOperands& op) {
+    return moe_gemm_tile_rows(TileShape{rows, E, {col_blocks(MODE, op.N), 0}, {op.K / BK, 0}, 0, {0, 0}});
+  };
   GemmOperands routed{}, dense{};
   TileList l{};
-  int dense_rows = 0;
+  int dense_rows = 0, dense_tiles = 0;
   long long dense_blocks = 0, grid = 0;
   if (dn) {
     if (int rc = check_operands(dn->op, dn->rows, 1, MODE, what)) return rc;
     dense = dn->op;
     dense.sc.out_through = through(dn->rows, 1, dense.N);
     dense_rows = dn->rows;
-    dense_blocks = 8 * (((long long)moe_tile_count(dense_rows) * col_blocks(MODE, dense.N) + 7) / 8);
+    dense_tiles = moe_tile_count(dense_rows, rt && rt->list_tile_rows ? rt->list_tile_rows : own_tile_rows(dense_rows, 1, dense));
+    dense_blocks = 8 * (((long long)dense_tiles * col_blocks(MODE, dense.N) + 7) / 8);
     grid = dense_blocks;
   }
   if (rt) {
@@ -802,7 +807,7 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
     if (rt->R > 0) {
       routed = rt->op;
       routed.sc.out_through = through(rt->R, rt->E, routed.N);
-      l = tile_list(rt->ws, rt->R, rt->E);
+      l = tile_list(rt->ws, rt->R, rt->E, rt->list_tile_rows ? rt->list_tile_rows : own_tile_rows(rt->R, rt->E, routed));
       // sized by the worst case of the largest XCD share (moe_xcd_share_cap_q) and of an XCD's draws from the pool;
       // surplus workgroups exit at once
       const long long max_items = (long long)l.max_tiles * col_blocks(MODE, routed.N);
@@ -812,21 +817,51 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
   }
   MOE_REQUIRE(grid < (1ll << 30), MOE_ERR_BAD_SHAPE, "%s: %lld work items exceed the grid limit", what, grid);
   if (grid == 0) return MOE_OK;
-  if (l.hdr && !rt->list_built)
+  if (l.hdr && !rt->list_tile_rows)
     hipLaunchKernelGGL(build_tiles_kernel, dim3(1), dim3(1024), 0, s, rt->group_offsets, rt->E, l);
   static std::atomic<unsigned long long> lds_raised[2] = {};
   auto* kernel = dn ? grouped_gemm_kernel<MODE, true> : grouped_gemm_kernel<MODE, false>;
   if (int rc = moe_raise_lds_limit((const void*)kernel, CLS_LDS_BYTES, lds_raised[dn != nullptr])) return rc;
   hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(NT), CLS_LDS_BYTES, s, routed, l.hdr, l.tiles, dense, dense_rows,
-                     (int)dense_blocks);
+                     dense_tiles, (int)dense_blocks);
   return moe_check_hip(hipGetLastError(), "gemm launch");
 }
 
 }  // namespace
 
+// Full tiles where they give every CU several work items; a smaller problem is cut so that its rounds over the 256 CUs
+// take the shortest time: a work item costs about (8 + height) per K step, in units of 32 rows, and some 50 of these
+// besides (list entry, first copies, epilogue).  8 experts of 64 rows were 16 work items of the down GEMM, on 256 CUs.
+// The groups are taken to be two standard deviations of an even routing above their mean, so that a count of tiles
+// that just fills a round does not spill into another one.
+int moe_gemm_tile_rows(const TileShape& t) {
+  const int groups = t.E < t.R ? t.E : t.R;
+  if (groups <= 0) return kTileRows;
+  const int mean = (t.R + groups - 1) / groups;
+  if (mean > kFullTileItems * kTileRows / groups) return kTileRows;
+  const int least = t.ncb[1] && t.ncb[1] < t.ncb[0] ? t.ncb[1] : t.ncb[0];
+  if (groups * ((mean + kTileRows - 1) / kTileRows) * least >= kFullTileItems) return kTileRows;
+  int spread = 0;
+  while (t.E > 1 && spread * spread < 4 * mean) ++spread;
+  const int units = (mean + spread + 31) / 32, dense_units = (t.dense_rows + 31) / 32;
+  int best = 0, best_u = kTileRows / 32;
+  for (int u = kTileRows / 32; u >= 1; --u) {
+    const int nt = (units + u - 1) / u, dense_nt = (dense_units + u - 1) / u, tallest = units > dense_units ? units : dense_units, height = tallest < u ? tallest : u;
+    int time = 0;
+    for (int g = 0; g < 2; ++g)
+      time += (groups * nt * t.ncb[g] + dense_nt * t.dense_ncb[g] + 255) / 256 * ((8 + height) * t.kb[g] + (t.kb[g] ? 50 : 0));
+    if (best == 0 || time < best) best = time, best_u = u;
+  }
+  return 32 * best_u;
+}
+
 extern "C" size_t moe_gemm_workspace_bytes(int R, int E, int N_out) {
   (void)N_out;   // the tile list does not depend on the number of output columns
-  return sizeof(TileHeader) + (size_t)max_tiles_for(R, E) * sizeof(TileEntry) + 256;
+  // lists of short tiles exist below kFullTileItems full tiles only
+  int tiles = max_tiles_for(R, E, kTileRows);
+  const int few = R < kFullTileItems * kTileRows ? R : kFullTileItems * kTileRows;
+  if (max_tiles_for(few, E, 32) > tiles) tiles = max_tiles_for(few, E, 32);
+  return sizeof(TileHeader) + (size_t)tiles * sizeof(TileEntry) + 256;
 }
 
 int moe_gemm_gateup_impl(const RoutedGemm* routed, const DenseGemm* dense, moe_stream_t stream) {
@@ -840,13 +875,13 @@ namespace {
 int gateup(const uint8_t* xq, const float* sx, const int32_t* row_ids, const uint8_t* w_gate, const float* sw_gate,
            const uint8_t* w_up, const float* sw_up, const int32_t* group_offsets, int E, int R, int D, int I, uint8_t* hq,
            float* sh, void* ws, size_t ws_bytes, GemmScales sc, moe_stream_t stream) {
-  const RoutedGemm r{{xq, sx, row_ids, w_gate, sw_gate, w_up, sw_up, D, I, hq, sh, sc}, group_offsets, E, R, ws, ws_bytes, false};
+  const RoutedGemm r{{xq, sx, row_ids, w_gate, sw_gate, w_up, sw_up, D, I, hq, sh, sc}, group_offsets, E, R, ws, ws_bytes, 0};
   return moe_gemm_gateup_impl(&r, nullptr, stream);
 }
 int down(const uint8_t* hq, const float* sh, const uint8_t* w_down, const float* sw_down, const int32_t* group_offsets, int E,
          int R, int I, int D, void* y_bf16, void* ws, size_t ws_bytes, GemmScales sc, moe_stream_t stream) {
   const RoutedGemm r{{hq, sh, nullptr, w_down, sw_down, nullptr, nullptr, I, D, y_bf16, nullptr, sc}, group_offsets, E, R, ws,
-                     ws_bytes, false};
+                     ws_bytes, 0};
   return moe_gemm_down_impl(&r, nullptr, stream);
 }
 }  // namespace
@@ -933,11 +968,11 @@ extern "C" int moe_gemm_down_fp8_layout(const uint8_t* hq, const float* sh, cons
   return down(hq, sh, w_down, sw_down, group_offsets, E, R, I, D, y_bf16, ws, ws_bytes, sc, stream);
 }
 
-// The tile list that the GEMM launches of (R rows, E experts) read from ws when they are told list_built = true.
-int moe_gemm_tile_list(int R, int E, void* ws, size_t ws_bytes, TileList* list) {
+// The tile list that the GEMM launches of (R rows, E experts) read from ws when they are told its list_tile_rows.
+int moe_gemm_tile_list(int R, int E, int tile_rows, void* ws, size_t ws_bytes, TileList* list) {
   MOE_REQUIRE(ws && list, MOE_ERR_NULL, "gemm tiles: null pointer");
   MOE_REQUIRE(E >= 1 && E <= 1024 && R >= 0, MOE_ERR_BAD_SHAPE, "gemm tiles: need 1 <= E <= 1024, got E=%d R=%d", E, R);
   MOE_REQUIRE(ws_bytes >= moe_gemm_workspace_bytes(R, E, 0), MOE_ERR_WORKSPACE_TOO_SMALL, "gemm tiles: workspace too small");
-  *list = tile_list(ws, R, E);
+  *list = tile_list(ws, R, E, tile_rows);
   return MOE_OK;
 }

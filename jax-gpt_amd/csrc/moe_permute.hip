@@ -85,10 +85,10 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(const int32_t* __r
       if (e == E - 1) o.group_offsets[E] = row_start + rows;
     }
     if (o.tl.tiles) {   // the grouped GEMMs' row tiles, an expert's tiles side by side (uniform branch)
-      const int nt = moe_tile_count(rows);
-      const int at = moe_tile_first(e, rows, total, before, o.tl.hdr, o.tl.max_tiles);
+      const int nt = moe_tile_count(rows, o.tl.tile_rows);
+      const int at = moe_tile_first(e, rows, nt, total, before, o.tl.hdr, o.tl.max_tiles);
       for (int t = 0; t < nt; ++t)
-        if (at + t < o.tl.max_tiles) o.tl.tiles[at + t] = TileEntry{e, row_start, rows, at};
+        if (at + t < o.tl.max_tiles) o.tl.tiles[at + t] = TileEntry{e | nt << 10, row_start, rows, at};
     }
     return;
   }
@@ -129,7 +129,7 @@ extern "C" int moe_permute(const int32_t* idx, int M, int k, int E, int32_t* gro
                            int32_t* group_offsets, int32_t* sorted_token_ids, int32_t* sort_order,
                            int32_t* inv_perm, void* ws, size_t ws_bytes, moe_stream_t stream) {
   return moe_permute_impl(idx, M, k, E, PermuteOut{group_sizes, group_offsets, sorted_token_ids, sort_order, inv_perm, k,
-                                                   TileList{0, nullptr, nullptr}}, ws, ws_bytes, nullptr, stream);
+                                                   TileList{}}, ws, ws_bytes, nullptr, stream);
 }
 
 int moe_permute_impl(const int32_t* idx, int M, int k, int E, const PermuteOut& o, void* ws, size_t ws_bytes, const QuantJob* quant,

@@ -68,7 +68,7 @@ __device__ __forceinline__ void permute_one_chunk(const int32_t* ids, int n, int
   int rows = 0;
   if (e < E)
     for (int w = 0; w < waves; ++w) rows += next[w * E + e];
-  const int nt = moe_tile_count(rows);
+  const int nt = o.tl.tiles ? moe_tile_count(rows, o.tl.tile_rows) : 0;
   int row_start = rows, tile_start = nt, rows_all, tiles_all;
   moe_scan_1024(row_start, tile_start, rows_all, tiles_all);
   if (e < E) {
@@ -83,7 +83,7 @@ __device__ __forceinline__ void permute_one_chunk(const int32_t* ids, int n, int
     if (e == E - 1) o.group_offsets[E] = row_start + rows;
     if (o.tl.tiles) {
       for (int t = 0; t < nt; ++t)
-        if (tile_start + t < o.tl.max_tiles) o.tl.tiles[tile_start + t] = TileEntry{e, row_start, rows, tile_start};
+        if (tile_start + t < o.tl.max_tiles) o.tl.tiles[tile_start + t] = TileEntry{e | nt << 10, row_start, rows, tile_start};
       if (e == 0) {
         const int all = min(tiles_all, o.tl.max_tiles);
         moe_tile_even_shares(o.tl.hdr, all, all);
