@@ -13,68 +13,78 @@ typedef moe_bf16x8 bf16x8;
 
 __global__ __launch_bounds__(256) void quant_act_kernel(const QuantJob q) { moe_quant_act_block(q, blockIdx.x); }
 
-// RMSNorm fused with the activation quantiser: one workgroup per row, the row stays in registers between the
-// two passes.  normed = bf16((x / sqrt(mean(x^2) + eps)) * (1 + weight)), the Qwen3.5 convention of
+// RMSNorm fused with the activation quantiser: one workgroup per row, thread t holds the row's 16-byte piece t between
+// the two passes, so that the 16 lanes of a quantisation group are neighbours as in quant_act_kernel.
+// normed = bf16((x / sqrt(mean(x^2) + eps)) * (1 + weight)), the Qwen3.5 convention of
 // jax_gpt/models/qwen35/primitives.py:16-32 (the step in front of the MoE layer, block.py:54 and :88), then
-// the 1x128 quantisation of the bf16 values.  Thread t holds the 16-byte pieces t, t + 256, ... of the row, so
-// the 16 lanes of a quantisation group are neighbours as in quant_act_kernel.  Sums are taken in a fixed order
-// with individually rounded operations.
+// the 1x128 quantisation of the bf16 values.  Sums are taken in a fixed order with individually rounded operations: the
+// first 256 threads add the squares of pieces t, t + 256, ... (through LDS where there are several).
+//   A launch of few rows is bound by latency, and straight-line code is part of it: some 0.3 us per KB that the first
+// wave has to fetch.  With four pieces per thread whatever D is (12.7 KB) and the weights read behind the sum 1 row of
+// 1024 took 6.3 us and 32 rows of 4096 9.7; this way
+// 2.6 and 5.0 (4096 rows of 4096: 51 and 25 us).
 constexpr int kNormPieces = 4;   // D <= 256 * 8 * 4 = 8192
 
-__global__ __launch_bounds__(256) void rmsnorm_quant_kernel(const void* __restrict__ x, int x_f32, const float* __restrict__ weight,
-                                                           float eps, int D, bf16x8* __restrict__ normed,
-                                                           uint2* __restrict__ xq, float* __restrict__ sx,
-                                                           float* __restrict__ sx_blocked) {
+template <int PIECES>
+__global__ __launch_bounds__(256 * PIECES) void rmsnorm_quant_kernel(const void* __restrict__ x, int x_f32,
+                                                                    const float* __restrict__ weight, float eps, int D,
+                                                                    bf16x8* __restrict__ normed, uint2* __restrict__ xq,
+                                                                    float* __restrict__ sx, float* __restrict__ sx_blocked) {
   __shared__ float wave_sum[4];
+  __shared__ v4i raw[PIECES > 1 ? 256 * PIECES : 1];
   const int row = blockIdx.x, P = D / 8, t = threadIdx.x;
-  float f[kNormPieces][8];
-  float ss = 0.f;
+  const bool ok = t < P;              // uniform over the 16 lanes of a group (P is a multiple of 16)
+  bf16x8 in = {};
+  float wt[8] = {};
+  if (ok) {
+    in = load_bf16x8(x, x_f32, (size_t)row * P + t);
 #pragma unroll
-  for (int i = 0; i < kNormPieces; ++i) {
-    const int p = t + 256 * i;
-    bf16x8 in = {};
-    if (p < P) in = load_bf16x8(x, x_f32, (size_t)row * P + p);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      f[i][j] = bf16_to_f32(in.v[j]);
-      ss = __fadd_rn(ss, __fmul_rn(f[i][j], f[i][j]));
-    }
+    for (int j = 0; j < 8; ++j) wt[j] = weight[t * 8 + j];
   }
+  if (PIECES > 1) {
+    raw[t] = __builtin_bit_cast(v4i, in);
+    __syncthreads();
+  }
+  if (t < 256) {
+    float ss = 0.f;
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) ss = __fadd_rn(ss, __shfl_xor(ss, off, MOE_WAVE));
-  if ((t & 63) == 0) wave_sum[t >> 6] = ss;
-  __syncthreads();
-  const float total = __fadd_rn(__fadd_rn(wave_sum[0], wave_sum[1]), __fadd_rn(wave_sum[2], wave_sum[3]));
-  const float rms = __fsqrt_rn(__fadd_rn(__fdiv_rn(total, (float)D), eps));
+    for (int i = 0; i < PIECES; ++i) {
+      const bf16x8 v = i == 0 ? in : __builtin_bit_cast(bf16x8, raw[t + 256 * i]);
 #pragma unroll
-  for (int i = 0; i < kNormPieces; ++i) {
-    const int p = t + 256 * i;
-    const bool ok = p < P;              // uniform over the 16 lanes of a group (P is a multiple of 16)
-    float amax = 0.f;
-    bf16x8 nb = {};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float wj = ok ? weight[p * 8 + j] : 0.f;
-      const float v = __fmul_rn(__fdiv_rn(f[i][j], rms), __fadd_rn(1.0f, wj));
-      nb.v[j] = f32_to_bf16(v);
-      f[i][j] = bf16_to_f32(nb.v[j]);
-      amax = fmaxf(amax, fabsf(f[i][j]));
-    }
-#pragma unroll
-    for (int off = 1; off < 16; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off, MOE_WAVE));
-    float scale, scale_inv;
-    fp8_scales(amax, scale, scale_inv);
-    if (ok) {
-      if (normed) normed[(size_t)row * P + p] = nb;
-      uint2 out;
-      out.x = pack4_e4m3(f[i][0] * scale, f[i][1] * scale, f[i][2] * scale, f[i][3] * scale);
-      out.y = pack4_e4m3(f[i][4] * scale, f[i][5] * scale, f[i][6] * scale, f[i][7] * scale);
-      xq[(size_t)row * P + p] = out;
-      if ((t & 15) == 0) {
-        sx[((size_t)row * P + p) >> 4] = scale_inv;
-        if (sx_blocked) sx_blocked[(size_t)(p >> 4) * gridDim.x + row] = scale_inv;   // the (K/128, M) array
+      for (int j = 0; j < 8; ++j) {
+        const float f = bf16_to_f32(v.v[j]);
+        ss = __fadd_rn(ss, __fmul_rn(f, f));
       }
     }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) ss = __fadd_rn(ss, __shfl_xor(ss, off, MOE_WAVE));
+    if ((t & 63) == 0) wave_sum[t >> 6] = ss;
+  }
+  __syncthreads();
+  if (!ok) return;
+  const float total = __fadd_rn(__fadd_rn(wave_sum[0], wave_sum[1]), __fadd_rn(wave_sum[2], wave_sum[3]));
+  const float rms = __fsqrt_rn(__fadd_rn(__fdiv_rn(total, (float)D), eps));
+  float f[8], amax = 0.f;
+  bf16x8 nb;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    nb.v[j] = f32_to_bf16(__fmul_rn(__fdiv_rn(bf16_to_f32(in.v[j]), rms), __fadd_rn(1.0f, wt[j])));
+    f[j] = bf16_to_f32(nb.v[j]);
+    amax = fmaxf(amax, fabsf(f[j]));
+  }
+#pragma unroll
+  for (int off = 1; off < 16; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off, MOE_WAVE));
+  float scale, scale_inv;
+  fp8_scales(amax, scale, scale_inv);
+  const size_t at = (size_t)row * P + t;
+  if (normed) normed[at] = nb;
+  uint2 out;
+  out.x = pack4_e4m3(f[0] * scale, f[1] * scale, f[2] * scale, f[3] * scale);
+  out.y = pack4_e4m3(f[4] * scale, f[5] * scale, f[6] * scale, f[7] * scale);
+  xq[at] = out;
+  if ((t & 15) == 0) {
+    sx[at >> 4] = scale_inv;
+    if (sx_blocked) sx_blocked[(size_t)(t >> 4) * gridDim.x + row] = scale_inv;   // the (K/128, M) array
   }
 }
 
@@ -158,8 +168,13 @@ int moe_rmsnorm_quant_impl(const void* x, int x_f32, const float* weight, float 
   MOE_REQUIRE(MOE_ALIGNED16(x) && MOE_ALIGNED16(xq) && MOE_ALIGNED16(normed_bf16), MOE_ERR_BAD_ALIGN,
               "rmsnorm_quant: pointers must be 16-byte aligned");
   if (M == 0) return MOE_OK;
-  hipLaunchKernelGGL(rmsnorm_quant_kernel, dim3(M), dim3(256), 0, (hipStream_t)stream, x, x_f32, weight, eps, D,
-                     (bf16x8*)normed_bf16, (uint2*)xq, sx, sx_blocked);
+  auto launch = [&](auto* kernel, int pieces) {
+    hipLaunchKernelGGL(kernel, dim3(M), dim3(256 * pieces), 0, (hipStream_t)stream, x, x_f32, weight, eps, D,
+                       (bf16x8*)normed_bf16, (uint2*)xq, sx, sx_blocked);
+  };
+  if (D <= 2048) launch(rmsnorm_quant_kernel<1>, 1);
+  else if (D <= 4096) launch(rmsnorm_quant_kernel<2>, 2);
+  else launch(rmsnorm_quant_kernel<kNormPieces>, kNormPieces);
   return moe_check_hip(hipGetLastError(), "rmsnorm_quant launch");
 }
 
