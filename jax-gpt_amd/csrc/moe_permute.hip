@@ -54,7 +54,8 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(const int32_t* __r
   const int c = (int)blockIdx.x - 1;   // chunk; workgroup 0 (started first) does the experts' side
   total[e] = 0;
   before[e] = 0;
-  const int waves = moe_place_waves(E);
+  const int first = c * chunk, n = c < 0 ? 0 : min(chunk, R - first);
+  const int waves = moe_place_waves(E, n);
   for (int i = e; i < waves * E; i += kPlaceThreads) smem[i] = 0;
   __syncthreads();
   // thread (part, e2) adds expert e2's counts in chunks part, part + parts, ...: independent coalesced loads
@@ -72,7 +73,6 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(const int32_t* __r
     if (all) atomicAdd(&total[e2], all);
     if (mine) atomicAdd(&before[e2], mine);
   }
-  const int first = c * chunk, n = min(chunk, R - first);
   if (c >= 0) place_pass<false>(ids + first, first, n, E, smem, o);
   __syncthreads();
   const int rows = total[e];
@@ -94,6 +94,7 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(const int32_t* __r
   }
   if (e < E) {
     int run = row_start + before[e];
+#pragma unroll 4
     for (int w = 0; w < waves; ++w) {
       const int v = smem[w * E + e];
       smem[w * E + e] = run;

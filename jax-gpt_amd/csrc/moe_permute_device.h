@@ -13,6 +13,11 @@ constexpr int kSmallRows = 2048;
 // waves that count and place: one counter per expert each, at most 32 KB of LDS in all
 __host__ __device__ inline int moe_place_waves(int E) { return E > 512 ? kPlaceWaves / 2 : kPlaceWaves; }
 __host__ __device__ inline size_t moe_place_lds_ints(int E) { return (size_t)moe_place_waves(E) * E; }
+// ... of a chunk of n entries: as many as have 64 entries to take (every wave's counters are cleared, added up and walked)
+__host__ __device__ inline int moe_place_waves(int E, int n) {
+  const int most = moe_place_waves(E), filled = (n + MOE_WAVE - 1) / MOE_WAVE;
+  return filled < 1 ? 1 : filled < most ? filled : most;
+}
 
 #ifdef __HIPCC__
 // lanes of this wave whose expert id equals mine (ids < 2^bits); inactive lanes pass id = -1
@@ -32,7 +37,7 @@ __device__ __forceinline__ int ilog2_ceil(int n) { return n <= 1 ? 0 : 32 - __cl
 // PLACE false: += the wave's entries per expert; true: next free output position, advanced as entries are placed.
 template <bool PLACE>
 __device__ __forceinline__ void place_pass(const int32_t* ids, int first, int n, int E, int* next, const PermuteOut& o) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, waves = moe_place_waves(E);
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, waves = moe_place_waves(E, n);
   if (wv >= waves) return;
   const int bits = ilog2_ceil(E);
   const int span = (n + waves * MOE_WAVE - 1) / (waves * MOE_WAVE) * MOE_WAVE;   // uniform
@@ -50,7 +55,7 @@ __device__ __forceinline__ void place_pass(const int32_t* ids, int first, int n,
       if (PLACE) {
         const int f = first + i;
         if (o.sort_order) o.sort_order[pos] = f;
-        if (o.sorted_token_ids) o.sorted_token_ids[pos] = f / o.k;
+        if (o.sorted_token_ids) o.sorted_token_ids[pos] = (int)((unsigned)f / (unsigned)o.k);   // (half the code of a signed division)
         if (o.inv_perm) o.inv_perm[f] = pos;
       }
     }
@@ -60,19 +65,21 @@ __device__ __forceinline__ void place_pass(const int32_t* ids, int first, int n,
 // The whole sort of one chunk (n entries starting at flat index 0) in one workgroup of kPlaceThreads; ids may be in
 // LDS.  next: moe_place_lds_ints(E) ints of LDS.  The caller synchronises before the call (ids written, LDS free).
 __device__ __forceinline__ void permute_one_chunk(const int32_t* ids, int n, int E, int* next, const PermuteOut& o) {
-  const int e = threadIdx.x, waves = moe_place_waves(E);
+  const int e = threadIdx.x, waves = moe_place_waves(E, n);
   for (int i = threadIdx.x; i < waves * E; i += kPlaceThreads) next[i] = 0;
   __syncthreads();
   place_pass<false>(ids, 0, n, E, next, o);
   __syncthreads();
   int rows = 0;
   if (e < E)
+#pragma unroll 4
     for (int w = 0; w < waves; ++w) rows += next[w * E + e];
   const int nt = o.tl.tiles ? moe_tile_count(rows, o.tl.tile_rows) : 0;
   int row_start = rows, tile_start = nt, rows_all, tiles_all;
   moe_scan_1024(row_start, tile_start, rows_all, tiles_all);
   if (e < E) {
     int run = row_start;
+#pragma unroll 4
     for (int w = 0; w < waves; ++w) {
       const int c = next[w * E + e];
       next[w * E + e] = run;
