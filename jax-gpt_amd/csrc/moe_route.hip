@@ -229,19 +229,44 @@ __device__ __forceinline__ int route_grouped_token(const RouteArgs& a, const flo
   return my_idx;
 }
 
-template <int N> __device__ __forceinline__ void add_slices(float& s, const float*& q, size_t stride) {
-  float v[N];
+// Columns [0, n) of the partial sums at p, added in slice order by the whole workgroup and rounded to bf16 (what the
+// router's own finishing pass computes).  The loads are what it waits for, so a thread has up to 8 slices of C columns
+// under way: past the last slice or column it reads the last one again.  (One column and batches of 8, 4, 1, 1, ...: the
+// launch took 24 us for 2047 tokens of 513 columns in 7 slices, 20 now.)
+template <int Z, int C>
+__device__ __forceinline__ void add_slices(float (&s)[C], const float* const (&q)[C], size_t slice, int z, int splits) {
+  float v[Z][C];
 #pragma unroll
-  for (int j = 0; j < N; ++j) v[j] = *(q += stride);
+  for (int j = 0; j < Z; ++j)
 #pragma unroll
-  for (int j = 0; j < N; ++j) s = __fadd_rn(s, v[j]);
+    for (int c = 0; c < C; ++c) v[j][c] = q[c][(size_t)min(z + j, splits - 1) * slice];
+#pragma unroll
+  for (int j = 0; j < Z; ++j)
+#pragma unroll
+    for (int c = 0; c < C; ++c) s[c] = z + j == 0 ? v[j][c] : z + j < splits ? __fadd_rn(s[c], v[j][c]) : s[c];
+}
+template <int C>
+__device__ __forceinline__ void sum_partials(const float* p, size_t slice, int splits, int n, float* rows) {
+  for (int i0 = threadIdx.x; i0 < n; i0 += C * blockDim.x) {
+    float s[C] = {};
+    const float* q[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) q[c] = p + min(i0 + c * (int)blockDim.x, n - 1);
+    int z = 0;
+    for (; splits - z > 4; z += 8) add_slices<8, C>(s, q, slice, z, splits);
+    if (splits - z > 1) add_slices<4, C>(s, q, slice, z, splits);
+    else if (splits - z == 1) add_slices<1, C>(s, q, slice, z, splits);
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+      if (i0 + c * (int)blockDim.x < n) rows[i0 + c * (int)blockDim.x] = bf16_to_f32(f32_to_bf16(s[c]));
+  }
 }
 
 // Workgroup c routes tokens [c * tokens_per_block, +tokens_per_block).  Around the selection:
 //  - LogitSource's partial sums are added by the whole workgroup for as many tokens as it has waves (a token's columns
-//    are contiguous in every slice: independent coalesced loads, eight in flight per thread) and the waves then read
-//    the rounded logits from LDS.  One wave summing its own token one load at a time took 87 us for 32 tokens of 513
-//    columns in 32 slices, most of the layer's overhead; this way 9 us.
+//    are contiguous in every slice: independent coalesced loads, see sum_partials) and the waves then read the rounded
+//    logits from LDS.  One wave summing its own token one load at a time took 87 us for 32 tokens of 513 columns in
+//    32 slices, most of the layer's overhead; this way 9 us.
 //  - chunk_hist: the workgroup's selections are counted for the sort by expert (one row of E counts per workgroup).
 //  - sort_here (one workgroup routes the whole batch): the sort itself follows in the same launch.
 //  - the blocks behind the routing blocks quantise the activations: independent work, one launch less.
@@ -273,15 +298,8 @@ __global__ __launch_bounds__(1024) void route_kernel(const RouteArgs a, const Ro
       if (t0 > first) __syncthreads();   // (the waves are done with the batch before)
       const size_t MN = (size_t)a.M * N;
       const float* p = a.src.partial + (size_t)t0 * N;
-      for (int i = threadIdx.x; i < nt * N; i += blockDim.x) {
-        const float* q = p + i;
-        float s = *q;
-        int z = 1;   // the slices in slice order, a batch of independent loads at a time
-        for (; z + 8 <= a.src.splits; z += 8) add_slices<8>(s, q, MN);
-        for (; z + 4 <= a.src.splits; z += 4) add_slices<4>(s, q, MN);
-        for (; z < a.src.splits; ++z) add_slices<1>(s, q, MN);
-        rows[i] = bf16_to_f32(f32_to_bf16(s));   // what the router's own finishing pass computes
-      }
+      if (nt * N > (int)blockDim.x) sum_partials<2>(p, MN, a.src.splits, nt * N, rows);
+      else sum_partials<1>(p, MN, a.src.splits, nt * N, rows);
       __syncthreads();
     }
     for (int tt = wave; tt < nt; tt += waves) {
