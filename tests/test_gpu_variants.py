@@ -1,0 +1,149 @@
+"""The kernels' variants against each other and against the oracle, at the sizes where the choice between them changes:
+row-tile heights and cache policies of the grouped GEMM, the shared expert inside or beside the routed launches, the
+one-launch sort, the remainders of the router's K slices, rows of the RMSNorm, f32 activations.
+
+Where two variants do the same individually rounded operations in the same order, the results must be equal bit for bit;
+a row's result does not depend on the tile that it is computed in (one scale block of K per matrix instruction, added in
+K order)."""
+import numpy as np
+import pytest
+
+from oracle import moe_oracle as O
+from tests import helpers as H
+from tests.test_gpu_parity import _check_logits, _ragged_case, jg, test_rmsnorm_quant_vs_oracle as check_rmsnorm  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+HEIGHTS = [257, 288, 289, 1, 32, 33, 576, 577, 0, 97, 128, 129, 160, 161, 192, 224, 225, 256]
+
+
+@pytest.mark.parametrize("E,D,I,sizes", [
+    (96, 2048, 1024, HEIGHTS),    # full tiles up to 288 rows; two tiles share their lines (K = 2048)
+    (64, 2304, 1536, HEIGHTS),    # K above 2048: two tiles do not; the down GEMM has fewer items and shorter tiles
+    (64, 2304, 2048, [1, 31, 32, 33, 40, 64, 65, 96, 97, 128]),   # a weight stream with outputs above 4 MB: written through
+])
+def test_row_tile_variants_give_the_same_bits(jg, E, D, I, sizes):
+    import torch
+    print("row tiles", E, D, I, flush=True)
+    sizes = [sizes[i % len(sizes)] for i in range(E)]
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    R = int(off[-1])
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(D + I)
+    rand = lambda *s: torch.randn(s, dtype=torch.bfloat16, device="cuda", generator=gen)
+    ex = {n: jg.quantize_weight_block(rand(E, *s).mul_(0.02))
+          for n, s in (("gate", (I, D)), ("up", (I, D)), ("down", (D, I)))}
+    xq, sx = jg.quant_act(rand(R, D))
+    doff = H.to_cuda(off)
+    hq, sh = jg.gemm_gateup_swiglu(xq, sx, ex["gate"], ex["up"], doff)
+    y = jg.gemm_down(hq, sh, ex["down"], doff)
+    for e in range(len(HEIGHTS)):
+        one = {n: {k: v[e:e + 1] for k, v in d.items()} for n, d in ex.items()}
+        for lo in range(int(off[e]), int(off[e + 1]), 32):      # the same rows, 32 at a time
+            hi = min(lo + 32, int(off[e + 1]))
+            o1 = H.to_cuda(np.array([0, hi - lo], np.int32))
+            hq1, sh1 = jg.gemm_gateup_swiglu(xq[lo:hi], sx[lo:hi].clone(), one["gate"], one["up"], o1)
+            y1 = jg.gemm_down(hq[lo:hi], sh[lo:hi].clone(), one["down"], o1)
+            assert torch.equal(hq1.view(torch.uint8), hq[lo:hi].view(torch.uint8)), f"expert {e}, row {lo}: h"
+            assert torch.equal(sh1, sh[lo:hi]), f"expert {e}, row {lo}: scales of h"
+            assert torch.equal(y1, y[lo:hi]), f"expert {e}, row {lo}: y"
+        if sizes[e] in (33, 97):                                 # and against the oracle (the classes agree with each other)
+            lo, hi = int(off[e]), int(off[e]) + 33
+            w, s = one["down"]["w"], one["down"]["scale_inv"]
+            want = O.grouped_gemm(H.codes_np(hq[lo:hi]), sh[lo:hi].cpu().numpy(), H.codes_np(w), s.cpu().numpy(), np.array([0, hi - lo], np.int32))
+            H.assert_close_out(H.bf16_to_np(y[lo:hi]), O.bf16_round(want.astype(np.float32)))
+
+
+def _layer(jg, D, E, I, SI, seed):
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(seed)
+    rand = lambda *s: torch.randn(s, dtype=torch.bfloat16, device="cuda", generator=gen)
+    q = lambda *s: jg.quantize_weight_block(rand(*s).mul_(0.02))
+    params = dict(gate_proj=q(E, I, D), up_proj=q(E, I, D), down_proj=q(E, D, I),
+                  gate_weight=rand(E, D).mul_(0.02).t(), shared_expert_gate_weight=rand(1, D).mul_(0.02).t())
+    if SI:
+        params.update(shared_gate_proj=q(1, SI, D), shared_up_proj=q(1, SI, D), shared_down_proj=q(1, D, SI))
+    return params, rand
+
+
+def test_shared_expert_beside_the_routing_gives_the_bits_of_the_joint_launches(jg):
+    """Above 16 M activation elements the shared expert runs on the side stream: same bits as a sub-batch that takes it
+    into the routed launches, and as every replay of a captured graph."""
+    import torch
+    print("forked shared expert", flush=True)
+    D, E, k = 4096, 8, 2
+    params, rand = _layer(jg, D, E, 128, 256, 3)
+    M = (1 << 24) // D + 40
+    x, lg = rand(M, D), rand(M, E).float()
+    kw = dict(top_k=k, experts={n: params[n] for n in ("gate_proj", "up_proj", "down_proj")},
+              shared={n: params["shared_" + n] for n in ("gate_proj", "up_proj", "down_proj")})
+    full = jg.moe_experts(x, lg, **kw)
+    part = jg.moe_experts(x[:1000].contiguous(), lg[:1000].contiguous(), **kw)
+    assert torch.equal(full[:1000], part)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = jg.moe_experts(x, lg, **kw)
+    for i in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, full), f"replay {i}"
+        assert torch.equal(jg.moe_experts(x, lg, **kw), full)
+
+
+@pytest.mark.parametrize("M,E,k,D", [
+    (1, 32, 2, 128), (8, 40, 3, 384),        # routed and sorted in one launch; 1 and 3 K slices
+    (9, 40, 3, 640), (8, 512, 10, 1152),     # one token more; 9 slices: a batch of eight and one
+    (33, 1000, 32, 1536),                    # eight counting waves, 12 slices
+    (70, 8, 2, 256), (2100, 33, 1, 1280),    # 3 waves of entries; several chunks, experts not a multiple of four
+    (1100, 1024, 4, 256),
+])
+def test_routing_inside_the_layer_is_exact(jg, M, E, k, D):
+    """Selection and sort against the oracle on the logits that the layer ranked, which are the router's own."""
+    import torch
+    print("routing", M, E, k, D, flush=True)
+    params, rand = _layer(jg, D, E, 128, 0, M + E)
+    x = rand(M, D)
+    out, dbg = jg.moe_experts(x, None, top_k=k, experts={n: params[n] for n in ("gate_proj", "up_proj", "down_proj")},
+                              gate_weight=params["gate_weight"], return_debug=True)
+    logits = dbg["logits"].cpu().numpy()
+    own = jg.router_logits(x, params["gate_weight"])
+    own = own[0] if isinstance(own, tuple) else own
+    assert np.array_equal(logits, own.cpu().numpy())
+    xn, wn = H.bf16_to_np(x), H.bf16_to_np(params["gate_weight"])
+    _check_logits(logits, O.router_logits(xn, wn), np.abs(xn).astype(np.float64) @ np.abs(wn).astype(np.float64))
+    idx, w = O.route_softmax_topk(logits, k)
+    assert np.array_equal(dbg["indices"].cpu().numpy(), idx)
+    assert np.allclose(dbg["weights"].cpu().numpy(), w, rtol=2e-6, atol=1e-9)
+    ref = O.sort_and_group(idx, E)
+    for name in ("group_sizes", "sorted_token_ids", "inv_perm"):
+        assert np.array_equal(dbg[name].cpu().numpy(), ref[name]), name
+    # the reference's two functions one after the other: the same path behind a selection that is handed in
+    sel = jg.moe_routing(x, params["gate_weight"], k)
+    assert torch.equal(sel[0], dbg["indices"]) and torch.equal(sel[1], dbg["weights"])
+    assert torch.equal(jg.expert_forward_single(x, *sel, params["gate_proj"], params["up_proj"], params["down_proj"]), out)
+
+
+@pytest.mark.parametrize("M,D", [(2, 2048), (2, 2176), (3, 4096), (1, 4224), (300, 1024)])
+def test_rmsnorm_row_lengths(jg, M, D):
+    check_rmsnorm(jg, M, D)
+
+
+@pytest.mark.parametrize("M,offset", [(3, 0), (300, 0)])
+def test_f32_activations_give_the_bits_of_their_bf16_rounding(jg, M, offset):
+    """moe.py:282: the layer computes from bf16(x) and returns the caller's dtype, also for a view at an odd offset."""
+    import torch
+    print("f32 activations", M, offset, flush=True)
+    D = 512
+    params, _ = _layer(jg, D, 16, 256, 128, 9)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M)
+    x = torch.randn(M * D + offset, device="cuda", generator=gen)[offset:].view(1, M, D)
+    norm = torch.randn(D, device="cuda", generator=gen) * 0.1
+    xb = x.to(torch.bfloat16)
+    got, want = jg.moe_layer(x, params, 4), jg.moe_layer(xb, params, 4)
+    assert got.dtype == torch.float32 and torch.equal(got, want.float())
+    got, want = jg.moe_sublayer(x, norm, params, 4), jg.moe_sublayer(xb, norm, params, 4)
+    assert got.dtype == torch.float32 and torch.equal(got, want.float())
