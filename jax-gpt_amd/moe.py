@@ -599,6 +599,8 @@ def moe_layer(x, params, n_experts_per_token, n_devices=1, axis_name="tp", mesh=
     x_flat = x.reshape(B * T, D)
     if x_flat.dtype not in (torch.bfloat16, torch.float32):
         raise TypeError(f"x: expected bf16 or f32 activations, got {x.dtype}")
+    if x_flat.dtype == torch.float32 and x_flat.data_ptr() % 16:
+        x_flat = x_flat.clone()   # (a view at an odd offset of its storage: the kernels read 16 bytes at a time)
     shared = None
     if params.get("shared_gate_proj") is not None:
         shared = dict(gate_proj=params["shared_gate_proj"], up_proj=params["shared_up_proj"],

@@ -131,7 +131,7 @@ def test_rmsnorm_row_lengths(jg, M, D):
     check_rmsnorm(jg, M, D)
 
 
-@pytest.mark.parametrize("M,offset", [(3, 0), (300, 0)])
+@pytest.mark.parametrize("M,offset", [(3, 0), (300, 0), (5, 1)])
 def test_f32_activations_give_the_bits_of_their_bf16_rounding(jg, M, offset):
     """moe.py:282: the layer computes from bf16(x) and returns the caller's dtype, also for a view at an odd offset."""
     import torch
