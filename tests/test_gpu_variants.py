@@ -126,6 +126,20 @@ def test_routing_inside_the_layer_is_exact(jg, M, E, k, D):
     assert torch.equal(jg.expert_forward_single(x, *sel, params["gate_proj"], params["up_proj"], params["down_proj"]), out)
 
 
+@pytest.mark.parametrize("M,E,k", [(9, 8, 2), (32, 8, 2), (33, 8, 2), (22, 40, 3), (17, 300, 4)])
+def test_ready_logits_routed_and_sorted_in_one_launch_or_two(jg, M, E, k):
+    print("routing of ready logits", M, E, k, flush=True)
+    params, rand = _layer(jg, 128, E, 128, 0, M)
+    lg = rand(M, E).float()
+    _, dbg = jg.moe_experts(rand(M, 128), lg, top_k=k, return_debug=True,
+                            experts={n: params[n] for n in ("gate_proj", "up_proj", "down_proj")})
+    idx, _ = O.route_softmax_topk(lg.cpu().numpy(), k)
+    assert np.array_equal(dbg["indices"].cpu().numpy(), idx)
+    ref = O.sort_and_group(idx, E)
+    for name in ("group_sizes", "sorted_token_ids", "inv_perm"):
+        assert np.array_equal(dbg[name].cpu().numpy(), ref[name]), name
+
+
 @pytest.mark.parametrize("M,D", [(2, 2048), (2, 2176), (3, 4096), (1, 4224), (300, 1024)])
 def test_rmsnorm_row_lengths(jg, M, D):
     check_rmsnorm(jg, M, D)
