@@ -235,8 +235,12 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
   // carries its blocks instead (QuantJob: the two are independent; one launch less and they overlap).  Not where the
   // router reads what the quantiser writes.
   const bool quant_in_route = !fork && !quantiser_feeds_router(a, io_f32);
+  // A few tokens behind an RMSNorm: norm, quantiser and router matmul are one launch, below.
+  const bool norm_router = !fork && !sx_blocked && a->norm_weight && a->w_router && !given_idx &&
+                           moe_norm_router_takes(a->M, a->D, a->E + (a->w_shared_gate ? 1 : 0), io_f32);
   QuantJob quant_job{};
-  if (quant_in_route) {
+  if (norm_router) {
+  } else if (quant_in_route) {
     if ((rc = moe_quant_act_job(a->x, io_f32, nullptr, a->M, a->D, b.xq, b.sx, sx_blocked, &quant_job))) return rc;
   } else if (!fork) {
     if ((rc = quantise(a, io_f32, b, sx_blocked, stream))) return rc;
@@ -275,9 +279,13 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
       quant_joined = true;
     }
     int splits = 0, n_cols = 0;
-    if ((rc = moe_router_partials(from_quantiser ? b.normed : a->x, a->M, a->D, a->w_router, a->E, a->w_shared_gate,
-                                  b.router_ws, b.router_ws_bytes, &splits, &n_cols, stream)))
-      return join(rc);
+    if (norm_router)
+      rc = moe_norm_router_partials(a->x, io_f32, a->norm_weight, a->norm_eps, a->M, a->D, a->w_router, a->E, a->w_shared_gate,
+                                    b.xq, b.sx, b.router_ws, b.router_ws_bytes, &splits, &n_cols, stream);
+    else
+      rc = moe_router_partials(from_quantiser ? b.normed : a->x, a->M, a->D, a->w_router, a->E, a->w_shared_gate,
+                               b.router_ws, b.router_ws_bytes, &splits, &n_cols, stream);
+    if (rc) return join(rc);
     float* gate_out = a->out_shared_gate ? a->out_shared_gate : b.shared_gate;   // (written by the routing kernel)
     if (a->w_shared_gate) shared_gate = gate_out;
     src = LogitSource{nullptr, (const float*)b.router_ws, splits, n_cols, a->out_logits, gate_out};

@@ -251,6 +251,11 @@ struct LogitSource {
 int moe_router_partials(const void* x_bf16, int M, int D, const void* w_router_bf16, int E,
                         const void* w_shared_gate_bf16, void* ws, size_t ws_bytes, int* splits_used, int* n_cols,
                         moe_stream_t stream);
+// RMSNorm, activation quantiser (row-major scales) and router matmul in one launch, for the calls that it takes (N as above)
+bool moe_norm_router_takes(int M, int D, int N, int x_f32);
+int moe_norm_router_partials(const void* x, int x_f32, const float* weight, float eps, int M, int D, const void* w_router_bf16,
+                             int E, const void* w_shared_gate_bf16, uint8_t* xq, float* sx, void* ws, size_t ws_bytes,
+                             int* splits_used, int* n_cols, moe_stream_t stream);
 // An activation quantisation (moe_quant_device.h): blocks of blockDim.x 16-byte pieces, in a launch of its own or
 // behind the routing kernel's own blocks.
 struct QuantJob {

@@ -115,6 +115,115 @@ __global__ __launch_bounds__(256, 2) void router_gemm_kernel(const bf16_t* __res
     }
 }
 
+// RMSNorm, activation quantiser and router matmul of up to kNormRouterTokens tokens in one launch: the sublayer's decode
+// step is a chain of launches, each of which costs some 3 us on the GPU and as much on the host, and for a few rows
+// every workgroup can add up the rows' squares itself while its weights travel.  Workgroup (column tile, K slice of 128
+// = one quantisation group): 4 waves of 32 columns; the slice's normalised pieces go through LDS to the MFMA's operand
+// lanes, the workgroups of column tile 0 write their group's codes and scale.  Sums, slices and instructions are those
+// of rmsnorm_quant_kernel and router_gemm_kernel in their order: the same bits.
+// 1 token of the mini sublayer 34 -> 32 us (6.2 of two launches became 4.7), of the Qwen3.5 sublayer 59.8 -> 57, 4 tokens
+// of it 122.1 -> 121; but 122.7 -> 123.4 from f32, where every workgroup rounds all rows: hence the limit on the pieces.
+constexpr int kNormRouterTokens = 4;
+inline int norm_row_pieces(int D) { return D <= 2048 ? 1 : D <= 4096 ? 2 : 4; }   // of 256 threads
+template <int PIECES, bool F32>
+__global__ __launch_bounds__(256) void norm_router_kernel(const void* __restrict__ x, const float* __restrict__ weight, float eps,
+                                                         int M, int D, const bf16_t* __restrict__ w, int E,
+                                                         const bf16_t* __restrict__ w_extra, int N, uint2* __restrict__ xq,
+                                                         float* __restrict__ sx, float* __restrict__ partial) {
+  constexpr int ROWS = PIECES < 4 ? kNormRouterTokens : 2;
+  __shared__ float wave_sum[ROWS][4];
+  __shared__ v4i a_lds[ROWS * 16];
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int fr = lane & 15, fq = lane >> 4;
+  const int z = blockIdx.y, n0 = blockIdx.x * RN + wave * 32, P = D / 8;
+  v4i b[2][4];
+  if (n0 < N) {
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const int n = min(n0 + 16 * g + fr, N - 1);
+      const v4i* src = (const v4i*)((n < E ? w + (size_t)n * D : w_extra) + z * 128) + fq;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) b[g][s] = src[4 * s];
+    }
+  }
+  // threads below 16 M: piece t % 16 of the slice, row t / 16
+  const bool mine = t < 16 * M;
+  const size_t at = (size_t)(t >> 4) * P + z * 16 + (t & 15);
+  moe_bf16x8 in = {};
+  float wt[8] = {};
+  if (mine) {
+    in = load_bf16x8(x, F32, at);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) wt[j] = weight[(z * 16 + (t & 15)) * 8 + j];
+  }
+  moe_bf16x8 row[ROWS][PIECES] = {};
+#pragma unroll
+  for (int m = 0; m < ROWS; ++m)
+    if (m < M)
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i)
+        if (t + 256 * i < P) row[m][i] = load_bf16x8(x, F32, (size_t)m * P + t + 256 * i);
+#pragma unroll
+  for (int m = 0; m < ROWS; ++m) {
+    if (m >= M) break;
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float f = bf16_to_f32(row[m][i].v[j]);
+        ss = __fadd_rn(ss, __fmul_rn(f, f));
+      }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) ss = __fadd_rn(ss, __shfl_xor(ss, off, MOE_WAVE));
+    if (lane == 0) wave_sum[m][wave] = ss;
+  }
+  __syncthreads();
+  if (mine) {
+    const float* q = wave_sum[t >> 4];
+    const float total = __fadd_rn(__fadd_rn(q[0], q[1]), __fadd_rn(q[2], q[3]));
+    const float rms = __fsqrt_rn(__fadd_rn(__fdiv_rn(total, (float)D), eps));
+    float f[8], amax = 0.f;
+    moe_bf16x8 nb;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      nb.v[j] = f32_to_bf16(__fmul_rn(__fdiv_rn(bf16_to_f32(in.v[j]), rms), __fadd_rn(1.0f, wt[j])));
+      f[j] = bf16_to_f32(nb.v[j]);
+      amax = fmaxf(amax, fabsf(f[j]));
+    }
+    a_lds[t] = __builtin_bit_cast(v4i, nb);
+    if (blockIdx.x == 0) {
+#pragma unroll
+      for (int off = 1; off < 16; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off, MOE_WAVE));
+      float scale, scale_inv;
+      fp8_scales(amax, scale, scale_inv);
+      uint2 out;
+      out.x = pack4_e4m3(f[0] * scale, f[1] * scale, f[2] * scale, f[3] * scale);
+      out.y = pack4_e4m3(f[4] * scale, f[5] * scale, f[6] * scale, f[7] * scale);
+      xq[at] = out;
+      if ((t & 15) == 0) sx[at >> 4] = scale_inv;
+    }
+  }
+  __syncthreads();
+  if (n0 >= N) return;
+  v4f acc[2] = {};
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const v4i av = fr < M ? a_lds[fr * 16 + 4 * s + fq] : (v4i){0, 0, 0, 0};
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+      acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av), __builtin_bit_cast(bf16x8_t, b[g][s]), acc[g], 0, 0, 0);
+  }
+  float* out = partial + (size_t)z * M * N;
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    const int n = n0 + 16 * g + fr;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (4 * fq + r < M && n < N) out[(size_t)(4 * fq + r) * N + n] = acc[g][r];
+  }
+}
+
 __global__ __launch_bounds__(256) void router_finish_kernel(const float* __restrict__ partial, int M, int E, int N,
                                                            int splits, float* __restrict__ logits,
                                                            float* __restrict__ shared_gate) {
@@ -157,34 +266,71 @@ extern "C" size_t moe_router_workspace_bytes(int M, int D, int E) {
   return (a > b ? a : b) + 256;
 }
 
-// The matmul alone: split-K partial sums [splits][M][N] at the start of ws (N = E, + 1 with the gate column).
-int moe_router_partials(const void* x_bf16, int M, int D, const void* w_router_bf16, int E,
-                        const void* w_shared_gate_bf16, void* ws, size_t ws_bytes, int* splits_used, int* n_cols,
-                        moe_stream_t stream) {
-  MOE_REQUIRE((M == 0 || x_bf16) && w_router_bf16 && ws, MOE_ERR_NULL, "router: null pointer");
+namespace {
+int check_partials(const void* x, int M, int D, const void* w_router_bf16, int E, const void* w_shared_gate_bf16, void* ws,
+                   size_t ws_bytes, int* k_per_split, int* splits_used, int* n_cols) {
+  MOE_REQUIRE((M == 0 || x) && w_router_bf16 && ws, MOE_ERR_NULL, "router: null pointer");
   MOE_REQUIRE(M >= 0 && D > 0 && D % 128 == 0 && E >= 1 && E <= 1024, MOE_ERR_BAD_SHAPE,
               "router: need D %% 128 == 0 and 1 <= E <= 1024, got M=%d D=%d E=%d", M, D, E);
-  MOE_REQUIRE(MOE_ALIGNED16(x_bf16) && MOE_ALIGNED16(w_router_bf16) && MOE_ALIGNED16(w_shared_gate_bf16) &&
+  MOE_REQUIRE(MOE_ALIGNED16(x) && MOE_ALIGNED16(w_router_bf16) && MOE_ALIGNED16(w_shared_gate_bf16) &&
                   MOE_ALIGNED16(ws),
               MOE_ERR_BAD_ALIGN, "router: pointers must be 16-byte aligned");
   MOE_REQUIRE(ws_bytes >= moe_router_workspace_bytes(M, D, E), MOE_ERR_WORKSPACE_TOO_SMALL,
               "router: workspace %zu < %zu", ws_bytes, moe_router_workspace_bytes(M, D, E));
   const int N = E + (w_shared_gate_bf16 ? 1 : 0);
-  int k_per_split = 0;
-  const int used = slices_used(M, N, D, &k_per_split);
+  const int used = slices_used(M, N, D, k_per_split);
   MOE_REQUIRE(ws_bytes >= (size_t)used * (size_t)M * N * sizeof(float), MOE_ERR_WORKSPACE_TOO_SMALL,
               "router: %d slices of %d x %d partial sums do not fit the workspace (%zu bytes)", used, M, N, ws_bytes);
   *splits_used = used;
   *n_cols = N;
+  return MOE_OK;
+}
+}  // namespace
+
+// The matmul alone: split-K partial sums [splits][M][N] at the start of ws (N = E, + 1 with the gate column).
+int moe_router_partials(const void* x_bf16, int M, int D, const void* w_router_bf16, int E,
+                        const void* w_shared_gate_bf16, void* ws, size_t ws_bytes, int* splits_used, int* n_cols,
+                        moe_stream_t stream) {
+  int k_per_split = 0;
+  if (int rc = check_partials(x_bf16, M, D, w_router_bf16, E, w_shared_gate_bf16, ws, ws_bytes, &k_per_split, splits_used, n_cols))
+    return rc;
   if (M == 0) return MOE_OK;
   MOE_REQUIRE((long long)M * D * 2 < (1ll << 32), MOE_ERR_BAD_SHAPE, "router: the activations must stay within 4 GB");
   hipStream_t s = (hipStream_t)stream;
   static std::atomic<unsigned long long> lds_raised{0};
   if (int rc = moe_raise_lds_limit((const void*)router_gemm_kernel, R_LDS, lds_raised)) return rc;
-  hipLaunchKernelGGL(router_gemm_kernel, dim3((M + RT - 1) / RT, (N + RN - 1) / RN, used), dim3(256), R_LDS, s,
+  const int N = *n_cols;
+  hipLaunchKernelGGL(router_gemm_kernel, dim3((M + RT - 1) / RT, (N + RN - 1) / RN, *splits_used), dim3(256), R_LDS, s,
                      (const bf16_t*)x_bf16, M, D, (const bf16_t*)w_router_bf16, E, (const bf16_t*)w_shared_gate_bf16, N,
                      k_per_split, (float*)ws);
   return moe_check_hip(hipGetLastError(), "router launch");
+}
+
+// Few tokens whose K slices are one quantisation group each (rows of up to 8192, as for the RMSNorm launch).
+bool moe_norm_router_takes(int M, int D, int N, int x_f32) {
+  int k_per_split = 0;
+  if (M < 1 || M > kNormRouterTokens || D < 128 || D > 8192 || D % 128 || M * norm_row_pieces(D) > (x_f32 ? 6 : 8)) return false;
+  slices_used(M, N, D, &k_per_split);
+  return k_per_split == 128;
+}
+int moe_norm_router_partials(const void* x, int x_f32, const float* weight, float eps, int M, int D, const void* w_router_bf16,
+                             int E, const void* w_shared_gate_bf16, uint8_t* xq, float* sx, void* ws, size_t ws_bytes,
+                             int* splits_used, int* n_cols, moe_stream_t stream) {
+  int k_per_split = 0;
+  if (int rc = check_partials(x, M, D, w_router_bf16, E, w_shared_gate_bf16, ws, ws_bytes, &k_per_split, splits_used, n_cols))
+    return rc;
+  const int N = *n_cols;
+  MOE_REQUIRE(weight && xq && sx && MOE_ALIGNED16(xq) && moe_norm_router_takes(M, D, N, x_f32), MOE_ERR_BAD_SHAPE,
+              "norm + router: not a call for this launch (M=%d D=%d N=%d)", M, D, N);
+  auto launch = [&](auto* kernel) {
+    hipLaunchKernelGGL(kernel, dim3((N + RN - 1) / RN, *splits_used), dim3(256), 0, (hipStream_t)stream, x, weight, eps, M, D,
+                       (const bf16_t*)w_router_bf16, E, (const bf16_t*)w_shared_gate_bf16, N, (uint2*)xq, sx, (float*)ws);
+  };
+  const int pieces = norm_row_pieces(D);
+  if (pieces == 1) x_f32 ? launch(norm_router_kernel<1, true>) : launch(norm_router_kernel<1, false>);
+  else if (pieces == 2) x_f32 ? launch(norm_router_kernel<2, true>) : launch(norm_router_kernel<2, false>);
+  else x_f32 ? launch(norm_router_kernel<4, true>) : launch(norm_router_kernel<4, false>);
+  return moe_check_hip(hipGetLastError(), "norm + router launch");
 }
 
 extern "C" int moe_router_logits(const void* x_bf16, int M, int D, const void* w_router_bf16, int E,

@@ -161,3 +161,18 @@ def test_f32_activations_give_the_bits_of_their_bf16_rounding(jg, M, offset):
     assert got.dtype == torch.float32 and torch.equal(got, want.float())
     got, want = jg.moe_sublayer(x, norm, params, 4), jg.moe_sublayer(xb, norm, params, 4)
     assert got.dtype == torch.float32 and torch.equal(got, want.float())
+
+
+@pytest.mark.parametrize("D,E,SI,dtype", [(512, 16, 128, "bf16"), (2176, 40, 0, "f32"), (4096, 130, 128, "bf16"), (4224, 8, 0, "bf16"),
+                                          (8192, 1000, 128, "bf16")])   # (the last: K slices longer than a quantisation group)
+def test_few_tokens_behind_the_norm_give_the_bits_of_a_larger_batch(jg, D, E, SI, dtype):
+    """Up to four tokens take norm, quantiser and router matmul in one launch, five take two."""
+    import torch
+    print("norm and router", D, E, SI, dtype, flush=True)
+    params, rand = _layer(jg, D, E, 128, SI, D)
+    x = rand(1, 5, D).to(torch.float32 if dtype == "f32" else torch.bfloat16) * 3
+    norm = rand(D).float() * 0.1
+    x[0, 1] = 0                                              # an all-zero row
+    want = jg.moe_sublayer(x, norm, params, 2)
+    for m in (1, 2, 3, 4):
+        assert torch.equal(jg.moe_sublayer(x[:, :m].contiguous(), norm, params, 2), want[:, :m]), f"{m} tokens"
