@@ -16,7 +16,7 @@
 // ONE activation row: one activation scale per lane per fragment, not four.
 //
 // Data movement.  A workgroup (8 waves, two per SIMD, one workgroup per CU) owns a
-// work item = (expert, <= 256 activation rows, 256 weight rows) and walks K in
+// work item = (expert, <= 288 activation rows, 256 weight rows) and walks K in
 // steps of 128 through a ring of LDS stages.  Tiles are copied global -> LDS by
 // global_load_lds (no registers in between) ahead of their use, by one wave of
 // each SIMD (wave set 0); the other (set 1) only computes.  In
@@ -105,10 +105,10 @@ __global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __rest
 // epilogue staging tile: 128-byte rows, chunk c of row r at position c ^ (r & 7)
 __device__ __forceinline__ int swz(int row, int chunk) { return row * BK + ((chunk ^ (row & 7)) << 4); }
 
-// One launch, row tiles of every height.  A work item's row tile (at most 256 rows, near-equal cuts of its
-// expert) is served by the smallest of eight compiled tile classes that holds it -- 32 XF rows, XF = 1 .. 8 MFMA
+// One launch, row tiles of every height.  A work item's row tile (at most 288 rows, near-equal cuts of its
+// expert) is served by the smallest of nine compiled tile classes that holds it -- 32 XF rows, XF = 1 .. 9 MFMA
 // groups per wave and K step -- each a branch-free, fully unrolled K loop of its own with its own LDS ring: the
-// short classes have short activation tiles and use the room for more stages (256 rows: two stages; 160 to 224
+// short classes have short activation tiles and use the room for more stages (256 and 288 rows: two stages; 160 to 224
 // rows: three weight stages, two activation stages; 64 to 128 rows: three stages, copies two steps ahead; 32 rows:
 // four stages, three steps ahead), because an item of a few rows only streams its 256 weight rows and lives on the
 // bytes it keeps in flight.  Rows past the end of a tile are multiplied like the others (their copies re-read the tile's last

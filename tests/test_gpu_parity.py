@@ -371,10 +371,9 @@ def test_reference_entry_points(jg):
 
 @pytest.mark.parametrize("M", [64, 4224])
 def test_graph_replay_matches_eager(jg, M):
-    """The whole path (side stream for the shared expert included) captured in a HIP graph: every replay, with
-    eager calls and synchronisations between the replays, gives the eager result bit for bit.  The two batch
-    sizes take the two launch orders of moe_forward: 64 tokens quantise on the caller's stream and enqueue the
-    shared expert after the routed GEMMs, 4224 tokens (more than 2 M activation elements) fork at once."""
+    """The whole path captured in a HIP graph: every replay, with eager calls and synchronisations between the
+    replays, gives the eager result bit for bit.  64 tokens sort in one chunk, 4224 in several and read
+    block-major scales."""
     import torch
     _say("graph replay", M)
     prob = H.make_problem(M=M, D=512, E=32, k=4, I=256, SI=256, seed=7, routing="sigmoid_grouped")
