@@ -176,3 +176,16 @@ def test_few_tokens_behind_the_norm_give_the_bits_of_a_larger_batch(jg, D, E, SI
     want = jg.moe_sublayer(x, norm, params, 2)
     for m in (1, 2, 3, 4):
         assert torch.equal(jg.moe_sublayer(x[:, :m].contiguous(), norm, params, 2), want[:, :m]), f"{m} tokens"
+
+
+@pytest.mark.parametrize("M,E", [(1030, 24), (1030, 16)])   # 2060 rows: scales read row-major up to 96 rows an expert, gathered above
+def test_scale_layouts_of_middle_sized_batches_give_the_same_bits(jg, M, E):
+    import torch
+    print("scale layouts", M, E, flush=True)
+    params, rand = _layer(jg, 512, E, 256, 128, M + E)
+    x, lg = rand(M, 512), rand(M, E).float()
+    kw = dict(top_k=2, experts={n: params[n] for n in ("gate_proj", "up_proj", "down_proj")},
+              shared={n: params["shared_" + n] for n in ("gate_proj", "up_proj", "down_proj")})
+    whole = jg.moe_experts(x, lg, **kw)
+    assert torch.equal(whole, jg.moe_experts(x, lg, return_debug=True, **kw)[0])      # (h scales row-major)
+    assert torch.equal(whole[:400], jg.moe_experts(x[:400].contiguous(), lg[:400].contiguous(), **kw))
