@@ -74,8 +74,10 @@ constexpr int ROTC = 2;       // MFMA groups by which wave set 1 trails wave set
 // ---- work list -----------------------------------------------------------
 
 // One workgroup lists the row tiles of every expert (an expert's tiles side by side; which expert where: see
-// moe_tile_first); thread e owns expert e.
-__global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __restrict__ group_offsets, int E, TileList l) {
+// moe_tile_first); thread e owns expert e.  Up to 8 rows an expert the tiles cost alike: plain expert order and equal XCD
+// shares do, for 2.4 us less a launch (expert-parallel shard of 32 experts, 64 rows 178.3 -> 173.3 us, 256 rows 213 ->
+// 208; with 800 unevenly spread rows it would be 239 -> 269).
+__global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __restrict__ group_offsets, int E, int R, TileList l) {
   __shared__ int s_rows[1024];
   __shared__ int s_key[1024];
   const int e = threadIdx.x;
@@ -85,7 +87,15 @@ __global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __rest
     rows = group_offsets[e + 1] - start;
   }
   const int tiles = moe_tile_count(rows, l.tile_rows);
-  const int first = moe_tile_first(e, rows, tiles, s_rows, s_key, l.hdr, l.max_tiles);
+  int first;
+  if (R <= 8 * E) {
+    int unused = 0, all, unused_all;
+    first = tiles;
+    moe_scan_1024(first, unused, all, unused_all);
+    if (e == 0) moe_tile_even_shares(l.hdr, min(all, l.max_tiles), min(all, l.max_tiles));
+  } else {
+    first = moe_tile_first(e, rows, tiles, s_rows, s_key, l.hdr, l.max_tiles);
+  }
   for (int t = 0; t < tiles; ++t)
     if (first + t < l.max_tiles) l.tiles[first + t] = TileEntry{e | tiles << 10, start, rows, first};   // (cannot overflow for consistent offsets)
 }
@@ -818,7 +828,7 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
   MOE_REQUIRE(grid < (1ll << 30), MOE_ERR_BAD_SHAPE, "%s: %lld work items exceed the grid limit", what, grid);
   if (grid == 0) return MOE_OK;
   if (l.hdr && !rt->list_tile_rows)
-    hipLaunchKernelGGL(build_tiles_kernel, dim3(1), dim3(1024), 0, s, rt->group_offsets, rt->E, l);
+    hipLaunchKernelGGL(build_tiles_kernel, dim3(1), dim3(1024), 0, s, rt->group_offsets, rt->E, rt->R, l);
   static std::atomic<unsigned long long> lds_raised[2] = {};
   auto* kernel = dn ? grouped_gemm_kernel<MODE, true> : grouped_gemm_kernel<MODE, false>;
   if (int rc = moe_raise_lds_limit((const void*)kernel, CLS_LDS_BYTES, lds_raised[dn != nullptr])) return rc;

@@ -189,3 +189,23 @@ def test_scale_layouts_of_middle_sized_batches_give_the_same_bits(jg, M, E):
     whole = jg.moe_experts(x, lg, **kw)
     assert torch.equal(whole, jg.moe_experts(x, lg, return_debug=True, **kw)[0])      # (h scales row-major)
     assert torch.equal(whole[:400], jg.moe_experts(x[:400].contiguous(), lg[:400].contiguous(), **kw))
+
+
+@pytest.mark.parametrize("E,sizes", [(32, [0, 200, 0, 1, 40] + [0] * 26 + [15]), (32, [0, 200, 0, 1, 40] + [0] * 26 + [16]), (1, [8]), (1, [9])])
+def test_work_lists_of_few_and_more_rows_give_the_same_bits(jg, E, sizes):
+    """8 rows an expert and one more: the two orders of the row-tile list (an expert of several tiles among empty ones)."""
+    import torch
+    print("work list", E, sum(sizes), flush=True)
+    D, I = 512, 256
+    params, rand = _layer(jg, D, E, I, 0, E)
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    xq, sx = jg.quant_act(rand(int(off[-1]), D))
+    hq, sh = jg.gemm_gateup_swiglu(xq, sx, params["gate_proj"], params["up_proj"], H.to_cuda(off))
+    y = jg.gemm_down(hq, sh, params["down_proj"], H.to_cuda(off))
+    for e in np.flatnonzero(sizes):
+        lo, hi = int(off[e]), int(off[e + 1])
+        one = {n: {k: v[e:e + 1] for k, v in params[n + "_proj"].items()} for n in ("gate", "up", "down")}
+        o1 = H.to_cuda(np.array([0, hi - lo], np.int32))
+        hq1, sh1 = jg.gemm_gateup_swiglu(xq[lo:hi], sx[lo:hi].clone(), one["gate"], one["up"], o1)
+        assert torch.equal(hq1.view(torch.uint8), hq[lo:hi].view(torch.uint8)) and torch.equal(sh1, sh[lo:hi]), f"expert {e}: h"
+        assert torch.equal(jg.gemm_down(hq1, sh1, one["down"], o1), y[lo:hi]), f"expert {e}: y"
