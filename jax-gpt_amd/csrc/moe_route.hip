@@ -117,8 +117,10 @@ __device__ __forceinline__ int route_softmax_token(const RouteArgs& a, const flo
     const int e = lane + 64 * s;
     v[s] = e < a.E ? row[e] : -INFINITY;
     key[s] = e < a.E ? make_key(v[s]) : 0u;
-    top = max(top, key[s]);
+    top = max(top, v[s] == v[s] ? key[s] : 0u);   // (a NaN ranks like any other value but is nobody's maximum: see below)
   }
+  // A NaN logit counts as exp_det's lower end and leaves the other experts' weights alone; as the maximum it would make
+  // every difference a NaN, every exponential that lower end, and all k weights equal.
   const float mx = key_value(wave_max(top));
   float part = 0.f;
 #pragma unroll

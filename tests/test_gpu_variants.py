@@ -140,6 +140,27 @@ def test_ready_logits_routed_and_sorted_in_one_launch_or_two(jg, M, E, k):
         assert np.array_equal(dbg[name].cpu().numpy(), ref[name]), name
 
 
+@pytest.mark.parametrize("E,k", [(32, 2), (130, 8), (1000, 4)])
+def test_nan_logits_leave_the_other_weights_alone(jg, E, k):
+    """A NaN's key ranks above (sign bit clear) or below every number; its probability is exp_det's lower end and the
+    others' are those of the numbers alone."""
+    print("NaN logits", E, k, flush=True)
+    rng = H.rng_for(E)
+    logits = rng.standard_normal((9, E), dtype=np.float32)
+    for t in range(8):
+        logits[t, rng.integers(E)] = np.nan if t % 2 else -np.nan
+    logits[7] = np.nan
+    idx, w = (a.cpu().numpy() for a in jg.route_softmax_topk(H.to_cuda(logits), k))
+    nan = np.isnan(logits)
+    rank = np.where(nan, np.where(np.signbit(logits), -np.inf, np.inf), logits)
+    assert np.array_equal(idx, np.argsort(-rank, axis=1, kind="stable")[:, :k])
+    number = np.where(nan, np.float32(-np.inf), logits)
+    number[7] = 0                                            # (no number at all: every expert the same)
+    e = O.exp_det(number - number.max(axis=1, keepdims=True))
+    p = np.take_along_axis(e / e.sum(axis=1, keepdims=True, dtype=np.float32), idx, axis=1)
+    assert np.allclose(w, p / p.sum(axis=1, keepdims=True), rtol=2e-6, atol=1e-9)
+
+
 @pytest.mark.parametrize("M,D", [(2, 2048), (2, 2176), (3, 4096), (1, 4224), (300, 1024)])
 def test_rmsnorm_row_lengths(jg, M, D):
     check_rmsnorm(jg, M, D)
