@@ -269,7 +269,8 @@ __device__ __forceinline__ void sum_partials(const float* p, size_t slice, int s
 //    are contiguous in every slice: independent coalesced loads, see sum_partials) and the waves then read the rounded
 //    logits from LDS.  One wave summing its own token one load at a time took 87 us for 32 tokens of 513 columns in
 //    32 slices, most of the layer's overhead; this way 9 us.
-//  - chunk_hist: the workgroup's selections are counted for the sort by expert (one row of E counts per workgroup).
+//  - chunk_hist: the workgroup's selections are counted for the sort by expert (one row of E counts per workgroup;
+//    not where so few rows would leave CUs idle, see moe_route_impl).
 //  - sort_here (one workgroup routes the whole batch): the sort itself follows in the same launch.
 //  - the blocks behind the routing blocks quantise the activations: independent work, one launch less.
 struct RouteJob {
@@ -333,6 +334,8 @@ __global__ __launch_bounds__(1024) void route_kernel(const RouteArgs a, const Ro
   }
 }
 
+constexpr int kCUs = 256;
+
 int check_route_args(int routing, const RouteArgs& a) {
   const LogitSource& src = a.src;
   const int M = a.M, E = a.E, k = a.k;
@@ -373,21 +376,30 @@ int moe_route_impl(int routing, const RouteArgs& a, const QuantJob* quant, const
   if (a.M == 0) return MOE_OK;
   const int R = a.M * a.k;
   RouteJob job{};
-  // Partial sums: a token per workgroup while there are few tokens (the summing is the work then); ready logits: a
-  // token per wave.  Many tokens: as many per workgroup as keep the sort's histograms few.
-  const int max_chunks = moe_permute_max_chunks(a.E);
-  int tpb = a.src.partial ? 1 : 4;
-  if ((a.M + max_chunks - 1) / max_chunks > tpb) tpb = (a.M + max_chunks - 1) / max_chunks;
   // One workgroup takes a batch whose partial sums (if any) it can add about as fast as many would: the sort needs no
   // launch of its own then.
   const bool sort_here = sort && route_sorts_here(a.M, a.k, a.src.partial) && R <= kSmallRows &&
                   (!a.src.partial || (long long)a.M * a.src.N * a.src.splits <= 65536);
+  const bool one_chunk = R <= kSmallRows;   // the placing kernel counts such a list itself
+  // Tokens per workgroup: one per wave, or one in all while there are few and their partial sums are the work (router
+  // of 4096 x 256 and routing, one token against four: 64 tokens 11.8 / 15.0 us, 1024 21.4 / 22.5, 2048 24.7 / 22.4).
+  int tpb = a.src.partial && a.M <= 1024 ? 1 : 4;
+  bool counts = sort && !sort_here && !one_chunk;
+  if (counts) {
+    // A workgroup that counts its selections for the sort owns a histogram, and those are few (moe_permute_max_chunks):
+    // 256, a workgroup of 16 waves on every CU, up to 256 experts, 64 for 1024.  Where that leaves CUs idle, the
+    // selections are counted by the sort's own first launch.  Ready logits, counted here / there: 300 experts, 1024
+    // tokens 39.4 / 36.3 us of a small layer, 8192 87.2 / 84.7; 512 experts, 4096 tokens 59.3 / 53.2; 1024 experts, 512
+    // tokens 53.9 / 52.4, 8192 163.7 / 93.3 (partial sums 231 / 114).  256 experts, 8192 tokens: 82.6 / 81.7.
+    const int max_chunks = moe_permute_max_chunks(a.E);
+    if (max_chunks < kCUs && a.M > 4 * max_chunks) counts = false;
+    else if ((a.M + max_chunks - 1) / max_chunks > tpb) tpb = (a.M + max_chunks - 1) / max_chunks;
+  }
   if (sort_here) tpb = a.M;
   const int threads = sort_here || tpb >= 8 ? 1024 : 256;
   job.tokens_per_block = tpb;
   job.blocks = (a.M + tpb - 1) / tpb;
-  const bool one_chunk = R <= kSmallRows;   // the placing kernel counts such a list itself
-  job.chunk_hist = sort && !sort_here && !one_chunk ? (int32_t*)permute_ws : nullptr;
+  job.chunk_hist = counts ? (int32_t*)permute_ws : nullptr;
   job.batch = tpb;
   size_t ints = (sort_here ? kSmallRows : 0) + (size_t)a.E;
   size_t tail = 0;
@@ -411,6 +423,7 @@ int moe_route_impl(int routing, const RouteArgs& a, const QuantJob* quant, const
   if (int rc = moe_check_hip(hipGetLastError(), "route launch")) return rc;
   if (!sort || sort_here) return MOE_OK;
   if (one_chunk) return moe_permute_place(a.idx, R, a.E, kSmallRows, 1, nullptr, o, nullptr, stream);
+  if (!counts) return moe_permute_impl(a.idx, a.M, a.k, a.E, o, permute_ws, permute_ws_bytes, nullptr, stream);
   return moe_permute_place(a.idx, R, a.E, tpb * a.k, job.blocks, job.chunk_hist, o, nullptr, stream);
 }
 

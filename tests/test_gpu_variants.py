@@ -99,6 +99,8 @@ def test_shared_expert_beside_the_routing_gives_the_bits_of_the_joint_launches(j
     (33, 1000, 32, 1536),                    # eight counting waves, 12 slices
     (70, 8, 2, 256), (2100, 33, 1, 1280),    # 3 waves of entries; several chunks, experts not a multiple of four
     (1100, 1024, 4, 256),
+    (872, 300, 3, 128), (873, 300, 3, 128),  # counted for the sort by the routing launch, and by the sort's own
+    (1024, 64, 3, 128), (1026, 64, 3, 128),  # a token per workgroup and four (two left over) where nothing is sorted
 ])
 def test_routing_inside_the_layer_is_exact(jg, M, E, k, D):
     """Selection and sort against the oracle on the logits that the layer ranked, which are the router's own."""
@@ -126,7 +128,7 @@ def test_routing_inside_the_layer_is_exact(jg, M, E, k, D):
     assert torch.equal(jg.expert_forward_single(x, *sel, params["gate_proj"], params["up_proj"], params["down_proj"]), out)
 
 
-@pytest.mark.parametrize("M,E,k", [(9, 8, 2), (32, 8, 2), (33, 8, 2), (22, 40, 3), (17, 300, 4)])
+@pytest.mark.parametrize("M,E,k", [(9, 8, 2), (32, 8, 2), (33, 8, 2), (22, 40, 3), (17, 300, 4), (513, 512, 5), (2049, 513, 1)])
 def test_ready_logits_routed_and_sorted_in_one_launch_or_two(jg, M, E, k):
     print("routing of ready logits", M, E, k, flush=True)
     params, rand = _layer(jg, 128, E, 128, 0, M)
