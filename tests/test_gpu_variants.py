@@ -10,7 +10,7 @@ import pytest
 
 from oracle import moe_oracle as O
 from tests import helpers as H
-from tests.test_gpu_parity import _check_logits, _ragged_case, jg, test_rmsnorm_quant_vs_oracle as check_rmsnorm  # noqa: F401
+from tests.test_gpu_parity import _check_logits, _ragged_case, jg, test_rmsnorm_quant_vs_oracle as check_rmsnorm, test_route_sigmoid_grouped_bit_exact as check_grouped  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
@@ -140,6 +140,12 @@ def test_ready_logits_routed_and_sorted_in_one_launch_or_two(jg, M, E, k):
     ref = O.sort_and_group(idx, E)
     for name in ("group_sizes", "sorted_token_ids", "inv_perm"):
         assert np.array_equal(dbg[name].cpu().numpy(), ref[name]), name
+
+
+@pytest.mark.parametrize("E,G,TG,k", [(60, 3, 2, 4), (300, 4, 2, 8), (640, 4, 1, 8), (1000, 10, 3, 32), (64, 64, 5, 5), (1024, 2, 1, 6), (130, 13, 4, 7)])
+def test_groups_across_lanes(jg, E, G, TG, k):
+    """Groups that are no run of 1, 2, 4, 8 or 16 lanes are scored one at a time (equal scores among them)."""
+    check_grouped(jg, 37, E, G, TG, k, 1.0)
 
 
 @pytest.mark.parametrize("E,k", [(32, 2), (130, 8), (1000, 4)])
