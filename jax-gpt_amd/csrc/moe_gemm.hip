@@ -154,8 +154,7 @@ template <int XF, int MODE = MODE_GATEUP, bool ONCE = true> struct Cls {
   // The weight copies' cache policy.  ONCE: the item's expert has one row tile (or two that stay close, see the
   // dispatch), so that its weight lines are fetched once and marked non-temporal, which leaves the memory-side cache
   // alone.  A read-only stream reaches 7.1 TB/s that way and 6.3 without (4 GiB, any grid); 64 tokens of the
-  // DeepSeek-V3 layer went from 1010 to 864 us, gate/up and down at 6.7 TB/s instead of 5.8.  Tiles of up to 128
-  // rows are their expert's only one in every launch that fills the chip, so these classes exist in this form only.
+  // DeepSeek-V3 layer went from 1010 to 864 us, gate/up and down at 6.7 TB/s instead of 5.8.
   static constexpr bool W_ONCE = ONCE;
   static constexpr int X_STAGE_S_OFF = BM * BK;                // the scales behind the tile
   // + 256: every copying wave copies 64 scale slots from its first one on (no lane mask, which would cut the
@@ -736,7 +735,10 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
   // Two row tiles of an expert read the same weight lines; over a short K they stay close enough to find them in L2
   // (non-temporal lines leave it first), over a long one the later tile needs the memory-side cache.  Qwen3-MoE, 4096
   // tokens (K = 2048, 768): 269 us with one-tile experts alone marked, 261 with two; DeepSeek-V3 gate/up (K = 7168) at
-  // 4096 tokens: 2426 / 2438 us of the step; all experts whatever their tiles: 8192 tokens 3731 / 3946 us.
+  // 4096 tokens: 2426 / 2438 us of the step; all experts whatever their tiles: 8192 tokens 3731 / 3946 us.  Tiles of
+  // 96 and 128 rows come in numbers where a small problem is cut (marked whatever their number against this rule: tiny
+  // layer, 2048 tokens 52.1 / 48.9 us, 1024 tokens 34.1 / 33.5).  Those of up to 64 rows are marked always: shards of 64
+  // to 4800 rows are the same within 0.3 % and a choice costs a launch of such tiles 0.5 us (Qwen3-MoE, 33 tokens).
   const bool once = __builtin_amdgcn_readfirstlane(item.tiles) <= (K <= 2048 ? 2 : 1);
 #define MOE_ITEM(XF, ONCE) item_body<MODE, XF, ONCE>(item, lds, xq, sx, row_ids, w0, sw0, w1, sw1, K, N, out, out_scale, sc)
 #define MOE_CLASS(XF) if (once) MOE_ITEM(XF, true); else MOE_ITEM(XF, false); break
@@ -746,8 +748,8 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
     case 7: MOE_CLASS(7);
     case 6: MOE_CLASS(6);
     case 5: MOE_CLASS(5);
-    case 4: MOE_ITEM(4, true); break;
-    case 3: MOE_ITEM(3, true); break;
+    case 4: MOE_CLASS(4);
+    case 3: MOE_CLASS(3);
     case 2: MOE_ITEM(2, true); break;
     default: MOE_ITEM(1, true); break;
   }
