@@ -210,8 +210,14 @@ constexpr int CLS_RING = cmax(cmax(cmax(cmax(Cls<9>::RING_BYTES, Cls<8>::RING_BY
                               cmax(cmax(Cls<4>::RING_BYTES, Cls<3>::RING_BYTES), cmax(Cls<2>::RING_BYTES, Cls<1>::RING_BYTES)));
 constexpr int CLS_WSCALE_OFF = CLS_RING;                       // [2][MAX_KB] weight block scales of the work item
 constexpr int CLS_FLAG_OFF = CLS_WSCALE_OFF + 2 * MAX_KB * 4;  // [4] early_flag: the step whose weight fragments wave (wi, 1) holds, + 1
-constexpr int CLS_LDS_BYTES = CLS_FLAG_OFF + 16;              // 160016; the epilogues stage through the ring (<= 128 KB)
+constexpr int CLS_LDS_BYTES = CLS_FLAG_OFF + 16;              // 160016
 static_assert(CLS_LDS_BYTES <= 160 * 1024, "LDS");
+// The epilogues stage their results where the rings were, all of CLS_RING whatever the class's own rings take: gate/up
+// four f32 maxima and 128 codes a row, down 256 bf16 a row -- 144 KB at 288 rows, whose rings are 139 KB.
+template <int XF> constexpr bool epilogue_fits() {
+  return Cls<XF>::BM * (4 * 4 + BK) <= CLS_RING && Cls<XF>::BM * 256 * 2 <= CLS_RING;
+}
+static_assert(epilogue_fits<9>(), "the tallest tile's epilogue stages inside the rings' space");
 
 struct Item { int expert, row_start, row_count, col_block, tiles; };
 
