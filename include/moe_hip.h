@@ -50,6 +50,7 @@ extern "C" {
 
 typedef void* moe_stream_t; /* a hipStream_t */
 
+/* 7.  Raised whenever an entry point is added or its arguments change (7: moe_routing, moe_forward_f32, moe_forward_selected). */
 MOE_API int moe_abi_version(void);
 MOE_API const char* moe_last_error(void);
 

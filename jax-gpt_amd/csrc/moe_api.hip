@@ -24,7 +24,7 @@ int moe_check_hip(hipError_t e, const char* what) {
   return moe_set_error(MOE_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
 }
 
-extern "C" int moe_abi_version(void) { return 6; }
+extern "C" int moe_abi_version(void) { return 7; }
 extern "C" const char* moe_last_error(void) { return g_err; }
 
 namespace {
