@@ -187,15 +187,15 @@ def test_config3_deepseek_v3_prefill(env, dsv3_layer):
 
 
 def _check_whole_expert(jg, torch, cfg, layer, dbg, x):
-    """Every row of one expert that is cut into two row tiles (257 .. 512 rows; both tiles, their first and last
+    """Every row of one expert that is cut into two row tiles (289 .. 576 rows; both tiles, their first and last
     rows, the rows either side of the cut) through the stage entry points at K = 7168: the gate/up GEMM's h against
     the oracle's, and the down GEMM's rows against the oracle continued from that h, to the plain tolerance."""
     experts = layer[0]
     E, D, I = cfg["E"], cfg["D"], cfg["I"]
     gs = dbg["group_sizes"].cpu().numpy()
-    cand = np.nonzero((gs > 256) & (gs <= 512))[0]
+    cand = np.nonzero((gs > 288) & (gs <= 576))[0]
     assert cand.size, "no expert with two row tiles in this routing"
-    e = int(cand[np.argmin(np.abs(gs[cand] - 292))])
+    e = int(cand[np.argmin(gs[cand])])
     off = np.concatenate([[0], np.cumsum(gs)]).astype(np.int32)
     a, b = int(off[e]), int(off[e + 1])
     _say(f"   whole expert {e}: rows {a}..{b} ({b - a} rows, two row tiles)")

@@ -190,10 +190,10 @@ def test_block_major_scales_give_the_same_bits(jg, E, D, I, sizes, gather):
     (8, 512, 1024, [64] * 8),
     (3, 384, 384, [257, 0, 1]),           # D % 256 != 0: the down GEMM's last column block is half full
     (6, 2048, 768, [300, 0, 0, 129, 7, 64]),
-    (8, 256, 256, [70, 0, 1, 33, 0, 16, 0, 0]),   # a few rows per expert: the 32- and 64-row tile classes, empty experts between
-    (2, 256, 256, [300, 150]),                    # two row tiles for one expert (near-equal cut), one 160-row tile for the other
-    (2, 256, 256, [4200, 100]),                   # 17 row tiles: the column blocks are walked once per group of 8-9 row tiles
-    (3, 1024, 256, [256, 0, 510]),                # 225-256 row tiles over 8 K steps: gate/up refills a weight stage inside the step that reads it
+    (8, 256, 256, [70, 0, 1, 33, 0, 16, 0, 0]),   # a few rows per expert: tiles of up to 96 rows, empty experts between
+    (2, 256, 256, [300, 150]),                    # (a problem this small is cut into 32-row tiles: ten and five)
+    (2, 256, 256, [4200, 100]),                   # 66 and 132 row tiles: the column blocks are walked once per group of 8 to 11 row tiles
+    (3, 1024, 256, [256, 0, 510]),                # 8 K steps, 8 and 16 row tiles
     # the smallest experts form a pool that every XCD draws from behind its fixed share: the eight smallest of the ranking here ...
     (64, 256, 128, [500] * 48 + [3, 40, 17, 0, 1, 33, 25, 8, 12, 0, 31, 2, 64, 5, 9, 20]),
     # ... and experts of two row tiles each in the pool here (of the ranking's last three groups of eight, one fits the pool's limit)
@@ -231,11 +231,14 @@ def test_gateup_full_height_tiles_same_bits_whatever_the_timing(jg):
     alone on an idle GPU and amid 63 others that keep every CU and the memory busy, the busy launch several times."""
     import torch
     _say("gateup timing independence")
-    E, D, I = 64, 2048, 256
+    E, D, I = 64, 2048, 1536      # 64 experts x 12 column blocks: fewer than 768 work items are cut into shorter tiles
     sizes = [250 + (i % 7) for i in range(E)]
-    off, xq, sx, ex = _ragged_case(650, E, D, I, sizes)
-    dex = H.experts_to_cuda(ex)
-    dxq, dsx, doff = H.to_cuda(xq), H.to_cuda(sx), H.to_cuda(off)
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(650)
+    rand = lambda *s: torch.randn(s, dtype=torch.bfloat16, device="cuda", generator=gen)
+    dex = {n: jg.quantize_weight_block(rand(E, I, D).mul_(0.03)) for n in ("gate_proj", "up_proj")}
+    (dxq, dsx), doff = jg.quant_act(rand(int(off[-1]), D)), H.to_cuda(off)
     hq0, sh0 = jg.gemm_gateup_swiglu(dxq, dsx, dex["gate_proj"], dex["up_proj"], doff)
     for _ in range(5):
         hq, sh = jg.gemm_gateup_swiglu(dxq, dsx, dex["gate_proj"], dex["up_proj"], doff)

@@ -18,6 +18,7 @@ HEIGHTS = [257, 288, 289, 1, 32, 33, 576, 577, 0, 97, 128, 129, 160, 161, 192, 2
 
 
 @pytest.mark.parametrize("E,D,I,sizes", [
+    (96, 1024, 1024, HEIGHTS),    # 8 K steps: little more than the rings' depth
     (96, 2048, 1024, HEIGHTS),    # full tiles up to 288 rows; two tiles share their lines (K = 2048)
     (64, 2304, 1536, HEIGHTS),    # K above 2048: two tiles do not; the down GEMM has fewer items and shorter tiles
     (64, 2304, 2048, [1, 31, 32, 33, 40, 64, 65, 96, 97, 128]),   # a weight stream with outputs above 4 MB: written through
@@ -91,6 +92,71 @@ def test_shared_expert_beside_the_routing_gives_the_bits_of_the_joint_launches(j
         torch.cuda.synchronize()
         assert torch.equal(out, full), f"replay {i}"
         assert torch.equal(jg.moe_experts(x, lg, **kw), full)
+
+
+@pytest.mark.parametrize("SI", [256, 0])
+def test_large_f32_activations_give_the_bits_of_their_bf16_rounding(jg, SI):
+    """Above 16 M activation elements, with a shared expert: the quantiser on the side stream feeds the router, and the
+    combine reads f32.  Eager, and every replay of a captured graph with eager calls between."""
+    import torch
+    print("large f32 activations", SI, flush=True)
+    D, k = 4096, 2
+    params, rand = _layer(jg, D, 8, 128, SI, 5)
+    M = (1 << 24) // D + 41
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(6)
+    x = torch.randn((1, M, D), device="cuda", generator=gen)
+    norm = rand(D).float() * 0.1
+    xb = x.to(torch.bfloat16)
+    for call in (lambda v: jg.moe_layer(v, params, k), lambda v: jg.moe_sublayer(v, norm, params, k)):
+        want = call(xb).float()
+        assert torch.equal(call(x), want)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = call(x)
+        for i in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), f"replay {i}"
+            assert torch.equal(call(x), want)
+
+
+def test_large_layer_with_its_router_is_its_stages(jg):
+    """The forked path with the router inside: its logits and gate are the router's own, its rows those of a smaller batch
+    that runs the shared expert in the routed launches, its output their combine."""
+    import torch
+    print("large layer with its router", flush=True)
+    D, k = 4096, 2
+    params, rand = _layer(jg, D, 8, 128, 256, 7)
+    x = rand((1 << 24) // D + 41, D)
+    ex, sh = ({n: params[p + n] for n in ("gate_proj", "up_proj", "down_proj")} for p in ("", "shared_"))
+    out, dbg = jg.moe_experts(x, None, top_k=k, experts=ex, shared=sh, gate_weight=params["gate_weight"],
+                              shared_expert_gate_weight=params["shared_expert_gate_weight"], return_debug=True)
+    logits, gate = jg.router_logits(x, params["gate_weight"], params["shared_expert_gate_weight"])
+    assert torch.equal(dbg["logits"], logits) and torch.equal(dbg["shared_gate"], gate)
+    idx, w = jg.route_softmax_topk(logits, k)
+    assert torch.equal(dbg["indices"], idx) and torch.equal(dbg["weights"], w)
+    _, part = jg.moe_experts(x[:1000].contiguous(), logits[:1000].contiguous(), top_k=k, experts=ex, shared=sh, return_debug=True)
+    rows = lambda d: d["y"][d["inv_perm"][:1000 * k].long()]
+    assert torch.equal(rows(dbg), rows(part)) and torch.equal(dbg["ys"][:1000], part["ys"])
+    assert torch.equal(out, jg.combine(dbg["y"], w, dbg["inv_perm"], dbg["ys"], gate))
+    assert torch.equal(jg.moe_layer(x[None], params, k)[0], out)      # (debug arrays keep h scales row-major)
+
+
+@pytest.mark.parametrize("M", [5, 300, (1 << 24) // 4096 + 9])
+def test_given_selection_with_a_shared_expert(jg, M):
+    """moe_forward_selected beside a shared expert, in the routed launches and forked: the routed call's bits."""
+    import torch
+    from jax_gpt_amd import moe
+    print("given selection with a shared expert", M, flush=True)
+    D, k = 4096, 2
+    params, rand = _layer(jg, D, 8, 128, 256, M)
+    x, lg = rand(M, D), rand(M, 8).float()
+    ex, sh = ({n: params[p + n] for n in ("gate_proj", "up_proj", "down_proj")} for p in ("", "shared_"))
+    want = jg.moe_experts(x, lg, top_k=k, experts=ex, shared=sh)
+    assert torch.equal(moe._forward(x, None, k, ex, shared=sh, selected=jg.route_softmax_topk(lg, k)), want)
 
 
 @pytest.mark.parametrize("M,E,k,D", [
