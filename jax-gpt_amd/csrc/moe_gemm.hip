@@ -151,10 +151,11 @@ template <int XF, int MODE = MODE_GATEUP, bool ONCE = true> struct Cls {
   static constexpr bool W_EARLY = XF >= 8 && MODE == MODE_GATEUP;
   static constexpr int EARLY_G = 3;   // the group behind which the weight copies of a W_EARLY step begin (2 and 4: within 1 %)
   static constexpr int X_PRE = X_NST - 1, W_PRE = W_NST - 1 + (W_EARLY ? 1 : 0);   // steps that a copy runs ahead of its use
-  // The weight copies' cache policy.  ONCE: the item's expert has one row tile (or two that stay close, see the
-  // dispatch), so that its weight lines are fetched once and marked non-temporal, which leaves the memory-side cache
-  // alone.  A read-only stream reaches 7.1 TB/s that way and 6.3 without (4 GiB, any grid); 64 tokens of the
-  // DeepSeek-V3 layer went from 1010 to 864 us, gate/up and down at 6.7 TB/s instead of 5.8.
+  // The weight copies' cache policy.  ONCE: the item's expert has one row tile (or two that stay close, see
+  // grouped_gemm_kernel) and comes from memory (launch()), so that its weight lines are fetched once and marked
+  // non-temporal, which leaves the memory-side cache alone.  A read-only stream reaches 7.1 TB/s that way and 6.3 without
+  // (4 GiB, any grid); 64 tokens of the DeepSeek-V3 layer went from 1010 to 864 us, gate/up and down at 6.7 TB/s instead
+  // of 5.8.
   static constexpr bool W_ONCE = ONCE;
   static constexpr int X_STAGE_S_OFF = BM * BK;                // the scales behind the tile
   // + 256: every copying wave copies 64 scale slots from its first one on (no lane mask, which would cut the
@@ -638,6 +639,9 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
   }
 }
 
+// row tiles of an expert up to which its weight lines are marked non-temporal (grouped_gemm_kernel)
+__host__ __device__ inline int once_tiles(int K) { return K <= 2048 ? 2 : 1; }
+
 // Column block and row tile of the `local`-th work item of an expert of nt row tiles and ncb column blocks.
 __device__ __forceinline__ void expert_item(int local, int nt, int ncb, int& col_block, int& rt) {
   if (nt < 16) {
@@ -675,7 +679,9 @@ __device__ __forceinline__ void expert_item(int local, int nt, int ncb, int& col
 // launches, the second stream and the events between them cost it more than the arithmetic.  DENSE false: routed
 // items only, as a kernel of its own, because choosing between the two operand sets costs every item of a large
 // launch some 0.7 us (0.8 % of the prefill step).
-template <int MODE, bool DENSE>
+// STREAM: weights come from memory and most experts have one row tile, so items mark their weight lines non-temporal
+// where that pays.  Otherwise every copy is a plain one (launch()).
+template <int MODE, bool DENSE, bool STREAM>
 __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands routed, TileHeader* hdr,
                                                             const TileEntry* __restrict__ tiles, const GemmOperands dense,
                                                             int dense_rows, int dense_tiles, int dense_blocks) {
@@ -738,28 +744,40 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
   float* out_scale = is_dense ? dense.out_scale : routed.out_scale;
   const GemmScales sc = is_dense ? dense.sc : routed.sc;
   const int rows = __builtin_amdgcn_readfirstlane(item.row_count);
-  // Two row tiles of an expert read the same weight lines; over a short K they stay close enough to find them in L2
-  // (non-temporal lines leave it first), over a long one the later tile needs the memory-side cache.  Qwen3-MoE, 4096
-  // tokens (K = 2048, 768): 269 us with one-tile experts alone marked, 261 with two; DeepSeek-V3 gate/up (K = 7168) at
-  // 4096 tokens: 2426 / 2438 us of the step; all experts whatever their tiles: 8192 tokens 3731 / 3946 us.  Tiles of
-  // 96 and 128 rows come in numbers where a small problem is cut (marked whatever their number against this rule: tiny
-  // layer, 2048 tokens 52.1 / 48.9 us, 1024 tokens 34.1 / 33.5).  Those of up to 64 rows are marked always: shards of 64
-  // to 4800 rows are the same within 0.3 % and a choice costs a launch of such tiles 0.5 us (Qwen3-MoE, 33 tokens).
-  const bool once = __builtin_amdgcn_readfirstlane(item.tiles) <= (K <= 2048 ? 2 : 1);
 #define MOE_ITEM(XF, ONCE) item_body<MODE, XF, ONCE>(item, lds, xq, sx, row_ids, w0, sw0, w1, sw1, K, N, out, out_scale, sc)
+  if constexpr (STREAM) {
+    // Two row tiles of an expert read the same weight lines; over a short K they stay close enough to find them in L2
+    // (non-temporal lines leave it first), over a long one the later tile needs the memory-side cache.  Qwen3-MoE, 4096
+    // tokens (K = 2048, 768): 269 us with one-tile experts alone marked, 261 with two; DeepSeek-V3 gate/up (K = 7168) at
+    // 4096 tokens: 2426 / 2438 us of the step; all experts whatever their tiles: 8192 tokens 3731 / 3946 us.  Tiles of up
+    // to 128 rows are their expert's only one in most of these launches (the host sees to it) and are always marked.
+    const bool once = __builtin_amdgcn_readfirstlane(item.tiles) <= once_tiles(K);
 #define MOE_CLASS(XF) if (once) MOE_ITEM(XF, true); else MOE_ITEM(XF, false); break
-  switch ((rows + 31) >> 5) {
-    case 9: MOE_CLASS(9);
-    case 8: MOE_CLASS(8);
-    case 7: MOE_CLASS(7);
-    case 6: MOE_CLASS(6);
-    case 5: MOE_CLASS(5);
-    case 4: MOE_CLASS(4);
-    case 3: MOE_CLASS(3);
-    case 2: MOE_ITEM(2, true); break;
-    default: MOE_ITEM(1, true); break;
-  }
+    switch ((rows + 31) >> 5) {
+      case 9: MOE_CLASS(9);
+      case 8: MOE_CLASS(8);
+      case 7: MOE_CLASS(7);
+      case 6: MOE_CLASS(6);
+      case 5: MOE_CLASS(5);
+      case 4: MOE_ITEM(4, true); break;
+      case 3: MOE_ITEM(3, true); break;
+      case 2: MOE_ITEM(2, true); break;
+      default: MOE_ITEM(1, true); break;
+    }
 #undef MOE_CLASS
+  } else {
+    switch ((rows + 31) >> 5) {
+      case 9: MOE_ITEM(9, false); break;
+      case 8: MOE_ITEM(8, false); break;
+      case 7: MOE_ITEM(7, false); break;
+      case 6: MOE_ITEM(6, false); break;
+      case 5: MOE_ITEM(5, false); break;
+      case 4: MOE_ITEM(4, false); break;
+      case 3: MOE_ITEM(3, false); break;
+      case 2: MOE_ITEM(2, false); break;
+      default: MOE_ITEM(1, false); break;
+    }
+  }
 #undef MOE_ITEM
 }
 int col_blocks(int mode, int N) { return mode == MODE_GATEUP ? N / 128 : (N + 255) / 256; }
@@ -837,9 +855,21 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
   if (grid == 0) return MOE_OK;
   if (l.hdr && !rt->list_tile_rows)
     hipLaunchKernelGGL(build_tiles_kernel, dim3(1), dim3(1024), 0, s, rt->group_offsets, rt->E, rt->R, l);
-  static std::atomic<unsigned long long> lds_raised[2] = {};
-  auto* kernel = dn ? grouped_gemm_kernel<MODE, true> : grouped_gemm_kernel<MODE, false>;
-  if (int rc = moe_raise_lds_limit((const void*)kernel, CLS_LDS_BYTES, lds_raised[dn != nullptr])) return rc;
+  // Non-temporal weight copies gain a stream from memory 2 to 3 % (four experts of 7168 x 2048 among others, 1 row each:
+  // 46.6 -> 45.4 us, 64 tokens of the DeepSeek-V3 layer 12 %) and cost
+  //  - a third where the memory-side cache (256 MB) still holds the weights from the call before (the same four experts
+  //    over and over 29.3 / 44.9 us; tiny layer, 64 tokens 23.9 / 26.0, 256 25.3 / 27.3; mini sublayer, 64 tokens 36.9 /
+  //    39.5, 256 37.8 / 40.6): layers of up to 192 MB, three projections of this size, go without;
+  //  - as much where the several short tiles of a small problem's experts read the same lines (four experts of 7168 x 2048
+  //    from memory, 40 rows each 49.7 / 55.0 us, 200 51.8 / 60.6; tiny layer, 2048 tokens 48.9 / 52.1).
+  const long long layer_bytes = (rt ? 3ll * rt->E * rt->op.N * rt->op.K : 0) + (dn ? 3ll * dn->op.N * dn->op.K : 0);
+  const bool shared_lines = l.hdr ? l.tile_rows <= 128 && rt->R > (long long)once_tiles(routed.K) * l.tile_rows * rt->E
+                                  : dense_tiles > once_tiles(dense.K) && dense_rows <= 128 * dense_tiles;
+  const bool stream = layer_bytes > (192ll << 20) && !shared_lines;
+  static std::atomic<unsigned long long> lds_raised[4] = {};
+  auto* kernel = dn ? (stream ? grouped_gemm_kernel<MODE, true, true> : grouped_gemm_kernel<MODE, true, false>)
+                    : (stream ? grouped_gemm_kernel<MODE, false, true> : grouped_gemm_kernel<MODE, false, false>);
+  if (int rc = moe_raise_lds_limit((const void*)kernel, CLS_LDS_BYTES, lds_raised[(dn ? 2 : 0) + stream])) return rc;
   hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(NT), CLS_LDS_BYTES, s, routed, l.hdr, l.tiles, dense, dense_rows,
                      dense_tiles, (int)dense_blocks);
   return moe_check_hip(hipGetLastError(), "gemm launch");

@@ -19,6 +19,8 @@ HEIGHTS = [257, 288, 289, 1, 32, 33, 576, 577, 0, 97, 128, 129, 160, 161, 192, 2
 
 @pytest.mark.parametrize("E,D,I,sizes", [
     (96, 1024, 1024, HEIGHTS),    # 8 K steps: little more than the rings' depth
+    (96, 512, 1024, HEIGHTS),     # weights that the memory-side cache holds: plain copies, tall gate/up tiles ...
+    (96, 2048, 256, HEIGHTS),     # ... and tall down tiles, over 4 and 2 K steps
     (96, 2048, 1024, HEIGHTS),    # full tiles up to 288 rows; two tiles share their lines (K = 2048)
     (64, 2304, 1536, HEIGHTS),    # K above 2048: two tiles do not; the down GEMM has fewer items and shorter tiles
     (64, 2304, 2048, [1, 31, 32, 33, 40, 64, 65, 96, 97, 128]),   # a weight stream with outputs above 4 MB: written through
