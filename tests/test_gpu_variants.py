@@ -288,6 +288,23 @@ def test_scale_layouts_of_middle_sized_batches_give_the_same_bits(jg, M, E):
     assert torch.equal(whole[:400], jg.moe_experts(x[:400].contiguous(), lg[:400].contiguous(), **kw))
 
 
+@pytest.mark.parametrize("R,D,I", [(4100, 256, 8192), (2090, 8192, 256)])
+def test_one_group_of_many_rows_gives_the_bits_of_fewer(jg, R, D, I):
+    """More than 768 work items of one group: its height follows from the rounds that its rows make."""
+    import torch
+    print("one group", R, D, I, flush=True)
+    params, rand = _layer(jg, D, 1, I, 0, R)
+    xq, sx = jg.quant_act(rand(R, D))
+    run = lambda lo, hi: jg.gemm_gateup_swiglu(xq[lo:hi], sx[lo:hi].clone(), params["gate_proj"], params["up_proj"],
+                                               H.to_cuda(np.array([0, hi - lo], np.int32)))
+    hq, sh = run(0, R)
+    y = jg.gemm_down(hq, sh, params["down_proj"], H.to_cuda(np.array([0, R], np.int32)))
+    for lo, hi in ((0, 300), (700, 1300), (R - 33, R)):
+        hq1, sh1 = run(lo, hi)
+        assert torch.equal(hq1.view(torch.uint8), hq[lo:hi].view(torch.uint8)) and torch.equal(sh1, sh[lo:hi])
+        assert torch.equal(jg.gemm_down(hq1, sh1, params["down_proj"], H.to_cuda(np.array([0, hi - lo], np.int32))), y[lo:hi])
+
+
 @pytest.mark.parametrize("D,I,E,sizes", [
     (1024, 1024, 8, [512, 600, 700, 33, 520, 96, 1, 1634]),   # several tiles of 96 to 160 rows an expert
     (512, 256, 32, [0, 200, 0, 1, 40] + [0] * 26 + [15]), (512, 256, 32, [0, 200, 0, 1, 40] + [0] * 26 + [16]),
