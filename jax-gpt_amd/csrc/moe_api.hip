@@ -295,7 +295,7 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
   const bool together = a->SI && !fork;   // the shared expert runs inside the routed launches
   const int tile_rows = moe_gemm_tile_rows(TileShape{R, a->E, {a->I / 128, (a->D + 255) / 256}, {a->D / 128, a->I / 128},
                                                      together ? a->M : 0, {a->SI / 128, (a->D + 255) / 256}});
-  if ((rc = moe_gemm_tile_list(R, a->E, tile_rows, b.gemm_ws, b.gemm_ws_bytes, &tiles))) return join(rc);
+  if ((rc = moe_gemm_tile_list(R, a->E, tile_rows, a->I / 128, (a->D + 255) / 256, b.gemm_ws, b.gemm_ws_bytes, &tiles))) return join(rc);
   const RouteArgs route{src, a->bias, a->M, a->E, a->k, a->renorm, a->n_group, a->topk_group, a->routed_scale, idx, w_own};
   const PermuteOut sort{gsz, b.group_offsets, stid, nullptr, inv, a->k, tiles};
   const QuantJob* carried = quant_in_route ? &quant_job : nullptr;

@@ -74,6 +74,8 @@ struct TileList {
   int tile_rows;      // rows of a full tile: a multiple of 32, at most kTileRows
   TileHeader* hdr;
   TileEntry* tiles;
+  int ncb[2];         // column blocks per row tile of the GEMMs that will read the list (0: none), ...
+  int round_q[2];     // ... and 32 work items in tiles, with kTileQBits fraction bits
 };
 // An expert with `rows` rows gets ceil(rows / tile_rows) row tiles whose heights, counted in units of 32 rows, differ by
 // at most one: no tile computes more than 31 rows of padding, and tiles that share a weight slab take about the same
@@ -151,7 +153,9 @@ __device__ __forceinline__ void moe_scan_1024(int& a, int& b, int& all_a, int& a
   b = in_b - b + (wv ? __builtin_amdgcn_readlane(sum_b, (wv - 1) & 15) : 0);
   __syncthreads();   // (the wave totals may be overwritten)
 }
-__device__ inline int moe_tile_first(int e, int rows, int nt, int* lds_a, int* lds_b, TileHeader* hdr, int max_tiles) {
+__device__ inline int moe_tile_first(int e, int rows, int nt, int* lds_a, int* lds_b, const TileList& l) {
+  TileHeader* const hdr = l.hdr;
+  const int max_tiles = l.max_tiles;
   __shared__ long long cut_q[9];
   __shared__ int tail_tiles[kTailRounds];   // tiles of the last, last but one, ... round of the ranking
   // rank: largest class first, inside a class in any order (1023 = the largest class and everything above it)
@@ -229,7 +233,16 @@ __device__ inline int moe_tile_first(int e, int rows, int nt, int* lds_a, int* l
     cut_q[0] = 0;
     cut_q[8] = (long long)ns << kTileQBits;
     bool fits = ns > 0 && total <= max_tiles;
-    for (int k = 0; k < 8 && fits; ++k) fits = cut_q[k + 1] - cut_q[k] <= moe_xcd_share_cap_q(max_tiles);
+    // A launch of one or two rounds over the CUs ends with whole items: an XCD with 33 of them takes as long as one with
+    // 64.  There no share may hold more than that many rounds' items.  (8 experts of 1024 rows of the tiny layer, 256 items:
+    // 67.5 -> 59.3 us; 9 tiles x 28 columns of 768 to 192 rows 46.8 -> 36.7.  Three rounds of unequal tiles lose by it, an
+    // expert-parallel shard of 8000 rows 481 -> 490.)
+    long long cap = moe_xcd_share_cap_q(max_tiles);
+    for (int g = 0; g < 2; ++g) {
+      const long long rounds = ((long long)n * l.ncb[g] + 255) >> 8;
+      if (rounds == 1 || rounds == 2) cap = min(cap, rounds * l.round_q[g]);
+    }
+    for (int k = 0; k < 8 && fits; ++k) fits = cut_q[k + 1] - cut_q[k] <= cap;
     moe_tile_even_shares(hdr, ns, n);   // (a share beyond what the launch provides workgroups for: equal counts always fit)
     if (fits)
       for (int k = 0; k <= 8; ++k) hdr->xcd_q[k] = cut_q[k];
@@ -298,7 +311,7 @@ int moe_permute_place(const int32_t* idx, int R, int E, int chunk, int n_chunks,
 // own.  moe_gemm_tile_list describes the list the GEMMs of (R rows, E experts) expect in ws, so that the permutation
 // kernels, which hold every expert's row range anyway, can write it (moe_permute_impl) and no launch is spent on it.
 // tile_rows: moe_gemm_tile_rows of the GEMMs that will read it.
-int moe_gemm_tile_list(int R, int E, int tile_rows, void* ws, size_t ws_bytes, TileList* list);
+int moe_gemm_tile_list(int R, int E, int tile_rows, int ncb_gateup, int ncb_down, void* ws, size_t ws_bytes, TileList* list);
 // Rows of a full tile for R rows in E groups and, in the same launches, dense_rows rows of a dense group; [0] gate/up,
 // [1] down: column blocks per row tile and K steps (0: that GEMM does not read the list).
 struct TileShape {

@@ -94,7 +94,7 @@ __global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __rest
     moe_scan_1024(first, unused, all, unused_all);
     if (e == 0) moe_tile_even_shares(l.hdr, min(all, l.max_tiles), min(all, l.max_tiles));
   } else {
-    first = moe_tile_first(e, rows, tiles, s_rows, s_key, l.hdr, l.max_tiles);
+    first = moe_tile_first(e, rows, tiles, s_rows, s_key, l);
   }
   for (int t = 0; t < tiles; ++t)
     if (first + t < l.max_tiles) l.tiles[first + t] = TileEntry{e | tiles << 10, start, rows, first};   // (cannot overflow for consistent offsets)
@@ -786,8 +786,9 @@ int max_tiles_for(int R, int E, int tile_rows) { return (int)(((long long)R + ti
 // fewest work items at which every launch takes full tiles (moe_gemm_tile_rows)
 constexpr int kFullTileItems = 768;
 
-TileList tile_list(void* ws, int R, int E, int tile_rows) {
-  return TileList{max_tiles_for(R, E, tile_rows), tile_rows, (TileHeader*)ws, (TileEntry*)((char*)ws + sizeof(TileHeader))};
+TileList tile_list(void* ws, int R, int E, int tile_rows, int ncb_gateup, int ncb_down) {
+  return TileList{max_tiles_for(R, E, tile_rows), tile_rows, (TileHeader*)ws, (TileEntry*)((char*)ws + sizeof(TileHeader)),
+                  {ncb_gateup, ncb_down}, {(32 << kTileQBits) / (ncb_gateup ? ncb_gateup : 1), (32 << kTileQBits) / (ncb_down ? ncb_down : 1)}};
 }
 
 int check_operands(const GemmOperands& op, int rows, int E, int mode, const char* what) {
@@ -843,7 +844,8 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
     if (rt->R > 0) {
       routed = rt->op;
       routed.sc.out_through = through(rt->R, rt->E, routed.N);
-      l = tile_list(rt->ws, rt->R, rt->E, rt->list_tile_rows ? rt->list_tile_rows : own_tile_rows(rt->R, rt->E, routed));
+      l = tile_list(rt->ws, rt->R, rt->E, rt->list_tile_rows ? rt->list_tile_rows : own_tile_rows(rt->R, rt->E, routed),
+                    col_blocks(MODE, routed.N), 0);   // (one launch reads a list that it builds itself)
       // sized by the worst case of the largest XCD share (moe_xcd_share_cap_q) and of an XCD's draws from the pool;
       // surplus workgroups exit at once
       const long long max_items = (long long)l.max_tiles * col_blocks(MODE, routed.N);
@@ -1019,10 +1021,10 @@ extern "C" int moe_gemm_down_fp8_layout(const uint8_t* hq, const float* sh, cons
 }
 
 // The tile list that the GEMM launches of (R rows, E experts) read from ws when they are told its list_tile_rows.
-int moe_gemm_tile_list(int R, int E, int tile_rows, void* ws, size_t ws_bytes, TileList* list) {
+int moe_gemm_tile_list(int R, int E, int tile_rows, int ncb_gateup, int ncb_down, void* ws, size_t ws_bytes, TileList* list) {
   MOE_REQUIRE(ws && list, MOE_ERR_NULL, "gemm tiles: null pointer");
   MOE_REQUIRE(E >= 1 && E <= 1024 && R >= 0, MOE_ERR_BAD_SHAPE, "gemm tiles: need 1 <= E <= 1024, got E=%d R=%d", E, R);
   MOE_REQUIRE(ws_bytes >= moe_gemm_workspace_bytes(R, E, 0), MOE_ERR_WORKSPACE_TOO_SMALL, "gemm tiles: workspace too small");
-  *list = tile_list(ws, R, E, tile_rows);
+  *list = tile_list(ws, R, E, tile_rows, ncb_gateup, ncb_down);
   return MOE_OK;
 }

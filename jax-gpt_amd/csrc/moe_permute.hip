@@ -86,7 +86,7 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(const int32_t* __r
     }
     if (o.tl.tiles) {   // the grouped GEMMs' row tiles, an expert's tiles side by side (uniform branch)
       const int nt = moe_tile_count(rows, o.tl.tile_rows);
-      const int at = moe_tile_first(e, rows, nt, total, before, o.tl.hdr, o.tl.max_tiles);
+      const int at = moe_tile_first(e, rows, nt, total, before, o.tl);
       for (int t = 0; t < nt; ++t)
         if (at + t < o.tl.max_tiles) o.tl.tiles[at + t] = TileEntry{e | nt << 10, row_start, rows, at};
     }

@@ -307,6 +307,7 @@ def test_one_group_of_many_rows_gives_the_bits_of_fewer(jg, R, D, I):
 
 @pytest.mark.parametrize("D,I,E,sizes", [
     (1024, 1024, 8, [512, 600, 700, 33, 520, 96, 1, 1634]),   # several tiles of 96 to 160 rows an expert
+    (7168, 256, 4, [768, 384, 256, 192]),                     # 9 unequal tiles x 28 column blocks: one round, equal counts
     (512, 256, 32, [0, 200, 0, 1, 40] + [0] * 26 + [15]), (512, 256, 32, [0, 200, 0, 1, 40] + [0] * 26 + [16]),
     (512, 256, 1, [8]), (512, 256, 1, [9])])
 def test_work_lists_of_few_and_more_rows_give_the_same_bits(jg, D, I, E, sizes):
