@@ -288,9 +288,9 @@ def test_scale_layouts_of_middle_sized_batches_give_the_same_bits(jg, M, E):
     assert torch.equal(whole[:400], jg.moe_experts(x[:400].contiguous(), lg[:400].contiguous(), **kw))
 
 
-@pytest.mark.parametrize("R,D,I", [(4100, 256, 8192), (2090, 8192, 256)])
+@pytest.mark.parametrize("R,D,I", [(4096, 256, 8192), (2090, 8192, 256), (5000, 512, 512)])   # (the last: lists of 53 and 79 tiles)
 def test_one_group_of_many_rows_gives_the_bits_of_fewer(jg, R, D, I):
-    """More than 768 work items of one group: its height follows from the rounds that its rows make."""
+    """More than 768 work items of one group, whose height follows from the rounds that its rows make; and many short tiles."""
     import torch
     print("one group", R, D, I, flush=True)
     params, rand = _layer(jg, D, 1, I, 0, R)
