@@ -1,6 +1,6 @@
 // Timing probe for the K loop of the grouped fp8 GEMM (moe_gemm.hip): skeletons of the loop -- the same
 // instruction mix, LDS traffic and copy traffic, no epilogue, results meaningless -- run on all 256 CUs, so
-// that the ceilings the design argues from can be measured again on any box:
+// that the ceilings the design argues from can be measured again:
 //   * what the compute pattern alone reaches (MFMAs + block-scale FMAs + fragment reads from LDS + barrier);
 //   * what the copies cost when every line is an L2 hit, when 4 workgroups of an XCD share each weight slab
 //     streamed from HBM (an expert of 4 row tiles), and when every workgroup streams its own (an expert of one);
@@ -35,6 +35,11 @@ __device__ __forceinline__ void dma16(const uint8_t* base, unsigned off, unsigne
   base = uniform_ptr(base);
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0v), "v"(off), "s"(base) : "memory", "m0");
 }
+__device__ __forceinline__ void dma16_nt(const uint8_t* base, unsigned off, unsigned lds_addr) {
+  const unsigned m0v = __builtin_amdgcn_readfirstlane(lds_addr);
+  base = uniform_ptr(base);
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(m0v), "v"(off), "s"(base) : "memory", "m0");
+}
 __device__ __forceinline__ void dma4(const uint8_t* base, unsigned off, unsigned lds_addr) {
   const unsigned m0v = __builtin_amdgcn_readfirstlane(lds_addr);
   base = uniform_ptr(base);
@@ -49,16 +54,16 @@ __device__ __forceinline__ size_t slab_of(int share, size_t wspan, int it) {
   return ((size_t)(((it * 32 + i) / share) * 8 + x) * (size_t)(256 * KROW)) % wspan;
 }
 
-// ---------------- A: the structure of grouped_gemm_kernel's 256-row class
-// COPY 0: no copies at all.  NGRP: MFMA groups per step (8 = the full tile's work, 0 = copies only).
+// ---------------- A: the structure of grouped_gemm_kernel's tallest classes, 32 XF rows
+// COPY 0: no copies at all.  NGRP: MFMA groups per step (XF = the full tile's work, 0 = copies only).
 // W2 1: the weight tile two steps ahead inside the two stages (issued once its fragments are in registers), the
-// activation tile one step ahead and issued first.
-template <int COPY, int NGRP = 8, int W2 = 0>
+// activation tile one step ahead and issued first.  NT: weight copies marked non-temporal.
+template <int COPY, int NGRP = 8, int W2 = 0, int XF = 8, int NT = 0>
 __global__ __launch_bounds__(512, 1) void kA(float* out, int items, const float* scp, const uint8_t* wsrc, size_t wspan,
                                              const uint8_t* xsrc, int share) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  constexpr int XF = 8;
-  constexpr int STAGE = 65536 + 1024 + 256;
+  constexpr int S_OFF = 32768 + XF * 4096, STAGE = S_OFF + XF * 128 + 256;
+  constexpr int S_OPS = XF > 8 ? 2 : 1;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wi = wave & 3, xj = wave >> 2;
   for (int i = threadIdx.x; i < 2 * STAGE / 4; i += 512) ((int*)lds)[i] = ((const int*)xsrc)[i + (blockIdx.x & 15) * 1000];
@@ -72,13 +77,11 @@ __global__ __launch_bounds__(512, 1) void kA(float* out, int items, const float*
   };
   const uint8_t* xb = xsrc + (size_t)((blockIdx.x >> 7) & 7) * (256 * KROW);
   const int drow = lane >> 3, dch = lane & 7;
-  unsigned woff[8], xoff[8];
+  unsigned woff[8], xoff[XF];
 #pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    woff[u] = (unsigned)((wi * 64 + u * 8 + drow) * KROW + ((dch ^ (drow >> 1)) << 4));
-    xoff[u] = (unsigned)(((u * 4 + wi) * 8 + drow) * KROW + ((dch ^ (drow >> 1)) << 4));
-  }
-  const unsigned soff = (unsigned)(wi * 64 + lane) * 4u;
+  for (int u = 0; u < 8; ++u) woff[u] = (unsigned)((wi * 64 + u * 8 + drow) * KROW + ((dch ^ (drow >> 1)) << 4));
+#pragma unroll
+  for (int u = 0; u < XF; ++u) xoff[u] = (unsigned)(((u * 4 + wi) * 8 + drow) * KROW + ((dch ^ (drow >> 1)) << 4));
   const unsigned lds0 = (unsigned)(uintptr_t)lds;
   v4f acc[4][XF];
   for (int f = 0; f < 4; ++f) for (int j = 0; j < XF; ++j) acc[f][j] = (v4f){0, 0, 0, 0};
@@ -88,13 +91,20 @@ __global__ __launch_bounds__(512, 1) void kA(float* out, int items, const float*
     auto issueW = [&](int kb) {
       const unsigned st = lds0 + (kb & 1) * STAGE;
 #pragma unroll
-      for (int u = 0; u < 8; ++u) dma16(wb + (size_t)kb * 128, woff[u], st + (wi * 8 + u) * 1024);
+      for (int u = 0; u < 8; ++u) {
+        if (NT) dma16_nt(wb + (size_t)kb * 128, woff[u], st + (wi * 8 + u) * 1024);
+        else dma16(wb + (size_t)kb * 128, woff[u], st + (wi * 8 + u) * 1024);
+      }
     };
     auto issueX = [&](int kb) {
       const unsigned st = lds0 + (kb & 1) * STAGE;
 #pragma unroll
-      for (int u = 0; u < 8; ++u) dma16(xb + (size_t)kb * 128, xoff[u], st + 32768 + (u * 4 + wi) * 1024);
-      dma4((const uint8_t*)scp, soff, st + 65536 + wi * 256);
+      for (int u = 0; u < XF; ++u) dma16(xb + (size_t)kb * 128, xoff[u], st + 32768 + (u * 4 + wi) * 1024);
+#pragma unroll
+      for (int i = 0; i < S_OPS; ++i) {   // (64 scale slots each; the second copy of a 288-row tile is the same for all four waves)
+        const int first = i ? 32 * XF - 64 : wi * 64;
+        dma4((const uint8_t*)scp, (unsigned)(first + lane) * 4u, st + S_OFF + first * 4);
+      }
     };
     auto issue = [&](int kb) { issueW(kb); issueX(kb); };
     if (COPY && xj == 0) { issue(0); if (W2) issueW(1); }
@@ -103,27 +113,50 @@ __global__ __launch_bounds__(512, 1) void kA(float* out, int items, const float*
       __builtin_amdgcn_s_barrier();
       if (COPY && xj == 0 && kb + 1 < KB) { if (W2) issueX(kb + 1); else issue(kb + 1); }
       const uint8_t* st = lds + (kb & 1) * STAGE;
+      const uint8_t* sp = st + S_OFF + xj * 64 * XF + fr * XF * 4;
       v8i wf[4], xf[2];
-      const v4f s0 = *(const v4f*)(st + 65536 + xj * 512 + fr * 32), s1 = *(const v4f*)(st + 65536 + xj * 512 + fr * 32 + 16);
-      const float sc[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
+      float sc[XF];
+      if constexpr (XF == 8) {
+        const v4f s0 = *(const v4f*)sp, s1 = *(const v4f*)(sp + 16);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sc[j] = s0[j], sc[4 + j] = s1[j];
+      }
 #pragma unroll
       for (int f = 0; f < 4; ++f) wf[f] = rd(st + (wi * 64 + f * 16) * 128);
       xf[0] = rd(st + 32768 + xj * 2048);
-      v4f p[2][4];
+      if constexpr (XF != 8) sc[0] = *(const float*)sp;
+      v4f p[XF == 8 ? 2 : 1][4];   // (288 rows: 144 of the registers are accumulators, one set of results)
 #pragma unroll
       for (int j = 0; j <= NGRP; ++j) {
         if (NGRP == 0) break;
-        if (j + 1 < NGRP) xf[(j + 1) & 1] = rd(st + 32768 + (2 * (j + 1) + xj) * 2048);
-#pragma unroll
-        for (int f = 0; f < 4; ++f) {
-          if (j < NGRP) p[j & 1][f] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[f], xf[j & 1], z, 0, 0, 0, 0, 0, 0);
-          if (j > 0) acc[f][j - 1] += p[(j - 1) & 1][f] * sc[j - 1];
+        if (j + 1 < NGRP) {
+          xf[(j + 1) & 1] = rd(st + 32768 + (2 * (j + 1) + xj) * 2048);
+          if constexpr (XF != 8) sc[j + 1] = *(const float*)(sp + (j + 1) * 4);
         }
 #pragma unroll
         for (int f = 0; f < 4; ++f) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
-          if (f < 2) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          if constexpr (XF == 8) {
+            if (j < NGRP) p[j & 1][f] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[f], xf[j & 1], z, 0, 0, 0, 0, 0, 0);
+            if (j > 0) acc[f][j - 1] += p[(j - 1) & 1][f] * sc[j - 1];
+          } else {
+            if (j > 0) acc[f][j - 1] += p[0][f] * sc[j - 1];
+            if (j < NGRP) p[0][f] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[f], xf[j & 1], z, 0, 0, 0, 0, 0, 0);
+          }
+        }
+        if constexpr (XF == 8) {
+#pragma unroll
+          for (int f = 0; f < 4; ++f) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+            if (f < 2) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          }
+        } else {
+          if (j + 1 < NGRP) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+#pragma unroll
+          for (int f = 0; f < 4; ++f) {
+            if (j > 0) __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          }
         }
         __builtin_amdgcn_sched_barrier(0);
         if (W2 && COPY && j == 1 && xj == 0) { issueW(kb + 2 < KB ? kb + 2 : KB - 1); __builtin_amdgcn_sched_barrier(0); }
@@ -136,7 +169,6 @@ __global__ __launch_bounds__(512, 1) void kA(float* out, int items, const float*
   for (int f = 0; f < 4; ++f) for (int j = 0; j < XF; ++j) s += acc[f][j][0] + acc[f][j][1] + acc[f][j][2] + acc[f][j][3];
   if (s == 12345.f) out[0] = s;
 }
-
 
 
 // ---------------- C: structure A with the 32x32x64 form of the MFMA (half the instructions and operand-register reads)
@@ -413,6 +445,14 @@ const Variant kVariants[] = {
     {"A  copies only: no MFMA work", kA<1, 0>, 2 * 66816, 0.0},
     {"A  half the MFMA work per step (4 groups: a 128-row tile's)", kA<1, 4>, 2 * 66816, 0.5},
     {"A2 weight tile two steps ahead inside the two stages, activation tile issued first", kA<1, 8, 1>, 2 * 66816, 1.0},
+    {"A  weight copies non-temporal", kA<1, 8, 0, 8, 1>, 2 * 66816, 1.0},
+    {"A  copies only, weight copies non-temporal", kA<1, 0, 0, 8, 1>, 2 * 66816, 0.0},
+    {"A2 weight copies non-temporal", kA<1, 8, 1, 8, 1>, 2 * 66816, 1.0},
+    {"A  288 rows", kA<1, 9, 0, 9>, 2 * 71040, 1.125},
+    {"A  288 rows, compute only", kA<0, 9, 0, 9>, 2 * 71040, 1.125},
+    {"A  288 rows, copies only", kA<1, 0, 0, 9>, 2 * 71040, 0.0},
+    {"A2 288 rows", kA<1, 9, 1, 9>, 2 * 71040, 1.125},
+    {"A2 288 rows, weight copies non-temporal", kA<1, 9, 1, 9, 1>, 2 * 71040, 1.125},
     {"B  8x1 wave grid: weights global->VGPR two steps ahead, activations lds-dma (4 stages), barrier per 2 steps", kB<1, 1, 2>, 4 * 34048, 1.0},
     {"B  the same with a barrier per step", kB<1, 1, 1>, 4 * 34048, 1.0},
     {"B  compute only", kB<0, 0, 2>, 4 * 34048, 1.0},
