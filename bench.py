@@ -43,8 +43,8 @@ def measured_traffic(workload, kernel="gateup_routed"):
     return None, None
 
 
-GATEUP_NAME = "grouped_gemm_kernel<0>, routed launch (gate/up + SwiGLU + h quantisation)"
-DOWN_NAME = "grouped_gemm_kernel<1>, routed launch (down, bf16 rows)"
+GATEUP_NAME = "grouped_gemm_kernel<0, ..>, routed launch (gate/up + SwiGLU + h quantisation)"
+DOWN_NAME = "grouped_gemm_kernel<1, ..>, routed launch (down, bf16 rows)"
 
 
 def kernel_roofline(bound, kern, workload, kernel_key, name):
@@ -61,12 +61,12 @@ def kernel_roofline(bound, kern, workload, kernel_key, name):
 
 
 WORKLOADS = {
-    # benchmark configs 3 and 4: DeepSeek-V3-style layer
+    # DeepSeek-V3-style layer: a full prompt batch and a decode batch
     "deepseek_v3_prefill": dict(M=8192, D=7168, E=256, k=8, I=2048, SI=2048, routing="sigmoid_grouped",
                                 n_group=8, topk_group=4),
     "deepseek_v3_decode": dict(M=64, D=7168, E=256, k=8, I=2048, SI=2048, routing="sigmoid_grouped",
                                n_group=8, topk_group=4),
-    # benchmark config 2: Qwen3-MoE-style layer
+    # Qwen3-MoE-style layer: a prompt batch
     "qwen3_moe_prefill": dict(M=4096, D=2048, E=128, k=8, I=768, SI=0, routing="softmax", n_group=1, topk_group=1),
 }
 
@@ -216,7 +216,7 @@ def run_workload(jg, torch, name, cfg, layer, steps, warmup, graph=True):
 
 
 def run_ep_shard(jg, torch, steps, warmup, seed=5):
-    """Benchmark config 5: one GPU's expert-parallel shard.  32 local experts of the DeepSeek-V3 shape receive
+    """One GPU's expert-parallel shard.  32 local experts of the DeepSeek-V3 shape receive
     16384 pre-dispatched rows (already in expert order: row_ids = NULL), group sizes from Zipf(1.2) with empty
     experts, combine with top-8 weights from Dirichlet(1) into 2048 tokens.  A step = gate/up GEMM, down GEMM,
     combine."""
@@ -270,7 +270,7 @@ def run_ep_shard(jg, torch, steps, warmup, seed=5):
 
 
 def run_probe(reps):
-    """`--probe`: the ceilings of the grouped GEMM's K loop on this box (jax-gpt_amd/csrc/moe_probe.hip: skeletons of
+    """`--probe`: the ceilings of the grouped GEMM's K loop on this machine (jax-gpt_amd/csrc/moe_probe.hip: skeletons of
     the loop on all 256 CUs, no epilogue, results meaningless).  Prints one JSON line with a list of measurements."""
     import ctypes as C
     path = os.path.join(ROOT, "jax-gpt_amd", "libmoe_probe.so")
@@ -310,7 +310,7 @@ def cpu_baseline(cfg, seconds_budget=25.0):
     import torch
     from oracle import reference_dataflow as RD
     cores = os.cpu_count() or 1
-    threads = min(cores, 16)                  # a one-GPU box gives this job 16 cores' worth
+    threads = min(cores, 16)                  # (one GPU's share of a host)
     rows = max(cfg["M"] * cfg["k"] // cfg["E"], 1)
     n_exp = 32                                # about 10-20 s of host work in total
     t0 = time.perf_counter()

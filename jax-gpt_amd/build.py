@@ -19,7 +19,7 @@ PROBE_PATH = os.path.join(HERE, "libmoe_probe.so")
 
 SOURCES = ["moe_api.hip", "moe_route.hip", "moe_router.hip", "moe_permute.hip", "moe_quant.hip", "moe_gemm.hip",
            "moe_combine.hip"]
-# no v_pk_*_f32 code generation (some packed-f32 forms misbehave on this hardware pool)
+# no v_pk_*_f32 code generation (some packed-f32 forms have given wrong results on this hardware)
 COMMON = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function",
           "-fvisibility=hidden",    # only the functions include/moe_hip.h declares (MOE_API) are exported
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

@@ -1,4 +1,5 @@
-"""Parity at the benchmark configurations' full sizes (configs 2-5 of BASELINE.json).
+"""Parity at the benchmark workloads' full sizes: Qwen3-MoE and DeepSeek-V3 prefill, DeepSeek-V3 decode, an expert-parallel
+shard.
 
 The oracle cannot run these sizes in full, so each test checks
   * every integer result (routing indices, group sizes, permutation) exactly against
@@ -8,7 +9,7 @@ The oracle cannot run these sizes in full, so each test checks
     intermediate h as helpers.check_layer_output does: the kernel's h rows against the oracle's,
     and the output rows against the oracle continued from the kernel's h, to the plain
     tolerance (1e-2 max-normalised and allclose);
-  * at config 3 every row of one expert that spans two row tiles, through the stage entry points;
+  * at the DeepSeek-V3 prefill every row of one expert that spans two row tiles, through the stage entry points;
   * size-independent properties: a sub-batch gives bit-identical rows; every routed
     row is written exactly once; empty experts are skipped.
 Weights are generated on the GPU (the DeepSeek-V3 shape is 11.3 GB of fp8) by the same
