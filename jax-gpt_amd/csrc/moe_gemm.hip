@@ -27,16 +27,16 @@
 // 16-row activation fragments 2j + xj (alternating between the two wave sets, so
 // a short tile still splits evenly).
 //
-// What bounds a work item.  A K step of a full tile moves 64 KB into LDS (72 copy instructions per CU) and holds
-// 2048 matrix-core cycles per SIMD.  The L2 can fill one CU's LDS at about 125 GB/s with this copy pattern (all CUs
-// at once); a CU streaming alone from HBM gets about 22 GB/s whatever its queue depth, and all 256 together reach
-// the memory's rate.  The activation tile is shared by the item's 16 column blocks and comes from L2, the weight
-// tile comes from L2 when a neighbouring row tile of the same expert has just fetched it and from HBM or the
-// memory-side cache otherwise (always, for an expert of one row tile).  An expert of few rows is therefore a
-// weight stream at the per-CU HBM rate whatever the kernel does with its rows; the kernel's part is to keep that
-// stream and the large experts' matrix work going side by side on different CUs, and to waste neither.  Measured
-// on full tiles, the copies cost the loop a quarter of its speed even from an L2-hot source: it is their issue
-// (address generation, back-pressure from the L1) in the instruction stream of the waves that feed the matrix core.
+// What bounds a work item.  A K step of a full tile moves 68 KB into LDS (76 copy instructions per CU) and holds
+// 2304 matrix-core cycles per SIMD.  Skeletons of the loop on all CUs: 3130 TFLOP/s without the copies, 2737 when every
+// weight line is an L2 hit, 2615 when four row tiles share a weight slab from memory, 2181 when each streams its own.
+// The activation tile is shared by the item's 16 column blocks and comes from L2, the weight tile comes from L2 when a
+// neighbouring row tile of the same expert has just fetched it and from HBM or the memory-side cache otherwise (always,
+// for an expert of one row tile).  An expert of few rows is therefore a weight stream at the per-CU HBM rate (31 GB/s of
+// both tiles, 41 with non-temporal weight copies) whatever the kernel does with its rows; the kernel's part is to keep that
+// stream and the large experts' matrix work going side by side on different CUs, and to waste neither.  The copies'
+// cost from an L2-hot source is their issue (address generation, back-pressure from the L1) in the instruction stream of
+// the waves that feed the matrix core.
 //
 // Row tiles are listed on the device (build_tiles_kernel here, or the permutation
 // kernels inside moe_forward: no host read-back of group sizes); a workgroup's
@@ -156,7 +156,7 @@ template <int XF, int MODE = MODE_GATEUP, bool ONCE = true> struct Cls {
   // the middle of the step, and not behind the next barrier: the weights of step kb + 2 are then in flight while step
   // kb still computes, as if the ring were a stage deeper, in the same LDS.  The weight rows that wave (wi, 0) copies
   // are read by itself and by wave (wi, 1) alone, so the release is a word in LDS between those two (early_flag)
-  // and no barrier.  Only the 256-row class of the gate/up GEMM, which has no room for a third stage: -4.5 % where
+  // and no barrier.  Only the 256- and 288-row classes of the gate/up GEMM, which have no room for a third stage: -4.5 % where
   // every workgroup streams its own weight slab, -3 % where 8 row tiles share one, -1 % on the mixed tile
   // heights of skewed routing; the down GEMM (16 K steps at the DeepSeek-V3 shape) gained 2 % in the first case and
   // lost 1 % in the second, and the classes with three weight stages cannot gain: their copies complete in issue
