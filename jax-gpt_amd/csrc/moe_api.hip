@@ -293,7 +293,7 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
   // routing, the sort by expert and the routed GEMMs' work list (the sort holds every expert's row range anyway)
   TileList tiles;
   const bool together = a->SI && !fork;   // the shared expert runs inside the routed launches
-  const int tile_rows = moe_gemm_tile_rows(TileShape{R, a->E, {a->I / 128, (a->D + 255) / 256}, {a->D / 128, a->I / 128},
+  const int tile_rows = moe_gemm_tile_rows(TileShape{R, a->E, a->M, {a->I / 128, (a->D + 255) / 256}, {a->D / 128, a->I / 128},
                                                      together ? a->M : 0, {a->SI / 128, (a->D + 255) / 256}});
   if ((rc = moe_gemm_tile_list(R, a->E, tile_rows, a->I / 128, (a->D + 255) / 256, b.gemm_ws, b.gemm_ws_bytes, &tiles))) return join(rc);
   const RouteArgs route{src, a->bias, a->M, a->E, a->k, a->renorm, a->n_group, a->topk_group, a->routed_scale, idx, w_own};

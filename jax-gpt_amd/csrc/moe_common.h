@@ -316,6 +316,7 @@ int moe_gemm_tile_list(int R, int E, int tile_rows, int ncb_gateup, int ncb_down
 // [1] down: column blocks per row tile and K steps (0: that GEMM does not read the list).
 struct TileShape {
   int R, E;
+  int max_rows;   // that a group may have
   int ncb[2], kb[2];
   int dense_rows, dense_ncb[2];
 };

@@ -48,12 +48,16 @@
 // the eight ranges as a pool from which the workgroups that follow an XCD's range
 // draw one item each through a counter (TileHeader), so an XCD that is ahead
 // takes more of them.
+//
+// Launches of many work items of short row tiles are taken by another kernel, with
+// the same items, operands and results: moe_gemm_stream.hip (moe_gemm_tile_rows and
+// moe_gemm_stream_stages say which).
 #include <stdlib.h>
 
 #include <mutex>
 #include <type_traits>
 
-#include "moe_common.h"
+#include "moe_gemm_device.h"
 
 // Tile list of moe_gemm_gateup_swiglu_fp8_static: one copy per GPU, held until the process ends.  In host code this
 // name is only a handle for hipGetSymbolAddress; kernels get the address that call returns.
@@ -61,14 +65,8 @@ static __device__ __align__(256) unsigned char scratch[MOE_STATIC_SCRATCH_BYTES]
 
 namespace {
 
-constexpr int BW = 256;       // weight rows per work item
-constexpr int BK = 128;       // K step = scale block
 constexpr int NWAVES = 8;
 constexpr int NT = 64 * NWAVES;
-constexpr int MODE_GATEUP = 0;
-constexpr int MODE_DOWN = 1;
-constexpr int MAX_KB = 256;   // K <= 32768
-constexpr int W_TILE_BYTES = BW * BK;   // 32 KB
 constexpr int ROTC = 2;       // MFMA groups by which wave set 1 trails wave set 0 (measured: 1 to 3 within 2 %)
 
 // ---- work list -----------------------------------------------------------
@@ -124,9 +122,6 @@ __global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __rest
 // global_load_lds_dwordx4 writes LDS base + lane * 16, i.e. one wave instruction fills 8
 // consecutive tile rows; the swizzle is applied by choosing which 16-byte piece of the row
 // each lane fetches.  No asynchronous load ever targets a register.
-
-// epilogue staging tile: 128-byte rows, chunk c of row r at position c ^ (r & 7)
-__device__ __forceinline__ int swz(int row, int chunk) { return row * BK + ((chunk ^ (row & 7)) << 4); }
 
 // One launch, row tiles of every height.  A work item's row tile (at most 288 rows, near-equal cuts of its
 // expert) is served by the smallest of nine compiled tile classes that holds it -- 32 XF rows, XF = 1 .. 9 MFMA
@@ -232,8 +227,6 @@ template <int XF> constexpr bool epilogue_fits() {
   return Cls<XF>::BM * (4 * 4 + BK) <= CLS_RING && Cls<XF>::BM * 256 * 2 <= CLS_RING;
 }
 static_assert(epilogue_fits<9>(), "the tallest tile's epilogue stages inside the rings' space");
-
-struct Item { int expert, row_start, row_count, col_block, tiles; };
 
 template <int MODE, int XF, bool ONCE>
 __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const uint8_t* __restrict__ xq,
@@ -567,124 +560,11 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
   else run(std::integral_constant<int, ROT1>{}, std::false_type{});
   __syncthreads();   // every wave is done reading the ring before the epilogue reuses LDS
 
-  // ---- epilogue.  Lane holds, for fragment (f, j): tile row (2j + xj)*16 + fr, weight rows (fragment base) + 4*fq + {0..3}.
-  if (MODE == MODE_GATEUP) {
-    float* amax_s = (float*)lds;                       // [4 weight-wave groups][BM rows]
-    uint8_t* tile = lds + 4 * BM * sizeof(float);      // [BM rows][128 B], swizzled
-#pragma unroll
-    for (int j = 0; j < XF; ++j) {
-      float m = 0.f;
-#pragma unroll
-      for (int f = 0; f < 2; ++f)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float g = acc[f][j][r], u = acc[f + 2][j][r];
-          float h = g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u;   // (reciprocal to 1 ulp: far inside the fp8 step)
-          acc[f][j][r] = h;
-          m = fmaxf(m, fabsf(h));
-        }
-      m = fmaxf(m, __shfl_xor(m, 16, MOE_WAVE));
-      m = fmaxf(m, __shfl_xor(m, 32, MOE_WAVE));
-      if (fq == 0) amax_s[wi * BM + (2 * j + xj) * 16 + fr] = m;
-    }
-    __syncthreads();
-    const int I = N;
-    uint8_t* hq = (uint8_t*)out;
-#pragma unroll
-    for (int j = 0; j < XF; ++j) {
-      const int xr = (2 * j + xj) * 16 + fr;
-      float m = fmaxf(fmaxf(amax_s[xr], amax_s[BM + xr]), fmaxf(amax_s[2 * BM + xr], amax_s[3 * BM + xr]));
-      float scale, scale_inv;
-      fp8_scales(m, scale, scale_inv);
-#pragma unroll
-      for (int f = 0; f < 2; ++f) {
-        int q = 0;   // (|h| <= amax, so the products stay within a rounding of +-448: one median clamps them)
-        q = __builtin_amdgcn_cvt_pk_fp8_f32(__builtin_amdgcn_fmed3f(acc[f][j][0] * scale, -MOE_FP8_MAX, MOE_FP8_MAX),
-                                            __builtin_amdgcn_fmed3f(acc[f][j][1] * scale, -MOE_FP8_MAX, MOE_FP8_MAX), q, false);
-        q = __builtin_amdgcn_cvt_pk_fp8_f32(__builtin_amdgcn_fmed3f(acc[f][j][2] * scale, -MOE_FP8_MAX, MOE_FP8_MAX),
-                                            __builtin_amdgcn_fmed3f(acc[f][j][3] * scale, -MOE_FP8_MAX, MOE_FP8_MAX), q, true);
-        const int col = wi * 32 + f * 16 + fq * 4;  // byte column within the 128-wide slab
-        *(unsigned*)(tile + swz(xr, col >> 4) + (col & 15)) = q;
-      }
-      if (wi == 0 && fq == 0 && xr < item.row_count)
-        out_scale[(size_t)(item.row_start + xr) * sc.out_row + (size_t)item.col_block * sc.out_cb] = scale_inv;
-    }
-    __syncthreads();
-    const int ld_chunk = tid & 7, ld_row = tid >> 3;   // 64 rows per pass
-#pragma unroll
-    for (int i = 0; i < (BM + 63) / 64; ++i) {
-      const int r = ld_row + 64 * i;
-      if (r < item.row_count) {
-        v4i v = *(const v4i*)(tile + swz(r, ld_chunk));
-        v4i* dst = (v4i*)(hq + (size_t)(item.row_start + r) * I + item.col_block * 128 + ld_chunk * 16);
-        store16(dst, v, sc.out_through);
-      }
-    }
-  } else {
-    // bf16 tile [BM rows][256 cols] = 512 B per row, 32 chunks of 16 B, swizzled with (row & 7)
-    uint8_t* tile = lds;
-#pragma unroll
-    for (int j = 0; j < XF; ++j) {
-      const int xr = (2 * j + xj) * 16 + fr;
-#pragma unroll
-      for (int f = 0; f < 4; ++f) {
-        const int col = wi * 64 + f * 16 + fq * 4;  // output column within the 256-wide slab
-        uint2 v;
-        v.x = pack2_bf16(acc[f][j][0], acc[f][j][1]);
-        v.y = pack2_bf16(acc[f][j][2], acc[f][j][3]);
-        const int chunk = col >> 3;  // 8 bf16 per 16-byte chunk
-        *(uint2*)(tile + xr * 512 + ((chunk ^ (xr & 7)) << 4) + (col & 7) * 2) = v;
-      }
-    }
-    __syncthreads();
-    bf16_t* y = (bf16_t*)out;
-    const int c32 = tid & 31, r16 = tid >> 5;          // 16 rows per pass
-    const int ncols = min(256, N - wrow0);
-#pragma unroll
-    for (int i = 0; i < BM / 16; ++i) {
-      const int r = r16 + 16 * i;
-      if (r < item.row_count && c32 * 8 < ncols) {
-        v4i v = *(const v4i*)(tile + r * 512 + ((c32 ^ (r & 7)) << 4));
-        v4i* dst = (v4i*)(y + (size_t)(item.row_start + r) * N + wrow0 + c32 * 8);
-        store16(dst, v, sc.out_through);
-      }
-    }
-  }
+  item_epilogue<MODE, 4, XF, BM, 32, NT>(acc, item, xj * 16 + fr, wi, lds, N, out, out_scale, sc);
 }
 
 // row tiles of an expert up to which its weight lines are marked non-temporal (grouped_gemm_kernel)
 __host__ __device__ inline int once_tiles(int K) { return K <= 2048 ? 2 : 1; }
-
-// Column block and row tile of the `local`-th work item of an expert of nt row tiles and ncb column blocks.
-__device__ __forceinline__ void expert_item(int local, int nt, int ncb, int& col_block, int& rt) {
-  if (nt < 16) {
-    col_block = nt == 1 ? local : local / nt;
-    rt = local - col_block * nt;
-    return;
-  }
-  // An expert of many row tiles goes through its column blocks once per group of 8 to 11 row tiles: the 32 CUs
-  // of an XCD then work on about 8 row tiles x 4 column blocks at a time (12 distinct operand tiles per K step)
-  // instead of 32 row tiles of one column block (33 distinct tiles, every CU pulling the same weight lines at
-  // once): 32 row tiles per expert ran 19 % slower than 8.  Below 16 tiles a split does not pay (11 tiles as
-  // 6 + 5 measured 1 % slower than unsplit).
-  const int ng = nt >> 3;
-  const int base = nt / ng, extra = nt - base * ng;   // the first `extra` groups hold base + 1 tiles
-  const int big = (base + 1) * ncb * extra;
-  int sz, l2, t0;
-  if (local < big) {
-    sz = base + 1;
-    const int g = local / (sz * ncb);
-    l2 = local - g * sz * ncb;
-    t0 = g * sz;
-  } else {
-    sz = base;
-    const int l = local - big, g = l / (sz * ncb);
-    l2 = l - g * sz * ncb;
-    t0 = extra * (base + 1) + g * sz;
-  }
-  col_block = l2 / sz;
-  rt = t0 + (l2 - col_block * sz);
-}
 
 // The first dense_blocks workgroups serve `dense`, one group of dense_rows rows (the shared expert), whose work items
 // follow from the row count alone; the rest serve the routed experts through the work list (hdr null: none).  A
@@ -700,52 +580,9 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
                                                             int dense_rows, int dense_tiles, int dense_blocks) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const bool is_dense = DENSE && (int)blockIdx.x < dense_blocks;   // (dense_blocks is a multiple of 8: the XCD is blockIdx % 8 for both)
-  const int xcd = blockIdx.x & 7;
   const int K = is_dense ? dense.K : routed.K, N = is_dense ? dense.N : routed.N;
-  const int ncb = MODE == MODE_GATEUP ? N / 128 : (N + 255) / 256;
   Item item;
-  if (is_dense) {
-    // contiguous eighths of the items, so that row tiles that share a weight slab run under one L2
-    const int nt = dense_tiles, items = nt * ncb;
-    const int per = dense_blocks >> 3;
-    const int local = xcd * per + (int)(blockIdx.x >> 3);
-    if (local >= items) return;
-    int rt, t0, tn;
-    expert_item(local, nt, ncb, item.col_block, rt);
-    moe_tile_span(dense_rows, nt, rt, t0, tn);
-    item.expert = 0;
-    item.tiles = nt;
-    item.row_start = t0;
-    item.row_count = tn;
-  } else {
-    // work items = (row tile, column block) pairs in [expert][column block][row tile] order, dealt to the 8 XCDs in
-    // contiguous ranges of about equal cost (workgroup ids are issued round-robin over XCDs)
-    int item_id = (int)((hdr->xcd_q[xcd] * ncb) >> kTileQBits) + (((int)blockIdx.x - (DENSE ? dense_blocks : 0)) >> 3);
-    const int share_end = (int)((hdr->xcd_q[xcd + 1] * ncb) >> kTileQBits);
-    if (item_id >= share_end) {
-      // behind the XCD's fixed share: the pool of the smallest experts' items, drawn one at a time by whoever gets
-      // there (TileHeader); an XCD may draw up to twice its eighth of it
-      const int pool_first = hdr->n_static * ncb;
-      const int pool_items = (hdr->n_tiles - hdr->n_static) * ncb;
-      if (pool_items == 0 || item_id - share_end >= moe_pool_workgroups(pool_items)) return;   // (uniform: the whole workgroup leaves)
-      int* slot = (int*)lds;
-      if (threadIdx.x == 0) *slot = atomicAdd(&hdr->pool_next[MODE], 1);   // (the one field of the list a GEMM writes)
-      __syncthreads();
-      const int drawn = *slot;
-      __syncthreads();   // (the work item's first copies overwrite the slot)
-      if (drawn >= pool_items) return;
-      item_id = pool_first + drawn;
-    }
-    const TileEntry te = tiles[item_id / ncb];   // entries [first_tile, first_tile + tiles) all describe this expert
-    const int nt = te.expert_tiles >> 10;
-    int rt, t0, tn;
-    expert_item(item_id - te.first_tile * ncb, nt, ncb, item.col_block, rt);
-    moe_tile_span(te.rows, nt, rt, t0, tn);
-    item.expert = te.expert_tiles & 1023;
-    item.tiles = nt;
-    item.row_start = te.row_start + t0;
-    item.row_count = tn;
-  }
+  if (!work_item<MODE, DENSE>(item, lds, N, is_dense, hdr, tiles, dense_rows, dense_tiles, dense_blocks)) return;
   const uint8_t* xq = is_dense ? dense.xq : routed.xq;
   const float* sx = is_dense ? dense.sx : routed.sx;
   const int32_t* row_ids = is_dense ? nullptr : routed.row_ids;
@@ -833,18 +670,19 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
     return (size_t)rows * N * (MODE == MODE_DOWN ? 2 : 1) > ((size_t)4 << 20) && rows <= 96ll * E;
   };
   auto own_tile_rows = [](int rows, int E, const GemmOperands& op) {
-    return moe_gemm_tile_rows(TileShape{rows, E, {col_blocks(MODE, op.N), 0}, {op.K / BK, 0}, 0, {0, 0}});
+    return moe_gemm_tile_rows(TileShape{rows, E, rows, {col_blocks(MODE, op.N), 0}, {op.K / BK, 0}, 0, {0, 0}});
   };
   GemmOperands routed{}, dense{};
   TileList l{};
-  int dense_rows = 0, dense_tiles = 0;
+  int dense_rows = 0, dense_tiles = 0, dense_tile_rows = 0;
   long long dense_blocks = 0, grid = 0;
   if (dn) {
     if (int rc = check_operands(dn->op, dn->rows, 1, MODE, what)) return rc;
     dense = dn->op;
     dense.sc.out_through = through(dn->rows, 1, dense.N);
     dense_rows = dn->rows;
-    dense_tiles = moe_tile_count(dense_rows, rt && rt->list_tile_rows ? rt->list_tile_rows : own_tile_rows(dense_rows, 1, dense));
+    dense_tile_rows = rt && rt->list_tile_rows ? rt->list_tile_rows : own_tile_rows(dense_rows, 1, dense);
+    dense_tiles = moe_tile_count(dense_rows, dense_tile_rows);
     dense_blocks = 8 * (((long long)dense_tiles * col_blocks(MODE, dense.N) + 7) / 8);
     grid = dense_blocks;
   }
@@ -881,6 +719,12 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
   const bool shared_lines = l.hdr ? l.tile_rows <= 128 && rt->R > (long long)once_tiles(routed.K) * l.tile_rows * rt->E
                                   : dense_tiles > once_tiles(dense.K) && dense_rows <= 128 * dense_tiles;
   const bool stream = layer_bytes > (192ll << 20) && !shared_lines;
+  const int tallest = l.hdr ? l.tile_rows : dense_tile_rows;   // (a dense group beside routed ones is cut as their list is)
+  long long items = dn ? (long long)dense_tiles * col_blocks(MODE, dense.N) : 0;
+  if (l.hdr) items += (long long)(rt->E < rt->R ? rt->E : rt->R) * col_blocks(MODE, routed.N);
+  if (const int stages = moe_gemm_stream_stages(MODE, tallest, items))
+    return moe_gemm_stream_launch(MODE, StreamLaunch{routed, l.hdr, l.tiles, dense, dense_rows, dense_tiles, (int)dense_blocks, stream,
+                                                     (unsigned)grid, tallest, stages}, s);
   static std::atomic<unsigned long long> lds_raised[4] = {};
   auto* kernel = dn ? (stream ? grouped_gemm_kernel<MODE, true, true> : grouped_gemm_kernel<MODE, true, false>)
                     : (stream ? grouped_gemm_kernel<MODE, false, true> : grouped_gemm_kernel<MODE, false, false>);
@@ -899,9 +743,17 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
 // that just fills a round does not spill into another one.  One group's size is known, and so are its rounds however many
 // items they hold: 8192 rows of 2048 x 8192 are 8 rounds of 256-row tiles or of 288-row ones, 287 -> 274 us (gate/up),
 // 138.6 -> 127.1 the down GEMM of 7168 x 2048.
+//   Before that: short tiles, which moe_gemm_stream.hip takes, where no expert can have more rows -- or hardly one will, with
+// eight times the mean to spare.  An expert that has more after all is cut, and its weights are read once for each tile, from
+// L2 at best (4000 tokens of the full layer, 78 rows an expert, tiles of 128 rows: 1329 us where the routing is even, 1340 ->
+// 1380 where 81 experts have 128 to 493).
 int moe_gemm_tile_rows(const TileShape& t) {
   const int groups = t.E < t.R ? t.E : t.R;
   if (groups <= 0) return kTileRows;
+  if ((long long)groups * (t.ncb[0] > t.ncb[1] ? t.ncb[0] : t.ncb[1]) >= kStreamItems) {
+    if (t.max_rows <= 32 || t.R <= 4 * t.E) return 32;
+    if (t.max_rows <= kStreamRows || t.R <= kStreamRows / 8 * t.E) return kStreamRows;
+  }
   const int mean = (t.R + groups - 1) / groups;
   if (mean > kFullTileItems * kTileRows / groups) return kTileRows;
   const int least = t.ncb[1] && t.ncb[1] < t.ncb[0] ? t.ncb[1] : t.ncb[0];

@@ -327,3 +327,64 @@ def test_work_lists_of_few_and_more_rows_give_the_same_bits(jg, D, I, E, sizes):
         hq1, sh1 = jg.gemm_gateup_swiglu(xq[lo:hi], sx[lo:hi].clone(), one["gate"], one["up"], o1)
         assert torch.equal(hq1.view(torch.uint8), hq[lo:hi].view(torch.uint8)) and torch.equal(sh1, sh[lo:hi]), f"expert {e}: h"
         assert torch.equal(jg.gemm_down(hq1, sh1, one["down"], o1), y[lo:hi]), f"expert {e}: y"
+
+
+SHORT = [33, 0, 1, 0, 2, 0, 0, 17, 0, 1, 0, 0, 16, 0, 3, 0, 0, 0, 32, 0, 0, 1, 0, 0, 0, 0, 0]   # at most 4 rows an expert on average
+TALL = [250, 129, 128, 97, 96, 65, 64, 33, 1] + [0] * 47                                             # at most 16
+
+
+@pytest.mark.parametrize("E,D,I,sizes", [
+    (108, 1024, 512, SHORT),      # 432 gate/up and down items: one stage, two stages
+    (162, 640, 512, SHORT),       # 648: two stages; the last column block of the down GEMM is half full
+    (108, 128, 512, SHORT),       # gate/up of one K step
+    (405, 256, 128, SHORT),       # 405 items each, of two K steps and of one
+    (54, 2176, 1280, SHORT),      # weights from memory: copies of experts of one tile are non-temporal
+    (56, 2048, 384, TALL),        # down tiles of up to 128 rows, plain copies ...
+    (56, 2048, 1024, TALL),       # ... and non-temporal ones
+])
+def test_streamed_short_tiles_give_the_same_bits(jg, E, D, I, sizes):
+    """Many short work items, which a kernel of their own takes: each expert's rows against a call of that expert alone
+    (too few items for it), and one expert's down rows against the oracle."""
+    import torch
+    print("streamed tiles", E, D, I, flush=True)
+    sizes = [sizes[i % len(sizes)] for i in range(E)]
+    params, rand = _layer(jg, D, E, I, 0, E + D)
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    R = int(off[-1])
+    ids = torch.randperm(R, device="cuda").to(torch.int32)
+    xq, sx = jg.quant_act(rand(R, D))
+    hq, sh = jg.gemm_gateup_swiglu(xq, sx, params["gate_proj"], params["up_proj"], H.to_cuda(off), row_ids=ids)
+    y = jg.gemm_down(hq, sh, params["down_proj"], H.to_cuda(off))
+    gathered = jg.gather_scales(sx, ids)
+    hb, sb = jg.gemm_gateup_swiglu(xq, gathered, params["gate_proj"], params["up_proj"], H.to_cuda(off), row_ids=ids, block_major=True)
+    assert torch.equal(hb.view(torch.uint8), hq.view(torch.uint8)) and torch.equal(sb.t(), sh)
+    assert torch.equal(jg.gemm_down(hb, sb, params["down_proj"], H.to_cuda(off), block_major=True), y)
+    for e in [e for e in range(min(E, 60)) if sizes[e]]:
+        lo, hi = int(off[e]), int(off[e + 1])
+        one = {n: {k: v[e:e + 1] for k, v in params[n + "_proj"].items()} for n in ("gate", "up", "down")}
+        o1 = H.to_cuda(np.array([0, hi - lo], np.int32))
+        hq1, sh1 = jg.gemm_gateup_swiglu(xq, sx, one["gate"], one["up"], o1, row_ids=ids[lo:hi].clone())
+        assert torch.equal(hq1.view(torch.uint8), hq[lo:hi].view(torch.uint8)) and torch.equal(sh1, sh[lo:hi]), f"expert {e}: h"
+        assert torch.equal(jg.gemm_down(hq1, sh1, one["down"], o1), y[lo:hi]), f"expert {e}: y"
+        if e == 0:
+            w, s = one["down"]["w"], one["down"]["scale_inv"]
+            want = O.grouped_gemm(H.codes_np(hq1), sh1.cpu().numpy(), H.codes_np(w), s.cpu().numpy(), np.array([0, hi - lo], np.int32))
+            H.assert_close_out(H.bf16_to_np(y[lo:hi]), O.bf16_round(want.astype(np.float32)))
+
+
+@pytest.mark.parametrize("routing", ["softmax", "sigmoid_grouped"])
+def test_batches_of_every_tile_height_give_the_bits_of_a_large_one(jg, routing):
+    """5 to 600 tokens of one layer with a shared expert: tiles of 32 and 128 rows in the two GEMMs' kernels."""
+    import torch
+    print("batches", routing, flush=True)
+    D, E, I, SI, k = 1152, 128, 512, 256, 4
+    params, rand = _layer(jg, D, E, I, SI, 11)
+    M = 4000
+    x, lg = rand(M, D), rand(M, E).float()
+    kw = dict(top_k=k, experts={n: params[n] for n in ("gate_proj", "up_proj", "down_proj")}, routing=routing,
+              shared={n: params["shared_" + n] for n in ("gate_proj", "up_proj", "down_proj")})
+    if routing == "sigmoid_grouped":
+        kw.update(n_group=8, topk_group=4, bias=0.1 * torch.arange(E, device="cuda").remainder(5).float())
+    whole = jg.moe_experts(x, lg, **kw)
+    for m in (5, 32, 33, 128, 129, 600):
+        assert torch.equal(jg.moe_experts(x[:m].contiguous(), lg[:m].contiguous(), **kw), whole[:m]), f"{m} tokens"
