@@ -388,3 +388,9 @@ def test_batches_of_every_tile_height_give_the_bits_of_a_large_one(jg, routing):
     whole = jg.moe_experts(x, lg, **kw)
     for m in (5, 32, 33, 128, 129, 600):
         assert torch.equal(jg.moe_experts(x[:m].contiguous(), lg[:m].contiguous(), **kw), whole[:m]), f"{m} tokens"
+
+
+@pytest.mark.parametrize("M,E,k", [(1793, 40, 2), (2047, 8, 1), (4099, 128, 8)])
+def test_many_tokens_a_workgroup_are_routed_exactly(jg, M, E, k):
+    """8 to 17 tokens of a routing workgroup, of eight waves beside the quantiser; the last one has fewer."""
+    test_ready_logits_routed_and_sorted_in_one_launch_or_two(jg, M, E, k)
