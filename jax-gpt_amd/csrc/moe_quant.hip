@@ -216,24 +216,36 @@ extern "C" int moe_convert(const void* src, int src_is_f32, void* dst, int dst_i
 
 namespace {
 // Activation scales, row-major (rows, KB) -> block-major (KB, n) in row-list order: out[kb][p] = sx[ids ? ids[p] : p][kb].
-// One thread per list position: it reads its row's KB scales (one or two lines) and writes one float into each of the
-// KB output rows, where neighbouring threads write neighbouring floats.
+// A thread takes kGatherScales neighbouring scales of one list position (half a line) and writes one float into each of as
+// many output rows, where neighbouring threads write neighbouring floats.  Bound by latency (7 MB for 16384 rows of 56): with
+// all scales of a row in one thread, 64 workgroups of 14 loads a thread, that took 8.2 us, now 4.5; 6216 rows of 56 6.4 -> 4.1.
+constexpr int kGatherScales = 16;
 __global__ __launch_bounds__(256) void gather_scales_kernel(const float* __restrict__ sx, const int32_t* __restrict__ ids,
                                                            int n, int KB, float* __restrict__ out) {
   const int p = blockIdx.x * 256 + threadIdx.x;
   if (p >= n) return;
-  const float* src = sx + (size_t)(ids ? ids[p] : p) * KB;
-  int kb = 0;
-  if ((KB & 3) == 0) {
-    for (; kb < KB; kb += 4) {
-      const float4 v = *(const float4*)(src + kb);
-      out[(size_t)kb * n + p] = v.x;
-      out[(size_t)(kb + 1) * n + p] = v.y;
-      out[(size_t)(kb + 2) * n + p] = v.z;
-      out[(size_t)(kb + 3) * n + p] = v.w;
+  const float* row = sx + (size_t)(ids ? ids[p] : p) * KB;
+  out += p;
+  for (int kb0 = blockIdx.y * kGatherScales; kb0 < KB; kb0 += gridDim.y * kGatherScales) {
+    const int m = min(kGatherScales, KB - kb0);
+    if ((KB & 3) == 0) {
+      float4 v[kGatherScales / 4];
+#pragma unroll
+      for (int i = 0; i < kGatherScales; i += 4)
+        if (i < m) v[i / 4] = *(const float4*)(row + kb0 + i);
+#pragma unroll
+      for (int i = 0; i < kGatherScales; i += 4) {
+        if (i >= m) break;
+        float* o = out + (size_t)(kb0 + i) * n;
+        o[0] = v[i / 4].x;
+        o[(size_t)n] = v[i / 4].y;
+        o[(size_t)2 * n] = v[i / 4].z;
+        o[(size_t)3 * n] = v[i / 4].w;
+      }
+    } else {
+      for (int i = kb0; i < kb0 + m; ++i) out[(size_t)i * n] = row[i];
     }
   }
-  for (; kb < KB; ++kb) out[(size_t)kb * n + p] = src[kb];
 }
 }  // namespace
 
@@ -243,7 +255,8 @@ extern "C" int moe_gather_scales(const float* sx, const int32_t* row_ids, int n,
   // (rows of a multiple of four scales are read 16 bytes at a time)
   MOE_REQUIRE((KB & 3) || MOE_ALIGNED16(sx), MOE_ERR_BAD_ALIGN, "gather_scales: sx must be 16-byte aligned when KB is a multiple of 4");
   if (n == 0) return MOE_OK;
-  hipLaunchKernelGGL(gather_scales_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, sx, row_ids,
+  const int parts = KB / kGatherScales + (KB % kGatherScales ? 1 : 0);
+  hipLaunchKernelGGL(gather_scales_kernel, dim3((unsigned)((n + 255) / 256), parts < 64 ? parts : 64), dim3(256), 0, (hipStream_t)stream, sx, row_ids,
                      n, KB, out);
   return moe_check_hip(hipGetLastError(), "gather_scales launch");
 }

@@ -394,3 +394,14 @@ def test_batches_of_every_tile_height_give_the_bits_of_a_large_one(jg, routing):
 def test_many_tokens_a_workgroup_are_routed_exactly(jg, M, E, k):
     """8 to 17 tokens of a routing workgroup, of eight waves beside the quantiser; the last one has fewer."""
     test_ready_logits_routed_and_sorted_in_one_launch_or_two(jg, M, E, k)
+
+
+@pytest.mark.parametrize("n,KB", [(1, 1), (257, 3), (300, 4), (255, 16), (70, 17), (513, 20), (256, 56), (5, 64 * 16 + 8), (5, 64 * 16 + 9)])
+def test_scales_are_gathered_whole(jg, n, KB):
+    """Rows of fewer and more scales than a thread takes and than the grid covers at once, a multiple of four or not."""
+    import torch
+    print("scales", n, KB, flush=True)
+    sx = torch.arange(2 * n * KB, dtype=torch.float32, device="cuda").reshape(2 * n, KB)
+    ids = torch.randperm(2 * n, device="cuda")[:n].to(torch.int32)
+    assert torch.equal(jg.gather_scales(sx, ids), sx[ids.long()].t())
+    assert torch.equal(jg.gather_scales(sx, n_rows=n), sx[:n].t())
