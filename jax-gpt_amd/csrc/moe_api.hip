@@ -295,7 +295,8 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
   const bool together = a->SI && !fork;   // the shared expert runs inside the routed launches
   const int tile_rows = moe_gemm_tile_rows(TileShape{R, a->E, a->M, {a->I / 128, (a->D + 255) / 256}, {a->D / 128, a->I / 128},
                                                      together ? a->M : 0, {a->SI / 128, (a->D + 255) / 256}});
-  if ((rc = moe_gemm_tile_list(R, a->E, tile_rows, a->I / 128, (a->D + 255) / 256, b.gemm_ws, b.gemm_ws_bytes, &tiles))) return join(rc);
+  if ((rc = moe_gemm_tile_list(R, a->E, tile_rows, a->I / 128, (a->D + 255) / 256,
+                               (a->I < a->D ? a->I : a->D) / 128, b.gemm_ws, b.gemm_ws_bytes, &tiles))) return join(rc);
   const RouteArgs route{src, a->bias, a->M, a->E, a->k, a->renorm, a->n_group, a->topk_group, a->routed_scale, idx, w_own};
   const PermuteOut sort{gsz, b.group_offsets, stid, nullptr, inv, a->k, tiles};
   const QuantJob* carried = quant_in_route ? &quant_job : nullptr;
@@ -320,10 +321,10 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
     sc.in_row = 1, sc.in_kb = R, sc.in_listed = true;
   }
   const RoutedGemm routed_gateup{{b.xq, sx_routed, stid, a->w_gate, a->sw_gate, a->w_up, a->sw_up, a->D, a->I, hq, sh, sc},
-                                 b.group_offsets, a->E, R, b.gemm_ws, b.gemm_ws_bytes, tile_rows};
+                                 b.group_offsets, a->E, R, b.gemm_ws, b.gemm_ws_bytes, tile_rows, tiles.pool_tiles};
   const RoutedGemm routed_down{{hq, sh, nullptr, a->w_down, a->sw_down, nullptr, nullptr, a->I, a->D, y, nullptr,
                                 GemmScales{sc.out_row, sc.out_cb, true, 0, 0}},
-                               b.group_offsets, a->E, R, b.gemm_ws, b.gemm_ws_bytes, tile_rows};
+                               b.group_offsets, a->E, R, b.gemm_ws, b.gemm_ws_bytes, tile_rows, tiles.pool_tiles};
   if ((rc = moe_gemm_gateup_impl(&routed_gateup, together ? &shared_gateup : nullptr, stream))) return join(rc);
   if ((rc = moe_gemm_down_impl(&routed_down, together ? &shared_down : nullptr, stream))) return join(rc);
   if ((rc = join(MOE_OK))) return rc;

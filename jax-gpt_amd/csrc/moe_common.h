@@ -53,11 +53,14 @@ struct TileHeader {
   long long pad2;
 };
 constexpr int kTileQBits = 20;
-// The pool holds at most max_tiles / 16 tiles, and an XCD may draw up to twice its eighth of it: the grouped GEMM
+// The pool holds at most TileList::pool_tiles tiles, and an XCD may draw up to twice its eighth of it: the grouped GEMM
 // launches this many workgroups per XCD beyond its fixed share for a GEMM of ncb column blocks per row tile.
-constexpr int kPoolShift = 4;    // (a pool of max_tiles / 8 and up to 4 or 6 tail rounds measured 0.5-1 % slower)
-constexpr int kTailRounds = 3;   // rounds of the ranking (8 experts each) that end a bin or go to the pool
-__host__ __device__ inline int moe_pool_tile_limit(int max_tiles) { return max_tiles >> kPoolShift; }
+//   It is max_tiles / 16 (a pool of max_tiles / 8 and up to 4 or 6 tail rounds measured 0.5-1 % slower), or a quarter of
+// max_tiles for lists of a few rounds of long items (moe_gemm_pool_tiles) if the groups are uneven: fixed shares cannot end
+// together there, and a draw (some 1 us) is little beside an item.  Expert-parallel shard, 32 experts of 7168 x 2048 with
+// Zipf(1.2) rows, 1/16, 1/4 and 1/2 of max_tiles: 1600 rows 265 / 253 / 248 us, 2400 294 / 279 / 268, 4800 355 / 337 / 359,
+// 6400 451 / 398 / 409, 8000 470 / 449 / 455, 12000 620 / 604 / 605, 16384 766 / 761 / 768.
+constexpr int kTailRounds = 3, kWideTailRounds = 8;   // rounds of the ranking (8 experts each) that end a bin or go to the pool
 __host__ __device__ inline int moe_pool_workgroups(long long pool_items) { return (int)(pool_items >> 2) + 1; }
 // The grouped GEMM launches ceil(max_tiles * ncb / 8) + 2 workgroups per XCD: a split whose largest share stays
 // within max_tiles / 8 tiles fits whatever ncb is (max_tiles is a worst case over all group sizes, so a real list
@@ -71,6 +74,8 @@ struct TileEntry {
 };
 struct TileList {
   int max_tiles;
+  int pool_tiles;     // more than max_tiles / 16: only where the groups are uneven
+  int rows;           // of all groups
   int tile_rows;      // rows of a full tile: a multiple of 32, at most kTileRows
   TileHeader* hdr;
   TileEntry* tiles;
@@ -157,11 +162,11 @@ __device__ inline int moe_tile_first(int e, int rows, int nt, int* lds_a, int* l
   TileHeader* const hdr = l.hdr;
   const int max_tiles = l.max_tiles;
   __shared__ long long cut_q[9];
-  __shared__ int tail_tiles[kTailRounds];   // tiles of the last, last but one, ... round of the ranking
+  __shared__ int tail_tiles[kWideTailRounds];   // tiles of the last, last but one, ... round of the ranking
   // rank: largest class first, inside a class in any order (1023 = the largest class and everything above it)
   const int cls = rows > 0 ? 1023 - min((rows + 31) >> 5, 1023) : 0;
   lds_a[e] = 0;
-  if (e < kTailRounds) tail_tiles[e] = 0;
+  if (e < kWideTailRounds) tail_tiles[e] = 0;
   __syncthreads();
   const int order = rows > 0 ? atomicAdd(&lds_a[cls], 1) : 0;
   __syncthreads();
@@ -171,7 +176,12 @@ __device__ inline int moe_tile_first(int e, int rows, int nt, int* lds_a, int* l
   __syncthreads();
   const int rank = lds_b[cls] + order;
   const int nr = (nz + 7) >> 3;   // rounds that hold a non-empty expert
-  const int tail = nr / 4 < kTailRounds ? nr / 4 : kTailRounds;   // (3 rounds = 24 experts over the 8 bins; 6 measured no better)
+  int tail = nr / 4 < kTailRounds ? nr / 4 : kTailRounds;   // (3 rounds = 24 experts over the 8 bins; 6 measured no better)
+  int pool_most = max_tiles >> 4;
+  if (l.pool_tiles > pool_most && __syncthreads_or((long long)rows * nz > 2ll * l.rows)) {   // (an expert of twice the mean)
+    tail = nr > kWideTailRounds ? kWideTailRounds : nr - 1;
+    pool_most = l.pool_tiles;
+  }
   const int round = rank >> 3;
   if (rows > 0 && round >= nr - tail) atomicAdd(&tail_tiles[nr - 1 - round], nt);
   __syncthreads();
@@ -179,7 +189,7 @@ __device__ inline int moe_tile_first(int e, int rows, int nt, int* lds_a, int* l
   int pooled = 0;
   for (int t = 0, sum = 0; t < tail; ++t) {
     sum += tail_tiles[t];
-    if (sum > moe_pool_tile_limit(max_tiles)) break;
+    if (sum > pool_most) break;
     pooled = t + 1;
   }
   const int n_fixed = pooled ? (nr - pooled) * 8 : nz;   // experts in fixed shares; the others, last in rank, are the pool
@@ -311,7 +321,8 @@ int moe_permute_place(const int32_t* idx, int R, int E, int chunk, int n_chunks,
 // own.  moe_gemm_tile_list describes the list the GEMMs of (R rows, E experts) expect in ws, so that the permutation
 // kernels, which hold every expert's row range anyway, can write it (moe_permute_impl) and no launch is spent on it.
 // tile_rows: moe_gemm_tile_rows of the GEMMs that will read it.
-int moe_gemm_tile_list(int R, int E, int tile_rows, int ncb_gateup, int ncb_down, void* ws, size_t ws_bytes, TileList* list);
+// kb: fewest K steps of these GEMMs.
+int moe_gemm_tile_list(int R, int E, int tile_rows, int ncb_gateup, int ncb_down, int kb, void* ws, size_t ws_bytes, TileList* list);
 // Rows of a full tile for R rows in E groups and, in the same launches, dense_rows rows of a dense group; [0] gate/up,
 // [1] down: column blocks per row tile and K steps (0: that GEMM does not read the list).
 struct TileShape {
@@ -368,7 +379,7 @@ struct RoutedGemm {
   int E, R;
   void* ws;
   size_t ws_bytes;
-  int list_tile_rows;   // of the list that is there already, or 0: none is
+  int list_tile_rows, list_pool_tiles;   // of the list that is there already, or 0: none is
 };
 // one group of all rows (the shared expert): no list, no workspace
 struct DenseGemm {

@@ -636,9 +636,20 @@ int max_tiles_for(int R, int E, int tile_rows) { return (int)(((long long)R + ti
 // fewest work items at which every launch takes full tiles (moe_gemm_tile_rows)
 constexpr int kFullTileItems = 768;
 
-TileList tile_list(void* ws, int R, int E, int tile_rows, int ncb_gateup, int ncb_down) {
-  return TileList{max_tiles_for(R, E, tile_rows), tile_rows, (TileHeader*)ws, (TileEntry*)((char*)ws + sizeof(TileHeader)),
-                  {ncb_gateup, ncb_down}, {(32 << kTileQBits) / (ncb_gateup ? ncb_gateup : 1), (32 << kTileQBits) / (ncb_down ? ncb_down : 1)}};
+// Lists whose pool may be large: of up to 8 rounds at most (the fewer, the larger a part the last one is; up to 10 the
+// expert-parallel shard of 16384 rows takes 786 us, up to 8 778), of items of 12 K steps (14 us) and more.  Shorter items lose
+// more by the draw (Qwen3-MoE, 2800 tokens 217 -> 221 us, 4000 of the mini layer 76 -> 79.5).
+int moe_gemm_pool_tiles(int max_tiles, int tile_rows, int ncb_least, int kb) {
+  const bool few = (long long)max_tiles * ncb_least <= 8 * 256 && kb >= 12 && tile_rows > kStreamRows;
+  return few ? max_tiles >> 2 : max_tiles >> 4;
+}
+
+// ncb: column blocks of the list's GEMMs (0: none); kb: the fewest K steps of these
+TileList tile_list(void* ws, int R, int E, int tile_rows, int ncb_gateup, int ncb_down, int kb) {
+  const int max_tiles = max_tiles_for(R, E, tile_rows), ncb = ncb_down && ncb_down < ncb_gateup ? ncb_down : ncb_gateup;
+  return TileList{max_tiles, moe_gemm_pool_tiles(max_tiles, tile_rows, ncb, kb), R, tile_rows, (TileHeader*)ws,
+                  (TileEntry*)((char*)ws + sizeof(TileHeader)), {ncb_gateup, ncb_down},
+                  {(32 << kTileQBits) / (ncb_gateup ? ncb_gateup : 1), (32 << kTileQBits) / (ncb_down ? ncb_down : 1)}};
 }
 
 int check_operands(const GemmOperands& op, int rows, int E, int mode, const char* what) {
@@ -696,11 +707,12 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
       routed = rt->op;
       routed.sc.out_through = through(rt->R, rt->E, routed.N);
       l = tile_list(rt->ws, rt->R, rt->E, rt->list_tile_rows ? rt->list_tile_rows : own_tile_rows(rt->R, rt->E, routed),
-                    col_blocks(MODE, routed.N), 0);   // (one launch reads a list that it builds itself)
+                    col_blocks(MODE, routed.N), 0, routed.K / BK);   // (one launch reads a list that it builds itself)
+      if (rt->list_tile_rows) l.pool_tiles = rt->list_pool_tiles;
       // sized by the worst case of the largest XCD share (moe_xcd_share_cap_q) and of an XCD's draws from the pool;
       // surplus workgroups exit at once
       const long long max_items = (long long)l.max_tiles * col_blocks(MODE, routed.N);
-      const long long pool_max = (long long)moe_pool_tile_limit(l.max_tiles) * col_blocks(MODE, routed.N);
+      const long long pool_max = (long long)l.pool_tiles * col_blocks(MODE, routed.N);
       grid += 8 * ((max_items + 7) / 8 + 2 + moe_pool_workgroups(pool_max));
     }
   }
@@ -792,13 +804,13 @@ namespace {
 int gateup(const uint8_t* xq, const float* sx, const int32_t* row_ids, const uint8_t* w_gate, const float* sw_gate,
            const uint8_t* w_up, const float* sw_up, const int32_t* group_offsets, int E, int R, int D, int I, uint8_t* hq,
            float* sh, void* ws, size_t ws_bytes, GemmScales sc, moe_stream_t stream) {
-  const RoutedGemm r{{xq, sx, row_ids, w_gate, sw_gate, w_up, sw_up, D, I, hq, sh, sc}, group_offsets, E, R, ws, ws_bytes, 0};
+  const RoutedGemm r{{xq, sx, row_ids, w_gate, sw_gate, w_up, sw_up, D, I, hq, sh, sc}, group_offsets, E, R, ws, ws_bytes, 0, 0};
   return moe_gemm_gateup_impl(&r, nullptr, stream);
 }
 int down(const uint8_t* hq, const float* sh, const uint8_t* w_down, const float* sw_down, const int32_t* group_offsets, int E,
          int R, int I, int D, void* y_bf16, void* ws, size_t ws_bytes, GemmScales sc, moe_stream_t stream) {
   const RoutedGemm r{{hq, sh, nullptr, w_down, sw_down, nullptr, nullptr, I, D, y_bf16, nullptr, sc}, group_offsets, E, R, ws,
-                     ws_bytes, 0};
+                     ws_bytes, 0, 0};
   return moe_gemm_down_impl(&r, nullptr, stream);
 }
 }  // namespace
@@ -886,10 +898,10 @@ extern "C" int moe_gemm_down_fp8_layout(const uint8_t* hq, const float* sh, cons
 }
 
 // The tile list that the GEMM launches of (R rows, E experts) read from ws when they are told its list_tile_rows.
-int moe_gemm_tile_list(int R, int E, int tile_rows, int ncb_gateup, int ncb_down, void* ws, size_t ws_bytes, TileList* list) {
+int moe_gemm_tile_list(int R, int E, int tile_rows, int ncb_gateup, int ncb_down, int kb, void* ws, size_t ws_bytes, TileList* list) {
   MOE_REQUIRE(ws && list, MOE_ERR_NULL, "gemm tiles: null pointer");
   MOE_REQUIRE(E >= 1 && E <= 1024 && R >= 0, MOE_ERR_BAD_SHAPE, "gemm tiles: need 1 <= E <= 1024, got E=%d R=%d", E, R);
   MOE_REQUIRE(ws_bytes >= moe_gemm_workspace_bytes(R, E, 0), MOE_ERR_WORKSPACE_TOO_SMALL, "gemm tiles: workspace too small");
-  *list = tile_list(ws, R, E, tile_rows, ncb_gateup, ncb_down);
+  *list = tile_list(ws, R, E, tile_rows, ncb_gateup, ncb_down, kb);
   return MOE_OK;
 }

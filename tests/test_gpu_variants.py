@@ -405,3 +405,52 @@ def test_scales_are_gathered_whole(jg, n, KB):
     ids = torch.randperm(2 * n, device="cuda")[:n].to(torch.int32)
     assert torch.equal(jg.gather_scales(sx, ids), sx[ids.long()].t())
     assert torch.equal(jg.gather_scales(sx, n_rows=n), sx[:n].t())
+
+
+@pytest.mark.parametrize("R", [2600, 6100, 9000])
+def test_uneven_groups_that_are_drawn_give_the_same_bits(jg, R):
+    """Few rounds of long items of uneven groups: most of the list is a pool that the XCDs draw from (empty experts, one of
+    many tiles and of one row among them).  And the even split of the same rows, whose pool is small."""
+    import torch
+    E, D, I = 32, 1536, 2048
+    print("uneven groups", R, flush=True)
+    params, rand = _layer(jg, D, E, I, 0, R)
+    p = 1.0 / np.arange(1, E + 1) ** 1.2
+    p[[5, 17, 30]] = 0.0
+    uneven = np.floor(p / p.sum() * (R - 40)).astype(np.int64)
+    uneven[31] = 1
+    uneven[0] += R - uneven.sum()
+    xq, sx = jg.quant_act(rand(R, D))
+    for sizes in (uneven, np.full(E, R // E) + (np.arange(E) < R % E)):
+        off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+        hq, sh = jg.gemm_gateup_swiglu(xq, sx, params["gate_proj"], params["up_proj"], H.to_cuda(off))
+        y = jg.gemm_down(hq, sh, params["down_proj"], H.to_cuda(off))
+        for e in np.flatnonzero(sizes):
+            lo, hi = int(off[e]), int(off[e + 1])
+            one = {n: {k: v[e:e + 1] for k, v in params[n + "_proj"].items()} for n in ("gate", "up", "down")}
+            o1 = H.to_cuda(np.array([0, hi - lo], np.int32))
+            hq1, sh1 = jg.gemm_gateup_swiglu(xq[lo:hi], sx[lo:hi].clone(), one["gate"], one["up"], o1)
+            assert torch.equal(hq1.view(torch.uint8), hq[lo:hi].view(torch.uint8)) and torch.equal(sh1, sh[lo:hi]), f"expert {e}: h"
+            assert torch.equal(jg.gemm_down(hq1, sh1, one["down"], o1), y[lo:hi]), f"expert {e}: y"
+
+
+def test_uneven_routing_of_a_layer_of_few_experts(jg):
+    """The same list inside the layer, written by the sort and read by both GEMMs: the output against its own stages."""
+    import torch
+    D, E, I, k, M = 1664, 16, 2048, 3, 1500
+    print("uneven layer", flush=True)
+    params, rand = _layer(jg, D, E, I, 0, 9)
+    x, lg = rand(M, D), rand(M, E).float() + 1.5 * torch.linspace(1, 0, E, device="cuda")
+    ex = {n: params[n] for n in ("gate_proj", "up_proj", "down_proj")}
+    out, dbg = jg.moe_experts(x, lg, top_k=k, experts=ex, return_debug=True)
+    assert torch.equal(out, jg.moe_experts(x, lg, top_k=k, experts=ex))
+    assert int(dbg["group_sizes"].max()) * E > 2 * M * k
+    off = torch.cat([torch.zeros(1, dtype=torch.int32, device="cuda"), dbg["group_sizes"].cumsum(0).to(torch.int32)])
+    xq, sx = jg.quant_act(x)
+    for e in range(E):
+        lo, hi = int(off[e]), int(off[e + 1])
+        one = {n: {k2: v[e:e + 1] for k2, v in ex[n].items()} for n in ex}
+        o1 = H.to_cuda(np.array([0, hi - lo], np.int32))
+        hq1, sh1 = jg.gemm_gateup_swiglu(xq, sx, one["gate_proj"], one["up_proj"], o1, row_ids=dbg["sorted_token_ids"][lo:hi].clone())
+        assert torch.equal(hq1.view(torch.uint8), dbg["hq"][lo:hi]), f"expert {e}: h"
+        assert torch.equal(jg.gemm_down(hq1, sh1, one["down_proj"], o1), dbg["y"][lo:hi]), f"expert {e}: y"
