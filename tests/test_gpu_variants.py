@@ -454,3 +454,25 @@ def test_uneven_routing_of_a_layer_of_few_experts(jg):
         hq1, sh1 = jg.gemm_gateup_swiglu(xq, sx, one["gate_proj"], one["up_proj"], o1, row_ids=dbg["sorted_token_ids"][lo:hi].clone())
         assert torch.equal(hq1.view(torch.uint8), dbg["hq"][lo:hi]), f"expert {e}: h"
         assert torch.equal(jg.gemm_down(hq1, sh1, one["down_proj"], o1), dbg["y"][lo:hi]), f"expert {e}: y"
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+def test_activations_in_any_strides(jg, dtype):
+    """The layer takes (B, T, D) activations as they lie; the flat entry points take two dimensions and refuse others."""
+    import torch
+    print("strides", dtype, flush=True)
+    params, rand = _layer(jg, 256, 8, 128, 128, 5)
+    x = rand(3, 5, 256).to(getattr(torch, dtype))
+    want = jg.moe_layer(x, params, 2)
+    assert want.shape == x.shape and want.dtype == x.dtype and want.is_contiguous()
+    for other in (x.transpose(0, 1).contiguous().transpose(0, 1), torch.cat([x, x], 2)[..., :256]):
+        assert not other.is_contiguous()
+        got = jg.moe_layer(other, params, 2)
+        assert torch.equal(got, want) and got.is_contiguous()
+    for bad in (x[0, 0], x[None]):
+        with pytest.raises(ValueError):
+            jg.moe_layer(bad, params, 2)
+    ex = {n: params[n] for n in ("gate_proj", "up_proj", "down_proj")}
+    for bad in (x.to(torch.bfloat16), x[0, 0].to(torch.bfloat16)):
+        with pytest.raises(ValueError):
+            jg.moe_experts(bad, rand(15, 8).float(), top_k=2, experts=ex)
