@@ -62,9 +62,52 @@ __device__ __forceinline__ void place_pass(const int32_t* ids, int first, int n,
   }
 }
 
+// The sort of at most kFewRows entries by one workgroup of kPlaceThreads, without counters or barriers: every wave that has
+// experts holds all entries, one a lane, and its threads go through them, eight at a time, for their experts' rows and what
+// stands in front of them.  An expert that has rows has one tile.  With the counters below the same step of the routing launch
+// takes 2.3 to 2.6 us, this way 1.2 for 8 entries and 2.0 for 32 (64: 3.2).
+constexpr int kFewRows = 32;   // (no tile is shorter)
+__device__ __forceinline__ void permute_few(const int32_t* ids, int n, int E, const PermuteOut& o) {
+  const int e = threadIdx.x, lane = e & 63;
+  if (e >= ((E + 63) & ~63)) return;   // (whole waves: no expert is theirs)
+  int id = lane < n ? ids[lane] : -1;
+  if (id >= E) id = -1;   // out-of-range ids are dropped
+  const unsigned long long same = match_any(id, ilog2_ceil(E));
+  const int rank = __popcll(same & ((1ull << lane) - 1ull)), first = id >= 0 && rank == 0;
+  int rows = 0, start = 0, tile = 0, pos = rank;   // (pos: of this lane's entry)
+  for (int j0 = 0; j0 < n; j0 += 8) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {   // (lanes past the last entry hold -1, as dropped ones: above every expert)
+      const unsigned other = (unsigned)__builtin_amdgcn_readlane(id, j0 + i);
+      const int new_expert = __builtin_amdgcn_readlane(first, j0 + i);
+      const bool before = other < (unsigned)e;
+      rows += other == (unsigned)e;
+      start += before;
+      tile += before ? new_expert : 0;
+      pos += other < (unsigned)id;
+    }
+  }
+  if (e < E) {
+    o.group_sizes[e] = rows;
+    o.group_offsets[e] = start;
+    if (e == E - 1) o.group_offsets[E] = start + rows;
+    if (o.tl.tiles && rows && tile < o.tl.max_tiles) o.tl.tiles[tile] = TileEntry{e | 1 << 10, start, rows, tile};
+  }
+  if (o.tl.tiles) {
+    const int all = min((int)__popcll(__ballot(first)), o.tl.max_tiles);
+    if (e == 0) moe_tile_even_shares(o.tl.hdr, all, all);
+  }
+  if (e < n && id >= 0) {
+    if (o.sort_order) o.sort_order[pos] = e;
+    if (o.sorted_token_ids) o.sorted_token_ids[pos] = (int)(((float)e + 0.5f) * __builtin_amdgcn_rcpf((float)o.k));   // e / k
+    if (o.inv_perm) o.inv_perm[e] = pos;
+  }
+}
+
 // The whole sort of one chunk (n entries starting at flat index 0) in one workgroup of kPlaceThreads; ids may be in
 // LDS.  next: moe_place_lds_ints(E) ints of LDS.  The caller synchronises before the call (ids written, LDS free).
 __device__ __forceinline__ void permute_one_chunk(const int32_t* ids, int n, int E, int* next, const PermuteOut& o) {
+  if (n <= kFewRows) return permute_few(ids, n, E, o);
   const int e = threadIdx.x, waves = moe_place_waves(E, n);
   for (int i = threadIdx.x; i < waves * E; i += kPlaceThreads) next[i] = 0;
   __syncthreads();

@@ -476,3 +476,35 @@ def test_activations_in_any_strides(jg, dtype):
     for bad in (x.to(torch.bfloat16), x[0, 0].to(torch.bfloat16)):
         with pytest.raises(ValueError):
             jg.moe_experts(bad, rand(15, 8).float(), top_k=2, experts=ex)
+
+
+@pytest.mark.parametrize("M,k,E", [(1, 1, 1), (1, 8, 256), (4, 8, 64), (31, 1, 65), (32, 1, 1), (1, 32, 1024), (3, 11, 130), (5, 7, 8)])
+def test_few_entries_are_sorted(jg, M, k, E):
+    """Up to 32 entries and one more, any number of one expert among them."""
+    import torch
+    print("few entries", M, k, E, flush=True)
+    rng = H.rng_for(M * 100 + k + E)
+    for idx in (rng.integers(0, E, (M, k)), np.full((M, k), E - 1), np.arange(M * k).reshape(M, k)[::-1] % E):
+        idx = np.ascontiguousarray(idx.astype(np.int32))
+        got, ref = jg.permute(H.to_cuda(idx), E), O.sort_and_group(idx, E)
+        for name in ("group_sizes", "group_offsets", "sorted_token_ids", "sort_order", "inv_perm"):
+            if name in ref:
+                assert np.array_equal(got[name].cpu().numpy(), ref[name]), name
+
+
+@pytest.mark.parametrize("M,k,E", [(4, 8, 24), (8, 4, 24), (16, 2, 8), (11, 3, 24)])
+def test_few_entries_of_a_layer(jg, M, k, E):
+    """The same inside the layer, routed (up to 32 entries are sorted by the routing launch) or given, all rows of one expert too."""
+    import torch
+    print("few entries of a layer", M, k, E, flush=True)
+    params, rand = _layer(jg, 256, E, 256, 0, M)
+    ex = [params[n] for n in ("gate_proj", "up_proj", "down_proj")]
+    x, lg = rand(200, 256), rand(200, E).float()
+    kw = dict(top_k=k, experts=dict(zip(("gate_proj", "up_proj", "down_proj"), ex)))
+    whole = jg.moe_experts(x, lg, **kw)
+    assert torch.equal(jg.moe_experts(x[:M].contiguous(), lg[:M].contiguous(), **kw), whole[:M])
+    w = rand(M, k).float()
+    same = torch.full((M, k), E - 2, dtype=torch.int32, device="cuda")
+    many = same.repeat(20, 1)
+    got = jg.expert_forward_single(x[:M].contiguous(), same, w, *ex)
+    assert torch.equal(got, jg.expert_forward_single(x[:M].repeat(20, 1), many, w.repeat(20, 1), *ex)[:M])
