@@ -18,7 +18,7 @@ LIB_PATH = os.path.join(HERE, "libmoe_hip.so")
 PROBE_PATH = os.path.join(HERE, "libmoe_probe.so")
 
 SOURCES = ["moe_api.hip", "moe_route.hip", "moe_router.hip", "moe_permute.hip", "moe_quant.hip", "moe_gemm.hip", "moe_gemm_stream.hip",
-           "moe_combine.hip"]
+           "moe_token.hip", "moe_combine.hip"]
 # no v_pk_*_f32 code generation (some packed-f32 forms have given wrong results on this hardware)
 COMMON = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function",
           "-fvisibility=hidden",    # only the functions include/moe_hip.h declares (MOE_API) are exported
@@ -29,7 +29,8 @@ PER_FILE = {"moe_route.hip": ["-ffp-contract=off"], "moe_combine.hip": ["-ffp-co
             "moe_router.hip": ["-ffp-contract=off", "-Wno-inline-asm"],
             # MFMA results go straight to VGPRs: the block-scale FMA consumes them on the vector ALU
             "moe_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-Wno-inline-asm"],   # m0 is clobbered on purpose
-            "moe_gemm_stream.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-Wno-inline-asm"]}
+            "moe_gemm_stream.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-Wno-inline-asm"],
+            "moe_token.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-Wno-inline-asm"]}
 
 
 def _hipcc() -> str:

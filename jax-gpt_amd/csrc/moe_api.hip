@@ -8,6 +8,7 @@
 #include <mutex>
 
 #include "moe_common.h"
+#include "moe_token.h"
 
 static thread_local char g_err[512] = "";
 
@@ -87,7 +88,7 @@ struct Carver {
 
 struct ForwardBuffers {
   int32_t *idx, *group_sizes, *group_offsets, *sorted_token_ids, *inv_perm;
-  float *w, *sx, *sh, *shs, *shared_gate, *sx_listed, *sx_blocked;
+  float *h32, *w, *sx, *sh, *shs, *shared_gate, *sx_listed, *sx_blocked;
   uint8_t *xq, *hq, *hsq;
   void *y, *ys, *permute_ws, *gemm_ws, *router_ws, *normed;
   size_t permute_ws_bytes, gemm_ws_bytes, router_ws_bytes, total;
@@ -120,6 +121,8 @@ ForwardBuffers carve(void* ws, int M, int D, int E, int k, int I, int SI, bool r
   b.shs = SI ? (float*)c.take((size_t)M * (SI / 128) * 4) : nullptr;
   b.ys = SI ? c.take((size_t)M * D * 2) : nullptr;
   b.shared_gate = router ? (float*)c.take((size_t)M * 4) : nullptr;
+  const size_t few = M < MOE_TOKEN_ROWS ? M : MOE_TOKEN_ROWS;
+  b.h32 = (float*)c.take(few * (k + 1) * (I > SI ? I : SI) * 4);   // h of single tokens
   b.router_ws_bytes = router ? moe_router_workspace_bytes(M, D, E) : 0;
   b.router_ws = router ? c.take(b.router_ws_bytes) : nullptr;
   b.normed = router ? c.take((size_t)M * D * 2) : nullptr;   // RMS-normalised activations (norm_weight)
@@ -290,6 +293,29 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
     if (a->w_shared_gate) shared_gate = gate_out;
     src = LogitSource{nullptr, (const float*)b.router_ws, splits, n_cols, a->out_logits, gate_out};
   }
+  const RouteArgs route{src, a->bias, a->M, a->E, a->k, a->renorm, a->n_group, a->topk_group, a->routed_scale, idx, w_own};
+  const QuantJob* carried = quant_in_route ? &quant_job : nullptr;
+  // A few tokens whose sort and rows nobody asks for: the experts straight from the selection.  (What the launches that this
+  // leaves out would have refused is refused here.)
+  const bool sorted_outputs = a->out_group_sizes || a->out_sorted_token_ids || a->out_inv_perm || a->out_hq || a->out_hsq || a->out_y || a->out_ys;
+  if (!fork && !sorted_outputs && moe_token_takes(a->M, a->D, a->k, a->I, a->SI)) {
+    const GemmScales sc = moe_row_major_scales(a->D, a->I);
+    if ((rc = moe_gemm_check(GemmOperands{b.xq, b.sx, nullptr, a->w_gate, a->sw_gate, a->w_up, a->sw_up, a->D, a->I, hq, sh, sc}, R, a->E, false))) return rc;
+    if ((rc = moe_gemm_check(GemmOperands{hq, sh, nullptr, a->w_down, a->sw_down, nullptr, nullptr, a->I, a->D, y, nullptr, sc}, R, a->E, true))) return rc;
+    if (a->SI && (rc = moe_gemm_check(shared_gateup.op, a->M, 1, false))) return rc;
+    if (a->SI && (rc = moe_gemm_check(shared_down.op, a->M, 1, true))) return rc;
+    MOE_REQUIRE(MOE_ALIGNED16(a->out) && (!a->add_residual || MOE_ALIGNED16(a->x)), MOE_ERR_BAD_ALIGN,
+                "combine: pointers must be 16-byte aligned");
+    if (given_idx) rc = carried ? moe_quant_act_impl(a->x, io_f32, nullptr, a->M, a->D, b.xq, b.sx, nullptr, stream) : MOE_OK;
+    else rc = moe_route_impl(a->routing, route, carried, nullptr, nullptr, 0, stream);
+    if (rc) return rc;
+    const TokenArgs tok{b.xq, b.sx, given_idx ? given_idx : idx, w,
+                        TokenExperts{a->w_gate, a->w_up, a->w_down, a->sw_gate, a->sw_up, a->sw_down},
+                        TokenExperts{a->ws_gate, a->ws_up, a->ws_down, a->sws_gate, a->sws_up, a->sws_down},
+                        a->M, a->D, a->E, a->k, a->I, a->SI, b.h32, a->I > a->SI ? a->I : a->SI,
+                        shared_gate, a->add_residual ? a->x : nullptr, io_f32, a->out};
+    return moe_token_experts(tok, moe_gemm_from_memory(((long long)a->E * a->I + a->SI) * a->D), stream);
+  }
   // routing, the sort by expert and the routed GEMMs' work list (the sort holds every expert's row range anyway)
   TileList tiles;
   const bool together = a->SI && !fork;   // the shared expert runs inside the routed launches
@@ -297,9 +323,7 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
                                                      together ? a->M : 0, {a->SI / 128, (a->D + 255) / 256}});
   if ((rc = moe_gemm_tile_list(R, a->E, tile_rows, a->I / 128, (a->D + 255) / 256,
                                (a->I < a->D ? a->I : a->D) / 128, b.gemm_ws, b.gemm_ws_bytes, &tiles))) return join(rc);
-  const RouteArgs route{src, a->bias, a->M, a->E, a->k, a->renorm, a->n_group, a->topk_group, a->routed_scale, idx, w_own};
   const PermuteOut sort{gsz, b.group_offsets, stid, nullptr, inv, a->k, tiles};
-  const QuantJob* carried = quant_in_route ? &quant_job : nullptr;
   rc = given_idx ? moe_permute_impl(given_idx, a->M, a->k, a->E, sort, b.permute_ws, b.permute_ws_bytes, carried, stream)
                  : moe_route_impl(a->routing, route, carried, &sort, b.permute_ws, b.permute_ws_bytes, stream);
   if (rc) return join(rc);

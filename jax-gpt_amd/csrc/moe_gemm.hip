@@ -669,6 +669,13 @@ int check_operands(const GemmOperands& op, int rows, int E, int mode, const char
   return MOE_OK;
 }
 
+}  // namespace
+
+int moe_gemm_check(const GemmOperands& op, int rows, int E, bool down) {
+  return check_operands(op, rows, E, down ? MODE_DOWN : MODE_GATEUP, down ? "gemm_down" : "gemm_gateup");
+}
+namespace {
+
 template <int MODE>
 int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
   const char* what = MODE == MODE_GATEUP ? "gemm_gateup" : "gemm_down";
@@ -724,13 +731,13 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
   // 46.6 -> 45.4 us, 64 tokens of the DeepSeek-V3 layer 12 %) and cost
   //  - a third where the memory-side cache (256 MB) still holds the weights from the call before (the same four experts
   //    over and over 29.3 / 44.9 us; tiny layer, 64 tokens 23.9 / 26.0, 256 25.3 / 27.3; mini sublayer, 64 tokens 36.9 /
-  //    39.5, 256 37.8 / 40.6): layers of up to 192 MB, three projections of this size, go without;
+  //    39.5, 256 37.8 / 40.6): layers of up to 192 MB, three projections of this size, go without (moe_gemm_from_memory);
   //  - as much where the several short tiles of a small problem's experts read the same lines (four experts of 7168 x 2048
   //    from memory, 40 rows each 49.7 / 55.0 us, 200 51.8 / 60.6; tiny layer, 2048 tokens 48.9 / 52.1).
-  const long long layer_bytes = (rt ? 3ll * rt->E * rt->op.N * rt->op.K : 0) + (dn ? 3ll * dn->op.N * dn->op.K : 0);
+  const bool from_memory = moe_gemm_from_memory((rt ? 1ll * rt->E * rt->op.N * rt->op.K : 0) + (dn ? 1ll * dn->op.N * dn->op.K : 0));
   const bool shared_lines = l.hdr ? l.tile_rows <= 128 && rt->R > (long long)once_tiles(routed.K) * l.tile_rows * rt->E
                                   : dense_tiles > once_tiles(dense.K) && dense_rows <= 128 * dense_tiles;
-  const bool stream = layer_bytes > (192ll << 20) && !shared_lines;
+  const bool stream = from_memory && !shared_lines;
   const int tallest = l.hdr ? l.tile_rows : dense_tile_rows;   // (a dense group beside routed ones is cut as their list is)
   long long items = dn ? (long long)dense_tiles * col_blocks(MODE, dense.N) : 0;
   if (l.hdr) items += (long long)(rt->E < rt->R ? rt->E : rt->R) * col_blocks(MODE, routed.N);

@@ -1,0 +1,28 @@
+// The experts of single tokens (moe_token.hip).
+#pragma once
+#include "moe_common.h"
+
+constexpr int MOE_TOKEN_ROWS = 16;    // tokens
+constexpr int MOE_TOKEN_SLOTS = 33;   // k <= 32 and the shared expert
+
+struct TokenExperts {   // (E, N, K) codes and block scales
+  const uint8_t *w_gate, *w_up, *w_down;
+  const float *s_gate, *s_up, *s_down;
+};
+struct TokenArgs {
+  const uint8_t* xq;   // (M, D) codes and their (M, D / 128) scales
+  const float* sx;
+  const int32_t* idx;  // (M, k)
+  const float* w;
+  TokenExperts routed, shared;
+  int M, D, E, k, I, SI;   // (SI 0: no shared expert)
+  float* h;                // (M, k + 1, h_stride) f32
+  int h_stride;            // the wider of I and SI
+  const float* shared_gate;
+  const void* residual;
+  int io_f32;              // of residual and out
+  void* out;
+};
+// whether a call of M tokens takes this route
+bool moe_token_takes(int M, int D, int k, int I, int SI);
+int moe_token_experts(const TokenArgs& a, bool from_memory, moe_stream_t stream);

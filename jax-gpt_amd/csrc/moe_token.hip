@@ -1,0 +1,276 @@
+// The experts of single tokens: gate/up, then down and combine, without a sort, a work list or y rows.
+//
+// A token's k experts (and the shared one) are k independent products of one row, so nothing has to be grouped: a workgroup
+// takes its expert from the selection itself.  Replaces jax_gpt/models/qwen35/moe.py:58-94 (sort, grouped SwiGLU, scatter
+// back), :225-232 and :281 for that batch size.  The grouped GEMMs' arithmetic, instruction for instruction (the same bits):
+// one v_mfma_f32_16x16x128_f8f6f4 a scale block, f32 accumulation on the vector ALU, SwiGLU in f32, 1x128 e4m3 quantisation
+// of h, bf16 rows, f32 sums in slot order.
+//   What bounds it: the stream of the experts' weights, and in small layers each launch's start and its chain of dependent
+// loads.  The grouped kernels give one token k * I / 128 work items of 256 weight rows (144 of the DeepSeek-V3 layer, 48 of
+// the Qwen3-MoE layer, on 256 CUs) because a quantisation group of h must not cross workgroups.  Here h stays in f32 between
+// the two launches and every wave of the second quantises the row that it multiplies -- a few KB from L2 -- so the first
+// launch's workgroups can be single waves of 16 columns (1152 and 384).  In the second a workgroup owns tiles of 16 output
+// columns of a token, one wave a slot, and adds the slots up itself: no y, no third launch.  Against the grouped route (us,
+// one token): DeepSeek-V3 layer 84 -> 76, Qwen3-MoE 28 -> 20, full layer behind its norm 57.5 -> 45, mini 31 -> 27, tiny
+// 23 -> 20; five tokens of Qwen3-MoE 46 -> 38.5, eight 55 -> 50.5; sixteen of the mini layer 34 -> 30.5, of tiny 23 -> 20.
+//   Rings of two K steps: more bytes in flight per wave lose (one token of DeepSeek-V3: rings of 2 / 3 / 4 / 6 steps 75.6 /
+// 76.8 / 78.1 / 88.2 in the first launch, 2 / 3 / 4 / 8 in the second 76.2 / 75.3 / 81.9 / 93.9).  Workgroups of four waves in
+// the first: 85.8, as 288 of them are uneven on 256 CUs.
+#include "moe_token.h"
+
+namespace {
+
+constexpr int BK = 128;
+constexpr int COLS = 16;         // output columns of a wave
+constexpr int STAGES = 2;        // K steps of a wave's ring
+constexpr int DOWN_TILES = 16;   // most tiles of a workgroup of the second launch
+constexpr int kLds = 160 * 1024, kDownLds = kLds - 8192;   // (the second launch has 5.3 KB of static LDS)
+
+template <int N> __device__ __forceinline__ void wait_copies() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
+// One wave's products of a row with tiles of FRAGS fragments of 16 weight rows, each fragment of a matrix of its own and the
+// tiles `stride` bytes apart: one stream of K steps through a ring, also from one tile to the next.
+// LDS: rows of 128 bytes, 16-byte chunk c of row r at c ^ ((r >> 1) & 7), as in the grouped kernels.
+template <int FRAGS, bool ONCE>
+struct WaveRows {
+  const uint8_t* w[FRAGS];   // the next K step to copy
+  unsigned off[2];
+  unsigned lds;              // the ring's LDS address
+  int KB, left, to_copy, copy_kb, slot;
+  size_t next_tile;          // from a tile's last K step to the next one's first
+
+  __device__ __forceinline__ void start(const uint8_t* const (&rows)[FRAGS], int K, int tiles, size_t stride, unsigned ring) {
+    const int lane = threadIdx.x & 63, drow = lane >> 3, piece = (lane & 7) ^ (drow >> 1);
+    KB = K / BK, lds = ring, left = to_copy = tiles * KB, copy_kb = 0, slot = 0, next_tile = stride - (size_t)(K - BK);
+#pragma unroll
+    for (int f = 0; f < FRAGS; ++f) w[f] = rows[f];
+    off[0] = (unsigned)drow * (unsigned)K + piece * 16;
+    off[1] = (unsigned)(drow + 8) * (unsigned)K + (piece ^ 4) * 16;
+    for (int t = 0; t < STAGES && to_copy; ++t) copy(t);
+  }
+  __device__ __forceinline__ void copy(int to) {
+    const size_t step = ++copy_kb == KB ? next_tile : BK;
+    if (copy_kb == KB) copy_kb = 0;
+#pragma unroll
+    for (int f = 0; f < FRAGS; ++f) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const unsigned dst = lds + (unsigned)(to * FRAGS + f) * (16 * BK) + g * 1024u;
+        if (ONCE) dma16_nt(w[f], off[g], dst);
+        else dma16(w[f], off[g], dst);
+      }
+      w[f] += step;
+    }
+    --to_copy;
+  }
+  // The next tile.  codes: the row's K codes in LDS; scale(kb, f): the product of its scale and the weights' for fragment f
+  template <class Scale>
+  __device__ __forceinline__ void run(const uint8_t* ring, const uint8_t* codes, v4f (&acc)[FRAGS], const Scale& scale) {
+    const int lane = threadIdx.x & 63, fr = lane & 15, fq = lane >> 4;
+    const int lane_off0 = fr * BK + ((fq ^ (fr >> 1)) << 4), lane_off1 = fr * BK + (((fq + 4) ^ (fr >> 1)) << 4);
+    for (int kb = 0; kb < KB; ++kb, --left) {
+      if (left > 1) wait_copies<2 * FRAGS>();     // the next step's copies may be under way
+      else wait_copies<0>();
+      static_assert(STAGES == 2, "");
+      v8i wf[FRAGS];
+#pragma unroll
+      for (int f = 0; f < FRAGS; ++f) {
+        const uint8_t* base = ring + (slot * FRAGS + f) * (16 * BK);
+        const v4i lo = *(const v4i*)(base + lane_off0), hi = *(const v4i*)(base + lane_off1);
+        wf[f] = (v8i){lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      }
+      // all sixteen columns of the matrix instruction are this row: the lanes of a quarter read one address
+      const v4i lo = *(const v4i*)(codes + kb * BK + fq * 16), hi = *(const v4i*)(codes + kb * BK + 64 + fq * 16);
+      const v8i xf = (v8i){lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      float c[FRAGS];
+#pragma unroll
+      for (int f = 0; f < FRAGS; ++f) c[f] = scale(kb, f);
+      if (to_copy) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the fragments are in registers: the stage may be overwritten
+        copy(slot);
+      }
+      slot = slot + 1 == STAGES ? 0 : slot + 1;
+#pragma unroll
+      for (int f = 0; f < FRAGS; ++f) {
+        const v4f p = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[f], xf, (v4f){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+        acc[f] += p * c[f];
+      }
+    }
+  }
+};
+
+__host__ __device__ constexpr int up_lds(int D) { return STAGES * 32 * BK + D + D / BK * 4 * 3; }
+
+template <bool ONCE>
+__global__ __launch_bounds__(64) void token_gateup_kernel(const TokenArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const int lane = threadIdx.x, t = blockIdx.y;
+  const int per = a.I / COLS, b = blockIdx.x, KB = a.D / BK;
+  const bool shared = b >= a.k * per;
+  const int slot = shared ? a.k : b / per, col = (b - slot * per) * COLS;
+  const TokenExperts& x = shared ? a.shared : a.routed;
+  const int N = shared ? a.SI : a.I;
+  const int e = __builtin_amdgcn_readfirstlane(shared ? 0 : a.idx[(size_t)t * a.k + slot]);
+  if (!shared && (unsigned)e >= (unsigned)a.E) return;   // (an index out of range: the second launch leaves its row out)
+  uint8_t* codes = lds + STAGES * 32 * BK;
+  float* sx = (float*)(codes + a.D);
+  float* sw = sx + KB;   // [2][KB]
+  const size_t row = ((size_t)e * N + col) * a.D;
+  WaveRows<2, ONCE> rows;
+  rows.start({x.w_gate + row, x.w_up + row}, a.D, 1, 0, __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)lds));
+  for (int i = lane; i < a.D / 16; i += 64) ((v4i*)codes)[i] = ((const v4i*)(a.xq + (size_t)t * a.D))[i];
+  const size_t block = ((size_t)e * (N / BK) + col / BK) * KB;
+  for (int i = lane; i < KB; i += 64) {
+    sx[i] = a.sx[(size_t)t * KB + i];
+    sw[i] = x.s_gate[block + i];
+    sw[KB + i] = x.s_up[block + i];
+  }
+  __syncthreads();
+  v4f acc[2] = {};
+  rows.run(lds, codes, acc, [&](int kb, int f) { return sx[kb] * sw[f * KB + kb]; });
+  v4f h;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float g = acc[0][r], u = acc[1][r];
+    h[r] = g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u;
+  }
+  if ((lane & 15) == 0) *(v4f*)(a.h + ((size_t)t * (a.k + 1) + slot) * a.h_stride + col + (lane >> 4) * 4) = h;
+}
+
+// LDS of a wave of the second launch: ring, codes and scales of its row, the weights' scales of its tiles
+__host__ __device__ constexpr int down_wave_lds(int I, int tiles) {
+  return STAGES * 16 * BK + I + ((tiles + 1) * (I / BK) * 4 + 15) / 16 * 16;
+}
+
+// A workgroup: `tiles` neighbouring tiles of 16 output columns of a token; a wave: a slot's row (several, if there are more
+// slots than waves; then tiles is 1).
+template <bool ONCE>
+__global__ __launch_bounds__(1024) void token_down_kernel(const TokenArgs a, const int tiles) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  __shared__ float y[2][MOE_TOKEN_SLOTS][COLS];
+  __shared__ float weight[MOE_TOKEN_SLOTS];
+  __shared__ float residual[DOWN_TILES * COLS];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
+  const int t = blockIdx.y, first = blockIdx.x * tiles, count = min(tiles, a.D / COLS - first), slots = a.k + (a.SI > 0);
+  uint8_t* ring = lds + w * down_wave_lds(a.h_stride, tiles);
+  uint8_t* codes = ring + STAGES * 16 * BK;
+  float* sx = (float*)(codes + a.h_stride);
+  float* sw = sx + a.h_stride / BK;   // [tile][kb]
+  const unsigned ring_at = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)ring);
+  if (w == waves - 1) {   // what the sums need, before copies are under way
+    for (int i = lane; i < slots; i += 64) weight[i] = i < a.k ? a.w[(size_t)t * a.k + i] : a.shared_gate ? a.shared_gate[t] : 0.f;
+    const size_t at = (size_t)t * a.D + first * COLS;
+    if (a.residual)
+      for (int i = lane; i < count * COLS; i += 64)
+        residual[i] = bf16_to_f32(a.io_f32 ? f32_to_bf16(((const float*)a.residual)[at + i]) : ((const bf16_t*)a.residual)[at + i]);
+  }
+  WaveRows<1, ONCE> rows;
+  int e = 0;   // (of the wave's only slot, where there are several tiles)
+  for (int j = 0; j < count; ++j) {
+    for (int slot = w; slot < slots; slot += waves) {
+      const bool shared = slot == a.k;
+      const int K = shared ? a.SI : a.I, KB = K / BK;
+      if (j == 0) e = __builtin_amdgcn_readfirstlane(shared ? 0 : a.idx[(size_t)t * a.k + slot]);
+      v4f acc[1] = {};
+      if (shared || (unsigned)e < (unsigned)a.E) {
+        if (j == 0) {
+          const TokenExperts& x = shared ? a.shared : a.routed;
+          rows.start({x.w_down + ((size_t)e * a.D + first * COLS) * K}, K, count, (size_t)COLS * K, ring_at);
+          for (int i = lane; i < count * KB; i += 64) {
+            const int tile = i / KB;
+            sw[i] = x.s_down[((size_t)e * (a.D / BK) + (first + tile) * COLS / BK) * KB + i - tile * KB];
+          }
+          // the row's quantisation groups, 32 lanes each
+          const float* h = a.h + ((size_t)t * (a.k + 1) + slot) * a.h_stride;
+          for (int i = lane; i < (K / 4 + 63) / 64 * 64; i += 64) {
+            const bool ok = i < K / 4;
+            const v4f v = ok ? ((const v4f*)h)[i] : (v4f){0.f, 0.f, 0.f, 0.f};
+            float m = 0.f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) m = fmaxf(m, fabsf(v[r]));
+#pragma unroll
+            for (int o = 1; o < 32; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, MOE_WAVE));
+            float scale, scale_inv;
+            fp8_scales(m, scale, scale_inv);
+            int q = 0;
+            q = __builtin_amdgcn_cvt_pk_fp8_f32(__builtin_amdgcn_fmed3f(v[0] * scale, -MOE_FP8_MAX, MOE_FP8_MAX),
+                                                __builtin_amdgcn_fmed3f(v[1] * scale, -MOE_FP8_MAX, MOE_FP8_MAX), q, false);
+            q = __builtin_amdgcn_cvt_pk_fp8_f32(__builtin_amdgcn_fmed3f(v[2] * scale, -MOE_FP8_MAX, MOE_FP8_MAX),
+                                                __builtin_amdgcn_fmed3f(v[3] * scale, -MOE_FP8_MAX, MOE_FP8_MAX), q, true);
+            if (ok) {
+              ((int*)codes)[i] = q;
+              if ((i & 31) == 0) sx[i >> 5] = scale_inv;
+            }
+          }
+        }
+        rows.run(ring, codes, acc, [&](int kb, int) { return sx[kb] * sw[j * KB + kb]; });
+      }
+      if ((lane & 15) == 0) {   // the row in bf16
+        const unsigned lo = pack2_bf16(acc[0][0], acc[0][1]), hi = pack2_bf16(acc[0][2], acc[0][3]);
+        float* dst = y[j & 1][slot] + 4 * (lane >> 4);
+        dst[0] = __uint_as_float(lo << 16), dst[1] = __uint_as_float(lo & 0xffff0000u);
+        dst[2] = __uint_as_float(hi << 16), dst[3] = __uint_as_float(hi & 0xffff0000u);
+      }
+    }
+    // this tile's rows are there (and those of the one before have been read: the sums below precede the next barrier);
+    // copies stay under way
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (tid < COLS) {
+#pragma clang fp contract(off)
+      float s = 0.f;
+      for (int i = 0; i < a.k; ++i) s = s + y[j & 1][i][tid] * weight[i];
+      if (a.SI > 0) s = s + (a.shared_gate ? y[j & 1][a.k][tid] * weight[a.k] : y[j & 1][a.k][tid]);
+      if (a.residual) s = s + residual[j * COLS + tid];
+      const size_t at = (size_t)t * a.D + (first + j) * COLS + tid;
+      const bf16_t o = f32_to_bf16(s);
+      if (a.io_f32) ((float*)a.out)[at] = bf16_to_f32(o);
+      else ((bf16_t*)a.out)[at] = o;
+    }
+  }
+}
+
+int launch_gateup(const TokenArgs& a, bool from_memory, hipStream_t s) {
+  static std::atomic<unsigned long long> raised[2] = {};
+  auto* kernel = from_memory ? token_gateup_kernel<true> : token_gateup_kernel<false>;
+  if (int rc = moe_raise_lds_limit((const void*)kernel, kLds, raised[from_memory])) return rc;
+  hipLaunchKernelGGL(kernel, dim3((a.k * a.I + a.SI) / COLS, a.M), dim3(64), up_lds(a.D), s, a);
+  return moe_check_hip(hipGetLastError(), "token gate/up launch");
+}
+
+// Up to a workgroup per CU, each with as many tiles as that takes: a row is quantised once, the copies run on from tile to
+// tile, and no CU has a second workgroup of about 80 KB of LDS to begin (full layer, 2 tokens, workgroups of 2 tiles against
+// 512 of one: 70.1 / 74.3 us; mini, 8: 31.3 / 32.9; one workgroup more than there are CUs -- 6 tokens of Qwen3-MoE in 258 --
+// 46.3 against 43.4 in 192).
+int launch_down(const TokenArgs& a, bool from_memory, hipStream_t s) {
+  static std::atomic<unsigned long long> raised[2] = {};
+  auto* kernel = from_memory ? token_down_kernel<true> : token_down_kernel<false>;
+  if (int rc = moe_raise_lds_limit((const void*)kernel, kDownLds, raised[from_memory])) return rc;
+  const int slots = a.k + (a.SI > 0), cols = a.D / COLS;
+  int tiles = 1;
+  while (tiles < DOWN_TILES && (cols + tiles - 1) / tiles * a.M > 256) ++tiles;
+  if (slots > 16 || slots * down_wave_lds(a.h_stride, tiles) > kDownLds) tiles = 1;   // (a wave of several slots)
+  const int per_wave = down_wave_lds(a.h_stride, tiles), fit = kDownLds / per_wave, most = fit < 16 ? fit : 16;
+  const int waves = slots < most ? slots : most;
+  hipLaunchKernelGGL(kernel, dim3((cols + tiles - 1) / tiles, a.M), dim3(64 * waves), waves * per_wave, s, a, tiles);
+  return moe_check_hip(hipGetLastError(), "token down launch");
+}
+
+}  // namespace
+
+// Every token reads its experts itself, where the grouped kernels read an expert once for all its rows, and 16-row streams
+// run at about 6 TB/s against their 6.9: what the launches left out and the finer split gain (7 to 13 us) covers that up to
+// some 300 MB of weights (Qwen3-MoE, 8 tokens = 302 MB 55.4 -> 50.6 us, 10 = 377 MB 60.6 -> 67.3; full
+// layer, 2 tokens = 277 MB 74.2 -> 69.4, 3 = 415 MB 87.2 -> 94.5; DeepSeek-V3, 2 tokens = 793 MB 113.6 -> 130).  One token
+// reads nothing twice and gains at any size (396 MB of DeepSeek-V3: 84 -> 76).  Of layers this small that keeps up to 16
+// tokens: at 24 the mini layer and tiny are even (34.6 / 34.9, 22.1 / 22.2), at 48 36 -> 47 and 23.4 -> 31.7.
+bool moe_token_takes(int M, int D, int k, int I, int SI) {
+  const int widest = I > SI ? I : SI;
+  if (M < 1 || M > MOE_TOKEN_ROWS || k < 1 || k >= MOE_TOKEN_SLOTS || up_lds(D) > kLds || down_wave_lds(widest, 1) > kDownLds) return false;
+  return M == 1 || 3ll * M * ((long long)k * I + SI) * D <= (320ll << 20);
+}
+
+int moe_token_experts(const TokenArgs& a, bool from_memory, moe_stream_t stream) {
+  hipStream_t s = (hipStream_t)stream;
+  if (int rc = launch_gateup(a, from_memory, s)) return rc;
+  return launch_down(a, from_memory, s);
+}

@@ -508,3 +508,52 @@ def test_few_entries_of_a_layer(jg, M, k, E):
     many = same.repeat(20, 1)
     got = jg.expert_forward_single(x[:M].contiguous(), same, w, *ex)
     assert torch.equal(got, jg.expert_forward_single(x[:M].repeat(20, 1), many, w.repeat(20, 1), *ex)[:M])
+
+
+@pytest.mark.parametrize("M,D,E,k,I,SI", [
+    (1, 128, 8, 2, 128, 0),       # one K step, eight tiles
+    (16, 512, 8, 2, 1024, 0),     # the most tokens, tiles of different scale blocks in a workgroup
+    (13, 384, 33, 3, 256, 384),   # tiles that do not divide, a shared expert wider than the routed ones
+    (3, 896, 40, 17, 128, 128),   # more slots than waves
+    (2, 256, 40, 32, 256, 128),   # the most slots
+    (16, 4096, 4, 1, 128, 128),   # sixteen tiles a workgroup
+    (1, 2048, 8, 8, 2432, 128),   # rows whose rings do not fit beside each other for every slot
+    (1, 7168, 16, 8, 512, 512),   # one token of a layer from memory (non-temporal copies)
+])
+@pytest.mark.parametrize("f32", [False, True])
+def test_experts_of_single_tokens_give_the_grouped_bits(jg, M, D, E, k, I, SI, f32):
+    """Batches that go from the selection straight to the experts: the bits of the grouped kernels (the call that returns
+    the sorted intermediates), routed or given, with norm, gate and residual, also where h or the rows hold infinities and NaN."""
+    import torch
+    print("single tokens", M, D, E, k, I, SI, f32, flush=True)
+    params, rand = _layer(jg, D, E, I, SI, M + D)
+    names = ("gate_proj", "up_proj", "down_proj")
+    ex = {n: params[n] for n in names}
+    x = rand(M, D)
+    for hard in (False, True):
+        if hard:
+            x[0, 5], x[M - 1, D - 1] = 3e38, -3e38
+            if M > 2:
+                x[1, 0], x[2, 1] = float("inf"), float("nan")
+        kw = dict(top_k=k, experts=ex, gate_weight=params["gate_weight"])
+        if SI:
+            kw.update(shared={n: params["shared_" + n] for n in names}, norm_weight=torch.rand(D, device="cuda") + 0.5,
+                      shared_expert_gate_weight=params["shared_expert_gate_weight"], add_residual=True)
+        if f32:
+            fwd = lambda **o: jg.moe._forward(x.float(), None, io_f32=True, **kw, **o)
+        else:
+            fwd = lambda **o: jg.moe_experts(x, None, **kw, **o)
+        want, dbg = fwd(return_debug=True)
+        assert torch.equal(fwd().nan_to_num(7.0), want.nan_to_num(7.0))
+        if not SI:
+            got = jg.expert_forward_single(x, dbg["indices"], dbg["weights"], *(params[n] for n in names))
+            assert torch.equal(got.nan_to_num(7.0), want.to(got.dtype).nan_to_num(7.0))
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = fwd()
+    for i in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.nan_to_num(7.0), want.nan_to_num(7.0)), f"replay {i}"
