@@ -238,9 +238,9 @@ __device__ __forceinline__ int route_grouped_token(const RouteArgs& a, const flo
 }
 
 // Columns [0, n) of the partial sums at p, added in slice order by the whole workgroup and rounded to bf16 (what the
-// router's own finishing pass computes).  The loads are what it waits for, so a thread has up to 8 slices of C columns
-// under way: past the last slice or column it reads the last one again.  (One column and batches of 8, 4, 1, 1, ...: the
-// launch took 24 us for 2047 tokens of 513 columns in 7 slices, 20 now.)
+// router's own finishing pass computes).  The loads are what it waits for, so a thread has 8 slices of two columns or 16
+// of one under way: past the last slice or column it reads the last one again.  (One column and batches of 8, 4, 1, 1, ...:
+// the launch took 24 us for 2047 tokens of 513 columns in 7 slices, 20 now.)
 template <int Z, int C>
 __device__ __forceinline__ void add_slices(float (&s)[C], const float* const (&q)[C], size_t slice, int z, int splits) {
   float v[Z][C];
@@ -261,6 +261,8 @@ __device__ __forceinline__ void sum_partials(const float* p, size_t slice, int s
 #pragma unroll
     for (int c = 0; c < C; ++c) q[c] = p + min(i0 + c * (int)blockDim.x, n - 1);
     int z = 0;
+    if (C == 1)
+      for (; splits - z > 8; z += 16) add_slices<16, C>(s, q, slice, z, splits);
     for (; splits - z > 4; z += 8) add_slices<8, C>(s, q, slice, z, splits);
     if (splits - z > 1) add_slices<4, C>(s, q, slice, z, splits);
     else if (splits - z == 1) add_slices<1, C>(s, q, slice, z, splits);
@@ -406,7 +408,10 @@ int moe_route_impl(int routing, const RouteArgs& a, const QuantJob* quant, const
   // sixteen fits beside another on a CU only when all of its slots are free, and the quantiser's blocks stood waiting.
   // Qwen3-MoE, 4096 tokens 14.7 -> 11.0 us, 4000 of the mini layer 9.4 -> 8.4, 8000 of the tiny layer 10.0 -> 9.3 (four waves
   // 16.1, 11.9 and 13.9); without it 2500 tokens of the mini layer from f32 take 66.7 us with sixteen, 68.4 with eight.
-  const int threads = sort_here || (tpb >= 8 && !quant) ? 1024 : tpb >= 8 ? 512 : 256;
+  //   A token whose partial sums are the work and that has a CU to itself: a thread a column (513 columns in 32 slices: the
+  // launch 10.5 -> 9.2 us for 1 token, 12.0 -> 10.6 for 200).
+  const bool own_cu = a.src.partial && tpb == 1 && a.M <= kCUs;
+  const int threads = sort_here || (tpb >= 8 && !quant) || (own_cu && a.src.N > 512) ? 1024 : tpb >= 8 || (own_cu && a.src.N > 256) ? 512 : 256;
   job.tokens_per_block = tpb;
   job.blocks = (a.M + tpb - 1) / tpb;
   job.chunk_hist = counts ? (int32_t*)permute_ws : nullptr;

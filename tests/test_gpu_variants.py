@@ -557,3 +557,19 @@ def test_experts_of_single_tokens_give_the_grouped_bits(jg, M, D, E, k, I, SI, f
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out.nan_to_num(7.0), want.nan_to_num(7.0)), f"replay {i}"
+
+
+@pytest.mark.parametrize("E", [256, 257, 512, 640])
+@pytest.mark.parametrize("M,D", [(1, 4096), (3, 2304), (256, 1152), (257, 2176)])
+def test_partial_sums_of_wide_routers(jg, M, D, E):
+    """Routing that adds the router's partial sums itself (9, 17, 18 and 32 slices; a thread a column up to 256 tokens)
+    selects what the router's own logits select."""
+    import torch
+    print("wide routers", M, D, E, flush=True)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + E)
+    x = torch.randn((M, D), dtype=torch.bfloat16, device="cuda", generator=gen)
+    gate = torch.randn((E, D), dtype=torch.bfloat16, device="cuda", generator=gen).mul_(0.02).t()
+    idx, w = jg.moe_routing(x, gate, 7)
+    want_idx, want_w = jg.route_softmax_topk(jg.router_logits(x, gate), 7)
+    assert torch.equal(idx.reshape(M, 7), want_idx) and torch.equal(w.reshape(M, 7), want_w.to(w.dtype))
