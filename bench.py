@@ -43,8 +43,8 @@ def measured_traffic(workload, kernel="gateup_routed"):
     return None, None
 
 
-GATEUP_NAME = "grouped_gemm_kernel<0, ..>, routed launch (gate/up + SwiGLU + h quantisation)"
-DOWN_NAME = "grouped_gemm_kernel<1, ..>, routed launch (down, bf16 rows)"
+GATEUP_NAME = "grouped_gemm_kernel<0, ..> or, short tiles, stream_gemm_kernel<0, ..>, routed launch (gate/up + SwiGLU + h quantisation)"
+DOWN_NAME = "grouped_gemm_kernel<1, ..> or, short tiles, stream_gemm_kernel<1, ..>, routed launch (down, bf16 rows)"
 
 
 def kernel_roofline(bound, kern, workload, kernel_key, name):
