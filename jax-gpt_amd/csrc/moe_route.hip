@@ -238,9 +238,10 @@ __device__ __forceinline__ int route_grouped_token(const RouteArgs& a, const flo
 }
 
 // Columns [0, n) of the partial sums at p, added in slice order by the whole workgroup and rounded to bf16 (what the
-// router's own finishing pass computes).  The loads are what it waits for, so a thread has 8 slices of two columns or 16
-// of one under way: past the last slice or column it reads the last one again.  (One column and batches of 8, 4, 1, 1, ...:
-// the launch took 24 us for 2047 tokens of 513 columns in 7 slices, 20 now.)
+// router's own finishing pass computes).  The loads are what it waits for, so a thread has up to 8 slices of C columns
+// under way: past the last slice or column it reads the last one again.  (One column and batches of 8, 4, 1, 1, ...: the
+// launch took 24 us for 2047 tokens of 513 columns in 7 slices, 20 now.  Sixteen slices of one column: 9.2 against 9.3 us for
+// 1 token of 32 slices, and the code alone costs 0.7 us where there are few: mini layer, 3000 tokens 5.2 -> 6.0.)
 template <int Z, int C>
 __device__ __forceinline__ void add_slices(float (&s)[C], const float* const (&q)[C], size_t slice, int z, int splits) {
   float v[Z][C];
@@ -261,8 +262,6 @@ __device__ __forceinline__ void sum_partials(const float* p, size_t slice, int s
 #pragma unroll
     for (int c = 0; c < C; ++c) q[c] = p + min(i0 + c * (int)blockDim.x, n - 1);
     int z = 0;
-    if (C == 1)
-      for (; splits - z > 8; z += 16) add_slices<16, C>(s, q, slice, z, splits);
     for (; splits - z > 4; z += 8) add_slices<8, C>(s, q, slice, z, splits);
     if (splits - z > 1) add_slices<4, C>(s, q, slice, z, splits);
     else if (splits - z == 1) add_slices<1, C>(s, q, slice, z, splits);
