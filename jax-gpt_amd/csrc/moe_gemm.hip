@@ -768,6 +768,7 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
 // 1380 where 81 experts have 128 to 493).  A shared expert beside them is cut alike: where the two tiles that 84 tokens of the
 // DeepSeek-V3 layer have more than in one tile of 96 rows begin another round of items, 837 -> 856 us; 80 tokens 817 -> 813,
 // 96 911 -> 908, 126 990 -> 982.
+// 32 experts of 7168 x 2048, uneven, 150 / 190 / 220 / 472 rows: 257 / 270 / 259 / 353 us by the rounds, 241 / 262 / 267 / 312 so.
 int moe_gemm_tile_rows(const TileShape& t) {
   const int groups = t.E < t.R ? t.E : t.R;
   if (groups <= 0) return kTileRows;
