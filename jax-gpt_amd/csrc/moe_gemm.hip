@@ -51,7 +51,7 @@
 //
 // Launches of many work items of short row tiles are taken by another kernel, with
 // the same items, operands and results: moe_gemm_stream.hip (moe_gemm_tile_rows and
-// moe_gemm_stream_stages say which).
+// moe_gemm_streams say which).
 #include <stdlib.h>
 
 #include <mutex>
@@ -741,9 +741,9 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
   const int tallest = l.hdr ? l.tile_rows : dense_tile_rows;   // (a dense group beside routed ones is cut as their list is)
   long long items = dn ? (long long)dense_tiles * col_blocks(MODE, dense.N) : 0;
   if (l.hdr) items += (long long)(rt->E < rt->R ? rt->E : rt->R) * col_blocks(MODE, routed.N);
-  if (const int stages = moe_gemm_stream_stages(MODE, tallest, items))
-    return moe_gemm_stream_launch(MODE, StreamLaunch{routed, l.hdr, l.tiles, dense, dense_rows, dense_tiles, (int)dense_blocks, stream,
-                                                     (unsigned)grid, tallest, stages}, s);
+  if (moe_gemm_streams(MODE, tallest, items))
+    return moe_gemm_stream_launch(MODE, StreamLaunch{routed, l.hdr, l.tiles, l.rows, dense, dense_rows, dense_tiles, (int)dense_blocks,
+                                                     stream, (unsigned)grid, tallest}, s);
   static std::atomic<unsigned long long> lds_raised[4] = {};
   auto* kernel = dn ? (stream ? grouped_gemm_kernel<MODE, true, true> : grouped_gemm_kernel<MODE, true, false>)
                     : (stream ? grouped_gemm_kernel<MODE, false, true> : grouped_gemm_kernel<MODE, false, false>);

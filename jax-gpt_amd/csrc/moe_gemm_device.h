@@ -4,20 +4,21 @@
 
 #include "moe_common.h"
 
-// moe_gemm_stream.hip: the launch, and the weight stages that it is to have (0: it is none for that kernel)
+// moe_gemm_stream.hip: the launch, and whether it is one for that kernel
 struct StreamLaunch {
   GemmOperands routed;
   TileHeader* hdr;
   const TileEntry* tiles;
+  int rows;   // of all routed groups
   GemmOperands dense;
   int dense_rows, dense_tiles, dense_blocks;
   bool from_memory;
   unsigned grid;
-  int tile_rows, stages;
+  int tile_rows;
 };
 constexpr int kStreamItems = 384;   // fewest work items, and
 constexpr int kStreamRows = 128;    // tallest tiles of such a launch
-int moe_gemm_stream_stages(int mode, int tile_rows, long long items);
+bool moe_gemm_streams(int mode, int tile_rows, long long items);
 int moe_gemm_stream_launch(int mode, const StreamLaunch& l, hipStream_t s);
 
 constexpr int BW = 256;       // weight rows per work item
@@ -26,6 +27,19 @@ constexpr int MODE_GATEUP = 0;
 constexpr int MODE_DOWN = 1;
 constexpr int MAX_KB = 256;   // K <= 32768
 constexpr int W_TILE_BYTES = BW * BK;   // 32 KB
+
+// Weight stages of that kernel's items of up to 32 rows.  The list's own sizes say which: the host knows only what they can be at most.
+//  - Gate/up: one where every item runs at once but some CUs have two of them, two where each CU has one or there are more
+//    rounds.  32 experts of 7168 x 2048, gate/up + down + combine, one stage / two: 16 of them with rows (256 items) 130 / 115
+//    us, 12 120 / 97, 17 142 / 153, 24 163 / 169; Qwen3-MoE, 9 tokens, 53 experts (318 items) 57.5 / 59.1, 33 49.0 / 45.5, 20
+//    42.4 / 37.2; full layer, 7 tokens (some 560) 184 / 169.
+//  - Down, in lists that may have taller tiles: two while a tile has ten rows or fewer on average, so that most of the
+//    stream is theirs.  The same 32 experts, one stage / two: 160 rows in 24 tiles 187 / 178, 264 in 27 198 / 194, 320 in 28 211 /
+//    215, 512 in 30 220 / 225; Qwen3-MoE, 80 tokens in 81 tiles 81.8 / 78.5, in 44 63.9 / 65.7; 200 tokens in 128 113.6 / 114.5.
+__host__ __device__ inline int moe_stream_depth(int mode, bool short_only, int tiles, int items, int rows) {
+  if (mode == MODE_GATEUP) return items > 256 && items <= 512 ? 1 : 2;
+  return short_only || rows <= 10 * tiles ? 2 : 1;
+}
 
 // epilogue staging tile: 128-byte rows, chunk c of row r at position c ^ (r & 7)
 __device__ __forceinline__ int swz(int row, int chunk) { return row * BK + ((chunk ^ (row & 7)) << 4); }

@@ -2,8 +2,9 @@
 //
 // The class kernel (moe_gemm.hip) keeps one workgroup on a CU, with all of its LDS as one deep ring.  An item of few K steps
 // then spends as long on its start (list entry, row ids, first copies) and its end as on its stream, and nobody on the CU
-// streams meanwhile.  Here two workgroups share a CU, each with rings of one or two stages, so that one streams while the other
-// starts or ends; there is more than one SIMD's worth of waves to hide a step's latencies, and the loop is rolled.
+// streams meanwhile.  Here two workgroups share a CU, each with rings of one or (items of up to 32 rows, moe_stream_depth) two
+// stages, so that one streams while the other starts or ends; there is more than one SIMD's worth of waves to hide a step's
+// latencies, and the loop is rolled.
 // Wave w copies the weight rows that it alone multiplies and takes its fragments to registers as a step begins: the rows'
 // place is free at once and is refilled in mid-step, with no barrier, so one stage is nearly always in flight.  The activation
 // tile is shared by all waves: one barrier a step, and one stage more than the weights' ring.
@@ -23,19 +24,23 @@ constexpr int RG = 32 / WAVES;       // weight row groups of 8 rows that a wave 
 __host__ __device__ constexpr int x_stage_bytes(int bm) { return bm * BK + bm * 4 + 256; }
 __host__ __device__ constexpr int wscale_off(int nst, int bm) { return nst * W_TILE_BYTES + (nst + 1) * x_stage_bytes(bm); }
 // the epilogues stage where the rings were
-static_assert(128 * 256 * 2 <= wscale_off(1, 128) && 32 * (8 * 4 + BK) <= wscale_off(1, 32), "the epilogue stages inside the rings' space");
+static_assert(kStreamRows * 256 * 2 <= wscale_off(1, kStreamRows) && 32 * (8 * 4 + BK) <= wscale_off(1, 32), "the epilogue stages inside the rings' space");
+// every item's rings and weight scales fit where two stages of 32-row tiles do
+static_assert(wscale_off(1, kStreamRows) <= wscale_off(2, 32), "rings of the tallest tile");
+static_assert(wscale_off(2, 32) + 2 * MAX_KB * 4 <= 80 * 1024, "two workgroups on a CU");
 
-// One item of up to 32 XF rows; MAXXF: the launch's tallest, which the rings are laid out for.  nst: weight stages (1 or 2).
-template <int MODE, int XF, int MAXXF, bool ONCE>
-__device__ __forceinline__ void stream_item(const Item& item, uint8_t* lds, const GemmOperands& op, int nst) {
+// One item of up to 32 XF rows.  depth: weight stages of an item of up to 32 rows (1 or 2); a taller one has one.
+template <int MODE, int XF, bool ONCE>
+__device__ __forceinline__ void stream_item(const Item& item, uint8_t* lds, const GemmOperands& op, int depth) {
   constexpr int BM = 32 * XF, NF = 2 * XF;
-  constexpr int X_STAGE = x_stage_bytes(32 * MAXXF), S_OFF = BM * BK;
+  constexpr int X_STAGE = x_stage_bytes(BM), S_OFF = BM * BK;
+  const int nst = XF == 1 ? depth : 1;
   // copies per wave and step: its weight rows, activation row groups w, w + WAVES, ... (4 XF in all), and one wave for every
   // 64 rows the scales
   constexpr int X_OPS = (4 * XF + WAVES - 1) / WAVES;
   constexpr bool SHORT = 4 * XF < WAVES;          // waves 4 XF .. copy no activations, and the first of them the scales
   constexpr int S_WAVES = (BM + 63) / 64;
-  constexpr int OPS = RG + (SHORT ? 0 : X_OPS);   // ... of a wave that has no more than the others (two stages: XF 1 and 2)
+  constexpr int OPS = RG + (SHORT ? 0 : X_OPS);   // ... of a wave that has no more than the others
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fq = lane >> 4;
@@ -95,7 +100,7 @@ __device__ __forceinline__ void stream_item(const Item& item, uint8_t* lds, cons
     copy_x(t, t);
     copy_w(t, t);
   }
-  float* wscale = (float*)(lds + wscale_off(nst, 32 * MAXXF));
+  float* wscale = (float*)(lds + wscale_off(nst, BM));
   for (int i = tid; i < 2 * KB; i += NT) {
     const int h = i >= KB, kk = h ? i - KB : i;
     float v;
@@ -124,7 +129,7 @@ __device__ __forceinline__ void stream_item(const Item& item, uint8_t* lds, cons
     constexpr bool MORE = decltype(more)::value;
     // this wave's copies of stage kb have landed, and its reads of the stage before are done; then everyone's
     // (copies complete in issue order; behind them, with two stages, those of the next step)
-    if (XF > 2 || nst == 1 || kb == KB - 1) wait_vm<0>();
+    if (XF > 1 || nst == 1 || kb == KB - 1) wait_vm<0>();
     else if (more_ops) wait_vm<OPS + 1>();
     else wait_vm<OPS>();
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -175,17 +180,22 @@ __device__ __forceinline__ void stream_item(const Item& item, uint8_t* lds, cons
 }
 
 // STREAM: weights come from memory, and those of experts of one row tile are marked as read once (grouped_gemm_kernel).
+// rows: of all routed groups.
 template <int MODE, bool DENSE, bool STREAM, int MAXXF>
 __global__ __launch_bounds__(NT, 4) void stream_gemm_kernel(const GemmOperands routed, TileHeader* hdr, const TileEntry* __restrict__ tiles,
-                                                           const GemmOperands dense, int dense_rows, int dense_tiles,
-                                                           int dense_blocks, int nst) {
+                                                           int rows, const GemmOperands dense, int dense_rows, int dense_tiles,
+                                                           int dense_blocks) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const bool is_dense = DENSE && (int)blockIdx.x < dense_blocks;
   const GemmOperands op = is_dense ? dense : routed;
   Item item;
   if (!work_item<MODE, DENSE>(item, lds, op.N, is_dense, hdr, tiles, dense_rows, dense_tiles, dense_blocks)) return;
+  auto ncb = [](int N) { return MODE == MODE_GATEUP ? N / 128 : (N + 255) / 256; };
+  const int listed = !DENSE || hdr ? hdr->n_tiles : 0;
+  const int depth = __builtin_amdgcn_readfirstlane(moe_stream_depth(
+      MODE, MAXXF == 1, listed + (DENSE ? dense_tiles : 0), listed * ncb(routed.N) + (DENSE ? dense_tiles * ncb(dense.N) : 0), rows + (DENSE ? dense_rows : 0)));
   const bool once = STREAM && __builtin_amdgcn_readfirstlane(item.tiles) == 1;
-#define MOE_CLASS(XF) if (once) stream_item<MODE, XF, MAXXF, true>(item, lds, op, nst); else stream_item<MODE, XF, MAXXF, false>(item, lds, op, nst)
+#define MOE_CLASS(XF) if (once) stream_item<MODE, XF, true>(item, lds, op, depth); else stream_item<MODE, XF, false>(item, lds, op, depth)
   if constexpr (MAXXF == 1) {
     MOE_CLASS(1);
   } else {
@@ -205,14 +215,13 @@ int launch(const StreamLaunch& l, hipStream_t s) {
   auto* kernel = l.dense_blocks ? (l.from_memory ? stream_gemm_kernel<MODE, true, true, MAXXF> : stream_gemm_kernel<MODE, true, false, MAXXF>)
                                 : (l.from_memory ? stream_gemm_kernel<MODE, false, true, MAXXF> : stream_gemm_kernel<MODE, false, false, MAXXF>);
   const int kb = (l.routed.K > l.dense.K ? l.routed.K : l.dense.K) / BK;
-  // (no less than 56 KB: a third workgroup on the CU makes launches of many items 1 to 4 % slower)
-  const int need = wscale_off(l.stages, 32 * MAXXF) + 2 * kb * (int)sizeof(float), bytes = need > 56 * 1024 ? need : 56 * 1024;
+  // (the same for one stage: a third workgroup on the CU makes launches of many items 1 to 4 % slower)
+  const int bytes = wscale_off(2, 32) + 2 * kb * (int)sizeof(float);
   if (int rc = moe_raise_lds_limit((const void*)kernel, 80 * 1024, lds_raised[(l.dense_blocks ? 2 : 0) + l.from_memory])) return rc;
-  hipLaunchKernelGGL(kernel, dim3(l.grid), dim3(NT), bytes, s, l.routed, l.hdr, l.tiles, l.dense, l.dense_rows, l.dense_tiles,
-                     l.dense_blocks, l.stages);
+  hipLaunchKernelGGL(kernel, dim3(l.grid), dim3(NT), bytes, s, l.routed, l.hdr, l.tiles, l.rows, l.dense, l.dense_rows,
+                     l.dense_tiles, l.dense_blocks);
   return moe_check_hip(hipGetLastError(), "gemm launch");
 }
-static_assert(wscale_off(2, 32) + 2 * MAX_KB * 4 <= 80 * 1024 && wscale_off(1, 128) + 2 * MAX_KB * 4 <= 80 * 1024, "two workgroups on a CU");
 
 }  // namespace
 
@@ -222,12 +231,8 @@ static_assert(wscale_off(2, 32) + 2 * MAX_KB * 4 <= 80 * 1024 && wscale_off(1, 1
 //    gate/up 48 us; 50 here with two stages, 75 with one).
 //  - Gate/up of tiles above 32 rows: its items are longer, and rounds over 2 x 256 workgroups do not come out even (128 experts
 //    of 2048 x 768, 60 rows 75.7 us, 79.4 here).  The down GEMM's items are half as long or less: 49.9 -> 45.5.
-//  - One stage does where all items run at once (Qwen3-MoE, 8 tokens 61.8 us; with one stage 55.8, two 58); with more rounds
-//    the last one, with one workgroup on a CU, needs two (64 tokens of the DeepSeek-V3 layer 733 / 753 / 731).
-int moe_gemm_stream_stages(int mode, int tile_rows, long long items) {
-  if (items < kStreamItems || tile_rows > (mode == MODE_GATEUP ? 32 : kStreamRows)) return 0;
-  if (mode == MODE_GATEUP) return items <= 560 ? 1 : 2;
-  return tile_rows <= 32 ? 2 : 1;
+bool moe_gemm_streams(int mode, int tile_rows, long long items) {
+  return items >= kStreamItems && tile_rows <= (mode == MODE_GATEUP ? 32 : kStreamRows);
 }
 int moe_gemm_stream_launch(int mode, const StreamLaunch& l, hipStream_t s) {
   if (mode == MODE_GATEUP) return launch<MODE_GATEUP, 1>(l, s);

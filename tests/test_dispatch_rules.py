@@ -1,0 +1,39 @@
+"""The rules that choose between kernels, asked on the host (no GPU call is made): the objects that the library was linked
+from, linked once more with a program that calls the rules themselves."""
+import glob
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PACKAGE = os.path.join(ROOT, "jax-gpt_amd")
+GATEUP, DOWN = 0, 1
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    objects = sorted(glob.glob(os.path.join(PACKAGE, "build", "*.o")))
+    if not os.path.exists(hipcc) or not objects:
+        pytest.skip("needs hipcc and the library's objects")
+    exe = str(tmp_path_factory.mktemp("rules") / "rules")
+    flags = ["--offload-arch=gfx950", "-O1", "-std=c++17", "-w", "-I", os.path.join(ROOT, "include"), "-I", os.path.join(PACKAGE, "csrc")]
+    subprocess.run([hipcc, *flags, "-c", os.path.join(ROOT, "tests", "dispatch_rules.hip"), "-o", exe + ".o"], check=True)
+    subprocess.run([hipcc, "--offload-arch=gfx950", exe + ".o", *objects, "-o", exe], check=True)
+
+    def run(*commands):
+        text = "\n".join(" ".join(str(int(v) if isinstance(v, bool) else v) for v in c) for c in commands)
+        return subprocess.run([exe], input=text, capture_output=True, text=True, check=True).stdout.splitlines()
+    return run
+
+
+def test_ring_depth_follows_the_items_that_there_are(ask):
+    """Short row tiles: one weight stage where all items run at once and some CUs have two, two stages otherwise -- by the
+    list's items, not by what they could be at most (12 of 32 experts with rows: 192 items of at most 512)."""
+    items = [192, 256, 257, 512, 513, 2048]
+    assert ask(*[("depth", GATEUP, True, n // 16, n, n // 8) for n in items]) == ["2", "2", "1", "1", "2", "2"]
+    # down, lists with taller tiles: by the rows of a tile
+    assert ask(*[("depth", DOWN, False, 24, 672, r) for r in (24, 240, 241, 700)]) == ["2", "2", "1", "1"]
+    assert ask(("depth", DOWN, True, 24, 672, 700)) == ["2"]

@@ -331,16 +331,21 @@ def test_work_lists_of_few_and_more_rows_give_the_same_bits(jg, D, I, E, sizes):
 
 SHORT = [33, 0, 1, 0, 2, 0, 0, 17, 0, 1, 0, 0, 16, 0, 3, 0, 0, 0, 32, 0, 0, 1, 0, 0, 0, 0, 0]   # at most 4 rows an expert on average
 TALL = [250, 129, 128, 97, 96, 65, 64, 33, 1] + [0] * 47                                             # at most 16
+MIXED = [129, 128, 97, 65, 33, 0, 1, 2, 2, 1, 0, 1] + [2] * 48 + [0] * 46                             # 574 rows in 64 tiles: two stages of the short ones
 
 
 @pytest.mark.parametrize("E,D,I,sizes", [
-    (108, 1024, 512, SHORT),      # 432 gate/up and down items: one stage, two stages
-    (162, 640, 512, SHORT),       # 648: two stages; the last column block of the down GEMM is half full
+    (108, 1024, 512, SHORT),      # 160 items of each GEMM: two stages
+    (108, 1024, 1024, SHORT),     # 320 gate/up items: one stage
+    (162, 256, 1536, SHORT),      # 720: more than all that run at once, two stages
+    (162, 640, 512, SHORT),       # the last column block of the down GEMM is half full
     (108, 128, 512, SHORT),       # gate/up of one K step
-    (405, 256, 128, SHORT),       # 405 items each, of two K steps and of one
+    (405, 256, 128, SHORT),       # 150 items each, of two K steps and of one
+    (405, 256, 256, SHORT),       # 300 gate/up items of two K steps, one stage
     (54, 2176, 1280, SHORT),      # weights from memory: copies of experts of one tile are non-temporal
     (56, 2048, 384, TALL),        # down tiles of up to 128 rows, plain copies ...
     (56, 2048, 1024, TALL),       # ... and non-temporal ones
+    (106, 2048, 384, MIXED), (106, 2048, 1024, MIXED), (106, 1024, 128, MIXED),   # (the last: one K step)
 ])
 def test_streamed_short_tiles_give_the_same_bits(jg, E, D, I, sizes):
     """Many short work items, which a kernel of their own takes: each expert's rows against a call of that expert alone
