@@ -688,7 +688,9 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
     return (size_t)rows * N * (MODE == MODE_DOWN ? 2 : 1) > ((size_t)4 << 20) && rows <= 96ll * E;
   };
   auto own_tile_rows = [](int rows, int E, const GemmOperands& op) {
-    return moe_gemm_tile_rows(TileShape{rows, E, rows, {col_blocks(MODE, op.N), 0}, {op.K / BK, 0}, 0, {0, 0}});
+    TileShape t{rows, E, rows, {0, 0}, {0, 0}, 0, {0, 0}};
+    t.ncb[MODE] = col_blocks(MODE, op.N), t.kb[MODE] = op.K / BK;
+    return moe_gemm_tile_rows(t);
   };
   GemmOperands routed{}, dense{};
   TileList l{};
@@ -762,23 +764,26 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
 // that just fills a round does not spill into another one.  One group's size is known, and so are its rounds however many
 // items they hold: 8192 rows of 2048 x 8192 are 8 rounds of 256-row tiles or of 288-row ones, 287 -> 274 us (gate/up),
 // 138.6 -> 127.1 the down GEMM of 7168 x 2048.
-//   Before that: short tiles, which moe_gemm_stream.hip takes, where no expert can have more rows -- or hardly one will, with
-// eight times the mean to spare.  An expert that has more after all is cut, and its weights are read once for each tile, from
-// L2 at best (4000 tokens of the full layer, 78 rows an expert, tiles of 128 rows: 1329 us where the routing is even, 1340 ->
-// 1380 where 81 experts have 128 to 493).  A shared expert beside them is cut alike: where the two tiles that 84 tokens of the
-// DeepSeek-V3 layer have more than in one tile of 96 rows begin another round of items, 837 -> 856 us; 80 tokens 817 -> 813,
-// 96 911 -> 908, 126 990 -> 982.
-// 32 experts of 7168 x 2048, uneven, 150 / 190 / 220 / 472 rows: 257 / 270 / 259 / 353 us by the rounds, 241 / 262 / 267 / 312 so.
+//   Before that: short tiles, which moe_gemm_stream.hip takes -- 32 rows, or 128 where a down GEMM reads the list (no gate/up
+// launch of these goes there, and on the class kernel it is better off with tall tiles and their larger pool: 264 to 512 rows
+// for 32 experts of 7168 x 2048, uneven, -6.5 to +2 %, -1.5 on average) -- where no expert can have more rows, or hardly one
+// will, with eight times the mean to spare.  An expert that has more after all is cut, and its weights are read once for each
+// tile, from L2 at best.  That is why the lines lie at 4 and 16 rows an expert (4000 tokens of the full layer, 78 rows an
+// expert, cut to 128 rows: 1329 us where the routing is even, 1380 for 1340 where 81 experts have 128 to 493).  Below them, against
+// the heights by the rounds, routing even or uneven by normal offsets of 1 and 2 on the logits: Qwen3-MoE, 20 tokens 86 / 93, 59 /
+// 63, 41 / 42.5 us; 100 tokens 110.7 / 114.5, 84.9 / 84.5, 67.2 / 69.7; 64 tokens 103 / 111, 73.5 / 79.5, but 57.7 / 54.3, where five
+// experts of 33 to 52 rows begin another round; 128 tokens of DeepSeek-V3 984 / 994, 644 / 643, 353 / 349; full layer, 100 tokens
+// 844 / 855, 400 1037 / 1062, 256 1028 / 1019.  A shared expert beside them is cut alike: where the two tiles that 84 tokens of the
+// DeepSeek-V3 layer have more than in one of 96 rows begin another round of items (125 experts touched, which the host does
+// not know) 852 / 835; 33 to 128 tokens otherwise -1.0 to +1.5 %, -0.2 on average.
 int moe_gemm_tile_rows(const TileShape& t) {
   const int groups = t.E < t.R ? t.E : t.R;
   if (groups <= 0) return kTileRows;
-  if ((long long)groups * (t.ncb[0] > t.ncb[1] ? t.ncb[0] : t.ncb[1]) >= kStreamItems) {
-    if (t.max_rows <= 32 || t.R <= 4 * t.E) return 32;
-    if (t.max_rows <= kStreamRows || t.R <= kStreamRows / 8 * t.E) return kStreamRows;
-  }
+  if ((t.max_rows <= 32 || t.R <= 4 * t.E) && (long long)groups * (t.ncb[0] > t.ncb[1] ? t.ncb[0] : t.ncb[1]) >= kStreamItems) return 32;
+  if ((t.max_rows <= kStreamRows || t.R <= kStreamRows / 8 * t.E) && (long long)groups * t.ncb[1] >= kStreamItems) return kStreamRows;
   const int mean = (t.R + groups - 1) / groups;
   if (mean > kFullTileItems * kTileRows / groups) return kTileRows;
-  const int least = t.ncb[1] && t.ncb[1] < t.ncb[0] ? t.ncb[1] : t.ncb[0];
+  const int least = !t.ncb[0] || (t.ncb[1] && t.ncb[1] < t.ncb[0]) ? t.ncb[1] : t.ncb[0];
   if (t.E > 1 && groups * ((mean + kTileRows - 1) / kTileRows) * least >= kFullTileItems) return kTileRows;
   int spread = 0;
   while (t.E > 1 && spread * spread < 4 * mean) ++spread;

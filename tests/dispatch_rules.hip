@@ -12,6 +12,10 @@ int main() {
       int mode, short_only, tiles, items, rows;
       std::cin >> mode >> short_only >> tiles >> items >> rows;
       std::cout << moe_stream_depth(mode, short_only, tiles, items, rows) << "\n";
+    } else if (what == "tile_rows") {   // rows, groups, most rows of a group; column blocks, K steps of gate/up and down; dense rows and column blocks
+      TileShape t;
+      std::cin >> t.R >> t.E >> t.max_rows >> t.ncb[0] >> t.ncb[1] >> t.kb[0] >> t.kb[1] >> t.dense_rows >> t.dense_ncb[0] >> t.dense_ncb[1];
+      std::cout << moe_gemm_tile_rows(t) << "\n";
     } else {
       return 1;
     }

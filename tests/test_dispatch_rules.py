@@ -37,3 +37,18 @@ def test_ring_depth_follows_the_items_that_there_are(ask):
     # down, lists with taller tiles: by the rows of a tile
     assert ask(*[("depth", DOWN, False, 24, 672, r) for r in (24, 240, 241, 700)]) == ["2", "2", "1", "1"]
     assert ask(("depth", DOWN, True, 24, 672, 700)) == ["2"]
+
+
+def test_lists_are_cut_for_the_kernels_that_read_them(ask):
+    """128-row tiles are for the down GEMM's short-tile kernel: a list that a gate/up launch alone reads has none."""
+    def rows(R, ncb, kb, E=32, most=None, dense=(0, 0, 0)):
+        return ("tile_rows", R, E, R if most is None else most, *ncb, *kb, *dense)
+    gateup, down, both = ((16, 0), (56, 0)), ((0, 28), (0, 16)), ((16, 28), (56, 16))
+    for R, want in ((64, ("32", "32", "32")), (128, ("32", "32", "32")), (129, ("288", "128", "128")), (512, ("288", "128", "128")),
+                    (513, ("288", "288", "288")), (16384, ("288", "288", "288"))):
+        assert tuple(ask(rows(R, *gateup), rows(R, *down), rows(R, *both))) == want, R
+    # too few items of the down GEMM for that kernel, whatever the gate/up GEMM has
+    assert ask(rows(512, (16, 2), (4, 16), E=64)) != ["128"]
+    # most rows of a group, and a shared expert beside
+    assert ask(rows(256, (6, 8), (16, 6), E=128, most=32), rows(1024, (6, 8), (16, 6), E=128, most=128),
+               rows(672, *both, E=256, most=84, dense=(84, 16, 28))) == ["32", "128", "32"]
