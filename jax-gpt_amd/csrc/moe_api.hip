@@ -298,7 +298,7 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
   // A few tokens whose sort and rows nobody asks for: the experts straight from the selection.  (What the launches that this
   // leaves out would have refused is refused here.)
   const bool sorted_outputs = a->out_group_sizes || a->out_sorted_token_ids || a->out_inv_perm || a->out_hq || a->out_hsq || a->out_y || a->out_ys;
-  if (!fork && !sorted_outputs && moe_token_takes(a->M, a->D, a->k, a->I, a->SI)) {
+  if (!fork && !sorted_outputs && moe_token_takes(a->M, a->D, a->E, a->k, a->I, a->SI)) {
     const GemmScales sc = moe_row_major_scales(a->D, a->I);
     if ((rc = moe_gemm_check(GemmOperands{b.xq, b.sx, nullptr, a->w_gate, a->sw_gate, a->w_up, a->sw_up, a->D, a->I, hq, sh, sc}, R, a->E, false))) return rc;
     if ((rc = moe_gemm_check(GemmOperands{hq, sh, nullptr, a->w_down, a->sw_down, nullptr, nullptr, a->I, a->D, y, nullptr, sc}, R, a->E, true))) return rc;

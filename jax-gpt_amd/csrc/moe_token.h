@@ -24,5 +24,5 @@ struct TokenArgs {
   void* out;
 };
 // whether a call of M tokens takes this route
-bool moe_token_takes(int M, int D, int k, int I, int SI);
+bool moe_token_takes(int M, int D, int E, int k, int I, int SI);
 int moe_token_experts(const TokenArgs& a, bool from_memory, moe_stream_t stream);

@@ -241,13 +241,18 @@ int launch_gateup(const TokenArgs& a, bool from_memory, hipStream_t s) {
 // tile, and no CU has a second workgroup of about 80 KB of LDS to begin (full layer, 2 tokens, workgroups of 2 tiles against
 // 512 of one: 70.1 / 74.3 us; mini, 8: 31.3 / 32.9; one workgroup more than there are CUs -- 6 tokens of Qwen3-MoE in 258 --
 // 46.3 against 43.4 in 192).
+int down_tiles(int D, int M) {
+  const int cols = D / COLS;
+  int tiles = 1;
+  while (tiles < DOWN_TILES && (cols + tiles - 1) / tiles * M > 256) ++tiles;
+  return tiles;
+}
 int launch_down(const TokenArgs& a, bool from_memory, hipStream_t s) {
   static std::atomic<unsigned long long> raised[2] = {};
   auto* kernel = from_memory ? token_down_kernel<true> : token_down_kernel<false>;
   if (int rc = moe_raise_lds_limit((const void*)kernel, kDownLds, raised[from_memory])) return rc;
   const int slots = a.k + (a.SI > 0), cols = a.D / COLS;
-  int tiles = 1;
-  while (tiles < DOWN_TILES && (cols + tiles - 1) / tiles * a.M > 256) ++tiles;
+  int tiles = down_tiles(a.D, a.M);
   if (slots > 16 || slots * down_wave_lds(a.h_stride, tiles) > kDownLds) tiles = 1;   // (a wave of several slots)
   const int per_wave = down_wave_lds(a.h_stride, tiles), fit = kDownLds / per_wave, most = fit < 16 ? fit : 16;
   const int waves = slots < most ? slots : most;
@@ -257,16 +262,29 @@ int launch_down(const TokenArgs& a, bool from_memory, hipStream_t s) {
 
 }  // namespace
 
-// Every token reads its experts itself, where the grouped kernels read an expert once for all its rows, and 16-row streams
-// run at about 6 TB/s against their 6.9: what the launches left out and the finer split gain (7 to 13 us) covers that up to
-// some 300 MB of weights (Qwen3-MoE, 8 tokens = 302 MB 55.4 -> 50.6 us, 10 = 377 MB 60.6 -> 67.3; full
-// layer, 2 tokens = 277 MB 74.2 -> 69.4, 3 = 415 MB 87.2 -> 94.5; DeepSeek-V3, 2 tokens = 793 MB 113.6 -> 130).  One token
-// reads nothing twice and gains at any size (396 MB of DeepSeek-V3: 84 -> 76).  Of layers this small that keeps up to 16
-// tokens: at 24 the mini layer and tiny are even (34.6 / 34.9, 22.1 / 22.2), at 48 36 -> 47 and 23.4 -> 31.7.
-bool moe_token_takes(int M, int D, int k, int I, int SI) {
+// Every token reads its experts itself, where the grouped kernels read an expert once for all its rows, and a wave of the second
+// launch walks its tiles' K steps one after the other.  What the launches left out and the finer split gain (3 to 13 us) covers
+//  - up to some 320 MB of weights, which 16-row streams read at about 6 TB/s against 6.9 (Qwen3-MoE, 8 tokens = 302 MB 55.4 ->
+//    50.6 us, 10 = 377 MB 60.6 -> 67.3; full layer, 2 tokens = 277 MB 74.2 -> 69.4, 3 = 415 MB 87.2 -> 94.5; DeepSeek-V3, 2
+//    tokens = 793 MB 113.6 -> 130);
+//  - of these, megabytes that are read again, and eight times the K steps that the second launch's longest chain has beyond one
+//    tile's, up to 300 (grouped / this way, us, of layers that the memory-side cache holds).  A shared expert eight times as
+//    wide, D 1024, 2 of 32 experts of 512: 4 tokens (no further steps) 31.6 / 25.9, 8 (32) 33.4 / 33.6, 12 (64) 34.8 / 47.0, 16 (96)
+//    35.1 / 49.6.  D 4096, 2 of 4 experts of 1024: 4 tokens (24) 31.5 / 27.3, 8 (56, 144 MB again) 32.3 / 34.6, 12 32.6 / 44.5.
+//    8 of 8 experts, D 1024 x 1024: 8 tokens (8, 168 MB) 24.5 / 22.1, 12 (24, 264 MB) 25.7 / 29.0; 8 of 8, 16 and 32 experts of
+//    2048 x 768, 8 tokens (18 and 252, 216 and 144 MB) 28.0 / 27.7, 29.5 / 29.0, 38.3 / 36.0.  In some 170 layers and batches of such
+//    kinds the choice by this line is 0.3 % slower than the better route on average, 13 % at worst (by the first line alone:
+//    2.3 and 41 %).
+// One token reads nothing twice and gains at any size (396 MB of DeepSeek-V3: 84 -> 76).  Of layers this small that keeps up to
+// 16 tokens: at 24 the mini layer and tiny are even (34.6 / 34.9, 22.1 / 22.2), at 48 36 -> 47 and 23.4 -> 31.7.
+bool moe_token_takes(int M, int D, int E, int k, int I, int SI) {
   const int widest = I > SI ? I : SI;
   if (M < 1 || M > MOE_TOKEN_ROWS || k < 1 || k >= MOE_TOKEN_SLOTS || up_lds(D) > kLds || down_wave_lds(widest, 1) > kDownLds) return false;
-  return M == 1 || 3ll * M * ((long long)k * I + SI) * D <= (320ll << 20);
+  if (M == 1) return true;
+  const long long touched = (long long)M * k < E ? (long long)M * k : E;
+  const long long bytes = 3ll * M * ((long long)k * I + SI) * D, once = 3ll * (touched * I + SI) * D;
+  const long long steps = (long long)(down_tiles(D, M) - 1) * (widest / BK);
+  return bytes <= (320ll << 20) && 8 * steps + ((bytes - once) >> 20) <= 300;
 }
 
 int moe_token_experts(const TokenArgs& a, bool from_memory, moe_stream_t stream) {

@@ -16,6 +16,10 @@ int main() {
       TileShape t;
       std::cin >> t.R >> t.E >> t.max_rows >> t.ncb[0] >> t.ncb[1] >> t.kb[0] >> t.kb[1] >> t.dense_rows >> t.dense_ncb[0] >> t.dense_ncb[1];
       std::cout << moe_gemm_tile_rows(t) << "\n";
+    } else if (what == "token") {   // tokens, D, experts, k, I, SI
+      int M, D, E, k, I, SI;
+      std::cin >> M >> D >> E >> k >> I >> SI;
+      std::cout << moe_token_takes(M, D, E, k, I, SI) << "\n";
     } else {
       return 1;
     }

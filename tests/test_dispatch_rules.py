@@ -52,3 +52,18 @@ def test_lists_are_cut_for_the_kernels_that_read_them(ask):
     # most rows of a group, and a shared expert beside
     assert ask(rows(256, (6, 8), (16, 6), E=128, most=32), rows(1024, (6, 8), (16, 6), E=128, most=128),
                rows(672, *both, E=256, most=84, dense=(84, 16, 28))) == ["32", "128", "32"]
+
+
+def test_few_tokens_go_straight_to_their_experts_where_that_is_cheaper(ask):
+    """By the weights read, those read again, and the second launch's chain: not a wide shared expert beside small routed
+    ones, nor sixteen tokens that all read the same few experts."""
+    taken = [(1, 7168, 256, 8, 2048, 2048), (8, 2048, 128, 8, 768, 0), (2, 4096, 512, 10, 1024, 1024), (16, 1024, 32, 2, 512, 512), (16, 512, 8, 2, 1024, 0),
+             (4, 1024, 32, 2, 512, 4096), (4, 4096, 4, 2, 1024, 0), (8, 2048, 32, 8, 768, 0), (8, 1024, 8, 8, 1024, 0), (16, 512, 16, 16, 512, 0)]
+    left = [(2, 7168, 256, 8, 2048, 2048), (9, 2048, 128, 8, 768, 0), (3, 4096, 512, 10, 1024, 1024), (17, 1024, 32, 2, 512, 512),
+            (12, 1024, 32, 2, 512, 4096), (16, 1024, 32, 2, 256, 4096), (8, 4096, 4, 2, 1024, 0), (8, 4096, 2, 2, 1024, 1024), (12, 1024, 8, 8, 1024, 0), (12, 768, 8, 8, 1536, 0)]
+    assert ask(*[("token", *c) for c in taken]) == ["1"] * len(taken)
+    assert ask(*[("token", *c) for c in left]) == ["0"] * len(left)
+    # the batches that test_gpu_variants.py compares with the grouped route do take the other one
+    from tests.test_gpu_variants import test_experts_of_single_tokens_give_the_grouped_bits as single
+    marks = [m.args[1] for m in single.pytestmark if m.name == "parametrize" and "M,D" in m.args[0]]
+    assert marks and ask(*[("token", *c) for c in marks[0]]) == ["1"] * len(marks[0])
