@@ -13,9 +13,10 @@
 // columns of a token, one wave a slot, and adds the slots up itself: no y, no third launch.  Against the grouped route (us,
 // one token): DeepSeek-V3 layer 84 -> 76, Qwen3-MoE 28 -> 20, full layer behind its norm 57.5 -> 45, mini 31 -> 27, tiny
 // 23 -> 20; five tokens of Qwen3-MoE 46 -> 38.5, eight 55 -> 50.5; sixteen of the mini layer 34 -> 30.5, of tiny 23 -> 20.
-//   Rings of two K steps: more bytes in flight per wave lose (one token of DeepSeek-V3: rings of 2 / 3 / 4 / 6 steps 75.6 /
-// 76.8 / 78.1 / 88.2 in the first launch, 2 / 3 / 4 / 8 in the second 76.2 / 75.3 / 81.9 / 93.9).  Workgroups of four waves in
-// the first: 85.8, as 288 of them are uneven on 256 CUs.
+//   Rings of two K steps: more bytes in flight per wave lose or change nothing (one token of DeepSeek-V3: rings of 2 / 3 / 4 / 6
+// steps 75.6 / 76.8 / 78.1 / 88.2 in the first launch; in the second 2 / 3 are even -- four draws 74.4 to 75.2 / 74.4 to 75.4, 1
+// to 8 tokens of Qwen3-MoE 22.0 to 49.0 / 21.6 to 48.9, 1 and 16 of the mini layer 26.5 and 30.2 / 27.3 and 30.5 -- and 4 / 8 are
+// 7 and 23 % slower).  Workgroups of four waves in the first: 85.8, as 288 of them are uneven on 256 CUs.
 #include "moe_token.h"
 
 namespace {
