@@ -390,7 +390,7 @@ struct DenseGemm {
 inline bool moe_gemm_from_memory(long long projection) { return 3 * projection > (192ll << 20); }
 // The checks of a GEMM launch's operands (gate/up or down), for a route that reads them without that launch.
 int moe_gemm_check(const GemmOperands& op, int rows, int E, bool down);
-// One launch for either or both (nullptr: none).
+// One launch for either or both (nullptr: none); both: the routed list has to be there.
 int moe_gemm_gateup_impl(const RoutedGemm* routed, const DenseGemm* dense, moe_stream_t stream);
 int moe_gemm_down_impl(const RoutedGemm* routed, const DenseGemm* dense, moe_stream_t stream);
 

@@ -697,11 +697,13 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
   int dense_rows = 0, dense_tiles = 0, dense_tile_rows = 0;
   long long dense_blocks = 0, grid = 0;
   if (dn) {
+    // (both groups in one launch are cut alike: it goes to one kernel by the height of one list's tiles)
+    MOE_REQUIRE(!rt || rt->list_tile_rows, MOE_ERR_BAD_SHAPE, "%s: a dense group beside routed rows needs their list to be there", what);
     if (int rc = check_operands(dn->op, dn->rows, 1, MODE, what)) return rc;
     dense = dn->op;
     dense.sc.out_through = through(dn->rows, 1, dense.N);
     dense_rows = dn->rows;
-    dense_tile_rows = rt && rt->list_tile_rows ? rt->list_tile_rows : own_tile_rows(dense_rows, 1, dense);
+    dense_tile_rows = rt ? rt->list_tile_rows : own_tile_rows(dense_rows, 1, dense);
     dense_tiles = moe_tile_count(dense_rows, dense_tile_rows);
     dense_blocks = 8 * (((long long)dense_tiles * col_blocks(MODE, dense.N) + 7) / 8);
     grid = dense_blocks;

@@ -20,6 +20,13 @@ int main() {
       int M, D, E, k, I, SI;
       std::cin >> M >> D >> E >> k >> I >> SI;
       std::cout << moe_token_takes(M, D, E, k, I, SI) << "\n";
+    } else if (what == "both") {   // routed rows without a list beside a dense group: refused before any GPU call
+      alignas(256) static unsigned char memory[1 << 16];
+      const float* f = (const float*)memory;
+      const GemmOperands op{memory, f, nullptr, memory, f, memory, f, 256, 256, memory, (float*)memory, moe_row_major_scales(256, 256)};
+      const RoutedGemm routed{op, (const int32_t*)memory, 8, 64, memory, sizeof memory, 0, 0};
+      const DenseGemm dense{op, 64};
+      std::cout << moe_gemm_gateup_impl(&routed, &dense, nullptr) << " " << moe_gemm_down_impl(&routed, &dense, nullptr) << " " << moe_last_error() << "\n";
     } else {
       return 1;
     }

@@ -67,3 +67,8 @@ def test_few_tokens_go_straight_to_their_experts_where_that_is_cheaper(ask):
     from tests.test_gpu_variants import test_experts_of_single_tokens_give_the_grouped_bits as single
     marks = [m.args[1] for m in single.pytestmark if m.name == "parametrize" and "M,D" in m.args[0]]
     assert marks and ask(*[("token", *c) for c in marks[0]]) == ["1"] * len(marks[0])
+
+
+def test_a_dense_group_beside_routed_rows_needs_their_list(ask):
+    """Cut on its own it could have taller tiles than the kernel that the routed list's height chooses."""
+    assert ask(("both",))[0].startswith("-1 -1 gemm_down: a dense group")
