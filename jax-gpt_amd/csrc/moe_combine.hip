@@ -35,7 +35,9 @@ __global__ __launch_bounds__(256) void combine_kernel(const bf16x8* __restrict__
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int s = 0; s < k; ++s) {
       bf16x8 v;   // (read once, written once: non-temporal accesses leave the caches to the GEMMs' operands, -0.3 to -1 % step time)
-      *(v4i*)&v = __builtin_nontemporal_load((const v4i*)&y[(size_t)pos[s] * D8 + c]);
+      // (an entry that the sort dropped has no row: zeros)
+      const v4i raw = __builtin_nontemporal_load((const v4i*)&y[(size_t)max(pos[s], 0) * D8 + c]);
+      *(v4i*)&v = pos[s] < 0 ? (v4i){0, 0, 0, 0} : raw;
       const float ws = wt[s];
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[i] = __fadd_rn(acc[i], __fmul_rn(bf16_to_f32(v.v[i]), ws));

@@ -58,6 +58,8 @@ __device__ __forceinline__ void place_pass(const int32_t* ids, int first, int n,
         if (o.sorted_token_ids) o.sorted_token_ids[pos] = (int)((unsigned)f / (unsigned)o.k);   // (half the code of a signed division)
         if (o.inv_perm) o.inv_perm[f] = pos;
       }
+    } else if (PLACE && i < n && o.inv_perm) {
+      o.inv_perm[first + i] = -1;   // (a dropped entry has no row)
     }
   }
 }
@@ -101,6 +103,8 @@ __device__ __forceinline__ void permute_few(const int32_t* ids, int n, int E, co
     if (o.sort_order) o.sort_order[pos] = e;
     if (o.sorted_token_ids) o.sorted_token_ids[pos] = (int)(((float)e + 0.5f) * __builtin_amdgcn_rcpf((float)o.k));   // e / k
     if (o.inv_perm) o.inv_perm[e] = pos;
+  } else if (e < n && o.inv_perm) {
+    o.inv_perm[e] = -1;   // (a dropped entry has no row)
   }
 }
 

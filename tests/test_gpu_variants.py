@@ -564,6 +564,36 @@ def test_experts_of_single_tokens_give_the_grouped_bits(jg, M, D, E, k, I, SI, f
         assert torch.equal(out.nan_to_num(7.0), want.nan_to_num(7.0)), f"replay {i}"
 
 
+@pytest.mark.parametrize("M,k", [(1, 2), (5, 3), (16, 8),     # straight to the experts: both of its kernels leave the rows out
+                                 (17, 1), (32, 1), (17, 3),   # the sort without counters, and with them
+                                 (700, 2), (1100, 2), (3000, 3)])   # scales read row-major, and gathered; several chunks
+def test_selected_experts_that_there_are_not_count_as_zero_rows(jg, M, k):
+    """A given selection may hold indices outside [0, E): their entries are dropped by the sort and add nothing."""
+    import torch
+    print("dropped entries", M, k, flush=True)
+    D, E, I = 512, 10, 256
+    params, rand = _layer(jg, D, E, I, 0, M + k)
+    ex = [params[n] for n in ("gate_proj", "up_proj", "down_proj")]
+    rng = H.rng_for(M * 10 + k)
+    idx = rng.integers(0, E, (M, k))
+    drop = rng.random((M, k)) < 0.3
+    drop[0] = True                                            # a token with no expert at all
+    bad = np.where(drop, rng.choice([-1, E, 2 ** 31 - 1, -2 ** 31], (M, k)), idx).astype(np.int32)
+    w = np.abs(rng.standard_normal((M, k))).astype(np.float32)
+    x = rand(M, D)
+    got = jg.expert_forward_single(x, H.to_cuda(bad), H.to_cuda(w), *ex)
+    want = jg.expert_forward_single(x, H.to_cuda(idx.astype(np.int32)), H.to_cuda(np.where(drop, np.float32(0), w)), *ex)
+    assert torch.equal(got, want) and not got[0].any()
+    p = jg.permute(H.to_cuda(bad), E)
+    n, flat = int((~drop).sum()), np.flatnonzero(~drop.reshape(-1))
+    order = flat[np.argsort(bad.reshape(-1)[flat], kind="stable")]
+    inv = np.full(M * k, -1)
+    inv[order] = np.arange(n)
+    assert np.array_equal(p["sort_order"].cpu().numpy()[:n], order) and np.array_equal(p["sorted_token_ids"].cpu().numpy()[:n], order // k)
+    assert np.array_equal(p["inv_perm"].cpu().numpy(), inv) and int(p["group_offsets"][-1]) == n
+    assert np.array_equal(p["group_sizes"].cpu().numpy(), np.bincount(bad.reshape(-1)[flat], minlength=E))
+
+
 @pytest.mark.parametrize("E", [256, 257, 512, 640])
 @pytest.mark.parametrize("M,D", [(1, 4096), (3, 2304), (256, 1152), (257, 2176)])
 def test_partial_sums_of_wide_routers(jg, M, D, E):
