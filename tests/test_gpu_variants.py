@@ -349,7 +349,7 @@ MIXED = [129, 128, 97, 65, 33, 0, 1, 2, 2, 1, 0, 1] + [2] * 48 + [0] * 46       
 ])
 def test_streamed_short_tiles_give_the_same_bits(jg, E, D, I, sizes):
     """Many short work items, which a kernel of their own takes: each expert's rows against a call of that expert alone
-    (too few items for it), and one expert's down rows against the oracle."""
+    (too few items for it), and one expert of every height against the oracle."""
     import torch
     print("streamed tiles", E, D, I, flush=True)
     sizes = [sizes[i % len(sizes)] for i in range(E)]
@@ -364,6 +364,7 @@ def test_streamed_short_tiles_give_the_same_bits(jg, E, D, I, sizes):
     hb, sb = jg.gemm_gateup_swiglu(xq, gathered, params["gate_proj"], params["up_proj"], H.to_cuda(off), row_ids=ids, block_major=True)
     assert torch.equal(hb.view(torch.uint8), hq.view(torch.uint8)) and torch.equal(sb.t(), sh)
     assert torch.equal(jg.gemm_down(hb, sb, params["down_proj"], H.to_cuda(off), block_major=True), y)
+    seen = set()
     for e in [e for e in range(min(E, 60)) if sizes[e]]:
         lo, hi = int(off[e]), int(off[e + 1])
         one = {n: {k: v[e:e + 1] for k, v in params[n + "_proj"].items()} for n in ("gate", "up", "down")}
@@ -371,9 +372,13 @@ def test_streamed_short_tiles_give_the_same_bits(jg, E, D, I, sizes):
         hq1, sh1 = jg.gemm_gateup_swiglu(xq, sx, one["gate"], one["up"], o1, row_ids=ids[lo:hi].clone())
         assert torch.equal(hq1.view(torch.uint8), hq[lo:hi].view(torch.uint8)) and torch.equal(sh1, sh[lo:hi]), f"expert {e}: h"
         assert torch.equal(jg.gemm_down(hq1, sh1, one["down"], o1), y[lo:hi]), f"expert {e}: y"
-        if e == 0:
-            w, s = one["down"]["w"], one["down"]["scale_inv"]
-            want = O.grouped_gemm(H.codes_np(hq1), sh1.cpu().numpy(), H.codes_np(w), s.cpu().numpy(), np.array([0, hi - lo], np.int32))
+        if sizes[e] not in seen:                                 # one expert of every height: both GEMMs against the oracle
+            seen.add(sizes[e])
+            rows, o1 = ids[lo:hi].long(), np.array([0, hi - lo], np.int32)
+            experts = {n: (H.codes_np(one[n]["w"]), one[n]["scale_inv"].cpu().numpy()) for n in one}
+            xe = H.codes_np(xq[rows]), sx[rows].cpu().numpy()
+            H.assert_h_close(H.codes_np(hq[lo:hi]), sh[lo:hi].cpu().numpy(), *O.expert_swiglu(*xe, experts, o1)[1:], f"h of {sizes[e]} rows")
+            want = O.grouped_gemm(H.codes_np(hq[lo:hi]), sh[lo:hi].cpu().numpy(), *experts["down"], o1)
             H.assert_close_out(H.bf16_to_np(y[lo:hi]), O.bf16_round(want.astype(np.float32)))
 
 
@@ -531,6 +536,7 @@ def test_experts_of_single_tokens_give_the_grouped_bits(jg, M, D, E, k, I, SI, f
     the sorted intermediates), routed or given, with norm, gate and residual, also where h or the rows hold infinities and NaN."""
     import torch
     print("single tokens", M, D, E, k, I, SI, f32, flush=True)
+    same = lambda a, b: torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(7.0, float("inf"), -float("inf")), b.nan_to_num(7.0, float("inf"), -float("inf")))
     params, rand = _layer(jg, D, E, I, SI, M + D)
     names = ("gate_proj", "up_proj", "down_proj")
     ex = {n: params[n] for n in names}
@@ -549,10 +555,16 @@ def test_experts_of_single_tokens_give_the_grouped_bits(jg, M, D, E, k, I, SI, f
         else:
             fwd = lambda **o: jg.moe_experts(x, None, **kw, **o)
         want, dbg = fwd(return_debug=True)
-        assert torch.equal(fwd().nan_to_num(7.0), want.nan_to_num(7.0))
+        assert same(fwd(), want)
         if not SI:
-            got = jg.expert_forward_single(x, dbg["indices"], dbg["weights"], *(params[n] for n in names))
-            assert torch.equal(got.nan_to_num(7.0), want.to(got.dtype).nan_to_num(7.0))
+            given = [params[n] for n in names]
+            got = jg.expert_forward_single(x, dbg["indices"], dbg["weights"], *given)
+            assert same(got, want.to(got.dtype))
+            w = dbg["weights"].clone()                           # infinite rows of the output, by a weight; the same tokens
+            w[M - 1, 0] = float("inf")                           # often enough to be grouped
+            got = jg.expert_forward_single(x, dbg["indices"], w, *given)
+            many = jg.expert_forward_single(x.repeat(20, 1), dbg["indices"].repeat(20, 1), w.repeat(20, 1), *given)
+            assert same(got, many[:M]) and (hard or got[M - 1].isinf().any())
     graph = torch.cuda.CUDAGraph()
     torch.cuda.synchronize()
     with torch.cuda.graph(graph):
@@ -561,7 +573,7 @@ def test_experts_of_single_tokens_give_the_grouped_bits(jg, M, D, E, k, I, SI, f
         out.zero_()
         graph.replay()
         torch.cuda.synchronize()
-        assert torch.equal(out.nan_to_num(7.0), want.nan_to_num(7.0)), f"replay {i}"
+        assert same(out, want), f"replay {i}"
 
 
 @pytest.mark.parametrize("M,k", [(1, 2), (5, 3), (16, 8),     # straight to the experts: both of its kernels leave the rows out
