@@ -356,7 +356,7 @@ def test_streamed_short_tiles_give_the_same_bits(jg, E, D, I, sizes):
     params, rand = _layer(jg, D, E, I, 0, E + D)
     off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
     R = int(off[-1])
-    ids = torch.randperm(R, device="cuda").to(torch.int32)
+    ids = H.to_cuda(H.rng_for(E + D + I).permutation(R).astype(np.int32))
     xq, sx = jg.quant_act(rand(R, D))
     hq, sh = jg.gemm_gateup_swiglu(xq, sx, params["gate_proj"], params["up_proj"], H.to_cuda(off), row_ids=ids)
     y = jg.gemm_down(hq, sh, params["down_proj"], H.to_cuda(off))
@@ -364,7 +364,7 @@ def test_streamed_short_tiles_give_the_same_bits(jg, E, D, I, sizes):
     hb, sb = jg.gemm_gateup_swiglu(xq, gathered, params["gate_proj"], params["up_proj"], H.to_cuda(off), row_ids=ids, block_major=True)
     assert torch.equal(hb.view(torch.uint8), hq.view(torch.uint8)) and torch.equal(sb.t(), sh)
     assert torch.equal(jg.gemm_down(hb, sb, params["down_proj"], H.to_cuda(off), block_major=True), y)
-    seen = set()
+    seen, got_h, want_h = set(), [], []
     for e in [e for e in range(min(E, 60)) if sizes[e]]:
         lo, hi = int(off[e]), int(off[e + 1])
         one = {n: {k: v[e:e + 1] for k, v in params[n + "_proj"].items()} for n in ("gate", "up", "down")}
@@ -377,9 +377,13 @@ def test_streamed_short_tiles_give_the_same_bits(jg, E, D, I, sizes):
             rows, o1 = ids[lo:hi].long(), np.array([0, hi - lo], np.int32)
             experts = {n: (H.codes_np(one[n]["w"]), one[n]["scale_inv"].cpu().numpy()) for n in one}
             xe = H.codes_np(xq[rows]), sx[rows].cpu().numpy()
-            H.assert_h_close(H.codes_np(hq[lo:hi]), sh[lo:hi].cpu().numpy(), *O.expert_swiglu(*xe, experts, o1)[1:], f"h of {sizes[e]} rows")
+            got_h.append((H.codes_np(hq[lo:hi]), sh[lo:hi].cpu().numpy()))
+            want_h.append(O.expert_swiglu(*xe, experts, o1)[1:])
             want = O.grouped_gemm(H.codes_np(hq[lo:hi]), sh[lo:hi].cpu().numpy(), *experts["down"], o1)
             H.assert_close_out(H.bf16_to_np(y[lo:hi]), O.bf16_round(want.astype(np.float32)))
+    # (all of them together, 11000 codes at least: one row of 512 codes has some one that lie on a rounding boundary, and more
+    # than the helper's two in one row of twelve -- Poisson at the 0.2 % that it tells of)
+    H.assert_h_close(*map(np.concatenate, zip(*got_h)), *map(np.concatenate, zip(*want_h)), "h of the sampled experts")
 
 
 @pytest.mark.parametrize("routing", ["softmax", "sigmoid_grouped"])
