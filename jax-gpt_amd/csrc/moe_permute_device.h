@@ -48,19 +48,17 @@ __device__ __forceinline__ void place_pass(const int32_t* ids, int first, int n,
     if (id >= E) id = -1;   // out-of-range ids are dropped rather than corrupting LDS
     const unsigned long long m = match_any(id, bits);
     const int rank = __popcll(m & ((1ull << lane) - 1ull));
+    int pos = -1;   // (a dropped entry has no row)
     if (id >= 0) {
-      int pos = 0;
       if (PLACE) pos = mine[id] + rank;             // every lane of a class reads before its leader bumps the counter
       if (rank == 0) mine[id] += __popcll(m);       // (one writer per counter and instruction)
       if (PLACE) {
         const int f = first + i;
         if (o.sort_order) o.sort_order[pos] = f;
         if (o.sorted_token_ids) o.sorted_token_ids[pos] = (int)((unsigned)f / (unsigned)o.k);   // (half the code of a signed division)
-        if (o.inv_perm) o.inv_perm[f] = pos;
       }
-    } else if (PLACE && i < n && o.inv_perm) {
-      o.inv_perm[first + i] = -1;   // (a dropped entry has no row)
     }
+    if (PLACE && i < n && o.inv_perm) o.inv_perm[first + i] = pos;
   }
 }
 
@@ -102,10 +100,8 @@ __device__ __forceinline__ void permute_few(const int32_t* ids, int n, int E, co
   if (e < n && id >= 0) {
     if (o.sort_order) o.sort_order[pos] = e;
     if (o.sorted_token_ids) o.sorted_token_ids[pos] = (int)(((float)e + 0.5f) * __builtin_amdgcn_rcpf((float)o.k));   // e / k
-    if (o.inv_perm) o.inv_perm[e] = pos;
-  } else if (e < n && o.inv_perm) {
-    o.inv_perm[e] = -1;   // (a dropped entry has no row)
   }
+  if (e < n && o.inv_perm) o.inv_perm[e] = id >= 0 ? pos : -1;   // (a dropped entry has no row)
 }
 
 // The whole sort of one chunk (n entries starting at flat index 0) in one workgroup of kPlaceThreads; ids may be in
