@@ -408,7 +408,7 @@ int moe_route_impl(int routing, const RouteArgs& a, const QuantJob* quant, const
   // Qwen3-MoE, 4096 tokens 14.7 -> 11.0 us, 4000 of the mini layer 9.4 -> 8.4, 8000 of the tiny layer 10.0 -> 9.3 (four waves
   // 16.1, 11.9 and 13.9); without it 2500 tokens of the mini layer from f32 take 66.7 us with sixteen, 68.4 with eight.
   //   A token whose partial sums are the work and that has a CU to itself: a thread a column (513 columns in 32 slices: the
-  // launch 10.5 -> 9.2 us for 1 token, 12.0 -> 10.6 for 200).
+  // launch 10.5 -> 9.3 us for 1 token, 12.0 -> 10.6 for 200).
   const bool own_cu = a.src.partial && tpb == 1 && a.M <= kCUs;
   const int threads = sort_here || (tpb >= 8 && !quant) || (own_cu && a.src.N > 512) ? 1024 : tpb >= 8 || (own_cu && a.src.N > 256) ? 512 : 256;
   job.tokens_per_block = tpb;
