@@ -210,15 +210,17 @@ __device__ __forceinline__ void item_epilogue(v4f (&acc)[NW][NF], const Item& it
     }
     __syncthreads();
     bf16_t* y = (bf16_t*)out;
+    const bool through = sc.out_through;
+    const int wrow0 = item.col_block * 256;
     const int c32 = tid & 31, ld_row = tid >> 5;       // THREADS / 32 rows per pass
-    const int ncols = min(256, N - item.col_block * 256);
+    const int ncols = min(256, N - wrow0);
 #pragma unroll
     for (int i = 0; i < BM / (THREADS / 32); ++i) {
       const int r = ld_row + THREADS / 32 * i;
       if (r < item.row_count && c32 * 8 < ncols) {
         v4i v = *(const v4i*)(tile + r * 512 + ((c32 ^ (r & 7)) << 4));
-        v4i* dst = (v4i*)(y + (size_t)(item.row_start + r) * N + item.col_block * 256 + c32 * 8);
-        store16(dst, v, sc.out_through);
+        v4i* dst = (v4i*)(y + (size_t)(item.row_start + r) * N + wrow0 + c32 * 8);
+        store16(dst, v, through);
       }
     }
   }
