@@ -69,8 +69,8 @@ MOE_API int moe_route_sigmoid_grouped(const float* logits, const float* bias, in
 /* moe.py:58-80 (_sort_and_group): stable counting sort of the flat (token, slot)
  * list by expert id.  Outputs group_sizes (E), group_offsets (E+1), sorted_token_ids
  * (R), sort_order (R), inv_perm (R); any of the last three may be NULL.  An entry whose expert is not in [0, E) is
- * dropped: it has no place in the sorted lists (which end at group_offsets[E]), its inv_perm is -1, and a combine counts
- * its row as zeros. */
+ * dropped: it has no place in the sorted lists (which go on with zeros behind group_offsets[E]), its inv_perm is -1, and a
+ * combine counts its row as zeros. */
 MOE_API size_t moe_permute_workspace_bytes(int M, int k, int E);
 MOE_API int moe_permute(const int32_t* idx, int M, int k, int E, int32_t* group_sizes,
                 int32_t* group_offsets, int32_t* sorted_token_ids, int32_t* sort_order,

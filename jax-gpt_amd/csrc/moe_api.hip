@@ -340,9 +340,7 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
   const bool gather_x = blocked_scales && (R > 96ll * a->E || (long long)R * (a->D / 128) * (a->I / 128) > (1ll << 20));
   if (blocked_scales && !a->out_sh) sc.out_row = 1, sc.out_cb = R;
   if (gather_x) {
-    // (a given selection may hold experts that there are not: their entries are not in the list)
-    const int32_t* listed = given_idx ? b.group_offsets + a->E : nullptr;
-    if ((rc = moe_gather_scales_impl(b.sx, stid, R, listed, a->D / 128, b.sx_listed, stream))) return join(rc);
+    if ((rc = moe_gather_scales(b.sx, stid, R, a->D / 128, b.sx_listed, stream))) return join(rc);
     sx_routed = b.sx_listed;
     sc.in_row = 1, sc.in_kb = R, sc.in_listed = true;
   }

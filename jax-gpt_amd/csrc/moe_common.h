@@ -342,8 +342,6 @@ int moe_rmsnorm_quant_impl(const void* x, int x_f32, const float* weight, float 
 // the combine with the residual and the output in bf16 or (io_f32) f32, the output rounded to bf16 either way
 int moe_combine_impl(const void* y_bf16, const float* w, const int32_t* inv_perm, const void* shared_bf16, const float* shared_gate,
                      const void* residual, int io_f32, int M, int k, int D, void* out, moe_stream_t stream);
-// moe_gather_scales of the first *listed positions (null: n) of a list of n
-int moe_gather_scales_impl(const float* sx, const int32_t* row_ids, int n, const int32_t* listed, int KB, float* out, moe_stream_t stream);
 // the whole sort; its first launch carries the quantisation, if any
 int moe_permute_impl(const int32_t* idx, int M, int k, int E, const PermuteOut& o, void* ws, size_t ws_bytes, const QuantJob* quant,
                      moe_stream_t stream);

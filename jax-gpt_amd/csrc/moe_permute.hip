@@ -84,6 +84,7 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(const int32_t* __r
       o.group_offsets[e] = row_start;
       if (e == E - 1) o.group_offsets[E] = row_start + rows;
     }
+    zero_list_ends(rows_all, R, o);
     if (o.tl.tiles) {   // the grouped GEMMs' row tiles, an expert's tiles side by side (uniform branch)
       const int nt = moe_tile_count(rows, o.tl.tile_rows);
       const int at = moe_tile_first(e, rows, nt, total, before, o.tl);

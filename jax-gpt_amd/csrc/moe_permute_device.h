@@ -62,6 +62,15 @@ __device__ __forceinline__ void place_pass(const int32_t* ids, int first, int n,
   }
 }
 
+// Behind the kept entries, where dropped ones leave the sorted lists without any: zeros, so that whoever walks a list to its
+// end stays inside the rows.  (Whole workgroup; kept: entries that have a place.)
+__device__ __forceinline__ void zero_list_ends(int kept, int R, const PermuteOut& o) {
+  for (int i = kept + (int)threadIdx.x; i < R; i += kPlaceThreads) {
+    if (o.sort_order) o.sort_order[i] = 0;
+    if (o.sorted_token_ids) o.sorted_token_ids[i] = 0;
+  }
+}
+
 // The sort of at most kFewRows entries by one workgroup of kPlaceThreads, without counters or barriers: every wave that has
 // experts holds all entries, one a lane, and its threads go through them, eight at a time, for their experts' rows and what
 // stands in front of them.  An expert that has rows has one tile.  With the counters below the same step of the routing launch
@@ -102,6 +111,7 @@ __device__ __forceinline__ void permute_few(const int32_t* ids, int n, int E, co
     if (o.sorted_token_ids) o.sorted_token_ids[pos] = (int)(((float)e + 0.5f) * __builtin_amdgcn_rcpf((float)o.k));   // e / k
   }
   if (e < n && o.inv_perm) o.inv_perm[e] = id >= 0 ? pos : -1;   // (a dropped entry has no row)
+  zero_list_ends((int)__popcll(__ballot(id >= 0)), n, o);   // (n <= 32: threads of the first wave)
 }
 
 // The whole sort of one chunk (n entries starting at flat index 0) in one workgroup of kPlaceThreads; ids may be in
@@ -140,6 +150,7 @@ __device__ __forceinline__ void permute_one_chunk(const int32_t* ids, int n, int
       }
     }
   }
+  zero_list_ends(rows_all, n, o);
   __syncthreads();
   place_pass<true>(ids, 0, n, E, next, o);
 }

@@ -221,9 +221,9 @@ namespace {
 // all scales of a row in one thread, 64 workgroups of 14 loads a thread, that took 8.2 us, now 4.5; 6216 rows of 56 6.4 -> 4.1.
 constexpr int kGatherScales = 16;
 __global__ __launch_bounds__(256) void gather_scales_kernel(const float* __restrict__ sx, const int32_t* __restrict__ ids,
-                                                           int n, const int32_t* __restrict__ listed, int KB, float* __restrict__ out) {
+                                                           int n, int KB, float* __restrict__ out) {
   const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p >= (listed ? min(n, *listed) : n)) return;
+  if (p >= n) return;
   const float* row = sx + (size_t)(ids ? ids[p] : p) * KB;
   out += p;
   for (int kb0 = blockIdx.y * kGatherScales; kb0 < KB; kb0 += gridDim.y * kGatherScales) {
@@ -250,9 +250,6 @@ __global__ __launch_bounds__(256) void gather_scales_kernel(const float* __restr
 }  // namespace
 
 extern "C" int moe_gather_scales(const float* sx, const int32_t* row_ids, int n, int KB, float* out, moe_stream_t stream) {
-  return moe_gather_scales_impl(sx, row_ids, n, nullptr, KB, out, stream);
-}
-int moe_gather_scales_impl(const float* sx, const int32_t* row_ids, int n, const int32_t* listed, int KB, float* out, moe_stream_t stream) {
   MOE_REQUIRE(n >= 0 && KB >= 1, MOE_ERR_BAD_SHAPE, "gather_scales: bad sizes n=%d KB=%d", n, KB);
   MOE_REQUIRE(n == 0 || (sx && out), MOE_ERR_NULL, "gather_scales: null pointer");
   // (rows of a multiple of four scales are read 16 bytes at a time)
@@ -260,6 +257,6 @@ int moe_gather_scales_impl(const float* sx, const int32_t* row_ids, int n, const
   if (n == 0) return MOE_OK;
   const int parts = KB / kGatherScales + (KB % kGatherScales ? 1 : 0);
   hipLaunchKernelGGL(gather_scales_kernel, dim3((unsigned)((n + 255) / 256), parts < 64 ? parts : 64), dim3(256), 0, (hipStream_t)stream, sx, row_ids,
-                     n, listed, KB, out);
+                     n, KB, out);
   return moe_check_hip(hipGetLastError(), "gather_scales launch");
 }

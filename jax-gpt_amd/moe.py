@@ -105,7 +105,7 @@ def route_sigmoid_grouped(logits, bias, n_group, topk_group, k, renorm=True, rou
 def permute(expert_indices, n_experts):
     """Stable sort of the flat (token, slot) list by expert.  Returns a dict with
     group_sizes (E,), group_offsets (E+1,), sorted_token_ids, sort_order, inv_perm (R,).  Entries outside [0, n_experts)
-    are dropped: the sorted lists end at group_offsets[E], and inv_perm is -1 where an entry has no place."""
+    are dropped: the sorted lists go on with zeros behind group_offsets[E], and inv_perm is -1 where an entry has no place."""
     idx = _dev(expert_indices, torch.int32, "expert_indices")
     M, k = idx.shape
     R = M * k

@@ -606,6 +606,9 @@ def test_selected_experts_that_there_are_not_count_as_zero_rows(jg, M, k):
     inv = np.full(M * k, -1)
     inv[order] = np.arange(n)
     assert np.array_equal(p["sort_order"].cpu().numpy()[:n], order) and np.array_equal(p["sorted_token_ids"].cpu().numpy()[:n], order // k)
+    assert not p["sort_order"][n:].any() and not p["sorted_token_ids"][n:].any()   # (a walk to the lists' ends stays inside the rows)
+    _, sx = jg.quant_act(x)
+    assert torch.equal(jg.gather_scales(sx, p["sorted_token_ids"]), sx[p["sorted_token_ids"].long()].t())
     assert np.array_equal(p["inv_perm"].cpu().numpy(), inv) and int(p["group_offsets"][-1]) == n
     assert np.array_equal(p["group_sizes"].cpu().numpy(), np.bincount(bad.reshape(-1)[flat], minlength=E))
 
