@@ -599,8 +599,13 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
     // Two row tiles of an expert read the same weight lines; over a short K they stay close enough to find them in L2
     // (non-temporal lines leave it first), over a long one the later tile needs the memory-side cache.  Qwen3-MoE, 4096
     // tokens (K = 2048, 768): 269 us with one-tile experts alone marked, 261 with two; DeepSeek-V3 gate/up (K = 7168) at
-    // 4096 tokens: 2426 / 2438 us of the step; all experts whatever their tiles: 8192 tokens 3731 / 3946 us.  Tiles of up
-    // to 128 rows are their expert's only one in most of these launches (the host sees to it) and are always marked.
+    // 4096 tokens: 2426 / 2438 us of the step; all experts whatever their tiles: 8192 tokens 3731 / 3946 us.
+    //   Tiles of up to 128 rows are always marked: without a second K loop each the tall classes are 0.1 to 0.3 % faster (shard
+    // of 16384 rows 786 / 788 us, Qwen3-MoE of 4096 tokens 267 / 268), and where the lists are short most experts have one
+    // tile.  An uneven batch pays for it, as an expert cut into several short tiles is marked too (so / by the rule, normal
+    // offsets of 1 to 3 on the logits): full layer, 500 tokens 604 / 602, 394 / 385, 269 / 262 and 211 / 205 us; DeepSeek-V3, 192
+    // tokens 1102 / 1097, 467 / 443 and 320 / 315, 256 1055 / 1053, 618 / 601 and 343 / 343, 384 1095 / 1084, 556 / 560 and 543 /
+    // 550, 512 1253 / 1256, 682 / 690 and 427 / 430.
     const bool once = __builtin_amdgcn_readfirstlane(item.tiles) <= once_tiles(K);
 #define MOE_CLASS(XF) if (once) MOE_ITEM(XF, true); else MOE_ITEM(XF, false); break
     switch ((rows + 31) >> 5) {

@@ -448,20 +448,23 @@ def test_uneven_groups_that_are_drawn_give_the_same_bits(jg, R):
             assert torch.equal(jg.gemm_down(hq1, sh1, one["down"], o1), y[lo:hi]), f"expert {e}: y"
 
 
-def test_uneven_routing_of_a_layer_of_few_experts(jg):
+@pytest.mark.parametrize("D,E,I,k,M,spread", [
+    (1664, 16, 2048, 3, 1500, 1.5),
+    (4096, 32, 640, 2, 250, 20.0),   # tiles of up to 128 rows, weights from memory
+])
+def test_uneven_routing_of_a_layer_of_few_experts(jg, D, E, I, k, M, spread):
     """The same list inside the layer, written by the sort and read by both GEMMs: the output against its own stages."""
     import torch
-    D, E, I, k, M = 1664, 16, 2048, 3, 1500
-    print("uneven layer", flush=True)
+    print("uneven layer", D, E, flush=True)
     params, rand = _layer(jg, D, E, I, 0, 9)
-    x, lg = rand(M, D), rand(M, E).float() + 1.5 * torch.linspace(1, 0, E, device="cuda")
+    x, lg = rand(M, D), rand(M, E).float() + spread * torch.linspace(1, 0, E, device="cuda")
     ex = {n: params[n] for n in ("gate_proj", "up_proj", "down_proj")}
     out, dbg = jg.moe_experts(x, lg, top_k=k, experts=ex, return_debug=True)
     assert torch.equal(out, jg.moe_experts(x, lg, top_k=k, experts=ex))
-    assert int(dbg["group_sizes"].max()) * E > 2 * M * k
+    assert int(dbg["group_sizes"].max()) > max(2 * M * k // E, 128)
     off = torch.cat([torch.zeros(1, dtype=torch.int32, device="cuda"), dbg["group_sizes"].cumsum(0).to(torch.int32)])
     xq, sx = jg.quant_act(x)
-    for e in range(E):
+    for e in [e for e in range(E) if off[e + 1] > off[e]]:
         lo, hi = int(off[e]), int(off[e + 1])
         one = {n: {k2: v[e:e + 1] for k2, v in ex[n].items()} for n in ex}
         o1 = H.to_cuda(np.array([0, hi - lo], np.int32))
