@@ -25,4 +25,7 @@ struct TokenArgs {
 };
 // whether a call of M tokens takes this route
 bool moe_token_takes(int M, int D, int E, int k, int I, int SI);
+// the second launch: tiles of 16 output columns and waves of a workgroup, LDS of a wave
+struct TokenDownPlan { int tiles, waves, wave_lds; };
+TokenDownPlan moe_token_down_plan(int M, int D, int k, int I, int SI);
 int moe_token_experts(const TokenArgs& a, bool from_memory, moe_stream_t stream);

@@ -242,10 +242,6 @@ int launch_gateup(const TokenArgs& a, bool from_memory, hipStream_t s) {
   return moe_check_hip(hipGetLastError(), "token gate/up launch");
 }
 
-// Up to a workgroup per CU, each with as many tiles as that takes: a row is quantised once, the copies run on from tile to
-// tile, and no CU has a second workgroup of about 80 KB of LDS to begin (full layer, 2 tokens, workgroups of 2 tiles against
-// 512 of one: 70.1 / 74.3 us; mini, 8: 31.3 / 32.9; one workgroup more than there are CUs -- 6 tokens of Qwen3-MoE in 258 --
-// 46.3 against 43.4 in 192).
 int down_tiles(int D, int M) {
   const int cols = D / COLS;
   int tiles = 1;
@@ -256,16 +252,24 @@ int launch_down(const TokenArgs& a, bool from_memory, hipStream_t s) {
   static std::atomic<unsigned long long> raised[2] = {};
   auto* kernel = from_memory ? token_down_kernel<true> : token_down_kernel<false>;
   if (int rc = moe_raise_lds_limit((const void*)kernel, kDownLds, raised[from_memory])) return rc;
-  const int slots = a.k + (a.SI > 0), cols = a.D / COLS;
-  int tiles = down_tiles(a.D, a.M);
-  if (slots > 16 || slots * down_wave_lds(a.h_stride, tiles) > kDownLds) tiles = 1;   // (a wave of several slots)
-  const int per_wave = down_wave_lds(a.h_stride, tiles), fit = kDownLds / per_wave, most = fit < 16 ? fit : 16;
-  const int waves = slots < most ? slots : most;
-  hipLaunchKernelGGL(kernel, dim3((cols + tiles - 1) / tiles, a.M), dim3(64 * waves), waves * per_wave, s, a, tiles);
+  const TokenDownPlan p = moe_token_down_plan(a.M, a.D, a.k, a.I, a.SI);
+  hipLaunchKernelGGL(kernel, dim3((a.D / COLS + p.tiles - 1) / p.tiles, a.M), dim3(64 * p.waves), p.waves * p.wave_lds, s, a, p.tiles);
   return moe_check_hip(hipGetLastError(), "token down launch");
 }
 
 }  // namespace
+
+// Up to a workgroup per CU, each with as many tiles as that takes: a row is quantised once, the copies run on from tile to
+// tile, and no CU has a second workgroup of about 80 KB of LDS to begin (full layer, 2 tokens, workgroups of 2 tiles against
+// 512 of one: 70.1 / 74.3 us; mini, 8: 31.3 / 32.9; one workgroup more than there are CUs -- 6 tokens of Qwen3-MoE in 258 --
+// 46.3 against 43.4 in 192).
+TokenDownPlan moe_token_down_plan(int M, int D, int k, int I, int SI) {
+  const int slots = k + (SI > 0), widest = I > SI ? I : SI;
+  int tiles = down_tiles(D, M);
+  if (slots > 16 || slots * down_wave_lds(widest, tiles) > kDownLds) tiles = 1;   // (a wave of several slots)
+  const int wave_lds = down_wave_lds(widest, tiles), fit = kDownLds / wave_lds, most = fit < 16 ? fit : 16;
+  return {tiles, slots < most ? slots : most, wave_lds};
+}
 
 // Every token reads its experts itself, where the grouped kernels read an expert once for all its rows, and a wave of the second
 // launch walks its tiles' K steps one after the other.  What the launches left out and the finer split gain (3 to 13 us) covers

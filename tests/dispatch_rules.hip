@@ -20,6 +20,15 @@ int main() {
       int M, D, E, k, I, SI;
       std::cin >> M >> D >> E >> k >> I >> SI;
       std::cout << moe_token_takes(M, D, E, k, I, SI) << "\n";
+    } else if (what == "down") {   // tokens, D, k, I, SI: tiles and waves of a workgroup, and whether LDS sets the waves
+      int M, D, k, I, SI;
+      std::cin >> M >> D >> k >> I >> SI;
+      const TokenDownPlan p = moe_token_down_plan(M, D, k, I, SI);
+      std::cout << p.tiles << " " << p.waves << " " << (p.waves < 16 && p.waves < k + (SI > 0)) << "\n";
+    } else if (what == "memory") {   // experts, D, I, SI of a layer
+      long long E, D, I, SI;
+      std::cin >> E >> D >> I >> SI;
+      std::cout << moe_gemm_from_memory((E * I + SI) * D) << "\n";
     } else if (what == "both") {   // routed rows without a list beside a dense group: refused before any GPU call
       alignas(256) static unsigned char memory[1 << 16];
       const float* f = (const float*)memory;

@@ -63,10 +63,24 @@ def test_few_tokens_go_straight_to_their_experts_where_that_is_cheaper(ask):
             (12, 1024, 32, 2, 512, 4096), (16, 1024, 32, 2, 256, 4096), (8, 4096, 4, 2, 1024, 0), (8, 4096, 2, 2, 1024, 1024), (12, 1024, 8, 8, 1024, 0), (12, 768, 8, 8, 1536, 0)]
     assert ask(*[("token", *c) for c in taken]) == ["1"] * len(taken)
     assert ask(*[("token", *c) for c in left]) == ["0"] * len(left)
-    # the batches that test_gpu_variants.py compares with the grouped route do take the other one
+
+
+def test_the_compared_batches_of_single_tokens_reach_what_they_are_for(ask):
+    """The batches that test_gpu_variants.py compares with the grouped route take the other one, and among them are: a last
+    workgroup of fewer tiles, one over two scale blocks, more slots than waves, waves that LDS limits, weights from memory."""
     from tests.test_gpu_variants import test_experts_of_single_tokens_give_the_grouped_bits as single
-    marks = [m.args[1] for m in single.pytestmark if m.name == "parametrize" and "M,D" in m.args[0]]
-    assert marks and ask(*[("token", *c) for c in marks[0]]) == ["1"] * len(marks[0])
+    cases, = [m.args[1] for m in single.pytestmark if m.name == "parametrize" and "M,D" in m.args[0]]
+    assert ask(*[("token", *c) for c in cases]) == ["1"] * len(cases)
+    memory = [v == "1" for v in ask(*[("memory", E, D, I, SI) for M, D, E, k, I, SI in cases])]
+    plans = [tuple(map(int, v.split())) for v in ask(*[("down", M, D, k, I, SI) for M, D, E, k, I, SI in cases])]
+    reached = {"from memory": memory}
+    reached["last workgroup"] = [D // 16 % t > 0 for (M, D, *_), (t, _, _) in zip(cases, plans)]
+    reached["two scale blocks"] = [any(b * t % 8 + min(t, D // 16 - b * t) > 8 for b in range(-(-D // 16 // t))) for (M, D, *_), (t, _, _) in zip(cases, plans)]
+    reached["sixteen waves"] = [w == 16 < k + (SI > 0) for (*_, k, I, SI), (_, w, _) in zip(cases, plans)]
+    reached["lds"] = [bool(limited) for _, _, limited in plans]
+    reached["several tokens from memory"] = [m and c[0] > 1 for m, c in zip(memory, cases)]
+    assert all(map(any, reached.values())), reached
+    assert {t for t, _, _ in plans} >= {1, 2, 3, 16}
 
 
 def test_a_dense_group_beside_routed_rows_needs_their_list(ask):

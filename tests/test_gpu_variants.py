@@ -155,9 +155,10 @@ def test_given_selection_with_a_shared_expert(jg, M):
     print("given selection with a shared expert", M, flush=True)
     D, k = 4096, 2
     params, rand = _layer(jg, D, 8, 128, 256, M)
-    x, lg = rand(M, D), rand(M, 8).float()
+    x, lg = rand(max(M, 40), D), rand(max(M, 40), 8).float()
     ex, sh = ({n: params[p + n] for n in ("gate_proj", "up_proj", "down_proj")} for p in ("", "shared_"))
-    want = jg.moe_experts(x, lg, top_k=k, experts=ex, shared=sh)
+    want = jg.moe_experts(x, lg, top_k=k, experts=ex, shared=sh)[:M]      # (five tokens go straight to their experts, forty do not)
+    x, lg = x[:M], lg[:M]
     assert torch.equal(moe._forward(x, None, k, ex, shared=sh, selected=jg.route_softmax_topk(lg, k)), want)
 
 
@@ -271,6 +272,11 @@ def test_few_tokens_behind_the_norm_give_the_bits_of_a_larger_batch(jg, D, E, SI
     norm = rand(D).float() * 0.1
     x[0, 1] = 0                                              # an all-zero row
     want = jg.moe_sublayer(x, norm, params, 2)
+    names = ("gate_proj", "up_proj", "down_proj")
+    sorted_want, _ = jg.moe._forward(x[0], None, 2, params, shared={n: params["shared_" + n] for n in names} if SI else None,   # the grouped route
+                                     gate_weight=params["gate_weight"], norm_weight=norm, add_residual=True, io_f32=dtype == "f32",
+                                     shared_expert_gate_weight=params["shared_expert_gate_weight"] if SI else None, return_debug=True)
+    assert torch.equal(sorted_want, want[0])
     for m in (1, 2, 3, 4):
         assert torch.equal(jg.moe_sublayer(x[:, :m].contiguous(), norm, params, 2), want[:, :m]), f"{m} tokens"
 
@@ -520,6 +526,11 @@ def test_few_entries_of_a_layer(jg, M, k, E):
     kw = dict(top_k=k, experts=dict(zip(("gate_proj", "up_proj", "down_proj"), ex)))
     whole = jg.moe_experts(x, lg, **kw)
     assert torch.equal(jg.moe_experts(x[:M].contiguous(), lg[:M].contiguous(), **kw), whole[:M])
+    got, dbg = jg.moe_experts(x[:M].contiguous(), lg[:M].contiguous(), return_debug=True, **kw)   # (sorted, not straight to the experts)
+    ref = O.sort_and_group(dbg["indices"].cpu().numpy(), E)
+    assert torch.equal(got, whole[:M])
+    for name in ("group_sizes", "sorted_token_ids", "inv_perm"):
+        assert np.array_equal(dbg[name].cpu().numpy(), ref[name]), name
     w = rand(M, k).float()
     same = torch.full((M, k), E - 2, dtype=torch.int32, device="cuda")
     many = same.repeat(20, 1)
@@ -529,13 +540,16 @@ def test_few_entries_of_a_layer(jg, M, k, E):
 
 @pytest.mark.parametrize("M,D,E,k,I,SI", [
     (1, 128, 8, 2, 128, 0),       # one K step, eight tiles
-    (16, 512, 8, 2, 1024, 0),     # the most tokens, tiles of different scale blocks in a workgroup
-    (13, 384, 33, 3, 256, 384),   # tiles that do not divide, a shared expert wider than the routed ones
+    (16, 512, 8, 2, 1024, 0),     # the most tokens, two tiles a workgroup
+    (9, 1024, 8, 2, 256, 0),      # three: some span two scale blocks, and the last workgroup has one
+    (13, 384, 33, 3, 256, 384),   # a shared expert wider than the routed ones
     (3, 896, 40, 17, 128, 128),   # more slots than waves
     (2, 256, 40, 32, 256, 128),   # the most slots
     (16, 4096, 4, 1, 128, 128),   # sixteen tiles a workgroup
-    (1, 2048, 8, 8, 2432, 128),   # rows whose rings do not fit beside each other for every slot
-    (1, 7168, 16, 8, 512, 512),   # one token of a layer from memory (non-temporal copies)
+    (1, 2048, 8, 8, 2432, 128),   # longer rows of the routed experts than of the shared one
+    (1, 128, 8, 8, 13312, 128),   # rows whose rings do not fit beside each other for every slot
+    (1, 7168, 18, 8, 512, 512),   # one token of a layer from memory (non-temporal copies) ...
+    (2, 7168, 18, 8, 512, 512),   # ... and two
 ])
 @pytest.mark.parametrize("f32", [False, True])
 def test_experts_of_single_tokens_give_the_grouped_bits(jg, M, D, E, k, I, SI, f32):
