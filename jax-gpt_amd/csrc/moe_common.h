@@ -170,15 +170,17 @@ __device__ inline int moe_tile_first(int e, int rows, int nt, int* lds_a, int* l
   __syncthreads();
   const int order = rows > 0 ? atomicAdd(&lds_a[cls], 1) : 0;
   __syncthreads();
-  int before = lds_a[e], unused = 0, nz, unused_all;   // nz: experts with rows
-  moe_scan_1024(before, unused, nz, unused_all);
+  int before = lds_a[e], tiles_to = nt, nz, all_tiles;   // nz: experts with rows
+  moe_scan_1024(before, tiles_to, nz, all_tiles);
   lds_b[e] = before;
   __syncthreads();
   const int rank = lds_b[cls] + order;
   const int nr = (nz + 7) >> 3;   // rounds that hold a non-empty expert
   int tail = nr / 4 < kTailRounds ? nr / 4 : kTailRounds;   // (3 rounds = 24 experts over the 8 bins; 6 measured no better)
   int pool_most = max_tiles >> 4;
-  if (l.pool_tiles > pool_most && __syncthreads_or((long long)rows * nz > 2ll * l.rows)) {   // (an expert of twice the mean)
+  const long long all_items = (long long)all_tiles * (l.ncb[0] ? l.ncb[0] : l.ncb[1]);
+  const bool whole = all_items == 256 || all_items == 512;   // one or two full rounds: equal shares end together, draws do not
+  if (l.pool_tiles > pool_most && !whole && __syncthreads_or((long long)rows * nz > 2ll * l.rows)) {   // (an expert of twice the mean)
     tail = nr > kWideTailRounds ? kWideTailRounds : nr - 1;
     pool_most = l.pool_tiles;
   }

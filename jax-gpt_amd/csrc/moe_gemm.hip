@@ -644,10 +644,11 @@ constexpr int kFullTileItems = 768;
 // Lists whose pool may be large: of up to 8 rounds at most (the fewer, the larger a part the last one is; up to 10 the
 // expert-parallel shard of 16384 rows takes 786 us, up to 8 778), of items of 12 K steps (14 us) and more.  Shorter items lose
 // more by the draw (Qwen3-MoE, 2800 tokens 217 -> 221 us, 4000 of the mini layer 76 -> 79.5).
-//   What it gains hangs on how a launch's last round comes out.  32 experts of 7168 x 2048 with Zipf(1.2) rows, 720 to 9600 of them
-// in 28 steps, large pool against small: gate/up -4.6 % on average (-20 %, 229 / 286 us, at 6400), down -3.1 % (even up to 1640
-// rows, -17 % at 4320).  It loses where equal shares are whole rounds: gate/up +2 % at 880 and 960 rows, +1 to +13 % from 1760 to
-// 2240 (161 / 143 us at 1920), down +2 to +6 % from 1760 to 2080.
+//   32 experts of 7168 x 2048, all or 29 of them with rows, Zipf(0.8 / 1.2 / 1.6), 560 to 3600 rows in 80s, large pool against small:
+// gate/up -6.3 % on average (-28 % where the last round came out worst), down -4.0 %; up to 10000 rows alike.  Not for lists of one
+// or two full rounds of items (moe_tile_first): equal shares end together there and draws do not (2000 to 2240 rows, 32 tiles of 16
+// columns: 154 to 173 us, 176 to 184 with the large pool; else +0.6 to +4.5 %).  It still loses now and then where the shares
+// nearly are whole rounds (31 tiles, 1200 to 1440 rows of Zipf(1.6): +5 to +13 %; other 31 tiles -1 to -11 %).
 int moe_gemm_pool_tiles(int max_tiles, int tile_rows, int ncb_least, int kb) {
   const bool few = (long long)max_tiles * ncb_least <= 8 * 256 && kb >= 12 && tile_rows > kStreamRows;
   return few ? max_tiles >> 2 : max_tiles >> 4;

@@ -427,7 +427,7 @@ def test_scales_are_gathered_whole(jg, n, KB):
     assert torch.equal(jg.gather_scales(sx, n_rows=n), sx[:n].t())
 
 
-@pytest.mark.parametrize("R", [2600, 6100, 9000])
+@pytest.mark.parametrize("R", [2100, 2600, 6100, 9000])   # (the first: 32 tiles of 16 column blocks, two full rounds: no large pool)
 def test_uneven_groups_that_are_drawn_give_the_same_bits(jg, R):
     """Few rounds of long items of uneven groups: most of the list is a pool that the XCDs draw from (empty experts, one of
     many tiles and of one row among them).  And the even split of the same rows, whose pool is small."""
