@@ -17,6 +17,9 @@ LIB_PATH = os.path.join(HERE, "libmoe_hip.so")
 # the timing probe of the grouped GEMM's K loop (`python bench.py --probe`): its own library, nothing of the product links it
 PROBE_PATH = os.path.join(HERE, "libmoe_probe.so")
 
+# the layer calls' host work (a Python extension over torch's headers; it gets the library's functions by address)
+CALL_PATH = os.path.join(HERE, "moe_call.so")
+
 SOURCES = ["moe_api.hip", "moe_route.hip", "moe_router.hip", "moe_permute.hip", "moe_quant.hip", "moe_gemm.hip", "moe_gemm_stream.hip",
            "moe_token.hip", "moe_combine.hip"]
 # no v_pk_*_f32 code generation (some packed-f32 forms have given wrong results on this hardware)
@@ -40,12 +43,27 @@ def _hipcc() -> str:
     raise RuntimeError("hipcc not found: the MI355X kernels cannot be built")
 
 
+def _call_command() -> list[str]:
+    import sysconfig
+
+    import torch
+    base = os.path.dirname(torch.__file__)
+    return [shutil.which("g++") or "g++", "-O2", "-shared", "-fPIC", "-std=c++17", "-Wall", "-fvisibility=hidden",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", "-I", os.path.join(ROOT, "include"),
+            "-isystem", os.path.join(base, "include"), "-isystem", sysconfig.get_paths()["include"],
+            os.path.join(CSRC, "moe_call.cpp"), "-o", CALL_PATH, "-L", os.path.join(base, "lib"), "-lc10", "-ltorch_cpu", "-ltorch_python"]
+
+
 def build(verbose: bool = True, jobs: int = 6) -> str:
     hipcc = _hipcc()
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
     procs = []
     objs = []
+    call = _call_command()
+    if verbose:
+        print(" ".join(call), flush=True)
+    procs.append(("moe_call.cpp", subprocess.Popen(call, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
     for src in SOURCES:
         obj = os.path.join(objdir, src.replace(".hip", ".o"))
         objs.append(obj)
@@ -76,7 +94,7 @@ def _drain(procs):
         if out:
             print(out, flush=True)
         if p.returncode != 0:
-            raise RuntimeError(f"hipcc failed on {src}")
+            raise RuntimeError(f"the compiler failed on {src}")
 
 
 if __name__ == "__main__":
