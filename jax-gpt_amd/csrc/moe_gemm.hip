@@ -124,7 +124,7 @@ __global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __rest
 // each lane fetches.  No asynchronous load ever targets a register.
 
 // One launch, row tiles of every height.  A work item's row tile (at most 288 rows, near-equal cuts of its
-// expert) is served by the smallest of nine compiled tile classes that holds it -- 32 XF rows, XF = 1 .. 9 MFMA
+// expert) is served by the smallest of nine (ten: TALL) compiled tile classes that holds it -- 32 XF rows, XF = 1 .. 9 MFMA
 // groups per wave and K step -- each a branch-free, fully unrolled K loop of its own with its own LDS ring: the
 // short classes have short activation tiles and use the room for more stages (256 and 288 rows: two stages; 160 to 224
 // rows: three weight stages, two activation stages; 64 to 128 rows: three stages, copies two steps ahead; 32 rows:
@@ -178,7 +178,10 @@ template <int XF, int MODE = MODE_GATEUP, bool ONCE = true> struct Cls {
   static constexpr int X_OPS = XF;                     // activation copies per copying wave and step
   static constexpr int S_OPS = BM > 256 ? 2 : 1;       // scale copies: 64 slots each, four waves
   static constexpr int XS_OPS = X_OPS + S_OPS;
-  static constexpr bool S_LATE = XF == 9;              // read a group's scale with its fragment (registers: 144 are accumulators)
+  // Result registers of a wave: the FMAs that scale an MFMA's results stand NP MFMAs behind it.  At 320 rows (160 accumulators)
+  // two quadruples are what the register file has left; with four 25 values of the K loop spill, with three 10.
+  static constexpr int NP = XF >= 10 ? 2 : 4;
+  static constexpr bool S_LATE = XF >= 9;              // read a group's scale with its fragment (registers: 144 are accumulators)
   static constexpr int OPS = 8 + XS_OPS;               // + 8 weight row groups
   // Copies complete in the order of their issue, so within a step those with the earlier deadline go first: with
   // the deeper weight ring the activation copies (and scales), then the weights; with rings of one depth the
@@ -215,18 +218,20 @@ template <int XF, int MODE = MODE_GATEUP, bool ONCE = true> struct Cls {
   }
 };
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
-constexpr int CLS_RING = cmax(cmax(cmax(cmax(Cls<9>::RING_BYTES, Cls<8>::RING_BYTES), Cls<7>::RING_BYTES), cmax(Cls<6>::RING_BYTES, Cls<5>::RING_BYTES)),
+constexpr int CLS_RING = cmax(cmax(cmax(cmax(cmax(Cls<10>::RING_BYTES, Cls<9>::RING_BYTES), Cls<8>::RING_BYTES), Cls<7>::RING_BYTES), cmax(Cls<6>::RING_BYTES, Cls<5>::RING_BYTES)),
                               cmax(cmax(Cls<4>::RING_BYTES, Cls<3>::RING_BYTES), cmax(Cls<2>::RING_BYTES, Cls<1>::RING_BYTES)));
 constexpr int CLS_WSCALE_OFF = CLS_RING;                       // [2][MAX_KB] weight block scales of the work item
 constexpr int CLS_FLAG_OFF = CLS_WSCALE_OFF + 2 * MAX_KB * 4;  // [4] early_flag: the step whose weight fragments wave (wi, 1) holds, + 1
 constexpr int CLS_LDS_BYTES = CLS_FLAG_OFF + 16;              // 160016
-static_assert(CLS_LDS_BYTES <= 160 * 1024, "LDS");
+constexpr int TALL_LDS_BYTES = 160 * 1024;
+static_assert(CLS_LDS_BYTES <= TALL_LDS_BYTES, "LDS");
 // The epilogues stage their results where the rings were, all of CLS_RING whatever the class's own rings take: gate/up
-// four f32 maxima and 128 codes a row, down 256 bf16 a row -- 144 KB at 288 rows, whose rings are 139 KB.
-template <int XF> constexpr bool epilogue_fits() {
-  return Cls<XF>::BM * (4 * 4 + BK) <= CLS_RING && Cls<XF>::BM * 256 * 2 <= CLS_RING;
+// four f32 maxima and 128 codes a row, down 256 bf16 a row -- 144 KB at 288 rows, whose rings are 139 KB; at 320 rows 160 KB,
+// the scales' and flags' places included.
+template <int XF> constexpr bool epilogue_fits(int bytes) {
+  return Cls<XF>::BM * (4 * 4 + BK) <= bytes && Cls<XF>::BM * 256 * 2 <= bytes;
 }
-static_assert(epilogue_fits<9>(), "the tallest tile's epilogue stages inside the rings' space");
+static_assert(epilogue_fits<9>(CLS_RING) && epilogue_fits<10>(TALL_LDS_BYTES), "the tallest tile's epilogue stages inside the LDS");
 
 template <int MODE, int XF, bool ONCE>
 __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const uint8_t* __restrict__ xq,
@@ -352,16 +357,29 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
 #pragma unroll
     for (int j = 0; j < XF; ++j) acc[f][j] = (v4f){0.f, 0.f, 0.f, 0.f};
   v8i wf[4];
-  v4f p[4];
+  v4f p[C::NP];
   float pc0 = 0.f, pc1 = 0.f;   // scales of the group whose FMAs are pending
   auto fm = [&](int f, int jj, float c0, float c1) {
-    acc[f][jj] += p[f] * ((MODE == MODE_GATEUP && f >= 2) ? c1 : c0);
+    acc[f][jj] += p[(4 * jj + f) % C::NP] * ((MODE == MODE_GATEUP && f >= 2) ? c1 : c0);
   };
-  auto mm = [&](int f, const v8i& x) {
-    p[f] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[f], x, (v4f){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+  auto mm = [&](int f, int jj, const v8i& x) {
+    p[(4 * jj + f) % C::NP] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[f], x, (v4f){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
   };
   auto fence = [&]() {
     __builtin_amdgcn_sched_barrier(0);
+  };
+  // group j's MFMAs, each behind the FMAs that finish the one NP before it, and the FMAs still pending behind a step's last group
+  auto group = [&](int j, bool pending, const v8i& x, float c0, float c1) {
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      if (f >= C::NP) fm(f - C::NP, j, c0, c1);
+      else if (pending) fm(f + 4 - C::NP, j - 1, pc0, pc1);
+      mm(f, j, x);
+    }
+  };
+  auto finish = [&]() {
+#pragma unroll
+    for (int f = 4 - C::NP; f < 4; ++f) fm(f, XF - 1, pc0, pc1);
   };
   // The two waves of a SIMD belong to different wave sets (xj = 0 / 1).  Set 1 runs ROT groups behind set 0: it
   // carries the last ROT activation fragments of a step (and their scales) in registers across the barrier and
@@ -399,11 +417,7 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
         if (!FIRST) {
 #pragma unroll
           for (int i = 0; i < ROT; ++i) {
-#pragma unroll
-            for (int f = 0; f < 4; ++f) {
-              fm(f, NG + i - 1, pc0, pc1);
-              mm(f, held[i]);
-            }
+            group(NG + i, true, held[i], hc0[i], hc1[i]);
             pc0 = hc0[i];
             pc1 = hc1[i];
             if (COPY) {
@@ -421,7 +435,11 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
       }
       const uint8_t* wt = lds + (kb % C::W_NST) * W_TILE_BYTES;
       const uint8_t* xs = lds + C::X_RING_OFF + (kb % C::X_NST) * C::X_STAGE_BYTES;
-      const float s0 = ws0[kb], s1 = MODE == MODE_GATEUP ? ws1[kb] : s0;
+      float s0 = ws0[kb], s1 = MODE == MODE_GATEUP ? ws1[kb] : s0;
+      if (C::NP < 4) {   // (in scalar registers)
+        s0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(s0)));
+        s1 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(s1)));
+      }
       const uint8_t* xt = xs + xj * 16 * BK;
       // Every wave of a wave set asks LDS for its first fragments at this moment: the reads come back in issue
       // order, so the first MFMA's operands (activation fragment 0, weight fragment 0) are asked for first and the
@@ -452,10 +470,7 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
           for (int j = 0; j < XF; ++j) sxv[j] = *(const float*)(sp + j * 4);
         }
       }
-      if (!FIRST) {
-#pragma unroll
-        for (int f = 0; f < 4; ++f) fm(f, XF - 1, pc0, pc1);
-      }
+      if (!FIRST) finish();
       fence();
 #pragma unroll
       for (int j = 0; j < NG; ++j) {
@@ -472,11 +487,9 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
             hc1[i] = sxv[NG + i] * s1;
           }
         }
-#pragma unroll
-        for (int f = 0; f < 4; ++f) {
-          if (j > 0) fm(f, j - 1, pc0, pc1);
-          mm(f, xf[j & 1]);
-        }
+        float c0 = 0.f, c1 = 0.f;
+        if (C::NP < 4) c0 = sxv[j] * s0, c1 = sxv[j] * s1;
+        group(j, j > 0, xf[j & 1], c0, c1);
         // pinned order: the next group's fragment reads first (a whole group of latency cover), then FMA quadruple f
         // just before MFMA f (left alone the compiler puts all 16 FMAs before the 4 MFMAs: down GEMM 3-6 % slower)
         if (j + 1 < NG) __builtin_amdgcn_sched_group_barrier(0x100, C::S_LATE ? 3 : 2, 0);
@@ -486,11 +499,11 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
         }
 #pragma unroll
         for (int f = 0; f < 4; ++f) {
-          if (j > 0) __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+          if (j > 0 || f >= C::NP) __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         }
-        pc0 = sxv[j] * s0;
-        pc1 = sxv[j] * s1;
+        pc0 = C::NP < 4 ? c0 : sxv[j] * s0;
+        pc1 = C::NP < 4 ? c1 : sxv[j] * s1;
         if (C::W_EARLY && COPY && KIND == 2 && ROT + j == C::EARLY_G) {
           // The weight copies from here on overwrite the stage that this step reads: this wave is past its own
           // fragment loads; the other reader of its rows, wave (wi, 1), says so through early_flag.  (It entered the
@@ -543,19 +556,15 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
     if constexpr (ROT > 0) {   // the groups carried out of the last step
 #pragma unroll
       for (int i = 0; i < ROT; ++i) {
-#pragma unroll
-        for (int f = 0; f < 4; ++f) {
-          fm(f, NG + i - 1, pc0, pc1);
-          mm(f, held[i]);
-        }
+        group(NG + i, true, held[i], hc0[i], hc1[i]);
         pc0 = hc0[i];
         pc1 = hc1[i];
       }
     }
-#pragma unroll
-    for (int f = 0; f < 4; ++f) fm(f, XF - 1, pc0, pc1);
+    finish();
   };
-  constexpr int ROT1 = XF == 9 ? 1 : XF > ROTC ? ROTC : XF - 1;   // (fewer groups than that: what there is)
+  // (fewer groups than that: what there is, or what the register file has room for)
+  constexpr int ROT1 = XF >= 10 ? 0 : XF == 9 ? 1 : XF > ROTC ? ROTC : XF - 1;
   if (xj == 0) run(std::integral_constant<int, 0>{}, std::true_type{});
   else run(std::integral_constant<int, ROT1>{}, std::false_type{});
   __syncthreads();   // every wave is done reading the ring before the epilogue reuses LDS
@@ -574,7 +583,8 @@ __host__ __device__ inline int once_tiles(int K) { return K <= 2048 ? 2 : 1; }
 // launch some 0.7 us (0.8 % of the prefill step).
 // STREAM: weights come from memory and most experts have one row tile, so items mark their weight lines non-temporal
 // where that pays.  Otherwise every copy is a plain one (launch()).
-template <int MODE, bool DENSE, bool STREAM>
+// TALL: tiles of up to 320 rows (moe_tile_rows_voted); a kernel of its own, as the tenth class costs the others 0.5 to 1.5 %.
+template <int MODE, bool DENSE, bool STREAM, bool TALL>
 __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands routed, TileHeader* hdr,
                                                             const TileEntry* __restrict__ tiles, const GemmOperands dense,
                                                             int dense_rows, int dense_tiles, int dense_blocks) {
@@ -609,6 +619,7 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
     const bool once = __builtin_amdgcn_readfirstlane(item.tiles) <= once_tiles(K);
 #define MOE_CLASS(XF) if (once) MOE_ITEM(XF, true); else MOE_ITEM(XF, false); break
     switch ((rows + 31) >> 5) {
+      case 10: if constexpr (TALL) { MOE_CLASS(10); }
       case 9: MOE_CLASS(9);
       case 8: MOE_CLASS(8);
       case 7: MOE_CLASS(7);
@@ -622,6 +633,7 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
 #undef MOE_CLASS
   } else {
     switch ((rows + 31) >> 5) {
+      case 10: if constexpr (TALL) { MOE_ITEM(10, false); break; }
       case 9: MOE_ITEM(9, false); break;
       case 8: MOE_ITEM(8, false); break;
       case 7: MOE_ITEM(7, false); break;
@@ -656,7 +668,7 @@ int moe_gemm_pool_tiles(int max_tiles, int tile_rows, int ncb_least, int kb) {
 
 // ncb: column blocks of the list's GEMMs (0: none); kb: the fewest K steps of these
 TileList tile_list(void* ws, int R, int E, int tile_rows, int ncb_gateup, int ncb_down, int kb) {
-  const int max_tiles = max_tiles_for(R, E, tile_rows), ncb = ncb_down && ncb_down < ncb_gateup ? ncb_down : ncb_gateup;
+  const int max_tiles = max_tiles_for(R, E, tile_rows < kTileRows ? tile_rows : kTileRows), ncb = ncb_down && ncb_down < ncb_gateup ? ncb_down : ncb_gateup;
   return TileList{max_tiles, moe_gemm_pool_tiles(max_tiles, tile_rows, ncb, kb), R, tile_rows, (TileHeader*)ws,
                   (TileEntry*)((char*)ws + sizeof(TileHeader)), {ncb_gateup, ncb_down},
                   {(32 << kTileQBits) / (ncb_gateup ? ncb_gateup : 1), (32 << kTileQBits) / (ncb_down ? ncb_down : 1)}};
@@ -758,11 +770,14 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
   if (moe_gemm_streams(MODE, tallest, items))
     return moe_gemm_stream_launch(MODE, StreamLaunch{routed, l.hdr, l.tiles, l.rows, dense, dense_rows, dense_tiles, (int)dense_blocks,
                                                      stream, (unsigned)grid, tallest}, s);
-  static std::atomic<unsigned long long> lds_raised[4] = {};
-  auto* kernel = dn ? (stream ? grouped_gemm_kernel<MODE, true, true> : grouped_gemm_kernel<MODE, true, false>)
-                    : (stream ? grouped_gemm_kernel<MODE, false, true> : grouped_gemm_kernel<MODE, false, false>);
-  if (int rc = moe_raise_lds_limit((const void*)kernel, CLS_LDS_BYTES, lds_raised[(dn ? 2 : 0) + stream])) return rc;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(NT), CLS_LDS_BYTES, s, routed, l.hdr, l.tiles, dense, dense_rows,
+  static std::atomic<unsigned long long> lds_raised[6] = {};
+  const bool tall = !dn && tallest > kTileRows;
+  auto* kernel = dn ? (stream ? grouped_gemm_kernel<MODE, true, true, false> : grouped_gemm_kernel<MODE, true, false, false>)
+               : tall ? (stream ? grouped_gemm_kernel<MODE, false, true, true> : grouped_gemm_kernel<MODE, false, false, true>)
+                      : (stream ? grouped_gemm_kernel<MODE, false, true, false> : grouped_gemm_kernel<MODE, false, false, false>);
+  const int lds = tall ? TALL_LDS_BYTES : CLS_LDS_BYTES;
+  if (int rc = moe_raise_lds_limit((const void*)kernel, lds, lds_raised[(dn ? 2 : tall ? 4 : 0) + stream])) return rc;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(NT), lds, s, routed, l.hdr, l.tiles, dense, dense_rows,
                      dense_tiles, (int)dense_blocks);
   return moe_check_hip(hipGetLastError(), "gemm launch");
 }
@@ -788,6 +803,13 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
 // 844 / 855, 400 1037 / 1062, 256 1028 / 1019.  A shared expert beside them is cut alike: where the two tiles that 84 tokens of the
 // DeepSeek-V3 layer have more than in one of 96 rows begin another round of items (125 experts touched, which the host does
 // not know) 852 / 835; 33 to 128 tokens otherwise -1.0 to +1.5 %, -0.2 on average.
+//   Tall tiles (320 rows, moe_tile_rows_voted) for lists of both GEMMs, of short K and at most eight rounds, where an even routing
+// puts the largest groups, 2.5 to 3 standard deviations above the mean, between whole full tiles and whole tall ones: with full
+// tiles alone a few of Qwen3-MoE's 128 experts have two at 4096 tokens, 130 tiles x 6 and x 8 columns, 3.05 and 4.06 rounds: gate/up
+// 135 -> 130, down 88.4 -> 84.3, the layer 256 -> 242 us; 3950 tokens through the two functions 269 -> 257, 8192 tokens 446 -> 428, 4600
+// 284 -> 278.  The kernel that has this height too runs the other heights 0.5 to 1.5 % slower, which is what a wrong guess costs
+// and why K = 7168 (64 experts of 266 rows 538 -> 504 and 298 -> 289, but sixteen rounds even) and rows that another GPU has
+// dispatched, which are uneven, go without.
 int moe_gemm_tile_rows(const TileShape& t) {
   const int groups = t.E < t.R ? t.E : t.R;
   if (groups <= 0) return kTileRows;
@@ -796,9 +818,13 @@ int moe_gemm_tile_rows(const TileShape& t) {
   const int mean = (t.R + groups - 1) / groups;
   if (mean > kFullTileItems * kTileRows / groups) return kTileRows;
   const int least = !t.ncb[0] || (t.ncb[1] && t.ncb[1] < t.ncb[0]) ? t.ncb[1] : t.ncb[0];
-  if (t.E > 1 && groups * ((mean + kTileRows - 1) / kTileRows) * least >= kFullTileItems) return kTileRows;
   int spread = 0;
   while (t.E > 1 && spread * spread < 4 * mean) ++spread;
+  if (t.E > 1 && groups * ((mean + kTileRows - 1) / kTileRows) * least >= kFullTileItems) {
+    const int n = moe_tall_tiles(t.R, t.E), longest = t.kb[0] > t.kb[1] ? t.kb[0] : t.kb[1];
+    const bool may_end_alike = 2 * mean + 3 * spread > 2 * n * kTileRows && 4 * mean + 5 * spread <= 4 * n * kTallTileRows;
+    return t.ncb[0] && t.ncb[1] && !t.dense_rows && longest <= 16 && (long long)groups * n * least <= 8 * 256 && may_end_alike ? kTallTileRows : kTileRows;
+  }
   const int units = (mean + spread + 31) / 32, dense_units = (t.dense_rows + 31) / 32;
   int best = 0, best_u = kTileRows / 32;
   for (int u = kTileRows / 32; u >= 1; --u) {

@@ -76,8 +76,8 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(const int32_t* __r
   if (c >= 0) place_pass<false>(ids + first, first, n, E, smem, o);
   __syncthreads();
   const int rows = total[e];
-  int row_start = rows, unused = 0, rows_all, unused_all;
-  moe_scan_1024(row_start, unused, rows_all, unused_all);
+  int row_start = rows, vote = o.tl.tile_rows > kTileRows ? moe_tall_vote(rows, moe_tall_tiles(R, E)) : 0, rows_all, votes;
+  moe_scan_1024(row_start, vote, rows_all, votes);
   if (c < 0) {
     if (e < E) {
       o.group_sizes[e] = rows;
@@ -86,7 +86,7 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(const int32_t* __r
     }
     zero_list_ends(rows_all, R, o);
     if (o.tl.tiles) {   // the grouped GEMMs' row tiles, an expert's tiles side by side (uniform branch)
-      const int nt = moe_tile_count(rows, o.tl.tile_rows);
+      const int nt = moe_tile_count(rows, moe_tile_rows_voted(o.tl.tile_rows, votes));
       const int at = moe_tile_first(e, rows, nt, total, before, o.tl);
       for (int t = 0; t < nt; ++t)
         if (at + t < o.tl.max_tiles) o.tl.tiles[at + t] = TileEntry{e | nt << 10, row_start, rows, at};

@@ -1,6 +1,7 @@
 // Prints what the library's host-side dispatch rules say: one command a line on stdin, one answer a line.
 #include <iostream>
 #include <string>
+#include <vector>
 
 #include "moe_gemm_device.h"
 #include "moe_token.h"
@@ -29,6 +30,13 @@ int main() {
       long long E, D, I, SI;
       std::cin >> E >> D >> I >> SI;
       std::cout << moe_gemm_from_memory((E * I + SI) * D) << "\n";
+    } else if (what == "voted") {   // rows of a full tile of a list that may have tall ones: groups, then the rows of each
+      int E, R = 0, votes = 0;
+      std::cin >> E;
+      std::vector<int> rows(E);
+      for (int& r : rows) std::cin >> r, R += r;
+      for (int r : rows) votes += moe_tall_vote(r, moe_tall_tiles(R, E));
+      std::cout << moe_tile_rows_voted(kTallTileRows, votes) << "\n";
     } else if (what == "both") {   // routed rows without a list beside a dense group: refused before any GPU call
       alignas(256) static unsigned char memory[1 << 16];
       const float* f = (const float*)memory;

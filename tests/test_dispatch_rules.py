@@ -54,6 +54,25 @@ def test_lists_are_cut_for_the_kernels_that_read_them(ask):
                rows(672, *both, E=256, most=84, dense=(84, 16, 28))) == ["32", "128", "32"]
 
 
+def test_tall_tiles_are_for_even_groups_of_short_k_in_few_rounds(ask):
+    """320 rows where the largest of even groups have more rows than whole full tiles and no more than whole tall ones."""
+    from tests.test_gpu_variants import TALL, test_tall_tiles_give_the_bits_of_full_ones as tall
+
+    def rows(R, E, D, I, dense=(0, 0, 0)):
+        return ("tile_rows", R, E, R, I // 128, -(-D // 256), D // 128, I // 128, *dense)
+    cases, = [m.args[1] for m in tall.pytestmark if m.name == "parametrize"]
+    E, D, I = TALL.values()
+    assert ask(*[rows(sum(c[i % len(c)] for i in range(E)), E, D, I) for c in cases]) == ["320"] * len(cases)
+    assert ask(*[("voted", E, *(c[i % len(c)] for i in range(E))) for c in cases]) == ["320", "320", "320", "288", "288", "320"]
+    even = {3500: "288", 3840: "288", 3860: "320", 4096: "320", 4400: "320", 4600: "288", 8000: "288", 8192: "320", 20000: "288"}
+    assert ask(*[rows(8 * M, 128, 2048, 768) for M in even]) == list(even.values())
+    # long K (twice), a dense group beside, more rounds
+    assert ask(rows(65536, 256, 7168, 2048), rows(32768, 128, 2176, 768), rows(32768, 128, 2048, 768, (4096, 6, 8)),
+               rows(131072, 512, 2048, 1024)) == ["288"] * 4
+    # a list of one GEMM has none
+    assert ask(("tile_rows", 32768, 128, 32768, 6, 0, 16, 0, 0, 0, 0), ("tile_rows", 32768, 128, 32768, 0, 8, 0, 6, 0, 0, 0)) == ["288", "288"]
+
+
 def test_few_tokens_go_straight_to_their_experts_where_that_is_cheaper(ask):
     """By the weights read, those read again, and the second launch's chain: not a wide shared expert beside small routed
     ones, nor sixteen tokens that all read the same few experts."""

@@ -644,3 +644,37 @@ def test_partial_sums_of_wide_routers(jg, M, D, E):
     idx, w = jg.moe_routing(x, gate, 7)
     want_idx, want_w = jg.route_softmax_topk(jg.router_logits(x, gate), 7)
     assert torch.equal(idx.reshape(M, 7), want_idx) and torch.equal(w.reshape(M, 7), want_w.to(w.dtype))
+
+
+TALL = dict(E=96, D=2048, I=1024)   # 8 column blocks and 16 or 8 K steps
+
+
+@pytest.mark.parametrize("sizes", [
+    [320, 289, 288, 200, 224, 225, 256, 240],     # one tile an expert, of 320 rows at most
+    [320, 289, 1, 319, 313, 304, 290, 270],       # ... and of all heights from 33 rows up to there
+    [320, 289, 0, 319, 313, 304, 290, 270],       # ... and none
+    [321, 289, 288, 200, 224, 225, 256, 240],     # one row too many: full tiles
+    [288, 287, 288, 224, 224, 225, 256, 240],     # ... no row too many
+    [640, 577, 576, 480, 449, 512, 500, 511],     # two tiles an expert
+])
+def test_tall_tiles_give_the_bits_of_full_ones(jg, sizes):
+    """Lists that may have tiles of 320 rows (what the host says of these batches: test_dispatch_rules.py) against the stage
+    functions, whose lists have none."""
+    import torch
+    print("tall tiles", sizes, flush=True)
+    E, D, I = TALL["E"], TALL["D"], TALL["I"]
+    rows = np.array([sizes[i % len(sizes)] for i in range(E)])
+    rng = np.random.default_rng(int(rows.sum()))
+    idx = rng.permutation(np.repeat(np.arange(E), rows)).astype(np.int32)[:, None]
+    M = len(idx)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M)
+    rand = lambda *s: torch.randn(s, dtype=torch.bfloat16, device="cuda", generator=gen)
+    ex = {n: jg.quantize_weight_block(rand(E, *s).mul_(0.02)) for n, s in (("gate_proj", (I, D)), ("up_proj", (I, D)), ("down_proj", (D, I)))}
+    x, w, didx = rand(M, D), torch.rand(M, 1, device="cuda", generator=gen), H.to_cuda(idx)
+    got = [jg.expert_forward_single(x, didx, w, *ex.values()) for _ in range(2)]
+    p = jg.permute(didx, E)
+    xq, sx = jg.quant_act(x)
+    hq, sh = jg.gemm_gateup_swiglu(xq, sx, ex["gate_proj"], ex["up_proj"], p["group_offsets"], row_ids=p["sorted_token_ids"])
+    want = jg.combine(jg.gemm_down(hq, sh, ex["down_proj"], p["group_offsets"]), w, p["inv_perm"])
+    assert torch.equal(got[0], want) and torch.equal(got[1], want)
