@@ -238,11 +238,14 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
   // carries its blocks instead (QuantJob: the two are independent; one launch less and they overlap).  Not where the
   // router reads what the quantiser writes.
   const bool quant_in_route = !fork && !quantiser_feeds_router(a, io_f32);
+  // A small router: norm, quantiser, router matmul and selection are one launch.
+  const int n_cols = a->E + (a->w_shared_gate ? 1 : 0);
+  const bool front = !fork && a->w_router && !given_idx && MOE_ALIGNED16(a->norm_weight) && moe_front_takes(a->M, a->D, a->E, n_cols);
   // A few tokens behind an RMSNorm: norm, quantiser and router matmul are one launch, below.
-  const bool norm_router = !fork && !sx_blocked && a->norm_weight && a->w_router && !given_idx &&
-                           moe_norm_router_takes(a->M, a->D, a->E + (a->w_shared_gate ? 1 : 0), io_f32);
+  const bool norm_router = !front && !fork && !sx_blocked && a->norm_weight && a->w_router && !given_idx &&
+                           moe_norm_router_takes(a->M, a->D, n_cols, io_f32);
   QuantJob quant_job{};
-  if (norm_router) {
+  if (norm_router || front) {
   } else if (quant_in_route) {
     if ((rc = moe_quant_act_job(a->x, io_f32, nullptr, a->M, a->D, b.xq, b.sx, sx_blocked, &quant_job))) return rc;
   } else if (!fork) {
@@ -274,27 +277,34 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
   // are written only when out_logits asks for them.
   LogitSource src{a->logits, nullptr, 0, a->E, nullptr, nullptr};
   const float* shared_gate = nullptr;
-  if (a->w_router && !given_idx) {
+  float* gate_out = a->out_shared_gate ? a->out_shared_gate : b.shared_gate;   // (written by the routing kernel)
+  if (a->w_shared_gate && !given_idx) shared_gate = gate_out;
+  if (front) {
+    src = LogitSource{nullptr, nullptr, 0, n_cols, a->out_logits, gate_out};
+  } else if (a->w_router && !given_idx) {
     const bool from_quantiser = quantiser_feeds_router(a, io_f32);
     if (from_quantiser && !quant_joined) {   // (the quantiser was forked)
       if (rc_shared) return join(rc_shared);
       if ((rc = moe_check_hip(hipStreamWaitEvent(main_s, ev->quant, 0), "forward: quant join"))) return join(rc);
       quant_joined = true;
     }
-    int splits = 0, n_cols = 0;
+    int splits = 0, used_cols = 0;
     if (norm_router)
       rc = moe_norm_router_partials(a->x, io_f32, a->norm_weight, a->norm_eps, a->M, a->D, a->w_router, a->E, a->w_shared_gate,
-                                    b.xq, b.sx, b.router_ws, b.router_ws_bytes, &splits, &n_cols, stream);
+                                    b.xq, b.sx, b.router_ws, b.router_ws_bytes, &splits, &used_cols, stream);
     else
       rc = moe_router_partials(from_quantiser ? b.normed : a->x, a->M, a->D, a->w_router, a->E, a->w_shared_gate,
-                               b.router_ws, b.router_ws_bytes, &splits, &n_cols, stream);
+                               b.router_ws, b.router_ws_bytes, &splits, &used_cols, stream);
     if (rc) return join(rc);
-    float* gate_out = a->out_shared_gate ? a->out_shared_gate : b.shared_gate;   // (written by the routing kernel)
-    if (a->w_shared_gate) shared_gate = gate_out;
-    src = LogitSource{nullptr, (const float*)b.router_ws, splits, n_cols, a->out_logits, gate_out};
+    src = LogitSource{nullptr, (const float*)b.router_ws, splits, used_cols, a->out_logits, gate_out};
   }
   const RouteArgs route{src, a->bias, a->M, a->E, a->k, a->renorm, a->n_group, a->topk_group, a->routed_scale, idx, w_own};
-  const QuantJob* carried = quant_in_route ? &quant_job : nullptr;
+  const QuantJob* carried = quant_in_route && !front ? &quant_job : nullptr;
+  const FrontArgs front_args{a->x, io_f32, a->D, a->norm_weight, a->norm_eps, a->w_router, a->w_shared_gate, b.xq, b.sx, sx_blocked};
+  auto select = [&](const PermuteOut* sort) {
+    return front ? moe_front_impl(a->routing, route, front_args, sort, b.permute_ws, b.permute_ws_bytes, stream)
+                 : moe_route_impl(a->routing, route, carried, sort, b.permute_ws, b.permute_ws_bytes, stream);
+  };
   // A few tokens whose sort and rows nobody asks for: the experts straight from the selection.  (What the launches that this
   // leaves out would have refused is refused here.)
   const bool sorted_outputs = a->out_group_sizes || a->out_sorted_token_ids || a->out_inv_perm || a->out_hq || a->out_hsq || a->out_y || a->out_ys;
@@ -307,7 +317,7 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
     MOE_REQUIRE(MOE_ALIGNED16(a->out) && (!a->add_residual || MOE_ALIGNED16(a->x)), MOE_ERR_BAD_ALIGN,
                 "combine: pointers must be 16-byte aligned");
     if (given_idx) rc = carried ? moe_quant_act_impl(a->x, io_f32, nullptr, a->M, a->D, b.xq, b.sx, nullptr, stream) : MOE_OK;
-    else rc = moe_route_impl(a->routing, route, carried, nullptr, nullptr, 0, stream);
+    else rc = select(nullptr);
     if (rc) return rc;
     const TokenArgs tok{b.xq, b.sx, given_idx ? given_idx : idx, w,
                         TokenExperts{a->w_gate, a->w_up, a->w_down, a->sw_gate, a->sw_up, a->sw_down},
@@ -325,7 +335,7 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
                                (a->I < a->D ? a->I : a->D) / 128, b.gemm_ws, b.gemm_ws_bytes, &tiles))) return join(rc);
   const PermuteOut sort{gsz, b.group_offsets, stid, nullptr, inv, a->k, tiles};
   rc = given_idx ? moe_permute_impl(given_idx, a->M, a->k, a->E, sort, b.permute_ws, b.permute_ws_bytes, carried, stream)
-                 : moe_route_impl(a->routing, route, carried, &sort, b.permute_ws, b.permute_ws_bytes, stream);
+                 : select(&sort);
   if (rc) return join(rc);
   if (!quant_joined) {
     if (rc_shared) return join(rc_shared);

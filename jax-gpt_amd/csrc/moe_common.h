@@ -288,6 +288,7 @@ struct LogitSource {
 int moe_router_partials(const void* x_bf16, int M, int D, const void* w_router_bf16, int E,
                         const void* w_shared_gate_bf16, void* ws, size_t ws_bytes, int* splits_used, int* n_cols,
                         moe_stream_t stream);
+int moe_router_k_slice(int M, int N, int D);   // K elements of a slice
 // RMSNorm, activation quantiser (row-major scales) and router matmul in one launch, for the calls that it takes (N as above)
 bool moe_norm_router_takes(int M, int D, int N, int x_f32);
 int moe_norm_router_partials(const void* x, int x_f32, const float* weight, float eps, int M, int D, const void* w_router_bf16,
@@ -326,6 +327,20 @@ struct RouteArgs {
 };
 int moe_route_impl(int routing, const RouteArgs& a, const QuantJob* quant, const PermuteOut* sort, void* permute_ws,
                    size_t permute_ws_bytes, moe_stream_t stream);
+// The same behind the router's matmul, the quantiser and, with norm, the RMSNorm, all in its one launch (small routers; N: columns
+// with the shared expert's gate).  a.src: out_logits and shared_gate alone.
+struct FrontArgs {
+  const void* x;    // (M, D) bf16, or f32 (x_f32), which is rounded to bf16 first
+  int x_f32, D;
+  const float* norm;
+  float eps;
+  const void *w_router, *w_shared_gate;
+  uint8_t* xq;      // optional: codes, scales and the scales' (D / 128, M) copy
+  float *sx, *sx_blocked;
+};
+bool moe_front_takes(int M, int D, int E, int N);
+int moe_front_impl(int routing, RouteArgs a, const FrontArgs& f, const PermuteOut* sort, void* permute_ws, size_t permute_ws_bytes,
+                   moe_stream_t stream);
 // chunks of the flat list that get a histogram each, at most
 int moe_permute_max_chunks(int E);
 // the sort's second launch: chunk_hist [n_chunks][E]; or, n_chunks == 1 and chunk_hist null, all of it (quant: carried along)

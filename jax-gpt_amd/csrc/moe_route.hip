@@ -341,6 +341,170 @@ __global__ __launch_bounds__(1024) void route_kernel(const RouteArgs a, const Ro
   }
 }
 
+// ---- small routers: all that stands in front of the experts' GEMMs but the sort ----------------------------------
+//
+// RMSNorm, activation quantiser, router matmul and selection are four launches' worth of dependent work on few bytes: with a
+// router of up to 64 experts over a hidden size of up to 1024 a workgroup can read all of the router's weights itself (66 KB for
+// 33 columns of 1024, from L2), so each does the whole chain for its tokens: one launch, no partial sums in memory.
+//   Its eight waves take a row's pieces of eight values 64 at a time, square, normalise and quantise them and put them into LDS,
+// while the weights travel into registers; then wave w multiplies K block w of all rows (128 values, a quantisation group) with
+// up to five fragments of 16 columns, the blocks' products meet in LDS, and a wave selects a token's experts.  Sums, blocks and
+// instructions are those of rmsnorm_quant_kernel, router_gemm_kernel (where its K slices are 128 long) and route_kernel in their
+// order: the same bits.
+//   What bounds it: the launch's start and four trips through memory and LDS.  Against the launches that it replaces (us): mini
+// layer (33 columns of 1024), 1 token 5.5 / 7.5, 64 7.3 / 9.5, 4096 12.1 / 14.0; behind its norm 1 token 6.0 / 7.9, 200 7.5 /
+// 13.1, 1000 8.6 / 14.4; tiny (8 of 512), 100 tokens 4.0 / 7.8.  Sixteen tokens a workgroup at any size: 11.1 for 64 tokens, 13.6
+// for 200 behind the norm.  The limits on columns and hidden size are what a wave has registers and a workgroup waves for.
+constexpr int kFrontTokens = 16, kFrontWaves = 8, kFrontColumns = 80, kFrontD = 128 * kFrontWaves;
+struct FrontJob {
+  const void* x;
+  int x_f32, D, tokens;         // tokens of a workgroup: a power of two up to kFrontTokens
+  const float* norm;            // NORM
+  float eps;
+  const bf16_t *w, *w_extra;    // (E, D) and the shared expert's gate (1, D) or null
+  uint8_t* xq;                  // null: no quantisation
+  float *sx, *sx_blocked;
+  int32_t* chunk_hist;          // [workgroups][E] or null
+};
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+
+template <int KIND, bool NORM>
+__global__ __launch_bounds__(64 * kFrontWaves) void front_kernel(const RouteArgs a, const FrontJob f) {
+  extern __shared__ __attribute__((aligned(16))) int lds[];   // [rows' pieces][the K blocks' products][logits][E counts]
+  constexpr int GROUPS = kFrontColumns / 16, UNITS = kFrontTokens * (kFrontD / 512) / kFrontWaves;
+  __shared__ float wave_sum[kFrontTokens][kFrontD / 512];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fr = lane & 15, fq = lane >> 4;
+  const int N = a.src.N, E = a.E, D = f.D, KB = D / 128, P = D / 8, T = f.tokens;
+  const int t0 = blockIdx.x * T;
+  v4i* pieces = (v4i*)lds;   // piece p of row r at p ^ (r & 7)
+  float* products = (float*)(pieces + T * P);
+  float* rows = products + KB * T * N;
+  int* hist = (int*)(rows + T * N);
+  // unit u: pieces [64 (u % per_row), +64) of row u / per_row; wave w has units w, w + 8, ...
+  const int per_row = P > 64 ? 2 : 1, units = T * per_row;
+  moe_bf16x8 in[UNITS] = {};
+  v4f wt[UNITS][2] = {};
+#pragma unroll
+  for (int i = 0; i < UNITS; ++i) {
+    const int u = w + kFrontWaves * i, p = (u & (per_row - 1)) * 64 + lane, t = t0 + (per_row == 2 ? u >> 1 : u);
+    if (u < units && p < P && t < a.M) {
+      in[i] = load_bf16x8(f.x, f.x_f32, (size_t)t * P + p);
+      if (NORM) wt[i][0] = ((const v4f*)f.norm)[2 * p], wt[i][1] = ((const v4f*)f.norm)[2 * p + 1];
+    }
+  }
+  v4i b[GROUPS][4];
+  if (w < KB) {
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) {
+      if (16 * g >= N) break;
+      const int n = min(16 * g + fr, N - 1);
+      const v4i* src = (const v4i*)((n < E ? f.w + (size_t)n * D : f.w_extra) + w * 128) + fq;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) b[g][s] = src[4 * s];
+    }
+  }
+  if (f.chunk_hist && tid < E) hist[tid] = 0;
+  if (NORM) {
+#pragma unroll
+    for (int i = 0; i < UNITS; ++i) {
+      const int u = w + kFrontWaves * i;
+      if (u >= units) break;
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float v = bf16_to_f32(in[i].v[j]);
+        ss = __fadd_rn(ss, __fmul_rn(v, v));
+      }
+      ss = wave_sum_f32(ss);
+      if (lane == 0) wave_sum[per_row == 2 ? u >> 1 : u][u & (per_row - 1)] = ss;
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < UNITS; ++i) {
+    const int u = w + kFrontWaves * i;
+    if (u >= units) break;
+    const int p = (u & (per_row - 1)) * 64 + lane, r = per_row == 2 ? u >> 1 : u;
+    if (NORM) {
+      const float total = per_row == 2 ? __fadd_rn(wave_sum[r][0], wave_sum[r][1]) : wave_sum[r][0];
+      const float rms = __fsqrt_rn(__fadd_rn(__fdiv_rn(total, (float)D), f.eps));
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        in[i].v[j] = f32_to_bf16(__fmul_rn(__fdiv_rn(bf16_to_f32(in[i].v[j]), rms), __fadd_rn(1.0f, wt[i][j / 4][j % 4])));
+    }
+    if (p < P) pieces[r * P + (p ^ (r & 7))] = __builtin_bit_cast(v4i, in[i]);
+  }
+  __syncthreads();
+  if (w < KB) {
+    v4f acc[GROUPS] = {};
+    v4i av[4];
+    const int r = fr & (T - 1);   // (rows beyond the tile's: any)
+#pragma unroll
+    for (int s = 0; s < 4; ++s) av[s] = pieces[r * P + ((w * 16 + 4 * s + fq) ^ (r & 7))];
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) {
+      if (16 * g >= N) break;
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av[s]), __builtin_bit_cast(bf16x8_t, b[g][s]), acc[g], 0, 0, 0);
+      const int n = 16 * g + fr;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (4 * fq + j < T && n < N) products[(w * T + 4 * fq + j) * N + n] = acc[g][j];
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < T * N; i += 64 * kFrontWaves) {
+    float s = products[i];
+    for (int kb = 1; kb < KB; ++kb) s = __fadd_rn(s, products[kb * T * N + i]);
+    rows[i] = bf16_to_f32(f32_to_bf16(s));
+  }
+  __syncthreads();
+  for (int tt = w; tt < min(T, a.M - t0); tt += kFrontWaves) {
+    const float* row = rows + tt * N;
+    if (a.src.out_logits && lane < E) a.src.out_logits[(size_t)(t0 + tt) * E + lane] = row[lane];
+    if (lane == 0 && a.src.shared_gate && N > E) a.src.shared_gate[t0 + tt] = bf16_to_f32(f32_to_bf16(sigmoid_det(row[E])));
+    const int chosen = KIND == ROUTE_SOFTMAX ? route_softmax_token<1>(a, row, t0 + tt) : route_grouped_token<1>(a, row, t0 + tt);
+    if (f.chunk_hist && lane < a.k) atomicAdd(&hist[chosen], 1);
+  }
+  if (f.xq) {   // (nobody in this launch waits for the codes)
+#pragma unroll
+    for (int i = 0; i < UNITS; ++i) {
+      const int u = w + kFrontWaves * i;
+      if (u >= units) break;
+      const int p = (u & (per_row - 1)) * 64 + lane, t = t0 + (per_row == 2 ? u >> 1 : u);
+      float v[8], amax = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        v[j] = bf16_to_f32(in[i].v[j]);
+        amax = fmaxf(amax, fabsf(v[j]));
+      }
+      unsigned m = __float_as_uint(amax);   // (not negative: ordered as integers; lanes of one group of 16)
+      m = max(m, dpp<DPP_XOR1>(m));
+      m = max(m, dpp<DPP_XOR2>(m));
+      m = max(m, dpp<DPP_MIRROR8>(m));
+      m = max(m, dpp<DPP_MIRROR16>(m));
+      float scale, scale_inv;
+      fp8_scales(__uint_as_float(m), scale, scale_inv);
+      if (p < P && t < a.M) {
+        uint2 out;
+        out.x = pack4_e4m3(v[0] * scale, v[1] * scale, v[2] * scale, v[3] * scale);
+        out.y = pack4_e4m3(v[4] * scale, v[5] * scale, v[6] * scale, v[7] * scale);
+        ((uint2*)f.xq)[(size_t)t * P + p] = out;
+        if ((p & 15) == 0) {
+          f.sx[(size_t)t * KB + p / 16] = scale_inv;
+          if (f.sx_blocked) f.sx_blocked[(size_t)(p / 16) * a.M + t] = scale_inv;
+        }
+      }
+    }
+  }
+  if (f.chunk_hist) {
+    __syncthreads();
+    if (tid < E) f.chunk_hist[(size_t)blockIdx.x * E + tid] = hist[tid];
+  }
+}
+
 constexpr int kCUs = 256;
 
 int check_route_args(int routing, const RouteArgs& a) {
@@ -441,6 +605,42 @@ int moe_route_impl(int routing, const RouteArgs& a, const QuantJob* quant, const
   return moe_permute_place(a.idx, R, a.E, tpb * a.k, job.blocks, job.chunk_hist, o, nullptr, stream);
 }
 
+// Routers that front_kernel takes: where the K slices of the router's matmul are its K blocks (the same sums).
+bool moe_front_takes(int M, int D, int E, int N) {
+  return M >= 1 && E <= 64 && N <= kFrontColumns && D >= 128 && D <= kFrontD && D % 128 == 0 && moe_router_k_slice(M, N, D) == 128;
+}
+int moe_front_impl(int routing, RouteArgs a, const FrontArgs& f, const PermuteOut* sort, void* permute_ws, size_t permute_ws_bytes,
+                   moe_stream_t stream) {
+  const int N = a.E + (f.w_shared_gate ? 1 : 0);
+  MOE_REQUIRE(f.x && f.w_router && (!f.w_shared_gate || a.src.shared_gate) && (!f.xq || f.sx), MOE_ERR_NULL, "router: null pointer");
+  MOE_REQUIRE(MOE_ALIGNED16(f.x) && MOE_ALIGNED16(f.w_router) && MOE_ALIGNED16(f.w_shared_gate) && MOE_ALIGNED16(f.norm) && MOE_ALIGNED16(f.xq),
+              MOE_ERR_BAD_ALIGN, "router: pointers must be 16-byte aligned");
+  MOE_REQUIRE(moe_front_takes(a.M, f.D, a.E, N), MOE_ERR_BAD_SHAPE, "router: not a call for this launch (M=%d D=%d N=%d)", a.M, f.D, N);
+  a.src.logits = nullptr, a.src.partial = (const float*)f.w_router, a.src.splits = 1, a.src.N = N;   // (no logits are given, and none are in memory)
+  if (int rc = check_route_args(routing, a)) return rc;
+  MOE_REQUIRE(!sort || (permute_ws && permute_ws_bytes >= moe_permute_workspace_bytes(a.M, a.k, a.E)), MOE_ERR_WORKSPACE_TOO_SMALL,
+              "route: permutation workspace too small");
+  MOE_REQUIRE((long long)a.M * a.k < (1ll << 31), MOE_ERR_BAD_SHAPE, "route: M*k overflows int32");
+  // Tokens of a workgroup: one, or as many as it takes to have one workgroup a CU.
+  int tokens = 1;
+  while (tokens < kFrontTokens && tokens * kCUs < a.M) tokens *= 2;
+  const int R = a.M * a.k, blocks = (a.M + tokens - 1) / tokens, KB = f.D / 128;
+  const bool one_chunk = R <= kSmallRows, counts = sort && !one_chunk && blocks <= moe_permute_max_chunks(a.E);
+  const FrontJob job{f.x, f.x_f32, f.D, tokens, f.norm, f.eps, (const bf16_t*)f.w_router, (const bf16_t*)f.w_shared_gate, f.xq, f.sx, f.sx_blocked,
+                     counts ? (int32_t*)permute_ws : nullptr};
+  const size_t lds = (size_t)tokens * f.D * 2 + ((size_t)tokens * N * (KB + 1) + a.E) * sizeof(float);   // (at most 78 KB)
+  auto* kernel = routing == MOE_ROUTING_SOFTMAX ? (f.norm ? front_kernel<ROUTE_SOFTMAX, true> : front_kernel<ROUTE_SOFTMAX, false>)
+                                                : (f.norm ? front_kernel<ROUTE_GROUPED, true> : front_kernel<ROUTE_GROUPED, false>);
+  static std::atomic<unsigned long long> lds_raised[4] = {};
+  if (int rc = moe_raise_lds_limit((const void*)kernel, 80 * 1024, lds_raised[(routing == MOE_ROUTING_SOFTMAX ? 0 : 2) + (f.norm ? 1 : 0)])) return rc;
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kFrontWaves), lds, (hipStream_t)stream, a, job);
+  if (int rc = moe_check_hip(hipGetLastError(), "route launch")) return rc;
+  if (!sort) return MOE_OK;
+  if (one_chunk) return moe_permute_place(a.idx, R, a.E, kSmallRows, 1, nullptr, *sort, nullptr, stream);
+  if (!counts) return moe_permute_impl(a.idx, a.M, a.k, a.E, *sort, permute_ws, permute_ws_bytes, nullptr, stream);
+  return moe_permute_place(a.idx, R, a.E, tokens * a.k, blocks, (const int32_t*)permute_ws, *sort, nullptr, stream);
+}
+
 extern "C" int moe_route_softmax_topk(const float* logits, int M, int E, int k, int renorm,
                                       int32_t* idx, float* w, moe_stream_t stream) {
   const RouteArgs a{LogitSource{logits, nullptr, 0, E, nullptr, nullptr}, nullptr, M, E, k, renorm, 1, 1, 1.f, idx, w};
@@ -459,6 +659,15 @@ extern "C" int moe_route_sigmoid_grouped(const float* logits, const float* bias,
 extern "C" int moe_routing(const void* x_bf16, int M, int D, const void* w_router_bf16, int E, int k, int renorm, int32_t* idx,
                            float* w, void* ws, size_t ws_bytes, moe_stream_t stream) {
   int splits = 0, n_cols = 0;
+  if (moe_front_takes(M, D, E, E)) {
+    MOE_REQUIRE(ws, MOE_ERR_NULL, "router: null pointer");
+    MOE_REQUIRE(MOE_ALIGNED16(ws), MOE_ERR_BAD_ALIGN, "router: pointers must be 16-byte aligned");
+    MOE_REQUIRE(ws_bytes >= moe_router_workspace_bytes(M, D, E), MOE_ERR_WORKSPACE_TOO_SMALL, "router: workspace %zu < %zu", ws_bytes,
+                moe_router_workspace_bytes(M, D, E));
+    const RouteArgs a{LogitSource{}, nullptr, M, E, k, renorm, 1, 1, 1.f, idx, w};
+    return moe_front_impl(MOE_ROUTING_SOFTMAX, a, FrontArgs{x_bf16, 0, D, nullptr, 0.f, w_router_bf16, nullptr, nullptr, nullptr, nullptr}, nullptr,
+                          nullptr, 0, stream);
+  }
   if (int rc = moe_router_partials(x_bf16, M, D, w_router_bf16, E, nullptr, ws, ws_bytes, &splits, &n_cols, stream)) return rc;
   const RouteArgs a{LogitSource{nullptr, (const float*)ws, splits, n_cols, nullptr, nullptr}, nullptr, M, E, k, renorm, 1, 1, 1.f, idx, w};
   return moe_route_impl(MOE_ROUTING_SOFTMAX, a, nullptr, nullptr, nullptr, 0, stream);

@@ -306,6 +306,12 @@ int moe_router_partials(const void* x_bf16, int M, int D, const void* w_router_b
   return moe_check_hip(hipGetLastError(), "router launch");
 }
 
+int moe_router_k_slice(int M, int N, int D) {
+  int k_per_split = 0;
+  slices_used(M, N, D, &k_per_split);
+  return k_per_split;
+}
+
 // Few tokens whose K slices are one quantisation group each (rows of up to 8192, as for the RMSNorm launch).
 bool moe_norm_router_takes(int M, int D, int N, int x_f32) {
   int k_per_split = 0;

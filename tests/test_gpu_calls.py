@@ -1,5 +1,7 @@
 """The layer calls' native way (csrc/moe_call.cpp) against the general one: the same bits where it takes a call, and nothing
 done where it does not."""
+import gc
+
 import numpy as np
 import pytest
 
@@ -38,7 +40,8 @@ def ways(jg, monkeypatch):
             if take:
                 taken = w.taken
         return out[0], out[1], taken
-    return both
+    yield both
+    gc.collect()   # (what the caught errors' frames still hold)
 
 
 def _weights(jg, E, D, I, gen, names=KEYS):

@@ -678,3 +678,49 @@ def test_tall_tiles_give_the_bits_of_full_ones(jg, sizes):
     hq, sh = jg.gemm_gateup_swiglu(xq, sx, ex["gate_proj"], ex["up_proj"], p["group_offsets"], row_ids=p["sorted_token_ids"])
     want = jg.combine(jg.gemm_down(hq, sh, ex["down_proj"], p["group_offsets"]), w, p["inv_perm"])
     assert torch.equal(got[0], want) and torch.equal(got[1], want)
+
+
+@pytest.mark.parametrize("M,D,E,SI,dtype,routing", [
+    (1, 1024, 64, 128, "bf16", "softmax"),        # the widest router: 65 columns
+    (3, 128, 1, 0, "f32", "softmax"),             # one K block, one expert
+    (17, 384, 33, 128, "f32", "softmax"),         # half a wave of pieces a row, two columns beyond two fragments
+    (256, 640, 16, 0, "bf16", "sigmoid_grouped"), # a wave and a quarter of pieces
+    (257, 1024, 8, 128, "bf16", "softmax"),       # two tokens a workgroup, the last one alone
+    (1025, 512, 40, 0, "bf16", "sigmoid_grouped"),   # eight, and selections counted for the sort
+    (2049, 896, 12, 128, "f32", "softmax"),       # sixteen, block-major scales
+    (4097, 256, 64, 0, "bf16", "softmax"),        # more workgroups than histograms
+])
+def test_small_routers_in_one_launch_give_the_bits_of_the_stages(jg, M, D, E, SI, dtype, routing):
+    import torch
+    print("one launch up to the selection", M, D, E, SI, dtype, routing, flush=True)
+    params, rand = _layer(jg, D, E, 128, SI, M + D)
+    names = ("gate_proj", "up_proj", "down_proj")
+    k = min(2, E)
+    kw = dict(routing=routing, n_group=4, topk_group=2, bias=rand(E).float() * 0.1, routed_scale=1.5) if routing != "softmax" else {}
+    experts, shared = {n: params[n] for n in names}, {n: params["shared_" + n] for n in names} if SI else None
+    x = rand(M, D).to(torch.float32 if dtype == "f32" else torch.bfloat16) * 3
+    x[M // 2] = 0                                            # an all-zero row
+    norm = rand(D).float() * 0.1
+    odd = torch.empty(D + 1, device="cuda")[1:]              # (read 16 bytes at a time: this one goes launch by launch)
+    odd.copy_(norm)
+    run = lambda norm, **o: jg.moe._forward(x, None, k, experts, shared=shared, gate_weight=params["gate_weight"], norm_weight=norm, io_f32=dtype == "f32",
+                                            shared_expert_gate_weight=params["shared_expert_gate_weight"] if SI else None, **kw, **o)
+    # with the norm: against the same call launch by launch
+    got, dbg = run(norm, add_residual=True, return_debug=True)
+    want, ref = run(odd, add_residual=True, return_debug=True)
+    for n in ref:
+        assert torch.equal(dbg[n], ref[n]), n
+    assert torch.equal(got, want) and torch.equal(run(norm, add_residual=True), want)
+    # without: against the stages
+    xb = x.bfloat16()
+    stage = jg.router_logits(xb, params["gate_weight"], params["shared_expert_gate_weight"] if SI else None)
+    logits, gate = stage if SI else (stage, None)
+    got, dbg = run(None, return_debug=True)
+    assert torch.equal(dbg["logits"], logits) and (not SI or torch.equal(dbg["shared_gate"], gate))
+    idx, w = jg.route_softmax_topk(logits, k) if routing == "softmax" else jg.route_sigmoid_grouped(logits, kw["bias"], 4, 2, k, True, 1.5)
+    assert torch.equal(dbg["indices"], idx) and torch.equal(dbg["weights"], w)
+    assert torch.equal(got, run(None))
+    if not SI:
+        assert torch.equal(got.bfloat16(), jg.expert_forward_single(xb, idx, w, *experts.values()))
+    if routing == "softmax":
+        assert all(map(torch.equal, jg.moe_routing(xb, params["gate_weight"], k), (idx, w)))
