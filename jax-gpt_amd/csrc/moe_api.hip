@@ -329,8 +329,26 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
   // routing, the sort by expert and the routed GEMMs' work list (the sort holds every expert's row range anyway)
   TileList tiles;
   const bool together = a->SI && !fork;   // the shared expert runs inside the routed launches
-  const int tile_rows = moe_gemm_tile_rows(TileShape{R, a->E, a->M, {a->I / 128, (a->D + 255) / 256}, {a->D / 128, a->I / 128},
-                                                     together ? a->M : 0, {a->SI / 128, (a->D + 255) / 256}});
+  const TileShape shape{R, a->E, a->M, {a->I / 128, (a->D + 255) / 256}, {a->D / 128, a->I / 128},
+                        together ? a->M : 0, {a->SI / 128, (a->D + 255) / 256}};
+  const bool from_memory = moe_gemm_from_memory(((long long)a->E * a->I + (together ? a->SI : 0)) * a->D);
+  if (const int scan_rows = fork || sorted_outputs ? 0 : moe_gemm_scan_rows(shape, from_memory)) {
+    // a small layer's few rows: the GEMMs read the selection itself
+    const int32_t* ids = given_idx ? given_idx : idx;
+    if (given_idx) rc = carried ? moe_quant_act_impl(a->x, io_f32, nullptr, a->M, a->D, b.xq, b.sx, nullptr, stream) : MOE_OK;
+    else rc = select(nullptr);
+    if (rc) return rc;
+    const GemmScales sc = moe_row_major_scales(a->D, a->I);
+    const RoutedGemm gateup{{b.xq, b.sx, nullptr, a->w_gate, a->sw_gate, a->w_up, a->sw_up, a->D, a->I, hq, sh, sc},
+                            nullptr, a->E, R, nullptr, 0, scan_rows, 0, ids, a->k};
+    const RoutedGemm down{{hq, sh, nullptr, a->w_down, a->sw_down, nullptr, nullptr, a->I, a->D, y, nullptr, moe_row_major_scales(a->I, a->D)},
+                          nullptr, a->E, R, nullptr, 0, scan_rows, 0, ids, a->k};
+    if ((rc = moe_gemm_gateup_impl(&gateup, together ? &shared_gateup : nullptr, stream))) return rc;
+    if ((rc = moe_gemm_down_impl(&down, together ? &shared_down : nullptr, stream))) return rc;
+    return moe_combine_impl(y, w, ids, a->E, a->SI ? ys : nullptr, shared_gate, a->add_residual ? a->x : nullptr, io_f32, a->M, a->k, a->D,
+                            a->out, stream);
+  }
+  const int tile_rows = moe_gemm_tile_rows(shape);
   if ((rc = moe_gemm_tile_list(R, a->E, tile_rows, a->I / 128, (a->D + 255) / 256,
                                (a->I < a->D ? a->I : a->D) / 128, b.gemm_ws, b.gemm_ws_bytes, &tiles))) return join(rc);
   const PermuteOut sort{gsz, b.group_offsets, stid, nullptr, inv, a->k, tiles};
@@ -362,7 +380,7 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
   if ((rc = moe_gemm_gateup_impl(&routed_gateup, together ? &shared_gateup : nullptr, stream))) return join(rc);
   if ((rc = moe_gemm_down_impl(&routed_down, together ? &shared_down : nullptr, stream))) return join(rc);
   if ((rc = join(MOE_OK))) return rc;
-  return moe_combine_impl(y, w, inv, a->SI ? ys : nullptr, shared_gate, a->add_residual ? a->x : nullptr, io_f32, a->M, a->k,
+  return moe_combine_impl(y, w, inv, 0, a->SI ? ys : nullptr, shared_gate, a->add_residual ? a->x : nullptr, io_f32, a->M, a->k,
                           a->D, a->out, stream);
 }
 

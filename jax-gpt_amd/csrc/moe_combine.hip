@@ -15,7 +15,7 @@ typedef moe_bf16x8 bf16x8;
 constexpr int kMaxK = 32;
 
 __global__ __launch_bounds__(256) void combine_kernel(const bf16x8* __restrict__ y, const float* __restrict__ w,
-                                                     const int32_t* __restrict__ inv_perm,
+                                                     const int32_t* __restrict__ inv_perm, int E,
                                                      const bf16x8* __restrict__ shared,
                                                      const float* __restrict__ shared_gate,
                                                      const void* __restrict__ residual, int io_f32, int k, int D8,
@@ -24,7 +24,9 @@ __global__ __launch_bounds__(256) void combine_kernel(const bf16x8* __restrict__
   __shared__ float wt[kMaxK];
   const int t = blockIdx.x;
   if (threadIdx.x < k) {
-    pos[threadIdx.x] = inv_perm[(size_t)t * k + threadIdx.x];
+    const size_t at = (size_t)t * k + threadIdx.x;
+    const int p = inv_perm[at];
+    pos[threadIdx.x] = E == 0 ? p : (unsigned)p < (unsigned)E ? (int)at : -1;
     wt[threadIdx.x] = w[(size_t)t * k + threadIdx.x];
   }
   __syncthreads();
@@ -79,9 +81,9 @@ __global__ __launch_bounds__(256) void combine_kernel(const bf16x8* __restrict__
 extern "C" int moe_combine(const void* y_bf16, const float* w, const int32_t* inv_perm,
                            const void* shared_bf16, const float* shared_gate, const void* residual_bf16, int M,
                            int k, int D, void* out_bf16, moe_stream_t stream) {
-  return moe_combine_impl(y_bf16, w, inv_perm, shared_bf16, shared_gate, residual_bf16, 0, M, k, D, out_bf16, stream);
+  return moe_combine_impl(y_bf16, w, inv_perm, 0, shared_bf16, shared_gate, residual_bf16, 0, M, k, D, out_bf16, stream);
 }
-int moe_combine_impl(const void* y_bf16, const float* w, const int32_t* inv_perm, const void* shared_bf16, const float* shared_gate,
+int moe_combine_impl(const void* y_bf16, const float* w, const int32_t* inv_perm, int E, const void* shared_bf16, const float* shared_gate,
                      const void* residual, int io_f32, int M, int k, int D, void* out, moe_stream_t stream) {
   MOE_REQUIRE(M == 0 || (y_bf16 && w && inv_perm && out), MOE_ERR_NULL, "combine: null pointer");
   MOE_REQUIRE(M >= 0 && k >= 1 && k <= kMaxK && D > 0 && D % 8 == 0, MOE_ERR_BAD_SHAPE,
@@ -94,7 +96,7 @@ int moe_combine_impl(const void* y_bf16, const float* w, const int32_t* inv_perm
   // about four workgroups per CU at least: split the columns of a token when there are few tokens
   int split = 1;
   while (split < 8 && (long long)M * split < 1024 && (D / 8) / (split * 2) >= 64) split *= 2;
-  hipLaunchKernelGGL(combine_kernel, dim3(M, split), dim3(256), 0, (hipStream_t)stream, (const bf16x8*)y_bf16, w, inv_perm,
+  hipLaunchKernelGGL(combine_kernel, dim3(M, split), dim3(256), 0, (hipStream_t)stream, (const bf16x8*)y_bf16, w, inv_perm, E,
                      (const bf16x8*)shared_bf16, shared_gate, residual, io_f32, k, D / 8, out);
   return moe_check_hip(hipGetLastError(), "combine launch");
 }

@@ -369,7 +369,8 @@ int moe_quant_act_impl(const void* x, int x_f32, void* x_bf16, int R, int K, uin
 int moe_rmsnorm_quant_impl(const void* x, int x_f32, const float* weight, float eps, int M, int D, void* normed_bf16,
                            uint8_t* xq, float* sx, float* sx_blocked, moe_stream_t stream);
 // the combine with the residual and the output in bf16 or (io_f32) f32, the output rounded to bf16 either way
-int moe_combine_impl(const void* y_bf16, const float* w, const int32_t* inv_perm, const void* shared_bf16, const float* shared_gate,
+// (E > 0: inv_perm holds the selections, and y's rows stand where these do: none for a selection outside [0, E))
+int moe_combine_impl(const void* y_bf16, const float* w, const int32_t* inv_perm, int E, const void* shared_bf16, const float* shared_gate,
                      const void* residual, int io_f32, int M, int k, int D, void* out, moe_stream_t stream);
 // the whole sort; its first launch carries the quantisation, if any
 int moe_permute_impl(const int32_t* idx, int M, int k, int E, const PermuteOut& o, void* ws, size_t ws_bytes, const QuantJob* quant,
@@ -409,7 +410,11 @@ struct RoutedGemm {
   void* ws;
   size_t ws_bytes;
   int list_tile_rows, list_pool_tiles;   // of the list that is there already, or 0: none is
+  const int32_t* ids = nullptr;          // the selections (flat, k a token) where the launch reads them itself: no list,
+  int k = 0;                             // no group_offsets; rows of gate/up's activations are tokens, all others flat indices
 };
+// rows of a full tile of such launches, or 0: the GEMMs read a list
+int moe_gemm_scan_rows(const TileShape& t, bool from_memory);
 // one group of all rows (the shared expert): no list, no workspace
 struct DenseGemm {
   GemmOperands op;

@@ -233,12 +233,14 @@ template <int XF> constexpr bool epilogue_fits(int bytes) {
 }
 static_assert(epilogue_fits<9>(CLS_RING) && epilogue_fits<10>(TALL_LDS_BYTES), "the tallest tile's epilogue stages inside the LDS");
 
-template <int MODE, int XF, bool ONCE>
+// listed (LDS), row_div: with LISTED, row r of the tile is row listed[r] / row_div of the activations and listed[r] of the output.
+template <int MODE, int XF, bool ONCE, bool LISTED = false>
 __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const uint8_t* __restrict__ xq,
                                           const float* __restrict__ sx, const int32_t* __restrict__ row_ids,
                                           const uint8_t* __restrict__ w0, const float* __restrict__ sw0,
                                           const uint8_t* __restrict__ w1, const float* __restrict__ sw1, int K, int N,
-                                          void* __restrict__ out, float* __restrict__ out_scale, const GemmScales sc) {
+                                          void* __restrict__ out, float* __restrict__ out_scale, const GemmScales sc,
+                                          const int* listed = nullptr, int row_div = 1) {
   using C = Cls<XF, MODE, ONCE>;
   constexpr int BM = C::BM, HALF = C::HALF;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -270,8 +272,13 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
     const int grp = i * 4 + cv;
     const int r = grp * 8 + drow;                              // row within the activation tile
     const int piece = dchunk ^ ((r >> 1) & 7);
-    int g = item.row_start + min(r, item.row_count - 1);
-    if (row_ids) g = row_ids[g];
+    int g = min(r, item.row_count - 1);
+    if constexpr (LISTED) {
+      g = (int)((unsigned)listed[g] / (unsigned)row_div);
+    } else {
+      g += item.row_start;
+      if (row_ids) g = row_ids[g];
+    }
     xoff[i] = (unsigned)g * (unsigned)K + piece * 16;
   }
   // first of the 64 scale slots that this wave copies (a second copy, all four waves the same, where 256 are not all)
@@ -282,8 +289,13 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
     const int p = min(sbase(i) + lane, BM - 1);   // slots past the tile land in the pad
     const int q = p % HALF;
     const int r = 16 * (2 * (q % XF) + p / HALF) + q / XF;
-    int g = item.row_start + min(r, item.row_count - 1);
-    if (row_ids && !sc.in_listed) g = row_ids[g];
+    int g = min(r, item.row_count - 1);
+    if constexpr (LISTED) {
+      g = (int)((unsigned)listed[g] / (unsigned)row_div);
+    } else {
+      g += item.row_start;
+      if (row_ids && !sc.in_listed) g = row_ids[g];
+    }
     soff[i] = (unsigned)g * (unsigned)sc.in_row * 4u;
   }
   const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)lds);
@@ -569,7 +581,7 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
   else run(std::integral_constant<int, ROT1>{}, std::false_type{});
   __syncthreads();   // every wave is done reading the ring before the epilogue reuses LDS
 
-  item_epilogue<MODE, 4, XF, BM, 32, NT>(acc, item, xj * 16 + fr, wi, lds, N, out, out_scale, sc);
+  item_epilogue<MODE, 4, XF, BM, 32, NT, LISTED>(acc, item, xj * 16 + fr, wi, lds, N, out, out_scale, sc, listed);
 }
 
 // row tiles of an expert up to which its weight lines are marked non-temporal (grouped_gemm_kernel)
@@ -647,6 +659,103 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
   }
 #undef MOE_ITEM
 }
+
+// ---- a small layer's batch, straight from the selection ----------------------------------------------------------
+//
+// Up to 2048 selections of up to 64 experts are read and counted by every workgroup itself, while it would otherwise wait for the
+// list header, the list entry and the row ids one after the other: no sort and no list in front of the two GEMMs, and rows of h
+// and y stay where their selections stand (flat index token * k + slot).  The same items, classes and bits.
+//   What bounds these launches: their start (arguments, instruction lines, the selections from memory), then the items' streams as in
+// the class kernel.  A GEMM launch is 0.5 to 1.5 us longer than one that reads a list, the sort's launch of 3.5 to 6 us (and as much
+// on the host) is gone: tiny layer, 32 tokens 22.6 -> 20 us, 256 25 -> 21.5, 1000 31 -> 28; mini layer, 64 tokens 30 -> 26.5, its
+// sublayer 200 tokens 31.6 -> 27.9, 1000 39 -> 35; uneven routings alike.  The limits are what a lane an expert and four
+// selections a thread hold.
+constexpr int kScanRows = 2048, kScanExperts = 64, kScanTileRows = 128;
+constexpr int SCAN_OFF = 150016;   // LDS: [64] experts' rows, [8] waves' rows of the item's expert, [128] the tile's rows
+constexpr int scan_ring() { return cmax(cmax(Cls<1>::RING_BYTES, Cls<2>::RING_BYTES), cmax(Cls<3>::RING_BYTES, Cls<4>::RING_BYTES)); }
+static_assert(scan_ring() <= SCAN_OFF && kScanTileRows * 512 <= SCAN_OFF && SCAN_OFF + (kScanExperts + NWAVES + kScanTileRows) * 4 <= CLS_RING, "LDS");
+
+// The workgroup's item among those of the routed rows (false: none is left) and its rows in listed.  MOST: selections of a thread at
+// most.  (Few instructions count for more here than few cycles, as every line of them is fetched cold: counts by ballots of the
+// selections' bits, with no atomics and two barriers fewer, take 1 to 2 us longer.)
+template <int MOST>
+__device__ __forceinline__ bool scan_item(Item& item, int* experts, int* counts, int* listed, const int32_t* __restrict__ ids, int R, int E,
+                                          int tile_rows, int ncb, int index) {
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), xcd = index & 7;
+  const int f = w * MOST * 64 + lane;   // the wave's selections: a run of 64 MOST
+  int mine[MOST];
+#pragma unroll
+  for (int j = 0; j < MOST; ++j) mine[j] = f + 64 * j < R ? ids[f + 64 * j] : -1;
+  if (tid < kScanExperts) experts[tid] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < MOST; ++j)
+    if ((unsigned)mine[j] < (unsigned)E) atomicAdd(&experts[mine[j]], 1);   // (a selection out of range has no row)
+  __syncthreads();
+  const int rows = experts[lane], nt = moe_tile_count(rows, tile_rows), to = moe_wave_scan(nt);   // lane = expert
+  const int n_items = __builtin_amdgcn_readlane(to, 63) * ncb;
+  const int id = (int)((unsigned)(n_items * xcd) >> 3) + (index >> 3);
+  if (id >= (int)((unsigned)(n_items * (xcd + 1)) >> 3)) return false;   // (uniform)
+  const int tile = id / ncb, e = (int)__builtin_ctzll(__ballot(to > tile));
+  const int e_rows = __builtin_amdgcn_readlane(rows, e), e_tiles = __builtin_amdgcn_readlane(nt, e);
+  const int first = __builtin_amdgcn_readlane(to, e) - e_tiles;
+  int rt, t0;
+  expert_item(id - first * ncb, e_tiles, ncb, item.col_block, rt);
+  moe_tile_span(e_rows, e_tiles, rt, t0, item.row_count);
+  item.expert = e;
+  item.tiles = e_tiles;
+  item.row_start = 0;
+  unsigned long long here[MOST];
+  int count = 0;
+#pragma unroll
+  for (int j = 0; j < MOST; ++j) {
+    here[j] = __ballot(mine[j] == e);
+    count += __popcll(here[j]);
+  }
+  if (lane == 0) counts[w] = count;
+  __syncthreads();
+  int place = -t0;   // in the tile, of the wave's first row
+  for (int v = 0; v < w; ++v) place += counts[v];
+#pragma unroll
+  for (int j = 0; j < MOST; ++j) {
+    const int p = place + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(here[j] >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)here[j], 0u));
+    if (mine[j] == e && (unsigned)p < (unsigned)item.row_count) listed[p] = f + 64 * j;
+    place += __popcll(here[j]);
+  }
+  __syncthreads();
+  return true;
+}
+
+template <int MODE, bool DENSE, int MOST>
+__global__ __launch_bounds__(NT, 1) void scan_gemm_kernel(const GemmOperands routed, const int32_t* __restrict__ ids, int R, int E, int k,
+                                                         int tile_rows, const GemmOperands dense, int dense_rows, int dense_tiles,
+                                                         int dense_blocks) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  int* const experts = (int*)(lds + SCAN_OFF);
+  int* const counts = experts + kScanExperts;
+  int* const listed = counts + NWAVES;
+  const bool is_dense = DENSE && (int)blockIdx.x < dense_blocks;
+  const GemmOperands op = is_dense ? dense : routed;
+  const int ncb = MODE == MODE_GATEUP ? op.N / 128 : (op.N + 255) / 256;
+  Item item;
+  if (is_dense) {
+    if (!work_item<MODE, true>(item, lds, op.N, true, nullptr, nullptr, dense_rows, dense_tiles, dense_blocks)) return;
+    if ((int)threadIdx.x < item.row_count) listed[threadIdx.x] = item.row_start + threadIdx.x;
+    __syncthreads();
+  } else if (!scan_item<MOST>(item, experts, counts, listed, ids, R, E, tile_rows, ncb, (int)blockIdx.x - (DENSE ? dense_blocks : 0))) {
+    return;
+  }
+  const int div = MODE == MODE_GATEUP && !is_dense ? k : 1;
+#define MOE_ITEM(XF) item_body<MODE, XF, false, true>(item, lds, op.xq, op.sx, nullptr, op.w0, op.sw0, op.w1, op.sw1, op.K, op.N, op.out, op.out_scale, op.sc, listed, div)
+  switch ((__builtin_amdgcn_readfirstlane(item.row_count) + 31) >> 5) {
+    case 4: MOE_ITEM(4); break;
+    case 3: MOE_ITEM(3); break;
+    case 2: MOE_ITEM(2); break;
+    default: MOE_ITEM(1); break;
+  }
+#undef MOE_ITEM
+}
+
 int col_blocks(int mode, int N) { return mode == MODE_GATEUP ? N / 128 : (N + 255) / 256; }
 
 int max_tiles_for(int R, int E, int tile_rows) { return (int)(((long long)R + tile_rows - 1) / tile_rows + (E < R ? E : R)); }
@@ -729,6 +838,21 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
     dense_tiles = moe_tile_count(dense_rows, dense_tile_rows);
     dense_blocks = 8 * (((long long)dense_tiles * col_blocks(MODE, dense.N) + 7) / 8);
     grid = dense_blocks;
+  }
+  if (rt && rt->ids) {   // (moe_gemm_scan_rows)
+    if (int rc = check_operands(rt->op, rt->R, rt->E, MODE, what)) return rc;
+    routed = rt->op;
+    routed.sc.out_through = through(rt->R, rt->E, routed.N);
+    grid += 8 * (((long long)max_tiles_for(rt->R, rt->E, rt->list_tile_rows) * col_blocks(MODE, routed.N) + 7) / 8);
+    static std::atomic<unsigned long long> lds_raised[6] = {};
+    const int most = rt->R <= NT ? 0 : rt->R <= 2 * NT ? 1 : 2;
+    auto* kernel = most == 0 ? (dn ? scan_gemm_kernel<MODE, true, 1> : scan_gemm_kernel<MODE, false, 1>)
+                 : most == 1 ? (dn ? scan_gemm_kernel<MODE, true, 2> : scan_gemm_kernel<MODE, false, 2>)
+                             : (dn ? scan_gemm_kernel<MODE, true, kScanRows / NT> : scan_gemm_kernel<MODE, false, kScanRows / NT>);
+    if (int rc = moe_raise_lds_limit((const void*)kernel, CLS_LDS_BYTES, lds_raised[2 * most + (dn != nullptr)])) return rc;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(NT), CLS_LDS_BYTES, s, routed, rt->ids, rt->R, rt->E, rt->k, rt->list_tile_rows,
+                       dense, dense_rows, dense_tiles, (int)dense_blocks);
+    return moe_check_hip(hipGetLastError(), "gemm launch");
   }
   if (rt) {
     MOE_REQUIRE(rt->group_offsets && rt->ws, MOE_ERR_NULL, "%s: null pointer", what);
@@ -835,6 +959,21 @@ int moe_gemm_tile_rows(const TileShape& t) {
     if (best == 0 || time < best) best = time, best_u = u;
   }
   return 32 * best_u;
+}
+
+// Batches whose GEMMs read the selection themselves: few rows of few experts whose launches are ones of the class kernel with plain
+// weight copies and tiles of up to 128 rows (a list's tiles may be allowed more where hardly any expert will have so many).
+int moe_gemm_scan_rows(const TileShape& t, bool from_memory) {
+  if (t.R < 1 || t.R > kScanRows || t.E > kScanExperts || from_memory) return 0;
+  const int groups = t.E < t.R ? t.E : t.R, mean = (t.R + groups - 1) / groups;
+  int spread = 0;
+  while (spread * spread < 4 * mean) ++spread;
+  const int list_rows = moe_gemm_tile_rows(t), rows = list_rows < kScanTileRows ? list_rows : kScanTileRows;
+  if (rows < list_rows && mean + spread > kScanTileRows) return 0;
+  for (int g = 0; g < 2; ++g)
+    if (moe_gemm_streams(g == 0 ? MODE_GATEUP : MODE_DOWN, rows, (long long)groups * t.ncb[g] + (long long)moe_tile_count(t.dense_rows, rows) * t.dense_ncb[g]))
+      return 0;
+  return rows;
 }
 
 extern "C" size_t moe_gemm_workspace_bytes(int R, int E, int N_out) {

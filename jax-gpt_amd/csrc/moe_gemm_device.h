@@ -133,10 +133,13 @@ __device__ __forceinline__ bool work_item(Item& item, uint8_t* lds, int N, bool 
 // 0 .. NW / 2 - 1 gate, the others up) or {16 NW wi ..} (down); a lane holds, for weight fragment f and activation fragment j,
 // the weight rows (fragment base) + 4 * (lane / 16) + {0..3} of tile row j * ROW_STEP + row0.  All of the workgroup calls it,
 // done with the LDS that it stages in: gate/up a f32 maximum per weight group and 128 codes a row, down 256 bf16 a row.
-template <int MODE, int NW, int NF, int BM, int ROW_STEP, int THREADS>
+// LISTED: row r of the tile is row listed[r] of the output (in LDS behind what the staging takes).
+template <int MODE, int NW, int NF, int BM, int ROW_STEP, int THREADS, bool LISTED = false>
 __device__ __forceinline__ void item_epilogue(v4f (&acc)[NW][NF], const Item& item, int row0, int wi, uint8_t* lds, int N,
-                                              void* __restrict__ out, float* __restrict__ out_scale, const GemmScales& sc) {
+                                              void* __restrict__ out, float* __restrict__ out_scale, const GemmScales& sc,
+                                              const int* listed = nullptr) {
   const int tid = threadIdx.x, fq = (tid & 63) >> 4;
+  auto out_row = [&](int r) { return (size_t)(LISTED ? listed[r] : item.row_start + r); };
   if (MODE == MODE_GATEUP) {
     constexpr int NG = NW / 2, GROUPS = 8 / NG;
     float* amax_s = (float*)lds;                            // [GROUPS][BM rows]
@@ -179,7 +182,7 @@ __device__ __forceinline__ void item_epilogue(v4f (&acc)[NW][NF], const Item& it
         *(unsigned*)(tile + swz(xr, col >> 4) + (col & 15)) = q;
       }
       if (wi == 0 && fq == 0 && xr < item.row_count)
-        out_scale[(size_t)(item.row_start + xr) * sc.out_row + (size_t)item.col_block * sc.out_cb] = scale_inv;
+        out_scale[out_row(xr) * sc.out_row + (size_t)item.col_block * sc.out_cb] = scale_inv;
     }
     __syncthreads();
     const int ld_chunk = tid & 7, ld_row = tid >> 3;   // THREADS / 8 rows per pass
@@ -188,7 +191,7 @@ __device__ __forceinline__ void item_epilogue(v4f (&acc)[NW][NF], const Item& it
       const int r = ld_row + THREADS / 8 * i;
       if (r < item.row_count) {
         v4i v = *(const v4i*)(tile + swz(r, ld_chunk));
-        v4i* dst = (v4i*)(hq + (size_t)(item.row_start + r) * I + item.col_block * 128 + ld_chunk * 16);
+        v4i* dst = (v4i*)(hq + out_row(r) * I + item.col_block * 128 + ld_chunk * 16);
         store16(dst, v, sc.out_through);
       }
     }
@@ -219,7 +222,7 @@ __device__ __forceinline__ void item_epilogue(v4f (&acc)[NW][NF], const Item& it
       const int r = ld_row + THREADS / 32 * i;
       if (r < item.row_count && c32 * 8 < ncols) {
         v4i v = *(const v4i*)(tile + r * 512 + ((c32 ^ (r & 7)) << 4));
-        v4i* dst = (v4i*)(y + (size_t)(item.row_start + r) * N + wrow0 + c32 * 8);
+        v4i* dst = (v4i*)(y + out_row(r) * N + wrow0 + c32 * 8);
         store16(dst, v, through);
       }
     }

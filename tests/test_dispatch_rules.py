@@ -84,6 +84,17 @@ def test_few_tokens_go_straight_to_their_experts_where_that_is_cheaper(ask):
     assert ask(*[("token", *c) for c in left]) == ["0"] * len(left)
 
 
+def test_small_layers_read_the_selection_themselves(ask):
+    """Few rows of few experts from the caches, in tiles of up to 128 rows; not where a list's tiles are taller for a reason, nor
+    where the short-tile kernel takes the launch."""
+    from tests.test_gpu_variants import SCANNED
+    assert all(32 <= int(r) <= 128 for r in ask(*[("scan", *c[:6]) for c in SCANNED]))
+    assert ask(*[("token", *c[:6]) for c in SCANNED]) == ["0"] * len(SCANNED)
+    left = [(1025, 512, 8, 2, 1024, 0), (100, 512, 65, 2, 256, 0), (100, 4096, 32, 2, 2048, 0),   # rows, experts, weights from memory
+            (512, 4096, 2, 2, 4096, 0), (128, 1536, 64, 8, 256, 0)]                              # 512 rows an expert in tall tiles; 384 items of short ones
+    assert ask(*[("scan", *c) for c in left]) == ["0"] * len(left)
+
+
 def test_the_compared_batches_of_single_tokens_reach_what_they_are_for(ask):
     """The batches that test_gpu_variants.py compares with the grouped route take the other one, and among them are: a last
     workgroup of fewer tiles, one over two scale blocks, more slots than waves, waves that LDS limits, weights from memory."""

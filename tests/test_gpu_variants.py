@@ -724,3 +724,44 @@ def test_small_routers_in_one_launch_give_the_bits_of_the_stages(jg, M, D, E, SI
         assert torch.equal(got.bfloat16(), jg.expert_forward_single(xb, idx, w, *experts.values()))
     if routing == "softmax":
         assert all(map(torch.equal, jg.moe_routing(xb, params["gate_weight"], k), (idx, w)))
+
+
+SCANNED = [   # M, D, E, k, I, SI, offsets on the logits
+    (17, 128, 1, 1, 128, 0, 0),       # one expert, one K step
+    (33, 384, 8, 2, 256, 0, 0),       # a half-full last column block
+    (64, 512, 64, 1, 128, 128, 0),    # as many experts as lanes; a shared expert beside
+    (100, 640, 7, 3, 384, 0, 30),     # a few experts take all: several tiles each, experts without rows
+    (512, 512, 8, 2, 1024, 0, 1),     # two selections a thread
+    (1024, 256, 60, 2, 128, 0, 0),    # four: all that they hold
+    (385, 256, 8, 4, 128, 128, 1),    # the last of four in a few waves
+    (511, 1024, 32, 2, 512, 512, 2),  # uneven, with a shared expert in several tiles
+    (128, 256, 33, 8, 256, 128, 0),   # eight selections a token
+]
+
+
+@pytest.mark.parametrize("M,D,E,k,I,SI,offset", SCANNED)
+def test_small_layers_without_a_list_give_the_bits_of_the_sorted_rows(jg, M, D, E, k, I, SI, offset):
+    """Where the GEMMs read the selection themselves (test_dispatch_rules.py says that these batches do) against the call whose
+    sorted rows are asked for, which has a list."""
+    import torch
+    print("selection read by the GEMMs", M, D, E, k, I, SI, offset, flush=True)
+    params, rand = _layer(jg, D, E, I, SI, M + D)
+    names = ("gate_proj", "up_proj", "down_proj")
+    experts = {n: params[n] for n in names}
+    kw = dict(top_k=k, experts=experts, shared={n: params["shared_" + n] for n in names} if SI else None)
+    x, lg = rand(M, D), rand(M, E).float() + offset * rand(E).float()
+    want, dbg = jg.moe_experts(x, lg, return_debug=True, **kw)
+    for _ in range(2):
+        assert torch.equal(jg.moe_experts(x, lg, **kw), want)
+    if SI:
+        return
+    assert torch.equal(jg.expert_forward_single(x, dbg["indices"], dbg["weights"], *experts.values()), want)
+    # selections outside [0, E) have no row
+    idx = dbg["indices"].clone()
+    idx[::3, 0] = E
+    idx[1::4, -1] = -7
+    idx[2] = 1 << 30
+    keep = (idx >= 0) & (idx < E)
+    got = jg.expert_forward_single(x, idx, dbg["weights"], *experts.values())
+    same = jg.expert_forward_single(x, torch.where(keep, idx, 0), torch.where(keep, dbg["weights"], 0.0), *experts.values())
+    assert torch.equal(got, same) and not got[2].any()
