@@ -88,18 +88,19 @@ __global__ __launch_bounds__(256 * PIECES) void rmsnorm_quant_kernel(const void*
   }
 }
 
-// One workgroup per 128x128 block.  A lane takes 16 bytes of a row (8 bf16 or 4 f32), 16 or 32 neighbouring lanes a whole
-// row, so a wave's loads and stores are whole lines; the block stays in registers, packed, between the maximum and the
-// rounding.  HBM-bound: every byte is read once and written once, hence non-temporal.  16 x 2048 x 7168 bf16: 158 us as
-// 64 consecutive elements per thread, 118 us now (5.97 TB/s; without the hints 130 us).
-template <typename T>
-__global__ __launch_bounds__(256) void quant_weight_kernel(const T* __restrict__ w, int N, int K,
-                                                          uint8_t* __restrict__ wq, float* __restrict__ sw) {
-  constexpr int V = 16 / sizeof(T), kRowLanes = 128 / V, kStepRows = 256 / kRowLanes, kSteps = 128 / kStepRows;
-  __shared__ float red[4];
-  const int kb = blockIdx.x, nb = blockIdx.y, e = blockIdx.z;
-  const int row0 = threadIdx.x / kRowLanes, col = (threadIdx.x % kRowLanes) * V;
-  const size_t off = ((size_t)e * N + (size_t)nb * 128 + row0) * K + (size_t)kb * 128 + col;
+// One workgroup per 128x128 block, or for two of them side by side (WIDE).  A lane takes 16 bytes of a row (8 bf16 or 4 f32), 16 or
+// 32 neighbouring lanes a block's row, so a wave's loads and stores are whole lines; the blocks stay in registers, packed,
+// between the maximum and the rounding.  HBM-bound: every byte is read once and written once, hence non-temporal.  16 x 2048 x 7168
+// bf16: 158 us as 64 consecutive elements per thread, 118 us as a block a workgroup of four waves (5.97 TB/s; without the hints 130
+// us), 111 as two of sixteen (6.3); f32 191 and, with sixteen waves, 182 (6.5).  Which form where: moe_quant_weight_block.
+template <typename T, int WIDE, int THREADS>
+__global__ __launch_bounds__(THREADS) void quant_weight_kernel(const T* __restrict__ w, int N, int K,
+                                                              uint8_t* __restrict__ wq, float* __restrict__ sw) {
+  constexpr int V = 16 / sizeof(T), kBlockLanes = 128 / V, kRowLanes = WIDE * kBlockLanes, kStepRows = THREADS / kRowLanes, kSteps = 128 / kStepRows;
+  __shared__ float red[kStepRows][WIDE];
+  const int nb = blockIdx.y, e = blockIdx.z;
+  const int row0 = threadIdx.x / kRowLanes, lane = threadIdx.x % kRowLanes, block = lane / kBlockLanes, kb = blockIdx.x * WIDE + block;
+  const size_t off = ((size_t)e * N + (size_t)nb * 128 + row0) * K + (size_t)blockIdx.x * (WIDE * 128) + lane * V;
   const size_t step = (size_t)kStepRows * K;
   v4i raw[kSteps];
 #pragma unroll
@@ -114,10 +115,11 @@ __global__ __launch_bounds__(256) void quant_weight_kernel(const T* __restrict__
 #pragma unroll
     for (int j = 0; j < V; ++j) amax = fmaxf(amax, fabsf(value(i, j)));
 #pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, MOE_WAVE));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
+  for (int o = kBlockLanes / 2; o >= 1; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, MOE_WAVE));
+  if (lane % kBlockLanes == 0) red[row0][block] = amax;
   __syncthreads();
-  amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+#pragma unroll
+  for (int i = 0; i < kStepRows; ++i) amax = fmaxf(amax, red[i][block]);
   float scale, scale_inv;
   fp8_scales(amax, scale, scale_inv);
 #pragma unroll
@@ -129,7 +131,7 @@ __global__ __launch_bounds__(256) void quant_weight_kernel(const T* __restrict__
       out[q] = pack4_e4m3(value(i, 4 * q) * scale, value(i, 4 * q + 1) * scale, value(i, 4 * q + 2) * scale, value(i, 4 * q + 3) * scale);
     __builtin_nontemporal_store(out, (codes_t*)(wq + off + i * step));
   }
-  if (threadIdx.x == 0) sw[((size_t)e * (N / 128) + nb) * (K / 128) + kb] = scale_inv;
+  if (row0 == 0 && lane % kBlockLanes == 0) sw[((size_t)e * (N / 128) + nb) * (K / 128) + kb] = scale_inv;
 }
 
 }  // namespace
@@ -184,11 +186,21 @@ extern "C" int moe_quant_weight_block(const void* w, int src_is_f32, int E, int 
   MOE_REQUIRE(E >= 1 && N > 0 && K > 0 && N % 128 == 0 && K % 128 == 0 && E < 65536 && N / 128 < 65536,
               MOE_ERR_BAD_SHAPE, "quant_weight_block: N=%d and K=%d must be multiples of 128 (E=%d)", N, K, E);
   MOE_REQUIRE(MOE_ALIGNED16(w) && MOE_ALIGNED16(wq), MOE_ERR_BAD_ALIGN, "quant_weight_block: pointers must be 16-byte aligned");
-  dim3 grid(K / 128, N / 128, E);
-  if (src_is_f32)
-    hipLaunchKernelGGL(quant_weight_kernel<float>, grid, dim3(256), 0, (hipStream_t)stream, (const float*)w, N, K, wq, sw);
-  else
-    hipLaunchKernelGGL(quant_weight_kernel<bf16_t>, grid, dim3(256), 0, (hipStream_t)stream, (const bf16_t*)w, N, K, wq, sw);
+  // Large arrays take workgroups of sixteen waves, bf16 two blocks wide: 512 bytes of a row, as f32 rows are with one.  Weights and
+  // codes together in MB, us with one block and four waves / this way, other weights and codes each time:
+  //   bf16 96 18.9 / 19.1, 129 24.7 / 25.3, 144 26.8 / 27.1, 185 33.7 / 33.3, 208 36.1 / 35.3, 270 48.0 / 47.7, 336 58.9 / 56.4, 562
+  // 98.8 / 93.2, 672 119.2 / 111.4, 2352 429 / 389;
+  //   f32 160 29.3 / 30.8, 216 37.8 / 37.3, 320 56.6 / 56.9, 347 60.0 / 56.9, 450 75.4 / 74.8, 560 94.9 / 89.8, 957 167 / 154, 1120 191 / 182.
+  // Below, f32 is 1 to 4 % faster with eight waves.  Plain stores look 9 % better only while the same codes are written again and
+  // again and stay in the memory-side cache (672 MB: 107; into other memory each time 123).
+  const long long n = (long long)E * N * K;
+  auto launch = [&](auto* kernel, auto* src, int width, int threads) {
+    hipLaunchKernelGGL(kernel, dim3(K / (128 * width), N / 128, E), dim3(threads), 0, (hipStream_t)stream, src, N, K, wq, sw);
+  };
+  if (src_is_f32) n * 5 > (320ll << 20) ? launch(quant_weight_kernel<float, 1, 1024>, (const float*)w, 1, 1024)
+                                        : launch(quant_weight_kernel<float, 1, 512>, (const float*)w, 1, 512);
+  else n * 3 > (160ll << 20) && K % 256 == 0 ? launch(quant_weight_kernel<bf16_t, 2, 1024>, (const bf16_t*)w, 2, 1024)
+                                             : launch(quant_weight_kernel<bf16_t, 1, 256>, (const bf16_t*)w, 1, 256);
   return moe_check_hip(hipGetLastError(), "quant_weight_block launch");
 }
 

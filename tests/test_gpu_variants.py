@@ -765,3 +765,18 @@ def test_small_layers_without_a_list_give_the_bits_of_the_sorted_rows(jg, M, D, 
     got = jg.expert_forward_single(x, idx, dbg["weights"], *experts.values())
     same = jg.expert_forward_single(x, torch.where(keep, idx, 0), torch.where(keep, dbg["weights"], 0.0), *experts.values())
     assert torch.equal(got, same) and not got[2].any()
+
+
+@pytest.mark.parametrize("E,N,K,dtype", [(9, 2560, 2560, "bf16"), (9, 2560, 2688, "bf16"), (11, 2560, 2432, "f32")])   # two blocks wide; an odd number of blocks; sixteen waves
+def test_large_weight_arrays_give_the_bits_of_their_experts(jg, E, N, K, dtype):
+    import torch
+    print("weight quantiser", E, N, K, dtype, flush=True)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(K)
+    w = torch.randn(E, N, K, dtype=torch.bfloat16 if dtype == "bf16" else torch.float32, device="cuda", generator=gen)
+    w[0, :128, :256] = 0                                     # all-zero blocks
+    w[-1, -1, -1] = 1e30
+    whole = jg.quantize_weight_block(w)
+    for e in range(E):
+        one = jg.quantize_weight_block(w[e])
+        assert torch.equal(whole["w"][e].view(torch.uint8), one["w"].view(torch.uint8)) and torch.equal(whole["scale_inv"][e], one["scale_inv"]), e
