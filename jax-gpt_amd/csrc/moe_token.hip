@@ -13,17 +13,16 @@
 // columns of a token, one wave a slot, and adds the slots up itself: no y, no third launch.  Against the grouped route (us,
 // one token): DeepSeek-V3 layer 84 -> 76, Qwen3-MoE 28 -> 20, full layer behind its norm 57.5 -> 45, mini 31 -> 27, tiny
 // 23 -> 20; five tokens of Qwen3-MoE 46 -> 38.5, eight 55 -> 50.5; sixteen of the mini layer 34 -> 30.5, of tiny 23 -> 20.
-//   Rings of two K steps: more bytes in flight per wave lose or change nothing (one token of DeepSeek-V3: rings of 2 / 3 / 4 / 6
-// steps 75.6 / 76.8 / 78.1 / 88.2 in the first launch; in the second 2 / 3 are even -- four draws 74.4 to 75.2 / 74.4 to 75.4, 1
-// to 8 tokens of Qwen3-MoE 22.0 to 49.0 / 21.6 to 48.9, 1 and 16 of the mini layer 26.5 and 30.2 / 27.3 and 30.5 -- and 4 / 8 are
-// 7 and 23 % slower).  Workgroups of four waves in the first: 85.8, as 288 of them are uneven on 256 CUs.
+//   Rings of two stages, of one or two K steps each (launch_gateup, launch_down); more of them lose or change nothing (of one
+// K step, one token of DeepSeek-V3: rings of 2 / 3 / 4 / 6 75.6 / 76.8 / 78.1 / 88.2 in the first launch; in the second 2 / 3 are
+// even and 4 / 8 are 7 and 23 % slower).  Workgroups of four waves in the first: 85.8, as 288 of them are uneven on 256 CUs.
 #include "moe_token.h"
 
 namespace {
 
 constexpr int BK = 128;
 constexpr int COLS = 16;         // output columns of a wave
-constexpr int STAGES = 2;        // K steps of a wave's ring
+constexpr int STAGES = 2;        // of a wave's ring
 constexpr int DOWN_TILES = 16;   // most tiles of a workgroup of the second launch
 constexpr int kLds = 160 * 1024, kDownLds = kLds - 8192;   // (the second launch has 5.3 KB of static LDS)
 
@@ -34,33 +33,38 @@ template <int N> __device__ __forceinline__ void wait_copies() { asm volatile("s
 // one of 4096 31.2 for 32.3, but 3 tokens of D 7168, 2 of 24 experts of 512 beside one of 512 41.4 for 39.7 and 16 of D 2048
 // 31.6 for 30.7; the other sizes tried are even.
 // One wave's products of a row with tiles of FRAGS fragments of 16 weight rows, each fragment of a matrix of its own and the
-// tiles `stride` bytes apart: one stream of K steps through a ring, also from one tile to the next.
-// LDS: rows of 128 bytes, 16-byte chunk c of row r at c ^ ((r >> 1) & 7), as in the grouped kernels.
-template <int FRAGS, bool ONCE>
+// tiles `stride` bytes apart: one stream of stages of KS K steps (1 or 2) through a ring, also from one tile to the next.
+// LDS: rows of 128 KS bytes, 16-byte chunk c of row r at c ^ ((r >> 1) & 7), as in the grouped kernels, or at c ^ r in rows of 256.
+template <int FRAGS, bool ONCE, int KS>
 struct WaveRows {
-  const uint8_t* w[FRAGS];   // the next K step to copy
-  unsigned off[2];
+  static constexpr int OPS = 2 * KS, ROW = KS * BK, ROWS = 8 / KS;   // copies of a fragment and stage, bytes and rows of one
+  static constexpr int FRAG = 16 * ROW;
+  const uint8_t* w[FRAGS];   // the next stage to copy
+  unsigned off[OPS];
   unsigned lds;              // the ring's LDS address
-  int KB, left, to_copy, copy_kb, slot;
-  size_t next_tile;          // from a tile's last K step to the next one's first
+  int KB, left, to_copy, copy_kb, slot, KM;
+  size_t next_tile;          // from a tile's last stage to the next one's first
 
   __device__ __forceinline__ void start(const uint8_t* const (&rows)[FRAGS], int K, int tiles, size_t stride, unsigned ring) {
-    const int lane = threadIdx.x & 63, drow = lane >> 3, piece = (lane & 7) ^ (drow >> 1);
-    KB = K / BK, lds = ring, left = to_copy = tiles * KB, copy_kb = 0, slot = 0, next_tile = stride - (size_t)(K - BK);
+    const int lane = threadIdx.x & 63;
+    KB = K / BK, KM = KB / KS, lds = ring, left = to_copy = tiles * KM, copy_kb = 0, slot = 0, next_tile = stride - (size_t)(K - ROW);
 #pragma unroll
     for (int f = 0; f < FRAGS; ++f) w[f] = rows[f];
-    off[0] = (unsigned)drow * (unsigned)K + piece * 16;
-    off[1] = (unsigned)(drow + 8) * (unsigned)K + (piece ^ 4) * 16;
+#pragma unroll
+    for (int g = 0; g < OPS; ++g) {
+      const int r = g * ROWS + lane / (8 * KS), at = lane % (8 * KS);
+      off[g] = (unsigned)r * (unsigned)K + (at ^ (KS == 1 ? (r >> 1) & 7 : r)) * 16;
+    }
     for (int t = 0; t < STAGES && to_copy; ++t) copy(t);
   }
   __device__ __forceinline__ void copy(int to) {
-    const size_t step = ++copy_kb == KB ? next_tile : BK;
-    if (copy_kb == KB) copy_kb = 0;
+    const size_t step = ++copy_kb == KM ? next_tile : ROW;
+    if (copy_kb == KM) copy_kb = 0;
 #pragma unroll
     for (int f = 0; f < FRAGS; ++f) {
 #pragma unroll
-      for (int g = 0; g < 2; ++g) {
-        const unsigned dst = lds + (unsigned)(to * FRAGS + f) * (16 * BK) + g * 1024u;
+      for (int g = 0; g < OPS; ++g) {
+        const unsigned dst = lds + (unsigned)(to * FRAGS + f) * FRAG + g * 1024u;
         if (ONCE) dma16_nt(w[f], off[g], dst);
         else dma16(w[f], off[g], dst);
       }
@@ -72,41 +76,44 @@ struct WaveRows {
   template <class Scale>
   __device__ __forceinline__ void run(const uint8_t* ring, const uint8_t* codes, v4f (&acc)[FRAGS], const Scale& scale) {
     const int lane = threadIdx.x & 63, fr = lane & 15, fq = lane >> 4;
-    const int lane_off0 = fr * BK + ((fq ^ (fr >> 1)) << 4), lane_off1 = fr * BK + (((fq + 4) ^ (fr >> 1)) << 4);
-    for (int kb = 0; kb < KB; ++kb, --left) {
-      if (left > 1) wait_copies<2 * FRAGS>();     // the next step's copies may be under way
+    for (int km = 0; km < KM; ++km, --left) {
+      if (left > 1) wait_copies<OPS * FRAGS>();     // the next stage's copies may be under way
       else wait_copies<0>();
       static_assert(STAGES == 2, "");
-      v8i wf[FRAGS];
+      v8i wf[KS][FRAGS];
 #pragma unroll
-      for (int f = 0; f < FRAGS; ++f) {
-        const uint8_t* base = ring + (slot * FRAGS + f) * (16 * BK);
-        const v4i lo = *(const v4i*)(base + lane_off0), hi = *(const v4i*)(base + lane_off1);
-        wf[f] = (v8i){lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-      }
-      // all sixteen columns of the matrix instruction are this row: the lanes of a quarter read one address
-      const v4i lo = *(const v4i*)(codes + kb * BK + fq * 16), hi = *(const v4i*)(codes + kb * BK + 64 + fq * 16);
-      const v8i xf = (v8i){lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-      float c[FRAGS];
+      for (int i = 0; i < KS; ++i)
 #pragma unroll
-      for (int f = 0; f < FRAGS; ++f) c[f] = scale(kb, f);
+        for (int f = 0; f < FRAGS; ++f) {
+          const uint8_t* base = ring + (slot * FRAGS + f) * FRAG + fr * ROW;
+          const int x = KS == 1 ? fr >> 1 : fr;
+          const v4i lo = *(const v4i*)(base + (((8 * i + fq) ^ x) << 4)), hi = *(const v4i*)(base + (((8 * i + 4 + fq) ^ x) << 4));
+          wf[i][f] = (v8i){lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        }
       if (to_copy) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the fragments are in registers: the stage may be overwritten
         copy(slot);
       }
       slot = slot + 1 == STAGES ? 0 : slot + 1;
 #pragma unroll
-      for (int f = 0; f < FRAGS; ++f) {
-        const v4f p = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[f], xf, (v4f){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
-        acc[f] += p * c[f];
+      for (int i = 0; i < KS; ++i) {
+        const int kb = km * KS + i;
+        // all sixteen columns of the matrix instruction are this row: the lanes of a quarter read one address
+        const v4i lo = *(const v4i*)(codes + kb * BK + fq * 16), hi = *(const v4i*)(codes + kb * BK + 64 + fq * 16);
+        const v8i xf = (v8i){lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+        for (int f = 0; f < FRAGS; ++f) {
+          const v4f p = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[i][f], xf, (v4f){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+          acc[f] += p * scale(kb, f);
+        }
       }
     }
   }
 };
 
-__host__ __device__ constexpr int up_lds(int D) { return STAGES * 32 * BK + D + D / BK * 4 * 3; }
+__host__ __device__ constexpr int up_lds(int D, int ks = 1) { return STAGES * 32 * BK * ks + D + D / BK * 4 * 3; }
 
-template <bool ONCE>
+template <bool ONCE, int KS>
 __global__ __launch_bounds__(64) void token_gateup_kernel(const TokenArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int lane = threadIdx.x, t = blockIdx.y;
@@ -117,11 +124,11 @@ __global__ __launch_bounds__(64) void token_gateup_kernel(const TokenArgs a) {
   const int N = shared ? a.SI : a.I;
   const int e = __builtin_amdgcn_readfirstlane(shared ? 0 : a.idx[(size_t)t * a.k + slot]);
   if (!shared && (unsigned)e >= (unsigned)a.E) return;   // (an index out of range: the second launch leaves its row out)
-  uint8_t* codes = lds + STAGES * 32 * BK;
+  uint8_t* codes = lds + STAGES * 32 * BK * KS;
   float* sx = (float*)(codes + a.D);
   float* sw = sx + KB;   // [2][KB]
   const size_t row = ((size_t)e * N + col) * a.D;
-  WaveRows<2, ONCE> rows;
+  WaveRows<2, ONCE, KS> rows;
   rows.start({x.w_gate + row, x.w_up + row}, a.D, 1, 0, __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)lds));
   for (int i = lane; i < a.D / 16; i += 64) ((v4i*)codes)[i] = ((const v4i*)(a.xq + (size_t)t * a.D))[i];
   const size_t block = ((size_t)e * (N / BK) + col / BK) * KB;
@@ -143,13 +150,13 @@ __global__ __launch_bounds__(64) void token_gateup_kernel(const TokenArgs a) {
 }
 
 // LDS of a wave of the second launch: ring, codes and scales of its row, the weights' scales of its tiles
-__host__ __device__ constexpr int down_wave_lds(int I, int tiles) {
-  return STAGES * 16 * BK + I + ((tiles + 1) * (I / BK) * 4 + 15) / 16 * 16;
+__host__ __device__ constexpr int down_wave_lds(int I, int tiles, int ks = 1) {
+  return STAGES * 16 * BK * ks + I + ((tiles + 1) * (I / BK) * 4 + 15) / 16 * 16;
 }
 
 // A workgroup: `tiles` neighbouring tiles of 16 output columns of a token; a wave: a slot's row (several, if there are more
 // slots than waves; then tiles is 1).
-template <bool ONCE>
+template <bool ONCE, int KS>
 __global__ __launch_bounds__(1024) void token_down_kernel(const TokenArgs a, const int tiles) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   __shared__ float y[2][MOE_TOKEN_SLOTS][COLS];
@@ -157,8 +164,8 @@ __global__ __launch_bounds__(1024) void token_down_kernel(const TokenArgs a, con
   __shared__ float residual[DOWN_TILES * COLS];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
   const int t = blockIdx.y, first = blockIdx.x * tiles, count = min(tiles, a.D / COLS - first), slots = a.k + (a.SI > 0);
-  uint8_t* ring = lds + w * down_wave_lds(a.h_stride, tiles);
-  uint8_t* codes = ring + STAGES * 16 * BK;
+  uint8_t* ring = lds + w * down_wave_lds(a.h_stride, tiles, KS);
+  uint8_t* codes = ring + STAGES * 16 * BK * KS;
   float* sx = (float*)(codes + a.h_stride);
   float* sw = sx + a.h_stride / BK;   // [tile][kb]
   const unsigned ring_at = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)ring);
@@ -169,7 +176,7 @@ __global__ __launch_bounds__(1024) void token_down_kernel(const TokenArgs a, con
       for (int i = lane; i < count * COLS; i += 64)
         residual[i] = bf16_to_f32(a.io_f32 ? f32_to_bf16(((const float*)a.residual)[at + i]) : ((const bf16_t*)a.residual)[at + i]);
   }
-  WaveRows<1, ONCE> rows;
+  WaveRows<1, ONCE, KS> rows;
   int e = 0;   // (of the wave's only slot, where there are several tiles)
   for (int j = 0; j < count; ++j) {
     for (int slot = w; slot < slots; slot += waves) {
@@ -234,11 +241,19 @@ __global__ __launch_bounds__(1024) void token_down_kernel(const TokenArgs a, con
   }
 }
 
+// Two K steps a stage, 256 bytes of a row (us, one / two).  In the first launch from the caches, or while a CU has up to four
+// workgroups: one token of Qwen3-MoE 19.8 / 17.9 for the call, two 21.8 / 21.2; 8 of the mini layer 17.0 / 16.5; with more of them
+// from memory their rows get in each other's way: one of DeepSeek-V3 (1152 workgroups) 74.7 / 75.5, 6 of Qwen3-MoE 42.8 / 44.7.  In
+// the second one from the caches, or where a wave walks up to 24 K steps: 16 tokens of tiny 16.5 / 15.5, of the mini layer 21.5 /
+// 20.7, 6 of Qwen3-MoE 43.7 / 42.8, 8 50.8 / 50.5, 2 of the full layer 61.5 / 61.1; DeepSeek-V3 (32 steps) 74.5 / 74.7.
 int launch_gateup(const TokenArgs& a, bool from_memory, hipStream_t s) {
-  static std::atomic<unsigned long long> raised[2] = {};
-  auto* kernel = from_memory ? token_gateup_kernel<true> : token_gateup_kernel<false>;
-  if (int rc = moe_raise_lds_limit((const void*)kernel, kLds, raised[from_memory])) return rc;
-  hipLaunchKernelGGL(kernel, dim3((a.k * a.I + a.SI) / COLS, a.M), dim3(64), up_lds(a.D), s, a);
+  static std::atomic<unsigned long long> raised[4] = {};
+  const unsigned columns = (a.k * a.I + a.SI) / COLS;
+  const int pairs = a.D % (2 * BK) == 0 && up_lds(a.D, 2) <= kLds && (!from_memory || columns * a.M <= 1024);
+  auto* kernel = pairs ? (from_memory ? token_gateup_kernel<true, 2> : token_gateup_kernel<false, 2>)
+                       : (from_memory ? token_gateup_kernel<true, 1> : token_gateup_kernel<false, 1>);
+  if (int rc = moe_raise_lds_limit((const void*)kernel, kLds, raised[2 * pairs + from_memory])) return rc;
+  hipLaunchKernelGGL(kernel, dim3(columns, a.M), dim3(64), up_lds(a.D, 1 + pairs), s, a);
   return moe_check_hip(hipGetLastError(), "token gate/up launch");
 }
 
@@ -249,11 +264,16 @@ int down_tiles(int D, int M) {
   return tiles;
 }
 int launch_down(const TokenArgs& a, bool from_memory, hipStream_t s) {
-  static std::atomic<unsigned long long> raised[2] = {};
-  auto* kernel = from_memory ? token_down_kernel<true> : token_down_kernel<false>;
-  if (int rc = moe_raise_lds_limit((const void*)kernel, kDownLds, raised[from_memory])) return rc;
+  static std::atomic<unsigned long long> raised[4] = {};
   const TokenDownPlan p = moe_token_down_plan(a.M, a.D, a.k, a.I, a.SI);
-  hipLaunchKernelGGL(kernel, dim3((a.D / COLS + p.tiles - 1) / p.tiles, a.M), dim3(64 * p.waves), p.waves * p.wave_lds, s, a, p.tiles);
+  const int pair_lds = down_wave_lds(a.h_stride, p.tiles, 2);
+  const int pairs = a.I % (2 * BK) == 0 && a.SI % (2 * BK) == 0 && p.waves * pair_lds <= kDownLds &&
+                    (!from_memory || p.tiles * (a.h_stride / BK) <= 24);
+  auto* kernel = pairs ? (from_memory ? token_down_kernel<true, 2> : token_down_kernel<false, 2>)
+                       : (from_memory ? token_down_kernel<true, 1> : token_down_kernel<false, 1>);
+  if (int rc = moe_raise_lds_limit((const void*)kernel, kDownLds, raised[2 * pairs + from_memory])) return rc;
+  hipLaunchKernelGGL(kernel, dim3((a.D / COLS + p.tiles - 1) / p.tiles, a.M), dim3(64 * p.waves), p.waves * (pairs ? pair_lds : p.wave_lds), s,
+                     a, p.tiles);
   return moe_check_hip(hipGetLastError(), "token down launch");
 }
 

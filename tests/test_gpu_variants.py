@@ -780,3 +780,14 @@ def test_large_weight_arrays_give_the_bits_of_their_experts(jg, E, N, K, dtype):
     for e in range(E):
         one = jg.quantize_weight_block(w[e])
         assert torch.equal(whole["w"][e].view(torch.uint8), one["w"].view(torch.uint8)) and torch.equal(whole["scale_inv"][e], one["scale_inv"]), e
+
+
+@pytest.mark.parametrize("M,D,E,k,I,SI", [
+    (3, 256, 8, 2, 384, 0),         # pairs of K steps in the first launch, an odd number of them in the second
+    (2, 384, 8, 2, 256, 128),       # odd in the first, and in the second for the shared expert
+    (5, 512, 8, 2, 512, 256),       # pairs in both
+    (6, 2048, 128, 8, 768, 0),      # from memory: nine workgroups a CU in the first, 18 K steps a wave in the second
+    (1, 7168, 18, 8, 2048, 2048),   # 1152 workgroups, 32 K steps
+])
+def test_single_tokens_in_stages_of_one_and_two_k_steps(jg, M, D, E, k, I, SI):
+    test_experts_of_single_tokens_give_the_grouped_bits(jg, M, D, E, k, I, SI, False)
