@@ -118,8 +118,8 @@ __host__ __device__ inline void moe_tile_span(int rows, int nt, int t, int& star
 // as skewed as a biased router makes them, natural expert order leaves one XCD with up to a tenth more work than the
 // average, and the launch ends with its slowest XCD.  The experts are therefore ranked by size (in units of 32 rows)
 // and dealt to eight bins in snake order (0..7, 7..0, ...); the list holds bin after bin.
-// Called by every thread of a workgroup of 1024; thread e owns expert e (rows = nt = 0 where there is none); lds_a and lds_b
-// are int[1024] in LDS.  Returns the index of expert e's first tile and writes the list header.
+// Called by every thread of a workgroup of 1024, or of a single wave (WAVE: up to 64 experts); thread e owns expert e (rows = nt = 0
+// where there is none); lds_a and lds_b are an int a thread in LDS.  Returns the index of expert e's first tile and writes the list header.
 //
 // The header's XCD shares are cut by cost, not by count: a row tile of u 32-row units costs about 8 + u (measured:
 // 63 us for a 32-row tile of the gate/up GEMM against 112 us for a 256-row one, and the same ratio for the down
@@ -170,29 +170,56 @@ __device__ __forceinline__ void moe_scan_1024(int& a, int& b, int& all_a, int& a
   b = in_b - b + (wv ? __builtin_amdgcn_readlane(sum_b, (wv - 1) & 15) : 0);
   __syncthreads();   // (the wave totals may be overwritten)
 }
+// the same over the workgroup's threads: 1024, or (WAVE) one wave's
+template <bool WAVE> __device__ __forceinline__ void moe_scan_threads(int& a, int& b, int& all_a, int& all_b) {
+  if constexpr (!WAVE) return moe_scan_1024(a, b, all_a, all_b);
+  const int in_a = moe_wave_scan(a), in_b = moe_wave_scan(b);
+  all_a = __builtin_amdgcn_readlane(in_a, 63);
+  all_b = __builtin_amdgcn_readlane(in_b, 63);
+  a = in_a - a;
+  b = in_b - b;
+}
+template <bool WAVE = false>
 __device__ inline int moe_tile_first(int e, int rows, int nt, int* lds_a, int* lds_b, const TileList& l) {
+  constexpr int THREADS = WAVE ? MOE_WAVE : 1024;
   TileHeader* const hdr = l.hdr;
   const int max_tiles = l.max_tiles;
   __shared__ long long cut_q[9];
   __shared__ int tail_tiles[kWideTailRounds];   // tiles of the last, last but one, ... round of the ranking
-  // rank: largest class first, inside a class in any order (1023 = the largest class and everything above it)
-  const int cls = rows > 0 ? 1023 - min((rows + 31) >> 5, 1023) : 0;
-  lds_a[e] = 0;
+  // rank: largest class first, inside a class in any order (1023 units = the largest class and everything above it)
+  const int units = min((rows + 31) >> 5, 1023);
+  int rank, nz, all_tiles;   // nz: experts with rows
   if (e < kWideTailRounds) tail_tiles[e] = 0;
-  __syncthreads();
-  const int order = rows > 0 ? atomicAdd(&lds_a[cls], 1) : 0;
-  __syncthreads();
-  int before = lds_a[e], tiles_to = nt, nz, all_tiles;   // nz: experts with rows
-  moe_scan_1024(before, tiles_to, nz, all_tiles);
-  lds_b[e] = before;
-  __syncthreads();
-  const int rank = lds_b[cls] + order;
+  if constexpr (WAVE) {   // bit by bit, the lanes of larger and of equal classes
+    unsigned long long larger = 0, equal = __ballot(rows > 0);
+    nz = (int)__popcll(equal);
+    for (int b = 9; b >= 0; --b) {
+      const bool mine = units >> b & 1;
+      const unsigned long long set = __ballot(mine);
+      if (!mine) larger |= equal & set;
+      equal &= mine ? set : ~set;
+    }
+    rank = (int)(__popcll(larger) + __popcll(equal & ((1ull << e) - 1)));
+    all_tiles = __builtin_amdgcn_readlane(moe_wave_scan(nt), 63);
+    __syncthreads();
+  } else {
+    const int cls = rows > 0 ? 1023 - units : 0;
+    lds_a[e] = 0;
+    __syncthreads();
+    const int order = rows > 0 ? atomicAdd(&lds_a[cls], 1) : 0;
+    __syncthreads();
+    int before = lds_a[e], tiles_to = nt;
+    moe_scan_1024(before, tiles_to, nz, all_tiles);
+    lds_b[e] = before;
+    __syncthreads();
+    rank = lds_b[cls] + order;
+  }
   const int nr = (nz + 7) >> 3;   // rounds that hold a non-empty expert
   int tail = nr / 4 < kTailRounds ? nr / 4 : kTailRounds;   // (3 rounds = 24 experts over the 8 bins; 6 measured no better)
   int pool_most = max_tiles >> 4;
   const long long all_items = (long long)all_tiles * (l.ncb[0] ? l.ncb[0] : l.ncb[1]);
   const bool whole = all_items == 256 || all_items == 512;   // one or two full rounds: equal shares end together, draws do not
-  if (l.pool_tiles > pool_most && !whole && __syncthreads_or((long long)rows * nz > 2ll * l.rows)) {   // (an expert of twice the mean)
+  if (l.pool_tiles > pool_most && !whole && (WAVE ? __any((long long)rows * nz > 2ll * l.rows) : __syncthreads_or((long long)rows * nz > 2ll * l.rows))) {   // (an expert of twice the mean)
     tail = nr > kWideTailRounds ? kWideTailRounds : nr - 1;
     pool_most = l.pool_tiles;
   }
@@ -234,12 +261,12 @@ __device__ inline int moe_tile_first(int e, int rows, int nt, int* lds_a, int* l
   }
   __syncthreads();
   int tiles_before = lds_a[e], cost_before = lds_b[e], total, cost_all;
-  moe_scan_1024(tiles_before, cost_before, total, cost_all);
+  moe_scan_threads<WAVE>(tiles_before, cost_before, total, cost_all);
   lds_a[e] = tiles_before;
   lds_b[e] = cost_before;
   __syncthreads();
-  const int first = lds_a[at & 1023], mine_before = lds_b[at & 1023];
-  const int fixed_tiles = n_fixed < 1024 ? lds_a[n_fixed] : total;
+  const int first = lds_a[at & (THREADS - 1)], mine_before = lds_b[at & (THREADS - 1)];
+  const int fixed_tiles = n_fixed < THREADS ? lds_a[n_fixed] : total;
   // cut k sits where the cost of the fixed shares reaches k/8 of their whole: inside exactly one expert, whose
   // thread places it
   if (rows > 0 && at < n_fixed) {

@@ -75,9 +75,14 @@ constexpr int ROTC = 2;       // MFMA groups by which wave set 1 trails wave set
 // moe_tile_first); thread e owns expert e.  Up to 8 rows an expert the tiles cost alike: plain expert order and equal XCD
 // shares do, for 2.4 us less a launch (expert-parallel shard of 32 experts, 64 rows 178.3 -> 173.3 us, 256 rows 213 ->
 // 208; with 800 unevenly spread rows it would be 239 -> 269).
-__global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __restrict__ group_offsets, int E, int R, TileList l) {
-  __shared__ int s_rows[1024];
-  __shared__ int s_key[1024];
+// WAVE: up to 64 experts, in one wave, with no other waves to start and to wait for at every step (launch 8.3 -> 5.1 us at 32
+// experts; their shard, two lists a pass, 320 rows 212 -> 209.5 us, 800 227.5 -> 224.2, 2400 285.2 -> 283.8, 16384 even).  Not where
+// an expert's tiles are written by 64 threads.
+__host__ __device__ inline bool many_tiles_each(int E, int max_tiles) { return E <= 16 && max_tiles >= 24 * E; }
+template <bool WAVE>
+__global__ __launch_bounds__(WAVE ? MOE_WAVE : 1024) void build_tiles_kernel(const int32_t* __restrict__ group_offsets, int E, int R, TileList l) {
+  __shared__ int s_rows[WAVE ? MOE_WAVE : 1024];
+  __shared__ int s_key[WAVE ? MOE_WAVE : 1024];
   const int e = threadIdx.x;
   int start = 0, rows = 0;
   if (e < E) {
@@ -89,14 +94,14 @@ __global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __rest
   if (R <= 8 * E) {
     int unused = 0, all, unused_all;
     first = tiles;
-    moe_scan_1024(first, unused, all, unused_all);
+    moe_scan_threads<WAVE>(first, unused, all, unused_all);
     if (e == 0) moe_tile_even_shares(l.hdr, min(all, l.max_tiles), min(all, l.max_tiles));
   } else {
-    first = moe_tile_first(e, rows, tiles, s_rows, s_key, l);
+    first = moe_tile_first<WAVE>(e, rows, tiles, s_rows, s_key, l);
   }
   // An expert of many tiles is written by 64 threads, not by its own (4096 rows of a 512 x 512 down GEMM in 128 tiles: 18.5
   // -> 11.9 us); below some 24 tiles that costs more than it saves (0.2 us).
-  if (E <= 16 && l.max_tiles >= 24 * E) {
+  if (!WAVE && many_tiles_each(E, l.max_tiles)) {
     __shared__ TileEntry entry[16];
     if (e < E) entry[e] = TileEntry{e | tiles << 10, start, rows, first};
     __syncthreads();
@@ -875,8 +880,11 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
   }
   MOE_REQUIRE(grid < (1ll << 30), MOE_ERR_BAD_SHAPE, "%s: %lld work items exceed the grid limit", what, grid);
   if (grid == 0) return MOE_OK;
-  if (l.hdr && !rt->list_tile_rows)
-    hipLaunchKernelGGL(build_tiles_kernel, dim3(1), dim3(1024), 0, s, rt->group_offsets, rt->E, rt->R, l);
+  if (l.hdr && !rt->list_tile_rows) {
+    const bool wave = rt->E <= MOE_WAVE && !many_tiles_each(rt->E, l.max_tiles);
+    hipLaunchKernelGGL(wave ? build_tiles_kernel<true> : build_tiles_kernel<false>, dim3(1), dim3(wave ? MOE_WAVE : 1024), 0, s,
+                       rt->group_offsets, rt->E, rt->R, l);
+  }
   // Non-temporal weight copies gain a stream from memory 2 to 3 % (four experts of 7168 x 2048 among others, 1 row each:
   // 46.6 -> 45.4 us, 64 tokens of the DeepSeek-V3 layer 12 %) and cost
   //  - a third where the memory-side cache (256 MB) still holds the weights from the call before (the same four experts

@@ -791,3 +791,35 @@ def test_large_weight_arrays_give_the_bits_of_their_experts(jg, E, N, K, dtype):
 ])
 def test_single_tokens_in_stages_of_one_and_two_k_steps(jg, M, D, E, k, I, SI):
     test_experts_of_single_tokens_give_the_grouped_bits(jg, M, D, E, k, I, SI, False)
+
+
+@pytest.mark.parametrize("E", [1, 17, 63, 64])
+@pytest.mark.parametrize("rows", ["one", "few", "uneven", "alike", "large"])
+def test_work_lists_of_one_wave_lead_to_the_same_rows(jg, E, rows):
+    """Up to 64 experts are listed by one wave, 65 (the last ones without rows) by a workgroup: which item is whose differs, no
+    row's bits do."""
+    import torch
+    print("one-wave list", E, rows, flush=True)
+    D, I = 256, 128
+    rng = H.rng_for(E)
+    sizes = np.zeros(65, np.int64)
+    sizes[:E] = {"one": 0, "few": rng.integers(0, 9, E), "uneven": rng.zipf(1.5, E).clip(0, 900) - 1, "alike": 40, "large": 13}[rows]
+    if not sizes.any():
+        sizes[E - 1] = 1
+    if rows == "large":                 # beyond the last size class, 1023 x 32 rows
+        sizes[E // 2] = 33000
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(E)
+    rand = lambda *shape: torch.randn(*shape, dtype=torch.bfloat16, device="cuda", generator=gen)
+    w = [jg.quantize_weight_block(rand(65, n, k).mul_(0.05)) for n, k in ((I, D), (I, D), (D, I))]
+    xq, sx = jg.quant_act(rand(int(off[-1]), D))
+
+    def rows_of(n):
+        gate, up, down = ({"w": d["w"][:n].contiguous(), "scale_inv": d["scale_inv"][:n].contiguous()} for d in w)
+        o = H.to_cuda(off[:n + 1].copy())
+        hq, sh = jg.gemm_gateup_swiglu(xq, sx, gate, up, o)
+        return hq.view(torch.uint8), sh, jg.gemm_down(hq, sh, down, o)
+
+    for got, want in zip(rows_of(E), rows_of(65)):
+        assert torch.equal(got, want)
