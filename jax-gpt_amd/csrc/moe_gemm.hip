@@ -75,9 +75,9 @@ constexpr int ROTC = 2;       // MFMA groups by which wave set 1 trails wave set
 // moe_tile_first); thread e owns expert e.  Up to 8 rows an expert the tiles cost alike: plain expert order and equal XCD
 // shares do, for 2.4 us less a launch (expert-parallel shard of 32 experts, 64 rows 178.3 -> 173.3 us, 256 rows 213 ->
 // 208; with 800 unevenly spread rows it would be 239 -> 269).
-// WAVE: up to 64 experts, in one wave, with no other waves to start and to wait for at every step (32 experts with 16384
-// rows 8.3 -> 6.2 us a launch; 4.8 for 320 rows; their shard, two lists a pass, 320 rows 212 -> 209.5 us, 800 227.5 -> 224.2, 2400 285.2 -> 283.8, 16384 even).  Not where
-// an expert's tiles are written by 64 threads.
+// WAVE: up to 64 experts, in one wave, with no other waves to start and to wait for at every step (32 experts with 16384 rows 8.3 ->
+// 6.2 us a launch, 4.8 for 320 rows; their shard, two lists a pass, 320 rows 212 -> 209.5 us, 800 227.5 -> 224.2, 2400 285.2 ->
+// 283.8, 16384 even).  Not where an expert's tiles are written by 64 threads.
 __host__ __device__ inline bool many_tiles_each(int E, int max_tiles) { return E <= 16 && max_tiles >= 24 * E; }
 template <bool WAVE>
 __global__ __launch_bounds__(WAVE ? MOE_WAVE : 1024) void build_tiles_kernel(const int32_t* __restrict__ group_offsets, int E, int R, TileList l) {
