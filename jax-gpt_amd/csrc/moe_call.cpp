@@ -10,6 +10,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include <climits>
 
@@ -115,6 +116,10 @@ struct Inputs {
 };
 PyObject* run(Call& c, const Inputs& in) {
   MoeForwardArgs& a = c.a;
+  // (the caller's dict alone may hold these two, and router_weight runs Python code, which lets other threads at it)
+  Py_XINCREF(in.router);
+  Py_XINCREF(in.shared_router);
+  const THPObjectPtr router(in.router), shared_router(in.shared_router);
   const at::Tensor* x = usable(in.x, in.io_f32 ? at::kFloat : at::kBFloat16, in.rank);
   if (!x || modes_active()) return general_way();
   const int64_t rows = in.rank == 2 ? x->size(0) : x->size(0) * x->size(1), D = x->size(in.rank - 1);

@@ -1,0 +1,99 @@
+"""The native host work of the layer calls (csrc/moe_call.cpp) without a GPU: the module built to take CPU tensors, over a library
+that records what it is called with."""
+import ctypes as C
+import importlib.machinery
+import importlib.util
+import os
+import shutil
+import subprocess
+import weakref
+
+import pytest
+import torch
+
+from jax_gpt_amd import _lib
+from tests.test_gpu_calls import KEYS
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def module(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("needs a C++ compiler")
+    spec = importlib.util.spec_from_file_location("_call_build", os.path.join(ROOT, "jax-gpt_amd", "build.py"))
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    out = tmp_path_factory.mktemp("call")
+    source, so = str(out / "host.cpp"), str(out / "moe_call.so")
+    headers = [line for line in open(os.path.join(build.CSRC, "moe_call.cpp")) if line.startswith("#include <")]
+    with open(source, "w") as f:   # (torch's headers first: the substitution reaches the module's own text alone)
+        f.write("".join(headers) + f'#define is_cuda is_cpu\n#include "{os.path.join(build.CSRC, "moe_call.cpp")}"\n')
+    command = build._call_command()
+    command[command.index(os.path.join(build.CSRC, "moe_call.cpp"))] = source
+    command[command.index("-o") + 1] = so
+    subprocess.run(command, check=True)
+    loader = importlib.machinery.ExtensionFileLoader("moe_call", so)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("moe_call", so, loader=loader))
+    loader.exec_module(module)
+    return module
+
+
+class Library:
+    """The functions that moe_call is bound to.  Every forward call's arguments are appended to `calls`."""
+
+    def __init__(self, module, router_weight=None):
+        self.calls, self.codes = [], []
+        size = C.CFUNCTYPE(C.c_size_t, *[C.c_int] * 6)(lambda *a: 64)
+        forward = C.CFUNCTYPE(C.c_int, C.POINTER(_lib.MoeForwardArgs), C.c_void_p, C.c_size_t, C.c_void_p)(self._forward)
+        selected = C.CFUNCTYPE(C.c_int, C.POINTER(_lib.MoeForwardArgs), *[C.c_void_p] * 3, C.c_size_t, C.c_void_p)(self._forward)
+        router_size = C.CFUNCTYPE(C.c_size_t, *[C.c_int] * 3)(lambda *a: 64)
+        routing = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_int, C.c_int, C.c_void_p, *[C.c_int] * 3, *[C.c_void_p] * 3, C.c_size_t, C.c_void_p)(
+            lambda *a: self.calls.append(a) or 0)
+        self.bound = size, forward, forward, selected, router_size, routing
+        module.bind(*(C.cast(f, C.c_void_p).value for f in self.bound), self.codes.append, router_weight or self._router_weight,
+                    lambda: 0, lambda device: 0)
+
+    def _forward(self, args, *rest):
+        got = _lib.MoeForwardArgs()
+        C.pointer(got)[0] = args[0]
+        self.calls.append(got)
+        return 0
+
+    @staticmethod
+    def _router_weight(w, name):
+        return w.t().contiguous()
+
+
+def _layer_params(D=256, E=8, I=128, SI=256):
+    def fp8(e, n, k):
+        return dict(w=torch.zeros(e, n, k, dtype=torch.float8_e4m3fn), scale_inv=torch.ones(e, n // 128, k // 128))
+    p = dict(zip(KEYS, (fp8(E, I, D), fp8(E, I, D), fp8(E, D, I))))
+    p.update(zip(("shared_" + n for n in KEYS), (fp8(1, SI, D), fp8(1, SI, D), fp8(1, D, SI))))
+    p["gate_weight"] = torch.zeros(E, D, dtype=torch.bfloat16).t()
+    p["shared_expert_gate_weight"] = torch.zeros(1, D, dtype=torch.bfloat16).t()
+    return p
+
+
+def test_router_weights_outlive_their_dict_entries(module):
+    """Fetching the router weight runs Python code; the shared expert's gate, which the dict alone may hold and which comes next, has
+    to outlive what that code, or another thread meanwhile, does to the dict."""
+    p = _layer_params()
+    old = {n: weakref.ref(p[n]) for n in ("gate_weight", "shared_expert_gate_weight")}
+    seen = []
+
+    def fetch(w, name):
+        if name == "gate_weight":
+            for n in old:
+                p[n] = torch.ones_like(old[n]())
+            if old["shared_expert_gate_weight"]() is None:
+                raise RuntimeError("freed while the call still needs it")   # (so that the call does not go on to read it)
+        assert w is old[name]()
+        seen.append(name)
+        return w.t().contiguous()
+
+    lib = Library(module, fetch)
+    x = torch.zeros(1, 5, 256, dtype=torch.bfloat16)
+    assert module.layer(x, p, 2, None, 1e-6, 0).shape == x.shape
+    assert seen == list(old) and len(lib.calls) == 1 and lib.calls[0].w_shared_gate
+    assert all(r() is None for r in old.values())   # (nor are they kept)
