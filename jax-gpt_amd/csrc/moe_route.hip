@@ -621,6 +621,7 @@ int moe_front_impl(int routing, RouteArgs a, const FrontArgs& f, const PermuteOu
   MOE_REQUIRE(!sort || (permute_ws && permute_ws_bytes >= moe_permute_workspace_bytes(a.M, a.k, a.E)), MOE_ERR_WORKSPACE_TOO_SMALL,
               "route: permutation workspace too small");
   MOE_REQUIRE((long long)a.M * a.k < (1ll << 31), MOE_ERR_BAD_SHAPE, "route: M*k overflows int32");
+  MOE_REQUIRE((long long)a.M * f.D * 2 < (1ll << 32), MOE_ERR_BAD_SHAPE, "router: the activations must stay within 4 GB");   // (as moe_router_partials)
   // Tokens of a workgroup: one, or as many as it takes to have one workgroup a CU.
   int tokens = 1;
   while (tokens < kFrontTokens && tokens * kCUs < a.M) tokens *= 2;

@@ -49,6 +49,11 @@ int main() {
       const RoutedGemm routed{op, (const int32_t*)memory, 8, 64, memory, sizeof memory, 0, 0};
       const DenseGemm dense{op, 64};
       std::cout << moe_gemm_gateup_impl(&routed, &dense, nullptr) << " " << moe_gemm_down_impl(&routed, &dense, nullptr) << " " << moe_last_error() << "\n";
+    } else if (what == "routing") {   // tokens, D, experts: what moe_routing refuses before any GPU call
+      int M, D, E;
+      std::cin >> M >> D >> E;
+      alignas(256) static unsigned char memory[256];
+      std::cout << moe_routing(memory, M, D, memory, E, 1, 1, (int32_t*)memory, (float*)memory, memory, ~(size_t)0, nullptr) << " " << moe_last_error() << "\n";
     } else {
       return 1;
     }

@@ -116,3 +116,9 @@ def test_the_compared_batches_of_single_tokens_reach_what_they_are_for(ask):
 def test_a_dense_group_beside_routed_rows_needs_their_list(ask):
     """Cut on its own it could have taller tiles than the kernel that the routed list's height chooses."""
     assert ask(("both",))[0].startswith("-1 -1 gemm_down: a dense group")
+
+
+def test_routers_refuse_activations_beyond_4_gb_whatever_the_launch(ask):
+    """128 columns and 64 experts go to the launch that has everything in one, 65 experts to the matmul's own."""
+    for E in (64, 65):
+        assert ask(("routing", 1 << 24, 128, E))[0].startswith("-1 router: the activations must stay within 4 GB"), E
