@@ -240,7 +240,8 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
   const bool quant_in_route = !fork && !quantiser_feeds_router(a, io_f32);
   // A small router: norm, quantiser, router matmul and selection are one launch.
   const int n_cols = a->E + (a->w_shared_gate ? 1 : 0);
-  const bool front = !fork && a->w_router && !given_idx && MOE_ALIGNED16(a->norm_weight) && moe_front_takes(a->M, a->D, a->E, n_cols);
+  const bool front = !fork && a->w_router && !given_idx && MOE_ALIGNED16(a->norm_weight) &&
+                     moe_front_takes(a->M, a->D, a->E, n_cols, a->norm_weight, io_f32, true);
   // A few tokens behind an RMSNorm: norm, quantiser and router matmul are one launch, below.
   const bool norm_router = !front && !fork && !sx_blocked && a->norm_weight && a->w_router && !given_idx &&
                            moe_norm_router_takes(a->M, a->D, n_cols, io_f32);

@@ -365,7 +365,7 @@ struct FrontArgs {
   uint8_t* xq;      // optional: codes, scales and the scales' (D / 128, M) copy
   float *sx, *sx_blocked;
 };
-bool moe_front_takes(int M, int D, int E, int N);
+bool moe_front_takes(int M, int D, int E, int N, bool norm, bool x_f32, bool sorted);   // sorted: a sort of the selections follows
 int moe_front_impl(int routing, RouteArgs a, const FrontArgs& f, const PermuteOut* sort, void* permute_ws, size_t permute_ws_bytes,
                    moe_stream_t stream);
 // chunks of the flat list that get a histogram each, at most

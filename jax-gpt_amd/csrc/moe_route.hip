@@ -605,9 +605,17 @@ int moe_route_impl(int routing, const RouteArgs& a, const QuantJob* quant, const
   return moe_permute_place(a.idx, R, a.E, tpb * a.k, job.blocks, job.chunk_hist, o, nullptr, stream);
 }
 
-// Routers that front_kernel takes: where the K slices of the router's matmul are its K blocks (the same sums).
-bool moe_front_takes(int M, int D, int E, int N) {
-  return M >= 1 && E <= 64 && N <= kFrontColumns && D >= 128 && D <= kFrontD && D % 128 == 0 && moe_router_k_slice(M, N, D) == 128;
+// Routers that front_kernel takes: where the K slices of the router's matmul are its K blocks (the same sums), and one workgroup a CU
+// has all tokens (4096).  With more of them there are more workgroups than histograms, and the sort counts in a launch of its own.
+// Layers of 64 experts, launch by launch / this way (us; 4096 tokens of 1024 behind the norm: 65.8 / 60.5):
+//   behind the norm, 4600 of 1024 69.1 / 76.5, 5000 of 640 67.4 / 72.6, 8192 of 512 66.5 / 64.1, 12000 of 256 67.1 / 66.4, 20000 of
+// 128 84.0 / 86.1, 65536 of it 189 / 218;
+//   without it, 4600 of 1024 60.4 / 62.7, 5000 of 640 58.8 / 59.7, 8192 of 512 58.5 / 57.6, 32000 of 256 101.0 / 96.5; from f32,
+// which else needs its rounding stored, 5000 of 640 69.7 / 66.8, 4097 of 1024 72.2 / 66.4;
+//   the routing alone, 4600 of 1024 15.1 / 13.1, 32000 of 256 28.5 / 24.1, 65536 of 128 42.1 / 39.8, 262144 132 / 157.
+bool moe_front_takes(int M, int D, int E, int N, bool norm, bool x_f32, bool sorted) {
+  if (M < 1 || E > 64 || N > kFrontColumns || D < 128 || D > kFrontD || D % 128 || moe_router_k_slice(M, N, D) != 128) return false;
+  return M <= kFrontTokens * kCUs || (M <= 32768 && !norm && (!sorted || x_f32 || D <= 512));
 }
 int moe_front_impl(int routing, RouteArgs a, const FrontArgs& f, const PermuteOut* sort, void* permute_ws, size_t permute_ws_bytes,
                    moe_stream_t stream) {
@@ -615,7 +623,7 @@ int moe_front_impl(int routing, RouteArgs a, const FrontArgs& f, const PermuteOu
   MOE_REQUIRE(f.x && f.w_router && (!f.w_shared_gate || a.src.shared_gate) && (!f.xq || f.sx), MOE_ERR_NULL, "router: null pointer");
   MOE_REQUIRE(MOE_ALIGNED16(f.x) && MOE_ALIGNED16(f.w_router) && MOE_ALIGNED16(f.w_shared_gate) && MOE_ALIGNED16(f.norm) && MOE_ALIGNED16(f.xq),
               MOE_ERR_BAD_ALIGN, "router: pointers must be 16-byte aligned");
-  MOE_REQUIRE(moe_front_takes(a.M, f.D, a.E, N), MOE_ERR_BAD_SHAPE, "router: not a call for this launch (M=%d D=%d N=%d)", a.M, f.D, N);
+  MOE_REQUIRE(moe_front_takes(a.M, f.D, a.E, N, f.norm, f.x_f32, sort), MOE_ERR_BAD_SHAPE, "router: not a call for this launch (M=%d D=%d N=%d)", a.M, f.D, N);
   a.src.logits = nullptr, a.src.partial = (const float*)f.w_router, a.src.splits = 1, a.src.N = N;   // (no logits are given, and none are in memory)
   if (int rc = check_route_args(routing, a)) return rc;
   MOE_REQUIRE(!sort || (permute_ws && permute_ws_bytes >= moe_permute_workspace_bytes(a.M, a.k, a.E)), MOE_ERR_WORKSPACE_TOO_SMALL,
@@ -660,7 +668,7 @@ extern "C" int moe_route_sigmoid_grouped(const float* logits, const float* bias,
 extern "C" int moe_routing(const void* x_bf16, int M, int D, const void* w_router_bf16, int E, int k, int renorm, int32_t* idx,
                            float* w, void* ws, size_t ws_bytes, moe_stream_t stream) {
   int splits = 0, n_cols = 0;
-  if (moe_front_takes(M, D, E, E)) {
+  if (moe_front_takes(M, D, E, E, false, false, false)) {
     MOE_REQUIRE(ws, MOE_ERR_NULL, "router: null pointer");
     MOE_REQUIRE(MOE_ALIGNED16(ws), MOE_ERR_BAD_ALIGN, "router: pointers must be 16-byte aligned");
     MOE_REQUIRE(ws_bytes >= moe_router_workspace_bytes(M, D, E), MOE_ERR_WORKSPACE_TOO_SMALL, "router: workspace %zu < %zu", ws_bytes,

@@ -49,6 +49,11 @@ int main() {
       const RoutedGemm routed{op, (const int32_t*)memory, 8, 64, memory, sizeof memory, 0, 0};
       const DenseGemm dense{op, 64};
       std::cout << moe_gemm_gateup_impl(&routed, &dense, nullptr) << " " << moe_gemm_down_impl(&routed, &dense, nullptr) << " " << moe_last_error() << "\n";
+    } else if (what == "front") {   // tokens, D, experts, columns, whether a norm, f32 input, a sort
+      int M, D, E, N;
+      bool norm, x_f32, sorted;
+      std::cin >> M >> D >> E >> N >> norm >> x_f32 >> sorted;
+      std::cout << moe_front_takes(M, D, E, N, norm, x_f32, sorted) << "\n";
     } else if (what == "routing") {   // tokens, D, experts: what moe_routing refuses before any GPU call
       int M, D, E;
       std::cin >> M >> D >> E;

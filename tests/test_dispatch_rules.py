@@ -118,6 +118,19 @@ def test_a_dense_group_beside_routed_rows_needs_their_list(ask):
     assert ask(("both",))[0].startswith("-1 -1 gemm_down: a dense group")
 
 
+def test_small_routers_of_many_tokens_go_launch_by_launch(ask):
+    """One workgroup a CU has 4096 tokens; more of them only where that is faster."""
+    def takes(*calls):
+        return ask(*[("front", M, D, E, E, *flags) for M, D, E, *flags in calls])
+    norm, bare, f32, alone = (True, False, True), (False, False, True), (False, True, True), (False, False, False)
+    taken = [(4096, 1024, 64, *norm), (4096, 128, 8, *norm), (4097, 512, 64, *bare), (32768, 256, 64, *bare), (4600, 1024, 64, *f32), (4600, 1024, 64, *alone),
+             (32768, 128, 64, *alone)]
+    left = [(4097, 1024, 64, *norm), (4097, 128, 8, *norm), (65536, 128, 64, *norm), (4097, 640, 64, *bare), (32769, 128, 64, *bare), (32769, 128, 64, *alone),
+            (262144, 128, 8, *alone)]
+    assert takes(*taken) == ["1"] * len(taken)
+    assert takes(*left) == ["0"] * len(left)
+
+
 def test_routers_refuse_activations_beyond_4_gb_whatever_the_launch(ask):
     """128 columns and 64 experts go to the launch that has everything in one, 65 experts to the matmul's own."""
     for E in (64, 65):
