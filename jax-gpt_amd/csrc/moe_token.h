@@ -28,4 +28,7 @@ bool moe_token_takes(int M, int D, int E, int k, int I, int SI);
 // the second launch: tiles of 16 output columns and waves of a workgroup, LDS of a wave
 struct TokenDownPlan { int tiles, waves, wave_lds; };
 TokenDownPlan moe_token_down_plan(int M, int D, int k, int I, int SI);
+// K steps of a ring's stage in the two launches: 1 or 2
+struct TokenStages { int gateup, down; };
+TokenStages moe_token_stages(int M, int D, int k, int I, int SI, bool from_memory);
 int moe_token_experts(const TokenArgs& a, bool from_memory, moe_stream_t stream);

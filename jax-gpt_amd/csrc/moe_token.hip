@@ -241,19 +241,13 @@ __global__ __launch_bounds__(1024) void token_down_kernel(const TokenArgs a, con
   }
 }
 
-// Two K steps a stage, 256 bytes of a row (us, one / two).  In the first launch from the caches, or while a CU has up to four
-// workgroups: one token of Qwen3-MoE 19.8 / 17.9 for the call, two 21.8 / 21.2; 8 of the mini layer 17.0 / 16.5; with more of them
-// from memory their rows get in each other's way: one of DeepSeek-V3 (1152 workgroups) 74.7 / 75.5, 6 of Qwen3-MoE 42.8 / 44.7.  In
-// the second one from the caches, or where a wave walks up to 24 K steps: 16 tokens of tiny 16.5 / 15.5, of the mini layer 21.5 /
-// 20.7, 6 of Qwen3-MoE 43.7 / 42.8, 8 50.8 / 50.5, 2 of the full layer 61.5 / 61.1; DeepSeek-V3 (32 steps) 74.5 / 74.7.
 int launch_gateup(const TokenArgs& a, bool from_memory, hipStream_t s) {
   static std::atomic<unsigned long long> raised[4] = {};
-  const unsigned columns = (a.k * a.I + a.SI) / COLS;
-  const int pairs = a.D % (2 * BK) == 0 && up_lds(a.D, 2) <= kLds && (!from_memory || columns * a.M <= 1024);
+  const bool pairs = moe_token_stages(a.M, a.D, a.k, a.I, a.SI, from_memory).gateup == 2;
   auto* kernel = pairs ? (from_memory ? token_gateup_kernel<true, 2> : token_gateup_kernel<false, 2>)
                        : (from_memory ? token_gateup_kernel<true, 1> : token_gateup_kernel<false, 1>);
   if (int rc = moe_raise_lds_limit((const void*)kernel, kLds, raised[2 * pairs + from_memory])) return rc;
-  hipLaunchKernelGGL(kernel, dim3(columns, a.M), dim3(64), up_lds(a.D, 1 + pairs), s, a);
+  hipLaunchKernelGGL(kernel, dim3((a.k * a.I + a.SI) / COLS, a.M), dim3(64), up_lds(a.D, 1 + pairs), s, a);
   return moe_check_hip(hipGetLastError(), "token gate/up launch");
 }
 
@@ -266,14 +260,12 @@ int down_tiles(int D, int M) {
 int launch_down(const TokenArgs& a, bool from_memory, hipStream_t s) {
   static std::atomic<unsigned long long> raised[4] = {};
   const TokenDownPlan p = moe_token_down_plan(a.M, a.D, a.k, a.I, a.SI);
-  const int pair_lds = down_wave_lds(a.h_stride, p.tiles, 2);
-  const int pairs = a.I % (2 * BK) == 0 && a.SI % (2 * BK) == 0 && p.waves * pair_lds <= kDownLds &&
-                    (!from_memory || p.tiles * (a.h_stride / BK) <= 24);
+  const bool pairs = moe_token_stages(a.M, a.D, a.k, a.I, a.SI, from_memory).down == 2;
   auto* kernel = pairs ? (from_memory ? token_down_kernel<true, 2> : token_down_kernel<false, 2>)
                        : (from_memory ? token_down_kernel<true, 1> : token_down_kernel<false, 1>);
   if (int rc = moe_raise_lds_limit((const void*)kernel, kDownLds, raised[2 * pairs + from_memory])) return rc;
-  hipLaunchKernelGGL(kernel, dim3((a.D / COLS + p.tiles - 1) / p.tiles, a.M), dim3(64 * p.waves), p.waves * (pairs ? pair_lds : p.wave_lds), s,
-                     a, p.tiles);
+  hipLaunchKernelGGL(kernel, dim3((a.D / COLS + p.tiles - 1) / p.tiles, a.M), dim3(64 * p.waves),
+                     p.waves * down_wave_lds(a.h_stride, p.tiles, 1 + pairs), s, a, p.tiles);
   return moe_check_hip(hipGetLastError(), "token down launch");
 }
 
@@ -314,6 +306,28 @@ bool moe_token_takes(int M, int D, int E, int k, int I, int SI) {
   const long long bytes = 3ll * M * ((long long)k * I + SI) * D, once = 3ll * (touched * I + SI) * D;
   const long long steps = (long long)(down_tiles(D, M) - 1) * (widest / BK);
   return bytes <= (320ll << 20) && 8 * steps + ((bytes - once) >> 20) <= 300;
+}
+
+// Two K steps a stage, 256 bytes of a row (us, one / two).  In the first launch
+//  - from memory while a CU has up to four workgroups: one token of Qwen3-MoE 19.8 / 17.9 for the call, two 21.8 / 21.2; with more of
+//    them their rows get in each other's way: one of DeepSeek-V3 (1152 workgroups) 74.7 / 75.5, 6 of Qwen3-MoE 42.8 / 44.7;
+//  - from the caches while the CUs hold all workgroups at once, eight or nine of 17 to 18 KB of LDS (the launch: 32 experts of
+//    2048 x 768, k = 8, 1 token 11.0 / 8.2, 4 of it (1536 workgroups) 15.2 / 14.5, 6 (2304) 18.2 / 20.2, 8 21.3 / 24.0; 16 of 1024 x 2048,
+//    k = 4, 4 tokens (2048) 11.8 / 11.1, 8 15.1 / 15.9; 8 of 1024 x 1024, k = 8, 8 tokens 9.9 / 11.4); rows of less than 1024 while
+//    a CU has up to four (8 of 512 x 1024, k = 2, 5 tokens (640) 5.0 / 4.8, 16 (2048) 5.5 / 5.8; 16 of 512 x 512, k = 16, 1 token 4.9 /
+//    4.8, 4 (2048) 5.4 / 5.7, 8 (4096) 6.8 / 8.6).
+// In the second one from the caches, or where a wave walks up to 24 K steps: 16 tokens of tiny 16.5 / 15.5 for the call, of the mini layer
+// 21.5 / 20.7, 6 of Qwen3-MoE 43.7 / 42.8, 8 50.8 / 50.5, 2 of the full layer 61.5 / 61.1; DeepSeek-V3 (32 steps) 74.5 / 74.7.  (The launch
+// of these layers, 1 to 16 tokens: -23 to +2 %.)
+TokenStages moe_token_stages(int M, int D, int k, int I, int SI, bool from_memory) {
+  const long long workgroups = (long long)M * ((k * I + SI) / COLS);
+  const int up = up_lds(D, 2);
+  const bool gateup = D % (2 * BK) == 0 && up <= kLds && workgroups <= (from_memory || D < 1024 ? 1024 : 256 * (kLds / up));
+  const TokenDownPlan p = moe_token_down_plan(M, D, k, I, SI);
+  const int widest = I > SI ? I : SI;
+  const bool down = I % (2 * BK) == 0 && SI % (2 * BK) == 0 && p.waves * down_wave_lds(widest, p.tiles, 2) <= kDownLds &&
+                    (!from_memory || p.tiles * (widest / BK) <= 24);
+  return {1 + gateup, 1 + down};
 }
 
 int moe_token_experts(const TokenArgs& a, bool from_memory, moe_stream_t stream) {

@@ -26,6 +26,11 @@ int main() {
       int M, D, E, k, I, SI;
       std::cin >> M >> D >> E >> k >> I >> SI;
       std::cout << moe_token_takes(M, D, E, k, I, SI) << "\n";
+    } else if (what == "stages") {   // tokens, D, experts, k, I, SI: K steps of a stage in the two launches of single tokens
+      int M, D, E, k, I, SI;
+      std::cin >> M >> D >> E >> k >> I >> SI;
+      const TokenStages st = moe_token_stages(M, D, k, I, SI, moe_gemm_from_memory(((long long)E * I + SI) * D));
+      std::cout << st.gateup << " " << st.down << "\n";
     } else if (what == "down") {   // tokens, D, k, I, SI: tiles and waves of a workgroup, and whether LDS sets the waves
       int M, D, k, I, SI;
       std::cin >> M >> D >> k >> I >> SI;

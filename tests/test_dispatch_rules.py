@@ -84,6 +84,19 @@ def test_few_tokens_go_straight_to_their_experts_where_that_is_cheaper(ask):
     assert ask(*[("token", *c) for c in left]) == ["0"] * len(left)
 
 
+def test_two_k_steps_a_stage_are_for_workgroups_that_run_at_once(ask):
+    """From the caches as many as the CUs' LDS holds, from memory and of short rows four a CU; whole pairs of K steps only.  The
+    batches that test_gpu_variants.py compares are on both sides of each."""
+    from tests.test_gpu_variants import test_single_tokens_in_stages_of_one_and_two_k_steps as compared
+    batches, = [m.args[1] for m in compared.pytestmark if m.name == "parametrize"]
+    assert ask(*[("token", *c) for c in batches]) == ["1"] * len(batches)
+    assert ask(*[("stages", *c) for c in batches]) == ["2 1", "1 1", "2 2", "1 2", "1 1", "1 2", "1 2"]
+    limits = {(4, 2048, 32, 8, 768, 0): "2", (6, 2048, 32, 8, 768, 0): "1", (4, 1024, 8, 8, 1024, 0): "2", (8, 1024, 8, 8, 1024, 0): "1",   # 1536, 2304, 2048, 4096 workgroups
+              (8, 512, 8, 2, 1024, 0): "2", (9, 512, 8, 2, 1024, 0): "1",                        # of short rows 1024, 1152
+              (2, 2048, 128, 8, 768, 0): "2", (3, 2048, 128, 8, 768, 0): "1"}                    # from memory 768, 1152
+    assert [a[0] for a in ask(*[("stages", *c) for c in limits])] == list(limits.values())
+
+
 def test_small_layers_read_the_selection_themselves(ask):
     """Few rows of few experts from the caches, in tiles of up to 128 rows; not where a list's tiles are taller for a reason, nor
     where the short-tile kernel takes the launch."""

@@ -788,6 +788,8 @@ def test_large_weight_arrays_give_the_bits_of_their_experts(jg, E, N, K, dtype):
     (5, 512, 8, 2, 512, 256),       # pairs in both
     (6, 2048, 128, 8, 768, 0),      # from memory: nine workgroups a CU in the first, 18 K steps a wave in the second
     (1, 7168, 18, 8, 2048, 2048),   # 1152 workgroups, 32 K steps
+    (8, 1024, 8, 8, 1024, 0),       # from the caches, more workgroups in the first launch than the CUs hold of two K steps a stage
+    (9, 512, 8, 2, 1024, 0),        # ... of short rows, more than four a CU
 ])
 def test_single_tokens_in_stages_of_one_and_two_k_steps(jg, M, D, E, k, I, SI):
     test_experts_of_single_tokens_give_the_grouped_bits(jg, M, D, E, k, I, SI, False)
