@@ -9,6 +9,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -17,8 +18,9 @@ LIB_PATH = os.path.join(HERE, "libmoe_hip.so")
 # the timing probe of the grouped GEMM's K loop (`python bench.py --probe`): its own library, nothing of the product links it
 PROBE_PATH = os.path.join(HERE, "libmoe_probe.so")
 
-# the layer calls' host work (a Python extension over torch's headers; it gets the library's functions by address)
-CALL_PATH = os.path.join(HERE, "moe_call.so")
+# the layer calls' host work (a Python extension over torch's headers; it gets the library's functions by address).  The suffix is the
+# interpreter's: another one does not find it.
+CALL_PATH = os.path.join(HERE, "moe_call" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 SOURCES = ["moe_api.hip", "moe_route.hip", "moe_router.hip", "moe_permute.hip", "moe_quant.hip", "moe_gemm.hip", "moe_gemm_stream.hip",
            "moe_token.hip", "moe_combine.hip"]
@@ -44,8 +46,6 @@ def _hipcc() -> str:
 
 
 def _call_command() -> list[str]:
-    import sysconfig
-
     import torch
     base = os.path.dirname(torch.__file__)
     return [shutil.which("g++") or "g++", "-O2", "-shared", "-fPIC", "-std=c++17", "-Wall", "-fvisibility=hidden",

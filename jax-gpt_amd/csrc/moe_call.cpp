@@ -11,6 +11,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
+#include <torch/headeronly/version.h>
 
 #include <climits>
 
@@ -326,5 +327,11 @@ PyMODINIT_FUNC PyInit_moe_call() {
       {&k_router, "gate_weight"}, {&k_shared_router, "shared_expert_gate_weight"}};
   for (const auto& k : keys)
     if (!(*k.at = PyUnicode_InternFromString(k.name))) return nullptr;
-  return PyModule_Create(&module);
+  PyObject* m = PyModule_Create(&module);
+  // (what this was compiled against: moe.py compares it with what there is)
+  if (!m || PyModule_AddIntConstant(m, "args_bytes", (long)sizeof(MoeForwardArgs)) || PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION)) {
+    Py_XDECREF(m);
+    return nullptr;
+  }
+  return m;
 }

@@ -21,6 +21,7 @@ block (a second rounding of the weights), cached for the life of the source tens
 from __future__ import annotations
 
 import ctypes as C
+import warnings
 import weakref
 
 import torch
@@ -40,18 +41,40 @@ ROUTING = {"softmax": 0, "sigmoid_grouped": 1}
 
 _FP8, _F32 = torch.float8_e4m3fn, torch.float32
 
-# The layer entry points hand their arguments to moe_call.so (csrc/moe_call.cpp) first: it makes the call where everything is
+# The layer entry points hand their arguments to the extension moe_call (csrc/moe_call.cpp) first: it makes the call where everything is
 # in its usual form, and returns None, having done nothing, where it is not.  Host time of a call behind a busy GPU, in Python /
 # this way (a launch takes 2.5 to 4 us of it): mini sublayer, 1 token 24.1 / 16.5 us, tiny layer, 1 token 18.5 / 13.5, 256 tokens
 # 22.8 / 21.1, its two functions 38.7 / 29.0.
 _calls = None
 
 
+class _NoCalls:
+    """moe_call where it cannot be loaded: takes nothing."""
+    experts = layer = routing = staticmethod(lambda *args: None)
+
+
+def _load_calls():
+    """moe_call, if there is one of this interpreter, this torch and this library's argument struct."""
+    try:
+        from . import moe_call
+        built = getattr(moe_call, "args_bytes", None), getattr(moe_call, "torch_version", None)
+        if built[0] != C.sizeof(MoeForwardArgs) or not torch.__version__.startswith(built[1]):
+            raise ImportError(f"{moe_call.__file__} is of another build (struct of {built[0]} bytes, torch {built[1]})")
+        return moe_call
+    except ImportError as e:
+        warnings.warn(f"layer calls take their arguments apart in Python, some 10 us a call slower: {e} (build it: "
+                      "python -c 'import __graft_entry__ as g; g.build()' at the repository root)", RuntimeWarning, stacklevel=4)
+        return None
+
+
 def _native():
     global _calls
     if _calls is None:
         L = lib()
-        from . import moe_call
+        moe_call = _load_calls()
+        if moe_call is None:
+            _calls = _NoCalls
+            return _calls
         names = ("moe_forward_workspace_bytes", "moe_forward", "moe_forward_f32", "moe_forward_selected",
                  "moe_router_workspace_bytes", "moe_routing")
         moe_call.bind(*(C.cast(getattr(L, n), C.c_void_p).value for n in names), check, _router_weight,

@@ -6,6 +6,8 @@ import importlib.util
 import os
 import shutil
 import subprocess
+import sys
+import types
 import weakref
 
 import pytest
@@ -97,3 +99,24 @@ def test_router_weights_outlive_their_dict_entries(module):
     assert module.layer(x, p, 2, None, 1e-6, 0).shape == x.shape
     assert seen == list(old) and len(lib.calls) == 1 and lib.calls[0].w_shared_gate
     assert all(r() is None for r in old.values())   # (nor are they kept)
+
+
+@pytest.mark.parametrize("there", [None, types.SimpleNamespace(__file__="old"),
+                                   types.SimpleNamespace(__file__="struct", args_bytes=C.sizeof(_lib.MoeForwardArgs) - 8, torch_version=torch.__version__),
+                                   types.SimpleNamespace(__file__="torch", args_bytes=C.sizeof(_lib.MoeForwardArgs), torch_version="1.13.0")],
+                         ids=["missing", "without versions", "another struct", "another torch"])
+def test_layer_calls_go_on_without_the_extension(lib, monkeypatch, there):
+    """The general way needs the library alone: where the extension is not there, or of another build, it is said once and every
+    call goes that way."""
+    from jax_gpt_amd import moe
+    monkeypatch.setitem(sys.modules, moe.__package__ + ".moe_call", there)
+    package = sys.modules[moe.__package__]
+    if there is None:
+        monkeypatch.delattr(package, "moe_call", raising=False)
+    else:
+        monkeypatch.setattr(package, "moe_call", there, raising=False)
+    monkeypatch.setattr(moe, "_calls", None)
+    with pytest.warns(RuntimeWarning, match="in Python"):
+        calls = moe._native()
+    assert calls.layer(0, 0, 0, 0, 0, 0) is calls.routing(0, 0, 0) is calls.experts(*range(19)) is None
+    assert moe._native() is calls
