@@ -19,13 +19,18 @@ from tests.test_gpu_calls import KEYS
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
+def _build_module():
+    spec = importlib.util.spec_from_file_location("_call_build", os.path.join(ROOT, "jax-gpt_amd", "build.py"))
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    return build
+
+
 @pytest.fixture(scope="module")
 def module(tmp_path_factory):
     if shutil.which("g++") is None:
         pytest.skip("needs a C++ compiler")
-    spec = importlib.util.spec_from_file_location("_call_build", os.path.join(ROOT, "jax-gpt_amd", "build.py"))
-    build = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(build)
+    build = _build_module()
     out = tmp_path_factory.mktemp("call")
     source, so = str(out / "host.cpp"), str(out / "moe_call.so")
     headers = [line for line in open(os.path.join(build.CSRC, "moe_call.cpp")) if line.startswith("#include <")]
@@ -120,3 +125,35 @@ def test_layer_calls_go_on_without_the_extension(lib, monkeypatch, there):
         calls = moe._native()
     assert calls.layer(0, 0, 0, 0, 0, 0) is calls.routing(0, 0, 0) is calls.experts(*range(19)) is None
     assert moe._native() is calls
+
+
+@pytest.mark.parametrize("trouble", ["no torch", "no compiler", "compile error"])
+def test_the_library_is_linked_whatever_becomes_of_the_extension(monkeypatch, tmp_path, trouble):
+    """The compilers' calls alone: only the extension's may fail, or be missing, and the library is linked before it."""
+    build, ran = _build_module(), []
+
+    class Process:
+        returncode = 0
+
+        def __init__(self, command, **kw):
+            ran.append(command)
+            if "-lc10" in command:
+                if trouble == "no compiler":
+                    raise FileNotFoundError(command[0])
+                self.returncode = 1
+
+        def communicate(self):
+            return "", None
+
+    monkeypatch.setattr(build, "HERE", str(tmp_path))
+    monkeypatch.setattr(build, "_hipcc", lambda: "hipcc")
+    monkeypatch.setattr(build.subprocess, "Popen", Process)
+    monkeypatch.setattr(build.subprocess, "run", lambda command, check: ran.append(command))
+    if trouble == "no torch":
+        monkeypatch.setitem(sys.modules, "torch", None)
+        assert build.build(verbose=False) == build.LIB_PATH
+    else:
+        with pytest.raises((RuntimeError, FileNotFoundError)):
+            build.build(verbose=False)
+    links = [i for i, c in enumerate(ran) if c[-1] == build.LIB_PATH]
+    assert len(links) == 1 and all(i > links[0] for i, c in enumerate(ran) if "-lc10" in c)
