@@ -518,12 +518,13 @@ def moe_experts(x, router_logits, *, top_k, experts, routing="softmax", bias=Non
 
 def _forward(x, router_logits, top_k, experts, routing="softmax", bias=None, n_group=1, topk_group=1, renorm=True,
              routed_scale=1.0, shared=None, return_debug=False, gate_weight=None, shared_expert_gate_weight=None,
-             norm_weight=None, norm_eps=1e-6, add_residual=False, io_f32=False, selected=None, rank=2):
+             norm_weight=None, norm_eps=1e-6, add_residual=False, io_f32=False, selected=None, rank=2, declined=False):
     """`moe_experts`, with x and the output in f32 if io_f32 (x is rounded to bf16, the output holds bf16 values), and
     with `selected` = (indices, weights) in place of the routing.  x and the output have `rank` dimensions, the last one D.
+    declined: moe_call has been offered these arguments already.
     (Host work, which a small call waits for: mini sublayer, 1 token 17.6 -> 14.1 us of Python without flattened views, with
     one allocation by the activations' likeness and the weights' usual form tested first.)"""
-    if not return_debug and isinstance(x, torch.Tensor) and x.is_cuda and isinstance(routing, str) and routing in ROUTING:
+    if not return_debug and not declined and isinstance(x, torch.Tensor) and x.is_cuda and isinstance(routing, str) and routing in ROUTING:
         out = (_calls or _native()).experts(x, router_logits, top_k, experts, ROUTING[routing], bias, n_group, topk_group, renorm,
                                             routed_scale, shared, gate_weight, shared_expert_gate_weight, norm_weight, norm_eps,
                                             add_residual, io_f32, selected, rank)
@@ -665,7 +666,8 @@ def moe_layer(x, params, n_experts_per_token, n_devices=1, axis_name="tp", mesh=
     io_f32 = x.dtype is _F32
     if not io_f32 and x.dtype != torch.bfloat16:
         raise TypeError(f"x: expected bf16 or f32 activations, got {x.dtype}")
-    if io_f32 and x.data_ptr() % 16:
+    unaligned = io_f32 and x.data_ptr() % 16 != 0
+    if unaligned:
         x = x.clone()   # (a view at an odd offset of its storage: the kernels read 16 bytes at a time)
     shared = None
     if params.get("shared_gate_proj") is not None:
@@ -674,4 +676,5 @@ def moe_layer(x, params, n_experts_per_token, n_devices=1, axis_name="tp", mesh=
     # f32 activations: the path computes from their bf16 rounding and returns the caller's dtype (moe.py:282)
     return _forward(x, None, n_experts_per_token, params, shared=shared, gate_weight=params["gate_weight"],
                     shared_expert_gate_weight=params.get("shared_expert_gate_weight") if shared is not None else None,
-                    norm_weight=_norm_weight, norm_eps=_norm_eps, add_residual=_add_residual, io_f32=io_f32, rank=3)
+                    norm_weight=_norm_weight, norm_eps=_norm_eps, add_residual=_add_residual, io_f32=io_f32, rank=3,
+                    declined=not unaligned)   # (for the alignment alone, maybe: the copy is offered again)

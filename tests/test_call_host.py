@@ -157,3 +157,32 @@ def test_the_library_is_linked_whatever_becomes_of_the_extension(monkeypatch, tm
             build.build(verbose=False)
     links = [i for i, c in enumerate(ran) if c[-1] == build.LIB_PATH]
     assert len(links) == 1 and all(i > links[0] for i, c in enumerate(ran) if "-lc10" in c)
+
+
+def test_layer_calls_in_other_forms_are_offered_once(monkeypatch):
+    """A layer whose weights the extension does not take (plain arrays) is declined once, not again on the general way."""
+    from jax_gpt_amd import moe
+    offered = []
+
+    class Declines:
+        def __getattr__(self, name):
+            return lambda *args: offered.append(name)
+
+    class OnGpu(torch.Tensor):
+        is_cuda = property(lambda self: True)
+
+    class Library:
+        moe_forward_workspace_bytes = staticmethod(lambda *a: 64)
+        moe_forward = moe_forward_f32 = staticmethod(lambda *a: 0)
+
+    monkeypatch.setattr(moe, "_calls", Declines())
+    monkeypatch.setattr(moe, "lib", Library)
+    monkeypatch.setattr(moe, "_stream", lambda: 0)
+    p = _layer_params()
+    on_gpu = lambda t: t.as_subclass(OnGpu)
+    p = {n: {k: on_gpu(t) for k, t in v.items()} if isinstance(v, dict) else on_gpu(v) for n, v in p.items()}
+    x, norm = on_gpu(torch.zeros(1, 5, 256, dtype=torch.bfloat16)), on_gpu(torch.zeros(256))
+    for call in (lambda: moe.moe_layer(x, p, 2), lambda: moe.moe_sublayer(x, norm, p, 2), lambda: moe.moe_layer(on_gpu(x.float()), p, 2),
+                 lambda: moe.moe_experts(x[0], on_gpu(torch.zeros(5, 8)), top_k=2, experts=p)):
+        offered.clear()
+        assert call().shape[-1] == 256 and len(offered) == 1, offered
