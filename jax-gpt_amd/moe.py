@@ -296,6 +296,9 @@ def _expert_weight(w, name, dense=False):
         return _codes(q, name + "['w']"), _dev(s, torch.float32, name + "['scale_inv']")
     if not isinstance(w, torch.Tensor):
         raise TypeError(f"{name}: expected a tensor or an fp8 dict")
+    hit = _derived.get(("plain", id(w)))   # (_cached's test, without its arguments: a call has three of these)
+    if hit is not None and hit[1] == w._version and hit[0]() is w:
+        return hit[2]
 
     def build():
         w3 = w.unsqueeze(0) if w.dim() == 2 else w
