@@ -138,7 +138,7 @@ PyObject* run(Call& c, const Inputs& in) {
   }
   if (in.bias) {
     const at::Tensor* b = usable(in.bias, at::kFloat, 1);
-    if (!b) return general_way();
+    if (!b || b->size(0) < a.E) return general_way();
     a.bias = (const float*)c.hold(*b);
   }
   if (in.norm_weight) {

@@ -589,6 +589,8 @@ def _forward(x, router_logits, top_k, experts, routing="softmax", bias=None, n_g
         a.w_shared_gate = wsg.data_ptr()
     if bias is not None:
         bias = _dev(bias, torch.float32, "bias")
+        if not selected and routing == "sigmoid_grouped" and bias.numel() < E:   # (softmax reads none)
+            raise ValueError(f"bias: expected {E} values, got {tuple(bias.shape)}")
         keep.append(bias)
         a.bias = bias.data_ptr()
     a.w_gate, a.w_up, a.w_down = wg.data_ptr(), wu.data_ptr(), wd.data_ptr()

@@ -159,8 +159,17 @@ def test_the_library_is_linked_whatever_becomes_of_the_extension(monkeypatch, tm
     assert len(links) == 1 and all(i > links[0] for i, c in enumerate(ran) if "-lc10" in c)
 
 
-def test_layer_calls_in_other_forms_are_offered_once(monkeypatch):
-    """A layer whose weights the extension does not take (plain arrays) is declined once, not again on the general way."""
+class OnGpu(torch.Tensor):
+    is_cuda = property(lambda self: True)
+
+
+def on_gpu(t):
+    return {k: on_gpu(v) for k, v in t.items()} if isinstance(t, dict) else t.as_subclass(OnGpu)
+
+
+@pytest.fixture
+def general(monkeypatch):
+    """moe.py whose extension declines every call (the names of its functions that were called) and whose library does nothing."""
     from jax_gpt_amd import moe
     offered = []
 
@@ -168,21 +177,43 @@ def test_layer_calls_in_other_forms_are_offered_once(monkeypatch):
         def __getattr__(self, name):
             return lambda *args: offered.append(name)
 
-    class OnGpu(torch.Tensor):
-        is_cuda = property(lambda self: True)
-
-    class Library:
+    class NoLibrary:
         moe_forward_workspace_bytes = staticmethod(lambda *a: 64)
         moe_forward = moe_forward_f32 = staticmethod(lambda *a: 0)
 
     monkeypatch.setattr(moe, "_calls", Declines())
-    monkeypatch.setattr(moe, "lib", Library)
+    monkeypatch.setattr(moe, "lib", NoLibrary)
     monkeypatch.setattr(moe, "_stream", lambda: 0)
-    p = _layer_params()
-    on_gpu = lambda t: t.as_subclass(OnGpu)
-    p = {n: {k: on_gpu(t) for k, t in v.items()} if isinstance(v, dict) else on_gpu(v) for n, v in p.items()}
+    return moe, offered
+
+
+def test_layer_calls_in_other_forms_are_offered_once(general):
+    """A call that the extension does not take is declined once, not again on the general way."""
+    moe, offered = general
+    p = on_gpu(_layer_params())
     x, norm = on_gpu(torch.zeros(1, 5, 256, dtype=torch.bfloat16)), on_gpu(torch.zeros(256))
     for call in (lambda: moe.moe_layer(x, p, 2), lambda: moe.moe_sublayer(x, norm, p, 2), lambda: moe.moe_layer(on_gpu(x.float()), p, 2),
                  lambda: moe.moe_experts(x[0], on_gpu(torch.zeros(5, 8)), top_k=2, experts=p)):
         offered.clear()
         assert call().shape[-1] == 256 and len(offered) == 1, offered
+
+
+def test_a_selection_bias_holds_a_value_an_expert(module, general):
+    """A shorter one is refused, not read beyond its end; softmax routing reads none, and a longer one's end is not read."""
+    moe, _ = general
+    lib, p, E = Library(module), _layer_params(), 8
+    x, logits = torch.zeros(5, 256, dtype=torch.bfloat16), torch.zeros(5, E)
+
+    def native(bias, routing):
+        return module.experts(x, logits, 2, p, routing, bias, 1, 1, 1, 1.0, None, None, None, None, 1e-6, 0, 0, None, 2)
+
+    def python(bias, routing):
+        return moe.moe_experts(on_gpu(x), on_gpu(logits), top_k=2, experts=on_gpu(p), routing=routing, bias=on_gpu(bias))
+    for n in (0, E - 1):
+        assert native(torch.zeros(n), 1) is None and not lib.calls
+        with pytest.raises(ValueError, match="bias"):
+            python(torch.zeros(n), "sigmoid_grouped")
+        assert python(torch.zeros(n), "softmax").shape == x.shape
+    for n in (E, E + 1):
+        assert native(torch.zeros(n), 1).shape == python(torch.zeros(n), "sigmoid_grouped").shape == x.shape
+    assert len(lib.calls) == 2
