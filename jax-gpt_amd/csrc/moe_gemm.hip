@@ -669,11 +669,17 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_kernel(const GemmOperands 
 //
 // Up to 2048 selections of up to 64 experts are read and counted by every workgroup itself, while it would otherwise wait for the
 // list header, the list entry and the row ids one after the other: no sort and no list in front of the two GEMMs, and rows of h
-// and y stay where their selections stand (flat index token * k + slot).  The same items, classes and bits.
+// and y stand where their selections stand (flat index token * k + slot).  The same bits; the items too, except where a list could
+// have tiles of more than 128 rows, and that an expert's neighbours in the list are others.
 //   What bounds these launches: their start (arguments, instruction lines, the selections from memory), then the items' streams as in
 // the class kernel.  A GEMM launch is 0.5 to 1.5 us longer than one that reads a list, the sort's launch of 3.5 to 6 us (and as much
 // on the host) is gone: tiny layer, 32 tokens 22.6 -> 20 us, 256 25 -> 21.5, 1000 31 -> 28; mini layer, 64 tokens 30 -> 26.5, its
-// sublayer 200 tokens 31.6 -> 27.9, 1000 39 -> 35; uneven routings alike.  The limits are what a lane an expert and four
+// sublayer 200 tokens 31.6 -> 27.9, 1000 39 -> 35.  Uneven routings (with a list / this way, us a call): normal offsets of 2 on the
+// logits, 64 experts of 1024 x 512, k = 8, 200 tokens 46.2 / 35.7, 256 49.0 / 35.1, mini layer of 1024 36.4 / 32.1, tiny of 1000 32.2 /
+// 29.6; all 2048 selections of 64 experts at one 46.2 / 36.6, half of 2048 of 32 experts of 1024 x 1024 at one 61.7 / 51.1.  Not every
+// one: where an even routing's items just fill the CUs and a few heavy experts begin another round, a list balances that better (the
+// 64 experts, 70 % of 200 tokens at eight of them, anywhere 44.9 / 47.8, side by side 46.8 / 42.1; 70 % of 2048 at one 52.0 / 57.7);
+// eight experts of 1024 x 2048, 1900 and 2048 rows, 47.7 / 48.5 and 48.9 / 49.8.  The limits are what a lane an expert and four
 // selections a thread hold.
 constexpr int kScanRows = 2048, kScanExperts = 64, kScanTileRows = 128;
 constexpr int SCAN_OFF = 150016;   // LDS: [64] experts' rows, [8] waves' rows of the item's expert, [128] the tile's rows
@@ -697,13 +703,16 @@ __device__ __forceinline__ bool scan_item(Item& item, int* experts, int* counts,
   for (int j = 0; j < MOST; ++j)
     if ((unsigned)mine[j] < (unsigned)E) atomicAdd(&experts[mine[j]], 1);   // (a selection out of range has no row)
   __syncthreads();
-  const int rows = experts[lane], nt = moe_tile_count(rows, tile_rows), to = moe_wave_scan(nt);   // lane = expert
+  // Experts side by side are eight lanes apart: the tiles of a heavy group of them go to all XCDs (of eight that have 70 % of the
+  // tokens, 64 experts of 1024 x 512, k = 8, 200 tokens 50.6 -> 42.1 us, 256 51.7 -> 42.2; 46.8 and 52.8 with a list).
+  auto swapped = [](int l) { return (l & 7) << 3 | l >> 3; };   // a lane's expert, an expert's lane
+  const int rows = experts[swapped(lane)], nt = moe_tile_count(rows, tile_rows), to = moe_wave_scan(nt);
   const int n_items = __builtin_amdgcn_readlane(to, 63) * ncb;
   const int id = (int)((unsigned)(n_items * xcd) >> 3) + (index >> 3);
   if (id >= (int)((unsigned)(n_items * (xcd + 1)) >> 3)) return false;   // (uniform)
-  const int tile = id / ncb, e = (int)__builtin_ctzll(__ballot(to > tile));
-  const int e_rows = __builtin_amdgcn_readlane(rows, e), e_tiles = __builtin_amdgcn_readlane(nt, e);
-  const int first = __builtin_amdgcn_readlane(to, e) - e_tiles;
+  const int tile = id / ncb, at = (int)__builtin_ctzll(__ballot(to > tile)), e = swapped(at);
+  const int e_rows = __builtin_amdgcn_readlane(rows, at), e_tiles = __builtin_amdgcn_readlane(nt, at);
+  const int first = __builtin_amdgcn_readlane(to, at) - e_tiles;
   int rt, t0;
   expert_item(id - first * ncb, e_tiles, ncb, item.col_block, rt);
   moe_tile_span(e_rows, e_tiles, rt, t0, item.row_count);
