@@ -10,6 +10,7 @@ import sys
 import types
 import weakref
 
+import numpy as np
 import pytest
 import torch
 
@@ -217,3 +218,24 @@ def test_a_selection_bias_holds_a_value_an_expert(module, general):
     for n in (E, E + 1):
         assert native(torch.zeros(n), 1).shape == python(torch.zeros(n), "sigmoid_grouped").shape == x.shape
     assert len(lib.calls) == 2
+
+
+@pytest.mark.parametrize("at,value", [(2, np.int64(2)), (2, 2.0), (2, "2"), (2, None), (2, 1 << 40), (2, -(1 << 40)), (4, 0.0), (6, np.int32(4)), (7, None),
+                                      (8, np.bool_(True)), (9, 2), (9, np.float32(2.5)), (14, 0), (14, np.float64(1e-6)), (15, np.bool_(True)), (16, None),
+                                      (18, 2.0), (18, 4)])
+def test_other_scalars_are_declined(module, at, value):
+    """A call that is taken, and the same with one number of another type, or beyond an int."""
+    lib, x = Library(module), torch.zeros(5, 256, dtype=torch.bfloat16)
+    call = [x, torch.zeros(5, 8), 2, _layer_params(), 1, None, 4, 2, True, 2.5, None, None, None, torch.zeros(256), 1e-6, True, False, None, 2]
+    assert module.experts(*call).shape == x.shape and len(lib.calls) == 1
+    a = lib.calls.pop()
+    assert (a.M, a.D, a.E, a.k, a.I, a.SI, a.routing, a.n_group, a.topk_group, a.renorm, a.routed_scale, a.add_residual) == (5, 256, 8, 2, 128, 0, 1, 4, 2, 1, 2.5, 1)
+    assert a.norm_eps == np.float32(1e-6) and a.x == x.data_ptr()
+    call[at] = value
+    assert module.experts(*call) is None and not lib.calls
+    if at == 2:
+        p = _layer_params()
+        assert module.routing(x, p["gate_weight"], 2) and len(lib.calls) == 1
+        assert module.routing(x, p["gate_weight"], value) is None and len(lib.calls) == 1
+        assert module.layer(x[None], p, 2, None, 1e-6, 0) is not None and len(lib.calls) == 2
+        assert module.layer(x[None], p, value, None, 1e-6, 0) is None and len(lib.calls) == 2

@@ -133,9 +133,18 @@ def test_a_dense_group_beside_routed_rows_needs_their_list(ask):
 
 def test_small_routers_of_many_tokens_go_launch_by_launch(ask):
     """One workgroup a CU has 4096 tokens; more of them only where that is faster."""
+    from tests.test_gpu_variants import test_small_routers_in_one_launch_give_the_bits_of_the_stages as small
+
     def takes(*calls):
         return ask(*[("front", M, D, E, E, *flags) for M, D, E, *flags in calls])
     norm, bare, f32, alone = (True, False, True), (False, False, True), (False, True, True), (False, False, False)
+    # what test_gpu_variants.py compares: all of it in one launch, but for the norm of the largest batch
+    compared, = [m.args[1] for m in small.pytestmark if m.name == "parametrize"]
+    for M, D, E, SI, dtype, _ in compared:
+        flags = [(has_norm, dtype == "f32", True) for has_norm in (True, False)] + [alone]
+        assert ask(*[("front", M, D, E, E + (SI > 0), *f) for f in flags]) == ["0" if M > 4096 else "1", "1", "1"], (M, D, E)
+    # too many experts, too long rows, rows of no whole blocks, K slices of more than one block
+    assert takes((100, 512, 65, *norm), (100, 1152, 8, *norm), (100, 192, 8, *norm), (12000, 1024, 64, *alone)) == ["0"] * 4
     taken = [(4096, 1024, 64, *norm), (4096, 128, 8, *norm), (4097, 512, 64, *bare), (32768, 256, 64, *bare), (4600, 1024, 64, *f32), (4600, 1024, 64, *alone),
              (32768, 128, 64, *alone)]
     left = [(4097, 1024, 64, *norm), (4097, 128, 8, *norm), (65536, 128, 64, *norm), (4097, 640, 64, *bare), (32769, 128, 64, *bare), (32769, 128, 64, *alone),

@@ -146,6 +146,35 @@ def test_calls_in_other_forms_go_the_general_way(jg, ways):
     assert not any(taken) and isinstance(a, Exception) and type(a) is type(b)
 
 
+@pytest.mark.gpu
+def test_calls_with_other_scalars_go_the_general_way(jg, ways):
+    """Calls that differ from a taken one in the type of one number alone: converted, or refused, as without the native way."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(11)
+    M, D, E, I, k = 5, 256, 8, 128, 2
+    ex, p = _weights(jg, E, D, I, gen), _layer_params(jg, gen)
+    r = lambda *s: torch.randn(s, device="cuda", generator=gen)
+    x, lg, norm = r(M, D).bfloat16(), r(M, E), r(D)
+    base = dict(top_k=k, experts=ex, routing="sigmoid_grouped", n_group=4, topk_group=2, renorm=True, routed_scale=2.5, norm_weight=norm, norm_eps=1e-6,
+                add_residual=True)
+    whole = (lambda **kw: jg.moe_experts(x, lg, **dict(base, **kw)))
+    a, b, taken = ways(whole)
+    assert taken == [True] and not isinstance(a, Exception)
+    _same(a, b)
+    for kw in (dict(top_k=np.int64(k)), dict(top_k=2.0), dict(top_k="2"), dict(top_k=None), dict(top_k=1 << 40), dict(n_group=np.int32(4)), dict(topk_group=2.0),
+               dict(renorm=np.bool_(True)), dict(renorm=1.0), dict(routed_scale=2), dict(routed_scale=np.float32(2.5)), dict(norm_eps=0), dict(norm_eps=np.float64(1e-6)),
+               dict(add_residual=np.bool_(True))):
+        a, b, taken = ways(lambda: whole(**kw))
+        assert taken == [False], kw
+        _same(a, b)
+    for call in (lambda: jg.moe_routing(x, p["gate_weight"], np.int64(k)), lambda: jg.moe_layer(x[None], p, np.int32(k)),
+                 lambda: jg.moe_sublayer(x[None], norm, p, k, 0)):
+        a, b, taken = ways(call)
+        assert not any(taken)
+        _same(a, b)
+
+
 def test_native_way_takes_nothing_from_the_cpu():
     """Without a GPU: every entry point of the module declines, and reads no address it was bound to."""
     import ctypes

@@ -688,7 +688,7 @@ def test_tall_tiles_give_the_bits_of_full_ones(jg, sizes):
     (257, 1024, 8, 128, "bf16", "softmax"),       # two tokens a workgroup, the last one alone
     (1025, 512, 40, 0, "bf16", "sigmoid_grouped"),   # eight, and selections counted for the sort
     (2049, 896, 12, 128, "f32", "softmax"),       # sixteen, block-major scales
-    (4097, 256, 64, 0, "bf16", "softmax"),        # more workgroups than histograms
+    (4097, 256, 64, 0, "bf16", "softmax"),        # more workgroups than histograms (with the norm: launch by launch)
 ])
 def test_small_routers_in_one_launch_give_the_bits_of_the_stages(jg, M, D, E, SI, dtype, routing):
     import torch
