@@ -128,10 +128,10 @@ __global__ __launch_bounds__(WAVE ? MOE_WAVE : 1024) void build_tiles_kernel(con
 // consecutive tile rows; the swizzle is applied by choosing which 16-byte piece of the row
 // each lane fetches.  No asynchronous load ever targets a register.
 
-// One launch, row tiles of every height.  A work item's row tile (at most 288 rows, near-equal cuts of its
+// One launch, row tiles of every height.  A work item's row tile (at most 288 rows, 320 with TALL, near-equal cuts of its
 // expert) is served by the smallest of nine (ten: TALL) compiled tile classes that holds it -- 32 XF rows, XF = 1 .. 9 MFMA
 // groups per wave and K step -- each a branch-free, fully unrolled K loop of its own with its own LDS ring: the
-// short classes have short activation tiles and use the room for more stages (256 and 288 rows: two stages; 160 to 224
+// short classes have short activation tiles and use the room for more stages (256 rows and more: two stages; 160 to 224
 // rows: three weight stages, two activation stages; 64 to 128 rows: three stages, copies two steps ahead; 32 rows:
 // four stages, three steps ahead), because an item of a few rows only streams its 256 weight rows and lives on the
 // bytes it keeps in flight.  Rows past the end of a tile are multiplied like the others (their copies re-read the tile's last
@@ -156,7 +156,7 @@ template <int XF, int MODE = MODE_GATEUP, bool ONCE = true> struct Cls {
   // the middle of the step, and not behind the next barrier: the weights of step kb + 2 are then in flight while step
   // kb still computes, as if the ring were a stage deeper, in the same LDS.  The weight rows that wave (wi, 0) copies
   // are read by itself and by wave (wi, 1) alone, so the release is a word in LDS between those two (early_flag)
-  // and no barrier.  Only the 256- and 288-row classes of the gate/up GEMM, which have no room for a third stage: -4.5 % where
+  // and no barrier.  Only the classes of 256 rows and more of the gate/up GEMM, which have no room for a third stage: -4.5 % where
   // every workgroup streams its own weight slab, -3 % where 8 row tiles share one, -1 % on the mixed tile
   // heights of skewed routing; the down GEMM (16 K steps at the DeepSeek-V3 shape) gained 2 % in the first case and
   // lost 1 % in the second, and the classes with three weight stages cannot gain: their copies complete in issue
@@ -946,11 +946,15 @@ int launch(const RoutedGemm* rt, const DenseGemm* dn, hipStream_t s) {
 // not know) 852 / 835; 33 to 128 tokens otherwise -1.0 to +1.5 %, -0.2 on average.
 //   Tall tiles (320 rows, moe_tile_rows_voted) for lists of both GEMMs, of short K and at most eight rounds, where an even routing
 // puts the largest groups, 2.5 to 3 standard deviations above the mean, between whole full tiles and whole tall ones: with full
-// tiles alone a few of Qwen3-MoE's 128 experts have two at 4096 tokens, 130 tiles x 6 and x 8 columns, 3.05 and 4.06 rounds: gate/up
-// 135 -> 130, down 88.4 -> 84.3, the layer 256 -> 242 us; 3950 tokens through the two functions 269 -> 257, 8192 tokens 446 -> 428, 4600
-// 284 -> 278.  The kernel that has this height too runs the other heights 0.5 to 1.5 % slower, which is what a wrong guess costs
-// and why K = 7168 (64 experts of 266 rows 538 -> 504 and 298 -> 289, but sixteen rounds even) and rows that another GPU has
-// dispatched, which are uneven, go without.
+// tiles alone a few of Qwen3-MoE's 128 experts have two at 4096 tokens, some 130 tiles x 6 and x 8 columns, 3.05 and 4.06 rounds.  Even
+// logits, six draws each, the launches' medians full / tall: 4096 tokens gate/up 134 / 128, down 91 / 84 (of these the two draws that have
+// an expert of more than 320 rows, and so full tiles, 146 / 143 and 130 / 135, 96 / 90 and 86 / 87), 8192 226 / 224 and 150 / 145, 9000 250 /
+// 236 and 167 / 155; the layer, 4096 tokens 258 / 244, 4300 267 / 256, 9000 482 / 476 and 490 / 474.  For 128 experts, k = 8, that is 3850 to
+// 4430 and 8120 to 9240 tokens.  The kernel that has this height too runs the other heights slower, which is what a wrong guess
+// costs: the layer with normal offsets of 0.15 to 2 on the logits -1.8 to +0.9 % at 3860 to 4430 tokens, -0.2 to +2 % at 8120 to 9240.  Hence
+// only where the guess has shown to be right more often than not: not for rows that another GPU has dispatched, which are uneven,
+// nor for longer K, of which one batch was measured (K = 7168, 64 experts of 266 rows each, gate/up 538 / 504, down 298 / 289) and no
+// uneven one, nor between 2048 and that.
 int moe_gemm_tile_rows(const TileShape& t) {
   const int groups = t.E < t.R ? t.E : t.R;
   if (groups <= 0) return kTileRows;

@@ -348,14 +348,16 @@ __global__ __launch_bounds__(1024) void route_kernel(const RouteArgs a, const Ro
 // 33 columns of 1024, from L2), so each does the whole chain for its tokens: one launch, no partial sums in memory.
 //   Its eight waves take a row's pieces of eight values 64 at a time, square, normalise and quantise them and put them into LDS,
 // while the weights travel into registers; then wave w multiplies K block w of all rows (128 values, a quantisation group) with
-// up to five fragments of 16 columns, the blocks' products meet in LDS, and a wave selects a token's experts.  Sums, blocks and
+// up to five fragments of 16 columns (65 in all), the blocks' products meet in LDS, and a wave selects a token's experts.  Sums, blocks and
 // instructions are those of rmsnorm_quant_kernel, router_gemm_kernel (where its K slices are 128 long) and route_kernel in their
 // order: the same bits.
 //   What bounds it: the launch's start and four trips through memory and LDS.  Against the launches that it replaces (us): mini
 // layer (33 columns of 1024), 1 token 5.5 / 7.5, 64 7.3 / 9.5, 4096 12.1 / 14.0; behind its norm 1 token 6.0 / 7.9, 200 7.5 /
 // 13.1, 1000 8.6 / 14.4; tiny (8 of 512), 100 tokens 4.0 / 7.8.  Sixteen tokens a workgroup at any size: 11.1 for 64 tokens, 13.6
 // for 200 behind the norm.  The limits on columns and hidden size are what a wave has registers and a workgroup waves for.
-constexpr int kFrontTokens = 16, kFrontWaves = 8, kFrontColumns = 80, kFrontD = 128 * kFrontWaves;
+constexpr int kFrontTokens = 16, kFrontWaves = 8, kFrontExperts = 64, kFrontColumns = kFrontExperts + 1, kFrontD = 128 * kFrontWaves;
+constexpr int front_lds(int tokens, int D, int N, int E) { return tokens * D * 2 + (tokens * N * (D / 128 + 1) + E) * 4; }
+constexpr int kFrontLds = front_lds(kFrontTokens, kFrontD, kFrontColumns, kFrontExperts);   // 70464
 struct FrontJob {
   const void* x;
   int x_f32, D, tokens;         // tokens of a workgroup: a power of two up to kFrontTokens
@@ -371,7 +373,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 template <int KIND, bool NORM>
 __global__ __launch_bounds__(64 * kFrontWaves) void front_kernel(const RouteArgs a, const FrontJob f) {
   extern __shared__ __attribute__((aligned(16))) int lds[];   // [rows' pieces][the K blocks' products][logits][E counts]
-  constexpr int GROUPS = kFrontColumns / 16, UNITS = kFrontTokens * (kFrontD / 512) / kFrontWaves;
+  constexpr int GROUPS = (kFrontColumns + 15) / 16, UNITS = kFrontTokens * (kFrontD / 512) / kFrontWaves;
   __shared__ float wave_sum[kFrontTokens][kFrontD / 512];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fq = lane >> 4;
@@ -614,7 +616,7 @@ int moe_route_impl(int routing, const RouteArgs& a, const QuantJob* quant, const
 // which else needs its rounding stored, 5000 of 640 69.7 / 66.8, 4097 of 1024 72.2 / 66.4;
 //   the routing alone, 4600 of 1024 15.1 / 13.1, 32000 of 256 28.5 / 24.1, 65536 of 128 42.1 / 39.8, 262144 132 / 157.
 bool moe_front_takes(int M, int D, int E, int N, bool norm, bool x_f32, bool sorted) {
-  if (M < 1 || E > 64 || N > kFrontColumns || D < 128 || D > kFrontD || D % 128 || moe_router_k_slice(M, N, D) != 128) return false;
+  if (M < 1 || E > kFrontExperts || D < 128 || D > kFrontD || D % 128 || moe_router_k_slice(M, N, D) != 128) return false;
   return M <= kFrontTokens * kCUs || (M <= 32768 && !norm && (!sorted || x_f32 || D <= 512));
 }
 int moe_front_impl(int routing, RouteArgs a, const FrontArgs& f, const PermuteOut* sort, void* permute_ws, size_t permute_ws_bytes,
@@ -633,15 +635,15 @@ int moe_front_impl(int routing, RouteArgs a, const FrontArgs& f, const PermuteOu
   // Tokens of a workgroup: one, or as many as it takes to have one workgroup a CU.
   int tokens = 1;
   while (tokens < kFrontTokens && tokens * kCUs < a.M) tokens *= 2;
-  const int R = a.M * a.k, blocks = (a.M + tokens - 1) / tokens, KB = f.D / 128;
+  const int R = a.M * a.k, blocks = (a.M + tokens - 1) / tokens;
   const bool one_chunk = R <= kSmallRows, counts = sort && !one_chunk && blocks <= moe_permute_max_chunks(a.E);
   const FrontJob job{f.x, f.x_f32, f.D, tokens, f.norm, f.eps, (const bf16_t*)f.w_router, (const bf16_t*)f.w_shared_gate, f.xq, f.sx, f.sx_blocked,
                      counts ? (int32_t*)permute_ws : nullptr};
-  const size_t lds = (size_t)tokens * f.D * 2 + ((size_t)tokens * N * (KB + 1) + a.E) * sizeof(float);   // (at most 78 KB)
+  const int lds = front_lds(tokens, f.D, N, a.E);
   auto* kernel = routing == MOE_ROUTING_SOFTMAX ? (f.norm ? front_kernel<ROUTE_SOFTMAX, true> : front_kernel<ROUTE_SOFTMAX, false>)
                                                 : (f.norm ? front_kernel<ROUTE_GROUPED, true> : front_kernel<ROUTE_GROUPED, false>);
   static std::atomic<unsigned long long> lds_raised[4] = {};
-  if (int rc = moe_raise_lds_limit((const void*)kernel, 80 * 1024, lds_raised[(routing == MOE_ROUTING_SOFTMAX ? 0 : 2) + (f.norm ? 1 : 0)])) return rc;
+  if (int rc = moe_raise_lds_limit((const void*)kernel, kFrontLds, lds_raised[(routing == MOE_ROUTING_SOFTMAX ? 0 : 2) + (f.norm ? 1 : 0)])) return rc;
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kFrontWaves), lds, (hipStream_t)stream, a, job);
   if (int rc = moe_check_hip(hipGetLastError(), "route launch")) return rc;
   if (!sort) return MOE_OK;
