@@ -191,14 +191,18 @@ extern "C" int moe_quant_weight_block(const void* w, int src_is_f32, int E, int 
   //   bf16 96 18.9 / 19.1, 129 24.7 / 25.3, 144 26.8 / 27.1, 185 33.7 / 33.3, 208 36.1 / 35.3, 270 48.0 / 47.7, 336 58.9 / 56.4, 562
   // 98.8 / 93.2, 672 119.2 / 111.4, 2352 429 / 389;
   //   f32 160 29.3 / 30.8, 216 37.8 / 37.3, 320 56.6 / 56.9, 347 60.0 / 56.9, 450 75.4 / 74.8, 560 94.9 / 89.8, 957 167 / 154, 1120 191 / 182.
-  // Below, f32 is 1 to 4 % faster with eight waves.  Plain stores look 9 % better only while the same codes are written again and
+  // Below, f32 takes eight waves, or four where a CU has between one and two blocks (blocks of 128 x 128, us with four / eight): 256 5.69 /
+  // 5.49, 320 7.07 / 6.87, 384 7.54 / 7.63, 440 7.85 / 8.09, 500 8.47 / 8.77, 520 10.45 / 10.26, 576 10.59 / 10.26, 768 12.60 / 12.36, 896
+  // 13.99 / 14.19, 1024 16.06 / 15.66, 1536 22.32 / 22.50, 2560 36.0 / 35.9.  Plain stores look 9 % better only while the same codes are written again and
   // again and stay in the memory-side cache (672 MB: 107; into other memory each time 123).
   const long long n = (long long)E * N * K;
   auto launch = [&](auto* kernel, auto* src, int width, int threads) {
     hipLaunchKernelGGL(kernel, dim3(K / (128 * width), N / 128, E), dim3(threads), 0, (hipStream_t)stream, src, N, K, wq, sw);
   };
+  const long long blocks = n / (128 * 128);
   if (src_is_f32) n * 5 > (320ll << 20) ? launch(quant_weight_kernel<float, 1, 1024>, (const float*)w, 1, 1024)
-                                        : launch(quant_weight_kernel<float, 1, 512>, (const float*)w, 1, 512);
+                  : blocks > 320 && blocks <= 512 ? launch(quant_weight_kernel<float, 1, 256>, (const float*)w, 1, 256)
+                                                  : launch(quant_weight_kernel<float, 1, 512>, (const float*)w, 1, 512);
   else n * 3 > (160ll << 20) && K % 256 == 0 ? launch(quant_weight_kernel<bf16_t, 2, 1024>, (const bf16_t*)w, 2, 1024)
                                              : launch(quant_weight_kernel<bf16_t, 1, 256>, (const bf16_t*)w, 1, 256);
   return moe_check_hip(hipGetLastError(), "quant_weight_block launch");

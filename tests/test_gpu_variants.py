@@ -767,7 +767,7 @@ def test_small_layers_without_a_list_give_the_bits_of_the_sorted_rows(jg, M, D, 
     assert torch.equal(got, same) and not got[2].any()
 
 
-@pytest.mark.parametrize("E,N,K,dtype", [(9, 2560, 2560, "bf16"), (9, 2560, 2688, "bf16"), (11, 2560, 2432, "f32")])   # two blocks wide; an odd number of blocks; sixteen waves
+@pytest.mark.parametrize("E,N,K,dtype", [(9, 2560, 2560, "bf16"), (9, 2560, 2688, "bf16"), (11, 2560, 2432, "f32"), (25, 512, 512, "f32")])   # two blocks wide; an odd number of blocks; sixteen waves; four, its experts eight
 def test_large_weight_arrays_give_the_bits_of_their_experts(jg, E, N, K, dtype):
     import torch
     print("weight quantiser", E, N, K, dtype, flush=True)
