@@ -24,7 +24,7 @@ PROBE_PATH = os.path.join(HERE, "libmoe_probe.so")
 CALL_PATH = os.path.join(HERE, "moe_call" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 SOURCES = ["moe_api.hip", "moe_route.hip", "moe_router.hip", "moe_permute.hip", "moe_quant.hip", "moe_gemm.hip", "moe_gemm_stream.hip",
-           "moe_token.hip", "moe_combine.hip"]
+           "moe_token.hip", "moe_small.hip", "moe_combine.hip"]
 # no v_pk_*_f32 code generation (some packed-f32 forms have given wrong results on this hardware)
 COMMON = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function",
           "-fvisibility=hidden",    # only the functions include/moe_hip.h declares (MOE_API) are exported
@@ -36,7 +36,8 @@ PER_FILE = {"moe_route.hip": ["-ffp-contract=off"], "moe_combine.hip": ["-ffp-co
             # MFMA results go straight to VGPRs: the block-scale FMA consumes them on the vector ALU
             "moe_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-Wno-inline-asm"],   # m0 is clobbered on purpose
             "moe_gemm_stream.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-Wno-inline-asm"],
-            "moe_token.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-Wno-inline-asm"]}
+            "moe_token.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-Wno-inline-asm"],
+            "moe_small.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-Wno-inline-asm"]}
 
 
 def _hipcc() -> str:

@@ -8,6 +8,7 @@
 #include <mutex>
 
 #include "moe_common.h"
+#include "moe_small.h"
 #include "moe_token.h"
 
 static thread_local char g_err[512] = "";
@@ -345,6 +346,15 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
     const RoutedGemm down{{hq, sh, nullptr, a->w_down, a->sw_down, nullptr, nullptr, a->I, a->D, y, nullptr, moe_row_major_scales(a->I, a->D)},
                           nullptr, a->E, R, nullptr, 0, scan_rows, 0, ids, a->k};
     if ((rc = moe_gemm_gateup_impl(&gateup, together ? &shared_gateup : nullptr, stream))) return rc;
+    // (what the launches that this one replaces would have refused is refused here)
+    if (const int lanes = moe_small_down_lanes(a->M, a->D, a->E, a->k, a->I, a->SI)) {
+      if ((rc = moe_gemm_check(down.op, R, a->E, true))) return rc;
+      if (together && (rc = moe_gemm_check(shared_down.op, a->M, 1, true))) return rc;
+      MOE_REQUIRE(MOE_ALIGNED16(a->out) && (!a->add_residual || MOE_ALIGNED16(a->x)), MOE_ERR_BAD_ALIGN,
+                  "combine: pointers must be 16-byte aligned");
+      return moe_small_down(SmallDown{hq, a->w_down, sh, a->sw_down, hsq, a->ws_down, shs, a->sws_down, ids, w, shared_gate,
+                                      a->add_residual ? a->x : nullptr, io_f32, a->out, a->M, a->D, a->E, a->k, a->I, a->SI}, lanes, stream);
+    }
     if ((rc = moe_gemm_down_impl(&down, together ? &shared_down : nullptr, stream))) return rc;
     return moe_combine_impl(y, w, ids, a->E, a->SI ? ys : nullptr, shared_gate, a->add_residual ? a->x : nullptr, io_f32, a->M, a->k, a->D,
                             a->out, stream);

@@ -4,6 +4,7 @@
 #include <vector>
 
 #include "moe_gemm_device.h"
+#include "moe_small.h"
 #include "moe_token.h"
 
 int main() {
@@ -22,6 +23,10 @@ int main() {
       std::cin >> M >> D >> E >> k >> I >> SI;
       const TileShape t{M * k, E, M, {I / 128, (D + 255) / 256}, {D / 128, I / 128}, SI ? M : 0, {SI / 128, (D + 255) / 256}};
       std::cout << moe_gemm_scan_rows(t, moe_gemm_from_memory(((long long)E * I + SI) * D)) << "\n";
+    } else if (what == "small") {   // tokens, D, experts, k, I, SI: selections a lane of a small layer's down launch holds, or 0
+      int M, D, E, k, I, SI;
+      std::cin >> M >> D >> E >> k >> I >> SI;
+      std::cout << moe_small_down_lanes(M, D, E, k, I, SI) << "\n";
     } else if (what == "token") {   // tokens, D, experts, k, I, SI
       int M, D, E, k, I, SI;
       std::cin >> M >> D >> E >> k >> I >> SI;

@@ -108,6 +108,20 @@ def test_small_layers_read_the_selection_themselves(ask):
     assert ask(*[("scan", *c) for c in left]) == ["0"] * len(left)
 
 
+def test_small_layers_down_launch_is_for_one_workgroup_a_cu(ask):
+    """64 selections a workgroup where that is no more than 256, else 128, while a workgroup's rows are few; the batches that
+    test_gpu_variants.py compares are of both kinds."""
+    from tests.test_gpu_variants import SMALL_DOWN
+    assert ask(*[("small", *c[:6]) for c in SMALL_DOWN]) == [str(c[6]) for c in SMALL_DOWN]
+    assert all(int(r) for r in ask(*[("scan", *c[:6]) for c in SMALL_DOWN]))
+    assert ask(*[("token", *c[:6]) for c in SMALL_DOWN]) == ["0"] * len(SMALL_DOWN)
+    limits = {(256, 512, 8, 2, 1024, 0): "1", (257, 512, 8, 2, 1024, 0): "2", (512, 512, 8, 2, 1024, 0): "2", (513, 512, 8, 2, 1024, 0): "0",
+              (128, 1024, 32, 2, 512, 512): "1", (256, 1024, 32, 2, 512, 512): "2", (257, 1024, 32, 2, 512, 512): "0",
+              (96, 1024, 32, 2, 2048, 0): "0", (128, 1024, 32, 4, 1024, 0): "0",          # too much for one workgroup
+              (33, 128, 4, 33, 128, 0): "0", (20, 128, 4, 2, 8320, 0): "0", (20, 128, 4, 2, 128, 8320): "0", (20, 128, 65, 2, 128, 0): "0"}
+    assert ask(*[("small", *c) for c in limits]) == list(limits.values())
+
+
 def test_the_compared_batches_of_single_tokens_reach_what_they_are_for(ask):
     """The batches that test_gpu_variants.py compares with the grouped route take the other one, and among them are: a last
     workgroup of fewer tiles, one over two scale blocks, more slots than waves, waves that LDS limits, weights from memory."""

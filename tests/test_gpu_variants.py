@@ -767,6 +767,40 @@ def test_small_layers_without_a_list_give_the_bits_of_the_sorted_rows(jg, M, D, 
     assert torch.equal(got, same) and not got[2].any()
 
 
+SMALL_DOWN = [   # M, D, E, k, I, SI, selections a lane
+    (17, 128, 1, 1, 128, 0, 1),        # one expert: units of 16 rows and of one
+    (64, 256, 64, 1, 128, 128, 1),     # a workgroup's 64 selections, and a unit for nearly each; four of the shared expert
+    (65, 128, 5, 1, 128, 0, 1),        # one more than a workgroup has
+    (43, 384, 7, 3, 384, 256, 1),      # 63 selections of 21 tokens; an odd number of K steps
+    (40, 256, 6, 20, 256, 0, 1),       # more of a token than there are experts, three tokens
+    (200, 512, 4, 2, 1024, 128, 1),    # several units of an expert
+    (17, 128, 1, 1, 8192, 0, 1),       # as many K steps as lanes
+    (129, 1024, 3, 2, 128, 640, 2),    # two selections a lane, one token in the last workgroup, a longer shared expert
+    (300, 512, 8, 3, 512, 0, 2),       # 126 selections
+    (512, 512, 64, 2, 128, 128, 2),    # all that two lanes hold, and units on both sides
+    (20, 512, 9, 26, 128, 0, 2),       # four tokens, selections of one in both of a lane's
+]
+
+
+@pytest.mark.parametrize("M,D,E,k,I,SI,lanes", SMALL_DOWN)
+def test_small_layers_down_launch_gives_the_bits_of_down_and_combine(jg, M, D, E, k, I, SI, lanes):
+    """Even routing, and one whose few experts have several units each; what a selection out of range leaves out."""
+    for offset in (0, 20):
+        test_small_layers_without_a_list_give_the_bits_of_the_sorted_rows(jg, M, D, E, min(k, E), I, SI, offset)
+    if k > E:   # (a selection that is given may name an expert more than once)
+        import torch
+        params, rand = _layer(jg, D, E, I, 0, M)
+        names = ("gate_proj", "up_proj", "down_proj")
+        x, idx = rand(M, D), (torch.arange(M * k, device="cuda") * 7 % (E + 1)).int().reshape(M, k)   # (E: out of range)
+        w = torch.rand(M, k, device="cuda")
+        got = jg.expert_forward_single(x, idx, w, *(params[n] for n in names))
+        parts = [jg.expert_forward_single(x, idx[:, s:s + 1].contiguous(), torch.ones(M, 1, device="cuda"), *(params[n] for n in names)) for s in range(k)]
+        want = torch.zeros(M, D, device="cuda")
+        for s in range(k):   # (one selection a token: its row in bf16)
+            want = want + parts[s].float() * w[:, s:s + 1]
+        assert torch.equal(got, want.bfloat16())
+
+
 @pytest.mark.parametrize("E,N,K,dtype", [(9, 2560, 2560, "bf16"), (9, 2560, 2688, "bf16"), (11, 2560, 2432, "f32"), (25, 512, 512, "f32")])   # two blocks wide; an odd number of blocks; sixteen waves; four, its experts eight
 def test_large_weight_arrays_give_the_bits_of_their_experts(jg, E, N, K, dtype):
     import torch
