@@ -91,7 +91,7 @@ struct ForwardBuffers {
   int32_t *idx, *group_sizes, *group_offsets, *sorted_token_ids, *inv_perm;
   float *h32, *w, *sx, *sh, *shs, *shared_gate, *sx_listed, *sx_blocked;
   uint8_t *xq, *hq, *hsq;
-  void *y, *ys, *permute_ws, *gemm_ws, *router_ws, *normed;
+  void *y, *ys, *permute_ws, *gemm_ws, *gemm_down_ws, *router_ws, *normed;
   size_t permute_ws_bytes, gemm_ws_bytes, router_ws_bytes, total;
 };
 
@@ -108,7 +108,8 @@ ForwardBuffers carve(void* ws, int M, int D, int E, int k, int I, int SI, bool r
   b.permute_ws_bytes = moe_permute_workspace_bytes(M, k, E);
   b.permute_ws = c.take(b.permute_ws_bytes);
   b.gemm_ws_bytes = moe_gemm_workspace_bytes((int)R, E, I > D ? I : D);
-  b.gemm_ws = c.take(b.gemm_ws_bytes);        // tile list of the routed GEMMs (gate/up and down share it)
+  b.gemm_ws = c.take(b.gemm_ws_bytes);        // tile list of the routed GEMMs, and
+  b.gemm_down_ws = c.take(b.gemm_ws_bytes);   // the down GEMM's own, if it has one
   b.xq = (uint8_t*)c.take((size_t)M * D);
   b.sx = (float*)c.take((size_t)M * (D / 128) * 4);
   // block-major copies of the activation scales for large batches (GemmScales): routed rows in sorted order,
@@ -360,9 +361,13 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
                             a->out, stream);
   }
   const int tile_rows = moe_gemm_tile_rows(shape);
-  if ((rc = moe_gemm_tile_list(R, a->E, tile_rows, a->I / 128, (a->D + 255) / 256,
-                               (a->I < a->D ? a->I : a->D) / 128, b.gemm_ws, b.gemm_ws_bytes, &tiles))) return join(rc);
-  const PermuteOut sort{gsz, b.group_offsets, stid, nullptr, inv, a->k, tiles};
+  const int down_rows = moe_gemm_down_tile_rows(shape, tile_rows);
+  TileList down_tiles{};
+  if ((rc = moe_gemm_tile_list(R, a->E, tile_rows, a->I / 128, down_rows ? 0 : (a->D + 255) / 256,
+                               (down_rows || a->D < a->I ? a->D : a->I) / 128, b.gemm_ws, b.gemm_ws_bytes, &tiles))) return join(rc);
+  if (down_rows && (rc = moe_gemm_tile_list(R, a->E, down_rows, 0, (a->D + 255) / 256, a->I / 128, b.gemm_down_ws, b.gemm_ws_bytes, &down_tiles)))
+    return join(rc);
+  const PermuteOut sort{gsz, b.group_offsets, stid, nullptr, inv, a->k, tiles, down_rows ? &down_tiles : nullptr};
   rc = given_idx ? moe_permute_impl(given_idx, a->M, a->k, a->E, sort, b.permute_ws, b.permute_ws_bytes, carried, stream)
                  : select(&sort);
   if (rc) return join(rc);
@@ -387,7 +392,8 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
                                  b.group_offsets, a->E, R, b.gemm_ws, b.gemm_ws_bytes, tile_rows, tiles.pool_tiles};
   const RoutedGemm routed_down{{hq, sh, nullptr, a->w_down, a->sw_down, nullptr, nullptr, a->I, a->D, y, nullptr,
                                 GemmScales{sc.out_row, sc.out_cb, true, 0, 0}},
-                               b.group_offsets, a->E, R, b.gemm_ws, b.gemm_ws_bytes, tile_rows, tiles.pool_tiles};
+                               b.group_offsets, a->E, R, down_rows ? b.gemm_down_ws : b.gemm_ws, b.gemm_ws_bytes,
+                               down_rows ? down_rows : tile_rows, down_rows ? down_tiles.pool_tiles : tiles.pool_tiles};
   if ((rc = moe_gemm_gateup_impl(&routed_gateup, together ? &shared_gateup : nullptr, stream))) return join(rc);
   if ((rc = moe_gemm_down_impl(&routed_down, together ? &shared_down : nullptr, stream))) return join(rc);
   if ((rc = join(MOE_OK))) return rc;

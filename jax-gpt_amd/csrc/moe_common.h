@@ -336,11 +336,16 @@ struct QuantJob {
 };
 inline unsigned moe_quant_blocks(const QuantJob& q, int threads) { return (unsigned)((q.n_pieces + threads - 1) / threads); }
 int moe_quant_act_job(const void* x, int x_f32, void* x_bf16, int R, int K, uint8_t* xq, float* sx, float* sx_blocked, QuantJob* job);
+// Batches up to this many (token, slot) entries are one chunk, and their few, short row tiles are listed in plain
+// expert order with equal XCD shares.
+constexpr int kSmallRows = 2048;
 // What the sort by expert writes (sort_order, sorted_token_ids, inv_perm: null to skip; tl.tiles null: no work list).
 struct PermuteOut {
   int32_t *group_sizes, *group_offsets, *sorted_token_ids, *sort_order, *inv_perm;
   int k;
   TileList tl;
+  // a list of its own for the down GEMM, or null: it reads tl.  Batches of more than kSmallRows entries only; read by the host.
+  const TileList* tl_down;
 };
 // One routing call: the selection, and with it (optional) an activation quantisation and the sort by expert.
 struct RouteArgs {
@@ -388,6 +393,8 @@ struct TileShape {
   int dense_rows, dense_ncb[2];
 };
 int moe_gemm_tile_rows(const TileShape& t);
+// ... of the down GEMM's own list, where gate/up's list has tiles of list_rows, or 0: they share that one
+int moe_gemm_down_tile_rows(const TileShape& t, int list_rows);
 // the activation quantisers with an optional second copy of the scales, block-major in row order ((K/128, R): what
 // GemmScales{1, R} reads) -- spares the shared expert of a large batch the separate transposition
 // (x_f32: x holds f32 values, rounded to bf16 first)

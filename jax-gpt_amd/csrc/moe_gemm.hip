@@ -982,6 +982,22 @@ int moe_gemm_tile_rows(const TileShape& t) {
   return 32 * best_u;
 }
 
+// The two GEMMs want different heights where K of the down GEMM is short: tall tiles for gate/up, and for down 128 rows, which the kernel
+// with two workgroups a CU takes (moe_gemm_stream.hip), because start and end are a good part of an item of 6 or 8 K steps and another
+// workgroup works meanwhile.  The placing launch writes both lists, in two workgroups.  The down launch alone, gate/up's list / its own, even
+// routing or uneven by normal offsets of 1 and 2 on the logits: Qwen3-MoE (6 K steps), 400 tokens 39.6 / 36.5 us, 1000 47.0 / 41.4, 2000
+// 63.0 / 55.6 and 60.4 / 56.8 and 49.2 / 46.2, 3000 71.8 / 64.8; full layer (8), 1000 389 / 367, 2047 405 / 381, 312 / 307 and 188 / 180.
+//   The lines (the call, one list / two, routed as above): Qwen3-MoE, 300 tokens 123.4 / 120.0, 109.9 / 105.7 and 76.4 / 74.9, 3000 (188
+// rows an expert) 217.5 / 215.9, 231.7 / 221.2 and 218.1 / 206.7, 3800 (238) 241.6 / 245.3, 269.6 / 262.1 and 241.0 / 234.2, 5000 323.9 / 322.7,
+// 313.6 / 309.2 and 308.2 / 309.7; full layer, 900 tokens 1046 / 1025, 692 / 678 and 324 / 318, 3000 (59 rows) 1216 / 1200, 1034 /
+// 1033 and 668 / 667, 4096 (80) 1315 / 1299, 1191 / 1198 and 879 / 884; DeepSeek-V3 (16 K steps), 777 (24) 1376 / 1378, 1058 / 1082 and
+// 519 / 523.
+int moe_gemm_down_tile_rows(const TileShape& t, int list_rows) {
+  const int groups = t.E < t.R ? t.E : t.R;
+  if (t.R <= kSmallRows || t.R > kFullTileItems * kTileRows || list_rows <= kStreamRows || list_rows > kTileRows) return 0;
+  return (long long)groups * t.ncb[1] >= kStreamItems && t.kb[1] <= 8 && t.R <= (t.kb[1] <= 6 ? 200ll : 64ll) * t.E ? kStreamRows : 0;
+}
+
 // Batches whose GEMMs read the selection themselves: few rows of few experts whose launches are ones of the class kernel with plain
 // weight copies and tiles of up to 128 rows (a list's tiles may be allowed more where hardly any expert will have so many).
 int moe_gemm_scan_rows(const TileShape& t, bool from_memory) {

@@ -37,11 +37,14 @@ __global__ __launch_bounds__(kHistThreads) void hist_kernel(const int32_t* __res
   for (int e = threadIdx.x; e < E; e += kHistThreads) chunk_hist[(size_t)blockIdx.x * E + e] = hist[e];
 }
 
+// TWO: there is a second work list, l2, for the same experts (a kernel of its own: with both lists' arguments in all launches, and the
+// choice between them, Qwen3-MoE of 4096 tokens took 1.2 us more)
+template <bool TWO>
 __global__ __launch_bounds__(kPlaceThreads) void place_kernel(const int32_t* __restrict__ ids, int R, int E, int chunk,
                                                              int n_chunks, const int32_t* __restrict__ chunk_hist,
-                                                             const PermuteOut o, const QuantJob quant) {
+                                                             const PermuteOut o, const QuantJob quant, const TileList l2) {
   extern __shared__ int smem[];   // [waves][E]
-  if (n_chunks == 1) {
+  if (!TWO && n_chunks == 1) {
     if (blockIdx.x > 0) {   // the blocks behind quantise the activations (QuantJob)
       moe_quant_act_block(quant, (int)blockIdx.x - 1);
       return;
@@ -51,7 +54,10 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(const int32_t* __r
   }
   __shared__ int total[kMaxE], before[kMaxE];
   const int e = threadIdx.x;
-  const int c = (int)blockIdx.x - 1;   // chunk; workgroup 0 (started first) does the experts' side
+  // chunk; workgroup 0 (started first) does the experts' side, and one behind it the second list
+  const int c = (int)blockIdx.x - (TWO ? 2 : 1);
+  const bool second = TWO && blockIdx.x == 1;
+  const TileList l = second ? l2 : o.tl;
   total[e] = 0;
   before[e] = 0;
   const int first = c * chunk, n = c < 0 ? 0 : min(chunk, R - first);
@@ -79,17 +85,17 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(const int32_t* __r
   int row_start = rows, vote = o.tl.tile_rows > kTileRows ? moe_tall_vote(rows, moe_tall_tiles(R, E)) : 0, rows_all, votes;
   moe_scan_1024(row_start, vote, rows_all, votes);
   if (c < 0) {
-    if (e < E) {
+    if (!second && e < E) {
       o.group_sizes[e] = rows;
       o.group_offsets[e] = row_start;
       if (e == E - 1) o.group_offsets[E] = row_start + rows;
     }
-    zero_list_ends(rows_all, R, o);
-    if (o.tl.tiles) {   // the grouped GEMMs' row tiles, an expert's tiles side by side (uniform branch)
-      const int nt = moe_tile_count(rows, moe_tile_rows_voted(o.tl.tile_rows, votes));
-      const int at = moe_tile_first(e, rows, nt, total, before, o.tl);
+    if (!second) zero_list_ends(rows_all, R, o);
+    if (l.tiles) {   // the grouped GEMMs' row tiles, an expert's tiles side by side (uniform branch)
+      const int nt = moe_tile_count(rows, moe_tile_rows_voted(l.tile_rows, votes));
+      const int at = moe_tile_first(e, rows, nt, total, before, l);
       for (int t = 0; t < nt; ++t)
-        if (at + t < o.tl.max_tiles) o.tl.tiles[at + t] = TileEntry{e | nt << 10, row_start, rows, at};
+        if (at + t < l.max_tiles) l.tiles[at + t] = TileEntry{e | nt << 10, row_start, rows, at};
     }
     return;
   }
@@ -120,10 +126,11 @@ extern "C" size_t moe_permute_workspace_bytes(int M, int k, int E) {
 
 int moe_permute_place(const int32_t* idx, int R, int E, int chunk, int n_chunks, const int32_t* chunk_hist, const PermuteOut& o,
                       const QuantJob* quant, moe_stream_t stream) {
+  MOE_REQUIRE(n_chunks > 1 || !o.tl_down, MOE_ERR_BAD_SHAPE, "permute: a list of one chunk has no second work list");
   const bool places = R > 0 && (o.sorted_token_ids || o.sort_order || o.inv_perm);
-  const unsigned blocks = n_chunks > 1 ? (places ? n_chunks + 1 : 1) : 1 + (quant ? moe_quant_blocks(*quant, kPlaceThreads) : 0);
-  hipLaunchKernelGGL(place_kernel, dim3(blocks), dim3(kPlaceThreads), moe_place_lds_ints(E) * sizeof(int), (hipStream_t)stream,
-                     idx, R, E, chunk, n_chunks, chunk_hist, o, quant ? *quant : QuantJob{});
+  const unsigned blocks = n_chunks > 1 ? (places ? n_chunks : 0) + (o.tl_down ? 2 : 1) : 1 + (quant ? moe_quant_blocks(*quant, kPlaceThreads) : 0);
+  hipLaunchKernelGGL(o.tl_down ? place_kernel<true> : place_kernel<false>, dim3(blocks), dim3(kPlaceThreads), moe_place_lds_ints(E) * sizeof(int), (hipStream_t)stream,
+                     idx, R, E, chunk, n_chunks, chunk_hist, o, quant ? *quant : QuantJob{}, o.tl_down ? *o.tl_down : TileList{});
   return moe_check_hip(hipGetLastError(), "permute launch");
 }
 
@@ -131,7 +138,7 @@ extern "C" int moe_permute(const int32_t* idx, int M, int k, int E, int32_t* gro
                            int32_t* group_offsets, int32_t* sorted_token_ids, int32_t* sort_order,
                            int32_t* inv_perm, void* ws, size_t ws_bytes, moe_stream_t stream) {
   return moe_permute_impl(idx, M, k, E, PermuteOut{group_sizes, group_offsets, sorted_token_ids, sort_order, inv_perm, k,
-                                                   TileList{}}, ws, ws_bytes, nullptr, stream);
+                                                   TileList{}, nullptr}, ws, ws_bytes, nullptr, stream);
 }
 
 int moe_permute_impl(const int32_t* idx, int M, int k, int E, const PermuteOut& o, void* ws, size_t ws_bytes, const QuantJob* quant,

@@ -6,9 +6,6 @@
 constexpr int kMaxE = 1024;
 constexpr int kPlaceThreads = 1024;
 constexpr int kPlaceWaves = kPlaceThreads / MOE_WAVE;
-// Batches up to this many (token, slot) entries are one chunk, and their few, short row tiles are listed in plain
-// expert order with equal XCD shares.
-constexpr int kSmallRows = 2048;
 
 // waves that count and place: one counter per expert each, at most 32 KB of LDS in all
 __host__ __device__ inline int moe_place_waves(int E) { return E > 512 ? kPlaceWaves / 2 : kPlaceWaves; }

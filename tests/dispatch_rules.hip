@@ -18,6 +18,11 @@ int main() {
       TileShape t;
       std::cin >> t.R >> t.E >> t.max_rows >> t.ncb[0] >> t.ncb[1] >> t.kb[0] >> t.kb[1] >> t.dense_rows >> t.dense_ncb[0] >> t.dense_ncb[1];
       std::cout << moe_gemm_tile_rows(t) << "\n";
+    } else if (what == "down_list") {   // tokens, D, experts, k, I, SI: rows of a full tile of the lists, gate/up's and the down GEMM's own (or 0)
+      int M, D, E, k, I, SI;
+      std::cin >> M >> D >> E >> k >> I >> SI;
+      const TileShape t{M * k, E, M, {I / 128, (D + 255) / 256}, {D / 128, I / 128}, SI ? M : 0, {SI / 128, (D + 255) / 256}};
+      std::cout << moe_gemm_tile_rows(t) << " " << moe_gemm_down_tile_rows(t, moe_gemm_tile_rows(t)) << "\n";
     } else if (what == "scan") {   // tokens, D, experts, k, I, SI: rows of a full tile where the GEMMs read the selection, or 0
       int M, D, E, k, I, SI;
       std::cin >> M >> D >> E >> k >> I >> SI;

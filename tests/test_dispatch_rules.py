@@ -97,6 +97,17 @@ def test_two_k_steps_a_stage_are_for_workgroups_that_run_at_once(ask):
     assert [a[0] for a in ask(*[("stages", *c) for c in limits])] == list(limits.values())
 
 
+def test_the_down_gemm_of_short_k_has_a_list_of_its_own(ask):
+    """Tiles of 128 rows beside gate/up's full ones: more rows than one workgroup sorts, few K steps, enough items and not too many rows."""
+    from tests.test_gpu_variants import TWO_LISTS
+    want = {(256, 2048, 128, 8, 768, 0): "128 0", (257, 2048, 128, 8, 768, 0): "288 128", (3200, 2048, 128, 8, 768, 0): "288 128", (3201, 2048, 128, 8, 768, 0): "288 0",
+            (4096, 2048, 128, 8, 768, 0): "320 0", (819, 4096, 512, 10, 1024, 1024): "128 0", (820, 4096, 512, 10, 1024, 1024): "288 128",
+            (3276, 4096, 512, 10, 1024, 1024): "288 128", (3277, 4096, 512, 10, 1024, 1024): "288 0", (777, 7168, 256, 8, 2048, 2048): "288 0",
+            (2000, 2048, 128, 8, 1152, 0): "288 0"}
+    assert ask(*[("down_list", *c) for c in want]) == list(want.values())
+    assert ask(*[("down_list", *c[:6]) for c in TWO_LISTS]) == ["288 128"] * len(TWO_LISTS)
+
+
 def test_small_layers_read_the_selection_themselves(ask):
     """Few rows of few experts from the caches, in tiles of up to 128 rows; not where a list's tiles are taller for a reason, nor
     where the short-tile kernel takes the launch."""

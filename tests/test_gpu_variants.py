@@ -767,6 +767,41 @@ def test_small_layers_without_a_list_give_the_bits_of_the_sorted_rows(jg, M, D, 
     assert torch.equal(got, same) and not got[2].any()
 
 
+TWO_LISTS = [   # M, D, E, k, I, SI, offset
+    (1300, 1536, 128, 2, 768, 0, 0),      # 20 rows an expert: a tile each in both lists
+    (3000, 1536, 128, 8, 768, 256, 0),    # about 188: one of gate/up, two of down; a shared expert beside
+    (2100, 1792, 128, 6, 768, 0, 2),      # uneven: experts without rows and of several tiles of each kind; a half last column block
+    (2000, 256, 800, 8, 768, 0, 0.5),     # more experts than the routing launch counts for
+    (1500, 2048, 100, 4, 1024, 0, 0),     # as many K steps as there may be
+]
+
+
+@pytest.mark.parametrize("M,D,E,k,I,SI,offset", TWO_LISTS)
+def test_a_down_gemm_with_its_own_list_gives_the_bits_of_small_batches(jg, M, D, E, k, I, SI, offset):
+    """The same tokens in batches that one workgroup sorts, which have one list; and the rows of h and y that the two GEMMs share."""
+    import torch
+    print("two work lists", M, D, E, k, I, SI, offset, flush=True)
+    params, rand = _layer(jg, D, E, I, SI, M)
+    names = ("gate_proj", "up_proj", "down_proj")
+    kw = dict(top_k=k, experts={n: params[n] for n in names}, shared={n: params["shared_" + n] for n in names} if SI else None)
+    x, lg = rand(M, D), rand(M, E).float() + offset * rand(E).float()
+    got = jg.moe_experts(x, lg, **kw)
+    part = 2048 // k
+    for t in range(0, M, part):
+        want = jg.moe_experts(x[t:t + part].contiguous(), lg[t:t + part].contiguous(), **kw)
+        assert torch.equal(got[t:t + part], want), t
+    again, dbg = jg.moe_experts(x, lg, return_debug=True, **kw)
+    assert torch.equal(again, got)
+    idx = dbg["indices"].clone()
+    idx[::5, 1] = E   # no expert: the lists are shorter than the batch
+    w = torch.where(idx < E, dbg["weights"], 0.0)
+    if not SI:
+        full = jg.expert_forward_single(x, idx, w, *(params[n] for n in names))
+        for t in range(0, M, part):
+            assert torch.equal(full[t:t + part], jg.expert_forward_single(x[t:t + part].contiguous(), idx[t:t + part].contiguous(), w[t:t + part].contiguous(),
+                                                                          *(params[n] for n in names))), t
+
+
 SMALL_DOWN = [   # M, D, E, k, I, SI, selections a lane
     (17, 128, 1, 1, 128, 0, 1),        # one expert: units of 16 rows and of one
     (64, 256, 64, 1, 128, 128, 1),     # a workgroup's 64 selections, and a unit for nearly each; four of the shared expert
