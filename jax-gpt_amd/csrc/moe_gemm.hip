@@ -329,6 +329,18 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
     else if (C::is_s(i)) copy_s(kb + C::X_PRE, C::s_index(i));
     else copy_x(kb + C::X_PRE, C::x_index(i));
   };
+  // The item's weight block scales and the flags.  In front of the first copies, in their own order: a load behind them would be waited
+  // for with all of them, where the first step needs its own stage alone.
+  volatile int* early_flag = (volatile int*)(lds + CLS_FLAG_OFF);
+  if (C::W_EARLY && tid < 4) early_flag[tid] = 0;
+  const unsigned my_flag = lds0 + CLS_FLAG_OFF + wi * 4;
+  const float* wscale = (const float*)(lds + CLS_WSCALE_OFF);   // [2][MAX_KB]
+  if (wave < 2) {
+    const float* from = MODE == MODE_GATEUP ? (wave ? sw1 : sw0) + ((size_t)e * (N / 128) + item.col_block) * KB
+                                            : sw0 + ((size_t)e * (N / 128) + min(item.col_block * 2 + wave, N / 128 - 1)) * KB;
+    for (int kk = 0; kk < KB; kk += 64)
+      dma4((const uint8_t*)from, (unsigned)min(kk + lane, KB - 1) * 4u, lds0 + CLS_WSCALE_OFF + (wave * MAX_KB + kk) * 4u);
+  }
   if (xj == 0) {
     // what the steps before the first would have issued, in their order (completion is counted in issue order)
 #pragma unroll
@@ -341,20 +353,9 @@ __device__ __forceinline__ void item_body(const Item& item, uint8_t* lds, const 
     }
   }
 
-  volatile int* early_flag = (volatile int*)(lds + CLS_FLAG_OFF);
-  if (C::W_EARLY && tid < 4) early_flag[tid] = 0;
-  const unsigned my_flag = lds0 + CLS_FLAG_OFF + wi * 4;
-  float* wscale = (float*)(lds + CLS_WSCALE_OFF);
-  for (int i = tid; i < 2 * KB; i += NT) {
-    const int h = i >= KB, kk = h ? i - KB : i;
-    float v;
-    if (MODE == MODE_GATEUP) v = (h ? sw1 : sw0)[((size_t)e * (N / 128) + item.col_block) * KB + kk];
-    else v = sw0[((size_t)e * (N / 128) + min(item.col_block * 2 + h, N / 128 - 1)) * KB + kk];
-    wscale[h * MAX_KB + kk] = v;
-  }
   const float* ws0 = wscale + (MODE == MODE_GATEUP ? 0 : (wi >> 1) * MAX_KB);
   const float* ws1 = wscale + MAX_KB;   // GATEUP only
-  __syncthreads();   // (the compiler waits here for the scale loads, and with them for the copies issued above)
+  wait_lgkm0();   // (the flags are there when the first step's barrier is passed)
 
   const int lane_off0 = fr * BK + ((fq ^ (fr >> 1)) << 4);         // K bytes [16 fq, +16)
   const int lane_off1 = fr * BK + (((fq + 4) ^ (fr >> 1)) << 4);   // K bytes [64 + 16 fq, +16)
