@@ -30,13 +30,13 @@ COMMON = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-
           "-fvisibility=hidden",    # only the functions include/moe_hip.h declares (MOE_API) are exported
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
           "-I", os.path.join(ROOT, "include"), "-I", CSRC]
-# routing and combine promise individually rounded f32 operations (bit-reproducible on a CPU)
+# routing (also of single tokens, moe_token.hip) and combine promise individually rounded f32 operations (bit-reproducible on a CPU)
 PER_FILE = {"moe_route.hip": ["-ffp-contract=off"], "moe_combine.hip": ["-ffp-contract=off"],
             "moe_router.hip": ["-ffp-contract=off", "-Wno-inline-asm"],
             # MFMA results go straight to VGPRs: the block-scale FMA consumes them on the vector ALU
             "moe_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-Wno-inline-asm"],   # m0 is clobbered on purpose
             "moe_gemm_stream.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-Wno-inline-asm"],
-            "moe_token.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-Wno-inline-asm"],
+            "moe_token.hip": ["-ffp-contract=off", "-mllvm", "-amdgpu-mfma-vgpr-form", "-Wno-inline-asm"],
             "moe_small.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-Wno-inline-asm"]}
 
 

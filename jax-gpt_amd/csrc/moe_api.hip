@@ -319,15 +319,20 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
     if (a->SI && (rc = moe_gemm_check(shared_down.op, a->M, 1, true))) return rc;
     MOE_REQUIRE(MOE_ALIGNED16(a->out) && (!a->add_residual || MOE_ALIGNED16(a->x)), MOE_ERR_BAD_ALIGN,
                 "combine: pointers must be 16-byte aligned");
+    const bool from_memory = moe_gemm_from_memory(((long long)a->E * a->I + a->SI) * a->D);
+    const bool fronts = front && moe_token_fronts(a->M, a->k, a->I, a->SI, a->norm_weight, from_memory);
+    const bool routes = carried && !given_idx && !a->w_router && !io_f32 && moe_token_routes(a->M, a->D, a->E, a->k, a->I, a->SI);
+    TokenRoute tok_route{a->routing, route, a->x, fronts ? &front_args : nullptr};
     if (given_idx) rc = carried ? moe_quant_act_impl(a->x, io_f32, nullptr, a->M, a->D, b.xq, b.sx, nullptr, stream) : MOE_OK;
-    else rc = select(nullptr);
+    else if (fronts) rc = moe_front_check(a->routing, tok_route.args, front_args, false);
+    else rc = routes ? moe_route_check(a->routing, route) : select(nullptr);
     if (rc) return rc;
     const TokenArgs tok{b.xq, b.sx, given_idx ? given_idx : idx, w,
                         TokenExperts{a->w_gate, a->w_up, a->w_down, a->sw_gate, a->sw_up, a->sw_down},
                         TokenExperts{a->ws_gate, a->ws_up, a->ws_down, a->sws_gate, a->sws_up, a->sws_down},
                         a->M, a->D, a->E, a->k, a->I, a->SI, b.h32, a->I > a->SI ? a->I : a->SI,
                         shared_gate, a->add_residual ? a->x : nullptr, io_f32, a->out};
-    return moe_token_experts(tok, moe_gemm_from_memory(((long long)a->E * a->I + a->SI) * a->D), stream);
+    return moe_token_experts(tok, from_memory, fronts || routes ? &tok_route : nullptr, stream);
   }
   // routing, the sort by expert and the routed GEMMs' work list (the sort holds every expert's row range anyway)
   TileList tiles;

@@ -357,6 +357,7 @@ struct RouteArgs {
   int32_t* idx;
   float* w;
 };
+int moe_route_check(int routing, const RouteArgs& a);   // what the routing launches refuse
 int moe_route_impl(int routing, const RouteArgs& a, const QuantJob* quant, const PermuteOut* sort, void* permute_ws,
                    size_t permute_ws_bytes, moe_stream_t stream);
 // The same behind the router's matmul, the quantiser and, with norm, the RMSNorm, all in its one launch (small routers; N: columns
@@ -371,6 +372,7 @@ struct FrontArgs {
   float *sx, *sx_blocked;
 };
 bool moe_front_takes(int M, int D, int E, int N, bool norm, bool x_f32, bool sorted);   // sorted: a sort of the selections follows
+int moe_front_check(int routing, RouteArgs& a, const FrontArgs& f, bool sorted);   // what the launch refuses; completes a.src
 int moe_front_impl(int routing, RouteArgs a, const FrontArgs& f, const PermuteOut* sort, void* permute_ws, size_t permute_ws_bytes,
                    moe_stream_t stream);
 // chunks of the flat list that get a histogram each, at most

@@ -12,230 +12,9 @@
 #include "moe_common.h"
 #include "moe_permute_device.h"
 #include "moe_quant_device.h"
+#include "moe_route_device.h"
 
 namespace {
-
-// 32-bit keys: larger key = larger value (-0 equals +0); 0 = absent
-__device__ __forceinline__ unsigned make_key(float v) {
-  const unsigned u = __float_as_uint(v + 0.0f);  // -0 -> +0
-  return max((u & 0x80000000u) ? ~u : (u | 0x80000000u), 1u);   // (a NaN of all ones is still present)
-}
-__device__ __forceinline__ float key_value(unsigned u) {
-  return __uint_as_float((u & 0x80000000u) ? (u & 0x7fffffffu) : ~u);
-}
-
-// Lane permutations inside a row of 16 lanes (DPP, a few cycles each): xor 1, xor 2, mirror of 8, mirror of 16 -- a
-// maximum does not care which partner it meets, only that the set closes.  Reductions over ds_bpermute cost about
-// 100 cycles per step, and routing is a chain of reductions.
-template <int CTRL> __device__ __forceinline__ unsigned dpp(unsigned v) {
-  return (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xF, 0xF, false);
-}
-constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_MIRROR8 = 0x141, DPP_MIRROR16 = 0x140, DPP_ROR4 = 0x124, DPP_ROR8 = 0x128;
-
-// wave-wide maximum, as a scalar: row maxima by DPP, the four rows as scalars
-__device__ __forceinline__ unsigned wave_max(unsigned k) {
-  k = max(k, dpp<DPP_XOR1>(k));
-  k = max(k, dpp<DPP_XOR2>(k));
-  k = max(k, dpp<DPP_MIRROR8>(k));
-  k = max(k, dpp<DPP_MIRROR16>(k));
-  const unsigned a = (unsigned)__builtin_amdgcn_readlane((int)k, 0), b = (unsigned)__builtin_amdgcn_readlane((int)k, 16);
-  const unsigned c = (unsigned)__builtin_amdgcn_readlane((int)k, 32), d = (unsigned)__builtin_amdgcn_readlane((int)k, 48);
-  return max(max(a, b), max(c, d));
-}
-// The two largest of a set of keys, equal ones counted: meet() joins disjoint sets.
-struct TwoBest {
-  unsigned m1 = 0u, m2 = 0u;
-  __device__ __forceinline__ void meet(unsigned o1, unsigned o2) {
-    m2 = max(min(m1, o1), max(m2, o2));
-    m1 = max(m1, o1);
-  }
-  template <int CTRL> __device__ __forceinline__ void meet_dpp() { meet(dpp<CTRL>(m1), dpp<CTRL>(m2)); }
-  __device__ __forceinline__ void meet_wave() {   // of all lanes' sets, as scalars
-    meet_dpp<DPP_XOR1>();
-    meet_dpp<DPP_XOR2>();
-    meet_dpp<DPP_MIRROR8>();
-    meet_dpp<DPP_MIRROR16>();
-    const unsigned r1 = m1, r2 = m2;
-    m1 = m2 = 0u;
-#pragma unroll
-    for (int row = 0; row < 64; row += 16)
-      meet((unsigned)__builtin_amdgcn_readlane((int)r1, row), (unsigned)__builtin_amdgcn_readlane((int)r2, row));
-  }
-};
-// wave-wide sum in the pairing of a butterfly (partner lane ^ 32, 16, 8, 4, 2, 1), which fixes the rounding.  After the
-// step over 8 lanes i and i ^ 8 hold the same value, so a rotation by 4 meets what lane ^ 4 holds.
-__device__ __forceinline__ float wave_sum_f32(float v) {
-  v = __fadd_rn(v, __shfl_xor(v, 32, MOE_WAVE));
-  v = __fadd_rn(v, __shfl_xor(v, 16, MOE_WAVE));
-  v = __fadd_rn(v, __uint_as_float(dpp<DPP_ROR8>(__float_as_uint(v))));
-  v = __fadd_rn(v, __uint_as_float(dpp<DPP_ROR4>(__float_as_uint(v))));
-  v = __fadd_rn(v, __uint_as_float(dpp<DPP_XOR2>(__float_as_uint(v))));
-  v = __fadd_rn(v, __uint_as_float(dpp<DPP_XOR1>(__float_as_uint(v))));
-  return v;
-}
-__device__ __forceinline__ float lane_f32(float v, int lane) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-
-// the k best of the wave's keys in order, ties to the lower index.  BLOCKED: element e lives in lane e / VPL, slot
-// e % VPL; otherwise in lane e % 64, slot e / 64.  Lane i keeps the i-th: its index, key and (SCORES) score.
-template <int VPL, bool BLOCKED, bool SCORES>
-__device__ __forceinline__ void select_topk(unsigned (&key)[VPL], const float* score, int k, int& my_idx, unsigned& my_key,
-                                            float& my_score) {
-  const int lane = threadIdx.x & 63;
-  for (int sel = 0; sel < k; ++sel) {
-    unsigned local = key[0];
-#pragma unroll
-    for (int s = 1; s < VPL; ++s) local = max(local, key[s]);
-    const unsigned best = wave_max(local);
-    int owner = 0, slot = 0;
-    if (BLOCKED) {
-      owner = (int)__builtin_ctzll(__ballot(local == best));
-#pragma unroll
-      for (int s = VPL - 1; s >= 0; --s)
-        if ((unsigned)__builtin_amdgcn_readlane((int)key[s], owner) == best) slot = s;
-    } else {
-#pragma unroll
-      for (int s = VPL - 1; s >= 0; --s) {
-        const unsigned long long in = __ballot(key[s] == best);
-        if (in) owner = (int)__builtin_ctzll(in), slot = s;
-      }
-    }
-    float sv = 0.f;
-#pragma unroll
-    for (int s = 0; s < VPL; ++s) {
-      if (SCORES) {
-        const float v = lane_f32(score[s], owner);
-        sv = s == slot ? v : sv;
-      }
-      if (s == slot && lane == owner) key[s] = 0u;
-    }
-    if (lane == sel) {
-      my_idx = BLOCKED ? owner * VPL + slot : owner + 64 * slot;
-      my_key = best;
-      my_score = sv;
-    }
-  }
-}
-// sum of the first k lanes' values in lane order
-__device__ __forceinline__ float sum_first(float v, int k) {
-  float s = 0.f;
-  for (int i = 0; i < k; ++i) s = __fadd_rn(s, lane_f32(v, i));
-  return s;
-}
-
-constexpr int ROUTE_SOFTMAX = MOE_ROUTING_SOFTMAX, ROUTE_GROUPED = MOE_ROUTING_SIGMOID_GROUPED;
-
-// One token's selection by one wave.  row: its logits (global memory or LDS).  Returns the chosen expert (lane < k).
-template <int VPL>
-__device__ __forceinline__ int route_softmax_token(const RouteArgs& a, const float* row, int t) {
-  const int lane = threadIdx.x & 63;
-  float v[VPL];
-  unsigned key[VPL], top = 0u;
-#pragma unroll
-  for (int s = 0; s < VPL; ++s) {
-    const int e = lane + 64 * s;
-    v[s] = e < a.E ? row[e] : -INFINITY;
-    key[s] = e < a.E ? make_key(v[s]) : 0u;
-    top = max(top, v[s] == v[s] ? key[s] : 0u);   // (a NaN ranks like any other value but is nobody's maximum: see below)
-  }
-  // A NaN logit counts as exp_det's lower end and leaves the other experts' weights alone; as the maximum it would make
-  // every difference a NaN, every exponential that lower end, and all k weights equal.
-  const float mx = key_value(wave_max(top));
-  float part = 0.f;
-#pragma unroll
-  for (int s = 0; s < VPL; ++s)
-    if (lane + 64 * s < a.E) part = __fadd_rn(part, exp_det(__fsub_rn(v[s], mx)));
-  const float denom = wave_sum_f32(part);
-  int my_idx = 0;
-  unsigned my_key = 0u;
-  float unused;
-  select_topk<VPL, false, false>(key, nullptr, a.k, my_idx, my_key, unused);
-  const float p = __fdiv_rn(exp_det(__fsub_rn(key_value(my_key), mx)), denom);
-  const float psum = sum_first(p, a.k);
-  if (lane < a.k) {
-    a.idx[(size_t)t * a.k + lane] = my_idx;
-    a.w[(size_t)t * a.k + lane] = a.renorm ? __fdiv_rn(p, psum) : p;
-  }
-  return my_idx;
-}
-
-template <int VPL>
-__device__ __forceinline__ int route_grouped_token(const RouteArgs& a, const float* row, int t) {
-  const int lane = threadIdx.x & 63, E = a.E, n_group = a.n_group;
-  float score[VPL];
-  unsigned key[VPL];
-#pragma unroll
-  for (int s = 0; s < VPL; ++s) {
-    const int e = lane * VPL + s;
-    const bool ok = e < E;
-    score[s] = ok ? sigmoid_det(row[e]) : 0.f;
-    const float choice = __fadd_rn(score[s], (ok && a.bias) ? a.bias[e] : 0.f);
-    key[s] = ok ? make_key(choice) : 0u;
-  }
-  if (a.topk_group < n_group) {
-    // group score = sum of the two best choice scores of the group; a group is kept if fewer than topk_group of the
-    // groups score higher (ties: lower index)
-    const int per = E / n_group, lpg = per / VPL;   // experts and lanes per group
-    if (lpg * VPL == per && (lpg & (lpg - 1)) == 0 && lpg >= 1 && lpg <= 16 && per >= 2) {
-      // every group is a run of 1, 2, 4, 8 or 16 lanes: all groups' two best at once, by DPP
-      TwoBest best;
-#pragma unroll
-      for (int s = 0; s < VPL; ++s) best.meet(key[s], 0u);
-      if (lpg > 1) best.meet_dpp<DPP_XOR1>();
-      if (lpg > 2) best.meet_dpp<DPP_XOR2>();
-      if (lpg > 4) best.meet_dpp<DPP_MIRROR8>();
-      if (lpg > 8) best.meet_dpp<DPP_MIRROR16>();
-      const int g = lane / lpg;
-      const unsigned gkey = make_key(__fadd_rn(key_value(best.m1), key_value(best.m2)));
-      int rank = 0;
-      for (int o = 0; o < n_group; ++o) {
-        const unsigned ok = (unsigned)__builtin_amdgcn_readlane((int)gkey, o * lpg);
-        rank += (ok > gkey || (ok == gkey && o < g)) ? 1 : 0;
-      }
-      const bool keep = rank < a.topk_group;
-#pragma unroll
-      for (int s = 0; s < VPL; ++s) key[s] = keep ? key[s] : 0u;
-    } else {
-      // groups that lie across lanes in any way: one at a time (lane g keeps group g's score).  (The second best as a
-      // second maximum over what lies below the first, with a count of the equals: 8192 tokens of 640 experts in 4
-      // groups 52 us, 46 this way.)
-      unsigned gkey = 0u;
-      int gid[VPL];
-#pragma unroll
-      for (int s = 0; s < VPL; ++s) gid[s] = lane * VPL + s < E ? (lane * VPL + s) / per : -1;
-      for (int g = 0; g < n_group; ++g) {
-        TwoBest best;
-#pragma unroll
-        for (int s = 0; s < VPL; ++s) best.meet(gid[s] == g ? key[s] : 0u, 0u);
-        best.meet_wave();
-        float gs = key_value(best.m1);
-        if (per >= 2) gs = __fadd_rn(gs, key_value(best.m2));
-        if (lane == g) gkey = make_key(gs);
-      }
-      int rank = 0;
-      for (int o = 0; o < n_group; ++o) {
-        const unsigned ok = (unsigned)__builtin_amdgcn_readlane((int)gkey, o);
-        rank += (ok > gkey || (ok == gkey && o < lane)) ? 1 : 0;
-      }
-      const unsigned long long keep = __ballot(lane < n_group && rank < a.topk_group);   // bit g set = group g kept
-#pragma unroll
-      for (int s = 0; s < VPL; ++s)
-        if (gid[s] < 0 || !((keep >> gid[s]) & 1ull)) key[s] = 0u;
-    }
-  }
-  int my_idx = 0;
-  unsigned my_key = 0u;
-  float my_w = 0.f;
-  select_topk<VPL, true, true>(key, score, a.k, my_idx, my_key, my_w);
-  const float wsum = sum_first(my_w, a.k);
-  if (lane < a.k) {
-    const float r = a.renorm ? __fdiv_rn(my_w, __fadd_rn(wsum, 1e-20f)) : my_w;
-    a.idx[(size_t)t * a.k + lane] = my_idx;
-    a.w[(size_t)t * a.k + lane] = __fmul_rn(r, a.routed_scale);
-  }
-  return my_idx;
-}
 
 // Columns [0, n) of the partial sums at p, added in slice order by the whole workgroup and rounded to bf16 (what the
 // router's own finishing pass computes).  The loads are what it waits for, so a thread has up to 8 slices of C columns
@@ -324,7 +103,7 @@ __global__ __launch_bounds__(1024) void route_kernel(const RouteArgs a, const Ro
         if (lane == 0 && a.src.shared_gate && N > a.E)   // the shared expert's gate rides in column E
           a.src.shared_gate[t] = bf16_to_f32(f32_to_bf16(sigmoid_det(row[a.E])));
       }
-      const int chosen = KIND == ROUTE_SOFTMAX ? route_softmax_token<VPL>(a, row, t) : route_grouped_token<VPL>(a, row, t);
+      const int chosen = KIND == ROUTE_SOFTMAX ? route_softmax_token<VPL>(a, row, t).expert : route_grouped_token<VPL>(a, row, t).expert;
       if (lane < a.k) {
         if (!SORT_HERE && job.chunk_hist) atomicAdd(&hist[chosen], 1);
         if (SORT_HERE) ids[t * a.k + lane] = chosen;
@@ -467,7 +246,7 @@ __global__ __launch_bounds__(64 * kFrontWaves) void front_kernel(const RouteArgs
     const float* row = rows + tt * N;
     if (a.src.out_logits && lane < E) a.src.out_logits[(size_t)(t0 + tt) * E + lane] = row[lane];
     if (lane == 0 && a.src.shared_gate && N > E) a.src.shared_gate[t0 + tt] = bf16_to_f32(f32_to_bf16(sigmoid_det(row[E])));
-    const int chosen = KIND == ROUTE_SOFTMAX ? route_softmax_token<1>(a, row, t0 + tt) : route_grouped_token<1>(a, row, t0 + tt);
+    const int chosen = KIND == ROUTE_SOFTMAX ? route_softmax_token<1>(a, row, t0 + tt).expert : route_grouped_token<1>(a, row, t0 + tt).expert;
     if (f.chunk_hist && lane < a.k) atomicAdd(&hist[chosen], 1);
   }
   if (f.xq) {   // (nobody in this launch waits for the codes)
@@ -509,7 +288,9 @@ __global__ __launch_bounds__(64 * kFrontWaves) void front_kernel(const RouteArgs
 
 constexpr int kCUs = 256;
 
-int check_route_args(int routing, const RouteArgs& a) {
+}  // namespace
+
+int moe_route_check(int routing, const RouteArgs& a) {
   const LogitSource& src = a.src;
   const int M = a.M, E = a.E, k = a.k;
   MOE_REQUIRE(M == 0 || ((src.logits || src.partial) && a.idx && a.w), MOE_ERR_NULL, "route: null pointer");
@@ -527,6 +308,8 @@ int check_route_args(int routing, const RouteArgs& a) {
   return MOE_OK;
 }
 
+namespace {
+
 template <int KIND, bool SORT_HERE>
 void launch_route(int vpl, dim3 grid, dim3 block, size_t lds, hipStream_t s, const RouteArgs& a, const RouteJob& job,
                   const QuantJob& q, const PermuteOut& o) {
@@ -541,7 +324,7 @@ void launch_route(int vpl, dim3 grid, dim3 block, size_t lds, hipStream_t s, con
 
 int moe_route_impl(int routing, const RouteArgs& a, const QuantJob* quant, const PermuteOut* sort, void* permute_ws,
                    size_t permute_ws_bytes, moe_stream_t stream) {
-  if (int rc = check_route_args(routing, a)) return rc;
+  if (int rc = moe_route_check(routing, a)) return rc;
   MOE_REQUIRE((!quant && !sort) || a.M > 0, MOE_ERR_BAD_SHAPE, "route: nothing to carry a quantisation or a sort with");
   MOE_REQUIRE(!sort || (permute_ws && permute_ws_bytes >= moe_permute_workspace_bytes(a.M, a.k, a.E)), MOE_ERR_WORKSPACE_TOO_SMALL,
               "route: permutation workspace too small");
@@ -619,15 +402,19 @@ bool moe_front_takes(int M, int D, int E, int N, bool norm, bool x_f32, bool sor
   if (M < 1 || E > kFrontExperts || D < 128 || D > kFrontD || D % 128 || moe_router_k_slice(M, N, D) != 128) return false;
   return M <= kFrontTokens * kCUs || (M <= 32768 && !norm && (!sorted || x_f32 || D <= 512));
 }
-int moe_front_impl(int routing, RouteArgs a, const FrontArgs& f, const PermuteOut* sort, void* permute_ws, size_t permute_ws_bytes,
-                   moe_stream_t stream) {
+int moe_front_check(int routing, RouteArgs& a, const FrontArgs& f, bool sorted) {
   const int N = a.E + (f.w_shared_gate ? 1 : 0);
   MOE_REQUIRE(f.x && f.w_router && (!f.w_shared_gate || a.src.shared_gate) && (!f.xq || f.sx), MOE_ERR_NULL, "router: null pointer");
   MOE_REQUIRE(MOE_ALIGNED16(f.x) && MOE_ALIGNED16(f.w_router) && MOE_ALIGNED16(f.w_shared_gate) && MOE_ALIGNED16(f.norm) && MOE_ALIGNED16(f.xq),
               MOE_ERR_BAD_ALIGN, "router: pointers must be 16-byte aligned");
-  MOE_REQUIRE(moe_front_takes(a.M, f.D, a.E, N, f.norm, f.x_f32, sort), MOE_ERR_BAD_SHAPE, "router: not a call for this launch (M=%d D=%d N=%d)", a.M, f.D, N);
+  MOE_REQUIRE(moe_front_takes(a.M, f.D, a.E, N, f.norm, f.x_f32, sorted), MOE_ERR_BAD_SHAPE, "router: not a call for this launch (M=%d D=%d N=%d)", a.M, f.D, N);
   a.src.logits = nullptr, a.src.partial = (const float*)f.w_router, a.src.splits = 1, a.src.N = N;   // (no logits are given, and none are in memory)
-  if (int rc = check_route_args(routing, a)) return rc;
+  return moe_route_check(routing, a);
+}
+int moe_front_impl(int routing, RouteArgs a, const FrontArgs& f, const PermuteOut* sort, void* permute_ws, size_t permute_ws_bytes,
+                   moe_stream_t stream) {
+  if (int rc = moe_front_check(routing, a, f, sort)) return rc;
+  const int N = a.src.N;
   MOE_REQUIRE(!sort || (permute_ws && permute_ws_bytes >= moe_permute_workspace_bytes(a.M, a.k, a.E)), MOE_ERR_WORKSPACE_TOO_SMALL,
               "route: permutation workspace too small");
   MOE_REQUIRE((long long)a.M * a.k < (1ll << 31), MOE_ERR_BAD_SHAPE, "route: M*k overflows int32");

@@ -17,7 +17,10 @@
 // K step, one token of DeepSeek-V3: rings of 2 / 3 / 4 / 6 75.6 / 76.8 / 78.1 / 88.2 in the first launch; in the second 2 / 3 are
 // even and 4 / 8 are 7 and 23 % slower).  Workgroups of four waves in the first: 85.8, as 288 of them are uneven on 256 CUs.
 #include "moe_token.h"
+#include "moe_route_device.h"
 
+//   Where all workgroups of the first launch run at once they route, and quantise, their token themselves (token_route_gateup_kernel,
+// token_front_gateup_kernel): the same work in each, but on otherwise idle CUs, and one launch less.
 //   Nothing that a wave has to wait for stands behind the weights' copies, which complete in order with everything else: codes and scales
 // are copied to LDS in front of them, and the second launch's wave has its whole row of h in registers (2048 values at a time) while the
 // selection's index travels, and quantises it while the first weights do.  With loads through registers behind the copies, and h piece by
@@ -25,6 +28,7 @@
 // 11.8, of the mini layer behind its norm 15.3 -> 15.0; 8 tokens of 2 of 8 experts of 1024 x 256 beside one of 4096 30.6 -> 24.2.
 namespace {
 
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 constexpr int BK = 128;
 constexpr int COLS = 16;         // output columns of a wave
 constexpr int STAGES = 2;        // of a wave's ring
@@ -109,7 +113,7 @@ struct WaveRows {
 #pragma unroll
         for (int f = 0; f < FRAGS; ++f) {
           const v4f p = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[i][f], xf, (v4f){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
-          acc[f] += p * scale(kb, f);
+          acc[f] = __builtin_elementwise_fma(p, (v4f)(scale(kb, f)), acc[f]);
         }
       }
     }
@@ -125,44 +129,212 @@ __device__ __forceinline__ void copy_floats(const float* from, int n, unsigned t
   for (int i = 0; i < n; i += 64) dma4((const uint8_t*)from, min(i + (int)threadIdx.x % 64, n - 1) * 4u, to + i * 4u);
 }
 
+// What a wave of the first launch does once its expert is known.  lds: ring, codes, [2] weights' scales (up_lds); the row's scales at sx
+template <bool ONCE, int KS>
+struct GateUpTile {
+  const TokenArgs& a;
+  int t, slot, col;
+  bool shared;
+  uint8_t* lds;
+  WaveRows<2, ONCE, KS> rows;
+  float *sx, *sw;   // sw: [2][up_scales / 4]
+
+  // Workgroup b of a token's: its slot and columns
+  __device__ __forceinline__ GateUpTile(const TokenArgs& args, int b, int token, uint8_t* base, int codes_bytes) : a(args), t(token), lds(base) {
+    const int per = a.I / COLS;
+    shared = b >= a.k * per;
+    slot = shared ? a.k : b / per, col = (b - slot * per) * COLS;
+    sx = (float*)(base + STAGES * 32 * BK * KS + codes_bytes), sw = sx + up_scales(a.D) / 4;
+  }
+  __device__ __forceinline__ uint8_t* codes() const { return lds + STAGES * 32 * BK * KS; }
+  static __device__ __forceinline__ unsigned address(const void* p) { return __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)p); }
+  __device__ __forceinline__ void start(int e) {
+    const TokenExperts& x = shared ? a.shared : a.routed;
+    const int N = shared ? a.SI : a.I, KB = a.D / BK;
+    const size_t block = ((size_t)e * (N / BK) + col / BK) * KB;
+    copy_floats(x.s_gate + block, KB, address(sw));
+    copy_floats(x.s_up + block, KB, address(sw) + up_scales(a.D));
+    const size_t row = ((size_t)e * N + col) * a.D;
+    rows.start({x.w_gate + row, x.w_up + row}, a.D, 1, 0, address(lds));
+  }
+  __device__ __forceinline__ void finish() {
+    const int lane = threadIdx.x & 63, per_scale = up_scales(a.D) / 4;
+    v4f acc[2] = {};
+    const float *rs = sx, *ws = sw;
+    rows.run(lds, codes(), acc, [&](int kb, int f) { return rs[kb] * ws[f * per_scale + kb]; });
+    v4f h;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float g = acc[0][r], u = acc[1][r];
+      h[r] = g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u;
+    }
+    if ((lane & 15) == 0) *(v4f*)(a.h + ((size_t)t * (a.k + 1) + slot) * a.h_stride + col + (lane >> 4) * 4) = h;
+  }
+};
+
 template <bool ONCE, int KS>
 __global__ __launch_bounds__(64) void token_gateup_kernel(const TokenArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int lane = threadIdx.x, t = blockIdx.y;
-  const int per = a.I / COLS, b = blockIdx.x, KB = a.D / BK;
-  const bool shared = b >= a.k * per;
-  const int slot = shared ? a.k : b / per, col = (b - slot * per) * COLS;
-  const TokenExperts& x = shared ? a.shared : a.routed;
-  const int N = shared ? a.SI : a.I;
-  const int chosen = shared ? 0 : a.idx[(size_t)t * a.k + slot];
-  uint8_t* codes = lds + STAGES * 32 * BK * KS;
-  float* sx = (float*)(codes + up_codes(a.D));
-  const int per_scale = up_scales(a.D) / 4;
-  float* sw = sx + per_scale;   // [2][per_scale]
+  GateUpTile<ONCE, KS> tile(a, blockIdx.x, t, lds, up_codes(a.D));
+  const int chosen = tile.shared ? 0 : a.idx[(size_t)t * a.k + tile.slot];
   // everything is copied by the wave itself, in the order of its use: what does not depend on the expert while its index travels
-  const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)lds), sx_at = lds0 + STAGES * 32 * BK * KS + up_codes(a.D);
-  for (int i = 0; i < a.D; i += 1024) dma16(a.xq + (size_t)t * a.D, min(i + lane * 16, a.D - 16), lds0 + STAGES * 32 * BK * KS + i);
-  copy_floats(a.sx + (size_t)t * KB, KB, sx_at);
+  const unsigned codes_at = tile.address(tile.codes());
+  for (int i = 0; i < a.D; i += 1024) dma16(a.xq + (size_t)t * a.D, min(i + lane * 16, a.D - 16), codes_at + i);
+  copy_floats(a.sx + (size_t)t * (a.D / BK), a.D / BK, tile.address(tile.sx));
   const int e = __builtin_amdgcn_readfirstlane(chosen);
-  if (!shared && (unsigned)e >= (unsigned)a.E) {   // (an index out of range: the second launch leaves its row out)
+  if (!tile.shared && (unsigned)e >= (unsigned)a.E) {   // (an index out of range: the second launch leaves its row out)
     wait_copies<0>();   // (none may land in LDS that is another workgroup's)
     return;
   }
-  const size_t block = ((size_t)e * (N / BK) + col / BK) * KB;
-  copy_floats(x.s_gate + block, KB, sx_at + per_scale * 4);
-  copy_floats(x.s_up + block, KB, sx_at + per_scale * 8);
-  const size_t row = ((size_t)e * N + col) * a.D;
-  WaveRows<2, ONCE, KS> rows;
-  rows.start({x.w_gate + row, x.w_up + row}, a.D, 1, 0, lds0);
-  v4f acc[2] = {};
-  rows.run(lds, codes, acc, [&](int kb, int f) { return sx[kb] * sw[f * per_scale + kb]; });
-  v4f h;
+  tile.start(e);
+  tile.finish();
+}
+
+// A piece of eight values of a token's row to its codes, scale and LDS; 16 lanes a group (moe_quant_act_block)
+__device__ __forceinline__ void quant_piece(const moe_bf16x8& in, int p, uint8_t* codes, float* sx) {
+  float v[8], amax = 0.f;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const float g = acc[0][r], u = acc[1][r];
-    h[r] = g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u;
+  for (int i = 0; i < 8; ++i) {
+    v[i] = bf16_to_f32(in.v[i]);
+    amax = fmaxf(amax, fabsf(v[i]));
   }
-  if ((lane & 15) == 0) *(v4f*)(a.h + ((size_t)t * (a.k + 1) + slot) * a.h_stride + col + (lane >> 4) * 4) = h;
+  unsigned m = __float_as_uint(amax);   // (not negative: ordered as integers)
+  m = max(m, dpp<DPP_XOR1>(m));
+  m = max(m, dpp<DPP_XOR2>(m));
+  m = max(m, dpp<DPP_MIRROR8>(m));
+  m = max(m, dpp<DPP_MIRROR16>(m));
+  float scale, scale_inv;
+  fp8_scales(__uint_as_float(m), scale, scale_inv);
+  uint2 out;
+  out.x = pack4_e4m3(v[0] * scale, v[1] * scale, v[2] * scale, v[3] * scale);
+  out.y = pack4_e4m3(v[4] * scale, v[5] * scale, v[6] * scale, v[7] * scale);
+  ((uint2*)codes)[p] = out;
+  if ((p & 15) == 0) sx[p >> 4] = scale_inv;
+}
+// LDS writes of all waves are there; the copies stay under way
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// The same with the token's routing and quantisation in front, from ready logits: the first wave selects its token's experts itself
+// and streams their weights, the others quantise the token meanwhile (rows above 4096: two of them).  What it waits for is the
+// selection's chain of dependent steps, as the launch before did, without that launch's end and this one's start.  One token of
+// DeepSeek-V3, launch by launch 71.0 us a call; this way with the selecting wave quantising behind its first copies 71.0 (110
+// instructions for 512 values), with one wave for that 70.2, with two 68.5, three 68.8.
+template <int KIND, int VPL, bool ONCE, int KS>
+__global__ __launch_bounds__(192) void token_route_gateup_kernel(const TokenArgs a, const RouteArgs r, const bf16_t* x) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const int lane = threadIdx.x & 63, t = blockIdx.y, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  GateUpTile<ONCE, KS> tile(a, blockIdx.x, t, lds, up_codes(a.D));
+  if (w > 0) {
+    const moe_bf16x8* row = (const moe_bf16x8*)(x + (size_t)t * a.D);
+    for (int p = threadIdx.x - 64; p < a.D / 8; p += blockDim.x - 64) quant_piece(row[p], p, tile.codes(), tile.sx);
+    lds_barrier();
+    return;
+  }
+  Chosen chosen{};
+  int e = 0;
+  if (!tile.shared) {
+    const float* row = r.src.logits + (size_t)t * a.E;
+    chosen = KIND == ROUTE_SOFTMAX ? route_softmax_token<VPL>(r, row, t, false) : route_grouped_token<VPL>(r, row, t, false);
+    e = __builtin_amdgcn_readlane(chosen.expert, tile.slot);
+  }
+  tile.start(e);
+  lds_barrier();
+  tile.finish();
+  if (blockIdx.x == 0 && lane < a.k) r.idx[(size_t)t * a.k + lane] = chosen.expert, r.w[(size_t)t * a.k + lane] = chosen.weight;
+}
+
+// The same behind a small router (front_kernel, whose sums, blocks and instructions these are): the workgroup's eight waves norm the
+// token and multiply a K block of the router each, and the first goes on alone with the selection and its experts' weights.  Bound by
+// its start and the chain behind it: mini layer behind its norm, one token, 14.8 us a call in three launches, 12.8 in two.
+constexpr int FRONT_WAVES = 8, FRONT_COLUMNS = 65;
+__host__ __device__ constexpr int front_up_lds(int D, int N, int ks) { return up_lds(D, ks) + D * 2 + (N * (D / 128 + 1) + 3) / 4 * 16; }
+template <int KIND, bool NORM, int KS>
+__global__ __launch_bounds__(64 * FRONT_WAVES) void token_front_gateup_kernel(const TokenArgs a, const RouteArgs r, const FrontArgs f) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];   // [the tile's][the row's pieces][the K blocks' products][logits]
+  constexpr int GROUPS = (FRONT_COLUMNS + 15) / 16;
+  __shared__ float wave_sum[2];
+  const int tid = threadIdx.x, lane = tid & 63, t = blockIdx.y, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fr = lane & 15, fq = lane >> 4, N = r.src.N, E = a.E, D = a.D, KB = D / BK, P = D / 8;
+  GateUpTile<false, KS> tile(a, blockIdx.x, t, lds, up_codes(D));
+  v4i* pieces = (v4i*)(lds + up_lds(D, KS));
+  float *products = (float*)(pieces + P), *logits = products + KB * N;
+  // the row's pieces: the last wave has the first 64, the one before it the rest
+  const int unit = FRONT_WAVES - 1 - w, p = unit * 64 + lane;
+  const bool has = unit < 2 && p < P;
+  moe_bf16x8 in = {};
+  v4f wt[2] = {};
+  if (has) {
+    in = load_bf16x8(f.x, f.x_f32, (size_t)t * P + p);
+    if (NORM) wt[0] = ((const v4f*)f.norm)[2 * p], wt[1] = ((const v4f*)f.norm)[2 * p + 1];
+  }
+  v4i b[GROUPS][4];
+  if (w < KB) {
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) {
+      if (16 * g >= N) break;
+      const int n = min(16 * g + fr, N - 1);
+      const v4i* src = (const v4i*)((const bf16_t*)(n < E ? f.w_router : f.w_shared_gate) + (n < E ? (size_t)n * D : 0) + w * 128) + fq;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) b[g][s] = src[4 * s];
+    }
+  }
+  if (NORM) {
+    if (unit < 2) {
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float v = bf16_to_f32(in.v[j]);
+        ss = __fadd_rn(ss, __fmul_rn(v, v));
+      }
+      ss = wave_sum_f32(ss);
+      if (lane == 0) wave_sum[unit] = ss;
+    }
+    lds_barrier();
+    const float total = P > 64 ? __fadd_rn(wave_sum[0], wave_sum[1]) : wave_sum[0];
+    const float rms = __fsqrt_rn(__fadd_rn(__fdiv_rn(total, (float)D), f.eps));
+#pragma unroll
+    for (int j = 0; j < 8; ++j) in.v[j] = f32_to_bf16(__fmul_rn(__fdiv_rn(bf16_to_f32(in.v[j]), rms), __fadd_rn(1.0f, wt[j / 4][j % 4])));
+  }
+  if (has) pieces[p] = __builtin_bit_cast(v4i, in);
+  lds_barrier();
+  if (w < KB) {
+    v4f acc[GROUPS] = {};
+    v4i av[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) av[s] = pieces[w * 16 + 4 * s + fq];   // (all sixteen rows of the matrix instruction are this one)
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) {
+      if (16 * g >= N) break;
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av[s]), __builtin_bit_cast(bf16x8_t, b[g][s]), acc[g], 0, 0, 0);
+      if (fq == 0 && 16 * g + fr < N) products[w * N + 16 * g + fr] = acc[g][0];
+    }
+  }
+  lds_barrier();
+  if (has) quant_piece(in, p, tile.codes(), tile.sx);
+  if (tid < 128)   // (N <= 65)
+    if (tid < N) {
+      float s = products[tid];
+      for (int kb = 1; kb < KB; ++kb) s = __fadd_rn(s, products[kb * N + tid]);
+      logits[tid] = bf16_to_f32(f32_to_bf16(s));
+    }
+  lds_barrier();
+  if (w > 0) return;
+  Chosen chosen{};
+  int e = 0;
+  if (!tile.shared) {
+    chosen = KIND == ROUTE_SOFTMAX ? route_softmax_token<1>(r, logits, t, false) : route_grouped_token<1>(r, logits, t, false);
+    e = __builtin_amdgcn_readlane(chosen.expert, tile.slot);
+  }
+  tile.start(e);
+  tile.finish();
+  if (blockIdx.x == 0) {   // (a routed tile: it has the selection)
+    if (lane < a.k) r.idx[(size_t)t * a.k + lane] = chosen.expert, r.w[(size_t)t * a.k + lane] = chosen.weight;
+    if (r.src.out_logits && lane < E) r.src.out_logits[(size_t)t * E + lane] = logits[lane];
+    if (lane == 0 && r.src.shared_gate && N > E) r.src.shared_gate[t] = bf16_to_f32(f32_to_bf16(sigmoid_det(logits[E])));
+  }
 }
 
 // LDS of a wave of the second launch: ring, codes and scales of its row, the weights' scales of its tiles
@@ -303,6 +475,37 @@ int launch_gateup(const TokenArgs& a, bool from_memory, hipStream_t s) {
   return moe_check_hip(hipGetLastError(), "token gate/up launch");
 }
 
+template <int KIND, bool ONCE, int KS>
+auto route_gateup_kernel(int E) {
+  return E <= 128 ? token_route_gateup_kernel<KIND, 2, ONCE, KS> : token_route_gateup_kernel<KIND, 4, ONCE, KS>;
+}
+template <int KIND>
+auto route_gateup_kernel(int E, bool from_memory, bool pairs) {
+  return pairs ? (from_memory ? route_gateup_kernel<KIND, true, 2>(E) : route_gateup_kernel<KIND, false, 2>(E))
+               : (from_memory ? route_gateup_kernel<KIND, true, 1>(E) : route_gateup_kernel<KIND, false, 1>(E));
+}
+template <int KIND>
+auto front_gateup_kernel(bool norm, bool pairs) {
+  return pairs ? (norm ? token_front_gateup_kernel<KIND, true, 2> : token_front_gateup_kernel<KIND, false, 2>)
+               : (norm ? token_front_gateup_kernel<KIND, true, 1> : token_front_gateup_kernel<KIND, false, 1>);
+}
+int launch_route_gateup(const TokenArgs& a, const TokenRoute& route, bool from_memory, hipStream_t s) {
+  static std::atomic<unsigned long long> raised[16] = {};
+  const int pairs = moe_token_stages(a.M, a.D, a.k, a.I, a.SI, from_memory).gateup == 2;
+  const bool softmax = route.routing == MOE_ROUTING_SOFTMAX;
+  const dim3 grid((a.k * a.I + a.SI) / COLS, a.M);
+  if (route.front) {   // (64 KB of LDS hold these)
+    auto* kernel = softmax ? front_gateup_kernel<ROUTE_SOFTMAX>(route.front->norm, pairs) : front_gateup_kernel<ROUTE_GROUPED>(route.front->norm, pairs);
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * FRONT_WAVES), front_up_lds(a.D, route.args.src.N, 1 + pairs), s, a, route.args, *route.front);
+    return moe_check_hip(hipGetLastError(), "token router and gate/up launch");
+  }
+  auto* kernel = softmax ? route_gateup_kernel<ROUTE_SOFTMAX>(a.E, from_memory, pairs) : route_gateup_kernel<ROUTE_GROUPED>(a.E, from_memory, pairs);
+  if (int rc = moe_raise_lds_limit((const void*)kernel, kLds, raised[(a.E > 128) * 8 + softmax * 4 + 2 * pairs + from_memory])) return rc;
+  const int quantisers = a.D > 4096 ? 2 : 1;
+  hipLaunchKernelGGL(kernel, grid, dim3(64 * (1 + quantisers)), up_lds(a.D, 1 + pairs), s, a, route.args, (const bf16_t*)route.x);
+  return moe_check_hip(hipGetLastError(), "token route and gate/up launch");
+}
+
 int down_tiles(int D, int M) {
   const int cols = D / COLS;
   int tiles = 1;
@@ -382,8 +585,23 @@ TokenStages moe_token_stages(int M, int D, int k, int I, int SI, bool from_memor
   return {1 + gateup, 1 + down};
 }
 
-int moe_token_experts(const TokenArgs& a, bool from_memory, moe_stream_t stream) {
+// Ready logits: while the CUs hold all workgroups at once (by LDS), which then route side by side: the launch that falls away took 3.6 to
+// 5.7 us and its end and the next one's start between them (us a call, launch by launch / this way): tiny, 1 token 11.3 / 8.9, 16 14.0 /
+// 11.6; Qwen3-MoE, 1 16.8 / 14.4, 4 31.4 / 28.7, 8 (3072 workgroups) 50.6 / 48.0; DeepSeek-V3, 1 71.0 / 68.5.  Nothing was measured above
+// 256 experts.
+bool moe_token_routes(int M, int D, int E, int k, int I, int SI) {
+  const int lds = up_lds(D);
+  return E <= 256 && lds <= kLds && (long long)M * ((k * I + SI) / COLS) <= 256 * (kLds / lds);
+}
+// Behind a small router every workgroup of eight waves repeats the router's matmul.  Mini layer, 96 workgroups a token, launch by
+// launch / this way: 1 token 14.0 / 11.6, 4 14.6 / 13.9, 5 15.2 / 14.6, 8 (768 workgroups) 15.4 / 17.9; behind its norm 1 14.8 / 12.8,
+// 2 15.1 / 12.9, 3 15.1 / 14.4, 4 15.2 / 15.3, 6 16.3 / 19.8.
+bool moe_token_fronts(int M, int k, int I, int SI, bool norm, bool from_memory) {
+  return !from_memory && (long long)M * ((k * I + SI) / COLS) <= (norm ? 320 : 512);
+}
+
+int moe_token_experts(const TokenArgs& a, bool from_memory, const TokenRoute* route, moe_stream_t stream) {
   hipStream_t s = (hipStream_t)stream;
-  if (int rc = launch_gateup(a, from_memory, s)) return rc;
+  if (int rc = route ? launch_route_gateup(a, *route, from_memory, s) : launch_gateup(a, from_memory, s)) return rc;
   return launch_down(a, from_memory, s);
 }

@@ -36,6 +36,14 @@ int main() {
       int M, D, E, k, I, SI;
       std::cin >> M >> D >> E >> k >> I >> SI;
       std::cout << moe_token_takes(M, D, E, k, I, SI) << "\n";
+    } else if (what == "token_routes") {   // tokens, D, experts, k, I, SI: whether the first launch routes ready logits
+      int M, D, E, k, I, SI;
+      std::cin >> M >> D >> E >> k >> I >> SI;
+      std::cout << moe_token_routes(M, D, E, k, I, SI) << "\n";
+    } else if (what == "token_fronts") {   // tokens, D, experts, k, I, SI, norm: whether it takes a small router too
+      int M, D, E, k, I, SI, norm;
+      std::cin >> M >> D >> E >> k >> I >> SI >> norm;
+      std::cout << moe_token_fronts(M, k, I, SI, norm, moe_gemm_from_memory(((long long)E * I + SI) * D)) << "\n";
     } else if (what == "stages") {   // tokens, D, experts, k, I, SI: K steps of a stage in the two launches of single tokens
       int M, D, E, k, I, SI;
       std::cin >> M >> D >> E >> k >> I >> SI;

@@ -97,6 +97,20 @@ def test_two_k_steps_a_stage_are_for_workgroups_that_run_at_once(ask):
     assert [a[0] for a in ask(*[("stages", *c) for c in limits])] == list(limits.values())
 
 
+def test_single_tokens_are_routed_by_workgroups_that_run_at_once(ask):
+    """Up to 256 experts and as many workgroups as the CUs' LDS holds; behind a small router about one a CU, two without a norm.  The
+    batches that test_gpu_variants.py compares are on both sides."""
+    from tests.test_gpu_variants import FRONTED_TOKENS, ROUTED_TOKENS
+    assert ask(*[("token", *c) for c in ROUTED_TOKENS]) == ["1"] * len(ROUTED_TOKENS)
+    assert ask(*[("token_routes", *c) for c in ROUTED_TOKENS]) == ["1"] * 5 + ["0", "1", "1", "1"]
+    assert ask(*[("token", *c[:6]) for c in FRONTED_TOKENS]) == ["1"] * len(FRONTED_TOKENS)
+    assert ask(*[("front", c[0], c[1], c[2], c[2] + (c[5] > 0), int(c[6]), 0, 1) for c in FRONTED_TOKENS]) == ["1"] * len(FRONTED_TOKENS)
+    assert ask(*[("token_fronts", *map(int, c)) for c in FRONTED_TOKENS]) == ["1", "1", "1", "0", "1", "1", "1", "1", "1"]
+    limits = {(1, 7168, 256, 8, 2048, 2048): "1", (8, 2048, 128, 8, 768, 0): "1", (1, 4096, 512, 10, 1024, 0): "0"}
+    assert ask(*[("token_routes", *c) for c in limits]) == list(limits.values())
+    assert ask(("token_fronts", 6, 1024, 32, 2, 512, 512, 0), ("token_fronts", 1, 1024, 64, 2, 1152, 0, 1)) == ["0", "0"]   # 576 workgroups; from memory
+
+
 def test_the_down_gemm_of_short_k_has_a_list_of_its_own(ask):
     """Tiles of 128 rows beside gate/up's full ones: more rows than one workgroup sorts, few K steps, enough items and not too many rows."""
     from tests.test_gpu_variants import TWO_LISTS

@@ -597,6 +597,85 @@ def test_experts_of_single_tokens_give_the_grouped_bits(jg, M, D, E, k, I, SI, f
         assert same(out, want), f"replay {i}"
 
 
+ROUTED_TOKENS = [   # M, D, E, k, I, SI of ready logits: routed by the experts' first launch, or just not
+    (1, 128, 1, 1, 128, 0), (3, 384, 128, 3, 256, 128), (3, 4096, 129, 4, 128, 0), (1, 4224, 256, 8, 256, 128), (1, 7168, 64, 8, 2048, 256),
+    (1, 512, 257, 2, 256, 0), (16, 512, 8, 2, 1024, 0), (16, 1024, 64, 8, 384, 0), (1, 7168, 32, 8, 3072, 0)]
+
+
+@pytest.mark.parametrize("routing", ["softmax", "sigmoid_grouped"])
+@pytest.mark.parametrize("M,D,E,k,I,SI", ROUTED_TOKENS)
+def test_ready_logits_of_single_tokens_give_the_grouped_bits(jg, M, D, E, k, I, SI, routing):
+    """Routing and quantiser inside the experts' first launch: the bits of the call that launches them one by one, also with logits
+    that are equal, infinite or NaN and rows that are zero or hold infinities and NaN; other rows in replays of a graph."""
+    import torch
+    print("ready logits of single tokens", M, D, E, k, I, SI, routing, flush=True)
+    params, rand = _layer(jg, D, E, I, SI, M + D + E)
+    names = ("gate_proj", "up_proj", "down_proj")
+    kw = dict(top_k=k, experts={n: params[n] for n in names}, routing=routing, shared={n: params["shared_" + n] for n in names} if SI else None)
+    if routing == "sigmoid_grouped":
+        groups = 8 if E % 8 == 0 else 1
+        kw.update(bias=0.1 * torch.arange(E, device="cuda").remainder(5).float(), routed_scale=2.5, n_group=groups, topk_group=max(groups // 2, 1))
+        if k > kw["topk_group"] * (E // groups):
+            kw.update(n_group=1, topk_group=1)
+    same = lambda a, b: torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(7.0, float("inf"), -float("inf")), b.nan_to_num(7.0, float("inf"), -float("inf")))
+    rows = []
+    for kind in ("plain", "ties", "odd logits", "zero rows", "odd rows"):
+        x, lg = rand(M, D), rand(M, E).float()
+        if kind == "ties":
+            lg = lg.round()
+        if kind == "odd logits":
+            lg[0, 0], lg[M - 1, E // 2], lg[0, E - 1] = float("nan"), float("inf"), -float("inf")
+        if kind == "zero rows":
+            x[M - 1] = 0
+        if kind == "odd rows":
+            x[0, 5], x[M - 1, D - 1] = float("inf"), float("nan")
+        want = jg.moe_experts(x, lg, return_debug=True, **kw)[0]
+        assert same(jg.moe_experts(x, lg, **kw), want), kind
+        rows.append((x, lg, want))
+    x, lg = rows[0][0].clone(), rows[0][1].clone()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = jg.moe_experts(x, lg, **kw)
+    for i, (xi, li, want) in enumerate(rows):
+        x.copy_(xi), lg.copy_(li), out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert same(out, want), f"replay {i}"
+
+
+FRONTED_TOKENS = [   # M, D, E, k, I, SI, norm: behind a small router, in the experts' first launch, or just not
+    (1, 1024, 32, 2, 512, 512, True), (3, 1024, 32, 2, 512, 512, True), (5, 1024, 32, 2, 512, 512, False), (4, 1024, 32, 2, 512, 512, True),
+    (2, 640, 64, 4, 128, 256, True), (1, 512, 64, 8, 256, 0, False), (2, 128, 1, 1, 128, 128, True), (16, 256, 16, 2, 256, 0, False), (1, 896, 17, 3, 384, 128, True)]
+
+
+@pytest.mark.parametrize("routing", ["softmax", "sigmoid_grouped"])
+@pytest.mark.parametrize("M,D,E,k,I,SI,norm", FRONTED_TOKENS)
+def test_small_routers_of_single_tokens_give_the_grouped_bits(jg, M, D, E, k, I, SI, norm, routing):
+    """Norm, router and selection inside the experts' first launch: the bits of the call that takes them launch by launch."""
+    import torch
+    print("small routers of single tokens", M, D, E, k, I, SI, norm, routing, flush=True)
+    params, rand = _layer(jg, D, E, I, SI, M + D + E)
+    names = ("gate_proj", "up_proj", "down_proj")
+    same = lambda a, b: torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(7.0, float("inf"), -float("inf")), b.nan_to_num(7.0, float("inf"), -float("inf")))
+    kw = dict(top_k=k, experts={n: params[n] for n in names}, routing=routing, gate_weight=params["gate_weight"], add_residual=True)
+    if SI:
+        kw.update(shared={n: params["shared_" + n] for n in names}, shared_expert_gate_weight=params["shared_expert_gate_weight"])
+    if norm:
+        kw.update(norm_weight=rand(D).float() * 0.1)
+    if routing == "sigmoid_grouped":
+        kw.update(bias=0.1 * torch.arange(E, device="cuda").remainder(5).float())
+    for kind in ("plain", "zero rows", "odd rows"):
+        x = rand(M, D)
+        if kind == "zero rows":
+            x[M - 1] = 0
+        if kind == "odd rows":
+            x[0, 5], x[M - 1, D - 1] = float("inf"), float("nan")
+        for f32 in (False, True):
+            run = lambda **o: jg.moe._forward(x.float() if f32 else x, None, io_f32=f32, **kw, **o)
+            assert same(run(), run(return_debug=True)[0]), (kind, f32)
+
+
 @pytest.mark.parametrize("M,k", [(1, 2), (5, 3), (16, 8),     # straight to the experts: both of its kernels leave the rows out
                                  (17, 1), (32, 1), (17, 3),   # the sort without counters, and with them
                                  (700, 2), (1100, 2), (3000, 3)])   # scales read row-major, and gathered; several chunks
