@@ -31,14 +31,15 @@ TokenDownPlan moe_token_down_plan(int M, int D, int k, int I, int SI);
 // K steps of a ring's stage in the two launches: 1 or 2
 struct TokenStages { int gateup, down; };
 TokenStages moe_token_stages(int M, int D, int k, int I, int SI, bool from_memory);
-// whether the first launch routes and quantises the tokens too: from ready logits and (M, D) bf16 activations, or behind a router that
-// moe_front_takes
-bool moe_token_routes(int M, int D, int E, int k, int I, int SI);
+// whether the first launch routes and quantises the tokens too: from ready logits (or a given selection) and (M, D) bf16 activations,
+// or behind a router that moe_front_takes
+bool moe_token_routes(int M, int D, int E, int k, int I, int SI, bool selected);
 bool moe_token_fronts(int M, int k, int I, int SI, bool norm, bool from_memory);
 struct TokenRoute {   // (checked: moe_route_check, moe_front_check)
   int routing;
   RouteArgs args;   // args.idx, args.w: the TokenArgs' own
   const void* x;
-  const FrontArgs* front;   // null: ready logits
+  const FrontArgs* front;   // null: ready logits, or
+  bool selected;            // nothing to route
 };
 int moe_token_experts(const TokenArgs& a, bool from_memory, const TokenRoute* route, moe_stream_t stream);   // route: null, or such a call's

@@ -215,11 +215,12 @@ __device__ __forceinline__ void quant_piece(const moe_bf16x8& in, int p, uint8_t
 // LDS writes of all waves are there; the copies stay under way
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// The same with the token's routing and quantisation in front, from ready logits: the first wave selects its token's experts itself
+// The same with the token's routing and quantisation in front, from ready logits (or a given selection): the first wave selects its token's experts itself
 // and streams their weights, the others quantise the token meanwhile (rows above 4096: two of them).  What it waits for is the
 // selection's chain of dependent steps, as the launch before did, without that launch's end and this one's start.  One token of
 // DeepSeek-V3, launch by launch 71.0 us a call; this way with the selecting wave quantising behind its first copies 71.0 (110
 // instructions for 512 values), with one wave for that 70.2, with two 68.5, three 68.8.
+constexpr int SELECTED = -1;   // (a KIND: nothing to route)
 template <int KIND, int VPL, bool ONCE, int KS>
 __global__ __launch_bounds__(192) void token_route_gateup_kernel(const TokenArgs a, const RouteArgs r, const bf16_t* x) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -233,7 +234,13 @@ __global__ __launch_bounds__(192) void token_route_gateup_kernel(const TokenArgs
   }
   Chosen chosen{};
   int e = 0;
-  if (!tile.shared) {
+  if (KIND == SELECTED) {
+    if (!tile.shared) e = __builtin_amdgcn_readfirstlane(a.idx[(size_t)t * a.k + tile.slot]);
+    if (!tile.shared && (unsigned)e >= (unsigned)a.E) {   // (out of range: the second launch leaves its row out)
+      lds_barrier();
+      return;
+    }
+  } else if (!tile.shared) {
     const float* row = r.src.logits + (size_t)t * a.E;
     chosen = KIND == ROUTE_SOFTMAX ? route_softmax_token<VPL>(r, row, t, false) : route_grouped_token<VPL>(r, row, t, false);
     e = __builtin_amdgcn_readlane(chosen.expert, tile.slot);
@@ -241,7 +248,7 @@ __global__ __launch_bounds__(192) void token_route_gateup_kernel(const TokenArgs
   tile.start(e);
   lds_barrier();
   tile.finish();
-  if (blockIdx.x == 0 && lane < a.k) r.idx[(size_t)t * a.k + lane] = chosen.expert, r.w[(size_t)t * a.k + lane] = chosen.weight;
+  if (KIND != SELECTED && blockIdx.x == 0 && lane < a.k) r.idx[(size_t)t * a.k + lane] = chosen.expert, r.w[(size_t)t * a.k + lane] = chosen.weight;
 }
 
 // The same behind a small router (front_kernel, whose sums, blocks and instructions these are): the workgroup's eight waves norm the
@@ -477,7 +484,8 @@ int launch_gateup(const TokenArgs& a, bool from_memory, hipStream_t s) {
 
 template <int KIND, bool ONCE, int KS>
 auto route_gateup_kernel(int E) {
-  return E <= 128 ? token_route_gateup_kernel<KIND, 2, ONCE, KS> : token_route_gateup_kernel<KIND, 4, ONCE, KS>;
+  if constexpr (KIND == SELECTED) return token_route_gateup_kernel<KIND, 1, ONCE, KS>;
+  else return E <= 128 ? token_route_gateup_kernel<KIND, 2, ONCE, KS> : token_route_gateup_kernel<KIND, 4, ONCE, KS>;
 }
 template <int KIND>
 auto route_gateup_kernel(int E, bool from_memory, bool pairs) {
@@ -490,7 +498,7 @@ auto front_gateup_kernel(bool norm, bool pairs) {
                : (norm ? token_front_gateup_kernel<KIND, true, 1> : token_front_gateup_kernel<KIND, false, 1>);
 }
 int launch_route_gateup(const TokenArgs& a, const TokenRoute& route, bool from_memory, hipStream_t s) {
-  static std::atomic<unsigned long long> raised[16] = {};
+  static std::atomic<unsigned long long> raised[20] = {};
   const int pairs = moe_token_stages(a.M, a.D, a.k, a.I, a.SI, from_memory).gateup == 2;
   const bool softmax = route.routing == MOE_ROUTING_SOFTMAX;
   const dim3 grid((a.k * a.I + a.SI) / COLS, a.M);
@@ -499,8 +507,11 @@ int launch_route_gateup(const TokenArgs& a, const TokenRoute& route, bool from_m
     hipLaunchKernelGGL(kernel, grid, dim3(64 * FRONT_WAVES), front_up_lds(a.D, route.args.src.N, 1 + pairs), s, a, route.args, *route.front);
     return moe_check_hip(hipGetLastError(), "token router and gate/up launch");
   }
-  auto* kernel = softmax ? route_gateup_kernel<ROUTE_SOFTMAX>(a.E, from_memory, pairs) : route_gateup_kernel<ROUTE_GROUPED>(a.E, from_memory, pairs);
-  if (int rc = moe_raise_lds_limit((const void*)kernel, kLds, raised[(a.E > 128) * 8 + softmax * 4 + 2 * pairs + from_memory])) return rc;
+  auto* kernel = route.selected ? route_gateup_kernel<SELECTED>(a.E, from_memory, pairs)
+                 : softmax      ? route_gateup_kernel<ROUTE_SOFTMAX>(a.E, from_memory, pairs)
+                                : route_gateup_kernel<ROUTE_GROUPED>(a.E, from_memory, pairs);
+  const int which = route.selected ? 4 : (a.E > 128) * 2 + softmax;
+  if (int rc = moe_raise_lds_limit((const void*)kernel, kLds, raised[which * 4 + 2 * pairs + from_memory])) return rc;
   const int quantisers = a.D > 4096 ? 2 : 1;
   hipLaunchKernelGGL(kernel, grid, dim3(64 * (1 + quantisers)), up_lds(a.D, 1 + pairs), s, a, route.args, (const bf16_t*)route.x);
   return moe_check_hip(hipGetLastError(), "token route and gate/up launch");
@@ -588,10 +599,11 @@ TokenStages moe_token_stages(int M, int D, int k, int I, int SI, bool from_memor
 // Ready logits: while the CUs hold all workgroups at once (by LDS), which then route side by side: the launch that falls away took 3.6 to
 // 5.7 us and its end and the next one's start between them (us a call, launch by launch / this way): tiny, 1 token 11.3 / 8.9, 16 14.0 /
 // 11.6; Qwen3-MoE, 1 16.8 / 14.4, 4 31.4 / 28.7, 8 (3072 workgroups) 50.6 / 48.0; DeepSeek-V3, 1 71.0 / 68.5.  Nothing was measured above
-// 256 experts.
-bool moe_token_routes(int M, int D, int E, int k, int I, int SI) {
+// 256 experts.  A given selection (the launch that falls away is the quantiser's): moe_routing and expert_forward_single of tiny, 1 to 16
+// tokens 20.0 / 17.8, of Qwen3-MoE, 1 24.0 / 22.6, 4 37.4 / 36.0, 8 56.7 / 54.8.
+bool moe_token_routes(int M, int D, int E, int k, int I, int SI, bool selected) {
   const int lds = up_lds(D);
-  return E <= 256 && lds <= kLds && (long long)M * ((k * I + SI) / COLS) <= 256 * (kLds / lds);
+  return (selected || E <= 256) && lds <= kLds && (long long)M * ((k * I + SI) / COLS) <= 256 * (kLds / lds);
 }
 // Behind a small router every workgroup of eight waves repeats the router's matmul.  Mini layer, 96 workgroups a token, launch by
 // launch / this way: 1 token 14.0 / 11.6, 4 14.6 / 13.9, 5 15.2 / 14.6, 8 (768 workgroups) 15.4 / 17.9; behind its norm 1 14.8 / 12.8,

@@ -36,10 +36,10 @@ int main() {
       int M, D, E, k, I, SI;
       std::cin >> M >> D >> E >> k >> I >> SI;
       std::cout << moe_token_takes(M, D, E, k, I, SI) << "\n";
-    } else if (what == "token_routes") {   // tokens, D, experts, k, I, SI: whether the first launch routes ready logits
+    } else if (what == "token_routes" || what == "token_selected") {   // tokens, D, experts, k, I, SI: whether the first launch routes ready logits, or takes a selection
       int M, D, E, k, I, SI;
       std::cin >> M >> D >> E >> k >> I >> SI;
-      std::cout << moe_token_routes(M, D, E, k, I, SI) << "\n";
+      std::cout << moe_token_routes(M, D, E, k, I, SI, what == "token_selected") << "\n";
     } else if (what == "token_fronts") {   // tokens, D, experts, k, I, SI, norm: whether it takes a small router too
       int M, D, E, k, I, SI, norm;
       std::cin >> M >> D >> E >> k >> I >> SI >> norm;

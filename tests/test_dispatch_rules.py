@@ -108,6 +108,7 @@ def test_single_tokens_are_routed_by_workgroups_that_run_at_once(ask):
     assert ask(*[("token_fronts", *map(int, c)) for c in FRONTED_TOKENS]) == ["1", "1", "1", "0", "1", "1", "1", "1", "1"]
     limits = {(1, 7168, 256, 8, 2048, 2048): "1", (8, 2048, 128, 8, 768, 0): "1", (1, 4096, 512, 10, 1024, 0): "0"}
     assert ask(*[("token_routes", *c) for c in limits]) == list(limits.values())
+    assert ask(*[("token_selected", *c) for c in limits]) == ["1", "1", "1"]   # (whatever the experts' number)
     assert ask(("token_fronts", 6, 1024, 32, 2, 512, 512, 0), ("token_fronts", 1, 1024, 64, 2, 1152, 0, 1)) == ["0", "0"]   # 576 workgroups; from memory
 
 
