@@ -339,13 +339,23 @@ int moe_quant_act_job(const void* x, int x_f32, void* x_bf16, int R, int K, uint
 // Batches up to this many (token, slot) entries are one chunk, and their few, short row tiles are listed in plain
 // expert order with equal XCD shares.
 constexpr int kSmallRows = 2048;
+// What the placing launch of a list of several chunks writes besides (a pointer to both, as these arguments' size is read cold by every
+// routing and placing launch)
+struct ScaleGather {   // the activation scales of the sorted rows, block-major
+  const float* sx;     // (tokens, KB)
+  int KB;
+  float* out;          // (KB, R)
+};
+struct PlaceMore {
+  const TileList* tl_down;     // a list of its own for the down GEMM, or null: it reads PermuteOut::tl
+  const ScaleGather* gather;   // or null
+};
 // What the sort by expert writes (sort_order, sorted_token_ids, inv_perm: null to skip; tl.tiles null: no work list).
 struct PermuteOut {
   int32_t *group_sizes, *group_offsets, *sorted_token_ids, *sort_order, *inv_perm;
   int k;
   TileList tl;
-  // a list of its own for the down GEMM, or null: it reads tl.  Batches of more than kSmallRows entries only; read by the host.
-  const TileList* tl_down;
+  const PlaceMore* more;   // or null; batches of more than kSmallRows entries only; read by the host
 };
 // One routing call: the selection, and with it (optional) an activation quantisation and the sort by expert.
 struct RouteArgs {

@@ -11,6 +11,8 @@
 // A launch of this size is bound by its start, not by its work (an idle launch takes 3 us, each chain of dependent
 // cold loads 1-2 us more), so the chunk count is capped to keep the second launch's redundant reads of the histograms
 // (chunks x E counts per workgroup, at most 256 KB from L2) cheaper than a third launch that would scan them once.
+#include <type_traits>
+
 #include "moe_common.h"
 #include "moe_permute_device.h"
 #include "moe_quant_device.h"
@@ -38,20 +40,23 @@ __global__ __launch_bounds__(kHistThreads) void hist_kernel(const int32_t* __res
 }
 
 // TWO: there is a second work list, l2, for the same experts (a kernel of its own: with both lists' arguments in all launches, and the
-// choice between them, Qwen3-MoE of 4096 tokens took 1.2 us more)
-template <bool TWO>
+// choice between them, Qwen3-MoE of 4096 tokens took 1.2 us more).  GATHER: the entries' activation scales are written to their places too
+// (more arguments for all launches: Qwen3-MoE of 1000 tokens +0.6 us)
+template <bool TWO, bool GATHER>
 __global__ __launch_bounds__(kPlaceThreads) void place_kernel(const int32_t* __restrict__ ids, int R, int E, int chunk,
                                                              int n_chunks, const int32_t* __restrict__ chunk_hist,
-                                                             const PermuteOut o, const QuantJob quant, const TileList l2) {
+                                                             const PermuteOut o, const std::conditional_t<GATHER, ScaleGather, QuantJob> job,
+                                                             const TileList l2) {
   extern __shared__ int smem[];   // [waves][E]
-  if (!TWO && n_chunks == 1) {
-    if (blockIdx.x > 0) {   // the blocks behind quantise the activations (QuantJob)
-      moe_quant_act_block(quant, (int)blockIdx.x - 1);
+  if constexpr (!TWO && !GATHER)
+    if (n_chunks == 1) {
+      if (blockIdx.x > 0) {   // the blocks behind quantise the activations (QuantJob)
+        moe_quant_act_block(job, (int)blockIdx.x - 1);
+        return;
+      }
+      permute_one_chunk(ids, R, E, smem, o);
       return;
     }
-    permute_one_chunk(ids, R, E, smem, o);
-    return;
-  }
   __shared__ int total[kMaxE], before[kMaxE];
   const int e = threadIdx.x;
   // chunk; workgroup 0 (started first) does the experts' side, and one behind it the second list
@@ -110,6 +115,15 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(const int32_t* __r
   }
   __syncthreads();
   place_pass<true>(ids + first, first, n, E, smem, o);
+  if constexpr (GATHER) {   // sixteen lanes an entry; its place from where the pass above has put it
+    __syncthreads();
+    for (int i = first + (e >> 4); i < first + n; i += kPlaceThreads / 16) {
+      const int pos = o.inv_perm[i];
+      const float* row = job.sx + (size_t)((unsigned)i / (unsigned)o.k) * job.KB;
+      if (pos >= 0)
+        for (int kb = e & 15; kb < job.KB; kb += 16) job.out[(size_t)kb * R + pos] = row[kb];
+    }
+  }
 }
 
 }  // namespace
@@ -126,11 +140,20 @@ extern "C" size_t moe_permute_workspace_bytes(int M, int k, int E) {
 
 int moe_permute_place(const int32_t* idx, int R, int E, int chunk, int n_chunks, const int32_t* chunk_hist, const PermuteOut& o,
                       const QuantJob* quant, moe_stream_t stream) {
-  MOE_REQUIRE(n_chunks > 1 || !o.tl_down, MOE_ERR_BAD_SHAPE, "permute: a list of one chunk has no second work list");
+  MOE_REQUIRE(n_chunks > 1 || !o.more, MOE_ERR_BAD_SHAPE, "permute: a list of one chunk has no second work list and gathers no scales");
+  const PlaceMore more = o.more ? *o.more : PlaceMore{};
   const bool places = R > 0 && (o.sorted_token_ids || o.sort_order || o.inv_perm);
-  const unsigned blocks = n_chunks > 1 ? (places ? n_chunks : 0) + (o.tl_down ? 2 : 1) : 1 + (quant ? moe_quant_blocks(*quant, kPlaceThreads) : 0);
-  hipLaunchKernelGGL(o.tl_down ? place_kernel<true> : place_kernel<false>, dim3(blocks), dim3(kPlaceThreads), moe_place_lds_ints(E) * sizeof(int), (hipStream_t)stream,
-                     idx, R, E, chunk, n_chunks, chunk_hist, o, quant ? *quant : QuantJob{}, o.tl_down ? *o.tl_down : TileList{});
+  const unsigned blocks = n_chunks > 1 ? (places ? n_chunks : 0) + (more.tl_down ? 2 : 1) : 1 + (quant ? moe_quant_blocks(*quant, kPlaceThreads) : 0);
+  const dim3 grid(blocks), block(kPlaceThreads);
+  const size_t lds = moe_place_lds_ints(E) * sizeof(int);
+  hipStream_t s = (hipStream_t)stream;
+  const TileList l2 = more.tl_down ? *more.tl_down : TileList{};
+  if (more.gather)
+    hipLaunchKernelGGL((more.tl_down ? place_kernel<true, true> : place_kernel<false, true>), grid, block, lds, s, idx, R, E, chunk, n_chunks, chunk_hist, o,
+                       *more.gather, l2);
+  else
+    hipLaunchKernelGGL((more.tl_down ? place_kernel<true, false> : place_kernel<false, false>), grid, block, lds, s, idx, R, E, chunk, n_chunks, chunk_hist, o,
+                       quant ? *quant : QuantJob{}, l2);
   return moe_check_hip(hipGetLastError(), "permute launch");
 }
 

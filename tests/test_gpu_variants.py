@@ -294,6 +294,29 @@ def test_scale_layouts_of_middle_sized_batches_give_the_same_bits(jg, M, E):
     assert torch.equal(whole[:400], jg.moe_experts(x[:400].contiguous(), lg[:400].contiguous(), **kw))
 
 
+@pytest.mark.parametrize("M,D", [(1030, 128), (1030, 384), (4097, 640), (8192, 2048), (8193, 2048), (1100, 2176)])   # the last two: by a launch of its own
+def test_scales_that_the_sort_places_give_the_bits_of_rows_read_in_place(jg, M, D):
+    """1, 3, 5, 16 and 17 scales a row, up to 2^18 of them and above, with dropped entries of a given selection and without."""
+    import torch
+    print("placed scales", M, D, flush=True)
+    E = 12
+    params, rand = _layer(jg, D, E, 128, 0, M + D)
+    names = ("gate_proj", "up_proj", "down_proj")
+    x, lg = rand(M, D), rand(M, E).float()
+    kw = dict(top_k=2, experts={n: params[n] for n in names})
+    whole, dbg = jg.moe_experts(x, lg, return_debug=True, **kw)
+    assert torch.equal(jg.moe_experts(x, lg, **kw), whole)
+    for lo in (0, M - 500):   # (1000 rows: scales read row-major)
+        assert torch.equal(jg.moe_experts(x[lo:lo + 500].contiguous(), lg[lo:lo + 500].contiguous(), **kw), whole[lo:lo + 500])
+    idx = dbg["indices"].clone()
+    idx[::7, 0] = -1
+    idx[3::11, 1] = E
+    run = lambda rows: jg.expert_forward_single(x[rows].contiguous(), idx[rows].contiguous(), dbg["weights"][rows].contiguous(), *[params[n] for n in names])
+    whole = run(slice(None))
+    for lo in (0, M - 500):
+        assert torch.equal(run(slice(lo, lo + 500)), whole[lo:lo + 500])
+
+
 @pytest.mark.parametrize("R,D,I", [(4096, 256, 8192), (2090, 8192, 256), (5000, 512, 512)])   # (the last: lists of 53 and 79 tiles)
 def test_one_group_of_many_rows_gives_the_bits_of_fewer(jg, R, D, I):
     """More than 768 work items of one group, whose height follows from the rounds that its rows make; and many short tiles."""
