@@ -419,7 +419,8 @@ __global__ __launch_bounds__(1024) void token_down_kernel(const TokenArgs a, con
                  ring_at + sw_at + i * 4u);
           }
           rows.start({x.w_down + ((size_t)e * a.D + first * COLS) * K}, K, count, (size_t)COLS * K, ring_at);
-          // the row's quantisation groups, 32 lanes each
+          // the row's quantisation groups, 32 lanes each (the maximum by DPP: where a wave has two slots the launch waits for its
+          // instructions, and with five shuffles 16 tokens of 32 of 256 experts of 1024 x 128 took 25.9 us for 24.0)
           for (int from = 0; from < K / 4; from += 64 * H_PIECES) {
             if (from || slot != w) load_h(slot, from);
 #pragma unroll
@@ -427,13 +428,17 @@ __global__ __launch_bounds__(1024) void token_down_kernel(const TokenArgs a, con
               const int i = from + 64 * p + lane;
               if (from + 64 * p >= K / 4) break;
               const v4f v = hv[p];   // (lanes past the row's end: half a wave, whose group is its own)
-              float m = 0.f;
+              float amax = 0.f;
 #pragma unroll
-              for (int r = 0; r < 4; ++r) m = fmaxf(m, fabsf(v[r]));
-#pragma unroll
-              for (int o = 1; o < 32; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, MOE_WAVE));
+              for (int r = 0; r < 4; ++r) amax = fmaxf(amax, fabsf(v[r]));
+              unsigned m = __float_as_uint(amax);   // (not negative: ordered as integers)
+              m = max(m, dpp<DPP_XOR1>(m));
+              m = max(m, dpp<DPP_XOR2>(m));
+              m = max(m, dpp<DPP_MIRROR8>(m));
+              m = max(m, dpp<DPP_MIRROR16>(m));
+              m = max(m, (unsigned)__shfl_xor((int)m, 16, MOE_WAVE));
               float scale, scale_inv;
-              fp8_scales(m, scale, scale_inv);
+              fp8_scales(__uint_as_float(m), scale, scale_inv);
               int q = 0;
               q = __builtin_amdgcn_cvt_pk_fp8_f32(__builtin_amdgcn_fmed3f(v[0] * scale, -MOE_FP8_MAX, MOE_FP8_MAX),
                                                   __builtin_amdgcn_fmed3f(v[1] * scale, -MOE_FP8_MAX, MOE_FP8_MAX), q, false);
