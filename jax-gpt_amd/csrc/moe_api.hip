@@ -321,7 +321,8 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
                 "combine: pointers must be 16-byte aligned");
     const bool from_memory = moe_gemm_from_memory(((long long)a->E * a->I + a->SI) * a->D);
     const bool fronts = front && moe_token_fronts(a->M, a->k, a->I, a->SI, a->norm_weight, from_memory);
-    const bool routes = carried && !a->w_router && !io_f32 && moe_token_routes(a->M, a->D, a->E, a->k, a->I, a->SI, given_idx);
+    const int chain = given_idx ? 0 : moe_token_chain(a->routing, a->E, a->k, a->n_group, a->topk_group);
+    const bool routes = carried && !a->w_router && !io_f32 && moe_token_routes(a->M, a->D, a->E, a->k, a->I, a->SI, given_idx, chain);
     TokenRoute tok_route{a->routing, route, a->x, fronts ? &front_args : nullptr, given_idx != nullptr};
     if (given_idx) rc = carried && !routes ? moe_quant_act_impl(a->x, io_f32, nullptr, a->M, a->D, b.xq, b.sx, nullptr, stream) : MOE_OK;
     else if (fronts) rc = moe_front_check(a->routing, tok_route.args, front_args, false);

@@ -33,7 +33,9 @@ struct TokenStages { int gateup, down; };
 TokenStages moe_token_stages(int M, int D, int k, int I, int SI, bool from_memory);
 // whether the first launch routes and quantises the tokens too: from ready logits (or a given selection) and (M, D) bf16 activations,
 // or behind a router that moe_front_takes
-bool moe_token_routes(int M, int D, int E, int k, int I, int SI, bool selected);
+// (chain: dependent steps of one token's selection)
+int moe_token_chain(int routing, int E, int k, int n_group, int topk_group);
+bool moe_token_routes(int M, int D, int E, int k, int I, int SI, bool selected, int chain = 0);
 bool moe_token_fronts(int M, int k, int I, int SI, bool norm, bool from_memory);
 struct TokenRoute {   // (checked: moe_route_check, moe_front_check)
   int routing;

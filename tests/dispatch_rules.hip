@@ -40,6 +40,10 @@ int main() {
       int M, D, E, k, I, SI;
       std::cin >> M >> D >> E >> k >> I >> SI;
       std::cout << moe_token_routes(M, D, E, k, I, SI, what == "token_selected") << "\n";
+    } else if (what == "token_chain") {   // the same of ready logits by the steps of their selection: routing, groups, kept groups
+      int M, D, E, k, I, SI, routing, n_group, topk_group;
+      std::cin >> M >> D >> E >> k >> I >> SI >> routing >> n_group >> topk_group;
+      std::cout << moe_token_routes(M, D, E, k, I, SI, false, moe_token_chain(routing, E, k, n_group, topk_group)) << "\n";
     } else if (what == "token_fronts") {   // tokens, D, experts, k, I, SI, norm: whether it takes a small router too
       int M, D, E, k, I, SI, norm;
       std::cin >> M >> D >> E >> k >> I >> SI >> norm;

@@ -112,6 +112,26 @@ def test_single_tokens_are_routed_by_workgroups_that_run_at_once(ask):
     assert ask(("token_fronts", 6, 1024, 32, 2, 512, 512, 0), ("token_fronts", 1, 1024, 64, 2, 1152, 0, 1)) == ["0", "0"]   # 576 workgroups; from memory
 
 
+def test_long_selections_are_not_repeated_by_many_workgroups(ask):
+    """Ready logits of 16 tokens, D 512: as many workgroups as 48 K steps of selection, a step more for each group that lies across
+    lanes, and one and a half for each of the grouped routing."""
+    softmax, grouped = 0, 1
+    want = {(16, 512, 256, 8, 512, 0, softmax, 1, 1): "1",      # 4096 workgroups, 32 K steps
+            (6, 512, 64, 32, 128, 0, softmax, 1, 1): "1",       # 1536, 48 K
+            (7, 512, 64, 32, 128, 0, softmax, 1, 1): "0",
+            (16, 512, 64, 32, 128, 0, softmax, 1, 1): "0",
+            (16, 512, 256, 8, 512, 0, grouped, 8, 4): "1",      # 48 K
+            (4, 512, 64, 32, 128, 0, grouped, 8, 4): "1",       # 1024, 48 K
+            (5, 512, 64, 32, 128, 0, grouped, 8, 4): "0",
+            (2, 512, 240, 8, 512, 0, grouped, 48, 24): "1",     # groups of five: 512 workgroups, 42 K
+            (3, 512, 240, 8, 512, 0, grouped, 48, 24): "0",
+            (16, 512, 240, 8, 512, 0, grouped, 48, 24): "0",
+            (16, 512, 240, 8, 512, 0, grouped, 48, 48): "1",    # (all groups are kept: nobody looks at them)
+            (2, 512, 192, 8, 512, 0, grouped, 0, 0): "1",       # (refused later)
+            (1, 7168, 256, 8, 2048, 2048, grouped, 8, 4): "1", (8, 2048, 128, 8, 768, 0, softmax, 1, 1): "1"}
+    assert ask(*[("token_chain", *c) for c in want]) == list(want.values())
+
+
 def test_the_down_gemm_of_short_k_has_a_list_of_its_own(ask):
     """Tiles of 128 rows beside gate/up's full ones: more rows than one workgroup sorts, few K steps, enough items and not too many rows."""
     from tests.test_gpu_variants import TWO_LISTS
