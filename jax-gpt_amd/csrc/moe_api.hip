@@ -320,7 +320,7 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
     MOE_REQUIRE(MOE_ALIGNED16(a->out) && (!a->add_residual || MOE_ALIGNED16(a->x)), MOE_ERR_BAD_ALIGN,
                 "combine: pointers must be 16-byte aligned");
     const bool from_memory = moe_gemm_from_memory(((long long)a->E * a->I + a->SI) * a->D);
-    const bool fronts = front && moe_token_fronts(a->M, a->k, a->I, a->SI, a->norm_weight, from_memory);
+    const bool fronts = front && moe_token_fronts(a->M, a->k, a->I, a->SI, a->norm_weight, from_memory, n_cols * a->D);
     const int chain = given_idx ? 0 : moe_token_chain(a->routing, a->E, a->k, a->n_group, a->topk_group);
     const bool routes = carried && !a->w_router && !io_f32 && moe_token_routes(a->M, a->D, a->E, a->k, a->I, a->SI, given_idx, chain);
     TokenRoute tok_route{a->routing, route, a->x, fronts ? &front_args : nullptr, given_idx != nullptr};

@@ -36,7 +36,7 @@ TokenStages moe_token_stages(int M, int D, int k, int I, int SI, bool from_memor
 // (chain: dependent steps of one token's selection)
 int moe_token_chain(int routing, int E, int k, int n_group, int topk_group);
 bool moe_token_routes(int M, int D, int E, int k, int I, int SI, bool selected, int chain = 0);
-bool moe_token_fronts(int M, int k, int I, int SI, bool norm, bool from_memory);
+bool moe_token_fronts(int M, int k, int I, int SI, bool norm, bool from_memory, int router = 0);   // router: its weights (columns x D)
 struct TokenRoute {   // (checked: moe_route_check, moe_front_check)
   int routing;
   RouteArgs args;   // args.idx, args.w: the TokenArgs' own

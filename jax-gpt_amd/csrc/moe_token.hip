@@ -626,8 +626,13 @@ bool moe_token_routes(int M, int D, int E, int k, int I, int SI, bool selected, 
 // Behind a small router every workgroup of eight waves repeats the router's matmul.  Mini layer, 96 workgroups a token, launch by
 // launch / this way: 1 token 14.0 / 11.6, 4 14.6 / 13.9, 5 15.2 / 14.6, 8 (768 workgroups) 15.4 / 17.9; behind its norm 1 14.8 / 12.8,
 // 2 15.1 / 12.9, 3 15.1 / 14.4, 4 15.2 / 15.3, 6 16.3 / 19.8.
-bool moe_token_fronts(int M, int k, int I, int SI, bool norm, bool from_memory) {
-  return !from_memory && (long long)M * ((k * I + SI) / COLS) <= (norm ? 320 : 512);
+//   One workgroup a CU gains with any router (10 to 30 %).  Where some CUs have two, the CU reads the router's weights twice, and the
+// line lies at their number (columns x D; this way against launch by launch): 320 to 512 workgroups without a norm, 33 K 0.93 to
+// 0.98, 42 K 0.99 to 1.01, 50 K 1.01 to 1.05, 66 K 1.06 to 1.09; behind a norm, 288 to 320, 25 K 0.92 to 0.99, 31 to 34 K 0.96 to 1.01, 44 K
+// 1.01 to 1.06, 66 K 1.08 to 1.12.  How many experts are chosen, and of which groups, changes little here.
+bool moe_token_fronts(int M, int k, int I, int SI, bool norm, bool from_memory, int router) {
+  const long long workgroups = (long long)M * ((k * I + SI) / COLS);
+  return !from_memory && (workgroups <= 256 || (workgroups <= (norm ? 320 : 512) && router <= (norm ? 34 : 42) * 1024));
 }
 
 int moe_token_experts(const TokenArgs& a, bool from_memory, const TokenRoute* route, moe_stream_t stream) {

@@ -48,6 +48,10 @@ int main() {
       int M, D, E, k, I, SI, norm;
       std::cin >> M >> D >> E >> k >> I >> SI >> norm;
       std::cout << moe_token_fronts(M, k, I, SI, norm, moe_gemm_from_memory(((long long)E * I + SI) * D)) << "\n";
+    } else if (what == "token_router") {   // the same of that router, with a column for the shared expert's gate
+      int M, D, E, k, I, SI, norm;
+      std::cin >> M >> D >> E >> k >> I >> SI >> norm;
+      std::cout << moe_token_fronts(M, k, I, SI, norm, moe_gemm_from_memory(((long long)E * I + SI) * D), (E + (SI > 0)) * D) << "\n";
     } else if (what == "stages") {   // tokens, D, experts, k, I, SI: K steps of a stage in the two launches of single tokens
       int M, D, E, k, I, SI;
       std::cin >> M >> D >> E >> k >> I >> SI;

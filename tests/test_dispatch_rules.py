@@ -132,6 +132,19 @@ def test_long_selections_are_not_repeated_by_many_workgroups(ask):
     assert ask(*[("token_chain", *c) for c in want]) == list(want.values())
 
 
+def test_wider_routers_are_repeated_by_one_workgroup_a_cu(ask):
+    """Behind a router the limit of workgroups is 256 where its weights are many; the batches that test_gpu_variants.py compares and
+    the mini layer's 3 (behind its norm) and 5 tokens are on the same sides as without that line."""
+    from tests.test_gpu_variants import FRONTED_TOKENS
+    assert ask(*[("token_router", *map(int, c)) for c in FRONTED_TOKENS]) == ask(*[("token_fronts", *map(int, c)) for c in FRONTED_TOKENS])
+    want = {(3, 1024, 64, 4, 256, 256, 0): "1", (3, 1024, 64, 4, 256, 256, 1): "1",      # 240 workgroups
+            (4, 1024, 64, 4, 256, 256, 0): "0", (4, 1024, 64, 4, 256, 256, 1): "0",      # 320, 65 K weights
+            (6, 768, 55, 4, 256, 256, 0): "1", (6, 768, 56, 4, 256, 256, 0): "0",        # 42 K and more
+            (4, 512, 67, 4, 256, 256, 1): "1", (4, 512, 68, 4, 256, 256, 1): "0",        # 34 K
+            (3, 1024, 32, 2, 512, 512, 1): "1", (5, 1024, 32, 2, 512, 512, 0): "1"}
+    assert ask(*[("token_router", *c) for c in want]) == list(want.values())
+
+
 def test_the_down_gemm_of_short_k_has_a_list_of_its_own(ask):
     """Tiles of 128 rows beside gate/up's full ones: more rows than one workgroup sorts, few K steps, enough items and not too many rows."""
     from tests.test_gpu_variants import TWO_LISTS
