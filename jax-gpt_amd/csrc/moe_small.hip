@@ -4,16 +4,19 @@
 // whose GEMMs read the selection themselves.  A workgroup owns 16 output columns of as many tokens as have 64 (or 128) selections,
 // whatever their experts; a lane holds a selection (or two).  Selections of one expert find each other by ballots of the id's bits;
 // every 16 of them are a unit of work, and so are 16 tokens of the shared expert.  A wave takes a unit through all of K in a ring of
-// its own -- 16 weight rows and 16 rows of h, no barrier, no other wave's copies to wait for -- and leaves its rows, rounded to bf16, in
+// its own -- 16 weight rows and 8 or 16 rows of h, no barrier, no other wave's copies to wait for -- and leaves its rows, rounded to bf16, in
 // LDS, where the workgroup adds a token's up in slot order.  The arithmetic of the grouped GEMM and the combine, instruction for
 // instruction: the same bits.
 //   What bounds it: a launch's start and its chain of dependent loads (ids, then rows and weights), then the bytes that a CU copies, some
-// 60 a ns.  A grouped GEMM has a work item for each 256 columns of an expert's rows, 40 of 288 KB for 256 tokens of 8 experts of 512 x
-// 1024, where 256 workgroups copy 192 KB here.  That launch and the combine 8.6 + 3.1 us, this one 6.2; the call 22.9 -> 17.7 us, 384
-// tokens 23.5 -> 20.7, 512 25.6 -> 21.4; 32 experts of 1024 x 512 with a shared one, 64 tokens 24.5 -> 21.6.
-//   Copies through LDS are what makes it: fragments loaded to registers are 64 bytes of each line, and the CU moves 38 bytes a ns
-// (20.3 us for the 17.7, 27.7 for the 22 of 512 tokens).  Sixteen waves a workgroup with rings of two K steps; eight with two or four are even
-// where there are no more units than waves, and slower where there are (mini, 64 tokens 21.6 / 23.7).
+// 70 a ns.  A unit copies 16 weight rows and 8 or 16 rows of h, whatever rows it has: some 240 KB a workgroup for 64 selections of 8
+// experts of 512 x 1024, of which 192 KB are distinct.  A grouped GEMM has a work item for each 256 columns of an expert's rows, 40 of 288 KB on 256 CUs for
+// 256 tokens of these.  That launch and the combine 8.6 + 3.1 us, this one 6.2; the call 22.9 -> 17.7 us, 384 tokens 23.5 -> 20.7, 512 25.6 ->
+// 21.4; 32 experts of 1024 x 512 with a shared one, 64 tokens 24.5 -> 21.6.
+//   Copies through LDS are what makes it: fragments loaded to registers are 64 bytes of each line, and the CU moves fewer bytes a ns
+// (20.3 us for the 17.7, 27.7 for the 22 of 512 tokens).  Sixteen waves a workgroup with rings of two K steps.  Nothing that a wave waits for
+// stands behind its copies: the unit's weight scales are copied in front of them.  With these in a register, whose first use in the K loop
+// waited for all copies at every step, and 16 rows of h for every unit: a shared expert of 256 x 4096 beside 8 small ones, 64 tokens 22.8 us a
+// call, so 18.6; tiny, 128 tokens 15.9 and 15.5.
 #include "moe_small.h"
 
 #include <math.h>
@@ -23,10 +26,11 @@ namespace {
 constexpr int BK = 128, COLS = 16;   // output columns of a workgroup
 
 constexpr int WAVES = 16, NST = 2;
-constexpr int kMostSteps = 64;           // K steps (a lane holds the weight scale of one)
+constexpr int kMostSteps = 64;           // K steps (a lane copies the weight scale of one)
 
-// LDS of a wave: NST stages of a K step, 16 weight rows and 16 rows of h with their scales (and 48 more)
+// LDS of a wave: NST stages of a K step, 16 weight rows and 16 rows of h with their scales (and 48 more), and the unit's weight scales
 constexpr int kStage = 2 * 16 * BK + 256;
+constexpr int kRing = NST * kStage, kWaveLds = kRing + kMostSteps * 4;
 
 // PL: selections of a lane
 template <int PL>
@@ -60,7 +64,7 @@ __global__ __launch_bounds__(64 * WAVES) void small_down_kernel(const SmallDown 
       if (a.shared_gate) gate[o] = a.shared_gate[t0 + t];
     }
   }
-  uint8_t* const ring = lds + w * (NST * kStage);
+  uint8_t* const ring = lds + w * kWaveLds;
   const unsigned ring_at = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)ring);
   if (tid < pairs) weight[tid] = a.w[p0 + tid];
   // each selection's place among those of its expert, and the first of every 16 of these: a unit
@@ -125,7 +129,7 @@ __global__ __launch_bounds__(64 * WAVES) void small_down_kernel(const SmallDown 
     const uint8_t* wp = (shared ? a.ws : a.wd) + ((size_t)e * a.D + ct * COLS) * K;
     const uint8_t* xp = (shared ? a.hsq : a.hq) + (size_t)row0 * K;
     const float* sx = (shared ? a.shs : a.sh) + (size_t)row0 * KB;
-    const float sw = ((shared ? a.sws : a.swd) + ((size_t)e * (a.D / BK) + ct / 8) * KB)[min(lane, KB - 1)];
+    const float* sw = (shared ? a.sws : a.swd) + ((size_t)e * (a.D / BK) + ct / 8) * KB;
     unsigned woff[2], xoff[2];
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
@@ -134,20 +138,24 @@ __global__ __launch_bounds__(64 * WAVES) void small_down_kernel(const SmallDown 
       xoff[g] = (unsigned)slot_of(r) * (unsigned)K + piece * 16;
     }
     const unsigned soff = (unsigned)slot_of(fr) * (unsigned)KB * 4u;
+    const bool wide = count > 8;
     auto copy = [&](int kb, int st) {
       const unsigned to = ring_at + st * kStage;
 #pragma unroll
       for (int g = 0; g < 2; ++g) dma16(wp + (size_t)kb * BK, woff[g], to + g * 1024u);
-#pragma unroll
-      for (int g = 0; g < 2; ++g) dma16(xp + (size_t)kb * BK, xoff[g], to + 2048u + g * 1024u);
+      dma16(xp + (size_t)kb * BK, xoff[0], to + 2048u);
+      if (wide) dma16(xp + (size_t)kb * BK, xoff[1], to + 3072u);
       dma4((const uint8_t*)(sx + kb), soff, to + 4096u);
     };
+    // (copied too, in front of the first stage: a load to a register would be waited for with everything behind it)
+    dma4((const uint8_t*)sw, (unsigned)min(lane, KB - 1) * 4u, ring_at + kRing);
     for (int t = 0; t < NST && t < KB; ++t) copy(t, t);
     v4f acc = {0.f, 0.f, 0.f, 0.f};
     int st = 0;
     for (int kb = 0; kb < KB; ++kb) {
-      if (KB - kb >= NST) wait_vm<5 * (NST - 1)>();
-      else wait_vm<0>();
+      if (KB - kb < NST) wait_vm<0>();
+      else if (wide) wait_vm<5 * (NST - 1)>();
+      else wait_vm<4 * (NST - 1)>();
       asm volatile("" ::: "memory");
       const uint8_t* base = ring + st * kStage;
       auto frag = [&](const uint8_t* p) {
@@ -155,7 +163,7 @@ __global__ __launch_bounds__(64 * WAVES) void small_down_kernel(const SmallDown 
         return (v8i){lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
       };
       const v8i wf = frag(base), xf = frag(base + 2048);
-      const float c = ((const float*)(base + 4096))[fr] * __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(sw), kb));
+      const float c = ((const float*)(base + 4096))[fr] * ((const float*)(ring + kRing))[kb];
       if (kb + NST < KB) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the fragments are in registers: the stage may be overwritten
         copy(kb + NST, st);
@@ -197,19 +205,20 @@ __global__ __launch_bounds__(64 * WAVES) void small_down_kernel(const SmallDown 
 // A group of tokens reads every expert's rows that it has a selection of again, so this is for batches that one workgroup a CU covers,
 // with 64 selections a workgroup or, where these are too many workgroups, with 128 (two of those on a CU are slower than 128: tiny, 384
 // tokens 20.6 / 22.7 us, mini 256 24.8 / 29.3, tiny 700 as 704 of 64 or 352 of 128 29.2 / 28.7 for 26.2 of the three launches).
-// Of these up to 600 and 400 KB a workgroup, by the experts that an even routing touches (three launches / this way, us a call, even
-// routing, then normal offsets of 2 on the logits): 32 experts of 1024 x 512 with a shared one, 128 tokens (one lane's selections, 350
-// KB) 24.7 / 22.7 and 23.4 / 18.8, 256 (two, 360 KB) 25.6 / 24.8 and 24.6 / 21.2; 32 of 1024 x 1024, 64 tokens of 4 (one, 510 KB) 30.7 /
-// 30.3 and 28.2 / 22.6, 128 (two, 640 KB) 31.0 / 32.6 and 32.7 / 27.2; 8 of 2048 x 2048 with one, 96 (two, 540 KB) 34.6 / 35.9
-// and 34.8 / 34.7; 48 of 512 x 1024, 128 (one, 630 KB) 30.1 / 32.5 and 28.3 / 20.6; 64 of 1024 x 512, 64 of 8 (two, 510 KB)
-// 31.7 / 33.6 and 27.3 / 23.0; 32 of 1024 x 2048, 96 of 2 (one, 1 MB) 44.6 / 49.8 and 34.1 / 29.9.  (Uneven routings touch fewer.)
+// Of these up to 500 KB of copies a workgroup, counted for an even routing: uneven ones have fewer units and gain more.  This way against
+// three launches, even and uneven (normal offsets of 1 on the logits) routing, 8 to 64 experts of 256 to 2048 x 256 to 2048: with 64 selections
+// up to 500 KB 0.74 to 0.99 and 0.74 to 0.92, up to 600 0.73 to 1.10 (64 experts of 256 x 512 1.02 to 1.09) and 0.75 to 0.97, up to 1000 0.81
+// to 1.14 and 0.81 to 1.00; with 128 up to 500 0.82 to 1.01 and 0.83 to 0.95, up to 600 0.83 to 1.01 and 0.81 to 1.00, up to 1000 0.86 to 1.19
+// and 0.84 to 1.05.
 int moe_small_down_lanes(int M, int D, int E, int k, int I, int SI) {
   if (M < 1 || E > 64 || k < 1 || k > 32 || I > kMostSteps * BK || SI > kMostSteps * BK) return 0;
   for (int lanes = 1; lanes <= 2; ++lanes) {
     const int tokens = 64 * lanes / k, most = tokens < M ? tokens : M;
     if ((long long)((M + tokens - 1) / tokens) * (D / COLS) > 256) continue;
-    const double touched = E * (1.0 - pow(1.0 - 1.0 / E, most * k));
-    return COLS * (touched * I + SI) + (double)most * (k * I + SI) <= (lanes == 1 ? 600 : 400) * 1024.0 ? lanes : 0;
+    const double touched = E * (1.0 - pow(1.0 - 1.0 / E, most * k)), rows = most * k / touched;   // experts, and rows of each
+    // a K step's KB of units of 16 rows: weights and scales, and h eight rows at a time
+    auto step = [](double rows) { return 2.25 * ceil(rows / 16 - 1e-9) + ceil(rows / 8 - 1e-9); };
+    return touched * step(rows) * (I / BK) + step(most) * (SI / BK) <= 500 ? lanes : 0;
   }
   return 0;
 }
@@ -217,7 +226,7 @@ int moe_small_down_lanes(int M, int D, int E, int k, int I, int SI) {
 namespace {
 template <int PL> int launch(const SmallDown& a, hipStream_t s) {
   static std::atomic<unsigned long long> raised = {};
-  const int tokens = 64 * PL / a.k, groups = (a.M + tokens - 1) / tokens, lds = WAVES * NST * kStage;
+  const int tokens = 64 * PL / a.k, groups = (a.M + tokens - 1) / tokens, lds = WAVES * kWaveLds;
   if (int rc = moe_raise_lds_limit((const void*)small_down_kernel<PL>, lds, raised)) return rc;
   hipLaunchKernelGGL(small_down_kernel<PL>, dim3((unsigned)groups * (a.D / COLS)), dim3(64 * WAVES), lds, s, a, tokens);
   return moe_check_hip(hipGetLastError(), "small layer's down launch");

@@ -181,6 +181,16 @@ def test_small_layers_down_launch_is_for_one_workgroup_a_cu(ask):
     assert ask(*[("small", *c) for c in limits]) == list(limits.values())
 
 
+def test_small_layers_down_launch_is_for_few_units(ask):
+    """By what a workgroup copies, 16 weight rows for every unit, which is more where many experts have a row or two each."""
+    want = {(64, 256, 64, 2, 512, 1024): "0", (128, 256, 64, 2, 512, 512): "0", (128, 512, 64, 4, 640, 512): "0", (17, 512, 64, 2, 1024, 0): "0",
+            (32, 512, 32, 4, 1024, 0): "0", (32, 256, 64, 8, 512, 0): "0", (32, 256, 64, 8, 256, 0): "1", (128, 1024, 32, 2, 512, 512): "1", (256, 1024, 32, 2, 512, 512): "2"}
+    assert ask(*[("small", *c) for c in want]) == list(want.values())
+    from tests.test_gpu_variants import UNITS
+    assert ask(*[("small", sum(c) // k, D, E, k, I, SI) for c, D, E, k, I, SI in UNITS]) == ["1", "1", "2"]
+    assert all(int(r) for r in ask(*[("scan", sum(c) // k, D, E, k, I, SI) for c, D, E, k, I, SI in UNITS]))
+
+
 def test_the_compared_batches_of_single_tokens_reach_what_they_are_for(ask):
     """The batches that test_gpu_variants.py compares with the grouped route take the other one, and among them are: a last
     workgroup of fewer tiles, one over two scale blocks, more slots than waves, waves that LDS limits, weights from memory."""

@@ -941,6 +941,42 @@ def test_small_layers_down_launch_gives_the_bits_of_down_and_combine(jg, M, D, E
         assert torch.equal(got, want.bfloat16())
 
 
+UNITS = [   # selections of each expert, D, E, k, I, SI
+    ((8, 9, 16, 17, 7, 1), 256, 6, 1, 384, 0),        # whole and half units of h, an odd number of K steps
+    ((24, 25, 1, 6, 8), 384, 9, 2, 128, 256),         # one K step; a shared expert; experts without rows
+    ((33, 40, 8, 9, 2, 64, 124), 1024, 8, 2, 512, 0), # two selections a lane
+]
+
+
+@pytest.mark.parametrize("counts,D,E,k,I,SI", UNITS)
+def test_small_layers_units_of_any_rows_give_the_grouped_bits(jg, counts, D, E, k, I, SI):
+    """Units of 1 to 8, 9 to 15 and 16 rows, also where rows are zero or hold infinities and NaN, against the same tokens often enough
+    for a sort."""
+    import torch
+    print("units of rows", counts, D, E, k, I, SI, flush=True)
+    params, rand = _layer(jg, D, E, I, SI, D + I)
+    names = ("gate_proj", "up_proj", "down_proj")
+    same = lambda a, b: torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(7.0, float("inf"), -float("inf")), b.nan_to_num(7.0, float("inf"), -float("inf")))
+    flat = np.repeat(np.arange(len(counts)), counts)
+    M = len(flat) // k
+    flat = H.rng_for(D).permutation(flat)[:M * k].reshape(M, k).astype(np.int32)
+    idx, w = H.to_cuda(flat), torch.rand(M, k, device="cuda")
+    for hard in (False, True):
+        x = rand(M, D)
+        if hard:
+            x[0] = 0
+            x[1, 5], x[2, 7], x[M - 1, D - 1] = float("inf"), float("nan"), -3e38
+        if SI:   # (ready logits that select these: the chosen ones are the largest)
+            lg = torch.full((M, E), -4.0, device="cuda").scatter_(1, (idx.long() + torch.arange(k, device="cuda") * 3) % E, 1.0)
+            run = lambda n: jg.moe_experts(x.repeat(n, 1), lg.repeat(n, 1), top_k=k, experts={n_: params[n_] for n_ in names},
+                                           shared={n_: params["shared_" + n_] for n_ in names})
+        else:
+            run = lambda n: jg.expert_forward_single(x.repeat(n, 1), idx.repeat(n, 1), w.repeat(n, 1), *(params[n_] for n_ in names))
+        got, many = run(1), run(2048 // (M * k) + 1)
+        assert same(got, many[:M]) and same(got, many[-M:])
+        assert same(run(1), got)
+
+
 @pytest.mark.parametrize("E,N,K,dtype", [(9, 2560, 2560, "bf16"), (9, 2560, 2688, "bf16"), (11, 2560, 2432, "f32"), (25, 512, 512, "f32")])   # two blocks wide; an odd number of blocks; sixteen waves; four, its experts eight
 def test_large_weight_arrays_give_the_bits_of_their_experts(jg, E, N, K, dtype):
     import torch
