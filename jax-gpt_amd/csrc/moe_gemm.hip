@@ -984,7 +984,7 @@ int moe_gemm_tile_rows(const TileShape& t) {
 }
 
 // The two GEMMs want different heights where K of the down GEMM is short: tall tiles for gate/up, and for down 128 rows, which the kernel
-// with two workgroups a CU takes (moe_gemm_stream.hip), because start and end are a good part of an item of 6 or 8 K steps and another
+// with two workgroups a CU takes (moe_gemm_stream.hip), because start and end are a good part of an item of up to 8 K steps and another
 // workgroup works meanwhile.  The placing launch writes both lists, in two workgroups.  The down launch alone, gate/up's list / its own, even
 // routing or uneven by normal offsets of 1 and 2 on the logits: Qwen3-MoE (6 K steps), 400 tokens 39.6 / 36.5 us, 1000 47.0 / 41.4, 2000
 // 63.0 / 55.6 and 60.4 / 56.8 and 49.2 / 46.2, 3000 71.8 / 64.8; full layer (8), 1000 389 / 367, 2047 405 / 381, 312 / 307 and 188 / 180.
@@ -992,11 +992,24 @@ int moe_gemm_tile_rows(const TileShape& t) {
 // rows an expert) 217.5 / 215.9, 231.7 / 221.2 and 218.1 / 206.7, 3800 (238) 241.6 / 245.3, 269.6 / 262.1 and 241.0 / 234.2, 5000 323.9 / 322.7,
 // 313.6 / 309.2 and 308.2 / 309.7; full layer, 900 tokens 1046 / 1025, 692 / 678 and 324 / 318, 3000 (59 rows) 1216 / 1200, 1034 /
 // 1033 and 668 / 667, 4096 (80) 1315 / 1299, 1191 / 1198 and 879 / 884; DeepSeek-V3 (16 K steps), 777 (24) 1376 / 1378, 1058 / 1082 and
-// 519 / 523.
+// 519 / 523.  Two lists (and the weights' scales in front of the copies, 1 to 3 %) against one without these, 128 experts of 2048 x 128 to
+// 1024 (1 to 8 K steps), k = 8, and others of 512 to 7168 x 256 to 768, 17 to 195 rows an expert, even routing and offsets of 1 and 4: 0.79 to
+// 1.02, on average 0.96; above 1.005 at six of 288, four of them with an offset of 4, where a few experts have most rows.
+//   A shared expert of long K beside is cut into short tiles too, and one such item can outlast the launch: not where it has more than 16
+// K steps, and 7/4 of those that a place (two workgroups a CU) has on average, unless the shared expert is one tall tile or two thirds of
+// the routed work.  Qwen3-MoE beside a shared expert of 3072 (24 K steps), 384 tokens 139 / 142 us, 640 151 / 150; of 4096, 384 140 / 150, 640 155 / 161,
+// 960 171 / 174; of 6144, 272 189 / 152, 384 151 / 167, 640 172 / 183, 1200 206 / 212, 1440 230 / 223; 256 experts of 1024 x 512 beside
+// one of 4096, 640 117 / 122; of 4096 x 512 beside one of 4096, 544 352 / 335.
 int moe_gemm_down_tile_rows(const TileShape& t, int list_rows) {
   const int groups = t.E < t.R ? t.E : t.R;
   if (t.R <= kSmallRows || t.R > kFullTileItems * kTileRows || list_rows <= kStreamRows || list_rows > kTileRows) return 0;
-  return (long long)groups * t.ncb[1] >= kStreamItems && t.kb[1] <= 8 && t.R <= (t.kb[1] <= 6 ? 200ll : 64ll) * t.E ? kStreamRows : 0;
+  if ((long long)groups * t.ncb[1] < kStreamItems || t.kb[1] > 8 || t.R > (t.kb[1] <= 6 ? 200ll : 64ll) * t.E) return 0;
+  const int dense_kb = t.dense_ncb[0];   // (the shared expert's columns in gate/up)
+  if (t.dense_rows > list_rows && dense_kb > 16) {
+    const long long routed = (long long)groups * t.ncb[1] * t.kb[1], dense = (long long)moe_tile_count(t.dense_rows, kStreamRows) * t.dense_ncb[1] * dense_kb;
+    if (4ll * 512 * dense_kb > 7 * (routed + dense) && 3 * dense < 2 * routed) return 0;
+  }
+  return kStreamRows;
 }
 
 // Batches whose GEMMs read the selection themselves: few rows of few experts whose launches are ones of the class kernel with plain

@@ -156,6 +156,16 @@ def test_the_down_gemm_of_short_k_has_a_list_of_its_own(ask):
     assert ask(*[("down_list", *c[:6]) for c in TWO_LISTS]) == ["288 128"] * len(TWO_LISTS)
 
 
+def test_a_shared_expert_of_long_k_keeps_the_list_of_tall_tiles(ask):
+    """Where one item of its short tiles would outlast the launch; not where it is one tall tile, or most of the work, or where the
+    routed experts' items take as long."""
+    want = {(384, 2048, 128, 8, 768, 2048): True, (384, 2048, 128, 8, 768, 3072): False, (640, 2048, 128, 8, 768, 3072): True,
+            (384, 2048, 128, 8, 768, 6144): False, (1200, 2048, 128, 8, 768, 6144): False, (1440, 2048, 128, 8, 768, 6144): True,
+            (272, 2048, 128, 8, 768, 6144): True, (544, 4096, 256, 8, 512, 4096): True,
+            (640, 1024, 256, 8, 512, 4096): False, (384, 2048, 128, 8, 768, 0): True, (2047, 4096, 512, 10, 1024, 1024): True}
+    assert [int(a.split()[1]) > 0 for a in ask(*[("down_list", *c) for c in want])] == list(want.values())
+
+
 def test_small_layers_read_the_selection_themselves(ask):
     """Few rows of few experts from the caches, in tiles of up to 128 rows; not where a list's tiles are taller for a reason, nor
     where the short-tile kernel takes the launch."""
