@@ -203,7 +203,7 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
   const int R = a->M * a->k;
   // large batches read their activation scales from block-major arrays (GemmScales); a decode-sized batch touches
   // few scale lines either way and is spared the extra launch
-  const bool blocked_scales = R > 2048;
+  const bool blocked_scales = R > kSmallRows;
   hipStream_t main_s = (hipStream_t)stream;
   MOE_REQUIRE(given_idx || a->routing == MOE_ROUTING_SOFTMAX || a->routing == MOE_ROUTING_SIGMOID_GROUPED, MOE_ERR_BAD_SHAPE,
               "forward: unknown routing %d", a->routing);
@@ -373,19 +373,10 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
                                (down_rows || a->D < a->I ? a->D : a->I) / 128, b.gemm_ws, b.gemm_ws_bytes, &tiles))) return join(rc);
   if (down_rows && (rc = moe_gemm_tile_list(R, a->E, down_rows, 0, (a->D + 255) / 256, a->I / 128, b.gemm_down_ws, b.gemm_ws_bytes, &down_tiles)))
     return join(rc);
-  // Gathering the activation scales is a launch (5 us); reading them row-major costs the gate/up GEMM a line per row and K
-  // step, which short tiles of a short launch hide.  Gathered against not: Qwen3-MoE (K blocks x column blocks = 96), 300
-  // tokens 124.6 / 121.9 us, 1024 145.5 / 142.9, 1500 163.0 / 162.4, 2000 189.0 / 191.3; mini layer, 1100 tokens 52.9 / 51.8;
-  // DeepSeek-V3 (896), 300 tokens 1176 / 1179, 1100 1530 / 1547.
-  const bool gather_x = blocked_scales && (R > 96ll * a->E || (long long)R * (a->D / 128) * (a->I / 128) > (1ll << 20));
-  // Few scales are written by the placing launch (the quantiser is in front of it where nothing is forked): no launch, but writes of
-  // four bytes.  Launch by launch / this way: tiny, 1100 tokens 36.2 / 33.9, 8192 76.7 / 75.2; mini sublayer, 2000 52.0 / 50.8, 9000 133.1 / 131.8;
-  // Qwen3-MoE, 1600 165.4 / 162.4, 2000 (256 K scales) 179.8 / 176.4, 4096 243.6 / 245.8; rows of 32 scales, full layer, 600 1016 / 1019, 1000
-  // 1046 / 1050; of 56, DeepSeek-V3, 300 and 777 even.
-  const bool placed_x = gather_x && !fork && a->D <= 2048 && (long long)R * (a->D / 128) <= (1ll << 18);
+  const ScalePlan plan = moe_scale_plan(R, a->E, a->D, a->I, fork);
   const ScaleGather gather{b.sx, a->D / 128, b.sx_listed};
-  const PlaceMore more{down_rows ? &down_tiles : nullptr, placed_x ? &gather : nullptr};
-  const PermuteOut sort{gsz, b.group_offsets, stid, nullptr, inv, a->k, tiles, down_rows || placed_x ? &more : nullptr};
+  const PlaceMore more{down_rows ? &down_tiles : nullptr, plan.placed ? &gather : nullptr};
+  const PermuteOut sort{gsz, b.group_offsets, stid, nullptr, inv, a->k, tiles, down_rows || plan.placed ? &more : nullptr};
   rc = given_idx ? moe_permute_impl(given_idx, a->M, a->k, a->E, sort, b.permute_ws, b.permute_ws_bytes, carried, stream)
                  : select(&sort);
   if (rc) return join(rc);
@@ -396,8 +387,8 @@ static int forward(const MoeForwardArgs* a, int io_f32, const int32_t* given_idx
   GemmScales sc = moe_row_major_scales(a->D, a->I);
   const float* sx_routed = b.sx;
   if (blocked_scales && !a->out_sh) sc.out_row = 1, sc.out_cb = R;
-  if (gather_x) {
-    if (!placed_x && (rc = moe_gather_scales(b.sx, stid, R, a->D / 128, b.sx_listed, stream))) return join(rc);
+  if (plan.gathered) {
+    if (!plan.placed && (rc = moe_gather_scales(b.sx, stid, R, a->D / 128, b.sx_listed, stream))) return join(rc);
     sx_routed = b.sx_listed;
     sc.in_row = 1, sc.in_kb = R, sc.in_listed = true;
   }

@@ -350,6 +350,10 @@ struct PlaceMore {
   const TileList* tl_down;     // a list of its own for the down GEMM, or null: it reads PermuteOut::tl
   const ScaleGather* gather;   // or null
 };
+// How the routed gate/up GEMM finds its activation scales: block-major in sorted order (gathered; placed: by the placing launch) or in the
+// quantiser's rows.  forked: the quantiser may run beside the sort
+struct ScalePlan { bool gathered, placed; };
+ScalePlan moe_scale_plan(int R, int E, int D, int I, bool forked);
 // What the sort by expert writes (sort_order, sorted_token_ids, inv_perm: null to skip; tl.tiles null: no work list).
 struct PermuteOut {
   int32_t *group_sizes, *group_offsets, *sorted_token_ids, *sort_order, *inv_perm;

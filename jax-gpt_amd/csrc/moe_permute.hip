@@ -39,9 +39,9 @@ __global__ __launch_bounds__(kHistThreads) void hist_kernel(const int32_t* __res
   for (int e = threadIdx.x; e < E; e += kHistThreads) chunk_hist[(size_t)blockIdx.x * E + e] = hist[e];
 }
 
-// TWO: there is a second work list, l2, for the same experts (a kernel of its own: with both lists' arguments in all launches, and the
-// choice between them, Qwen3-MoE of 4096 tokens took 1.2 us more).  GATHER: the entries' activation scales are written to their places too
-// (more arguments for all launches: Qwen3-MoE of 1000 tokens +0.6 us)
+// TWO: there is a second work list, l2, for the same experts (a kernel of its own: with the choice between them in all launches Qwen3-MoE of
+// 4096 tokens took 1.2 us more).  GATHER: the entries' activation scales are written to their places too, and what that needs stands where
+// the quantiser's arguments do, which a list of several chunks has none of (as an argument more, Qwen3-MoE of 1000 tokens +0.6 us).
 template <bool TWO, bool GATHER>
 __global__ __launch_bounds__(kPlaceThreads) void place_kernel(const int32_t* __restrict__ ids, int R, int E, int chunk,
                                                              int n_chunks, const int32_t* __restrict__ chunk_hist,
@@ -136,6 +136,20 @@ int moe_permute_max_chunks(int E) {
 extern "C" size_t moe_permute_workspace_bytes(int M, int k, int E) {
   (void)M, (void)k;
   return E > 0 ? (size_t)moe_permute_max_chunks(E) * E * sizeof(int32_t) + 256 : 256;
+}
+
+// Gathering the activation scales is a launch (5 us); reading them row-major costs the gate/up GEMM a line per row and K
+// step, which short tiles of a short launch hide.  Gathered against not: Qwen3-MoE (K blocks x column blocks = 96), 300
+// tokens 124.6 / 121.9 us, 1024 145.5 / 142.9, 1500 163.0 / 162.4, 2000 189.0 / 191.3; mini layer, 1100 tokens 52.9 / 51.8;
+// DeepSeek-V3 (896), 300 tokens 1176 / 1179, 1100 1530 / 1547.
+//   Few scales are written by the placing launch (the quantiser is in front of it where nothing is forked): no launch, but writes of
+// four bytes.  Launch by launch / this way: tiny, 1100 tokens 36.2 / 33.9, 8192 76.7 / 75.2; mini sublayer, 2000 52.0 / 50.8, 9000 133.1 / 131.8;
+// Qwen3-MoE, 1600 165.4 / 162.4, 2000 (256 K scales) 179.8 / 176.4, 4096 243.6 / 245.8; rows of 32 scales, full layer, 600 1016 / 1019, 1000
+// 1046 / 1050; of 56, DeepSeek-V3, 300 and 777 even.
+ScalePlan moe_scale_plan(int R, int E, int D, int I, bool forked) {
+  const long long scales = (long long)R * (D / 128);
+  const bool gathered = R > kSmallRows && (R > 96ll * E || scales * (I / 128) > (1ll << 20));
+  return {gathered, gathered && !forked && D <= 2048 && scales <= (1ll << 18)};
 }
 
 int moe_permute_place(const int32_t* idx, int R, int E, int chunk, int n_chunks, const int32_t* chunk_hist, const PermuteOut& o,

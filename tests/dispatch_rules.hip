@@ -23,6 +23,11 @@ int main() {
       std::cin >> M >> D >> E >> k >> I >> SI;
       const TileShape t{M * k, E, M, {I / 128, (D + 255) / 256}, {D / 128, I / 128}, SI ? M : 0, {SI / 128, (D + 255) / 256}};
       std::cout << moe_gemm_tile_rows(t) << " " << moe_gemm_down_tile_rows(t, moe_gemm_tile_rows(t)) << "\n";
+    } else if (what == "scales") {   // tokens, D, experts, k, I, forked: whether gate/up's activation scales are gathered, and by the placing launch
+      int M, D, E, k, I, forked;
+      std::cin >> M >> D >> E >> k >> I >> forked;
+      const ScalePlan p = moe_scale_plan(M * k, E, D, I, forked);
+      std::cout << p.gathered << " " << p.placed << "\n";
     } else if (what == "scan") {   // tokens, D, experts, k, I, SI: rows of a full tile where the GEMMs read the selection, or 0
       int M, D, E, k, I, SI;
       std::cin >> M >> D >> E >> k >> I >> SI;

@@ -156,6 +156,17 @@ def test_the_down_gemm_of_short_k_has_a_list_of_its_own(ask):
     assert ask(*[("down_list", *c[:6]) for c in TWO_LISTS]) == ["288 128"] * len(TWO_LISTS)
 
 
+def test_scales_are_placed_with_their_rows_where_they_are_few(ask):
+    """The batches that test_gpu_variants.py compares: placed, or by a launch of their own; beside two work lists one of each kind, and their
+    parts, which one workgroup sorts, read them in place."""
+    from tests.test_gpu_variants import PLACED, TWO_LISTS
+    assert ask(*[("scales", M, D, 12, 2, 128, 0) for M, D in PLACED]) == ["1 1"] * 4 + ["1 0"] * 2
+    assert ask(*[("scales", 500, D, 12, 2, 128, 0) for M, D in PLACED]) == ["0 0"] * 6
+    assert ask(*[("scales", M, D, E, k, I, 0) for M, D, E, k, I, SI, offset in TWO_LISTS]) == ["0 0", "1 0", "1 1", "0 0", "0 0"]
+    assert ask(("scales", 8192, 2048, 12, 2, 128, 1), ("scales", 4096, 2048, 128, 8, 768, 0), ("scales", 2000, 2048, 128, 8, 768, 0),
+               ("scales", 777, 7168, 256, 8, 2048, 0), ("scales", 1024, 2048, 128, 8, 768, 0)) == ["1 0", "1 0", "1 1", "1 0", "0 0"]
+
+
 def test_a_shared_expert_of_long_k_keeps_the_list_of_tall_tiles(ask):
     """Where one item of its short tiles would outlast the launch; not where it is one tall tile, or most of the work, or where the
     routed experts' items take as long."""

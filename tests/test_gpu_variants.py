@@ -294,7 +294,10 @@ def test_scale_layouts_of_middle_sized_batches_give_the_same_bits(jg, M, E):
     assert torch.equal(whole[:400], jg.moe_experts(x[:400].contiguous(), lg[:400].contiguous(), **kw))
 
 
-@pytest.mark.parametrize("M,D", [(1030, 128), (1030, 384), (4097, 640), (8192, 2048), (8193, 2048), (1100, 2176)])   # the last two: by a launch of its own
+PLACED = [(1030, 128), (1030, 384), (4097, 640), (8192, 2048), (8193, 2048), (1100, 2176)]   # M, D; the last two: by a launch of its own
+
+
+@pytest.mark.parametrize("M,D", PLACED)
 def test_scales_that_the_sort_places_give_the_bits_of_rows_read_in_place(jg, M, D):
     """1, 3, 5, 16 and 17 scales a row, up to 2^18 of them and above, with dropped entries of a given selection and without."""
     import torch
