@@ -167,6 +167,14 @@ def test_scales_are_placed_with_their_rows_where_they_are_few(ask):
                ("scales", 777, 7168, 256, 8, 2048, 0), ("scales", 1024, 2048, 128, 8, 768, 0)) == ["1 0", "1 0", "1 1", "1 0", "0 0"]
 
 
+def test_selections_that_a_quantiser_goes_in_front_of(ask):
+    """The dropped entries that test_gpu_variants.py compares: read by the launch that quantises too, and by the one that does not."""
+    from tests.test_gpu_variants import DROPPED
+    inside = [(M, 512, 10, k, 256, 0) for M, k in ((1, 2), (5, 3), (16, 8))]
+    assert ask(*[("token", *c) for c in inside + [DROPPED]]) == ["1"] * 4
+    assert ask(*[("token_selected", *c) for c in inside + [DROPPED]]) == ["1", "1", "1", "0"]
+
+
 def test_a_shared_expert_of_long_k_keeps_the_list_of_tall_tiles(ask):
     """Where one item of its short tiles would outlast the launch; not where it is one tall tile, or most of the work, or where the
     routed experts' items take as long."""

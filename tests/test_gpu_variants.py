@@ -705,7 +705,7 @@ def test_small_routers_of_single_tokens_give_the_grouped_bits(jg, M, D, E, k, I,
             assert same(run(), run(return_debug=True)[0]), (kind, f32)
 
 
-@pytest.mark.parametrize("M,k", [(1, 2), (5, 3), (16, 8),     # straight to the experts: both of its kernels leave the rows out
+@pytest.mark.parametrize("M,k", [(1, 2), (5, 3), (16, 8),     # straight to the experts, read by their first launch, which quantises too
                                  (17, 1), (32, 1), (17, 3),   # the sort without counters, and with them
                                  (700, 2), (1100, 2), (3000, 3)])   # scales read row-major, and gathered; several chunks
 def test_selected_experts_that_there_are_not_count_as_zero_rows(jg, M, k):
@@ -736,6 +736,30 @@ def test_selected_experts_that_there_are_not_count_as_zero_rows(jg, M, k):
     assert torch.equal(jg.gather_scales(sx, p["sorted_token_ids"]), sx[p["sorted_token_ids"].long()].t())
     assert np.array_equal(p["inv_perm"].cpu().numpy(), inv) and int(p["group_offsets"][-1]) == n
     assert np.array_equal(p["group_sizes"].cpu().numpy(), np.bincount(bad.reshape(-1)[flat], minlength=E))
+
+
+DROPPED = (16, 512, 128, 8, 1024, 0)   # more workgroups than run at once: the first launch finds the tokens quantised
+
+
+def test_selected_experts_that_there_are_not_leave_their_workgroups(jg):
+    """The same of the first launch behind a quantiser of its own: workgroups without an expert end with copies under way."""
+    import torch
+    print("dropped entries of many workgroups", flush=True)
+    M, D, E, k, I, _ = DROPPED
+    params, rand = _layer(jg, D, E, I, 0, 5)
+    ex = [params[n] for n in ("gate_proj", "up_proj", "down_proj")]
+    rng = H.rng_for(11)
+    idx = rng.integers(0, E, (M, k)).astype(np.int32)
+    drop = rng.random((M, k)) < 0.4
+    drop[3] = True
+    w, x = np.abs(rng.standard_normal((M, k))).astype(np.float32), rand(M, D)
+    bad = np.where(drop, rng.choice([-1, E, 2 ** 31 - 1, -2 ** 31], (M, k)), idx).astype(np.int32)
+    for _ in range(3):
+        got = jg.expert_forward_single(x, H.to_cuda(bad), H.to_cuda(w), *ex)
+        want = jg.expert_forward_single(x, H.to_cuda(idx), H.to_cuda(np.where(drop, np.float32(0), w)), *ex)
+        assert torch.equal(got, want) and not got[3].any()
+    many = jg.expert_forward_single(x.repeat(20, 1), H.to_cuda(bad).repeat(20, 1), H.to_cuda(w).repeat(20, 1), *ex)   # (sorted)
+    assert torch.equal(got, many[:M])
 
 
 @pytest.mark.parametrize("E", [256, 257, 512, 640])
