@@ -108,8 +108,7 @@ ForwardBuffers carve(void* ws, int M, int D, int E, int k, int I, int SI, bool r
   b.permute_ws_bytes = moe_permute_workspace_bytes(M, k, E);
   b.permute_ws = c.take(b.permute_ws_bytes);
   b.gemm_ws_bytes = moe_gemm_workspace_bytes((int)R, E, I > D ? I : D);
-  b.gemm_ws = c.take(b.gemm_ws_bytes);        // tile list of the routed GEMMs, and
-  b.gemm_down_ws = c.take(b.gemm_ws_bytes);   // the down GEMM's own, if it has one
+  b.gemm_ws = c.take(b.gemm_ws_bytes);   // tile list of the routed GEMMs
   b.xq = (uint8_t*)c.take((size_t)M * D);
   b.sx = (float*)c.take((size_t)M * (D / 128) * 4);
   // block-major copies of the activation scales for large batches (GemmScales): routed rows in sorted order,
@@ -126,7 +125,10 @@ ForwardBuffers carve(void* ws, int M, int D, int E, int k, int I, int SI, bool r
   const size_t few = M < MOE_TOKEN_ROWS ? M : MOE_TOKEN_ROWS;
   b.h32 = (float*)c.take(few * (k + 1) * (I > SI ? I : SI) * 4);   // h of single tokens
   b.router_ws_bytes = router ? moe_router_workspace_bytes(M, D, E) : 0;
-  b.router_ws = router ? c.take(b.router_ws_bytes) : nullptr;
+  // The router's sums and, once the routing launch has added them up, the down GEMM's own list, if it has one (lists of several chunks: the
+  // placing launch that writes them stands behind the routing launch).
+  const size_t down_list = R > kSmallRows ? b.gemm_ws_bytes : 0;
+  b.router_ws = b.gemm_down_ws = router ? c.take(b.router_ws_bytes > down_list ? b.router_ws_bytes : down_list) : nullptr;
   b.normed = router ? c.take((size_t)M * D * 2) : nullptr;   // RMS-normalised activations (norm_weight)
   b.total = c.used;
   return b;

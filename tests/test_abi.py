@@ -104,6 +104,14 @@ def test_argument_errors_come_back_as_codes(dll):
     assert dll.moe_forward(None, one, 0, None) == -5
 
 
+def test_workspace_of_a_layer_call_has_not_grown(dll):
+    """A caller may have sized its scratch memory once: what was enough before the down GEMM had a list of its own still is."""
+    was = {(256, 512, 8, 2, 1024, 0): 1723136, (1, 1024, 32, 2, 512, 512): 55040, (8192, 7168, 256, 8, 2048, 2048): 1443306752,
+           (4096, 2048, 128, 8, 768, 0): 222384384, (2047, 4096, 512, 10, 1024, 1024): 271416064, (1, 7168, 256, 8, 2048, 2048): 570112}
+    for shape, size in was.items():
+        assert dll.moe_forward_workspace_bytes(*shape) <= size, shape
+
+
 def test_workspace_sizes_are_monotone(dll):
     a = dll.moe_forward_workspace_bytes(64, 7168, 256, 8, 2048, 2048)
     b = dll.moe_forward_workspace_bytes(8192, 7168, 256, 8, 2048, 2048)
