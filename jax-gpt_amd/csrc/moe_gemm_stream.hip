@@ -100,6 +100,7 @@ __device__ __forceinline__ void stream_item(const Item& item, uint8_t* lds, cons
     copy_x(t, t);
     copy_w(t, t);
   }
+  // (loads to registers behind the copies: the first step waits for all of these, where the class kernel copies its scales in front of them)
   float* wscale = (float*)(lds + wscale_off(nst, BM));
   for (int i = tid; i < 2 * KB; i += NT) {
     const int h = i >= KB, kk = h ? i - KB : i;

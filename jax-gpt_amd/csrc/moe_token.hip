@@ -10,22 +10,23 @@
 // the Qwen3-MoE layer, on 256 CUs) because a quantisation group of h must not cross workgroups.  Here h stays in f32 between
 // the two launches and every wave of the second quantises the row that it multiplies -- a few KB from L2 -- so the first
 // launch's workgroups can be single waves of 16 columns (1152 and 384).  In the second a workgroup owns tiles of 16 output
-// columns of a token, one wave a slot, and adds the slots up itself: no y, no third launch.  Against the grouped route (us,
-// one token): DeepSeek-V3 layer 84 -> 76, Qwen3-MoE 28 -> 20, full layer behind its norm 57.5 -> 45, mini 31 -> 27, tiny
-// 23 -> 20; five tokens of Qwen3-MoE 46 -> 38.5, eight 55 -> 50.5; sixteen of the mini layer 34 -> 30.5, of tiny 23 -> 20.
+// columns of a token, one wave a slot, and adds the slots up itself: no y, no third launch.  Against the grouped route (us a
+// call): one token of the DeepSeek-V3 layer 82 -> 68, of Qwen3-MoE 29.3 -> 14.7, of the full layer behind its norm 55.4 -> 42.5, of mini behind
+// its norm 18.1 -> 12.5, of tiny 13.7 -> 9.1; five tokens of Qwen3-MoE 44.0 -> 33.0, eight 56.3 -> 46.8; sixteen of mini 23.0 -> 20.6, of tiny
+// 14.9 -> 11.1.
 //   Rings of two stages, of one or two K steps each (launch_gateup, launch_down); more of them lose or change nothing (of one
 // K step, one token of DeepSeek-V3: rings of 2 / 3 / 4 / 6 75.6 / 76.8 / 78.1 / 88.2 in the first launch; in the second 2 / 3 are
 // even and 4 / 8 are 7 and 23 % slower).  Workgroups of four waves in the first: 85.8, as 288 of them are uneven on 256 CUs.
-#include "moe_token.h"
-#include "moe_route_device.h"
-
-//   Where all workgroups of the first launch run at once they route, and quantise, their token themselves (token_route_gateup_kernel,
+//   Where the CUs' LDS holds all workgroups of the first launch they route, and quantise, their token themselves (token_route_gateup_kernel,
 // token_front_gateup_kernel): the same work in each, but on otherwise idle CUs, and one launch less.
-//   Nothing that a wave has to wait for stands behind the weights' copies, which complete in order with everything else: codes and scales
-// are copied to LDS in front of them, and the second launch's wave has its whole row of h in registers (2048 values at a time) while the
+//   Nothing that a wave has to wait for stands behind the weights' copies, which complete in order with everything else (but the rows of
+// further slots of a wave of the second launch, and what a row has beyond 2048 values): codes and scales are copied to LDS in front of them, and the second launch's wave has its whole row of h in registers (2048 values at a time) while the
 // selection's index travels, and quantises it while the first weights do.  With loads through registers behind the copies, and h piece by
 // piece (us a call): one token of DeepSeek-V3 73.8 -> 70.3, of the full layer 34.6 -> 32.3, of Qwen3-MoE 18.2 -> 17.0, of tiny 12.9 ->
 // 11.8, of the mini layer behind its norm 15.3 -> 15.0; 8 tokens of 2 of 8 experts of 1024 x 256 beside one of 4096 30.6 -> 24.2.
+#include "moe_token.h"
+#include "moe_route_device.h"
+
 namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -555,20 +556,23 @@ TokenDownPlan moe_token_down_plan(int M, int D, int k, int I, int SI) {
 }
 
 // Every token reads its experts itself, where the grouped kernels read an expert once for all its rows, and a wave of the second
-// launch walks its tiles' K steps one after the other.  What the launches left out and the finer split gain (3 to 13 us) covers
-//  - up to some 320 MB of weights, which 16-row streams read at about 6 TB/s against 6.9 (Qwen3-MoE, 8 tokens = 302 MB 55.4 ->
-//    50.6 us, 10 = 377 MB 60.6 -> 67.3; full layer, 2 tokens = 277 MB 74.2 -> 69.4, 3 = 415 MB 87.2 -> 94.5; DeepSeek-V3, 2
-//    tokens = 793 MB 113.6 -> 130);
+// launch walks its tiles' K steps one after the other.  What the launches left out and the finer split gain (3 to 15 us) covers (us a call,
+// grouped / this way)
+//  - up to some 320 MB of weights, which 16-row streams read at about 6 TB/s against 6.9 (Qwen3-MoE, 8 tokens = 302 MB 56.3 /
+//    46.8, 10 = 377 MB 66.4 / 64.2, 12 = 453 MB 71.5 / 73.5; full layer behind its norm, 2 tokens = 277 MB 72.0 / 65.4, 3 = 415 MB 82.3 /
+//    88.0).  The line is from before the launch in front of the experts fell away and is on the careful side (9 tokens of
+//    Qwen3-MoE 61.0 / 54.8; DeepSeek-V3, 2 tokens = 793 MB 154 / 125);
 //  - of these, megabytes that are read again, and eight times the K steps that the second launch's longest chain has beyond one
-//    tile's, up to 300 (grouped / this way, us, of layers that the memory-side cache holds).  A shared expert eight times as
-//    wide, D 1024, 2 of 32 experts of 512: 4 tokens (no further steps) 31.6 / 25.9, 8 (32) 33.4 / 33.6, 12 (64) 34.8 / 47.0, 16 (96)
-//    35.1 / 49.6.  D 4096, 2 of 4 experts of 1024: 4 tokens (24) 31.5 / 27.3, 8 (56, 144 MB again) 32.3 / 34.6, 12 32.6 / 44.5.
-//    8 of 8 experts, D 1024 x 1024: 8 tokens (8, 168 MB) 24.5 / 22.1, 12 (24, 264 MB) 25.7 / 29.0; 8 of 8, 16 and 32 experts of
-//    2048 x 768, 8 tokens (18 and 252, 216 and 144 MB) 28.0 / 27.7, 29.5 / 29.0, 38.3 / 36.0.  In some 170 layers and batches of such
-//    kinds the choice by this line is 0.3 % slower than the better route on average, 13 % at worst (by the first line alone:
-//    2.3 and 41 %).
-// One token reads nothing twice and gains at any size (396 MB of DeepSeek-V3: 84 -> 76).  Of layers this small that keeps up to
-// 16 tokens: at 24 the mini layer and tiny are even (34.6 / 34.9, 22.1 / 22.2), at 48 36 -> 47 and 23.4 -> 31.7.
+//    tile's, up to 300 (of layers that the memory-side cache holds).  A shared expert eight times as
+//    wide, D 1024, 2 of 32 experts of 512: 4 tokens (no further steps) 24.8 / 15.1, 8 (32) 26.6 / 20.8, 12 (64) 27.2 / 29.3, 16 (96)
+//    28.4 / 34.6.  D 4096, 2 of 4 experts of 1024: 4 tokens (24) 25.7 / 19.0, 8 (56, 144 MB again) 26.0 / 24.9, 12 26.2 / 33.5.
+//    8 of 8 experts, D 1024 x 1024: 8 tokens (8, 168 MB) 17.6 / 17.2, 12 (24, 264 MB) 17.8 / 25.5; 8 of 8, 16 and 32 experts of
+//    2048 x 768, 8 tokens (18 and 252, 216 and 144 MB) 20.8 / 22.5, 22.8 / 24.8, 32.0 / 34.8.  In 170 drawn layers and batches of 2 to 16
+//    tokens the choice by this line is 0.9 % slower than the better route on average (by the first line alone 2.4 %), 41 % at worst: small
+//    layers whose down projection is one launch with the combine (moe_small.hip) lose where an expert has many tokens (13 tokens of 8 of 8
+//    experts of 512 x 1408 17.1 / 24.2).
+// One token reads nothing twice and gains at any size (396 MB of DeepSeek-V3: 82 -> 68).  Above 16 tokens nothing is taken: 24 were even
+// with the grouped route when that had three launches more.
 bool moe_token_takes(int M, int D, int E, int k, int I, int SI) {
   const int widest = I > SI ? I : SI;
   if (M < 1 || M > MOE_TOKEN_ROWS || k < 1 || k >= MOE_TOKEN_SLOTS || up_lds(D) > kLds || down_wave_lds(widest, 1) > kDownLds) return false;

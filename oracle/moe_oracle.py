@@ -4,7 +4,7 @@ This module restates, in NumPy, the algorithm of jax-gpt's MoE layer
 (reference: jax_gpt/models/qwen35/moe.py) extended with the block-scaled fp8
 format and the DeepSeek-V3 group-limited router that the benchmark configs
 name.  Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may
-import it, and only as the checker; the product path never does.
+import it, and only to check against; the product path never does.
 
 What pins each function (tests/test_oracle.py holds the checks):
 
