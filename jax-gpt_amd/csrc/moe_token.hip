@@ -350,6 +350,10 @@ __host__ __device__ constexpr int down_wave_lds(int I, int tiles, int ks = 1) {
   return STAGES * 16 * BK * ks + I + (I / BK * 4 + 15) / 16 * 16 + ((tiles * (I / BK) + 63) / 64 * 256);
 }
 
+// with the lane that CTRL pairs this one with, in one instruction (0 from outside)
+template <int CTRL> __device__ __forceinline__ unsigned max_dpp(unsigned v) {
+  return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true));
+}
 constexpr int H_PIECES = 8;   // of four values a lane: 2048 of a row
 
 // A workgroup: `tiles` neighbouring tiles of 16 output columns of a token; a wave: a slot's row (several, if there are more
@@ -369,7 +373,8 @@ __global__ __launch_bounds__(1024) void token_down_kernel(const TokenArgs a, con
   const float* sw = (const float*)(ring + sw_at);   // [tile][kb]
   const unsigned ring_at = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)ring);
   // What the sums need, and what a wave needs first: all under way before anything is waited for (copies come behind them).
-  float wv = 0.f, rv[DOWN_TILES * COLS / 64];
+  float wv = 0.f;
+  unsigned rv[DOWN_TILES * COLS / 64];   // (bits, converted below: a conversion would wait here)
   if (w == waves - 1) {
     if (lane < a.k) wv = a.w[(size_t)t * a.k + lane];
     else if (a.shared_gate && lane == a.k) wv = a.shared_gate[t];
@@ -378,7 +383,7 @@ __global__ __launch_bounds__(1024) void token_down_kernel(const TokenArgs a, con
 #pragma unroll
       for (int i = 0; i < DOWN_TILES * COLS / 64; ++i)
         if (i * 64 + lane < count * COLS)
-          rv[i] = a.io_f32 ? ((const float*)a.residual)[at + i * 64 + lane] : bf16_to_f32(((const bf16_t*)a.residual)[at + i * 64 + lane]);
+          rv[i] = a.io_f32 ? ((const unsigned*)a.residual)[at + i * 64 + lane] : ((const bf16_t*)a.residual)[at + i * 64 + lane];
   }
   // the slot's row of h, some of it in registers: the loads of the first slot are under way before its expert is known
   v4f hv[H_PIECES];
@@ -400,7 +405,7 @@ __global__ __launch_bounds__(1024) void token_down_kernel(const TokenArgs a, con
     if (a.residual)
 #pragma unroll
       for (int i = 0; i < DOWN_TILES * COLS / 64; ++i)
-        if (i * 64 + lane < count * COLS) residual[i * 64 + lane] = bf16_to_f32(f32_to_bf16(rv[i]));   // (of bf16: itself)
+        if (i * 64 + lane < count * COLS) residual[i * 64 + lane] = bf16_to_f32(a.io_f32 ? f32_to_bf16(__uint_as_float(rv[i])) : (bf16_t)rv[i]);
   }
   for (int j = 0; j < count; ++j) {
     for (int slot = w; slot < slots; slot += waves) {
@@ -420,8 +425,8 @@ __global__ __launch_bounds__(1024) void token_down_kernel(const TokenArgs a, con
                  ring_at + sw_at + i * 4u);
           }
           rows.start({x.w_down + ((size_t)e * a.D + first * COLS) * K}, K, count, (size_t)COLS * K, ring_at);
-          // the row's quantisation groups, 32 lanes each (the maximum by DPP: where a wave has two slots the launch waits for its
-          // instructions, and with five shuffles 16 tokens of 32 of 256 experts of 1024 x 128 took 25.9 us for 24.0)
+          // the row's quantisation groups, 32 lanes each (the maximum by lane permutations: where a wave has two slots the launch waits
+          // for its instructions, and with five shuffles 16 tokens of 32 of 256 experts of 1024 x 128 took 25.9 us for 24.0)
           for (int from = 0; from < K / 4; from += 64 * H_PIECES) {
             if (from || slot != w) load_h(slot, from);
 #pragma unroll
@@ -433,11 +438,12 @@ __global__ __launch_bounds__(1024) void token_down_kernel(const TokenArgs a, con
 #pragma unroll
               for (int r = 0; r < 4; ++r) amax = fmaxf(amax, fabsf(v[r]));
               unsigned m = __float_as_uint(amax);   // (not negative: ordered as integers)
-              m = max(m, dpp<DPP_XOR1>(m));
-              m = max(m, dpp<DPP_XOR2>(m));
-              m = max(m, dpp<DPP_MIRROR8>(m));
-              m = max(m, dpp<DPP_MIRROR16>(m));
-              m = max(m, (unsigned)__shfl_xor((int)m, 16, MOE_WAVE));
+              m = max_dpp<DPP_XOR1>(m);
+              m = max_dpp<DPP_XOR2>(m);
+              m = max_dpp<DPP_MIRROR8>(m);
+              m = max_dpp<DPP_MIRROR16>(m);
+              const auto pair = __builtin_amdgcn_permlane16_swap(m, m, false, false);   // (even rows of 16 lanes twice, and odd ones)
+              m = max(pair[0], pair[1]);
               float scale, scale_inv;
               fp8_scales(__uint_as_float(m), scale, scale_inv);
               int q = 0;
