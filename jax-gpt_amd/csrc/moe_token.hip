@@ -617,11 +617,13 @@ TokenStages moe_token_stages(int M, int D, int k, int I, int SI, bool from_memor
 // 256 experts.  A given selection (the launch that falls away is the quantiser's): moe_routing and expert_forward_single of tiny, 1 to 16
 // tokens 20.0 / 17.8, of Qwen3-MoE, 1 24.0 / 22.6, 4 37.4 / 36.0, 8 56.7 / 54.8.
 //   The selection is a chain of k steps, and of a step for each group where groups lie across lanes, and all workgroups of a CU repeat it:
-// up to 48 K steps of them in all, a step of the grouped routing being one and a half.  This way against launch by launch, over hidden
-// sizes of 128 to 1024 (shorter rows lose first): softmax, 32 of 64 or 256 experts, 1536 workgroups (48 K) 0.91 to 0.99, 2048 0.93 to
-// 1.05, 3072 0.94 to 1.10, 4096 0.95 to 1.17; 16 of them, 2048 (32 K) 0.87 to 0.92; 8 of 256, 4096 (32 K) 0.88 to 0.96.  Grouped, 8 groups: 32,
-// 1024 (48 K) 0.92 to 1.01, 1536 0.95 to 1.07, 4096 0.99 to 1.28; 16, 2048 (48 K) 0.90 to 0.97; 8, 4096 (48 K) 0.92 to 1.02.  240
-// experts in 48 groups of five, k = 8: 512 (42 K) 0.94, 1024 (84 K) 0.94, 2048 1.01 to 1.10, 4096 1.15 to 1.57.
+// up to 48 K steps of them in all, a step of the grouped routing being one and a half; 64 K and, of more than 128 experts, 128 K
+// where rows of 1024 and more stream meanwhile.  This way against launch by launch, hidden sizes of 128 to 768: softmax, 32 of 64 or 256 experts,
+// 1536 workgroups (48 K) 0.91 to 1.00, 2048 0.93 to 1.05, 3072 0.99 to 1.10, 4096 0.97 to 1.17; 16 of them, 2048 (32 K) 0.87 to 0.92; 8 of 256,
+// 4096 (32 K) 0.88 to 0.96.  Grouped, 8 groups: 32, 1024 (48 K) 0.92 to 1.01, 1536 0.96 to 1.07, 4096 1.06 to 1.28; 16, 2048 (48 K)
+// 0.90 to 0.97; 8, 4096 (48 K) 0.92 to 1.02.  240 experts in 48 groups of five, k = 8: 512 (42 K) 0.94, 1024 (84 K) 0.94, 2048 1.01 to 1.10,
+// 4096 1.15 to 1.57.  D 1024: softmax, 32 of 256 experts, 4096 (128 K) 0.95, of 64, 2048 (64 K) 0.95, 4096 1.04; grouped, 32 of 256, 2560
+// (120 K) 0.97, 4096 0.99 to 1.00, 32 of 64, 1024 (48 K) 1.00, 2560 1.08; 16 of 256, 4096 (96 K) 0.95.
 int moe_token_chain(int routing, int E, int k, int n_group, int topk_group) {
   if (routing != MOE_ROUTING_SIGMOID_GROUPED) return k;
   const int lane_keys = E <= 128 ? 2 : 4, per = n_group > 0 ? E / n_group : 0, lanes = per / lane_keys;
@@ -631,7 +633,8 @@ int moe_token_chain(int routing, int E, int k, int n_group, int topk_group) {
 bool moe_token_routes(int M, int D, int E, int k, int I, int SI, bool selected, int chain) {
   const int lds = up_lds(D);
   const long long workgroups = (long long)M * ((k * I + SI) / COLS);
-  return (selected || (E <= 256 && workgroups * chain <= 48 * 1024)) && lds <= kLds && workgroups <= 256 * (kLds / lds);
+  const long long most = D < 1024 ? 48 : E > 128 ? 128 : 64;
+  return (selected || (E <= 256 && workgroups * chain <= most * 1024)) && lds <= kLds && workgroups <= 256 * (kLds / lds);
 }
 // Behind a small router every workgroup of eight waves repeats the router's matmul.  Mini layer, 96 workgroups a token, launch by
 // launch / this way: 1 token 14.0 / 11.6, 4 14.6 / 13.9, 5 15.2 / 14.6, 8 (768 workgroups) 15.4 / 17.9; behind its norm 1 14.8 / 12.8,

@@ -113,7 +113,7 @@ def test_single_tokens_are_routed_by_workgroups_that_run_at_once(ask):
 
 
 def test_long_selections_are_not_repeated_by_many_workgroups(ask):
-    """Ready logits of 16 tokens, D 512: as many workgroups as 48 K steps of selection, a step more for each group that lies across
+    """Ready logits: as many workgroups as 48 K steps of selection (64 or 128 K from D 1024 on), a step more for each group that lies across
     lanes, and one and a half for each of the grouped routing."""
     softmax, grouped = 0, 1
     want = {(16, 512, 256, 8, 512, 0, softmax, 1, 1): "1",      # 4096 workgroups, 32 K steps
@@ -128,6 +128,8 @@ def test_long_selections_are_not_repeated_by_many_workgroups(ask):
             (16, 512, 240, 8, 512, 0, grouped, 48, 24): "0",
             (16, 512, 240, 8, 512, 0, grouped, 48, 48): "1",    # (all groups are kept: nobody looks at them)
             (2, 512, 192, 8, 512, 0, grouped, 0, 0): "1",       # (refused later)
+            (16, 1024, 256, 32, 128, 0, softmax, 1, 1): "1", (8, 1024, 64, 32, 128, 0, softmax, 1, 1): "1", (9, 1024, 64, 32, 128, 0, softmax, 1, 1): "0",
+            (10, 1024, 256, 32, 128, 0, grouped, 8, 4): "1", (11, 1024, 256, 32, 128, 0, grouped, 8, 4): "0",   # longer rows stream meanwhile
             (1, 7168, 256, 8, 2048, 2048, grouped, 8, 4): "1", (8, 2048, 128, 8, 768, 0, softmax, 1, 1): "1"}
     assert ask(*[("token_chain", *c) for c in want]) == list(want.values())
 
