@@ -12,7 +12,7 @@
 #include "moe_common.h"
 #include "moe_permute_device.h"
 #include "moe_quant_device.h"
-#include "moe_route_device.h"
+#include "moe_front_device.h"
 
 namespace {
 
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(1024) void route_kernel(const RouteArgs a, const Ro
         if (a.src.out_logits)
           for (int e = lane; e < a.E; e += MOE_WAVE) a.src.out_logits[(size_t)t * a.E + e] = row[e];
         if (lane == 0 && a.src.shared_gate && N > a.E)   // the shared expert's gate rides in column E
-          a.src.shared_gate[t] = bf16_to_f32(f32_to_bf16(sigmoid_det(row[a.E])));
+          a.src.shared_gate[t] = front_gate(row[a.E]);
       }
       const int chosen = KIND == ROUTE_SOFTMAX ? route_softmax_token<VPL>(a, row, t).expert : route_grouped_token<VPL>(a, row, t).expert;
       if (lane < a.k) {
@@ -147,7 +147,6 @@ struct FrontJob {
   float *sx, *sx_blocked;
   int32_t* chunk_hist;          // [workgroups][E] or null
 };
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
 template <int KIND, bool NORM>
 __global__ __launch_bounds__(64 * kFrontWaves) void front_kernel(const RouteArgs a, const FrontJob f) {
@@ -175,29 +174,14 @@ __global__ __launch_bounds__(64 * kFrontWaves) void front_kernel(const RouteArgs
     }
   }
   v4i b[GROUPS][4];
-  if (w < KB) {
-#pragma unroll
-    for (int g = 0; g < GROUPS; ++g) {
-      if (16 * g >= N) break;
-      const int n = min(16 * g + fr, N - 1);
-      const v4i* src = (const v4i*)((n < E ? f.w + (size_t)n * D : f.w_extra) + w * 128) + fq;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) b[g][s] = src[4 * s];
-    }
-  }
+  if (w < KB) front_weights(b, f.w, f.w_extra, E, N, D, w);
   if (f.chunk_hist && tid < E) hist[tid] = 0;
   if (NORM) {
 #pragma unroll
     for (int i = 0; i < UNITS; ++i) {
       const int u = w + kFrontWaves * i;
       if (u >= units) break;
-      float ss = 0.f;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float v = bf16_to_f32(in[i].v[j]);
-        ss = __fadd_rn(ss, __fmul_rn(v, v));
-      }
-      ss = wave_sum_f32(ss);
+      const float ss = wave_sum_f32(front_squares(in[i]));
       if (lane == 0) wave_sum[per_row == 2 ? u >> 1 : u][u & (per_row - 1)] = ss;
     }
     __syncthreads();
@@ -209,16 +193,12 @@ __global__ __launch_bounds__(64 * kFrontWaves) void front_kernel(const RouteArgs
     const int p = (u & (per_row - 1)) * 64 + lane, r = per_row == 2 ? u >> 1 : u;
     if (NORM) {
       const float total = per_row == 2 ? __fadd_rn(wave_sum[r][0], wave_sum[r][1]) : wave_sum[r][0];
-      const float rms = __fsqrt_rn(__fadd_rn(__fdiv_rn(total, (float)D), f.eps));
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        in[i].v[j] = f32_to_bf16(__fmul_rn(__fdiv_rn(bf16_to_f32(in[i].v[j]), rms), __fadd_rn(1.0f, wt[i][j / 4][j % 4])));
+      front_norm(in[i], total, D, f.eps, wt[i]);
     }
     if (p < P) pieces[r * P + (p ^ (r & 7))] = __builtin_bit_cast(v4i, in[i]);
   }
   __syncthreads();
   if (w < KB) {
-    v4f acc[GROUPS] = {};
     v4i av[4];
     const int r = fr & (T - 1);   // (rows beyond the tile's: any)
 #pragma unroll
@@ -226,26 +206,20 @@ __global__ __launch_bounds__(64 * kFrontWaves) void front_kernel(const RouteArgs
 #pragma unroll
     for (int g = 0; g < GROUPS; ++g) {
       if (16 * g >= N) break;
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-        acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av[s]), __builtin_bit_cast(bf16x8_t, b[g][s]), acc[g], 0, 0, 0);
+      const v4f acc = front_products(av, b[g]);
       const int n = 16 * g + fr;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (4 * fq + j < T && n < N) products[(w * T + 4 * fq + j) * N + n] = acc[g][j];
+        if (4 * fq + j < T && n < N) products[(w * T + 4 * fq + j) * N + n] = acc[j];
     }
   }
   __syncthreads();
-  for (int i = tid; i < T * N; i += 64 * kFrontWaves) {
-    float s = products[i];
-    for (int kb = 1; kb < KB; ++kb) s = __fadd_rn(s, products[kb * T * N + i]);
-    rows[i] = bf16_to_f32(f32_to_bf16(s));
-  }
+  for (int i = tid; i < T * N; i += 64 * kFrontWaves) rows[i] = front_logit(products + i, KB, T * N);
   __syncthreads();
   for (int tt = w; tt < min(T, a.M - t0); tt += kFrontWaves) {
     const float* row = rows + tt * N;
     if (a.src.out_logits && lane < E) a.src.out_logits[(size_t)(t0 + tt) * E + lane] = row[lane];
-    if (lane == 0 && a.src.shared_gate && N > E) a.src.shared_gate[t0 + tt] = bf16_to_f32(f32_to_bf16(sigmoid_det(row[E])));
+    if (lane == 0 && a.src.shared_gate && N > E) a.src.shared_gate[t0 + tt] = front_gate(row[E]);
     const int chosen = KIND == ROUTE_SOFTMAX ? route_softmax_token<1>(a, row, t0 + tt).expert : route_grouped_token<1>(a, row, t0 + tt).expert;
     if (f.chunk_hist && lane < a.k) atomicAdd(&hist[chosen], 1);
   }
@@ -255,23 +229,9 @@ __global__ __launch_bounds__(64 * kFrontWaves) void front_kernel(const RouteArgs
       const int u = w + kFrontWaves * i;
       if (u >= units) break;
       const int p = (u & (per_row - 1)) * 64 + lane, t = t0 + (per_row == 2 ? u >> 1 : u);
-      float v[8], amax = 0.f;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        v[j] = bf16_to_f32(in[i].v[j]);
-        amax = fmaxf(amax, fabsf(v[j]));
-      }
-      unsigned m = __float_as_uint(amax);   // (not negative: ordered as integers; lanes of one group of 16)
-      m = max(m, dpp<DPP_XOR1>(m));
-      m = max(m, dpp<DPP_XOR2>(m));
-      m = max(m, dpp<DPP_MIRROR8>(m));
-      m = max(m, dpp<DPP_MIRROR16>(m));
-      float scale, scale_inv;
-      fp8_scales(__uint_as_float(m), scale, scale_inv);
+      float scale_inv;
+      const uint2 out = front_codes(in[i], scale_inv);
       if (p < P && t < a.M) {
-        uint2 out;
-        out.x = pack4_e4m3(v[0] * scale, v[1] * scale, v[2] * scale, v[3] * scale);
-        out.y = pack4_e4m3(v[4] * scale, v[5] * scale, v[6] * scale, v[7] * scale);
         ((uint2*)f.xq)[(size_t)t * P + p] = out;
         if ((p & 15) == 0) {
           f.sx[(size_t)t * KB + p / 16] = scale_inv;

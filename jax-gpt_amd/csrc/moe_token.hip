@@ -25,11 +25,10 @@
 // piece (us a call): one token of DeepSeek-V3 73.8 -> 70.3, of the full layer 34.6 -> 32.3, of Qwen3-MoE 18.2 -> 17.0, of tiny 12.9 ->
 // 11.8, of the mini layer behind its norm 15.3 -> 15.0; 8 tokens of 2 of 8 experts of 1024 x 256 beside one of 4096 30.6 -> 24.2.
 #include "moe_token.h"
-#include "moe_route_device.h"
+#include "moe_front_device.h"
 
 namespace {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 constexpr int BK = 128;
 constexpr int COLS = 16;         // output columns of a wave
 constexpr int STAGES = 2;        // of a wave's ring
@@ -192,25 +191,10 @@ __global__ __launch_bounds__(64) void token_gateup_kernel(const TokenArgs a) {
   tile.finish();
 }
 
-// A piece of eight values of a token's row to its codes, scale and LDS; 16 lanes a group (moe_quant_act_block)
+// A piece of eight values of a token's row to its codes and scale in LDS; 16 lanes a group
 __device__ __forceinline__ void quant_piece(const moe_bf16x8& in, int p, uint8_t* codes, float* sx) {
-  float v[8], amax = 0.f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    v[i] = bf16_to_f32(in.v[i]);
-    amax = fmaxf(amax, fabsf(v[i]));
-  }
-  unsigned m = __float_as_uint(amax);   // (not negative: ordered as integers)
-  m = max(m, dpp<DPP_XOR1>(m));
-  m = max(m, dpp<DPP_XOR2>(m));
-  m = max(m, dpp<DPP_MIRROR8>(m));
-  m = max(m, dpp<DPP_MIRROR16>(m));
-  float scale, scale_inv;
-  fp8_scales(__uint_as_float(m), scale, scale_inv);
-  uint2 out;
-  out.x = pack4_e4m3(v[0] * scale, v[1] * scale, v[2] * scale, v[3] * scale);
-  out.y = pack4_e4m3(v[4] * scale, v[5] * scale, v[6] * scale, v[7] * scale);
-  ((uint2*)codes)[p] = out;
+  float scale_inv;
+  ((uint2*)codes)[p] = front_codes(in, scale_inv);
   if ((p & 15) == 0) sx[p >> 4] = scale_inv;
 }
 // LDS writes of all waves are there; the copies stay under way
@@ -277,57 +261,32 @@ __global__ __launch_bounds__(64 * FRONT_WAVES) void token_front_gateup_kernel(co
     if (NORM) wt[0] = ((const v4f*)f.norm)[2 * p], wt[1] = ((const v4f*)f.norm)[2 * p + 1];
   }
   v4i b[GROUPS][4];
-  if (w < KB) {
-#pragma unroll
-    for (int g = 0; g < GROUPS; ++g) {
-      if (16 * g >= N) break;
-      const int n = min(16 * g + fr, N - 1);
-      const v4i* src = (const v4i*)((const bf16_t*)(n < E ? f.w_router : f.w_shared_gate) + (n < E ? (size_t)n * D : 0) + w * 128) + fq;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) b[g][s] = src[4 * s];
-    }
-  }
+  if (w < KB) front_weights(b, (const bf16_t*)f.w_router, (const bf16_t*)f.w_shared_gate, E, N, D, w);
   if (NORM) {
     if (unit < 2) {
-      float ss = 0.f;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float v = bf16_to_f32(in.v[j]);
-        ss = __fadd_rn(ss, __fmul_rn(v, v));
-      }
-      ss = wave_sum_f32(ss);
+      const float ss = wave_sum_f32(front_squares(in));
       if (lane == 0) wave_sum[unit] = ss;
     }
     lds_barrier();
-    const float total = P > 64 ? __fadd_rn(wave_sum[0], wave_sum[1]) : wave_sum[0];
-    const float rms = __fsqrt_rn(__fadd_rn(__fdiv_rn(total, (float)D), f.eps));
-#pragma unroll
-    for (int j = 0; j < 8; ++j) in.v[j] = f32_to_bf16(__fmul_rn(__fdiv_rn(bf16_to_f32(in.v[j]), rms), __fadd_rn(1.0f, wt[j / 4][j % 4])));
+    front_norm(in, P > 64 ? __fadd_rn(wave_sum[0], wave_sum[1]) : wave_sum[0], D, f.eps, wt);
   }
   if (has) pieces[p] = __builtin_bit_cast(v4i, in);
   lds_barrier();
   if (w < KB) {
-    v4f acc[GROUPS] = {};
     v4i av[4];
 #pragma unroll
     for (int s = 0; s < 4; ++s) av[s] = pieces[w * 16 + 4 * s + fq];   // (all sixteen rows of the matrix instruction are this one)
 #pragma unroll
     for (int g = 0; g < GROUPS; ++g) {
       if (16 * g >= N) break;
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-        acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av[s]), __builtin_bit_cast(bf16x8_t, b[g][s]), acc[g], 0, 0, 0);
-      if (fq == 0 && 16 * g + fr < N) products[w * N + 16 * g + fr] = acc[g][0];
+      const v4f acc = front_products(av, b[g]);
+      if (fq == 0 && 16 * g + fr < N) products[w * N + 16 * g + fr] = acc[0];
     }
   }
   lds_barrier();
   if (has) quant_piece(in, p, tile.codes(), tile.sx);
   if (tid < 128)   // (N <= 65)
-    if (tid < N) {
-      float s = products[tid];
-      for (int kb = 1; kb < KB; ++kb) s = __fadd_rn(s, products[kb * N + tid]);
-      logits[tid] = bf16_to_f32(f32_to_bf16(s));
-    }
+    if (tid < N) logits[tid] = front_logit(products + tid, KB, N);
   lds_barrier();
   if (w > 0) return;
   Chosen chosen{};
@@ -341,7 +300,7 @@ __global__ __launch_bounds__(64 * FRONT_WAVES) void token_front_gateup_kernel(co
   if (blockIdx.x == 0) {   // (a routed tile: it has the selection)
     if (lane < a.k) r.idx[(size_t)t * a.k + lane] = chosen.expert, r.w[(size_t)t * a.k + lane] = chosen.weight;
     if (r.src.out_logits && lane < E) r.src.out_logits[(size_t)t * E + lane] = logits[lane];
-    if (lane == 0 && r.src.shared_gate && N > E) r.src.shared_gate[t] = bf16_to_f32(f32_to_bf16(sigmoid_det(logits[E])));
+    if (lane == 0 && r.src.shared_gate && N > E) r.src.shared_gate[t] = front_gate(logits[E]);
   }
 }
 
